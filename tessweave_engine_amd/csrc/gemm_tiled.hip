@@ -2,11 +2,36 @@
 // weight layouts and the GLU form; this file holds the kernel, its epilogue and its launcher.
 #include "gemm_shared.h"
 
+// f(integral_constant<int, 0>), ..., f(integral_constant<int, N - 1>): a loop whose index is a constant
+// expression in the body (the scheduler's group barriers take constants only)
+template <int... Is, typename F>
+__device__ __forceinline__ void tw_unroll_impl(std::integer_sequence<int, Is...>, F&& f) {
+  (f(std::integral_constant<int, Is>{}), ...);
+}
+template <int N, typename F>
+__device__ __forceinline__ void tw_unroll(F&& f) {
+  tw_unroll_impl(std::make_integer_sequence<int, N>{}, f);
+}
+
+// A wave's private use of LDS: its own writes are seen by its own later reads (a wave's LDS operations are executed in
+// order), the compiler only has to leave them in that order.
+__device__ __forceinline__ void tw_wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
 // Epilogue of the tiled kernels: each wave passes its tile through LDS (32 rows at a time) so
 // that a lane stores 8 consecutive columns of one row, whole cache lines instead of 2- or 4-byte
 // pieces; bias, residual, the output type and the SiLU-multiply of GLU pairs are applied here.
-// `lds` must hold 4 waves x 32 rows x (32 * WN + 4) floats and no wave may still read its old contents
-// (the first __syncthreads below sees to that).
+// `lds` must hold 4 waves x (32 rows x (32 * WN + 4) + 32 * WN) floats and no wave may still read its old contents
+// (the __syncthreads below sees to that; afterwards every wave works in its own part).
+//
+// What bounds it is the instruction cache (64 KB, shared by two CUs). Unrolled over the row blocks, the rounds and the
+// eight values of a lane, with every activation inlined at every value, it was 14,000 (gated) to 26,000 instructions, and a
+// gated tile also spilled its accumulators: a tile spent a quarter of its time there. Now only the row blocks are written out
+// (the copy of the accumulators into LDS must name its registers), a round is a loop of a few hundred instructions, and the
+// activation is asked for once a round. 256x256 tiles, K = 3,584, bfloat16: the gated projection of 2,048 rows x 37,888
+// columns 653 -> 491 us, of 8,192 rows 2,479 -> 1,832 us (898 -> 1,215 TFLOP/s); plain products 2 to 5 %.
 template <typename OutT, int WM, int WN, bool GLU>
 __device__ __forceinline__ void tw_tiled_epilogue(f32x16 (&acc)[WM][WN], char* lds, const float* __restrict__ bias,
                                                   const float* residual, long ldr, OutT* C, long ldc, int M, int N,
@@ -14,8 +39,6 @@ __device__ __forceinline__ void tw_tiled_epilogue(f32x16 (&acc)[WM][WN], char* l
   const int r = lane & 31, g = lane >> 5;
   constexpr int WCOLS = 32 * WN;                             // columns of a wave tile
   constexpr int EROW = WCOLS + 4;                            // floats per staged row, padded
-  // (the launcher asks for max(pipeline stages, 4 waves x 32 rows x EROW floats) bytes of LDS)
-  float* stage = reinterpret_cast<float*>(lds) + wave * 32 * EROW;   // (the GLU form below may lay its rows out differently)
   constexpr int CPR = WCOLS / 8;                             // 8-column groups per row
   const bool vec_ok = (ldc % 8 == 0) && (residual == nullptr || ldr % 4 == 0) &&
                       ((uintptr_t)C % 16 == 0) && ((uintptr_t)residual % 16 == 0);
@@ -25,91 +48,59 @@ __device__ __forceinline__ void tw_tiled_epilogue(f32x16 (&acc)[WM][WN], char* l
   // wave tile's row is a multiple of 256 bytes the rows are not padded and the 16-byte pieces of row lr lie
   // at piece ^ (0, 1, 4, 5)[lr % 4]: the 16 lanes that a 16-byte read serves in one pass (four rows, four
   // column groups each) then find 16 different 16-byte columns.
-  // Bias: a lane's group of 8 columns in its round t of a pass through LDS is group (lane + 64 t) % CPR of
-  // the row, which repeats after NB rounds (1 where 64 is a multiple of the groups per row, 3 for 12 groups).
-  // Those NB groups' bias is read once, before the first barrier, instead of eight values at a time in front of
-  // every store (a fifth of a qkv projection's time at 2,048 rows went there).
-  constexpr int NB = 64 % CPR == 0 ? 1 : ((128 % CPR == 0) ? 2 : 3);
-  static_assert((64 * NB) % CPR == 0, "the column groups of a lane repeat after NB rounds");
-  float lane_bias[NB][8];
-  if (!GLU && bias) {
-#pragma unroll
-    for (int b = 0; b < NB; ++b) {
-      const int col = n0 + wn0 + ((lane + 64 * b) % CPR) * 8;
-      if (col + 8 <= N && (uintptr_t)bias % 16 == 0) {
-        const f32x4 b0 = *reinterpret_cast<const f32x4*>(bias + col), b1 = *reinterpret_cast<const f32x4*>(bias + col + 4);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) { lane_bias[b][e] = b0[e]; lane_bias[b][4 + e] = b1[e]; }
-      } else {
-#pragma unroll
-        for (int e = 0; e < 8; ++e) lane_bias[b][e] = col + e < N ? bias[col + e] : 0.f;
-      }
-    }
-  }
   constexpr bool SWIZZLED = GLU && WCOLS % 64 == 0;
   constexpr int SROW = SWIZZLED ? WCOLS : EROW;
-  if (SWIZZLED) stage = reinterpret_cast<float*>(lds) + wave * 32 * SROW;
+  float* stage = reinterpret_cast<float*>(lds) + wave * 32 * SROW;
+  // A plain product's bias: the wave's columns of it go to LDS once, behind all waves' rows (read from memory in front of
+  // every store it cost a fifth of a qkv projection's time at 2,048 rows; in registers a lane needs up to three groups of it).
+  float* bias_stage = reinterpret_cast<float*>(lds) + 4 * 32 * EROW + wave * WCOLS;
   auto swz = [](int row) { return SWIZZLED ? ((row & 1) | ((row & 2) << 1)) : 0; };
+
+  // A residual that is added to a whole tile: all of a row block's values of it are requested in front of the copy into LDS
+  // (in the loop every round would wait for its own: C may be the residual, so no load passes a store).
+  constexpr int ROUNDS = 32 * CPR / 64;
+  const bool ahead = !GLU && residual != nullptr && vec_ok && m0 + 64 * WM <= M && n0 + 64 * WN <= N;
+  f32x4 res[GLU ? 1 : ROUNDS][2];
+  auto request = [&](int i) {
 #pragma unroll
-  for (int i = 0; i < WM; ++i) {
-    __syncthreads();                                          // the pipeline's (or the last round's) LDS reads are done
-#pragma unroll
-    for (int j = 0; j < WN; ++j)
-#pragma unroll
-      for (int e = 0; e < 16; ++e) {
-        const int srow = 8 * (e / 4) + 4 * g + (e % 4);
-        stage[srow * SROW + (((j * 8 + (r >> 2)) ^ swz(srow)) << 2) + (r & 3)] = acc[i][j][e];
-      }
-    __syncthreads();
-    if (GLU) {
-      // a wave tile's columns are [gate 16 | up 16] pairs; a lane forms 8 outputs of one row
-      constexpr int GPR = WCOLS / 16;                         // 8-output groups per row
-#pragma unroll
-      for (int q = lane; q < 32 * GPR; q += 64) {
-        const int lr = q / GPR, og = q % GPR;
-        const int lc = (og >> 1) * 32 + (og & 1) * 8;         // gate columns lc.., up columns lc + 16..
-        const int row = m0 + wm0 + i * 32 + lr, col = n0 + wn0 + lc;
-        if (row >= M || col + 24 > N) continue;               // N is a multiple of 32: groups are whole
-        float v[8], gv[8], uv[8];
-        if (SWIZZLED) {
-          const float* base = stage + lr * SROW;
-          const int piece = lc >> 2, x = swz(lr);
-          const f32x4 g0 = *reinterpret_cast<const f32x4*>(base + ((piece ^ x) << 2));
-          const f32x4 g1 = *reinterpret_cast<const f32x4*>(base + (((piece + 1) ^ x) << 2));
-          const f32x4 u0 = *reinterpret_cast<const f32x4*>(base + (((piece + 4) ^ x) << 2));
-          const f32x4 u1 = *reinterpret_cast<const f32x4*>(base + (((piece + 5) ^ x) << 2));
-#pragma unroll
-          for (int e = 0; e < 4; ++e) { gv[e] = g0[e]; gv[4 + e] = g1[e]; uv[e] = u0[e]; uv[4 + e] = u1[e]; }
-        } else {
-#pragma unroll
-          for (int e = 0; e < 8; ++e) { gv[e] = stage[lr * SROW + lc + e]; uv[e] = stage[lr * SROW + lc + 16 + e]; }
-        }
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          if (bias) { gv[e] += bias[col + e]; uv[e] += bias[col + 16 + e]; }
-          v[e] = tw_glu(gv[e], uv[e], ldr);
-        }
-        OutT* dst = C + (size_t)row * ldc + (n0 + wn0) / 2 + (og >> 1) * 16 + (og & 1) * 8;
-        if (ldc % 8 == 0 && (uintptr_t)C % 16 == 0) {
-          if (sizeof(OutT) == 4) {
-            *reinterpret_cast<f32x4*>(dst) = f32x4{v[0], v[1], v[2], v[3]};
-            *reinterpret_cast<f32x4*>(dst + 4) = f32x4{v[4], v[5], v[6], v[7]};
-          } else {
-            bf16x8 o;
-#pragma unroll
-            for (int e = 0; e < 8; ++e) o[e] = (bf16_t)v[e];
-            *reinterpret_cast<bf16x8*>(dst) = o;
-          }
-        } else {
-#pragma unroll
-          for (int e = 0; e < 8; ++e) dst[e] = tw_from_float<OutT>(v[e]);
-        }
-      }
-      continue;
-    }
-#pragma unroll
-    for (int t = 0; t < 32 * CPR / 64; ++t) {
+    for (int t = 0; t < ROUNDS; ++t) {
       const int q = lane + 64 * t;
+      const float* src = residual + (size_t)(m0 + wm0 + i * 32 + q / CPR) * ldr + n0 + wn0 + (q % CPR) * 8;
+      res[t][0] = *reinterpret_cast<const f32x4*>(src);
+      res[t][1] = *reinterpret_cast<const f32x4*>(src + 4);
+    }
+  };
+  auto finish_ahead = [&](int i) {
+#pragma unroll
+    for (int t = 0; t < ROUNDS; ++t) {
+      const int q = lane + 64 * t;
+      const int lr = q / CPR, lc = (q % CPR) * 8;
+      float v[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v[e] = stage[lr * EROW + lc + e];
+      if (bias) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[e] += bias_stage[lc + e];
+      }
+#pragma unroll
+      for (int e = 0; e < 4; ++e) { v[e] += res[t][0][e]; v[4 + e] += res[t][1][e]; }
+      OutT* dst = C + (size_t)(m0 + wm0 + i * 32 + lr) * ldc + n0 + wn0 + lc;
+      if (sizeof(OutT) == 4) {
+        *reinterpret_cast<f32x4*>(dst) = f32x4{v[0], v[1], v[2], v[3]};
+        *reinterpret_cast<f32x4*>(dst + 4) = f32x4{v[4], v[5], v[6], v[7]};
+      } else {
+        bf16x8 o;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) o[e] = (bf16_t)v[e];
+        *reinterpret_cast<bf16x8*>(dst) = o;
+      }
+    }
+  };
+  // rows i * 32 .. + 31 of any other plain product
+  const long act = residual == nullptr ? ldr : 0;             // (no residual: the stride names an activation, see tw_act)
+  auto finish = [&](int i) {
+#pragma unroll 1
+    for (int q = lane; q < 32 * CPR; q += 64) {
       const int lr = q / CPR, lc = (q % CPR) * 8;
       const int row = m0 + wm0 + i * 32 + lr, col = n0 + wn0 + lc;
       if (row >= M || col >= N) continue;
@@ -118,11 +109,14 @@ __device__ __forceinline__ void tw_tiled_epilogue(f32x16 (&acc)[WM][WN], char* l
       for (int e = 0; e < 8; ++e) v[e] = stage[lr * EROW + lc + e];
       if (bias) {
 #pragma unroll
-        for (int e = 0; e < 8; ++e) v[e] += lane_bias[t % NB][e];
+        for (int e = 0; e < 8; ++e) v[e] += bias_stage[lc + e];
       }
-      if (residual == nullptr && ldr != 0) {                 // (no residual: the stride names an activation, see tw_act)
+      if (act == TW_ACT_RELU_SQUARED) {
 #pragma unroll
-        for (int e = 0; e < 8; ++e) v[e] = tw_act(v[e], ldr);
+        for (int e = 0; e < 8; ++e) v[e] = tw_act(v[e], TW_ACT_RELU_SQUARED);
+      } else if (act == TW_ACT_GELU_ERF) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[e] = tw_act(v[e], TW_ACT_GELU_ERF);
       }
       if (vec_ok && col + 8 <= N) {
         if (residual) {
@@ -150,6 +144,82 @@ __device__ __forceinline__ void tw_tiled_epilogue(f32x16 (&acc)[WM][WN], char* l
             C[(size_t)row * ldc + col + e] = tw_from_float<OutT>(x);
           }
       }
+    }
+  };
+  // the same rows of a gated product: a wave tile's columns are [gate 16 | up 16] pairs, a lane forms 8 outputs of one row
+  auto finish_glu = [&](int i) {
+    constexpr int GPR = WCOLS / 16;                           // 8-output groups per row
+#pragma unroll 1
+    for (int q = lane; q < 32 * GPR; q += 64) {
+      const int lr = q / GPR, og = q % GPR;
+      const int lc = (og >> 1) * 32 + (og & 1) * 8;           // gate columns lc.., up columns lc + 16..
+      const int row = m0 + wm0 + i * 32 + lr, col = n0 + wn0 + lc;
+      if (row >= M || col + 24 > N) continue;                 // N is a multiple of 32: groups are whole
+      float v[8], gv[8], uv[8];
+      if (SWIZZLED) {
+        const float* base = stage + lr * SROW;
+        const int piece = lc >> 2, x = swz(lr);
+        const f32x4 g0 = *reinterpret_cast<const f32x4*>(base + ((piece ^ x) << 2));
+        const f32x4 g1 = *reinterpret_cast<const f32x4*>(base + (((piece + 1) ^ x) << 2));
+        const f32x4 u0 = *reinterpret_cast<const f32x4*>(base + (((piece + 4) ^ x) << 2));
+        const f32x4 u1 = *reinterpret_cast<const f32x4*>(base + (((piece + 5) ^ x) << 2));
+#pragma unroll
+        for (int e = 0; e < 4; ++e) { gv[e] = g0[e]; gv[4 + e] = g1[e]; uv[e] = u0[e]; uv[4 + e] = u1[e]; }
+      } else {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) { gv[e] = stage[lr * SROW + lc + e]; uv[e] = stage[lr * SROW + lc + 16 + e]; }
+      }
+      if (bias) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) { gv[e] += bias[col + e]; uv[e] += bias[col + 16 + e]; }
+      }
+      if (ldr == 0) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[e] = tw_glu(gv[e], uv[e], 0);
+      } else {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[e] = tw_glu(gv[e], uv[e], ldr);
+      }
+      OutT* dst = C + (size_t)row * ldc + (n0 + wn0) / 2 + (og >> 1) * 16 + (og & 1) * 8;
+      if (ldc % 8 == 0 && (uintptr_t)C % 16 == 0) {
+        if (sizeof(OutT) == 4) {
+          *reinterpret_cast<f32x4*>(dst) = f32x4{v[0], v[1], v[2], v[3]};
+          *reinterpret_cast<f32x4*>(dst + 4) = f32x4{v[4], v[5], v[6], v[7]};
+        } else {
+          bf16x8 o;
+#pragma unroll
+          for (int e = 0; e < 8; ++e) o[e] = (bf16_t)v[e];
+          *reinterpret_cast<bf16x8*>(dst) = o;
+        }
+      } else {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) dst[e] = tw_from_float<OutT>(v[e]);
+      }
+    }
+  };
+
+  __syncthreads();                                            // the pipeline's LDS reads are done
+  if (!GLU && bias)
+    for (int c = lane; c < WCOLS; c += 64) bias_stage[c] = n0 + wn0 + c < N ? bias[n0 + wn0 + c] : 0.f;
+#pragma unroll
+  for (int i = 0; i < WM; ++i) {
+    if constexpr (!GLU) {
+      if (ahead) request(i);
+    }
+    tw_wave_lds_fence();                                      // (the last round's reads come first)
+#pragma unroll
+    for (int j = 0; j < WN; ++j)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) {
+        const int srow = 8 * (e / 4) + 4 * g + (e % 4);
+        stage[srow * SROW + (((j * 8 + (r >> 2)) ^ swz(srow)) << 2) + (r & 3)] = acc[i][j][e];
+      }
+    tw_wave_lds_fence();
+    if constexpr (GLU) {
+      finish_glu(i);
+    } else {
+      if (ahead) finish_ahead(i);
+      else finish(i);
     }
   }
 }
@@ -406,17 +476,6 @@ typedef __attribute__((address_space(3))) void* tw_lds_ptr;
 #define TW_DMA_STAGES 4       /* of W, one k-tile each */
 #define TW_DMA_A_SLOTS 3      /* of A, a pair of k-tiles each */
 
-// f(integral_constant<int, 0>), ..., f(integral_constant<int, N - 1>): a loop whose index is a constant
-// expression in the body (the scheduler's group barriers take constants only)
-template <int... Is, typename F>
-__device__ __forceinline__ void tw_unroll_impl(std::integer_sequence<int, Is...>, F&& f) {
-  (f(std::integral_constant<int, Is>{}), ...);
-}
-template <int N, typename F>
-__device__ __forceinline__ void tw_unroll(F&& f) {
-  tw_unroll_impl(std::make_integer_sequence<int, N>{}, f);
-}
-
 template <typename OutT, int WM, int WN, bool GLU>
 __global__ __launch_bounds__(256) void gemm_dma_kernel(const bf16_t* __restrict__ A, long lda,
                                                        const bf16_t* __restrict__ W, long k_steps,
@@ -667,7 +726,7 @@ static int launch_tiled(const T* A, long lda, const T* W, long ldw, const float*
   TW_REQUIRE(SHUF ? (long)(BN / 16) * ldw * 64 * EPF < (1L << 31) : (long)BN * ldw < (1L << 31));
   const int grid = (int)((n_blocks + 7) / 8 * 8);
   const size_t pipeline_bytes = 2 * (size_t)(BM + BN) * (KCH * 16 + 16);
-  const size_t epilogue_bytes = 4 * 32 * (size_t)(32 * WN + 4) * 4;
+  const size_t epilogue_bytes = 4 * (32 * (size_t)(32 * WN + 4) + 32 * WN) * 4;
   const size_t lds_bytes = pipeline_bytes > epilogue_bytes ? pipeline_bytes : epilogue_bytes;
   auto kernel = gemm_tiled_kernel<T, OutT, WM, WN, SHUF, GLU>;
   static bool attribute_set = false;   // per instantiation
@@ -706,7 +765,7 @@ static int launch_dma(const bf16_t* A, long lda, const bf16_t* W, long ldw, cons
   const int grid = (int)((n_blocks + 7) / 8 * 8);
   const size_t pipeline_bytes = TW_DMA_A_SLOTS * (size_t)BM * 128 + TW_DMA_STAGES * (size_t)BN * 64;
   static_assert(TW_DMA_A_SLOTS * BM * 128 + TW_DMA_STAGES * BN * 64 <= 160 * 1024, "a workgroup has 160 KB of LDS");
-  const size_t epilogue_bytes = 4 * 32 * (size_t)(32 * WN + 4) * 4;
+  const size_t epilogue_bytes = 4 * (32 * (size_t)(32 * WN + 4) + 32 * WN) * 4;
   const size_t lds_bytes = pipeline_bytes > epilogue_bytes ? pipeline_bytes : epilogue_bytes;
   auto kernel = gemm_dma_kernel<OutT, WM, WN, GLU>;
   static bool attribute_set = false;   // per instantiation

@@ -323,6 +323,36 @@ def test_linear_all_paths(ops, device, dtype, m, n, k):
         w = w_rows
 
 
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("m,n", [(256, 768), (255, 768), (512, 760), (257, 389)])
+def test_linear_epilogues_at_tile_edges(ops, device, dtype, m, n):
+    """Whole tiles (a residual is requested ahead of a row block), tiles that rows or columns end inside, rows that are no
+    multiple of 16 bytes; the residual another matrix of another stride, in place, and none, each with and without a bias.
+    K = 64: a float32 sum of 64 exact products is off by at most 64 x 2^-24 of the sum of their sizes (below 50 here)."""
+    x = rand((m, 64), dtype, device, 1.0, seed=1)
+    w = rand((n, 64), dtype, device, 0.05, seed=2)
+    bias = rand((n,), torch.float32, device, 0.5, seed=3)
+    wide = rand((m, n + 5), torch.float32, device, 1.0, seed=4)
+    want = (x.double() @ w.double().T).cpu()
+    shuffled = ops.shuffle_weight(w)
+    near = dict(atol=64 * 2.0 ** -24 * 50, rtol=1e-6)
+    big = (ops.GEMM_TILED_256, ops.GEMM_TILED_256X192) if dtype == torch.bfloat16 else ()
+    for force in (ops.GEMM_TILED, ops.GEMM_TILED_WIDE) + big:
+        for b in (None, bias):
+            plain = want + (0 if b is None else b.double().cpu())
+            for residual in (None, wide[:, :n], wide[:, 5:], wide[:, :n].contiguous()):
+                out = torch.full((m, n), float("nan"), device=device)
+                ops.linear(x, shuffled, out, bias=b, residual=residual, force=force)
+                torch.testing.assert_close(out.double().cpu(), plain + (0 if residual is None else residual.double().cpu()), **near)
+            acc = wide[:, :n].clone()
+            ops.linear(x, shuffled, acc, bias=b, residual=acc, force=force)
+            torch.testing.assert_close(acc.double().cpu(), plain + wide[:, :n].double().cpu(), **near)
+    for name, act in (("relu_squared", lambda z: torch.relu(z) ** 2), ("gelu", torch.nn.functional.gelu)):
+        out = torch.full((m, n), float("nan"), dtype=dtype, device=device)
+        ops.linear_act(x, shuffled, out, activation=name, bias=bias)
+        torch.testing.assert_close(out.double().cpu(), act(want + bias.double().cpu()), **tol(dtype, (1e-5, 1e-5), (1e-2, 1e-2)))
+
+
 @pytest.mark.parametrize("m,n,k", [(1024, 3584, 16384), (1100, 3000, 12288), (2048, 3584, 8192)])
 def test_linear_large_tiles_over_k_ranges(ops, device, m, n, k):
     """Many rows, few columns, long K (a down projection): the chosen plan may be 256x256 tiles whose K is
