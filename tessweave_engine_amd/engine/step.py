@@ -47,19 +47,27 @@ def _round_up(v, m):
 
 GRAPH_SEGMENT_RUNS = 8       # layer runs per captured graph after the first
 MIN_LENGTH_CLASS = 512       # steps whose longest sequence is shorter share one captured graph
+SECOND_FORM_REPLAYS = 16     # a captured step's other form (cut into segments or whole) is captured after so many replays
 MAX_GRAPHS = 96              # captured steps kept (one per batch size and length class met); the least recently
                              # replayed one goes first
 
 
 class _Graph:
-    """A captured decode step: several graphs launched one after the other (see Stepper._capture).
+    """A captured decode step: a list of graphs launched one after the other (see Stepper._capture), in one or both of two
+    forms, {cut into segments?: handles}.
 
     BUFFERS names the scratch buffers whose addresses the capture holds, each with its version at the
     time: the capture stays good until one of THOSE is allocated anew (a larger prompt portion growing a
     buffer that only prompt portions use leaves every captured decode step alone)."""
 
-    def __init__(self, handles, logits, generation, buffers):
-        self.handles, self.logits, self.generation, self.buffers = handles, logits, generation, buffers
+    def __init__(self, segmented, handles, logits, generation, buffers):
+        self.forms, self.logits, self.generation, self.buffers = {segmented: handles}, logits, generation, buffers
+        self.replays = 0
+
+    def destroy(self, lib):
+        for handles in self.forms.values():
+            for handle in handles:
+                lib.tw_graph_destroy(handle)
 
 
 class Stepper:
@@ -71,7 +79,8 @@ class Stepper:
         self.device = model.device
         self.dtype = model.dtype
         self.workspace = Workspace(self.device)
-        self.stream = torch.cuda.Stream(device=self.device)
+        self.stream = torch.cuda.Stream(device=self.device)     # captures run here; a step runs on its caller's stream
+        self._end, self._end_stream = None, None                 # the last step's end and the stream it ran on
         self.use_graphs = bool(use_graphs) and model.graph_safe_model
         self._defer_sums = bool(getattr(model, "defers_sums", False))
         self.position_axes = max(1, int(getattr(model, "position_axes", 1)))
@@ -130,18 +139,15 @@ class Stepper:
             torch.cuda.synchronize(self.device)
             lib = library()
             for graph in self._graphs.values():
-                for handle in graph.handles:
-                    lib.tw_graph_destroy(handle)
+                graph.destroy(lib)
         self._graphs = OrderedDict()
         self._warm = set()
 
     def _drop_graph(self, key):
-        """Destroy one captured step (it may still be running: wait for the step's stream first)."""
+        """Destroy one captured step (it may still be running: wait for the last step first)."""
         graph = self._graphs.pop(key)
-        self.stream.synchronize()
-        lib = library()
-        for handle in graph.handles:
-            lib.tw_graph_destroy(handle)
+        self.synchronize()
+        graph.destroy(library())
 
     def close(self):
         self._drop_graphs()
@@ -161,6 +167,9 @@ class Stepper:
             self.token_feed = feed
 
     def synchronize(self):
+        """Wait for the last step, and for whatever its caller has put on the stepper's own stream."""
+        if self._end is not None:
+            self._end.synchronize()
         self.stream.synchronize()
 
     # ---- the step ----------------------------------------------------------------------
@@ -173,23 +182,33 @@ class Stepper:
         if not entries:
             return torch.empty(0, self.model.vocab_size, dtype=torch.float32, device=self.device)
         ctx, ordered, graphable = self.prepare(entries)
-        # A caller that already works on the step's stream (the scheduler with lookahead) needs no hand-over
-        # between streams. Each hand-over is an event and a wait in another hardware queue, unless the two
-        # streams happen to share a queue (one engine in four of a process did, and ran 0.2 ms a step faster).
-        caller = torch.cuda.current_stream(self.device)
-        same = caller.cuda_stream == self.stream.cuda_stream
-        if not same:
-            self.stream.wait_stream(caller)
-        with torch.cuda.stream(self.stream):
-            self.upload(ctx)
+        # The step runs on its caller's stream. On a stream of its own it cost an event and a wait each way, barriers
+        # between two hardware queues unless the two streams happened to share one: 18 and 11 us of idle device a step
+        # (four layers of the 7B shape at batch 8: 734 us with them).
+        stream = torch.cuda.current_stream(self.device)
+        self._follow(stream)
+        try:
+            self._upload(ctx)
             if graphable:
-                logits = self._run_graphable(ctx, (ctx.n_seqs, ctx.kv_bound))
+                logits = self._run_graphable(ctx, (ctx.n_seqs, ctx.kv_bound), stream)
             else:
                 logits = self.model.forward(ctx)
-        if not same:
-            caller.wait_stream(self.stream)
+        finally:
+            # one event a step: the staging buffer is free again, and the next step knows what to follow
+            self._end, self._end_stream = torch.cuda.Event(), stream.cuda_stream
+            self._end.record(stream)
+            self._staging_events[ctx.staging_index] = self._end
         self.finish(ordered)
         return logits
+
+    def _follow(self, stream):
+        """A step on another stream than the last one's waits for that one's end (they share scratch memory), and the
+        scratch memory, which may have been allocated for the other stream, is marked as used on this one as well."""
+        if self._end is None or self._end_stream == stream.cuda_stream:
+            return
+        stream.wait_event(self._end)
+        for tensor in (self._meta_dev, *self.workspace.buffers.values()):
+            tensor.record_stream(stream)
 
     def finish(self, ordered):
         """Record in the cache that the step's tokens are now held."""
@@ -202,14 +221,17 @@ class Stepper:
         """Bring the step's packed metadata to the device (on the current stream): a kernel fetches the parts
         this step filled from the pinned staging buffer, which keeps the step in one queue (a memory copy
         would hand over to the copy engine and back, tens of microseconds of idle queue per step)."""
+        self._upload(ctx)
+        event = torch.cuda.Event()
+        event.record(torch.cuda.current_stream(self.device))
+        self._staging_events[ctx.staging_index] = event
+
+    def _upload(self, ctx):
         k = ctx.staging_index
         if ctx.staging_segments is not None and len(ctx.staging_segments) <= 16:
             ops.upload_words(self._staging[k], self._meta_dev, ctx.staging_segments)
         else:
             self._meta_dev.copy_(self._staging[k], non_blocking=True)
-        event = torch.cuda.Event()
-        event.record(torch.cuda.current_stream(self.device))
-        self._staging_events[k] = event
 
     def prepare(self, entries):
         """Check ENTRIES, take their pages, and build the step's context (host side; nothing runs yet).
@@ -341,15 +363,13 @@ class Stepper:
         return self.cache.layout.groups[group].spec.first_position(computed) // self.cache.page_size * self.cache.page_size
 
     # ---- HIP graphs for decode-only steps ------------------------------------------------
-    def _capture(self, ctx):
-        """Capture model.forward(ctx) as a chain of graphs.
+    def _capture(self, ctx, segmented):
+        """Capture model.forward(ctx) as a chain of graphs (on the stepper's own stream: nothing runs); returns
+        (handles, logits, the scratch buffers whose addresses they hold, each with its version).
 
-        Launching a graph costs host time per node before its first kernel starts. With
-        `segment_graphs` the step is therefore cut after the first layer run and then every
-        GRAPH_SEGMENT_RUNS runs: the first graph is short and starts at once, and every later one
-        is launched while its predecessor still runs. A caller that launches a step while the step
-        before still runs (the scheduler's lookahead) turns it off: the launch is hidden anyway, and
-        every cut costs about 8 us between two graphs.
+        Launching a graph costs host time per node before its first kernel starts. A SEGMENTED step is
+        therefore cut after the first layer run and then every GRAPH_SEGMENT_RUNS runs: the first graph
+        is short and starts at once, and every later one is launched while its predecessor still runs.
         """
         lib = library()
         stream = self.stream.cuda_stream
@@ -365,31 +385,32 @@ class Stepper:
             return code
 
         def segment_end(i):
-            if self.segment_graphs and i + 1 < n_runs and (i == 0 or (i + 1) % GRAPH_SEGMENT_RUNS == 0):
+            if segmented and i + 1 < n_runs and (i == 0 or (i + 1) % GRAPH_SEGMENT_RUNS == 0):
                 check(end_segment(), "graph capture end")
                 check(lib.tw_graph_begin(stream), "graph capture begin")
 
-        check(lib.tw_graph_begin(stream), "graph capture begin")
-        ctx.segment_end = segment_end
-        self.workspace.touched = touched = set()
-        try:
-            logits = self.model.forward(ctx)
-        except BaseException:
-            end_segment()
-            for handle in handles:
-                lib.tw_graph_destroy(handle)
-            raise
-        finally:
-            ctx.segment_end = None
-            self.workspace.touched = None
-        check(end_segment(), "graph capture end")
+        with torch.cuda.stream(self.stream):
+            check(lib.tw_graph_begin(stream), "graph capture begin")
+            ctx.segment_end = segment_end
+            self.workspace.touched = touched = set()
+            try:
+                logits = self.model.forward(ctx)
+            except BaseException:
+                end_segment()
+                for handle in handles:
+                    lib.tw_graph_destroy(handle)
+                raise
+            finally:
+                ctx.segment_end = None
+                self.workspace.touched = None
+            check(end_segment(), "graph capture end")
         if self.workspace.generation != generation:
             for handle in handles:
                 lib.tw_graph_destroy(handle)
             raise RuntimeError("a scratch buffer was allocated during graph capture")
-        return _Graph(handles, logits, generation, {key: self.workspace.versions[key] for key in touched})
+        return handles, logits, {key: self.workspace.versions[key] for key in touched}
 
-    def _run_graphable(self, ctx, key):
+    def _run_graphable(self, ctx, key, stream):
         """KEY = (batch size, length class) names the captured graph this step can be replayed from."""
         graph = self._graphs.get(key)
         if graph is not None and graph.generation != self.workspace.generation:
@@ -399,18 +420,28 @@ class Stepper:
             else:
                 self._drop_graph(key)
                 graph = None
+        # A step that is launched while the step before still runs goes out as one graph: its launch is hidden, and every
+        # cut costs about 8 us between two graphs. (The scheduler's lookahead, whose launches always are, turns cutting off.)
+        segmented = self.segment_graphs and (self._end is None or self._end.query())
         if graph is None:
             if key not in self._warm:
                 # First time at this batch size and length class: run eagerly so every scratch buffer exists.
                 self._warm.add(key)
                 return self.model.forward(ctx)
-            graph = self._graphs[key] = self._capture(ctx)
+            handles, logits, buffers = self._capture(ctx, segmented)
+            graph = self._graphs[key] = _Graph(segmented, handles, logits, self.workspace.generation, buffers)
             while len(self._graphs) > self.max_graphs:
                 self._drop_graph(next(iter(self._graphs)))
         else:
             self._graphs.move_to_end(key)
+            if segmented not in graph.forms:
+                if graph.replays >= SECOND_FORM_REPLAYS:     # (a capture costs as much as some steps)
+                    graph.forms[segmented] = self._capture(ctx, segmented)[0]
+                else:
+                    segmented = not segmented
         lib = library()
-        for handle in graph.handles:
-            check(lib.tw_graph_launch(handle, self.stream.cuda_stream), "graph launch")
+        for handle in graph.forms[segmented]:
+            check(lib.tw_graph_launch(handle, stream.cuda_stream), "graph launch")
+        graph.replays += 1
         self.graph_replays += 1
         return graph.logits

@@ -72,6 +72,37 @@ def test_bfloat16_generation_agrees_where_the_choice_is_clear(tiny):
     assert clear >= total // 4, (clear, total)       # otherwise this test would compare nothing
 
 
+def test_steps_called_from_changing_streams(tiny):
+    """A step runs on its caller's stream. Steps of one request from streams in turn, with other work in front of them and
+    scratch buffers growing in between, give what they give from one stream: each follows the one before."""
+    from tessweave_engine_amd.cache import CacheManager
+    from tessweave_engine_amd.engine import StepEntry, Stepper
+    from tessweave_engine_amd.weights import load_model
+    model = load_model(tiny["folder"], dtype="float32", device="cuda:0")
+    tokens = prompts_for(tiny, [90], seed=4)[0]
+    portions = [tokens[:9]] + [[t] for t in tokens[9:20]] + [tokens[20:70]] + [[t] for t in tokens[70:]]
+    streams = [torch.cuda.default_stream(), torch.cuda.Stream(), torch.cuda.Stream()]
+    busy = torch.randn(2048, 2048, device="cuda")
+
+    def run(turn):
+        cache = CacheManager(model.cache_layout(), tiny["page"], 100, 2, dtype="float32", device=model.device, prefix_cache=False)
+        stepper = Stepper(model, cache, max_step_tokens=16)
+        torch.cuda.synchronize()
+        seq, rows = cache.open("a"), []
+        for i, portion in enumerate(portions):
+            with torch.cuda.stream(streams[turn(i)]):
+                for _ in range(i % 3):
+                    busy @ busy
+                rows.append(stepper.step([StepEntry(seq, portion, [len(portion) - 1])]).clone())
+        stepper.synchronize()
+        torch.cuda.synchronize()
+        assert stepper.graph_replays > 20
+        stepper.close()
+        return torch.cat(rows)
+
+    assert torch.equal(run(lambda i: 0), run(lambda i: i % 3))
+
+
 def test_long_decoding_and_the_first_tokens(tiny):
     """One token after the other for hundreds of steps (pages fill and new ones are taken), from position 0."""
     from tessweave_engine_amd.cache import CacheManager
