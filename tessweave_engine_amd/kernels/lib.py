@@ -78,7 +78,8 @@ _SIGNATURES = {
     "tw_sigmoid_gate": (I, [I, P, L, P, L, I, I, I, P]),
     "tw_softcap_values": (I, [P, L, F, P]),
     "tw_qk_finish": (I, [I, P, L, I, I, P, P, P, P, P, L, P, P, P, I, I, I, I, I, I, I, I, F, P]),
-    "tw_mlstm": (I, [P, L, I, I, I, I, I, P, P, P, P, P, P, P, P, I, I, P, L, I, I, I, F, F, I, I, I, P]),
+    "tw_mlstm_workspace_floats": (L, [I, I, I, I, I]),
+    "tw_mlstm": (I, [P, L, I, I, I, I, I, P, P, P, P, P, P, P, P, I, I, P, L, I, I, I, F, F, I, I, I, I, P, L, P]),
     "tw_embed_sinusoid": (I, [I, P, P, P, P, P, P, P, F, I, I, I, P, I, P]),
     "tw_head_finish": (I, [I, P, L, I, I, I, P, P, L, P, P, P, I, I, I, I, I, I, I, I, F, F, P]),
     "tw_add_normed_sum": (I, [P, I, ctypes.POINTER(c_void_p), ctypes.POINTER(c_int), ctypes.POINTER(c_void_p),

@@ -1346,15 +1346,22 @@ def qk_finish(src, q_col, k_col, q_weight, k_weight, cos, sin, q_out, keys, valu
 MLSTM_WALK_TOKENS = 4          # sequences with up to this many tokens in a step are walked token by token
 
 
+def mlstm_workspace_floats(n_seqs, max_q_len, heads, dim, value_dim):
+    """float32 scratch the chunked form of `mlstm` needs for portions of up to max_q_len tokens (0: none)."""
+    up = lambda v: (int(v) + 15) // 16 * 16       # noqa: E731
+    return int(library().tw_mlstm_workspace_floats(int(n_seqs), int(max_q_len), int(heads), up(dim), up(value_dim)))
+
+
 def mlstm(proj, q_col, k_col, v_col, i_col, f_col, i_bias, f_bias, S, n_state, m_state, q_start, state_slots, phase, seq0,
-          n_seqs, out, heads, dim, value_dim, q_scale, cap, walk, first_row=None):
+          n_seqs, out, heads, dim, value_dim, q_scale, cap, walk, first_row=None, max_q_len=0, workspace=None):
     """The mLSTM's matrix memory over sequences seq0 .. seq0 + n_seqs - 1 of a step. proj float32 rows with q, k
     (heads * dim each), v (heads * value_dim) and the two gates' raw values (heads each) at the given columns; i_bias,
     f_bias float32 [heads]. S float32 [requests, heads, value_dev, dim_dev], n_state [requests, 2, heads, dim_dev], m_state
     [requests, 2, heads] (copy phase[s] is read, the other written). out float32 [rows, heads * value_dim]: S^T q over its
     denominator. walk: token by token (steps of a few tokens a sequence), else chunks of 16 on the matrix unit; then
     first_row, if given, says that the launch's sequences own the rows from there to proj's last: their gates are formed
-    first by a kernel of their own, IN PLACE of the raw values in proj."""
+    first by a kernel of their own, IN PLACE of the raw values in proj. With a workspace (float32, mlstm_workspace_floats of
+    max_q_len, which no sequence of the launch exceeds) long sequences are cut into segments for separate workgroups."""
     n, width, ld = _rows(proj, "proj")
     no, wo, ld_out = _rows(out, "out")
     dim_dev, value_dev = (dim + 15) // 16 * 16, (value_dim + 15) // 16 * 16
@@ -1370,11 +1377,15 @@ def mlstm(proj, q_col, k_col, v_col, i_col, f_col, i_bias, f_bias, S, n_state, m
         _need(t.dtype == torch.float32 and t.is_contiguous() and t.numel() == heads, f"{name} must be float32 [heads]")
     _need(q_start.numel() >= seq0 + n_seqs + 1 and state_slots.numel() >= seq0 + n_seqs and phase.numel() >= seq0 + n_seqs,
           "sequence metadata is too short")
+    _need(workspace is None or (workspace.dtype == torch.float32 and workspace.is_contiguous() and max_q_len > 0 and
+          workspace.numel() >= mlstm_workspace_floats(n_seqs, max_q_len, heads, dim, value_dim)), "mlstm: the workspace is too small")
     check(library().tw_mlstm(_dev(proj), ld, int(q_col), int(k_col), int(v_col), int(i_col), int(f_col), _dev(i_bias), _dev(f_bias),
                              _dev(S), _dev(n_state), _dev(m_state), _dev(q_start, torch.int32, "q_start"),
                              _dev(state_slots, torch.int32, "state_slots"), _dev(phase, torch.int32, "phase"), int(seq0),
                              int(n_seqs), _dev(out), ld_out, int(heads), int(dim), int(value_dim), float(q_scale), float(cap),
-                             1 if walk else 0, -1 if (walk or first_row is None) else int(first_row), n, _stream()), "mlstm")
+                             1 if walk else 0, -1 if (walk or first_row is None) else int(first_row), n, int(max_q_len),
+                             _dev(workspace) if workspace is not None else None, workspace.numel() if workspace is not None else 0,
+                             _stream()), "mlstm")
     return out
 
 

@@ -10,7 +10,7 @@ in range (Beck et al., "xLSTM: Extended Long Short-Term Memory").
 S, n and m (all zero when a request opens, m too) are the mixer's whole memory: float32 states in its cache slot. The
 packed product leaves float32 rows; gates, exponentials, the state and all products with it are float32 in both
 precisions. One-token (and few-token) sequences are walked token by token, longer portions run in chunks of 16 on the
-matrix unit: the same sums in another order.
+matrix unit, long ones in segments of chunks side by side: the same sums in another order.
 """
 from __future__ import annotations
 
@@ -96,7 +96,10 @@ class MatrixLSTM(Mixer):
                 ops.mlstm(*common, 0, ctx.n_decode, *tail, walk=True)
             if portions:
                 # (one-token sequences own the first rows of a step: the portions' rows are the rest)
-                ops.mlstm(*common, ctx.n_decode, portions, *tail, walk=False, first_row=ctx.n_decode)
+                floats = ops.mlstm_workspace_floats(portions, ctx.max_q_len, H, D, E)
+                ws = ctx.workspace.get("mlstm.segments", (floats,), torch.float32) if floats else None
+                ops.mlstm(*common, ctx.n_decode, portions, *tail, walk=False, first_row=ctx.n_decode, max_q_len=ctx.max_q_len,
+                          workspace=ws)
         act = ctx.scratch("mlstm.act", (n, H * E))
         ops.head_norm_gate(result, proj[:, col["g"]:col["g"] + H * E], self.norm_weight, act, H, E, self.eps,
                            gate_activation="sigmoid")

@@ -326,6 +326,39 @@ def test_mlstm_over_cut_sequences_in_reused_slots(device, H, D, E, walk):
         assert err < 5e-5, (s, float(err))          # (float32 sums in another order than the plain float64 walk)
 
 
+@pytest.mark.parametrize("H,D,E,open_gates", [(2, 128, 128, True), (3, 20, 72, False), (1, 200, 16, True)])
+def test_mlstm_in_segments(device, H, D, E, open_gates):
+    """Portions long enough to be cut into segments for separate workgroups (one that ends inside a chunk, one too short to
+    be cut, one of a single token), then portions that continue from the states they leave; forget gates near one (the state
+    remembers thousands of tokens) and around a half."""
+    from tessweave_engine_amd.kernels import ops
+    g = torch.Generator().manual_seed(H + D + E)
+    cap, width = 6.0, 2 * H * D + H * E + 2 * H
+    Dp, Ep = (D + 15) // 16 * 16, (E + 15) // 16 * 16
+    i_b, f_b = torch.randn(H, generator=g).to(device), ((5.0 if open_gates else 0.0) + torch.randn(H, generator=g)).to(device)
+    cuts = [[701, 400], [100, 513], [1, 64]]
+    proj = [torch.randn(sum(c), width, generator=g).to(device) for c in cuts]
+    wants = [mlstm_plain_heads(p, H, D, E, i_b, f_b, cap) for p in proj]
+    S, n_st, m_st = (torch.zeros(3, *shape, device=device) for shape in ((H, Ep, Dp), (2, H, Dp), (2, H)))
+    at, outs = [0, 0, 0], [[], [], []]
+    for step in range(2):
+        lens = [c[step] for c in cuts]
+        rows = torch.cat([p[a:a + n] for p, a, n in zip(proj, at, lens)]).contiguous()
+        q_start = [0, lens[0], lens[0] + lens[1], sum(lens)]
+        out = torch.full((len(rows), H * E), float("nan"), device=device)
+        floats = ops.mlstm_workspace_floats(3, max(lens), H, D, E)
+        assert floats > 0 and ops.mlstm_workspace_floats(3, 64, H, D, E) == 0
+        ops.mlstm(rows, 0, H * D, 2 * H * D, width - 2 * H, width - H, i_b, f_b, S, n_st, m_st, ints(q_start, device),
+                  ints([2, 0, 1], device), ints([step] * 3, device), 0, 3, out, H, D, E, D ** -0.5, cap, False, first_row=0,
+                  max_q_len=max(lens), workspace=torch.full((floats,), float("nan"), device=device))
+        for s in range(3):
+            outs[s].append(out[q_start[s]:q_start[s + 1]])
+            at[s] += lens[s]
+    for s in range(3):
+        err = (torch.cat(outs[s]).double().cpu() - wants[s]).abs().max() / wants[s].abs().max()
+        assert err < 5e-5, (s, float(err))          # (as above: float32 sums in another order than the plain float64 walk)
+
+
 # ---------------------------------------------------------------------------------------------------------
 # whole models
 
