@@ -19,8 +19,9 @@
 // chunk's tokens out, norm q and k, form beta and g, then all walk the chunk.
 #include "tw_common.h"
 
-#define TW_DELTA_CHUNK 16
+#define TW_DELTA_CHUNK 16             /* tokens the walk stages at a time */
 #define TW_DELTA_WALK_MOST 4          /* up to this many tokens a sequence, a step walks them one by one */
+#define TW_DELTA_SHORT_MOST 48        /* up to this many, it solves chunks of 16 tokens in one launch; beyond, of 32 in two */
 
 struct DeltaArgs {
   const float* qkv; long ld_qkv;      // q of key head j at q_col + j * D, k at k_col + j * D, v of head h at v_col + h * E
@@ -168,25 +169,412 @@ __device__ __forceinline__ void delta_lds_barrier() {
   asm volatile("" ::: "memory");
 }
 
-// ---- many tokens a sequence: chunks of 16 tokens, each solved at once ----------------------------------------------
+// ---- many tokens a sequence: chunks of 32 tokens, solved side by side, then walked ----------------------------------
 // Inside a chunk with state S0 at its start, L_i = sum_{m <= i} log g_m (so that G_i = exp(L_i) and every quotient
 // G_i / G_j, j <= i, is an exponential of a sum of logarithms that are at most 0):
 //   u_i = beta_i (v_i - G_i S0^T k_i) - sum_{j < i} A_ij u_j,      A_ij = beta_i (G_i / G_j) (k_i . k_j)
-//   o_i = G_i S0^T q_i + sum_{j <= i} (G_i / G_j) (q_i . k_j) u_j
+//   o_i = G_i S0^T q_i + sum_{j <= i} M_ij u_j,                    M_ij = (G_i / G_j) (q_i . k_j)
 //   S   = G_last S0 + sum_j (G_last / G_j) k_j u_j^T
-// which is the token-by-token rule written out. All products are float32 on the matrix unit (16x16x4). A workgroup
-// owns 16 value columns of one (sequence, head); its four waves own a quarter of the key elements each (NT tiles of 16),
-// and a wave's part of S stays in registers in the layout that is both the B operand of K S and the accumulator of
-// K^T W: lane (c, g) holds S[16 tile + 4 g + j][c]. Per chunk: the waves form their parts of K S0, Q S0, K K^T and
-// Q K^T from the same fragments (the key rows of a chunk are the A operand of the first and both operands of the third),
-// the parts meet in LDS and thread 16 i + j adds them up for the pair (i, j) and puts decay, beta and the unit norms on
-// (q and k are multiplied as they come; their squared lengths are the diagonals of K K^T and of one more product, Q Q^T); every lane solves
-// the triangular system of its column by substitution (after u_j is final every later row takes its term off: one
-// multiply-add deep a token); one wave reads the chunk's outputs out (one more product), every wave updates its part
-// of S. Tokens behind a sequence's end are staged as zeros with beta = 0 and g = 1: they change nothing. The next
-// chunk's rows are on their way from memory while this one is worked on.
+// which is the token-by-token rule written out. All of it but the products with S0 is the same whatever the state is: with
+// T = (I + A)^-1, W = T (beta G K) and U0 = T (beta V)
+//   U = U0 - W S0,    O = M U0 + (G Q - M W) S0,    S = G_last S0 + K'^T U.
+// delta_prepare forms W, Q' = G Q - M W, K', U0 and O0 = M U0 for every (chunk, head) at once; delta_chunk then goes through a
+// sequence's chunks with three products each. Everything is float32, the products on the matrix unit (16x16x4). T comes from
+// substitution, a column a lane, in blocks of 16 tokens (a series in powers of A would lose digits where keys are alike).
+//
+// What bounds them: delta_chunk the chain from chunk to chunk and the 48 KB of operands a chunk that each of its workgroups
+// reads (2 us a chunk, 30 GB/s a CU), delta_prepare its own length: written out over the 32 tokens with a thread a column it
+// was 4,000 instructions, executed once, and took 32 us for one chunk. Solved inside the chain (chunks of 16 tokens, four
+// barriers each) a chunk took 4.5 us. 16 heads of 128, the two launches
+// together: one sequence of 2,048 tokens 579 -> 170 us, two of 800 and 1,200 tokens 340 -> 120 us, 100 tokens 34 -> 24 us.
+#define TW_DELTA_PREP 32              /* tokens a chunk */
+
+struct DeltaPrepared {                // per (chunk, head), all in the order the walk's lanes read them, 16 bytes a lane
+  float* W;                           // [4 waves][NT][2][64][4]: A operands, row = token, reduction = the wave's key elements
+  float* Q;                           // the same of Q'
+  float* K;                           // [4][NT][2][64][4]: A operands of K'^T, row = key element, reduction = token
+  float* U;                           // [value tiles][2][64][4]: accumulators, row = token, column = value
+  float* O;                           // the same of O0
+  float* G;                           // [1]: G_last
+};
+
+// The number of the first chunk of a sequence: chunks of sequences never overlap whatever their lengths, and there are at
+// most rows / 32 + sequences of them.
+__device__ __forceinline__ int delta_first_chunk(const DeltaArgs& a, int seq0, int s) {
+  return (a.q_start[s] - a.q_start[seq0]) / TW_DELTA_PREP + (s - seq0);
+}
+
+// grid (chunk numbers, H), 256 threads
 template <int NT>
-__global__ __launch_bounds__(256) void delta_chunk_kernel(DeltaArgs a, int seq0) {
+__global__ __launch_bounds__(256) void delta_prepare_kernel(DeltaArgs a, DeltaPrepared out, int seq0, int n_seqs) {
+  constexpr int C = TW_DELTA_PREP, DP = 64 * NT, ROW = DP + 4, PW = C + 4;
+  __shared__ __attribute__((aligned(16))) float q_s[C][ROW];
+  __shared__ __attribute__((aligned(16))) float k_s[C][ROW];
+  __shared__ __attribute__((aligned(16))) float at_s[C][PW];     // k_j . k_i, then A_ij at [j][i] (0 unless j < i)
+  __shared__ __attribute__((aligned(16))) float m_s[C][PW];      // q_i . k_j, then M_ij at [i][j] (0 unless j <= i)
+  __shared__ __attribute__((aligned(16))) float t_s[C][PW];      // T (its block above the diagonal is never read)
+  __shared__ __attribute__((aligned(16))) float mt_s[C][PW];     // M T
+  __shared__ float beta_s[C], lg_s[C], g_s[C], kn_s[C], qn_s[C], tail_s[C];
+  const int chunk = blockIdx.x, head = blockIdx.y;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  // the sequence this chunk number belongs to: the last one whose first chunk is not behind it
+  int s = -1;
+  for (int s0 = 0; s0 < n_seqs; s0 += 64) {
+    const bool in = s0 + lane < n_seqs && delta_first_chunk(a, seq0, seq0 + s0 + lane) <= chunk;
+    const int n = __popcll(__ballot(in));
+    s = n ? s0 + n - 1 : s;
+    if (n < 64) break;
+  }
+  s += seq0;
+  const int t0 = a.q_start[s] + (chunk - delta_first_chunk(a, seq0, s)) * C, last = a.q_start[s + 1];
+  if (t0 >= last) return;                            // (a number that no chunk has)
+  const int kh = head / (a.H / a.G);
+
+  // ---- rows and gates into LDS (tokens behind the sequence's end: zeros, beta = 0, g = 1) -----------------------------
+  // (Loads are whole, from clamped places, and issued together: a load behind a condition waits for the one before.)
+  const int r = lane & 15, g = lane >> 4;
+  const int value_tiles = (a.E + 15) / 16;
+  auto values = [&](int x, f32x4* vf) {              // value tile x: the B operands of a product over tokens
+    const float* v = a.qkv + a.v_col + (size_t)head * a.E + min(16 * x + r, a.E - 1);
+#pragma unroll
+    for (int tt = 0; tt < 2; ++tt)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) vf[tt][j] = v[(size_t)min(t0 + 16 * tt + 4 * g + j, last - 1) * a.ld_qkv];
+  };
+  f32x4 vf[2];
+  values(min(wave, value_tiles - 1), vf);            // (needed at the end only)
+  const bool vec = a.D % 4 == 0 && a.ld_qkv % 4 == 0 && a.q_col % 4 == 0 && a.k_col % 4 == 0 && (uintptr_t)a.qkv % 16 == 0;
+  if (vec) {
+    constexpr int N = C * DP / 4 / 256;
+    f32x4 qv[N], kv[N];
+#pragma unroll
+    for (int n = 0; n < N; ++n) {
+      const int x = threadIdx.x + 256 * n, t = x / (DP / 4), d = (x % (DP / 4)) * 4;
+      const float* row = a.qkv + (size_t)min(t0 + t, last - 1) * a.ld_qkv + (size_t)kh * a.D + min(d, a.D - 4);
+      qv[n] = *reinterpret_cast<const f32x4*>(row + a.q_col);
+      kv[n] = *reinterpret_cast<const f32x4*>(row + a.k_col);
+    }
+#pragma unroll
+    for (int n = 0; n < N; ++n) {
+      const int x = threadIdx.x + 256 * n, t = x / (DP / 4), d = (x % (DP / 4)) * 4;
+      const bool in = t0 + t < last && d < a.D;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) { qv[n][j] = in ? qv[n][j] : 0.f; kv[n][j] = in ? kv[n][j] : 0.f; }
+      *reinterpret_cast<f32x4*>(&q_s[t][d]) = qv[n];
+      *reinterpret_cast<f32x4*>(&k_s[t][d]) = kv[n];
+    }
+  } else {
+    for (int x = threadIdx.x; x < C * DP; x += 256) {
+      const int t = x / DP, d = x % DP;
+      const bool in = t0 + t < last && d < a.D;
+      const float* row = a.qkv + (size_t)min(t0 + t, last - 1) * a.ld_qkv + (size_t)kh * a.D + min(d, a.D - 1);
+      const float qv = row[a.q_col], kv = row[a.k_col];
+      q_s[t][d] = in ? qv : 0.f;
+      k_s[t][d] = in ? kv : 0.f;
+    }
+  }
+  if (threadIdx.x < C) {
+    const bool in = t0 + threadIdx.x < last;
+    const float* ab = a.ab + (size_t)(in ? t0 + threadIdx.x : t0) * a.ld_ab;
+    beta_s[threadIdx.x] = in ? 1.f / (1.f + expf(-ab[a.b_col + head])) : 0.f;
+    lg_s[threadIdx.x] = in ? -expf(a.A_log[head]) * delta_softplus(ab[a.a_col + head] + a.dt_bias[head]) : 0.f;
+  }
+  __syncthreads();
+
+  // ---- K K^T and Q K^T, the three tiles on and below the diagonal by a wave each; the fourth wave: squared lengths ------
+  if (wave < 3) {
+    const int ti = wave ? 1 : 0, tj = wave == 2 ? 1 : 0;
+    f32x4 kk = {0.f, 0.f, 0.f, 0.f}, qk = kk;
+#pragma unroll
+    for (int x = 0; x < 4 * NT; ++x) {
+      const f32x4 kj = *reinterpret_cast<const f32x4*>(&k_s[16 * tj + r][16 * x + 4 * g]);
+      tw_mma16(kk, *reinterpret_cast<const f32x4*>(&k_s[16 * ti + r][16 * x + 4 * g]), kj);
+      tw_mma16(qk, *reinterpret_cast<const f32x4*>(&q_s[16 * ti + r][16 * x + 4 * g]), kj);
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      at_s[16 * tj + r][16 * ti + 4 * g + j] = kk[j];
+      m_s[16 * ti + 4 * g + j][16 * tj + r] = qk[j];
+    }
+  } else {
+    const int t = lane >> 1;
+    float qq = 0.f, kk = 0.f;
+    for (int d = (lane & 1) * 4; d < DP; d += 8) {
+      const f32x4 qv = *reinterpret_cast<const f32x4*>(&q_s[t][d]), kv = *reinterpret_cast<const f32x4*>(&k_s[t][d]);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) { qq = __fmaf_rn(qv[j], qv[j], qq); kk = __fmaf_rn(kv[j], kv[j], kk); }
+    }
+    qq += __shfl_xor(qq, 1, TW_WAVE);
+    kk += __shfl_xor(kk, 1, TW_WAVE);
+    if (!(lane & 1)) {
+      kn_s[t] = 1.f / sqrtf(kk + 1e-6f);
+      qn_s[t] = a.q_scale / sqrtf(qq + 1e-6f);
+    }
+  }
+  __syncthreads();
+
+  // ---- the decay between tokens, beta and the unit norms put on them ----------------------------------------------------
+  {
+    const int j = threadIdx.x % C, i0 = threadIdx.x / C;         // this thread's pairs: (i0 + 8 p, j)
+    float between[4] = {0.f, 0.f, 0.f, 0.f};         // logs of G_i / G_j (j <= i), summed over the tokens in between
+#pragma unroll 8
+    for (int m = 0; m < C; ++m) {
+      const float lg = m > j ? lg_s[m] : 0.f;
+#pragma unroll
+      for (int p = 0; p < 4; ++p) between[p] += m <= i0 + 8 * p ? lg : 0.f;
+    }
+#pragma unroll
+    for (int p = 0; p < 4; ++p) {
+      const int i = i0 + 8 * p;
+      const float decay = expf(between[p]);
+      at_s[j][i] = j < i ? beta_s[i] * decay * (kn_s[i] * kn_s[j]) * at_s[j][i] : 0.f;
+      m_s[i][j] = j <= i ? decay * (qn_s[i] * kn_s[j]) * m_s[i][j] : 0.f;
+      if (i == C - 1) tail_s[j] = decay * kn_s[j];
+      if (j == 0) g_s[i] = expf(between[p] + lg_s[0]);
+    }
+  }
+  __syncthreads();
+
+  // ---- T = (I + A)^-1, by the first wave: the two diagonal blocks by substitution (a lane a column), then the block below ---
+  if (wave == 0) {
+    if (lane < 32) {
+      const int b = lane & 16;                       // the block's first token
+      float x[16];
+#pragma unroll
+      for (int i = 0; i < 16; ++i) x[i] = i == r ? 1.f : 0.f;
+#pragma unroll
+      for (int j = 0; j < 15; ++j)
+#pragma unroll
+        for (int i4 = (j + 1) / 4 * 4; i4 < 16; i4 += 4) {
+          const f32x4 v = *reinterpret_cast<const f32x4*>(&at_s[b + j][b + i4]);
+#pragma unroll
+          for (int y = 0; y < 4; ++y)
+            if (i4 + y > j) x[i4 + y] = __fmaf_rn(-v[y], x[j], x[i4 + y]);
+        }
+#pragma unroll
+      for (int i = 0; i < 16; ++i) t_s[b + i][b + r] = x[i];
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    f32x4 below, left, p = {0.f, 0.f, 0.f, 0.f}, t21 = p;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      below[j] = at_s[4 * g + j][16 + r];            // A of the lower tokens on the upper ones, row r
+      left[j] = t_s[4 * g + j][r];
+    }
+    tw_mma16(p, below, left);                        // an accumulator, and the next product's B operand
+    tw_mma16(t21, *reinterpret_cast<const f32x4*>(&t_s[16 + r][16 + 4 * g]), p);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) t_s[16 + 4 * g + j][r] = -t21[j];
+  }
+  __syncthreads();
+
+  // ---- M T, its three tiles on and below the diagonal by a wave each --------------------------------------------------------
+  if (wave < 3) {
+    const int ti = wave ? 1 : 0, tj = wave == 2 ? 1 : 0;
+    f32x4 mt = {0.f, 0.f, 0.f, 0.f};
+    for (int tk = tj; tk <= ti; ++tk) {
+      f32x4 tf;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) tf[j] = t_s[16 * tk + 4 * g + j][16 * tj + r];
+      tw_mma16(mt, *reinterpret_cast<const f32x4*>(&m_s[16 * ti + r][16 * tk + 4 * g]), tf);
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) mt_s[16 * ti + 4 * g + j][16 * tj + r] = mt[j];
+  }
+  __syncthreads();
+
+  // ---- the five results -----------------------------------------------------------------------------------------------------
+  const size_t unit = (size_t)chunk * a.H + head;
+  if (threadIdx.x == 0) out.G[unit] = g_s[C - 1];
+  // rows of T and M T (tiles 00, 10, 11), their columns times beta G / |k| for the keys and times beta for the values
+  f32x4 tk[3], mk[3], tv[3], mv[3];
+#pragma unroll
+  for (int t = 0; t < 3; ++t) {
+    const int row = (t ? 16 : 0) + r, col = (t == 2 ? 16 : 0) + 4 * g;
+    const f32x4 tr = *reinterpret_cast<const f32x4*>(&t_s[row][col]), mr = *reinterpret_cast<const f32x4*>(&mt_s[row][col]);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const float bv = beta_s[col + j], bk = bv * g_s[col + j] * kn_s[col + j];
+      tk[t][j] = tr[j] * bk;
+      mk[t][j] = mr[j] * bk;
+      tv[t][j] = tr[j] * bv;
+      mv[t][j] = mr[j] * bv;
+    }
+  }
+  // keys, a tile of 16 a wave and round: K^T is the A operand, so that a lane ends with four key elements of one token, which
+  // is how the walk takes W and Q', and K' is K^T itself
+  float* W = out.W + unit * C * DP + lane * 4;
+  float* Q = out.Q + unit * C * DP + lane * 4;
+  float* K = out.K + unit * C * DP + lane * 4;
+#pragma unroll 1
+  for (int x = wave; x < 4 * NT; x += 4) {
+    f32x4 kf[2], w[2], q[2];
+#pragma unroll
+    for (int tt = 0; tt < 2; ++tt) {
+      f32x4 tail;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        kf[tt][j] = k_s[16 * tt + 4 * g + j][16 * x + r];
+        tail[j] = kf[tt][j] * tail_s[16 * tt + 4 * g + j];
+      }
+      *reinterpret_cast<f32x4*>(K + (x * 2 + tt) * 256) = tail;
+      w[tt] = q[tt] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+    tw_mma16(w[0], kf[0], tk[0]);
+    tw_mma16(q[0], kf[0], mk[0]);
+    tw_mma16(w[1], kf[0], tk[1]);
+    tw_mma16(q[1], kf[0], mk[1]);
+    tw_mma16(w[1], kf[1], tk[2]);
+    tw_mma16(q[1], kf[1], mk[2]);
+#pragma unroll
+    for (int tt = 0; tt < 2; ++tt) {
+      const float gq = g_s[16 * tt + r] * qn_s[16 * tt + r];
+      const f32x4 qv = *reinterpret_cast<const f32x4*>(&q_s[16 * tt + r][16 * x + 4 * g]);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) q[tt][j] = __fmaf_rn(gq, qv[j], -q[tt][j]);
+      *reinterpret_cast<f32x4*>(W + (x * 2 + tt) * 256) = w[tt];
+      *reinterpret_cast<f32x4*>(Q + (x * 2 + tt) * 256) = q[tt];
+    }
+  }
+  // values, a tile of 16 columns a wave and round (columns behind the last one: the last one's, which nobody reads)
+  float* U = out.U + unit * C * 16 * value_tiles + lane * 4;
+  float* O = out.O + unit * C * 16 * value_tiles + lane * 4;
+#pragma unroll 1
+  for (int x = wave; x < value_tiles; x += 4) {
+    f32x4 u[2], o[2], next[2];
+    values(min(x + 4, value_tiles - 1), next);
+#pragma unroll
+    for (int tt = 0; tt < 2; ++tt) u[tt] = o[tt] = f32x4{0.f, 0.f, 0.f, 0.f};
+    tw_mma16(u[0], tv[0], vf[0]);
+    tw_mma16(o[0], mv[0], vf[0]);
+    tw_mma16(u[1], tv[1], vf[0]);
+    tw_mma16(o[1], mv[1], vf[0]);
+    tw_mma16(u[1], tv[2], vf[1]);
+    tw_mma16(o[1], mv[2], vf[1]);
+#pragma unroll
+    for (int tt = 0; tt < 2; ++tt) {
+      *reinterpret_cast<f32x4*>(U + (x * 2 + tt) * 256) = u[tt];
+      *reinterpret_cast<f32x4*>(O + (x * 2 + tt) * 256) = o[tt];
+      vf[tt] = next[tt];
+    }
+  }
+}
+
+// grid (H * value tiles, n_seqs). A workgroup owns 16 value columns of one (sequence, head); its four waves own a quarter of
+// the key elements each (NT tiles of 16), and a wave's part of S stays in registers in the layout that is both the B operand of
+// W S and Q' S and the accumulator of K'^T U: lane (c, g) holds S[16 tile + 4 g + j][c]. Per chunk the waves' parts of the two
+// products meet in LDS (twice, so that one barrier a chunk is enough), every wave adds them up and updates its part of S, two
+// waves write the outputs. A chunk's operands are requested two chunks ahead.
+template <int NT>
+__global__ __launch_bounds__(256) void delta_chunk_kernel(DeltaArgs a, DeltaPrepared in, int seq0) {
+  constexpr int C = TW_DELTA_PREP, DP = 64 * NT;
+  __shared__ __attribute__((aligned(16))) f32x4 part_s[2][4][4][64];   // [copy][wave][W S of two token tiles, Q' S of two][lane]
+  const int value_tiles = (a.E + 15) / 16;
+  const int eb = blockIdx.x % value_tiles, head = blockIdx.x / value_tiles;
+  const int s = seq0 + blockIdx.y;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int r = lane & 15, g = lane >> 4;
+  const int e = eb * 16 + r;                         // this lane's value column
+  const bool live = e < a.E;
+  const int first = a.q_start[s], last = a.q_start[s + 1];
+  if (first >= last) return;
+  const int chunks = (last - first + C - 1) / C;
+  const size_t unit0 = (size_t)delta_first_chunk(a, seq0, s) * a.H + head;
+  const int d_wave = 16 * NT * wave;                 // the wave's first key element
+  float* S_mem = a.state + (((size_t)a.state_slots[s] * a.H + head) * a.E + (live ? e : 0)) * a.Dk;
+  f32x4 S[NT];
+#pragma unroll
+  for (int mm = 0; mm < NT; ++mm) {
+    const int d0 = d_wave + 16 * mm + 4 * g;
+    S[mm] = f32x4{0.f, 0.f, 0.f, 0.f};
+    if (live && d0 < a.Dk) S[mm] = *reinterpret_cast<const f32x4*>(S_mem + d0);
+  }
+  struct Operands {
+    f32x4 w[NT][2], q[NT][2], k[NT][2], u[2], o;
+    float G;
+  };
+  auto request = [&](int chunk, Operands& x) __attribute__((always_inline)) {
+    const size_t unit = unit0 + (size_t)chunk * a.H;
+    const size_t keys = unit * C * DP + (size_t)wave * NT * 512 + lane * 4;
+    const size_t values = (unit * value_tiles + eb) * 512 + lane * 4;
+#pragma unroll
+    for (int mm = 0; mm < NT; ++mm)
+#pragma unroll
+      for (int tt = 0; tt < 2; ++tt) {
+        x.w[mm][tt] = *reinterpret_cast<const f32x4*>(in.W + keys + (mm * 2 + tt) * 256);
+        x.q[mm][tt] = *reinterpret_cast<const f32x4*>(in.Q + keys + (mm * 2 + tt) * 256);
+        x.k[mm][tt] = *reinterpret_cast<const f32x4*>(in.K + keys + (mm * 2 + tt) * 256);
+      }
+#pragma unroll
+    for (int tt = 0; tt < 2; ++tt) x.u[tt] = *reinterpret_cast<const f32x4*>(in.U + values + tt * 256);
+    x.o = *reinterpret_cast<const f32x4*>(in.O + values + (wave & 1) * 256);
+    x.G = in.G[unit];
+  };
+  auto link = [&](int chunk, int copy, Operands& x) __attribute__((always_inline)) {
+    f32x4 pw[2], pq[2];
+#pragma unroll
+    for (int tt = 0; tt < 2; ++tt) pw[tt] = pq[tt] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int mm = 0; mm < NT; ++mm)
+#pragma unroll
+      for (int tt = 0; tt < 2; ++tt) {
+        tw_mma16(pw[tt], x.w[mm][tt], S[mm]);        // [token][column]
+        tw_mma16(pq[tt], x.q[mm][tt], S[mm]);
+      }
+#pragma unroll
+    for (int tt = 0; tt < 2; ++tt) {
+      part_s[copy][wave][tt][lane] = pw[tt];
+      part_s[copy][wave][2 + tt][lane] = pq[tt];
+    }
+    delta_lds_barrier();
+    // U of tokens 16 tt + 4 g .. + 3: an accumulator, and the B operand of the product over tokens
+#pragma unroll
+    for (int tt = 0; tt < 2; ++tt)
+      x.u[tt] -= (part_s[copy][0][tt][lane] + part_s[copy][1][tt][lane]) + (part_s[copy][2][tt][lane] + part_s[copy][3][tt][lane]);
+#pragma unroll
+    for (int mm = 0; mm < NT; ++mm) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) S[mm][j] *= x.G;
+#pragma unroll
+      for (int tt = 0; tt < 2; ++tt) tw_mma16(S[mm], x.k[mm][tt], x.u[tt]);
+    }
+    if (wave < 2) {
+      const f32x4 o = x.o + ((part_s[copy][0][2 + wave][lane] + part_s[copy][1][2 + wave][lane]) +
+                             (part_s[copy][2][2 + wave][lane] + part_s[copy][3][2 + wave][lane]));
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int t = first + chunk * C + 16 * wave + 4 * g + j;
+        if (live && t < last) a.out[(size_t)t * a.ld_out + (size_t)head * a.E + e] = o[j];
+      }
+    }
+    if (chunk + 2 < chunks) request(chunk + 2, x);   // (its registers are free again)
+  };
+  Operands even, odd;
+  request(0, even);
+  if (chunks > 1) request(1, odd);
+  for (int c = 0; c < chunks; c += 2) {
+    link(c, 0, even);
+    if (c + 1 < chunks) link(c + 1, 1, odd);
+  }
+#pragma unroll
+  for (int mm = 0; mm < NT; ++mm) {
+    const int d0 = d_wave + 16 * mm + 4 * g;
+    if (live && d0 < a.Dk) *reinterpret_cast<f32x4*>(S_mem + d0) = S[mm];
+  }
+}
+
+// ---- portions of a few dozen tokens: chunks of 16 tokens, each solved inside the chain --------------------------------
+// One launch instead of two: up to 48 tokens (three chunks of 4.5 us behind 2.5 us of start) it ends before delta_prepare and
+// delta_chunk would (13 + 7 us at 33 tokens, 16 heads of 128). A workgroup owns 16 value columns of one (sequence, head) and its
+// waves a quarter of the key elements each, as above. Per chunk: the waves form their parts of K S0, Q S0, K K^T and Q K^T from
+// the same fragments, the parts meet in LDS and thread 16 i + j adds them up for the pair (i, j) and puts decay, beta and the
+// unit norms on (q and k are multiplied as they come; their squared lengths are the diagonals of K K^T and of one more product,
+// Q Q^T); every lane solves the triangular system of its column by substitution; one wave reads the chunk's outputs out, every
+// wave updates its part of S. Tokens behind a sequence's end are staged as zeros with beta = 0 and g = 1: they change nothing.
+// The next chunk's rows are on their way from memory while this one is worked on.
+template <int NT>
+__global__ __launch_bounds__(256) void delta_short_kernel(DeltaArgs a, int seq0) {
   constexpr int C = 16, DP = 64 * NT;                // key elements, rounded up: 16 NT a wave
   constexpr int ROW = DP + 4;                        // (+ 4: the four token rows a transposed read meets lie 16 banks apart)
   constexpr int PW = C + 4;
@@ -383,10 +771,35 @@ __global__ __launch_bounds__(256) void delta_chunk_kernel(DeltaArgs a, int seq0)
   }
 }
 
+// float32 scratch of a launch over n_seqs sequences of up to `rows` rows together (0: it needs none)
+extern "C" long tw_delta_workspace_floats(int rows, int n_seqs, int max_q_len, int H, int E, int Dk) {
+  if (n_seqs <= 0 || rows <= 0 || max_q_len <= TW_DELTA_SHORT_MOST) return 0;
+  const long units = ((long)rows / TW_DELTA_PREP + n_seqs) * H;
+  const long DP = Dk <= 64 ? 64 : Dk <= 128 ? 128 : 256;
+  return units * (TW_DELTA_PREP * (3 * DP + 2L * tw_div_up(E, 16) * 16) + 4);
+}
+
+template <int NT>
+static int delta_chunks(const DeltaArgs& a, int seq0, int n_seqs, int rows, float* workspace, hipStream_t stream) {
+  const size_t chunks = (size_t)rows / TW_DELTA_PREP + n_seqs, units = chunks * a.H;
+  const size_t keys = units * TW_DELTA_PREP * 64 * NT, values = units * TW_DELTA_PREP * 16 * tw_div_up(a.E, 16);
+  DeltaPrepared p;
+  p.W = workspace;
+  p.Q = p.W + keys;
+  p.K = p.Q + keys;
+  p.U = p.K + keys;
+  p.O = p.U + values;
+  p.G = p.O + values;
+  delta_prepare_kernel<NT><<<dim3((unsigned)chunks, a.H), 256, 0, stream>>>(a, p, seq0, n_seqs);
+  delta_chunk_kernel<NT><<<dim3(a.H * tw_div_up(a.E, 16), n_seqs), 256, 0, stream>>>(a, p, seq0);
+  return TW_LAUNCH_RESULT();
+}
+
 extern "C" int tw_delta_rule(const float* qkv, long ld_qkv, int q_col, int k_col, int v_col, const float* ab, long ld_ab,
                              int b_col, int a_col, const float* A_log, const float* dt_bias, float* state,
                              const int* q_start, const int* state_slots, float* out, long ld_out, int seq0, int n_seqs,
-                             int max_q_len, int H, int G, int D, int E, int Dk, float q_scale, hipStream_t stream) {
+                             int max_q_len, int H, int G, int D, int E, int Dk, float q_scale, int rows, float* workspace,
+                             long workspace_floats, hipStream_t stream) {
   TW_REQUIRE(qkv && ab && A_log && dt_bias && state && q_start && state_slots && out);
   TW_REQUIRE(H > 0 && G > 0 && H % G == 0 && D > 0 && D <= 256 && E > 0 && Dk >= D && Dk % 4 == 0 && Dk <= 256);
   TW_REQUIRE(max_q_len >= 1);
@@ -397,12 +810,18 @@ extern "C" int tw_delta_rule(const float* qkv, long ld_qkv, int q_col, int k_col
   if (n_seqs == 0) return 0;
   DeltaArgs a{qkv, ld_qkv, q_col, k_col, v_col, ab, ld_ab, b_col, a_col, A_log, dt_bias, state, q_start, state_slots,
               out, ld_out, H, G, D, E, Dk, q_scale};
-  if (max_q_len > TW_DELTA_WALK_MOST) {
-    // some sequence brings many tokens: every sequence of the step goes through the kernel that solves chunks at once
+  if (max_q_len > TW_DELTA_SHORT_MOST) {
+    // some sequence brings many tokens: every sequence of the step goes through the chunks
+    TW_REQUIRE(workspace != nullptr && (uintptr_t)workspace % 16 == 0 && rows > 0 && H <= 65535 &&
+               workspace_floats >= tw_delta_workspace_floats(rows, n_seqs, max_q_len, H, E, Dk));
+    if (Dk <= 64) return delta_chunks<1>(a, seq0, n_seqs, rows, workspace, stream);
+    if (Dk <= 128) return delta_chunks<2>(a, seq0, n_seqs, rows, workspace, stream);
+    return delta_chunks<4>(a, seq0, n_seqs, rows, workspace, stream);
+  } else if (max_q_len > TW_DELTA_WALK_MOST) {
     const dim3 grid(H * tw_div_up(E, 16), n_seqs);
-    if (Dk <= 64) delta_chunk_kernel<1><<<grid, 256, 0, stream>>>(a, seq0);
-    else if (Dk <= 128) delta_chunk_kernel<2><<<grid, 256, 0, stream>>>(a, seq0);
-    else delta_chunk_kernel<4><<<grid, 256, 0, stream>>>(a, seq0);
+    if (Dk <= 64) delta_short_kernel<1><<<grid, 256, 0, stream>>>(a, seq0);
+    else if (Dk <= 128) delta_short_kernel<2><<<grid, 256, 0, stream>>>(a, seq0);
+    else delta_short_kernel<4><<<grid, 256, 0, stream>>>(a, seq0);
   } else if (Dk <= 16) {
     delta_walk_kernel<4, 4><<<dim3(H * tw_div_up(E, 64), n_seqs), 256, 0, stream>>>(a, seq0);
   } else {

@@ -1098,8 +1098,14 @@ def delta_key_extent(dim):
     return (int(dim) + 3) // 4 * 4
 
 
+def delta_workspace_floats(rows, n_seqs, max_q_len, heads, value_dim, dim):
+    """float32 scratch `delta_rule` needs for sequences of up to max_q_len tokens in a step of that many rows (0: none)."""
+    return int(library().tw_delta_workspace_floats(int(rows), int(n_seqs), int(max_q_len), int(heads), int(value_dim),
+                                                   delta_key_extent(dim)))
+
+
 def delta_rule(qkv, q_col, k_col, v_col, ab, b_col, a_col, A_log, dt_bias, state, q_start, state_slots, seq0, n_seqs, out,
-               kv_heads, dim, q_scale, max_q_len=1):
+               kv_heads, dim, q_scale, max_q_len=1, workspace=None):
     """The gated delta rule over sequences seq0 .. seq0 + n_seqs - 1, from and to state float32
     [requests, H, E, Dk] (a column of S is contiguous; Dk = delta_key_extent(dim)):
 
@@ -1109,8 +1115,9 @@ def delta_rule(qkv, q_col, k_col, v_col, ab, b_col, a_col, A_log, dt_bias, state
     qkv float32 [n, .]: q of key head j at q_col + j * dim, k at k_col + j * dim, v of head h at v_col + h * E;
     ab float32 [n, .]: b of head h at b_col + h, a at a_col + h; value head h reads key head h // (H / kv_heads).
     out float32 [n, H * E]. max_q_len: the most tokens a sequence brings (an upper bound will do). Up to a few tokens
-    a sequence the tokens are walked one by one; beyond, chunks of 16 tokens are solved at once (the same sums in another
-    order: a triangular system a chunk in place of a chain of updates)."""
+    a sequence the tokens are walked one by one; beyond, chunks of 16 or 32 tokens are solved at once (the same sums in another
+    order: a triangular system a chunk in place of a chain of updates), with a float32 workspace of delta_workspace_floats
+    (allocated here if none is given)."""
     n, wq, ld_qkv = _rows(qkv, "qkv")
     na, wa, ld_ab = _rows(ab, "ab")
     _need(qkv.dtype == torch.float32 and ab.dtype == torch.float32 and na == n, "the delta rule reads float32 rows")
@@ -1125,10 +1132,16 @@ def delta_rule(qkv, q_col, k_col, v_col, ab, b_col, a_col, A_log, dt_bias, state
     _need(A_log.numel() == H and dt_bias.numel() == H and A_log.dtype == torch.float32 and dt_bias.dtype == torch.float32,
           "one float32 A_log and dt_bias per head")
     _need(seq0 >= 0 and q_start.numel() >= seq0 + n_seqs + 1 and state_slots.numel() >= seq0 + n_seqs, "sequence metadata is too short")
+    floats = delta_workspace_floats(n, n_seqs, max(1, int(max_q_len)), H, E, D)
+    if floats and workspace is None:
+        workspace = torch.empty(floats, dtype=torch.float32, device=qkv.device)
+    _need(not floats or (workspace.dtype == torch.float32 and workspace.is_contiguous() and workspace.numel() >= floats),
+          "delta_rule: the workspace is too small")
     check(library().tw_delta_rule(_dev(qkv), ld_qkv, int(q_col), int(k_col), int(v_col), _dev(ab), ld_ab, int(b_col), int(a_col),
                                   _dev(A_log), _dev(dt_bias), _dev(state), _dev(q_start, torch.int32, "q_start"),
                                   _dev(state_slots, torch.int32, "state_slots"), _dev(out), ldo, int(seq0), int(n_seqs),
-                                  max(1, int(max_q_len)), H, G, D, E, Dk, float(q_scale), _stream()), "delta_rule")
+                                  max(1, int(max_q_len)), H, G, D, E, Dk, float(q_scale), n, _dev(workspace) if floats else None,
+                                  workspace.numel() if floats else 0, _stream()), "delta_rule")
     return out
 
 

@@ -204,6 +204,31 @@ def test_delta_rule_long_portions_solved_in_chunks(device, H, G, D, E):
         assert (res - ref).abs().max() < 1e-4 * max(1.0, ref.abs().max().item()), (res - ref).abs().max()
 
 
+@pytest.mark.parametrize("H,G,D,E", [(2, 1, 20, 24), (1, 1, 130, 40)])
+def test_delta_rule_chunks_of_many_sequences(device, H, G, D, E):
+    """84 sequences of lengths around a chunk's 32 tokens in one launch that leaves its step's first sequence alone: every
+    chunk finds its sequence, against the same sequences walked token by token (both float32: twice the bar above)."""
+    from tessweave_engine_amd.kernels import ops
+    g = torch.Generator().manual_seed(D)
+    lens = [7] + [1, 31, 32, 33, 64, 65, 5] * 12
+    n = sum(lens)
+    starts, slots = ints(np.cumsum([0] + lens).tolist(), device), ints(torch.randperm(len(lens), generator=g).tolist(), device)
+    qkv, ab = torch.randn(n, 2 * G * D + H * E, generator=g).to(device), torch.randn(n, 2 * H, generator=g).to(device)
+    A_log, dt_bias = (-2.0 + 0.5 * torch.randn(H, generator=g)).to(device), (-3.0 + torch.randn(H, generator=g)).to(device)
+    first = torch.randn(len(lens), H, E, ops.delta_key_extent(D), generator=g).to(device)
+    first[..., D:] = 0
+    results = []
+    for most in (1, 48, 65):                # (48: the kernel for short portions, which takes longer ones as well)
+        state, out = first.clone(), torch.zeros(n, H * E, device=device)
+        ops.delta_rule(qkv, 0, G * D, 2 * G * D, ab, 0, H, A_log, dt_bias, state, starts, slots, 1, len(lens) - 1, out, G, D,
+                       D ** -0.5, max_q_len=most)
+        results.append((out, state))
+    for result in results:
+        assert not result[0][:7].any() and torch.equal(result[1][slots[0]], first[slots[0]])
+        for walked, chunked in zip(results[0], result):
+            assert (walked - chunked).abs().max() < 4e-5 * max(1.0, walked.abs().max().item())
+
+
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 def test_head_norm_with_gate(device, dtype):
     from tessweave_engine_amd.kernels import ops
