@@ -326,6 +326,38 @@ def test_mlstm_over_cut_sequences_in_reused_slots(device, H, D, E, walk):
         assert err < 5e-5, (s, float(err))          # (float32 sums in another order than the plain float64 walk)
 
 
+@pytest.mark.parametrize("hidden", [4, 1023, 2048, 6000, 12000, 16388])
+@pytest.mark.parametrize("splits", [0, 1, 9])
+def test_row_norms_of_every_length(device, hidden, splits):
+    """Rows in one, two and four groups a thread, longer ones and ones of no whole groups; a strided result, one and nine
+    partial sums (more than are requested at a time). Float32 sums of `hidden` squares: 1e-5 of the values is twenty times
+    what rounding leaves of them."""
+    from tessweave_engine_amd.kernels import ops
+    g = torch.Generator().manual_seed(hidden + splits)
+    n = 3
+    x, w, b, scale = torch.randn(n, hidden, generator=g), 1 + torch.randn(hidden, generator=g), torch.randn(hidden, generator=g), torch.randn(hidden, generator=g)
+    wide, parts = torch.randn(n, hidden + 4, generator=g), torch.randn(max(1, splits), n, hidden, generator=g)
+    y = (parts.double().sum(0) if splits else wide[:, 4:].double())
+    given = dict(add=parts.to(device)) if splits else dict(y=wide.to(device)[:, 4:])
+
+    def layer(v, weight, bias):
+        v = v - v.mean(-1, keepdim=True)
+        return v / torch.sqrt((v * v).mean(-1, keepdim=True) + 1e-5) * weight.double() + bias.double()
+    cases = [(ops.add_normed, (w, 1e-5, 0.7), x.double() + 0.7 * plain.rms_norm(y, w.double(), 1e-5), None),
+             (ops.residual_norm, (w, 1e-5), plain.rms_norm(0.5 * x.double() + scale.double() * y, w.double(), 1e-5), dict(scale=scale.to(device), alpha=0.5)),
+             (ops.layer_norm, (1e-5,), None, dict(post=(w.to(device), b.to(device)), norm=(scale.to(device), b.to(device))))]
+    for op, args, want, more in cases:
+        got, out = x.clone().to(device), torch.full((n, hidden), float("nan"), device=device)
+        op(got, *(a.to(device) if torch.is_tensor(a) else a for a in args), out=out, **given, **(more or {}))
+        if want is None:
+            stream = x.double() + layer(y, w, b)
+            want, want_out = stream, layer(stream, scale, b)
+        else:
+            want_out = want
+        for a, ref in ((got, want), (out, want_out)):
+            assert ((a.double().cpu() - ref).abs() <= 1e-5 * (1 + ref.abs())).all(), op.__name__
+
+
 @pytest.mark.parametrize("H,D,E,open_gates", [(2, 128, 128, True), (3, 20, 72, False), (1, 200, 16, True)])
 def test_mlstm_in_segments(device, H, D, E, open_gates):
     """Portions long enough to be cut into segments for separate workgroups (one that ends inside a chunk, one too short to
