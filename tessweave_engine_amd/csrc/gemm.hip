@@ -1,10 +1,12 @@
 // Linear layers: C[M, N] = A[M, K] * W[N, K]^T (+ bias[N]) (+ residual[M, N]).
 // A and W are both contiguous along K (the checkpoint's [out, in] layout), in
 // float32 or bfloat16; accumulation is float32 on the MFMA units (true float32
-// MFMA for float32 inputs, no reduced-precision matrix mode). Three kernels:
+// MFMA for float32 inputs, no reduced-precision matrix mode). The kernels:
 //   gemm_tiled      - many rows (prompt portions): LDS-staged 32x32 MFMA tiles
 //   gemm_skinny_lds - few rows (decode): weights streamed once from HBM straight
 //                     into 16x16 MFMA fragments, split over K when N is small
+//   gemm_stream_cu  - 17 to 64 rows: the same with one workgroup per CU
+//   gemm_narrow     - up to 16 rows, few columns: a workgroup has the whole of K
 //   gemm_generic    - any K (rows not 16-byte aligned): one output per thread
 //
 // Weight layouts. Row-major [N][K] as in the checkpoint, or SHUFFLED (an exact permutation,
@@ -473,6 +475,100 @@ __global__ __launch_bounds__(TW_CU_WAVES * 64) void gemm_stream_cu_kernel(
 }
 
 // =====================================================================================
+// Few rows against a matrix with few columns (M <= 16, shuffled weights): one workgroup owns 16 output
+// columns (GLU: a gate and an up tile of 16) over the WHOLE of K. Its waves take k-steps in turn (wave w:
+// steps w, w + WAVES, ..., so that the workgroup reads consecutive kilobytes), weights and activations
+// straight into MFMA fragments, two batches of U steps in flight; the waves' float32 sums meet in LDS, are
+// added in the waves' order, and the epilogue runs here: no partial sums in memory and no second kernel.
+// Bound by the weights' latency and bytes, and by the activations that every workgroup reads from L2 (with K
+// above 4096 these cost more than they save).
+// =====================================================================================
+template <typename T, typename OutT, int WAVES, bool GLU>
+__global__ __launch_bounds__(WAVES * 64) void gemm_narrow_kernel(const T* __restrict__ A, long lda,
+                                                                 const T* __restrict__ W, long ldw,
+                                                                 const float* __restrict__ bias,
+                                                                 const float* residual, long ldr, OutT* C, long ldc,
+                                                                 int M, int N, int K) {
+  typedef typename Elem<T>::Frag Frag;
+  constexpr int EPF = Elem<T>::kPerFrag, U = 4, NT = GLU ? 2 : 1;
+  __shared__ float sums[NT * WAVES * 16 * 16];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int r = lane & 15, g = lane >> 4;
+  const int chunks = K / EPF, steps = (chunks + 3) / 4;
+  const int mine = steps > wave ? (steps - wave + WAVES - 1) / WAVES : 0;      // this wave's steps
+  const T* w_base = W + ((size_t)blockIdx.x * NT * ldw * 64 + lane) * EPF;
+  const size_t w_tile = (size_t)ldw * 64 * EPF;
+  const T* x_base = A + (size_t)min(r, M - 1) * lda;                            // (rows past M: never stored)
+
+  // Loads carry no predicate: steps are clamped to the last one and chunks to the last chunk, and activations
+  // past either are replaced by zeros before the product.
+  Frag wf[2][NT][U], xf[2][U];
+  auto load = [&](const int buf, int i0) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int s = wave + (i0 + u) * WAVES;
+#pragma unroll
+      for (int t = 0; t < NT; ++t)
+        wf[buf][t][u] = tw_load_frag_stream(w_base + t * w_tile + (size_t)min(s, steps - 1) * 64 * EPF);
+      xf[buf][u] = tw_load_frag(x_base + (size_t)min(s * 4 + g, chunks - 1) * EPF);
+    }
+  };
+  f32x4 acc[NT];
+#pragma unroll
+  for (int t = 0; t < NT; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+  auto multiply = [&](const int buf, int i0) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int s = wave + (i0 + u) * WAVES;
+      const Frag x = s * 4 + g < chunks ? xf[buf][u] : Elem<T>::zero();
+#pragma unroll
+      for (int t = 0; t < NT; ++t) tw_mma16(acc[t], wf[buf][t][u], x);
+    }
+  };
+  load(0, 0);
+  load(1, U);
+  // what the epilogue adds, requested behind the first weights: thread t < 256 finishes row t / 16, column t % 16
+  const int row = tid >> 4, c = tid & 15, col = blockIdx.x * 16 + c;
+  const bool store = row < M && col < N / NT;
+  float add[NT], res = 0.f;
+#pragma unroll
+  for (int t = 0; t < NT; ++t) add[t] = store && bias ? bias[(blockIdx.x * NT + t) * 16 + c] : 0.f;
+  if (!GLU && store && residual) res = residual[(size_t)row * ldr + col];
+  for (int i = 0; i < mine; i += 2 * U) {
+    multiply(0, i);
+    if (i + 2 * U < mine) load(0, i + 2 * U);
+    __builtin_amdgcn_sched_barrier(0);           // the compiler would sink the loads below the waits
+    if (i + U < mine) {
+      multiply(1, i + U);
+      if (i + 3 * U < mine) load(1, i + 3 * U);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+  // acc[t][j] = sum over this wave's steps of W[16 tile + 4g + j][k] * A[r][k]; columns swapped about by row,
+  // so that the 16 rows of a write meet different banks
+#pragma unroll
+  for (int t = 0; t < NT; ++t)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) sums[((t * WAVES + wave) * 16 + r) * 16 + ((4 * g + j) ^ r)] = acc[t][j];
+  __syncthreads();
+  if (!store) return;
+  float v[NT];
+#pragma unroll
+  for (int t = 0; t < NT; ++t) {
+    v[t] = 0.f;
+#pragma unroll
+    for (int w = 0; w < WAVES; ++w) v[t] += sums[((t * WAVES + w) * 16 + row) * 16 + (c ^ row)];
+    v[t] += add[t];
+  }
+  if constexpr (GLU) {
+    C[(size_t)row * ldc + col] = tw_from_float<OutT>(tw_glu(v[0], v[1], ldr));
+  } else {
+    if (residual) v[0] += res;
+    C[(size_t)row * ldc + col] = tw_from_float<OutT>(v[0]);
+  }
+}
+
+// =====================================================================================
 // Generic kernel: any K. One thread per output element, float32 accumulation.
 // =====================================================================================
 template <typename T>
@@ -690,14 +786,51 @@ static int launch_skinny_lds_m(const T* A, long lda, const T* W, long ldw, const
   return launch_skinny_lds<T, OutT, 4, PARTIAL, SHUF, GLU>(A, lda, W, ldw, bias, residual, ldr, C, ldc, partial, partial_bytes, M, N, K, stream);
 }
 
+// Up to 16 rows of a shuffled weight: is the kernel with 16 output columns (GLU: 16 pairs) over the whole of K a
+// workgroup faster than the one with K ranges? Measured with weights from HBM, back to back, at 8 rows (bf16; us,
+// K ranges and their reduction / whole K):
+//    N x K        1536 x 512   2048 x 1024   2048 x 2048   3584 x 3584   896 x 4864   4608 x 3584   8192 x 2048
+//                 4.7 / 3.1    6.1 / 3.5     6.6 / 4.4     9.8 / 7.0     8.5 / 8.4    10.7 / 11.3   10.7 / 7.6
+//    N x 256:     3584 4.0 / 3.2, 4608 4.0 / 4.2;   N x 1536: 24576 15.7 / 15.1, with 16 rows 15.8 / 18.9
+//    GLU (K ranges: always one):   8192 x 512 4.7 / 4.0,   9728 x 896 6.5 / 6.2,   8192 x 2048 9.9 / 7.3,
+//                 37888 x 512 9.2 / 10.6,   22016 x 2048 17.7 / 16.6,   9728 x 3584 16.2 / 16.8
+// Up to 256 workgroups (one a CU): as long as a wave's share of K is about what it keeps in flight (8 k-steps of 16
+// waves), K <= 4096 in bf16. With more, the CUs are uneven and every workgroup reads the activations again: only
+// where the other kernel's waves sit through a chain of stages and the weights outweigh the activations.
+// `sums`: float32 sums for the caller's next kernel, no reduction saved: only where the other kernel has one range too
+// (4096 x 896: 5.6 / 3.4).
+static bool narrow_pays(int N, int K, int epf, bool glu, bool sums) {
+  const int steps = tw_div_up(K / epf, 4), groups = glu ? N / 32 : tw_div_up(N, 16);
+  if (sums) return groups <= 256 && steps >= 16 && steps < 32;
+  if (groups <= 256) return steps <= 128;
+  if (glu) return steps >= 28 && steps <= 64;
+  return groups <= 512 && steps >= 16 && steps <= 64;
+}
+
+// Waves a workgroup: as few as have a wave's whole share of K in flight at once (8 k-steps), up to 16. (2048 x 1024, 8
+// rows: 4 / 8 / 16 waves 3.5 / 4.0 / 5.6 us; 2048 x 2048: 5.2 / 4.4 / 5.9; 2048 x 4096: 8.1 / 6.7 / 6.5)
+template <typename T, typename OutT, bool GLU>
+static int launch_narrow(const T* A, long lda, const T* W, long ldw, const float* bias, const float* residual, long ldr,
+                         OutT* C, long ldc, int M, int N, int K, hipStream_t stream) {
+  const int steps = tw_div_up(K / Elem<T>::kPerFrag, 4), groups = GLU ? N / 32 : tw_div_up(N, 16);
+  if (steps <= 48)
+    gemm_narrow_kernel<T, OutT, 4, GLU><<<groups, 256, 0, stream>>>(A, lda, W, ldw, bias, residual, ldr, C, ldc, M, N, K);
+  else if (steps <= 96)
+    gemm_narrow_kernel<T, OutT, 8, GLU><<<groups, 512, 0, stream>>>(A, lda, W, ldw, bias, residual, ldr, C, ldc, M, N, K);
+  else
+    gemm_narrow_kernel<T, OutT, 16, GLU><<<groups, 1024, 0, stream>>>(A, lda, W, ldw, bias, residual, ldr, C, ldc, M, N, K);
+  return TW_LAUNCH_RESULT();
+}
+
 // force: 0 = choose, 1 = generic, 3 = tiled 128x128, 4 = tiled 128x256, 5 = skinny, 6 = tiled 256x256,
-// 7 = tiled 256x192, 8 = streaming with one workgroup per CU (shuffled weights, up to 64 rows)
+// 7 = tiled 256x192, 8 = streaming with one workgroup per CU (shuffled weights, up to 64 rows),
+// 9 = whole K per workgroup (shuffled weights, up to 16 rows)
 template <typename T, typename OutT, bool SHUF, bool GLU>
 static int linear_dispatch(const T* A, long lda, const T* W, long ldw, const float* bias,
                            const float* residual, long ldr, OutT* C, long ldc, float* partial,
                            long partial_bytes, int M, int N, int K, int force, hipStream_t stream) {
   constexpr int EPF = Elem<T>::kPerFrag;
-  TW_REQUIRE(force == 0 || force == 1 || (force >= 3 && force <= 8));
+  TW_REQUIRE(force == 0 || force == 1 || (force >= 3 && force <= 9));
   // the shuffled layout exists only for K that is a multiple of 16 bytes and is always aligned
   const bool aligned = K % EPF == 0 && lda % EPF == 0 && ((uintptr_t)A % 16 == 0) && ((uintptr_t)W % 16 == 0) &&
                        (SHUF || ldw % EPF == 0);
@@ -713,6 +846,12 @@ static int linear_dispatch(const T* A, long lda, const T* W, long ldw, const flo
     TW_REQUIRE(M <= 64 && SHUF);
     if constexpr (SHUF)
       return launch_stream_cu<T, OutT, false, GLU>(A, lda, W, ldw, bias, residual, ldr, C, ldc, partial, partial_bytes, M, N, K, stream);
+  }
+  if constexpr (SHUF) {
+    if (force == 9 || (force == 0 && M <= 16 && narrow_pays(N, K, EPF, GLU, false))) {
+      TW_REQUIRE(M <= 16);
+      return launch_narrow<T, OutT, GLU>(A, lda, W, ldw, bias, residual, ldr, C, ldc, M, N, K, stream);
+    }
   }
   if (force == 5 || (force == 0 && M <= 64)) {
     TW_REQUIRE(M <= 64);
@@ -829,6 +968,10 @@ static int partials_layout(int shuffled, const T* A, long lda, const T* W, long 
                            long partial_bytes, int M, int N, int K, hipStream_t stream) {
   if (shuffled && M > TW_CU_ABOVE_ROWS)
     return launch_stream_cu<T, float, true, false>(A, lda, W, ldw, nullptr, nullptr, 0, (float*)nullptr, N, partial, partial_bytes, M, N, K, stream);
+  if (shuffled && M <= 16 && narrow_pays(N, K, Elem<T>::kPerFrag, false, true)) {
+    TW_REQUIRE(partial != nullptr && partial_bytes >= (long)M * N * 4);
+    return launch_narrow<T, float, false>(A, lda, W, ldw, nullptr, nullptr, 0, partial, N, M, N, K, stream);
+  }
   if (shuffled)
     return launch_skinny_lds_m<T, float, true, true, false>(A, lda, W, ldw, nullptr, nullptr, 0, (float*)nullptr, N, partial, partial_bytes, M, N, K, stream);
   return launch_skinny_lds_m<T, float, true, false, false>(A, lda, W, ldw, nullptr, nullptr, 0, (float*)nullptr, N, partial, partial_bytes, M, N, K, stream);

@@ -353,6 +353,53 @@ def test_linear_epilogues_at_tile_edges(ops, device, dtype, m, n):
         torch.testing.assert_close(out.double().cpu(), act(want + bias.double().cpu()), **tol(dtype, (1e-5, 1e-5), (1e-2, 1e-2)))
 
 
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("m,n,k", [(1, 16, 8), (16, 15, 40), (3, 33, 1536), (8, 389, 1576), (16, 256, 3104), (5, 96, 4096), (16, 64, 8200)])
+def test_linear_of_few_rows_over_whole_k(ops, device, dtype, m, n, k):
+    """A workgroup with the whole of K: one k-step and fewer steps than waves, a last step that K ends inside, every number
+    of waves and the most and more than they keep in flight, columns that end inside a tile, rows of another stride; with
+    and without bias, the residual apart and in place, float32 sums for the next kernel, gated pairs. A float32 sum of K
+    products of sizes below 5 x 0.25, added as chains of at most K / 4, is off by at most K / 4 x 2^-24 of their sum of sizes."""
+    wide = rand((m, k + 16), dtype, device, 1.0, seed=1)
+    x = wide[:, :k]
+    w = rand((n, k), dtype, device, 0.05, seed=2)
+    bias = rand((n,), torch.float32, device, 0.5, seed=3)
+    res = rand((m, n + 5), torch.float32, device, 1.0, seed=4)[:, :n]
+    want = (x.double() @ w.double().T).cpu()
+    size = (x.double().abs() @ w.double().abs().T).max().item()
+    near = dict(atol=(k / 4 + 4) * 2.0 ** -24 * size + 1e-6, rtol=1e-6)
+    shuffled = ops.shuffle_weight(w)
+    for rows in (x, x.contiguous()):
+        for b in (None, bias):
+            plain = want + (0 if b is None else b.double().cpu())
+            for residual in (None, res):
+                out = torch.full((m, n + 3), float("nan"), device=device)
+                ops.linear(rows, shuffled, out[:, :n], bias=b, residual=residual, force=ops.GEMM_NARROW)
+                torch.testing.assert_close(out[:, :n].double().cpu(), plain + (0 if residual is None else residual.double().cpu()), **near)
+                assert out[:, n:].isnan().all()
+            acc = res.clone()
+            ops.linear(rows, shuffled, acc, bias=b, residual=acc, force=ops.GEMM_NARROW)
+            torch.testing.assert_close(acc.double().cpu(), plain + res.double().cpu(), **near)
+        low = torch.full((m, n), float("nan"), dtype=dtype, device=device)
+        ops.linear(rows, shuffled, low, force=ops.GEMM_NARROW)
+        torch.testing.assert_close(low.double().cpu(), want, **near if dtype == torch.float32 else dict(atol=near["atol"], rtol=2.0 ** -8))
+        splits = ops.linear_partial_splits_rows(shuffled, m, rows.stride(0))
+        part = torch.full((splits, m, n), float("nan"), device=device)
+        ops.linear_partials(rows, shuffled, part)
+        torch.testing.assert_close(part.double().sum(0).cpu(), want, **near)
+    pairs = n // 16 * 16
+    if pairs:
+        gate, up = w[:pairs], rand((pairs, k), dtype, device, 0.05, seed=5)
+        both = ops.shuffle_weight(ops.interleave_glu_rows(gate, up))
+        biases = ops.interleave_glu_rows(bias[:pairs], 0.5 * bias[:pairs])
+        g = (x.double() @ gate.double().T + bias[:pairs].double()).cpu()
+        u = (x.double() @ up.double().T + 0.5 * bias[:pairs].double()).cpu()
+        out = torch.full((m, pairs), float("nan"), dtype=dtype, device=device)
+        ops.linear_glu(x, both, out, bias=biases, force=ops.GEMM_NARROW)
+        bound = near["atol"] * (1.1 * u.abs().max().item() + g.abs().max().item() + 1) + 1e-6
+        torch.testing.assert_close(out.double().cpu(), g * torch.sigmoid(g) * u, atol=bound, rtol=1e-5 if dtype == torch.float32 else 2.0 ** -7)
+
+
 @pytest.mark.parametrize("m,n,k", [(1024, 3584, 16384), (1100, 3000, 12288), (2048, 3584, 8192)])
 def test_linear_large_tiles_over_k_ranges(ops, device, m, n, k):
     """Many rows, few columns, long K (a down projection): the chosen plan may be 256x256 tiles whose K is
