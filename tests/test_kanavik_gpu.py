@@ -112,6 +112,26 @@ def test_mixed_head_attention(device, dtype, H, G, D, E, window, T, q_len, page)
 
 
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("H,G,D,E,window,T,q_len,page", [
+    (7, 7, 128, 128, 33, 61, 61, 8),       # queries in registers (bfloat16), one head a wave, tiles that rows end inside
+    (16, 4, 128, 128, 60, 300, 35, 16),    # two heads of shared keys a wave, key ranges
+    (13, 13, 128, 128, 40, 90, 90, 16),    # two heads of different keys, the last wave with one
+    (16, 4, 64, 128, 100, 200, 1, 16),     # the same in registers in float32; decode
+    (14, 2, 192, 128, 50, 70, 70, 16),     # more k-steps than are requested at a time, a last one that the size ends inside
+    (18, 9, 128, 128, 24, 77, 40, 16),     # nine waves and twelve: three a SIMD
+    (24, 6, 144, 64, 50, 260, 20, 16),
+    (23, 23, 64, 144, 30, 64, 64, 16),
+    (16, 8, 128, 256, 0, 50, 50, 16),      # a k-step at a time
+    (26, 2, 128, 128, 90, 150, 1, 16),
+])
+def test_mixed_head_attention_forms(device, dtype, H, G, D, E, window, T, q_len, page):
+    """The same against the same oracle for every way a wave can hold its queries, keys and heads. (Windows of at most 100: a
+    float32 score holds slope x distance, off by 2^-24 of it for each of H mixed heads, and 300 keys away with a slope of
+    0.8 that alone is the tolerance.)"""
+    test_mixed_head_attention(device, dtype, H, G, D, E, window, T, q_len, page)
+
+
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 @pytest.mark.parametrize("taps,norm,C", [(3, True, 40), (4, False, 40), (1, True, 38), (2, False, 38), (8, True, 38)])
 def test_causal_conv_over_portions_and_reused_slots(device, dtype, taps, norm, C):
     """Sequences in portions of 1 to 9 tokens, two at a time, in state slots that were used before."""
