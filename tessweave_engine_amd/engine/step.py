@@ -100,8 +100,15 @@ class Stepper:
 
     # ---- metadata buffers ------------------------------------------------------------
     def _reserve(self, max_tokens, max_seqs):
-        """(Re)allocate the metadata buffers for steps of up to MAX_TOKENS rows and MAX_SEQS requests."""
+        """(Re)allocate the metadata buffers for steps of up to MAX_TOKENS rows and MAX_SEQS requests.
+
+        Steps already issued are waited for first: the kernel that fetches a step's metadata reads the pinned buffer when
+        it runs, the allocator does not know of it, and would hand the same memory to the new buffers at once."""
         self._drop_graphs()
+        self.synchronize()
+        for event in self._staging_events:
+            if event is not None:
+                event.synchronize()
         self.max_tokens, self.max_seqs = max_tokens, max_seqs
         width = self.cache.table_width
         n_groups = len(self.cache.pools)

@@ -103,6 +103,33 @@ def test_steps_called_from_changing_streams(tiny):
     assert torch.equal(run(lambda i: 0), run(lambda i: i % 3))
 
 
+def test_step_buffers_grow_behind_a_busy_device(tiny):
+    """Every request is longer than any before, so every step grows the stepper's buffers while the step before still waits
+    for the device: its metadata must reach it all the same."""
+    from tessweave_engine_amd.cache import CacheManager
+    from tessweave_engine_amd.engine import StepEntry, Stepper
+    from tessweave_engine_amd.weights import load_model
+    model = load_model(tiny["folder"], dtype="float32", device="cuda:0")
+    prompts = prompts_for(tiny, [20, 300, 301, 700, 701], seed=9)
+    busy = torch.randn(4096, 4096, device="cuda")
+
+    def run(wait):
+        cache = CacheManager(model.cache_layout(), tiny["page"], 2200 // tiny["page"] + 20, 5, dtype="float32", device=model.device,
+                             prefix_cache=False, max_request_tokens=768)
+        stepper, rows = Stepper(model, cache, max_step_tokens=16), []
+        for i, tokens in enumerate(prompts):
+            for _ in range(20):
+                busy @ busy
+            rows.append(stepper.step([StepEntry(cache.open(i), tokens, [len(tokens) - 1])]).clone())
+            if wait:
+                torch.cuda.synchronize()
+        torch.cuda.synchronize()
+        stepper.close()
+        return torch.cat(rows)
+
+    assert torch.equal(run(True), run(False))
+
+
 def test_long_decoding_and_the_first_tokens(tiny):
     """One token after the other for hundreds of steps (pages fill and new ones are taken), from position 0."""
     from tessweave_engine_amd.cache import CacheManager
