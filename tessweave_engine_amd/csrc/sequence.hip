@@ -96,8 +96,12 @@ __device__ __forceinline__ void conv_store4(bf16_t* p, f32x4 v) {
 }
 
 // VEC: four consecutive channels a thread, 16-byte (8-byte for bfloat16) accesses; the launcher asks for it when
-// the channel count, the row strides and the pointers allow.
-template <typename SrcT, typename OutT, bool NORM, bool VEC>
+// the channel count, the row strides and the pointers allow; a row's squares are then summed four such loads at a time
+// (one channel a load, each waited for: 8 rows of 2,048 with 3 taps behind a norm 6.9 us, now 5.2).
+// FOUR: four taps, a channel's being one 16-byte read: what a thread's channels need (rows, state, weights, taps) is
+// requested before the rows' squares are summed (the same rows: 7.8 -> 4.0 us, without a norm 4.5 -> 3.2; other numbers of taps read one
+// by one with the rows were no faster, and at 300 rows slower, than where they are used).
+template <typename SrcT, typename OutT, bool NORM, bool VEC, bool FOUR = false>
 __global__ __launch_bounds__(256) void causal_conv_kernel(ConvArgs a) {
   __shared__ float red[TW_CONV_MAX_TAPS][4];
   __shared__ float rinv[TW_CONV_MAX_TAPS];
@@ -107,7 +111,7 @@ __global__ __launch_bounds__(256) void causal_conv_kernel(ConvArgs a) {
   const int len = a.kv_len[s];
   const int start = len - q_len;                 // position of the step's first token of this sequence
   const int pos = start + (row - first);
-  const int K = a.K, C = a.C;
+  const int K = FOUR ? 4 : a.K, C = a.C;
   const int slot = a.state_slots[s], ph = a.phase[s] & 1;
   const float* old_state = a.state + ((size_t)slot * 2 + ph) * (size_t)(K - 1) * C;
   float* new_state = a.state + ((size_t)slot * 2 + (1 - ph)) * (size_t)(K - 1) * C;
@@ -122,6 +126,22 @@ __global__ __launch_bounds__(256) void causal_conv_kernel(ConvArgs a) {
     from_src[j] = (j < K && p >= start) ? src + (size_t)(first + p - start) * a.ld_src : nullptr;
     from_state[j] = (j < K && p < start && p >= 0) ? old_state + (size_t)(p - start + K - 1) * C : nullptr;
   }
+  const int share = ((C + gridDim.y - 1) / gridDim.y + 3) / 4 * 4;
+  const int c_end = min(C, (int)(blockIdx.y + 1) * share);
+  const int c_first = blockIdx.y * share + threadIdx.x * 4;
+  f32x4 v4[4], tap4[4], acc4, nw4;
+  auto request = [&](int c) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      v4[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+      if (from_src[j]) v4[j] = conv_load4(from_src[j] + c);
+      else if (from_state[j]) v4[j] = conv_load4(from_state[j] + c);
+      tap4[j] = conv_load4(a.taps + (size_t)(c + j) * 4);
+    }
+    acc4 = a.bias ? conv_load4(a.bias + c) : f32x4{0.f, 0.f, 0.f, 0.f};
+    nw4 = NORM ? conv_load4(a.norm_w + c) : f32x4{1.f, 1.f, 1.f, 1.f};
+  };
+  if (FOUR && c_first < c_end) request(c_first);
   if (NORM && a.row_rinv) {
     if (threadIdx.x < TW_CONV_MAX_TAPS) {
       const int j = threadIdx.x, p = pos - (K - 1) + j;
@@ -130,24 +150,33 @@ __global__ __launch_bounds__(256) void causal_conv_kernel(ConvArgs a) {
     __syncthreads();
   } else if (NORM) {
     // every block sums whole rows, whatever share of the channels it then writes
-    float sums[TW_CONV_MAX_TAPS];
-#pragma unroll
-    for (int j = 0; j < TW_CONV_MAX_TAPS; ++j) sums[j] = 0.f;
-    for (int c = threadIdx.x; c < C; c += blockDim.x) {
-#pragma unroll
-      for (int j = 0; j < TW_CONV_MAX_TAPS; ++j)
-        if (from_src[j]) {
-          const float v = tw_to_float(from_src[j][c]);
-          sums[j] += v * v;
-        }
-    }
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+#pragma unroll 1
+    for (int j = 0; j < K; ++j) {
+      const int p = pos - (K - 1) + j;
+      float sum = 0.f;
+      if (p >= start) {
+        const SrcT* from = src + (size_t)(first + p - start) * a.ld_src;
+        if constexpr (VEC) {
+          for (int c0 = threadIdx.x * 4; c0 < C; c0 += blockDim.x * 16) {
+            f32x4 v[4];
 #pragma unroll
-    for (int j = 0; j < TW_CONV_MAX_TAPS; ++j) {
-      if (j < K) {
-        const float t = tw_wave_sum(sums[j]);
-        if (lane == 0) red[j][wave] = t;
+            for (int u = 0; u < 4; ++u) v[u] = conv_load4(from + min(c0 + u * (int)blockDim.x * 4, C - 4));
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+              const float t = v[u][0] * v[u][0] + v[u][1] * v[u][1] + v[u][2] * v[u][2] + v[u][3] * v[u][3];
+              sum += c0 + u * (int)blockDim.x * 4 < C ? t : 0.f;
+            }
+          }
+        } else {
+          for (int c = threadIdx.x; c < C; c += blockDim.x) {
+            const float v = tw_to_float(from[c]);
+            sum += v * v;
+          }
+        }
+        sum = tw_wave_sum(sum);
       }
+      if (lane == 0) red[j][wave] = sum;
     }
     __syncthreads();
     if (threadIdx.x < K) {
@@ -156,27 +185,40 @@ __global__ __launch_bounds__(256) void causal_conv_kernel(ConvArgs a) {
     }
     __syncthreads();
   }
-  const int share = ((C + gridDim.y - 1) / gridDim.y + 3) / 4 * 4;
-  const int c_end = min(C, (int)(blockIdx.y + 1) * share);
   if constexpr (VEC) {
-    for (int c = blockIdx.y * share + threadIdx.x * 4; c < c_end; c += blockDim.x * 4) {
-      f32x4 v[TW_CONV_MAX_TAPS];
+    for (int c = c_first; c < c_end; c += blockDim.x * 4) {
+      f32x4 acc;
+      if constexpr (FOUR) {
+        if (c != c_first) request(c);
+        acc = acc4;
 #pragma unroll
-      for (int j = 0; j < TW_CONV_MAX_TAPS; ++j) {
-        v[j] = f32x4{0.f, 0.f, 0.f, 0.f};
-        if (from_src[j]) v[j] = conv_load4(from_src[j] + c);
-        else if (from_state[j]) v[j] = conv_load4(from_state[j] + c);
-      }
-      f32x4 acc = a.bias ? conv_load4(a.bias + c) : f32x4{0.f, 0.f, 0.f, 0.f};
-      const f32x4 nw = NORM ? conv_load4(a.norm_w + c) : f32x4{1.f, 1.f, 1.f, 1.f};
+        for (int j = 0; j < 4; ++j) {
+          f32x4 v = v4[j];
+          if (NORM && from_src[j]) v = v * rinv[j] * nw4;
 #pragma unroll
-      for (int j = 0; j < TW_CONV_MAX_TAPS; ++j) {
-        if (j < K) {
-          if (NORM && from_src[j]) v[j] = v[j] * rinv[j] * nw;
+          for (int e = 0; e < 4; ++e) acc[e] += tap4[e][j] * v[e];
+          if (j == 3) acc += a.identity * v;
+          if (last && j >= 1) conv_store4(new_state + (size_t)(j - 1) * C + c, v);
+        }
+      } else {
+        f32x4 v[TW_CONV_MAX_TAPS];
 #pragma unroll
-          for (int e = 0; e < 4; ++e) acc[e] += a.taps[(size_t)(c + e) * K + j] * v[j][e];
-          if (j == K - 1) acc += a.identity * v[j];
-          if (last && j >= 1) conv_store4(new_state + (size_t)(j - 1) * C + c, v[j]);
+        for (int j = 0; j < TW_CONV_MAX_TAPS; ++j) {
+          v[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+          if (from_src[j]) v[j] = conv_load4(from_src[j] + c);
+          else if (from_state[j]) v[j] = conv_load4(from_state[j] + c);
+        }
+        acc = a.bias ? conv_load4(a.bias + c) : f32x4{0.f, 0.f, 0.f, 0.f};
+        const f32x4 nw = NORM ? conv_load4(a.norm_w + c) : f32x4{1.f, 1.f, 1.f, 1.f};
+#pragma unroll
+        for (int j = 0; j < TW_CONV_MAX_TAPS; ++j) {
+          if (j < K) {
+            if (NORM && from_src[j]) v[j] = v[j] * rinv[j] * nw;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) acc[e] += a.taps[(size_t)(c + e) * K + j] * v[j][e];
+            if (j == K - 1) acc += a.identity * v[j];
+            if (last && j >= 1) conv_store4(new_state + (size_t)(j - 1) * C + c, v[j]);
+          }
         }
       }
       acc = conv_act(acc, a.act);
@@ -369,6 +411,7 @@ extern "C" int tw_causal_conv(int dtype, int src_f32, const void* src, long ld_s
     const dim3 tiles(tw_div_up(n_tokens, TW_CONV_TILE), tw_div_up(C, 1024));                       \
     if (tiled && four) causal_conv_tile_kernel<S, O, N, 4><<<tiles, 256, 0, stream>>>(a, n_tokens); \
     else if (tiled) causal_conv_tile_kernel<S, O, N, 0><<<tiles, 256, 0, stream>>>(a, n_tokens);   \
+    else if (vec && four) causal_conv_kernel<S, O, N, true, true><<<n_blocks, 256, 0, stream>>>(a); \
     else if (vec) causal_conv_kernel<S, O, N, true><<<n_blocks, 256, 0, stream>>>(a);              \
     else causal_conv_kernel<S, O, N, false><<<n_blocks, 256, 0, stream>>>(a);                      \
   } while (0)

@@ -187,6 +187,15 @@ def test_causal_conv_over_portions_and_reused_slots(device, dtype, taps, norm, C
 
 
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("norm,C", [(True, 4), (True, 40), (True, 1028), (True, 4100), (False, 4), (False, 1028)])
+def test_causal_conv_of_four_taps(device, dtype, norm, C):
+    """Four taps, requested with the rows: fewer channels than threads, a last share that the channels end inside, more
+    channels than one round of 16-byte loads sums; with and without the norm."""
+    test_causal_conv_over_portions_and_reused_slots(device, dtype, 4, norm, C)
+
+
+
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 @pytest.mark.parametrize("taps,norm,C", [(4, True, 48), (3, False, 48), (1, True, 48), (8, False, 48), (2, True, 48), (4, False, 2308),
                                          (5, True, 1028)])
 def test_causal_conv_of_many_rows(device, dtype, taps, norm, C):
