@@ -180,7 +180,11 @@ __device__ __forceinline__ void delta_lds_barrier() {
 //   U = U0 - W S0,    O = M U0 + (G Q - M W) S0,    S = G_last S0 + K'^T U.
 // delta_prepare forms W, Q' = G Q - M W, K', U0 and O0 = M U0 for every (chunk, head) at once; delta_chunk then goes through a
 // sequence's chunks with three products each. Everything is float32, the products on the matrix unit (16x16x4). T comes from
-// substitution, a column a lane, in blocks of 16 tokens (a series in powers of A would lose digits where keys are alike).
+// substitution, a column a lane, in blocks of 16 tokens (a series in powers of A would lose digits where keys are alike). For
+// the same reason the products of keys are sums of eight elements added in 64 bits, and a chunk's change of the state is summed
+// before it meets the state. Errors against 64 bits (400 tokens, heads of 128), outputs and state: 1.9e-7 and 1.5e-7, with keys
+// that share half of their length 3.0e-7 and 2.8e-7 (with one float32 chain each 2.6e-7 and 2.2e-7, 7.4e-7 and 6.9e-7; chunks
+// of 16 solved in the chain of tokens 2.3e-7 and 2.2e-7, 3.6e-7 and 3.4e-7). The time is the same.
 //
 // What bounds them: delta_chunk the chain from chunk to chunk and the 48 KB of operands a chunk that each of its workgroups
 // reads (2 us a chunk, 30 GB/s a CU), delta_prepare its own length: written out over the 32 tokens with a thread a column it
@@ -284,25 +288,45 @@ __global__ __launch_bounds__(256) void delta_prepare_kernel(DeltaArgs a, DeltaPr
   // ---- K K^T and Q K^T, the three tiles on and below the diagonal by a wave each; the fourth wave: squared lengths ------
   if (wave < 3) {
     const int ti = wave ? 1 : 0, tj = wave == 2 ? 1 : 0;
-    f32x4 kk = {0.f, 0.f, 0.f, 0.f}, qk = kk;
+    // (sums of eight elements, added in 64 bits: where keys are alike, rounding here doubled the error of the results)
+    double kk[4] = {0., 0., 0., 0.}, qk[4] = {0., 0., 0., 0.};
 #pragma unroll
     for (int x = 0; x < 4 * NT; ++x) {
       const f32x4 kj = *reinterpret_cast<const f32x4*>(&k_s[16 * tj + r][16 * x + 4 * g]);
-      tw_mma16(kk, *reinterpret_cast<const f32x4*>(&k_s[16 * ti + r][16 * x + 4 * g]), kj);
-      tw_mma16(qk, *reinterpret_cast<const f32x4*>(&q_s[16 * ti + r][16 * x + 4 * g]), kj);
+      const f32x4 ki = *reinterpret_cast<const f32x4*>(&k_s[16 * ti + r][16 * x + 4 * g]);
+      const f32x4 qi = *reinterpret_cast<const f32x4*>(&q_s[16 * ti + r][16 * x + 4 * g]);
+#pragma unroll
+      for (int h = 0; h < 4; h += 2) {
+        f32x4 kp = {0.f, 0.f, 0.f, 0.f}, qp = kp;
+#pragma unroll
+        for (int e = h; e < h + 2; ++e) {
+          kp = __builtin_amdgcn_mfma_f32_16x16x4f32(ki[e], kj[e], kp, 0, 0, 0);
+          qp = __builtin_amdgcn_mfma_f32_16x16x4f32(qi[e], kj[e], qp, 0, 0, 0);
+        }
+#pragma unroll
+        for (int j = 0; j < 4; ++j) { kk[j] += kp[j]; qk[j] += qp[j]; }
+      }
     }
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-      at_s[16 * tj + r][16 * ti + 4 * g + j] = kk[j];
-      m_s[16 * ti + 4 * g + j][16 * tj + r] = qk[j];
+      at_s[16 * tj + r][16 * ti + 4 * g + j] = (float)kk[j];
+      m_s[16 * ti + 4 * g + j][16 * tj + r] = (float)qk[j];
     }
   } else {
     const int t = lane >> 1;
     float qq = 0.f, kk = 0.f;
-    for (int d = (lane & 1) * 4; d < DP; d += 8) {
-      const f32x4 qv = *reinterpret_cast<const f32x4*>(&q_s[t][d]), kv = *reinterpret_cast<const f32x4*>(&k_s[t][d]);
+#pragma unroll 1
+    for (int y = 0; y < NT; ++y) {                   // (sums of eight squares, added in pairs)
+      f32x4 qp = {0.f, 0.f, 0.f, 0.f}, kp = qp;
 #pragma unroll
-      for (int j = 0; j < 4; ++j) { qq = __fmaf_rn(qv[j], qv[j], qq); kk = __fmaf_rn(kv[j], kv[j], kk); }
+      for (int i = 0; i < 8; ++i) {
+        const int d = 64 * y + 8 * i + (lane & 1) * 4;
+        const f32x4 qv = *reinterpret_cast<const f32x4*>(&q_s[t][d]), kv = *reinterpret_cast<const f32x4*>(&k_s[t][d]);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) { qp[j] = __fmaf_rn(qv[j], qv[j], qp[j]); kp[j] = __fmaf_rn(kv[j], kv[j], kp[j]); }
+      }
+      qq += (qp[0] + qp[1]) + (qp[2] + qp[3]);
+      kk += (kp[0] + kp[1]) + (kp[2] + kp[3]);
     }
     qq += __shfl_xor(qq, 1, TW_WAVE);
     kk += __shfl_xor(kk, 1, TW_WAVE);
@@ -327,9 +351,11 @@ __global__ __launch_bounds__(256) void delta_prepare_kernel(DeltaArgs a, DeltaPr
     for (int p = 0; p < 4; ++p) {
       const int i = i0 + 8 * p;
       const float decay = expf(between[p]);
-      at_s[j][i] = j < i ? beta_s[i] * decay * (kn_s[i] * kn_s[j]) * at_s[j][i] : 0.f;
-      m_s[i][j] = j <= i ? decay * (qn_s[i] * kn_s[j]) * m_s[i][j] : 0.f;
-      if (i == C - 1) tail_s[j] = decay * kn_s[j];
+      // (one rounding each)
+      const double unit = (double)decay * kn_s[j];
+      at_s[j][i] = j < i ? (float)(beta_s[i] * unit * kn_s[i] * at_s[j][i]) : 0.f;
+      m_s[i][j] = j <= i ? (float)(unit * qn_s[i] * m_s[i][j]) : 0.f;
+      if (i == C - 1) tail_s[j] = (float)unit;
       if (j == 0) g_s[i] = expf(between[p] + lg_s[0]);
     }
   }
@@ -534,10 +560,12 @@ __global__ __launch_bounds__(256) void delta_chunk_kernel(DeltaArgs a, DeltaPrep
       x.u[tt] -= (part_s[copy][0][tt][lane] + part_s[copy][1][tt][lane]) + (part_s[copy][2][tt][lane] + part_s[copy][3][tt][lane]);
 #pragma unroll
     for (int mm = 0; mm < NT; ++mm) {
+      // (the chunk's change is summed by itself: summed onto the state, every one of its products rounds at the state's size)
+      f32x4 change = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int j = 0; j < 4; ++j) S[mm][j] *= x.G;
+      for (int tt = 0; tt < 2; ++tt) tw_mma16(change, x.k[mm][tt], x.u[tt]);
 #pragma unroll
-      for (int tt = 0; tt < 2; ++tt) tw_mma16(S[mm], x.k[mm][tt], x.u[tt]);
+      for (int j = 0; j < 4; ++j) S[mm][j] = __fmaf_rn(x.G, S[mm][j], change[j]);
     }
     if (wave < 2) {
       const f32x4 o = x.o + ((part_s[copy][0][2 + wave][lane] + part_s[copy][1][2 + wave][lane]) +
