@@ -1104,8 +1104,21 @@ def delta_workspace_floats(rows, n_seqs, max_q_len, heads, value_dim, dim):
                                                    delta_key_extent(dim)))
 
 
+DELTA_WALK_TOKENS = 4          # launches whose sequences bring up to this many tokens walk them one by one
+
+
+def delta_walks_apart(one_token_seqs, max_q_len, heads, value_dim):
+    """Beside portions of up to max_q_len tokens: is a launch of its own, which walks their tokens, faster for a step's one-token
+    sequences than the portions' launch, which takes each for a chunk of 16 or 32 tokens?
+
+    From eight workgroups (of 16 value columns) a CU on; below, a small step's launch from the host costs what it saves. 16 heads
+    of 128, us: 64 sequences beside a portion of 512 154 -> 84, beside one of 100 123 -> 55, 24 beside 512 94 -> 70 (8 beside
+    256 52 -> 44, but 7 beside 49 33 -> 37); 32 heads: 24 beside 512 144 -> 90; 16 heads of 256: 64 beside 100 467 -> 177."""
+    return max_q_len > DELTA_WALK_TOKENS and one_token_seqs * heads * ((value_dim + 15) // 16) >= 2048
+
+
 def delta_rule(qkv, q_col, k_col, v_col, ab, b_col, a_col, A_log, dt_bias, state, q_start, state_slots, seq0, n_seqs, out,
-               kv_heads, dim, q_scale, max_q_len=1, workspace=None):
+               kv_heads, dim, q_scale, max_q_len=1, workspace=None, rows=None):
     """The gated delta rule over sequences seq0 .. seq0 + n_seqs - 1, from and to state float32
     [requests, H, E, Dk] (a column of S is contiguous; Dk = delta_key_extent(dim)):
 
@@ -1117,7 +1130,7 @@ def delta_rule(qkv, q_col, k_col, v_col, ab, b_col, a_col, A_log, dt_bias, state
     out float32 [n, H * E]. max_q_len: the most tokens a sequence brings (an upper bound will do). Up to a few tokens
     a sequence the tokens are walked one by one; beyond, chunks of 16 or 32 tokens are solved at once (the same sums in another
     order: a triangular system a chunk in place of a chain of updates), with a float32 workspace of delta_workspace_floats
-    (allocated here if none is given)."""
+    (allocated here if none is given). rows: the most rows these sequences bring together (default: all of qkv's)."""
     n, wq, ld_qkv = _rows(qkv, "qkv")
     na, wa, ld_ab = _rows(ab, "ab")
     _need(qkv.dtype == torch.float32 and ab.dtype == torch.float32 and na == n, "the delta rule reads float32 rows")
@@ -1132,7 +1145,9 @@ def delta_rule(qkv, q_col, k_col, v_col, ab, b_col, a_col, A_log, dt_bias, state
     _need(A_log.numel() == H and dt_bias.numel() == H and A_log.dtype == torch.float32 and dt_bias.dtype == torch.float32,
           "one float32 A_log and dt_bias per head")
     _need(seq0 >= 0 and q_start.numel() >= seq0 + n_seqs + 1 and state_slots.numel() >= seq0 + n_seqs, "sequence metadata is too short")
-    floats = delta_workspace_floats(n, n_seqs, max(1, int(max_q_len)), H, E, D)
+    rows = n if rows is None else int(rows)
+    _need(0 <= rows <= n, "delta_rule: rows must be at most qkv's")
+    floats = delta_workspace_floats(rows, n_seqs, max(1, int(max_q_len)), H, E, D)
     if floats and workspace is None:
         workspace = torch.empty(floats, dtype=torch.float32, device=qkv.device)
     _need(not floats or (workspace.dtype == torch.float32 and workspace.is_contiguous() and workspace.numel() >= floats),
@@ -1140,7 +1155,7 @@ def delta_rule(qkv, q_col, k_col, v_col, ab, b_col, a_col, A_log, dt_bias, state
     check(library().tw_delta_rule(_dev(qkv), ld_qkv, int(q_col), int(k_col), int(v_col), _dev(ab), ld_ab, int(b_col), int(a_col),
                                   _dev(A_log), _dev(dt_bias), _dev(state), _dev(q_start, torch.int32, "q_start"),
                                   _dev(state_slots, torch.int32, "state_slots"), _dev(out), ldo, int(seq0), int(n_seqs),
-                                  max(1, int(max_q_len)), H, G, D, E, Dk, float(q_scale), n, _dev(workspace) if floats else None,
+                                  max(1, int(max_q_len)), H, G, D, E, Dk, float(q_scale), rows, _dev(workspace) if floats else None,
                                   workspace.numel() if floats else 0, _stream()), "delta_rule")
     return out
 

@@ -99,10 +99,16 @@ class GatedDeltaRule(Mixer):
         self.conv.forward(ctx, run, proj[:, :channels], out32=qkv, activation="silu")
         result = ctx.scratch("delta.o", (n, H * E), torch.float32)
         state = ctx.cache.states[run.cache_slot][self.STATE]
-        floats = ops.delta_workspace_floats(n, ctx.n_seqs, max(1, ctx.max_q_len), H, E, D)
+        common = (qkv, col["q"], col["k"], col["v"], proj, col["b"], col["a"], self.A_log, self.dt_bias, state, ctx.q_start,
+                  ctx.state_slots)
+        # (one-token sequences own the first rows of a step)
+        apart = ctx.n_decode if ctx.n_decode < ctx.n_seqs and ops.delta_walks_apart(ctx.n_decode, ctx.max_q_len, H, E) else 0
+        if apart:
+            ops.delta_rule(*common, 0, apart, result, G, D, D ** -0.5)
+        rows, sequences = n - apart, ctx.n_seqs - apart
+        floats = ops.delta_workspace_floats(rows, sequences, max(1, ctx.max_q_len), H, E, D)
         ws = ctx.workspace.get("delta.chunks", (floats,), torch.float32) if floats else None
-        ops.delta_rule(qkv, col["q"], col["k"], col["v"], proj, col["b"], col["a"], self.A_log, self.dt_bias, state,
-                       ctx.q_start, ctx.state_slots, 0, ctx.n_seqs, result, G, D, D ** -0.5, max_q_len=ctx.max_q_len, workspace=ws)
+        ops.delta_rule(*common, apart, sequences, result, G, D, D ** -0.5, max_q_len=ctx.max_q_len, workspace=ws, rows=rows)
         act = ctx.scratch("delta.act", (n, H * E))
         ops.head_norm_gate(result, proj[:, col["g"]:col["g"] + H * E], self.norm_weight, act, H, E, self.eps)
         self.o.forward(ctx, act, x, residual=x if accumulate else None)

@@ -71,6 +71,33 @@ def test_cache_layout_and_schedule():
     assert [r.block for r in one.schedule] == [0, 0, 0]
 
 
+@pytest.mark.parametrize("n_decode,portions,launches", [
+    (64, [512], [(0, 64, 1), (64, 1, 512)]), (16, [20, 60], [(0, 16, 1), (16, 2, 60)]), (15, [512], [(0, 16, 512)]),
+    (64, [], [(0, 64, 0)]), (0, [300], [(0, 1, 300)]), (64, [3], [(0, 65, 3)])])
+def test_delta_layers_walk_a_steps_one_token_sequences_apart(monkeypatch, n_decode, portions, launches):
+    """Beside prompt portions a step's one-token sequences get a launch of their own, which walks them, once they are
+    eight workgroups a CU; the portions' launch and its scratch are then sized without them."""
+    from types import SimpleNamespace
+    from tessweave_engine_amd.kernels import ops
+    from tessweave_engine_amd.parts.delta import GatedDeltaRule
+    H, G, D, E = 16, 4, 128, 128
+    mixer = GatedDeltaRule("m.", 64, H, G, D, E, 4, 1e-6)
+    n, calls, sizes = n_decode + sum(portions), [], []
+    for part in (mixer.proj, mixer.conv, mixer.o):
+        part.forward = lambda *a, **k: None
+    monkeypatch.setattr(ops, "head_norm_gate", lambda *a, **k: None)
+    monkeypatch.setattr(ops, "delta_workspace_floats", lambda *a: sizes.append(a) or 0)
+    monkeypatch.setattr(ops, "delta_rule", lambda *a, max_q_len=1, rows=None, **k: calls.append((a[12], a[13], max_q_len, rows)))
+    longest = max(portions, default=0)
+    ctx = SimpleNamespace(n_tokens=n, n_seqs=n_decode + len(portions), n_decode=n_decode, max_q_len=longest, q_start=None,
+                          state_slots=None, scratch=lambda tag, shape, dtype=None: torch.empty(shape, device="meta"),
+                          cache=SimpleNamespace(states={0: {mixer.STATE: None}}))
+    mixer.forward(ctx, SimpleNamespace(cache_slot=0), None, None)
+    assert [c[:3] for c in calls] == launches
+    own = n if len(launches) == 1 else sum(portions)
+    assert calls[-1][3] == own and sizes[-1] == (own, launches[-1][1], max(1, longest), H, E, D)
+
+
 def test_random_weights_and_inspect_on_the_command_line(tmp_path, capsys):
     from tessweave_engine_amd.cli import main
     from tessweave_engine_amd.config import read_model_config
