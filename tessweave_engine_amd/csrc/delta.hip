@@ -21,7 +21,6 @@
 
 #define TW_DELTA_CHUNK 16             /* tokens the walk stages at a time */
 #define TW_DELTA_WALK_MOST 4          /* up to this many tokens a sequence, a step walks them one by one */
-#define TW_DELTA_SHORT_MOST 48        /* up to this many, it solves chunks of 16 tokens in one launch; beyond, of 32 in two */
 
 struct DeltaArgs {
   const float* qkv; long ld_qkv;      // q of key head j at q_col + j * D, k at k_col + j * D, v of head h at v_col + h * E
@@ -593,7 +592,7 @@ __global__ __launch_bounds__(256) void delta_chunk_kernel(DeltaArgs a, DeltaPrep
 }
 
 // ---- portions of a few dozen tokens: chunks of 16 tokens, each solved inside the chain --------------------------------
-// One launch instead of two: up to 48 tokens (three chunks of 4.5 us behind 2.5 us of start) it ends before delta_prepare and
+// One launch instead of two (see delta_in_chunks): a few chunks of 4.5 us behind 2.5 us of start end before delta_prepare and
 // delta_chunk would (13 + 7 us at 33 tokens, 16 heads of 128). A workgroup owns 16 value columns of one (sequence, head) and its
 // waves a quarter of the key elements each, as above. Per chunk: the waves form their parts of K S0, Q S0, K K^T and Q K^T from
 // the same fragments, the parts meet in LDS and thread 16 i + j adds them up for the pair (i, j) and puts decay, beta and the
@@ -799,9 +798,24 @@ __global__ __launch_bounds__(256) void delta_short_kernel(DeltaArgs a, int seq0)
   }
 }
 
+// Chunks of 32 tokens in two launches (or of 16 in one)? Two launches start later but their chain is less than half as long;
+// where workgroups queue, a sequence of a few tokens costs a whole chunk either way, one of 32 more than one of 16.
+// Measured, one launch / two, us:                 one portion of 49    64          80          96          128
+//   16 heads of 128 (128 workgroups of the chain)   22.5 / 21.3   23.0 / 21.1   27.4 / 23.4   31.7 / 24.6   41.4 / 28.1
+//   32 heads of 128 (256)                           21.5 / 24.0   22.1 / 25.0   26.7 / 29.4   31.2 / 28.9   40.1 / 31.8
+//   16 heads of 256 (256)                           25.7 / 30.8   26.4 / 31.4   31.6 / 35.9   37.1 / 37.8   47.9 / 39.7
+//   32 heads of 256 (512)                           34.5 / 44.1   35.9 / 42.8   43.6 / 48.4   50.5 / 49.7   64.6 / 54.3
+// 60 portions of 5 and one of 64: 16 heads of 128 119 / 111, 32 heads 215 / 222, 16 heads of 256 269 / 421; 30 of 17 and one of
+// 64: 108 / 66, 196 / 118, 250 / 208; 30 of 40 and one of 64: 148 / 107, 279 / 203, 363 / 374; 16 of 60: 97 / 69, 188 / 119,
+// 243 / 196.
+static bool delta_in_chunks(int rows, int n_seqs, int max_q_len, int H, int E, int Dk) {
+  const long groups = (long)n_seqs * H * tw_div_up(E, 16);
+  return max_q_len > (groups > 128 && groups <= 512 ? 88 : 48) && rows >= (Dk <= 128 ? 8L : 48L) * n_seqs;
+}
+
 // float32 scratch of a launch over n_seqs sequences of up to `rows` rows together (0: it needs none)
 extern "C" long tw_delta_workspace_floats(int rows, int n_seqs, int max_q_len, int H, int E, int Dk) {
-  if (n_seqs <= 0 || rows <= 0 || max_q_len <= TW_DELTA_SHORT_MOST) return 0;
+  if (n_seqs <= 0 || rows <= 0 || !delta_in_chunks(rows, n_seqs, max_q_len, H, E, Dk)) return 0;
   const long units = ((long)rows / TW_DELTA_PREP + n_seqs) * H;
   const long DP = Dk <= 64 ? 64 : Dk <= 128 ? 128 : 256;
   return units * (TW_DELTA_PREP * (3 * DP + 2L * tw_div_up(E, 16) * 16) + 4);
@@ -838,9 +852,8 @@ extern "C" int tw_delta_rule(const float* qkv, long ld_qkv, int q_col, int k_col
   if (n_seqs == 0) return 0;
   DeltaArgs a{qkv, ld_qkv, q_col, k_col, v_col, ab, ld_ab, b_col, a_col, A_log, dt_bias, state, q_start, state_slots,
               out, ld_out, H, G, D, E, Dk, q_scale};
-  if (max_q_len > TW_DELTA_SHORT_MOST) {
-    // some sequence brings many tokens: every sequence of the step goes through the chunks
-    TW_REQUIRE(workspace != nullptr && (uintptr_t)workspace % 16 == 0 && rows > 0 && H <= 65535 &&
+  if (rows > 0 && H <= 65535 && delta_in_chunks(rows, n_seqs, max_q_len, H, E, Dk)) {
+    TW_REQUIRE(workspace != nullptr && (uintptr_t)workspace % 16 == 0 &&
                workspace_floats >= tw_delta_workspace_floats(rows, n_seqs, max_q_len, H, E, Dk));
     if (Dk <= 64) return delta_chunks<1>(a, seq0, n_seqs, rows, workspace, stream);
     if (Dk <= 128) return delta_chunks<2>(a, seq0, n_seqs, rows, workspace, stream);

@@ -1129,8 +1129,8 @@ def delta_rule(qkv, q_col, k_col, v_col, ab, b_col, a_col, A_log, dt_bias, state
     ab float32 [n, .]: b of head h at b_col + h, a at a_col + h; value head h reads key head h // (H / kv_heads).
     out float32 [n, H * E]. max_q_len: the most tokens a sequence brings (an upper bound will do). Up to a few tokens
     a sequence the tokens are walked one by one; beyond, chunks of 16 or 32 tokens are solved at once (the same sums in another
-    order: a triangular system a chunk in place of a chain of updates), with a float32 workspace of delta_workspace_floats
-    (allocated here if none is given). rows: the most rows these sequences bring together (default: all of qkv's)."""
+    order: a triangular system a chunk in place of a chain of updates), those of 32 with a float32 workspace of
+    delta_workspace_floats (allocated here if none is given). rows: the most rows these sequences bring together (default: all of qkv's)."""
     n, wq, ld_qkv = _rows(qkv, "qkv")
     na, wa, ld_ab = _rows(ab, "ab")
     _need(qkv.dtype == torch.float32 and ab.dtype == torch.float32 and na == n, "the delta rule reads float32 rows")

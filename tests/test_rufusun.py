@@ -98,6 +98,18 @@ def test_delta_layers_walk_a_steps_one_token_sequences_apart(monkeypatch, n_deco
     assert calls[-1][3] == own and sizes[-1] == (own, launches[-1][1], max(1, longest), H, E, D)
 
 
+def test_delta_launches_of_short_portions_keep_the_one_launch_form():
+    """Which launches take the two-launch form (they are the ones that need scratch): long portions, many of them, but not one
+    of a few dozen tokens whose heads fill the chip, nor many that are mostly a chunk's padding."""
+    from tessweave_engine_amd.kernels import ops
+    in_chunks = lambda lens, H, D: ops.delta_workspace_floats(sum(lens), len(lens), max(lens), H, D, D) > 0      # noqa: E731
+    for lens, H, D, want in (([48], 16, 128, False), ([49], 16, 128, True), ([64], 32, 128, False), ([64], 16, 256, False),
+                             ([96], 32, 128, True), ([96], 32, 256, True), ([49] * 16, 32, 128, True), ([60] * 16, 16, 256, True),
+                             ([5] * 60 + [64], 16, 256, False), ([5] * 60 + [64], 32, 128, False), ([17] * 30 + [64], 32, 128, True),
+                             ([1, 1, 500], 16, 256, True), ([2048], 32, 256, True)):
+        assert in_chunks(lens, H, D) is want, (lens, H, D)
+
+
 def test_random_weights_and_inspect_on_the_command_line(tmp_path, capsys):
     from tessweave_engine_amd.cli import main
     from tessweave_engine_amd.config import read_model_config

@@ -229,6 +229,31 @@ def test_delta_rule_chunks_of_many_sequences(device, H, G, D, E):
             assert (walked - chunked).abs().max() < 4e-5 * max(1.0, walked.abs().max().item())
 
 
+@pytest.mark.parametrize("H,G,D,E", [(2, 1, 20, 24), (2, 1, 130, 40)])
+def test_delta_rule_chunks_of_many_longer_sequences(device, H, G, D, E):
+    """Sequences of 49 tokens and more on average with a longest one of 129, which take the chunks of 32 whatever their keys'
+    size, against the same sequences walked token by token (bar as above)."""
+    from tessweave_engine_amd.kernels import ops
+    g = torch.Generator().manual_seed(3)
+    lens = [7] + [1, 97, 64, 33, 129, 2] * 9
+    n = sum(lens)
+    starts, slots = ints(np.cumsum([0] + lens).tolist(), device), ints(torch.randperm(len(lens), generator=g).tolist(), device)
+    qkv, ab = torch.randn(n, 2 * G * D + H * E, generator=g).to(device), torch.randn(n, 2 * H, generator=g).to(device)
+    A_log, dt_bias = (-2.0 + 0.5 * torch.randn(H, generator=g)).to(device), (-3.0 + torch.randn(H, generator=g)).to(device)
+    first = torch.randn(len(lens), H, E, ops.delta_key_extent(D), generator=g).to(device)
+    first[..., D:] = 0
+    results = []
+    for most in (1, 129):
+        assert (ops.delta_workspace_floats(n - 7, len(lens) - 1, most, H, E, D) > 0) == (most > 1)
+        state, out = first.clone(), torch.zeros(n, H * E, device=device)
+        ops.delta_rule(qkv, 0, G * D, 2 * G * D, ab, 0, H, A_log, dt_bias, state, starts, slots, 1, len(lens) - 1, out, G, D,
+                       D ** -0.5, max_q_len=most, rows=n - 7)
+        results.append((out, state))
+    for walked, chunked in zip(*results):
+        assert (walked - chunked).abs().max() < 4e-5 * max(1.0, walked.abs().max().item())
+    assert not results[1][0][:7].any() and torch.equal(results[1][1][slots[0]], first[slots[0]])
+
+
 @pytest.mark.parametrize("D,E", [(64, 20), (128, 64), (200, 32)])
 @pytest.mark.parametrize("alike", [0.5, 0.9])
 def test_delta_rule_chunks_lose_no_precision_where_keys_are_alike(device, D, E, alike):
