@@ -33,6 +33,7 @@ struct DeltaArgs {
   float* out; long ld_out;            // float32 [n][>= H * E]: head h at h * E
   int H, G, D, E, Dk;
   float q_scale;
+  int row0, row1;                     // chunks of 32: of the launch's rows, those that this pair of launches takes
 };
 
 template <int CTRL>
@@ -201,10 +202,19 @@ struct DeltaPrepared {                // per (chunk, head), all in the order the
   float* G;                           // [1]: G_last
 };
 
-// The number of the first chunk of a sequence: chunks of sequences never overlap whatever their lengths, and there are at
-// most rows / 32 + sequences of them.
+// A sequence's rows among those that a pair of launches takes (none: first == last).
+__device__ __forceinline__ void delta_rows(const DeltaArgs& a, int seq0, int s, int& first, int& last) {
+  const int lo = a.q_start[seq0] + a.row0, hi = a.q_start[seq0] + a.row1;
+  first = min(max(a.q_start[s], lo), hi);
+  last = min(max(a.q_start[s + 1], lo), hi);
+}
+
+// The number of a sequence's first chunk: chunks of sequences never overlap whatever their lengths, and there are at most
+// rows / 32 + sequences of them.
 __device__ __forceinline__ int delta_first_chunk(const DeltaArgs& a, int seq0, int s) {
-  return (a.q_start[s] - a.q_start[seq0]) / TW_DELTA_PREP + (s - seq0);
+  int first, last;
+  delta_rows(a, seq0, s, first, last);
+  return (first - a.q_start[seq0] - a.row0) / TW_DELTA_PREP + (s - seq0);
 }
 
 // grid (chunk numbers, H), 256 threads
@@ -229,7 +239,9 @@ __global__ __launch_bounds__(256) void delta_prepare_kernel(DeltaArgs a, DeltaPr
     if (n < 64) break;
   }
   s += seq0;
-  const int t0 = a.q_start[s] + (chunk - delta_first_chunk(a, seq0, s)) * C, last = a.q_start[s + 1];
+  int first, last;
+  delta_rows(a, seq0, s, first, last);
+  const int t0 = first + (chunk - delta_first_chunk(a, seq0, s)) * C;
   if (t0 >= last) return;                            // (a number that no chunk has)
   const int kh = head / (a.H / a.G);
 
@@ -502,7 +514,8 @@ __global__ __launch_bounds__(256) void delta_chunk_kernel(DeltaArgs a, DeltaPrep
   const int r = lane & 15, g = lane >> 4;
   const int e = eb * 16 + r;                         // this lane's value column
   const bool live = e < a.E;
-  const int first = a.q_start[s], last = a.q_start[s + 1];
+  int first, last;
+  delta_rows(a, seq0, s, first, last);
   if (first >= last) return;
   const int chunks = (last - first + C - 1) / C;
   const size_t unit0 = (size_t)delta_first_chunk(a, seq0, s) * a.H + head;
@@ -813,17 +826,33 @@ static bool delta_in_chunks(int rows, int n_seqs, int max_q_len, int H, int E, i
   return max_q_len > (groups > 128 && groups <= 512 ? 88 : 48) && rows >= (Dk <= 128 ? 8L : 48L) * n_seqs;
 }
 
+// Chunks of 32: the scratch of a chunk of one head, and how many rows a pair of launches takes. A step's rows go through in
+// pieces (a sequence's state passes from one to the next through its memory, as from step to step), so that the scratch stays
+// below 512 MB unless 512 rows and the sequences alone need more: 9,200 rows of 16 heads of 128, 3,200 of 32 heads of 256, whose
+// 8,192 rows take 1.4 GB at once. What pieces cost is the sequences that wait for the ones before them: one of 8,192 or 16,384
+// tokens is as fast either way (32 heads of 256 2.7 and 2.8 ms, 5.4 and 5.6), four of 4,096 lose at 16 heads of 128
+// (734 us in one piece, 933 in two, 1,138 in four), less at 32 heads of 256 (5.4 and 5.6 ms), so pieces are no smaller than they
+// have to be.
+static long delta_unit_floats(int E, int Dk) {
+  const long DP = Dk <= 64 ? 64 : Dk <= 128 ? 128 : 256;
+  return TW_DELTA_PREP * (3 * DP + 2L * tw_div_up(E, 16) * 16) + 4;
+}
+static int delta_piece_rows(int rows, int n_seqs, int H, int E, int Dk) {
+  long chunks = (128L << 20) / (delta_unit_floats(E, Dk) * H) - n_seqs;
+  if (chunks < 16) chunks = 16;
+  return chunks * TW_DELTA_PREP < rows ? (int)chunks * TW_DELTA_PREP : rows;
+}
+
 // float32 scratch of a launch over n_seqs sequences of up to `rows` rows together (0: it needs none)
 extern "C" long tw_delta_workspace_floats(int rows, int n_seqs, int max_q_len, int H, int E, int Dk) {
   if (n_seqs <= 0 || rows <= 0 || !delta_in_chunks(rows, n_seqs, max_q_len, H, E, Dk)) return 0;
-  const long units = ((long)rows / TW_DELTA_PREP + n_seqs) * H;
-  const long DP = Dk <= 64 ? 64 : Dk <= 128 ? 128 : 256;
-  return units * (TW_DELTA_PREP * (3 * DP + 2L * tw_div_up(E, 16) * 16) + 4);
+  return ((long)delta_piece_rows(rows, n_seqs, H, E, Dk) / TW_DELTA_PREP + n_seqs) * H * delta_unit_floats(E, Dk);
 }
 
 template <int NT>
-static int delta_chunks(const DeltaArgs& a, int seq0, int n_seqs, int rows, float* workspace, hipStream_t stream) {
-  const size_t chunks = (size_t)rows / TW_DELTA_PREP + n_seqs, units = chunks * a.H;
+static int delta_chunks(DeltaArgs a, int seq0, int n_seqs, int rows, float* workspace, hipStream_t stream) {
+  const int piece = delta_piece_rows(rows, n_seqs, a.H, a.E, a.Dk);
+  const size_t chunks = (size_t)piece / TW_DELTA_PREP + n_seqs, units = chunks * a.H;
   const size_t keys = units * TW_DELTA_PREP * 64 * NT, values = units * TW_DELTA_PREP * 16 * tw_div_up(a.E, 16);
   DeltaPrepared p;
   p.W = workspace;
@@ -832,8 +861,11 @@ static int delta_chunks(const DeltaArgs& a, int seq0, int n_seqs, int rows, floa
   p.U = p.K + keys;
   p.O = p.U + values;
   p.G = p.O + values;
-  delta_prepare_kernel<NT><<<dim3((unsigned)chunks, a.H), 256, 0, stream>>>(a, p, seq0, n_seqs);
-  delta_chunk_kernel<NT><<<dim3(a.H * tw_div_up(a.E, 16), n_seqs), 256, 0, stream>>>(a, p, seq0);
+  for (a.row0 = 0; a.row0 < rows; a.row0 += piece) {
+    a.row1 = min(rows, a.row0 + piece);
+    delta_prepare_kernel<NT><<<dim3((unsigned)chunks, a.H), 256, 0, stream>>>(a, p, seq0, n_seqs);
+    delta_chunk_kernel<NT><<<dim3(a.H * tw_div_up(a.E, 16), n_seqs), 256, 0, stream>>>(a, p, seq0);
+  }
   return TW_LAUNCH_RESULT();
 }
 
@@ -851,7 +883,7 @@ extern "C" int tw_delta_rule(const float* qkv, long ld_qkv, int q_col, int k_col
   TW_REQUIRE(ld_ab >= (long)max(a_col, b_col) + H);
   if (n_seqs == 0) return 0;
   DeltaArgs a{qkv, ld_qkv, q_col, k_col, v_col, ab, ld_ab, b_col, a_col, A_log, dt_bias, state, q_start, state_slots,
-              out, ld_out, H, G, D, E, Dk, q_scale};
+              out, ld_out, H, G, D, E, Dk, q_scale, 0, 0};
   if (rows > 0 && H <= 65535 && delta_in_chunks(rows, n_seqs, max_q_len, H, E, Dk)) {
     TW_REQUIRE(workspace != nullptr && (uintptr_t)workspace % 16 == 0 &&
                workspace_floats >= tw_delta_workspace_floats(rows, n_seqs, max_q_len, H, E, Dk));

@@ -110,6 +110,15 @@ def test_delta_launches_of_short_portions_keep_the_one_launch_form():
         assert in_chunks(lens, H, D) is want, (lens, H, D)
 
 
+def test_delta_scratch_is_bounded():
+    """Scratch of the two-launch form: up to 512 MB however many rows a step has (its rows go through in pieces then)."""
+    from tessweave_engine_amd.kernels import ops
+    sizes = [4 * ops.delta_workspace_floats(rows, 2, rows, 32, 256, 256) for rows in (512, 2048, 4096, 8192, 1 << 20)]
+    assert sizes == sorted(sizes) and 0 < sizes[0] < sizes[1] < sizes[2] == sizes[4] <= 1 << 29
+    # (a piece has 512 rows at least)
+    assert 4 * ops.delta_workspace_floats(8192, 1, 8192, 256, 256, 256) == 4 * ops.delta_workspace_floats(512, 1, 512, 256, 256, 256)
+
+
 def test_random_weights_and_inspect_on_the_command_line(tmp_path, capsys):
     from tessweave_engine_amd.cli import main
     from tessweave_engine_amd.config import read_model_config

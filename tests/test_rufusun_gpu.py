@@ -254,6 +254,32 @@ def test_delta_rule_chunks_of_many_longer_sequences(device, H, G, D, E):
     assert not results[1][0][:7].any() and torch.equal(results[1][1][slots[0]], first[slots[0]])
 
 
+def test_delta_rule_rows_in_pieces(device):
+    """More rows than the scratch takes at once: pieces that end inside sequences and inside chunks, a sequence that ends where
+    a piece does, one behind it and one of no rows, against chunks of 16 in one launch (bar as above)."""
+    from tessweave_engine_amd.kernels import ops
+    H, G, D, E = 64, 1, 256, 256
+    piece = 32 * ((128 << 20) // ((32 * 5 * 256 + 4) * H) - 5)
+    lens = [3, 40, piece - 40, 700, 0, piece + 37]
+    n = sum(lens)
+    g = torch.Generator(device=device).manual_seed(5)
+    qkv, ab = torch.randn(n, 2 * G * D + H * E, generator=g, device=device), torch.randn(n, 2 * H, generator=g, device=device)
+    A_log, dt_bias = -2.0 + 0.5 * torch.randn(H, generator=g, device=device), -3.0 + torch.randn(H, generator=g, device=device)
+    starts, slots = ints(np.cumsum([0] + lens).tolist(), device), ints([2, 0, 5, 1, 3, 4], device)
+    first = torch.randn(6, H, E, D, generator=g, device=device)
+    floats = ops.delta_workspace_floats(n - 3, 5, max(lens), H, E, D)
+    assert floats == (piece // 32 + 5) * H * (32 * 5 * 256 + 4)
+    results = []
+    for most, scratch in ((max(lens), torch.full((floats,), float("nan"), device=device)), (48, None)):
+        state, out = first.clone(), torch.full((n, H * E), float("nan"), device=device)
+        ops.delta_rule(qkv, 0, G * D, 2 * G * D, ab, 0, H, A_log, dt_bias, state, starts, slots, 1, 5, out, G, D, D ** -0.5,
+                       max_q_len=most, workspace=scratch, rows=n - 3)
+        results.append((out, state))
+    assert results[0][0][:3].isnan().all() and torch.equal(results[0][1][2], first[2]) and torch.equal(results[0][1][3], first[3])
+    for pieces, whole in zip((results[0][0][3:], results[0][1]), (results[1][0][3:], results[1][1])):
+        assert (pieces - whole).abs().max() < 4e-5 * max(1.0, whole.abs().max().item())
+
+
 @pytest.mark.parametrize("D,E", [(64, 20), (128, 64), (200, 32)])
 @pytest.mark.parametrize("alike", [0.5, 0.9])
 def test_delta_rule_chunks_lose_no_precision_where_keys_are_alike(device, D, E, alike):
