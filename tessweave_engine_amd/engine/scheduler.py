@@ -191,18 +191,23 @@ class Engine:
     def _admit(self):
         """Admit from the head of the queue while a request slot and every page the head can ever need are
         to be had. A head that does not fit stops admission: nobody overtakes it, so it cannot starve."""
+        if not self.waiting:
+            return
         budget = self.config.step_token_budget
-        while self.waiting and len(self.active) < self.config.max_active:
-            r = self.waiting[0]
-            try:
-                r.seq = self.cache.admit(r.id, r.prompt, len(r.prompt) + r.max_tokens, budget, r.namespace)
-            except CapacityError:
-                return
-            self.waiting.popleft()
-            r.cached = r.published = r.seq.cached
-            r.status = "active"
-            self.active.append(r)
-            self.trace.emit("admit", request_id=r.id, reused_tokens=r.cached, **self.cache.stats())
+        # On the steps' own stream: opening a request clears its slot's recurrent state, behind the step in flight, which may
+        # still write what the slot's last request left there, and in front of the request's first step.
+        with self._sampling_stream():
+            while self.waiting and len(self.active) < self.config.max_active:
+                r = self.waiting[0]
+                try:
+                    r.seq = self.cache.admit(r.id, r.prompt, len(r.prompt) + r.max_tokens, budget, r.namespace)
+                except CapacityError:
+                    return
+                self.waiting.popleft()
+                r.cached = r.published = r.seq.cached
+                r.status = "active"
+                self.active.append(r)
+                self.trace.emit("admit", request_id=r.id, reused_tokens=r.cached, **self.cache.stats())
 
     # ---- one turn ----------------------------------------------------------------------
     def plan(self):

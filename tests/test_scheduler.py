@@ -633,3 +633,29 @@ def test_prompt_blocks_are_shared_early_under_lookahead_too():
     e.close()
     e.cache.check()
     assert len(e.cache.pools[0].free) == 32
+
+
+def test_requests_are_admitted_on_the_steps_stream(monkeypatch):
+    """Opening a request clears its slot's recurrent state on the device. With lookahead the step in flight may still write the
+    slot's last request there, so the clearing goes to the stream of the steps, like everything else of a turn."""
+    import contextlib
+    engine = make(max_active=1)[0]
+    inside, seen = [], []
+
+    @contextlib.contextmanager
+    def stream():
+        inside.append(True)
+        yield
+        inside.pop()
+
+    monkeypatch.setattr(engine, "_sampling_stream", stream)
+    opened, step = engine.cache.open, engine.stepper.step
+    monkeypatch.setattr(engine.cache, "open", lambda seq_id: seen.append(("open", bool(inside))) or opened(seq_id))
+    monkeypatch.setattr(engine.stepper, "step", lambda entries: seen.append(("step", bool(inside))) or step(entries))
+    FakeStepper.full = {}
+    for prompt in ([1, 2, 3], [4, 5]):
+        r = engine.submit(prompt, max_tokens=2, ignore_eos=True)
+        FakeStepper.full[r.id] = r.tokens
+    while engine.step():
+        pass
+    assert [kind for kind, _ in seen].count("open") >= 2 and all(on_stream for _, on_stream in seen), seen
