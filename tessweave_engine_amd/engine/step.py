@@ -80,7 +80,8 @@ class Stepper:
         self.dtype = model.dtype
         self.workspace = Workspace(self.device)
         self.stream = torch.cuda.Stream(device=self.device)     # captures run here; a step runs on its caller's stream
-        self._end, self._end_stream = None, None                 # the last step's end and the stream it ran on
+        self._end, self._end_stream = None, None                 # the end of the last work issued here, and its stream
+        self._by_hand = None             # the stream of work that its caller issues by hand (upload, model.forward)
         self.use_graphs = bool(use_graphs) and model.graph_safe_model
         self._defer_sums = bool(getattr(model, "defers_sums", False))
         self.position_axes = max(1, int(getattr(model, "position_axes", 1)))
@@ -105,7 +106,9 @@ class Stepper:
         Steps already issued are waited for first: the kernel that fetches a step's metadata reads the pinned buffer when
         it runs, the allocator does not know of it, and would hand the same memory to the new buffers at once."""
         self._drop_graphs()
+        stream = torch.cuda.current_stream(self.device)
         self.synchronize()
+        self._follow(stream)
         for event in self._staging_events:
             if event is not None:
                 event.synchronize()
@@ -136,6 +139,9 @@ class Stepper:
         self._staging_np = [t.numpy() for t in self._staging]
         self._staging_events = [None] * 4
         self._staging_next = 0
+        # a first step on another stream comes behind this stream's work: the clearing of the new buffers, and the model's and
+        # the cache's initialisation if they were made here
+        self._mark(stream)
 
     def _dev(self, name, count=None):
         off, cap = self._sections[name]
@@ -174,9 +180,11 @@ class Stepper:
             self.token_feed = feed
 
     def synchronize(self):
-        """Wait for the last step, and for whatever its caller has put on the stepper's own stream."""
+        """Wait for the last step, and for whatever its caller has put on the stepper's own stream or issued by hand."""
         if self._end is not None:
             self._end.synchronize()
+        if self._by_hand is not None:
+            self._by_hand.synchronize()
         self.stream.synchronize()
 
     # ---- the step ----------------------------------------------------------------------
@@ -202,17 +210,25 @@ class Stepper:
                 logits = self.model.forward(ctx)
         finally:
             # one event a step: the staging buffer is free again, and the next step knows what to follow
-            self._end, self._end_stream = torch.cuda.Event(), stream.cuda_stream
-            self._end.record(stream)
+            self._mark(stream)
             self._staging_events[ctx.staging_index] = self._end
         self.finish(ordered)
         return logits
 
+    def _mark(self, stream):
+        """What has been issued here so far ends where STREAM is now."""
+        self._end, self._end_stream = torch.cuda.Event(), stream.cuda_stream
+        self._end.record(stream)
+
     def _follow(self, stream):
-        """A step on another stream than the last one's waits for that one's end (they share scratch memory), and the
-        scratch memory, which may have been allocated for the other stream, is marked as used on this one as well."""
+        """Work on another stream than the last one's waits for that one's end (they share scratch memory and the metadata
+        buffer), and this memory, which may have been allocated for the other stream, is marked as used on this one as well.
+        Work issued by hand is waited for up to where its stream is now: its caller went on there behind `upload`."""
+        by_hand, self._by_hand = self._by_hand, None
         if self._end is None or self._end_stream == stream.cuda_stream:
             return
+        if by_hand is not None:
+            stream.wait_stream(by_hand)
         stream.wait_event(self._end)
         for tensor in (self._meta_dev, *self.workspace.buffers.values()):
             tensor.record_stream(stream)
@@ -228,10 +244,12 @@ class Stepper:
         """Bring the step's packed metadata to the device (on the current stream): a kernel fetches the parts
         this step filled from the pinned staging buffer, which keeps the step in one queue (a memory copy
         would hand over to the copy engine and back, tens of microseconds of idle queue per step)."""
+        stream = torch.cuda.current_stream(self.device)
+        self._follow(stream)
         self._upload(ctx)
-        event = torch.cuda.Event()
-        event.record(torch.cuda.current_stream(self.device))
-        self._staging_events[ctx.staging_index] = event
+        self._mark(stream)
+        self._by_hand = stream
+        self._staging_events[ctx.staging_index] = self._end
 
     def _upload(self, ctx):
         k = ctx.staging_index

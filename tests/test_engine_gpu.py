@@ -103,6 +103,41 @@ def test_steps_called_from_changing_streams(tiny):
     assert torch.equal(run(lambda i: 0), run(lambda i: i % 3))
 
 
+def test_first_step_and_work_by_hand_are_followed(tiny):
+    """A first step from another stream than the one the stepper and its cache were made on, while that one is busy; work issued
+    by hand on the stepper's stream, behind a busy device, and a step from the default stream behind it: the same as from one
+    stream."""
+    from tessweave_engine_amd.cache import CacheManager
+    from tessweave_engine_amd.engine import StepEntry, Stepper
+    from tessweave_engine_amd.weights import load_model
+    model = load_model(tiny["folder"], dtype="float32", device="cuda:0")
+    tokens = prompts_for(tiny, [24], seed=12)[0]
+    busy, default, side = torch.randn(4096, 4096, device="cuda"), torch.cuda.default_stream(), torch.cuda.Stream()
+
+    def run(mixed):
+        torch.cuda.synchronize()
+        for _ in range(20 * mixed):
+            busy @ busy
+        cache = CacheManager(model.cache_layout(), tiny["page"], 60, 2, dtype="float32", device=model.device, prefix_cache=False)
+        stepper, rows = Stepper(model, cache, max_step_tokens=16), []
+        seq = cache.open("a")
+        with torch.cuda.stream(side if mixed else default):
+            rows.append(stepper.step([StepEntry(seq, tokens[:9], [8])]).clone())
+        ctx, ordered, _ = stepper.prepare([StepEntry(seq, tokens[9:20], [10])])
+        with torch.cuda.stream(stepper.stream if mixed else default):
+            stepper.upload(ctx)
+            for _ in range(20 * mixed):
+                busy @ busy
+            rows.append(model.forward(ctx).clone())
+        stepper.finish(ordered)
+        rows += [stepper.step([StepEntry(seq, [t], [0])]).clone() for t in tokens[20:]]
+        torch.cuda.synchronize()
+        stepper.close()
+        return torch.cat(rows)
+
+    assert torch.equal(run(False), run(True))
+
+
 def test_step_buffers_grow_behind_a_busy_device(tiny):
     """Every request is longer than any before, so every step grows the stepper's buffers while the step before still waits
     for the device: its metadata must reach it all the same."""
