@@ -70,6 +70,38 @@ class _Graph:
                 lib.tw_graph_destroy(handle)
 
 
+class _Staging:
+    """Pinned buffers in which steps' metadata waits for the device, taken in turn.
+
+    The kernel that fetches a step's metadata reads its buffer when it runs. The allocator of pinned memory does not know
+    of it and would hand the memory to its next taker at once, so the buffers are let go only once their readers are done."""
+
+    def __init__(self, words, count=4):
+        self.buffers = [torch.zeros(words, dtype=torch.int32, pin_memory=True) for _ in range(count)]
+        self.arrays = [t.numpy() for t in self.buffers]
+        self.readers = [None] * count        # per buffer: an event behind its last reader
+        self.next = 0
+
+    def take(self):
+        """Index of the next buffer, whose last reader is done."""
+        k = self.next
+        self.next = (k + 1) % len(self.buffers)
+        if self.readers[k] is not None:
+            self.readers[k].synchronize()
+        return k
+
+    def wait(self):
+        for event in self.readers:
+            if event is not None:
+                event.synchronize()
+
+    def __del__(self):
+        try:
+            self.wait()
+        except Exception:       # noqa: BLE001  (half made, or the interpreter is going down)
+            pass
+
+
 class Stepper:
     def __init__(self, model, cache, max_step_tokens=256, max_step_seqs=None, use_graphs=True, max_graphs=MAX_GRAPHS):
         if model.device is None or model.device.type != "cuda":
@@ -92,9 +124,7 @@ class Stepper:
         self.max_graphs = max(1, int(max_graphs))
         self.token_feed = None
         self.segment_graphs = True
-        self._staging = []
-        self._staging_events = []
-        self._staging_next = 0
+        self._staging = None
         self.steps = 0
         self.graph_replays = 0
         self._reserve(max(1, int(max_step_tokens)), int(max_step_seqs or cache.max_requests))
@@ -103,15 +133,11 @@ class Stepper:
     def _reserve(self, max_tokens, max_seqs):
         """(Re)allocate the metadata buffers for steps of up to MAX_TOKENS rows and MAX_SEQS requests.
 
-        Steps already issued are waited for first: the kernel that fetches a step's metadata reads the pinned buffer when
-        it runs, the allocator does not know of it, and would hand the same memory to the new buffers at once."""
+        Steps already issued are waited for first (see _Staging)."""
         self._drop_graphs()
         stream = torch.cuda.current_stream(self.device)
         self.synchronize()
         self._follow(stream)
-        for event in self._staging_events:
-            if event is not None:
-                event.synchronize()
         self.max_tokens, self.max_seqs = max_tokens, max_seqs
         width = self.cache.table_width
         n_groups = len(self.cache.pools)
@@ -135,10 +161,8 @@ class Stepper:
             add(f"table{g}", max_seqs * width)
         self._sections, self._meta_ints = sections, offset
         self._meta_dev = torch.zeros(offset, dtype=torch.int32, device=self.device)
-        self._staging = [torch.zeros(offset, dtype=torch.int32, pin_memory=True) for _ in range(4)]
-        self._staging_np = [t.numpy() for t in self._staging]
-        self._staging_events = [None] * 4
-        self._staging_next = 0
+        self._staging = None                 # (the old buffers go first)
+        self._staging = _Staging(offset)
         # a first step on another stream comes behind this stream's work: the clearing of the new buffers, and the model's and
         # the cache's initialisation if they were made here
         self._mark(stream)
@@ -163,7 +187,10 @@ class Stepper:
         graph.destroy(library())
 
     def close(self):
+        """Let go of captured steps and wait for what has been issued."""
         self._drop_graphs()
+        self.synchronize()
+        self._staging.wait()
 
     accepts_token_feed = True
 
@@ -211,7 +238,7 @@ class Stepper:
         finally:
             # one event a step: the staging buffer is free again, and the next step knows what to follow
             self._mark(stream)
-            self._staging_events[ctx.staging_index] = self._end
+            self._staging.readers[ctx.staging_index] = self._end
         self.finish(ordered)
         return logits
 
@@ -249,14 +276,14 @@ class Stepper:
         self._upload(ctx)
         self._mark(stream)
         self._by_hand = stream
-        self._staging_events[ctx.staging_index] = self._end
+        self._staging.readers[ctx.staging_index] = self._end
 
     def _upload(self, ctx):
         k = ctx.staging_index
         if ctx.staging_segments is not None and len(ctx.staging_segments) <= 16:
-            ops.upload_words(self._staging[k], self._meta_dev, ctx.staging_segments)
+            ops.upload_words(self._staging.buffers[k], self._meta_dev, ctx.staging_segments)
         else:
-            self._meta_dev.copy_(self._staging[k], non_blocking=True)
+            self._meta_dev.copy_(self._staging.buffers[k], non_blocking=True)
 
     def prepare(self, entries):
         """Check ENTRIES, take their pages, and build the step's context (host side; nothing runs yet).
@@ -308,11 +335,8 @@ class Stepper:
         n_logits = len(rows)
 
         # pack the metadata into a pinned buffer and upload it once
-        k = self._staging_next
-        self._staging_next = (k + 1) % len(self._staging)
-        if self._staging_events[k] is not None:
-            self._staging_events[k].synchronize()
-        host = self._staging_np[k]
+        k = self._staging.take()
+        host = self._staging.arrays[k]
 
         segments = []                        # (offset, words) of what this step fills: all that has to travel
 

@@ -103,6 +103,36 @@ def test_steps_called_from_changing_streams(tiny):
     assert torch.equal(run(lambda i: 0), run(lambda i: i % 3))
 
 
+@pytest.mark.parametrize("close", [True, False], ids=["closed", "dropped"])
+def test_stepper_let_go_behind_a_busy_device(tiny, close):
+    """A stepper closed or dropped while its step still waits for the device, and another one made at once, whose staging
+    buffers are cleared by the host: the step's metadata must reach the device all the same."""
+    from tessweave_engine_amd.cache import CacheManager
+    from tessweave_engine_amd.engine import StepEntry, Stepper
+    from tessweave_engine_amd.weights import load_model
+    model = load_model(tiny["folder"], dtype="float32", device="cuda:0")
+    prompts = prompts_for(tiny, [20, 31, 12, 25], seed=13)
+    busy = torch.randn(4096, 4096, device="cuda")
+
+    def run(wait):
+        rows = []
+        for i, tokens in enumerate(prompts):
+            cache = CacheManager(model.cache_layout(), tiny["page"], 20, 1, dtype="float32", device=model.device, prefix_cache=False)
+            stepper = Stepper(model, cache, max_step_tokens=32)
+            for _ in range(20):
+                busy @ busy
+            rows.append(stepper.step([StepEntry(cache.open(i), tokens, [len(tokens) - 1])]).clone())
+            if wait:
+                torch.cuda.synchronize()
+            if close:
+                stepper.close()
+            del stepper
+        torch.cuda.synchronize()
+        return torch.cat(rows)
+
+    assert torch.equal(run(True), run(False))
+
+
 def test_first_step_and_work_by_hand_are_followed(tiny):
     """A first step from another stream than the one the stepper and its cache were made on, while that one is busy; work issued
     by hand on the stepper's stream, behind a busy device, and a step from the default stream behind it: the same as from one

@@ -659,3 +659,26 @@ def test_requests_are_admitted_on_the_steps_stream(monkeypatch):
     while engine.step():
         pass
     assert [kind for kind, _ in seen].count("open") >= 2 and all(on_stream for _, on_stream in seen), seen
+
+
+def test_staging_memory_outlives_its_readers():
+    """Kernels read a stepper's pinned staging buffers when they run. Closing a stepper waits for them whether or not it has
+    captured steps, and the buffers themselves wait where a stepper is dropped."""
+    from types import SimpleNamespace
+    from tessweave_engine_amd.engine.step import Stepper, _Staging
+
+    def event(done):
+        return SimpleNamespace(synchronize=lambda: done.append(True))
+
+    done, staging = [], _Staging.__new__(_Staging)
+    staging.buffers, staging.readers, staging.next = [None] * 3, [None, event(done), event(done)], 0
+    assert staging.take() == 0 and not done and staging.take() == 1 and len(done) == 1
+    done.clear()
+    stepper = Stepper.__new__(Stepper)
+    stepper._graphs, stepper._warm, stepper._staging, stepper._by_hand = {}, set(), staging, None
+    stepper._end, stepper.stream = event(done), event([])
+    stepper.close()
+    assert len(done) == 3
+    done.clear()
+    del stepper, staging
+    assert len(done) == 2
