@@ -47,25 +47,26 @@ def _round_up(v, m):
 
 GRAPH_SEGMENT_RUNS = 8       # layer runs per captured graph after the first
 MIN_LENGTH_CLASS = 512       # steps whose longest sequence is shorter share one captured graph
-SECOND_FORM_REPLAYS = 16     # a captured step's other form (cut into segments or whole) is captured after so many replays
+SECOND_FORM_MISSES = 16      # a captured step's other form (cut into segments or whole) is captured after so many launches
+                             # that wanted it
 MAX_GRAPHS = 96              # captured steps kept (one per batch size and length class met); the least recently
                              # replayed one goes first
 
 
 class _Graph:
-    """A captured decode step: a list of graphs launched one after the other (see Stepper._capture), in one or both of two
-    forms, {cut into segments?: handles}.
+    """A captured decode step in one or both of two forms, {cut into segments?: (graphs launched one after the other, the
+    logits they leave)} (see Stepper._capture).
 
-    BUFFERS names the scratch buffers whose addresses the capture holds, each with its version at the
-    time: the capture stays good until one of THOSE is allocated anew (a larger prompt portion growing a
+    BUFFERS names the scratch buffers whose addresses the captures hold, each with its version at the
+    time: the captures stay good until one of THOSE is allocated anew (a larger prompt portion growing a
     buffer that only prompt portions use leaves every captured decode step alone)."""
 
-    def __init__(self, segmented, handles, logits, generation, buffers):
-        self.forms, self.logits, self.generation, self.buffers = {segmented: handles}, logits, generation, buffers
-        self.replays = 0
+    def __init__(self, generation):
+        self.forms, self.generation, self.buffers = {}, generation, {}
+        self.missed = 0                      # launches that wanted the form that is not there
 
     def destroy(self, lib):
-        for handles in self.forms.values():
+        for handles, _ in self.forms.values():
             for handle in handles:
                 lib.tw_graph_destroy(handle)
 
@@ -469,28 +470,35 @@ class Stepper:
             else:
                 self._drop_graph(key)
                 graph = None
-        # A step that is launched while the step before still runs goes out as one graph: its launch is hidden, and every
-        # cut costs about 8 us between two graphs. (The scheduler's lookahead, whose launches always are, turns cutting off.)
-        segmented = self.segment_graphs and (self._end is None or self._end.query())
         if graph is None:
             if key not in self._warm:
                 # First time at this batch size and length class: run eagerly so every scratch buffer exists.
                 self._warm.add(key)
                 return self.model.forward(ctx)
-            handles, logits, buffers = self._capture(ctx, segmented)
-            graph = self._graphs[key] = _Graph(segmented, handles, logits, self.workspace.generation, buffers)
+            # (the device runs dry while the host captures: the form for an idle one, where cutting is on)
+            graph = _Graph(self.workspace.generation)
+            self._add_form(graph, ctx, self.segment_graphs)
+            self._graphs[key] = graph
             while len(self._graphs) > self.max_graphs:
                 self._drop_graph(next(iter(self._graphs)))
         else:
             self._graphs.move_to_end(key)
-            if segmented not in graph.forms:
-                if graph.replays >= SECOND_FORM_REPLAYS:     # (a capture costs as much as some steps)
-                    graph.forms[segmented] = self._capture(ctx, segmented)[0]
-                else:
-                    segmented = not segmented
+        # A step that is launched while the step before still runs goes out as one graph: its launch is hidden, and every
+        # cut costs about 8 us between two graphs. (The scheduler's lookahead, whose launches always are, turns cutting off.)
+        segmented = wanted = self.segment_graphs and (self._end is None or self._end.query())
+        if wanted not in graph.forms:
+            segmented = not wanted
+            graph.missed += 1
+        handles, logits = graph.forms[segmented]
         lib = library()
-        for handle in graph.forms[segmented]:
+        for handle in handles:
             check(lib.tw_graph_launch(handle, stream.cuda_stream), "graph launch")
-        graph.replays += 1
         self.graph_replays += 1
-        return graph.logits
+        if graph.missed >= SECOND_FORM_MISSES and wanted not in graph.forms:
+            self._add_form(graph, ctx, wanted)       # (behind the launch: the device has this step to run meanwhile)
+        return logits
+
+    def _add_form(self, graph, ctx, segmented):
+        handles, logits, buffers = self._capture(ctx, segmented)
+        graph.forms[segmented] = (handles, logits)
+        graph.buffers.update(buffers)

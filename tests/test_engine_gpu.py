@@ -168,6 +168,42 @@ def test_first_step_and_work_by_hand_are_followed(tiny):
     assert torch.equal(run(False), run(True))
 
 
+def test_both_forms_of_a_captured_step(tiny):
+    """A decode step is captured cut into segments (the device is idle behind a capture), whether or not it was busy before;
+    steps launched behind a busy device get the whole form after a while, once and with the same logits, an idle one never."""
+    from tessweave_engine_amd.cache import CacheManager
+    from tessweave_engine_amd.engine import StepEntry, Stepper
+    from tessweave_engine_amd.engine.step import SECOND_FORM_MISSES
+    from tessweave_engine_amd.weights import load_model
+    model = load_model(tiny["folder"], dtype="float32", device="cuda:0")
+    tokens = prompts_for(tiny, [2 * SECOND_FORM_MISSES + 20], seed=14)[0]
+    busy = torch.randn(4096, 4096, device="cuda")
+
+    def run(is_busy):
+        cache = CacheManager(model.cache_layout(), tiny["page"], 100, 1, dtype="float32", device=model.device, prefix_cache=False)
+        stepper, rows, forms = Stepper(model, cache, max_step_tokens=16), [], []
+        captures, capture = [], stepper._capture
+        stepper._capture = lambda ctx, segmented: captures.append(segmented) or capture(ctx, segmented)
+        seq = cache.open("a")
+        for t in tokens:
+            for _ in range(3 * is_busy):
+                busy @ busy
+            rows.append(stepper.step([StepEntry(seq, [t], [0])]).clone())
+            forms.append(len(captures))
+            if not is_busy:
+                torch.cuda.synchronize()
+        torch.cuda.synchronize()
+        (graph,) = stepper._graphs.values()
+        assert stepper.graph_replays == len(tokens) - 1 and set(graph.forms) == set(captures)
+        stepper.close()
+        return torch.cat(rows), captures, forms
+
+    (idle, captures, _), (queued, both, at) = run(False), run(True)
+    assert captures == [True] and both == [True, False]
+    assert at[1] == 1 and at.index(2) >= SECOND_FORM_MISSES
+    assert torch.equal(idle, queued)
+
+
 def test_step_buffers_grow_behind_a_busy_device(tiny):
     """Every request is longer than any before, so every step grows the stepper's buffers while the step before still waits
     for the device: its metadata must reach it all the same."""
