@@ -787,23 +787,34 @@ static int launch_skinny_lds_m(const T* A, long lda, const T* W, long ldw, const
 }
 
 // Up to 16 rows of a shuffled weight: is the kernel with 16 output columns (GLU: 16 pairs) over the whole of K a
-// workgroup faster than the one with K ranges? Measured with weights from HBM, back to back, at 8 rows (bf16; us,
-// K ranges and their reduction / whole K):
-//    N x K        1536 x 512   2048 x 1024   2048 x 2048   3584 x 3584   896 x 4864   4608 x 3584   8192 x 2048
-//                 4.7 / 3.1    6.1 / 3.5     6.6 / 4.4     9.8 / 7.0     8.5 / 8.4    10.7 / 11.3   10.7 / 7.6
-//    N x 256:     3584 4.0 / 3.2, 4608 4.0 / 4.2;   N x 1536: 24576 15.7 / 15.1, with 16 rows 15.8 / 18.9
-//    GLU (K ranges: always one):   8192 x 512 4.7 / 4.0,   9728 x 896 6.5 / 6.2,   8192 x 2048 9.9 / 7.3,
-//                 37888 x 512 9.2 / 10.6,   22016 x 2048 17.7 / 16.6,   9728 x 3584 16.2 / 16.8
+// workgroup faster than the one with K ranges? Measured with weights from HBM, back to back (us, K ranges and their
+// reduction / whole K), at 1, 8 and 16 rows:
+//    N x K, bf16       256 x 1024          256 x 3072          256 x 4096         1536 x 4096         4096 x 4096
+//      1           4.9 / 2.4           6.0 / 4.3           6.0 / 4.9           7.6 / 5.3          11.2 / 7.4
+//      8           5.5 / 3.0           6.5 / 5.3           6.6 / 5.9           7.8 / 6.4          11.5 / 7.8
+//     16           6.0 / 3.5           6.9 / 6.6           6.9 / 7.5           8.3 / 8.0          12.4 / 9.0
+//                  4608 x 256          4608 x 512         6144 x 1536         8192 x 2048         4608 x 3584
+//      1           3.8 / 3.5           4.8 / 3.8           8.5 / 5.6          10.5 / 7.3          10.4 / 9.9
+//      8           4.1 / 4.2           5.0 / 4.4           8.8 / 6.5          10.8 / 7.6          10.7 / 11.5
+//     16           4.3 / 5.0           5.3 / 5.2           9.6 / 7.7          11.5 / 8.8          11.7 / 13.9
+//    gated             2048 x 4096         8192 x 4096         9728 x 896         9728 x 2048         16384 x 2048        22016 x 2048       37888 x 512
+//      1          14.4 / 7.4          19.2 / 12.9          6.2 / 5.7          10.0 / 9.4          14.1 / 12.4         17.1 / 16.0        8.7 / 9.7
+//      8          14.7 / 8.4          17.5 / 13.4          6.3 / 6.1          10.2 / 10.1         13.6 / 12.2         16.7 / 16.0        9.0 / 10.6
+//     16          15.1 / 9.8          17.9 / 16.5          6.6 / 6.8          10.5 / 11.5         13.9 / 12.7         17.3 / 17.1        9.6 / 11.7
+//    float32, K halved (the same k-steps): the same signs, but gated 9728 x 768 9.2 / 9.4, 9.3 / 9.8, 9.5 / 10.3 and
+//    x 1024 12.1 / 11.0, 11.3 / 11.3, 11.5 / 12.4 (bf16 9728 x 1536 8.3 / 8.0, 8.4 / 8.6, 8.6 / 9.3).
 // Up to 256 workgroups (one a CU): as long as a wave's share of K is about what it keeps in flight (8 k-steps of 16
-// waves), K <= 4096 in bf16. With more, the CUs are uneven and every workgroup reads the activations again: only
-// where the other kernel's waves sit through a chain of stages and the weights outweigh the activations.
+// waves), K <= 4096 in bf16; where few workgroups leave the chip to the K ranges, more than 8 rows end sooner.
+// With more workgroups every one reads the activations again: only where the other kernel's waves sit through a chain
+// of stages and the weights outweigh the activations. Gated, between one and two a CU, the second round is nearly empty
+// and up to 8 rows (in float32 fewer k-steps too) are the most that pays.
 // `sums`: float32 sums for the caller's next kernel, no reduction saved: only where the other kernel has one range too
-// (4096 x 896: 5.6 / 3.4).
-static bool narrow_pays(int N, int K, int epf, bool glu, bool sums) {
+// (bf16, 1 and 16 rows: 256 x 512 2.9 / 2.2, 3.2 / 2.9; 4096 x 896 5.4 / 3.4, 6.1 / 4.1; float32 4096 x 448 6.3 / 3.9, 6.9 / 4.4).
+static bool narrow_pays(int M, int N, int K, int epf, bool glu, bool sums) {
   const int steps = tw_div_up(K / epf, 4), groups = glu ? N / 32 : tw_div_up(N, 16);
   if (sums) return groups <= 256 && steps >= 16 && steps < 32;
-  if (groups <= 256) return steps <= 128;
-  if (glu) return steps >= 28 && steps <= 64;
+  if (groups <= 256) return steps <= (M > 8 && groups < 96 && !glu ? 96 : 128);
+  if (glu) return steps >= 28 && steps <= (groups < 512 && epf == 4 ? 32 : 64) && (M <= 8 || groups >= 512);
   return groups <= 512 && steps >= 16 && steps <= 64;
 }
 
@@ -848,7 +859,7 @@ static int linear_dispatch(const T* A, long lda, const T* W, long ldw, const flo
       return launch_stream_cu<T, OutT, false, GLU>(A, lda, W, ldw, bias, residual, ldr, C, ldc, partial, partial_bytes, M, N, K, stream);
   }
   if constexpr (SHUF) {
-    if (force == 9 || (force == 0 && M <= 16 && narrow_pays(N, K, EPF, GLU, false))) {
+    if (force == 9 || (force == 0 && M <= 16 && narrow_pays(M, N, K, EPF, GLU, false))) {
       TW_REQUIRE(M <= 16);
       return launch_narrow<T, OutT, GLU>(A, lda, W, ldw, bias, residual, ldr, C, ldc, M, N, K, stream);
     }
@@ -968,7 +979,7 @@ static int partials_layout(int shuffled, const T* A, long lda, const T* W, long 
                            long partial_bytes, int M, int N, int K, hipStream_t stream) {
   if (shuffled && M > TW_CU_ABOVE_ROWS)
     return launch_stream_cu<T, float, true, false>(A, lda, W, ldw, nullptr, nullptr, 0, (float*)nullptr, N, partial, partial_bytes, M, N, K, stream);
-  if (shuffled && M <= 16 && narrow_pays(N, K, Elem<T>::kPerFrag, false, true)) {
+  if (shuffled && M <= 16 && narrow_pays(M, N, K, Elem<T>::kPerFrag, false, true)) {
     TW_REQUIRE(partial != nullptr && partial_bytes >= (long)M * N * 4);
     return launch_narrow<T, float, false>(A, lda, W, ldw, nullptr, nullptr, 0, partial, N, M, N, K, stream);
   }

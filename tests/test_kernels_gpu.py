@@ -430,8 +430,8 @@ def test_linear_large_tiles_over_k_ranges(ops, device, m, n, k):
                                    (64, 3584, 2368), (48, 1000, 520)])
 def test_linear_partials(ops, device, dtype, m, n, k):
     """Sums of K ranges left for the next kernel: row-major weights through the kernel with four column tiles a
-    workgroup, shuffled ones through the same (up to 16 rows: identical bits) or, above 16 rows, through the
-    kernel with one workgroup per CU, which names its own number of ranges."""
+    workgroup, shuffled ones through the same (up to 16 rows, at these sizes: identical bits) or, above 16 rows, through
+    the kernel with one workgroup per CU, which names its own number of ranges."""
     x = rand((m, k), dtype, device, 1.0, seed=1)
     w = rand((n, k), dtype, device, 0.05, seed=2)
     want = x.double().cpu() @ w.double().cpu().T
@@ -451,6 +451,59 @@ def test_linear_partials(ops, device, dtype, m, n, k):
     if m <= 16:
         assert ops.linear_partial_splits_rows(w, m) == ops.linear_partial_splits(dtype, n, k)
         torch.testing.assert_close(sums[0], sums[1], atol=0, rtol=0)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("m,n,steps", [(1, 16, 16), (8, 389, 16), (16, 64, 28), (5, 4096, 28), (16, 130, 31), (3, 2048, 31), (8, 48, 32), (8, 48, 15)])
+def test_linear_partials_of_whole_k(ops, device, dtype, m, n, steps):
+    """Up to 16 rows of shuffled weights over 16 to 31 k-steps (K of about 512 to 992 in bfloat16): one sum over the whole of K
+    from the kernel that gives a workgroup all of it, whose rounding is that of GEMM_NARROW's; at 15 and 32 k-steps the kernel
+    with K ranges. Rows of another stride; bounds as for GEMM_NARROW."""
+    k = steps * (16 if dtype == torch.float32 else 32) - (4 if dtype == torch.float32 else 8)      # (K ends inside a k-step)
+    x = rand((m, k + 16), dtype, device, 1.0, seed=1)[:, :k]
+    w = rand((n, k), dtype, device, 0.05, seed=2)
+    want = (x.double() @ w.double().T).cpu()
+    size = (x.double().abs() @ w.double().abs().T).max().item()
+    shuffled = ops.shuffle_weight(w)
+    splits = ops.linear_partial_splits_rows(shuffled, m, x.stride(0))
+    part = torch.full((splits, m, n), float("nan"), device=device)
+    ops.linear_partials(x, shuffled, part)
+    torch.testing.assert_close(part.double().sum(0).cpu(), want, atol=(k / 4 + 4) * 2.0 ** -24 * size + 1e-6, rtol=1e-6)
+    if 16 <= steps < 32:
+        out = torch.empty(m, n, device=device)
+        ops.linear(x, shuffled, out, force=ops.GEMM_NARROW)
+        assert splits == 1 and torch.equal(part[0], out)
+
+
+@pytest.mark.parametrize("m,n,k,narrow", [
+    (16, 256, 3072, True), (8, 256, 4096, True), (16, 256, 4096, False), (16, 1536, 4096, True),
+    (1, 256, 4128, False), (16, 8192, 2048, True), (8, 8192, 2080, False), (8, 8208, 1024, False)])
+@pytest.mark.parametrize("dtype", DTYPES)
+def test_linear_of_few_rows_chooses_by_rows_and_type(ops, device, dtype, m, n, k, narrow):
+    """Which of the two kernels of up to 16 rows a product takes (float32 at half the K): their sums are in different orders,
+    so the bits tell."""
+    k //= 2 if dtype == torch.float32 else 1
+    x, w = rand((m, k), dtype, device, 1.0, seed=1), ops.shuffle_weight(rand((n, k), dtype, device, 0.05, seed=2))
+    workspace = torch.empty(max(4, ops.linear_workspace_bytes(dtype, 64, n, k) // 4), device=device)
+    got = {}
+    for force in (ops.GEMM_AUTO, ops.GEMM_SKINNY, ops.GEMM_NARROW):
+        got[force] = ops.linear(x, w, torch.empty(m, n, device=device), workspace=workspace, force=force)
+    assert not torch.equal(got[ops.GEMM_SKINNY], got[ops.GEMM_NARROW])
+    assert torch.equal(got[ops.GEMM_AUTO], got[ops.GEMM_NARROW if narrow else ops.GEMM_SKINNY])
+
+
+@pytest.mark.parametrize("dtype,m,n,k,narrow", [
+    (torch.bfloat16, 16, 8192, 4096, True), (torch.bfloat16, 8, 9728, 896, True), (torch.bfloat16, 9, 9728, 896, False),
+    (torch.bfloat16, 8, 11264, 2048, True), (torch.bfloat16, 16, 16384, 2048, True), (torch.bfloat16, 8, 16384, 2080, False),
+    (torch.float32, 8, 9728, 512, True), (torch.float32, 1, 9728, 768, False), (torch.float32, 16, 9728, 448, False),
+    (torch.float32, 16, 16384, 1024, True)])
+def test_linear_glu_of_few_rows_chooses_by_rows_and_type(ops, device, dtype, m, n, k, narrow):
+    """The same for gated products (in bfloat16 the rounded results still differ somewhere)."""
+    x, w = rand((m, k), dtype, device, 1.0, seed=1), ops.shuffle_weight(rand((n, k), dtype, device, 0.05, seed=2))
+    got = {force: ops.linear_glu(x, w, torch.empty(m, n // 2, dtype=dtype, device=device), force=force)
+           for force in (ops.GEMM_AUTO, ops.GEMM_SKINNY, ops.GEMM_NARROW)}
+    assert not torch.equal(got[ops.GEMM_SKINNY], got[ops.GEMM_NARROW])
+    assert torch.equal(got[ops.GEMM_AUTO], got[ops.GEMM_NARROW if narrow else ops.GEMM_SKINNY])
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
