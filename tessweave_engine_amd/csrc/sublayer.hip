@@ -204,8 +204,8 @@ extern "C" int tw_relu_squared(int dtype, void* x, long ld, int n, int cols, con
 // y is a sublayer's float32 result (or split-K partial sums that are added up here, in index order); its statistic is
 // float32; the sum goes back into the float32 stream x and, rounded once, to `out` in the compute type, which is what
 // the next sublayer's products read (such an arrangement's sublayers read the stream itself). A block a row, four
-// elements a thread and pass where rows and addresses allow; the row of y stays in registers between the two passes
-// up to 4,096 elements, longer rows are read again.
+// elements a thread and round where rows and addresses allow; the row of y stays in registers between the two passes
+// up to 16,384 elements (4,096 where they do not allow), of longer rows the rest is read again.
 struct AddNormedArgs {
   float* x;
   const float* y; long ldy;
@@ -260,31 +260,76 @@ __global__ __launch_bounds__(1024) void add_normed_vec4_kernel(AddNormedArgs a) 
   }
 }
 
-// Any row (rows that are no multiple of 16 bytes, longer than 16,384 elements): a column a thread and round, the row's
-// values formed twice.
-template <typename T>
-__global__ __launch_bounds__(256) void add_normed_kernel(AddNormedArgs a) {
+// Any row: W columns a thread and round (four where the result's rows allow: longer rows than the above and streams or weights
+// that do not start at 16 bytes), the first KEEP rounds' values in registers between the two passes, the rest formed twice.
+// (With one column a round and every value formed twice, us: 8 rows of 16,388 22.2, with four partial sums 66.8, now 5.5 and 7.8;
+// 2,048 such rows 128 and 363, now 91 and 174; 8 rows of 3,001 6.3 and 14.7, now 3.8 and 4.7.)
+template <typename T, int W>
+__global__ __launch_bounds__(1024) void add_normed_kernel(AddNormedArgs a) {
   __shared__ float lds[16];
-  const int row = blockIdx.x;
+  constexpr int KEEP = 4;
+  const int row = blockIdx.x, units = a.hidden / W;
   float* x = a.x + (size_t)row * a.hidden;
-  auto load = [&](int c) {
-    if (!a.add) return a.y[(size_t)row * a.ldy + c];
-    float v = 0.f;
-    for (int s = 0; s < a.splits; ++s) v += a.add[s * a.add_stride + (size_t)row * a.hidden + c];
-    return v;
+  auto load = [&](int u, float (&v)[W]) {
+    if constexpr (W == 4) {
+      const f32x4 t = a.add ? sub_partial_sums(a.add + (size_t)row * a.hidden + 4 * u, a.splits, a.add_stride)
+                            : *reinterpret_cast<const f32x4*>(a.y + (size_t)row * a.ldy + 4 * u);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] = t[e];
+    } else {
+      v[0] = 0.f;
+      if (!a.add) v[0] = a.y[(size_t)row * a.ldy + u];
+      else
+        for (int s = 0; s < a.splits; ++s) v[0] += a.add[s * a.add_stride + (size_t)row * a.hidden + u];
+    }
   };
-  float ss = 0.f;
-  for (int c = threadIdx.x; c < a.hidden; c += blockDim.x) {
-    const float v = load(c);
-    ss = __fmaf_rn(v, v, ss);
+  float kept[KEEP][W], ss = 0.f;
+#pragma unroll
+  for (int i = 0; i < KEEP; ++i) {
+    const int u = threadIdx.x + i * blockDim.x;
+    if (u < units) {
+      load(u, kept[i]);
+#pragma unroll
+      for (int e = 0; e < W; ++e) ss = __fmaf_rn(kept[i][e], kept[i][e], ss);
+    }
+  }
+  for (int u = threadIdx.x + KEEP * blockDim.x; u < units; u += blockDim.x) {
+    float v[W];
+    load(u, v);
+#pragma unroll
+    for (int e = 0; e < W; ++e) ss = __fmaf_rn(v[e], v[e], ss);
   }
   const float total = tw_block_sum(ss, lds);
   const float f = a.mult / sqrtf(total / (float)a.hidden + a.eps);
   T* out = a.out ? (T*)a.out + (size_t)row * a.hidden : nullptr;
-  for (int c = threadIdx.x; c < a.hidden; c += blockDim.x) {
-    const float r = __fmaf_rn(load(c) * f, a.w[c], x[c]);
-    x[c] = r;
-    if (out) out[c] = tw_from_float<T>(r);
+  const bool whole = W == 4 && (uintptr_t)a.x % 16 == 0 && (uintptr_t)a.w % 16 == 0;
+  auto store = [&](int u, const float (&v)[W]) {
+    if constexpr (W == 4) {
+      if (whole) {
+        const f32x4 wv = *reinterpret_cast<const f32x4*>(a.w + 4 * u), xv = *reinterpret_cast<const f32x4*>(x + 4 * u);
+        f32x4 r;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) r[e] = __fmaf_rn(v[e] * f, wv[e], xv[e]);
+        *reinterpret_cast<f32x4*>(x + 4 * u) = r;
+        if (out) sub_store4(out + 4 * u, r);
+        return;
+      }
+    }
+#pragma unroll
+    for (int e = 0; e < W; ++e) {
+      const int c = u * W + e;
+      const float r = __fmaf_rn(v[e] * f, a.w[c], x[c]);
+      x[c] = r;
+      if (out) out[c] = tw_from_float<T>(r);
+    }
+  };
+#pragma unroll
+  for (int i = 0; i < KEEP; ++i)
+    if ((int)(threadIdx.x + i * blockDim.x) < units) store(threadIdx.x + i * blockDim.x, kept[i]);
+  for (int u = threadIdx.x + KEEP * blockDim.x; u < units; u += blockDim.x) {
+    float v[W];
+    load(u, v);
+    store(u, v);
   }
 }
 
@@ -292,14 +337,21 @@ template <typename T>
 static void add_normed_launch(const AddNormedArgs& a, int n, hipStream_t stream) {
   auto ok = [](const void* p) { return (uintptr_t)p % 16 == 0; };            // (null is)
   const int chunks = a.hidden / 4;
-  if (a.hidden % 4 == 0 && ok(a.x) && ok(a.w) && ok(a.y) && a.ldy % 4 == 0 && ok(a.add) && a.add_stride % 4 == 0 && chunks <= 4096) {
+  const bool whole = ok(a.x) && ok(a.w);
+  // (a result that is one row is read column by column where the stream and the weight have to be, partial sums are not)
+  const bool vec = a.hidden % 4 == 0 && ok(a.y) && a.ldy % 4 == 0 && ok(a.add) && a.add_stride % 4 == 0 && (whole || a.add);
+  if (vec && whole && chunks <= 4096) {
     const int per = chunks <= 1024 ? 1 : chunks <= 2048 ? 2 : 4;
     const int threads = (tw_div_up(chunks, per) + 63) / 64 * 64;
     if (per == 1) add_normed_vec4_kernel<T, 1><<<n, threads, 0, stream>>>(a);
     else if (per == 2) add_normed_vec4_kernel<T, 2><<<n, threads, 0, stream>>>(a);
     else add_normed_vec4_kernel<T, 4><<<n, threads, 0, stream>>>(a);
   } else {
-    add_normed_kernel<T><<<n, 256, 0, stream>>>(a);
+    // (many rows share the chip: a short one's few columns a thread then pay for the block's sums)
+    const int units = vec ? chunks : a.hidden, most = n >= 512 && units <= 2048 ? 256 : 1024;
+    const int threads = units < most ? (units + 63) / 64 * 64 : most;
+    if (vec) add_normed_kernel<T, 4><<<n, threads, 0, stream>>>(a);
+    else add_normed_kernel<T, 1><<<n, threads, 0, stream>>>(a);
   }
 }
 

@@ -358,6 +358,26 @@ def test_row_norms_of_every_length(device, hidden, splits):
             assert ((a.double().cpu() - ref).abs() <= 1e-5 * (1 + ref.abs())).all(), op.__name__
 
 
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("n,hidden,off", [(3, 5001, 0), (3, 20480, 0), (3, 2048, 1), (3, 17000, 3), (600, 1023, 0), (600, 2048, 1),
+                                          (513, 8196, 2)])
+def test_add_normed_of_any_row(device, dtype, n, hidden, off):
+    """Rows longer than a block keeps, of no whole groups of four, many of them, and streams and weights that do not start at
+    16 bytes; one result and five partial sums. Bound as above, and half a bfloat16 step for the rounded copy."""
+    from tessweave_engine_amd.kernels import ops
+    g = torch.Generator(device=device).manual_seed(hidden + off)
+    x, y = torch.randn(n, hidden, generator=g, device=device), torch.randn(n, hidden, generator=g, device=device)
+    w = torch.randn(hidden + off, generator=g, device=device)[off:]
+    parts = torch.randn(5, n, hidden, generator=g, device=device)
+    for given, total in (({"y": y}, y.double()), ({"add": parts}, parts.double().sum(0))):
+        want = x.double() + 0.7 * total / torch.sqrt((total * total).mean(-1, keepdim=True) + 1e-5) * w.double()
+        got = torch.empty(n * hidden + off, device=device)[off:].view(n, hidden).copy_(x)
+        out = torch.full((n, hidden), float("nan"), dtype=getattr(torch, dtype), device=device)
+        ops.add_normed(got, w, 1e-5, 0.7, out=out, **given)
+        assert ((got.double() - want).abs() <= 1e-5 * (1 + want.abs())).all()
+        assert torch.equal(out, got.to(out.dtype))
+
+
 @pytest.mark.parametrize("H,D,E,open_gates", [(2, 128, 128, True), (3, 20, 72, False), (1, 200, 16, True)])
 def test_mlstm_in_segments(device, H, D, E, open_gates):
     """Portions long enough to be cut into segments for separate workgroups (one that ends inside a chunk, one too short to
