@@ -845,7 +845,7 @@ static int delta_piece_rows(int rows, int n_seqs, int H, int E, int Dk) {
 
 // float32 scratch of a launch over n_seqs sequences of up to `rows` rows together (0: it needs none)
 extern "C" long tw_delta_workspace_floats(int rows, int n_seqs, int max_q_len, int H, int E, int Dk) {
-  if (n_seqs <= 0 || rows <= 0 || !delta_in_chunks(rows, n_seqs, max_q_len, H, E, Dk)) return 0;
+  if (n_seqs <= 0 || rows <= 0 || H <= 0 || E <= 0 || Dk <= 0 || !delta_in_chunks(rows, n_seqs, max_q_len, H, E, Dk)) return 0;
   return ((long)delta_piece_rows(rows, n_seqs, H, E, Dk) / TW_DELTA_PREP + n_seqs) * H * delta_unit_floats(E, Dk);
 }
 

@@ -436,7 +436,7 @@ static void ml_segments(int n_seqs, int max_q_len, int H, int Ep, int* len, int*
 
 // float32 scratch that sequences of up to max_q_len tokens in chunks need (0: none)
 extern "C" long tw_mlstm_workspace_floats(int n_seqs, int max_q_len, int H, int Dp, int Ep) {
-  if (n_seqs <= 0 || max_q_len <= 0) return 0;
+  if (n_seqs <= 0 || max_q_len <= 0 || H <= 0 || Dp <= 0 || Ep <= 0) return 0;
   int len, count;
   ml_segments(n_seqs, max_q_len, H, Ep, &len, &count);
   return count > 1 ? (long)n_seqs * H * count * ((long)Ep * Dp + Dp + 4) : 0;

@@ -35,3 +35,14 @@ def test_block_size_is_checked_when_the_engine_configuration_is_made():
     assert EngineConfig(block_size=12).block_size == 12
     with pytest.raises(ValueError, match="multiple of 4"):
         EngineConfig(block_size=6)
+
+
+def test_scratch_sizes_of_nothing_are_zero():
+    """Sizes that a launch refuses need no scratch: asking for it is answered, not ended by a division."""
+    from tessweave_engine_amd.kernels import ops
+    for zero in range(5):
+        sizes = [2, 2048, 16, 128, 128]
+        sizes[zero] = 0
+        assert ops.mlstm_workspace_floats(*sizes) == 0
+        assert ops.delta_workspace_floats(sizes[1], sizes[0], sizes[1], *sizes[2:]) == 0
+    assert ops.mlstm_workspace_floats(2, 2048, 16, 128, 128) > 0 and ops.delta_workspace_floats(2048, 2, 2048, 16, 128, 128) > 0
