@@ -19,28 +19,40 @@ struct ResidualNormArgs {
   float alpha, eps;
 };
 
-// Four columns of split-K partial sums, `stride` apart, requested eight at a time and added in index order.
+// Four columns of split-K partial sums, `stride` apart, requested up to eight at a time and added in index order. (Four, two and
+// one behind the whole eights: eight loads with a condition each cost a row of one partial sum 0.3 to 1.2 us.)
+template <int N>
+__device__ __forceinline__ void sub_add_parts(f32x4& sum, const float* p, size_t stride) {
+  f32x4 part[N];
+#pragma unroll
+  for (int i = 0; i < N; ++i) part[i] = *reinterpret_cast<const f32x4*>(p + (size_t)i * stride);
+#pragma unroll
+  for (int i = 0; i < N; ++i) sum += part[i];
+}
 __device__ __forceinline__ f32x4 sub_partial_sums(const float* p, int splits, size_t stride) {
   f32x4 sum = {0.f, 0.f, 0.f, 0.f};
-  for (int s0 = 0; s0 < splits; s0 += 8) {
-    f32x4 part[8];
-#pragma unroll
-    for (int i = 0; i < 8; ++i)
-      if (s0 + i < splits) part[i] = *reinterpret_cast<const f32x4*>(p + (size_t)(s0 + i) * stride);
-#pragma unroll
-    for (int i = 0; i < 8; ++i)
-      if (s0 + i < splits) sum += part[i];
-  }
+  int s = 0;
+  for (; s + 8 <= splits; s += 8) sub_add_parts<8>(sum, p + (size_t)s * stride, stride);
+  if (splits & 4) { sub_add_parts<4>(sum, p + (size_t)s * stride, stride); s += 4; }
+  if (splits & 2) { sub_add_parts<2>(sum, p + (size_t)s * stride, stride); s += 2; }
+  if (splits & 1) sub_add_parts<1>(sum, p + (size_t)s * stride, stride);
   return sum;
 }
 
-// Four neighbouring values (hidden % 4 == 0, so that they are aligned wherever the tensor's start is).
+// Rows up to which a row's kernel requests its weights with the row (EARLY): with few rows its time is a chain of trips to
+// memory; with more than a CU has at a time, the registers that hold them are rows that are not there. 300 rows, weights with
+// the row / where they are used, us: layer_norm (two norms) of 5,120 11.5 / 8.5, 8,192 14.1 / 10.9; residual_norm of 8,192 8.7 / 7.7;
+// 2,048 rows of 5,120 43.8 / 33.2. (Few rows: residual_norm of 8 rows of 2,048 with four and nine partial sums 3.5 and 3.8 with
+// the row, 3.7 and 4.2 where they are used.)
+#define TW_EARLY_ROWS 256
+
+// Four neighbouring values of a row; `whole`: the tensor starts where four of them are aligned (hidden % 4 == 0: then all are).
 template <typename T>
-__device__ __forceinline__ void sub_store4(T* dst, f32x4 r) {
+__device__ __forceinline__ void sub_store4(T* dst, f32x4 r, bool whole) {
   T packed[4];
 #pragma unroll
   for (int e = 0; e < 4; ++e) packed[e] = tw_from_float<T>(r[e]);
-  if ((uintptr_t)dst % (4 * sizeof(T)) != 0) {
+  if (!whole) {
 #pragma unroll
     for (int e = 0; e < 4; ++e) dst[e] = packed[e];
   } else if constexpr (sizeof(T) == 2) {
@@ -49,31 +61,35 @@ __device__ __forceinline__ void sub_store4(T* dst, f32x4 r) {
     *reinterpret_cast<f32x4*>(dst) = *reinterpret_cast<const f32x4*>(packed);
   }
 }
+template <typename T>
+__device__ __forceinline__ bool sub_whole4(const void* out) { return (uintptr_t)out % (4 * sizeof(T)) == 0; }
 
 // PER groups of four consecutive elements a thread, the row in registers between the two passes.
-template <typename T, int PER>
+template <typename T, int PER, bool EARLY>
 __global__ __launch_bounds__(1024) void residual_norm_vec4_kernel(ResidualNormArgs a) {
   __shared__ float lds[16];
   const int row = blockIdx.x;
   const int chunks = a.hidden / 4;
   float* x = a.x + (size_t)row * a.hidden;
-  // (every load of the row is requested before the first one is waited for)
   f32x4 v[PER], xv[PER], wv[PER], sv[PER];
 #pragma unroll
   for (int i = 0; i < PER; ++i) {
     const int c = min((int)(threadIdx.x + i * blockDim.x), chunks - 1);
-    xv[i] = *reinterpret_cast<const f32x4*>(x + 4 * c);
-    wv[i] = *reinterpret_cast<const f32x4*>(a.w + 4 * c);
-    if (a.scale) sv[i] = *reinterpret_cast<const f32x4*>(a.scale + 4 * c);
+    if (EARLY) xv[i] = *reinterpret_cast<const f32x4*>(x + 4 * c);
+    if (EARLY) wv[i] = *reinterpret_cast<const f32x4*>(a.w + 4 * c);
+    if (EARLY && a.scale) sv[i] = *reinterpret_cast<const f32x4*>(a.scale + 4 * c);
   }
   float ss = 0.f;
 #pragma unroll
   for (int i = 0; i < PER; ++i) {
     const int c = min((int)(threadIdx.x + i * blockDim.x), chunks - 1);
     f32x4 yv = {0.f, 0.f, 0.f, 0.f};
-    if (a.add) yv = sub_partial_sums(a.add + (size_t)row * a.hidden + 4 * c, a.splits, a.add_stride);
+    if (!EARLY) xv[i] = *reinterpret_cast<const f32x4*>(x + 4 * c);
+    if (EARLY && a.add) yv = sub_partial_sums(a.add + (size_t)row * a.hidden + 4 * c, a.splits, a.add_stride);
+    else if (a.add)
+      for (int s = 0; s < a.splits; ++s) yv += *reinterpret_cast<const f32x4*>(a.add + s * a.add_stride + (size_t)row * a.hidden + 4 * c);
     else if (a.y) yv = *reinterpret_cast<const f32x4*>(a.y + (size_t)row * a.ldy + 4 * c);
-    if (a.scale) yv *= sv[i];
+    if (a.scale) yv *= EARLY ? sv[i] : *reinterpret_cast<const f32x4*>(a.scale + 4 * c);
 #pragma unroll
     for (int e = 0; e < 4; ++e) v[i][e] = __fmaf_rn(a.alpha, xv[i][e], yv[e]);
     if (threadIdx.x + i * blockDim.x < chunks) {
@@ -87,11 +103,12 @@ __global__ __launch_bounds__(1024) void residual_norm_vec4_kernel(ResidualNormAr
   for (int i = 0; i < PER; ++i) {
     const int c = threadIdx.x + i * blockDim.x;
     if (c >= chunks) continue;
+    if (!EARLY) wv[i] = *reinterpret_cast<const f32x4*>(a.w + 4 * c);
     f32x4 r;
 #pragma unroll
     for (int e = 0; e < 4; ++e) r[e] = v[i][e] * rinv * wv[i][e];
     *reinterpret_cast<f32x4*>(x + 4 * c) = r;
-    if (a.out) sub_store4((T*)a.out + (size_t)row * a.hidden + 4 * c, r);
+    if (a.out) sub_store4((T*)a.out + (size_t)row * a.hidden + 4 * c, r, sub_whole4<T>(a.out));
   }
 }
 
@@ -135,9 +152,13 @@ static void residual_norm_launch(const ResidualNormArgs& a, int n, hipStream_t s
     const int per = chunks <= 1024 ? 1 : (chunks <= 2048 ? 2 : 4);
     int threads = (chunks + per - 1) / per;
     threads = (threads + 63) / 64 * 64;
-    if (per == 1) residual_norm_vec4_kernel<T, 1><<<n, threads, 0, stream>>>(a);
-    else if (per == 2) residual_norm_vec4_kernel<T, 2><<<n, threads, 0, stream>>>(a);
-    else residual_norm_vec4_kernel<T, 4><<<n, threads, 0, stream>>>(a);
+#define TW_ROWS(PER) \
+  (n <= TW_EARLY_ROWS ? residual_norm_vec4_kernel<T, PER, true><<<n, threads, 0, stream>>>(a) \
+                      : residual_norm_vec4_kernel<T, PER, false><<<n, threads, 0, stream>>>(a))
+    if (per == 1) TW_ROWS(1);
+    else if (per == 2) TW_ROWS(2);
+    else TW_ROWS(4);
+#undef TW_ROWS
   } else {
     residual_norm_kernel<T><<<n, 256, 0, stream>>>(a);
   }
@@ -256,7 +277,7 @@ __global__ __launch_bounds__(1024) void add_normed_vec4_kernel(AddNormedArgs a) 
 #pragma unroll
     for (int e = 0; e < 4; ++e) r[e] = __fmaf_rn(v[i][e] * f, wv[i][e], xv[i][e]);
     *reinterpret_cast<f32x4*>(x + 4 * c) = r;
-    if (a.out) sub_store4((T*)a.out + (size_t)row * a.hidden + 4 * c, r);
+    if (a.out) sub_store4((T*)a.out + (size_t)row * a.hidden + 4 * c, r, sub_whole4<T>(a.out));
   }
 }
 
@@ -311,7 +332,7 @@ __global__ __launch_bounds__(1024) void add_normed_kernel(AddNormedArgs a) {
 #pragma unroll
         for (int e = 0; e < 4; ++e) r[e] = __fmaf_rn(v[e] * f, wv[e], xv[e]);
         *reinterpret_cast<f32x4*>(x + 4 * u) = r;
-        if (out) sub_store4(out + 4 * u, r);
+        if (out) sub_store4(out + 4 * u, r, sub_whole4<T>(a.out));
         return;
       }
     }
@@ -605,23 +626,19 @@ struct LayerNormArgs {
 };
 
 // PER groups of four consecutive elements a thread, the row in registers.
-template <typename T, int PER>
+template <typename T, int PER, bool EARLY>
 __global__ __launch_bounds__(1024) void layer_norm_vec4_kernel(LayerNormArgs a) {
   __shared__ float lds[16];
   const int row = a.rows ? a.rows[blockIdx.x] : blockIdx.x;
   const int chunks = a.hidden / 4;
   float* x = a.x + (size_t)row * a.hidden;
   const bool has_y = a.y || a.add || a.top > 0;
-  // Every load of the row, its weights included, is requested before the first one is waited for (rows longer than 8,192
-  // elements, four groups a thread, read the second norm's weights where they are used: with them a thread runs out of
-  // registers).
-  constexpr bool EARLY = PER <= 2;
   f32x4 xv[PER], yv[PER], w1[PER], b1[PER], w2[PER], b2[PER];
 #pragma unroll
   for (int i = 0; i < PER; ++i) {
     const int c = min((int)(threadIdx.x + i * blockDim.x), chunks - 1);
     xv[i] = *reinterpret_cast<const f32x4*>(x + 4 * c);
-    if (a.w1) {
+    if (EARLY && a.w1) {
       w1[i] = *reinterpret_cast<const f32x4*>(a.w1 + 4 * c);
       b1[i] = *reinterpret_cast<const f32x4*>(a.b1 + 4 * c);
     }
@@ -634,8 +651,12 @@ __global__ __launch_bounds__(1024) void layer_norm_vec4_kernel(LayerNormArgs a) 
   for (int i = 0; i < PER; ++i) {
     const int c = min((int)(threadIdx.x + i * blockDim.x), chunks - 1);
     yv[i] = f32x4{0.f, 0.f, 0.f, 0.f};
-    if (a.add) yv[i] = sub_partial_sums(a.add + (size_t)row * a.hidden + 4 * c, a.splits, a.add_stride);
-    else if (a.y) yv[i] = *reinterpret_cast<const f32x4*>(a.y + (size_t)row * a.ldy + 4 * c);
+    if (EARLY && a.add) yv[i] = sub_partial_sums(a.add + (size_t)row * a.hidden + 4 * c, a.splits, a.add_stride);
+    else if (a.add) {
+      const float* p = a.add + (size_t)row * a.hidden + 4 * c;
+#pragma unroll 8
+      for (int s = 0; s < a.splits; ++s) yv[i] += *reinterpret_cast<const f32x4*>(p + s * a.add_stride);
+    } else if (a.y) yv[i] = *reinterpret_cast<const f32x4*>(a.y + (size_t)row * a.ldy + 4 * c);
 #pragma unroll 4
     for (int r = 0; r < a.top; ++r) {
       const int at = a.pos[(size_t)row * a.top + r];
@@ -666,6 +687,10 @@ __global__ __launch_bounds__(1024) void layer_norm_vec4_kernel(LayerNormArgs a) 
       const int c = threadIdx.x + i * blockDim.x;
       if (c < chunks) {
         if (a.w1) {
+          if (!EARLY) {
+            w1[i] = *reinterpret_cast<const f32x4*>(a.w1 + 4 * c);
+            b1[i] = *reinterpret_cast<const f32x4*>(a.b1 + 4 * c);
+          }
 #pragma unroll
           for (int e = 0; e < 4; ++e) yv[i][e] = __fmaf_rn((yv[i][e] - mean) * rinv, w1[i][e], b1[i][e]);
         }
@@ -689,7 +714,7 @@ __global__ __launch_bounds__(1024) void layer_norm_vec4_kernel(LayerNormArgs a) 
       f32x4 r;
 #pragma unroll
       for (int e = 0; e < 4; ++e) r[e] = __fmaf_rn((xv[i][e] - mean) * rinv, w2[i][e], b2[i][e]);
-      sub_store4(out + 4 * c, r);
+      sub_store4(out + 4 * c, r, sub_whole4<T>(a.out));
     }
   }
 }
@@ -749,9 +774,13 @@ static void layer_norm_launch(const LayerNormArgs& a, int n, hipStream_t stream)
   if (vec && chunks <= 4096) {
     const int per = chunks <= 1024 ? 1 : chunks <= 2048 ? 2 : 4;
     const int threads = (tw_div_up(chunks, per) + 63) / 64 * 64;
-    if (per == 1) layer_norm_vec4_kernel<T, 1><<<n, threads, 0, stream>>>(a);
-    else if (per == 2) layer_norm_vec4_kernel<T, 2><<<n, threads, 0, stream>>>(a);
-    else layer_norm_vec4_kernel<T, 4><<<n, threads, 0, stream>>>(a);
+    // (rows longer than 8,192 elements, four groups a thread, with all their weights run a thread out of registers)
+    const bool early = n <= TW_EARLY_ROWS && per <= 2;
+    if (per == 1 && early) layer_norm_vec4_kernel<T, 1, true><<<n, threads, 0, stream>>>(a);
+    else if (per == 2 && early) layer_norm_vec4_kernel<T, 2, true><<<n, threads, 0, stream>>>(a);
+    else if (per == 1) layer_norm_vec4_kernel<T, 1, false><<<n, threads, 0, stream>>>(a);
+    else if (per == 2) layer_norm_vec4_kernel<T, 2, false><<<n, threads, 0, stream>>>(a);
+    else layer_norm_vec4_kernel<T, 4, false><<<n, threads, 0, stream>>>(a);
   } else {
     layer_norm_kernel<T><<<n, 256, 0, stream>>>(a);
   }

@@ -358,6 +358,32 @@ def test_row_norms_of_every_length(device, hidden, splits):
             assert ((a.double().cpu() - ref).abs() <= 1e-5 * (1 + ref.abs())).all(), op.__name__
 
 
+@pytest.mark.parametrize("n", [256, 257])
+@pytest.mark.parametrize("hidden", [64, 4096, 8192, 12292])
+@pytest.mark.parametrize("splits", [0, 1, 7])
+def test_row_norms_of_many_rows(device, n, hidden, splits):
+    """The last number of rows whose weights are requested with the row and the first behind it, in one, two and four groups a
+    thread; seven partial sums are four, two and one. Bound as above."""
+    from tessweave_engine_amd.kernels import ops
+    g = torch.Generator(device=device).manual_seed(hidden + splits)
+    rand = lambda *shape: torch.randn(*shape, generator=g, device=device)      # noqa: E731
+    x, parts, w, b, scale = rand(n, hidden), rand(max(1, splits), n, hidden), 1 + rand(hidden), rand(hidden), rand(hidden)
+    y = parts.double().sum(0)
+    given = dict(add=parts) if splits else dict(y=parts[0])
+
+    def layer(v, weight, bias):
+        v = v - v.mean(-1, keepdim=True)
+        return v / torch.sqrt((v * v).mean(-1, keepdim=True) + 1e-5) * weight.double() + bias.double()
+    normed = plain.rms_norm(0.5 * x.double() + scale.double() * y, w.double(), 1e-5)
+    stream = x.double() + layer(y, w, b)
+    for op, args, more, want in ((ops.residual_norm, (w, 1e-5), dict(scale=scale, alpha=0.5), (normed, normed)),
+                                 (ops.layer_norm, (1e-5,), dict(post=(w, b), norm=(scale, b)), (stream, layer(stream, scale, b)))):
+        got, out = x.clone(), torch.full((n, hidden), float("nan"), device=device)
+        op(got, *args, out=out, **given, **more)
+        for a, ref in zip((got, out), want):
+            assert ((a.double() - ref).abs() <= 1e-5 * (1 + ref.abs())).all(), op.__name__
+
+
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 @pytest.mark.parametrize("n,hidden,off", [(3, 5001, 0), (3, 20480, 0), (3, 2048, 1), (3, 17000, 3), (600, 1023, 0), (600, 2048, 1),
                                           (513, 8196, 2)])
