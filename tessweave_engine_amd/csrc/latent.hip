@@ -416,6 +416,7 @@ __global__ __launch_bounds__(256) void latent_decode_kernel(LatentDecodeArgs a) 
     const bool edge = t * 16 + 16 > len, more = t + 4 < t_end;
     // S^T for 16 keys: this lane holds key t * 16 + r
     f32x4 S = {0.f, 0.f, 0.f, 0.f};
+    const T* krow = AHEAD ? nullptr : key_row(t, k_page);
 #pragma unroll
     for (int kc = 0; kc < KC_MAX; ++kc)
       if (kc < KC) {
@@ -424,7 +425,7 @@ __global__ __launch_bounds__(256) void latent_decode_kernel(LatentDecodeArgs a) 
           if (K % STEP != 0 && col >= K) kf[kc] = Elem<T>::zero();
           tw_mma16(S, kf[kc], qf[kc]);            // S[j]: key t * 16 + 4 g + j against head r
         } else {
-          const Frag one = col < K ? tw_load_frag(key_row(t, k_page) + col) : Elem<T>::zero();
+          const Frag one = col < K ? tw_load_frag(krow + col) : Elem<T>::zero();
           tw_mma16(S, one, qf[kc]);
         }
       }
