@@ -422,11 +422,14 @@ __global__ __launch_bounds__(256) void mlstm_scan_kernel(MlstmArgs a, MlstmSegme
 
 // Segments of a launch whose longest portion has max_q_len tokens: as many as make one round of workgroups (at a key size
 // of 128 a CU holds two), each at least four chunks long (a segment costs its state written, scanned and read: as much
-// memory traffic as the rows of four chunks at a head size of 128). 16 heads of 128: 128 tokens 49 -> 45 us, two segments.
+// memory traffic as the rows of four chunks at a head size of 128). 16 heads of 128: 128 tokens 49 -> 45 us, two segments. Where
+// there is room for two only, they are worth two launches more from 24 chunks on (16 sequences of 128 tokens, 16 heads of 64
+// 45 us whole, 50 in two; five of 300, 24 heads of 128 124.8 and 125.4; four of 700 269 and 241).
 static void ml_segments(int n_seqs, int max_q_len, int H, int Ep, int* len, int* count) {
   const int chunks = tw_div_up(max_q_len, ML_L);
   const long groups = (long)n_seqs * H * ((Ep + 63) / 64);
   long want = 512 / groups;
+  if (want == 2 && chunks < 24) want = 1;
   if (want > chunks / 4) want = chunks / 4;
   if (want < 1) want = 1;
   const int per = tw_div_up(chunks, want);

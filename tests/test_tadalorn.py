@@ -276,3 +276,12 @@ def test_layer_arrangement_shared_weights_and_soft_cap():
     assert torch.allclose(layers[4], x + mult * plain.rms_norm(y, weights["l4.norm1"], eps))           # no feed-forward
     raw = plain.rms_norm(layers[5], weights["final.norm"], eps) @ weights["head"].T
     assert torch.allclose(logits, 9.0 * torch.tanh(raw / 9.0)) and logits.abs().max() < 9.0
+
+
+def test_mlstm_launches_that_are_cut_into_segments():
+    """Long portions are (they need scratch); portions that fill the chip are not, nor are short ones where there is room for two
+    segments only."""
+    from tessweave_engine_amd.kernels import ops
+    for n, tokens, heads, dim, cut in ((1, 64, 16, 128, False), (1, 128, 16, 128, True), (16, 128, 16, 64, False),
+                                       (5, 300, 24, 128, False), (4, 700, 24, 128, True), (16, 2048, 16, 128, False)):
+        assert (ops.mlstm_workspace_floats(n, tokens, heads, dim, dim) > 0) is cut, (n, tokens, heads, dim)
