@@ -131,6 +131,27 @@ def test_mixed_head_attention_forms(device, dtype, H, G, D, E, window, T, q_len,
     test_mixed_head_attention(device, dtype, H, G, D, E, window, T, q_len, page)
 
 
+def test_mixed_head_attention_does_not_round_the_first_heads_product(device):
+    """Distance slopes make the first head's score the largest; its product with the mixing weight goes into the sum unrounded.
+    Here w0 r0 = 2^20 (1 + 2^-12)^2 and w1 r1 = -2^20 (1 + 2^-11), both factors exact in float32: the sum is 2^-4, and nothing
+    if the first product is rounded by itself. A second key's score is zero."""
+    from tessweave_engine_amd.kernels import ops
+    H, D, E, page = 4, 64, 64, 16
+    w0, r0, r1 = 1 + 2.0 ** -12, 2.0 ** 20 * (1 + 2.0 ** -12), 2.0 ** 20 * (1 + 2.0 ** -11)
+    q, k, v = torch.zeros(1, H, D), torch.zeros(2, H, D), torch.zeros(2, H, E)
+    q[0, :, 0] = 1
+    k[0, 0, 0], k[0, 1, 0] = r0, r1
+    v[0] = 1
+    talk = torch.eye(H)
+    talk[0, 0], talk[0, 1] = w0, -1.0
+    kp, vp, table = paged(k.to(device), v.to(device), page, [0])
+    out = torch.empty(1, H * E, device=device)
+    ops.attn_mixed(q.reshape(1, H * D).to(device), kp, vp, table, torch.tensor([0, 1], dtype=torch.int32, device=device),
+                   torch.tensor([2], dtype=torch.int32, device=device), 0, 1, 1, out, H, H, 1.0, talk=talk.to(device))
+    want = 1 / (1 + math.exp(-2.0 ** -4))
+    assert abs(float(out[0, 0]) - want) < 1e-6, (float(out[0, 0]), want)
+
+
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 @pytest.mark.parametrize("taps,norm,C", [(3, True, 40), (4, False, 40), (1, True, 38), (2, False, 38), (8, True, 38)])
 def test_causal_conv_over_portions_and_reused_slots(device, dtype, taps, norm, C):
