@@ -265,6 +265,9 @@ __global__ __launch_bounds__(WMAX * 64) void attn_mixed_kernel(MixedAttnArgs a) 
               for (int o = 0; o < QB; ++o) kf[o] = tw_load_frag(k_row + min((st0 + o) * 4 + g, chunks - 1) * EPF);
               q_frags(head, st0, qf);
 #pragma unroll
+              for (int o = 0; o < QB; ++o)     // (an infinite key times the zero of a query would be no number)
+                if ((st0 + o) * 4 + g >= chunks) kf[o] = Elem<T>::zero();
+#pragma unroll
               for (int o = 0; o < QB; ++o) tw_mma16(s, kf[o], qf[o]);
             }
           }

@@ -152,6 +152,33 @@ def test_mixed_head_attention_does_not_round_the_first_heads_product(device):
     assert abs(float(out[0, 0]) - want) < 1e-6, (float(out[0, 0]), want)
 
 
+@pytest.mark.parametrize("dtype,D", [("float32", 80), ("bfloat16", 144), ("bfloat16", 80), ("bfloat16", 48)])
+@pytest.mark.parametrize("H,G", [(3, 3), (12, 4), (20, 4)])
+def test_mixed_head_attention_of_an_infinite_score(device, dtype, D, H, G):
+    """A key whose last element is infinite, against queries that are negative there: its score is minus infinity in every head
+    and it weighs nothing. (In bfloat16 the last k-step of these key sizes ends inside itself: what stands in for its missing elements
+    must not meet the infinity. Mixing weights are positive, or infinities of two signs would meet.)"""
+    from tessweave_engine_amd.kernels import ops
+    g = torch.Generator().manual_seed(D + H)
+    dt, T, E, page, bad = tdtype(dtype), 40, 32, 16, 5
+    q, k, v = torch.randn(T, H, D, generator=g), torch.randn(T, G, D, generator=g), torch.randn(T, G, E, generator=g)
+    q[..., -1] = -q[..., -1].abs() - 0.1
+    talk, sink = (0.1 + torch.rand(H, H, generator=g)) / H, torch.randn(H, generator=g)
+    q, k, v = (t.to(dt).float() for t in (q, k, v))
+    k[bad, :, -1] = float("inf")
+    want = plain.mixed_head_attention(q.double(), k.double(), v.double(), 0.3 / math.sqrt(D), 10 ** 9, talk.double(),
+                                      sink.double()).reshape(T, H * E)[bad + 1:]
+    assert torch.isfinite(want).all()
+    kp, vp, table = paged(k.to(dt).to(device), v.to(dt).to(device), page, [2, 0, 1])
+    out = torch.empty(T, H * E, dtype=dt, device=device)
+    slopes = torch.tensor(plain.distance_slopes(H).tolist(), dtype=torch.float32, device=device)
+    ops.attn_mixed(q.reshape(T, H * D).to(dt).to(device), kp, vp, table, torch.tensor([0, T], dtype=torch.int32, device=device),
+                   torch.tensor([T], dtype=torch.int32, device=device), 0, 1, T, out, H, G, 0.3 / math.sqrt(D),
+                   talk=talk.to(device), sink=sink.to(device), slopes=slopes)
+    err = row_error(out[bad + 1:].float().cpu().numpy(), want.numpy()).max()
+    assert err < (1e-5 if dtype == "float32" else 2e-2), err
+
+
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 @pytest.mark.parametrize("taps,norm,C", [(3, True, 40), (4, False, 40), (1, True, 38), (2, False, 38), (8, True, 38)])
 def test_causal_conv_over_portions_and_reused_slots(device, dtype, taps, norm, C):
