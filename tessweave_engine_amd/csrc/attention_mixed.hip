@@ -175,19 +175,38 @@ __global__ __launch_bounds__(WMAX * 64) void attn_mixed_kernel(MixedAttnArgs a) 
   typedef const __attribute__((address_space(3))) Frag* LdsFrag;
   // k-steps whose fragments are requested together where they are used (one where registers are short)
   constexpr int QB = (AHEAD || WMAX <= 12) && !(HPW == 2 && VT == 16) ? 4 : 1;
-  auto q_frags = [&](int head, int st0, Frag (&f)[QB]) {          // k-steps st0 ...; zeros past the last chunk
+  const bool ragged = !EXACT && chunks % 4 != 0;           // the last k-step ends inside itself
+  auto past_zero = [&](int st0, auto& f) {                 // (zeros past the last chunk, in both operands: an infinite key
+    if (ragged) {                                          // times the zero of a query would be no number)
+#pragma unroll
+      for (int o = 0; o < (int)(sizeof(f) / sizeof(Frag)); ++o)
+        if ((st0 + o) * 4 + g >= chunks) f[o] = Elem<T>::zero();
+    }
+  };
+  auto q_frags = [&](int head, int st0, auto& f) {         // k-steps st0, st0 + 1, ..., as many as f holds
+    constexpr int N = sizeof(f) / sizeof(Frag);
     if (a.q_in_lds) {
 #pragma unroll
-      for (int o = 0; o < QB; ++o)
+      for (int o = 0; o < N; ++o)
         f[o] = *(LdsFrag)(lds_q + ((size_t)head * 16 + r) * qrow + min((st0 + o) * 4 + g, chunks - 1) * EPF);
     } else {
 #pragma unroll
-      for (int o = 0; o < QB; ++o)
+      for (int o = 0; o < N; ++o)
         f[o] = tw_load_frag(q_global + (size_t)head * D + min((st0 + o) * 4 + g, chunks - 1) * EPF);
     }
-#pragma unroll
-    for (int o = 0; o < QB; ++o)
-      if ((st0 + o) * 4 + g >= chunks) f[o] = Elem<T>::zero();
+    past_zero(st0, f);
+  };
+  // body(number of k-steps, the first of them) over all k-steps, QB at a time and the rest at once (products for k-steps
+  // that are not there: 32 sequences of 1,500, 5 heads of 32, one token each 35.4 -> 44.3 us, now 35.4)
+  auto over_steps = [&](auto&& body) {
+    int st0 = 0;
+    for (; st0 + QB <= steps; st0 += QB) body(std::integral_constant<int, QB>{}, st0);
+    if constexpr (QB > 1) {
+      const int rest = steps - st0;
+      if (rest == 1) body(std::integral_constant<int, 1>{}, st0);
+      else if (rest == 2) body(std::integral_constant<int, 2>{}, st0);
+      else if (rest == 3) body(std::integral_constant<int, 3>{}, st0);
+    }
   };
   int kv_head[KVN];                                        // (SHARE: the wave's first head stands for all)
 #pragma unroll
@@ -249,27 +268,37 @@ __global__ __launch_bounds__(WMAX * 64) void attn_mixed_kernel(MixedAttnArgs a) 
         if (head < H) {
           f32x4 s = {0.f, 0.f, 0.f, 0.f};
           if (AHEAD && ahead) {
+            if constexpr (Q_REGS) {
 #pragma unroll
-            for (int st0 = 0; st0 < KP; st0 += QB) {
-              Frag qf[QB];
-              if constexpr (!Q_REGS) q_frags(head, st0, qf);
+              for (int st = 0; st < KP; ++st) tw_mma16(s, kpre[SHARE ? 0 : i][st], q_own[i][st % 4]);
+            } else if constexpr (QB == KP) {
+              over_steps([&](auto count, int st0) {        // (all k-steps are one group: st0 is 0)
+                Frag qf[decltype(count)::value];
+                q_frags(head, st0, qf);
 #pragma unroll
-              for (int o = 0; o < QB; ++o)
-                tw_mma16(s, kpre[SHARE ? 0 : i][(st0 + o) % KP], Q_REGS ? q_own[i][(st0 + o) % 4] : qf[o]);
+                for (int o = 0; o < decltype(count)::value; ++o) tw_mma16(s, kpre[SHARE ? 0 : i][o], qf[o]);
+              });
+            } else {
+#pragma unroll
+              for (int st = 0; st < KP; ++st)
+                if (st < steps) {
+                  Frag qf[1];
+                  q_frags(head, st, qf);
+                  tw_mma16(s, kpre[SHARE ? 0 : i][st], qf[0]);
+                }
             }
           } else {
             const T* k_row = keys + (((size_t)(page < 0 ? 0 : page) * a.G + kv_head[SHARE ? 0 : i]) * P + in_page(p)) * D;
-            for (int st0 = 0; st0 < steps; st0 += QB) {
-              Frag kf[QB], qf[QB];
+            over_steps([&](auto count, int st0) {
+              constexpr int N = decltype(count)::value;
+              Frag kf[N], qf[N];
 #pragma unroll
-              for (int o = 0; o < QB; ++o) kf[o] = tw_load_frag(k_row + min((st0 + o) * 4 + g, chunks - 1) * EPF);
+              for (int o = 0; o < N; ++o) kf[o] = tw_load_frag(k_row + min((st0 + o) * 4 + g, chunks - 1) * EPF);
               q_frags(head, st0, qf);
+              past_zero(st0, kf);
 #pragma unroll
-              for (int o = 0; o < QB; ++o)     // (an infinite key times the zero of a query would be no number)
-                if ((st0 + o) * 4 + g >= chunks) kf[o] = Elem<T>::zero();
-#pragma unroll
-              for (int o = 0; o < QB; ++o) tw_mma16(s, kf[o], qf[o]);
-            }
+              for (int o = 0; o < N; ++o) tw_mma16(s, kf[o], qf[o]);
+            });
           }
 #pragma unroll
           for (int e = 0; e < 4; ++e) s[e] = s[e] * a.scale - slope[i] * (float)(t_row - (p0 + 4 * g + e));
@@ -310,7 +339,8 @@ __global__ __launch_bounds__(WMAX * 64) void attn_mixed_kernel(MixedAttnArgs a) 
     }
     const f32x4* raw_lane = lds_s + (size_t)buf * H * 64 + lane;
     int other = 0;
-#pragma unroll 2
+    // (two rounds at a time where two heads share them and registers are left: 5 % slower otherwise at 16 heads with values of 256)
+#pragma unroll(HPW == 1 || VT == 16 ? 1 : 2)
     for (; other + 4 <= H; other += 4) {                   // four heads' reads in flight at a time
       f32x4 raw[4];
 #pragma unroll
@@ -324,6 +354,7 @@ __global__ __launch_bounds__(WMAX * 64) void attn_mixed_kernel(MixedAttnArgs a) 
         }
       }
     }
+#pragma unroll 1
     for (; other < H; ++other) {
       const f32x4 raw = raw_lane[other * 64];
 #pragma unroll
