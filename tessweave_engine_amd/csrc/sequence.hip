@@ -97,7 +97,10 @@ __device__ __forceinline__ void conv_store4(bf16_t* p, f32x4 v) {
 
 // VEC: four consecutive channels a thread, 16-byte (8-byte for bfloat16) accesses; the launcher asks for it when
 // the channel count, the row strides and the pointers allow; a row's squares are then summed four such loads at a time
-// (one channel a load, each waited for: 8 rows of 2,048 with 3 taps behind a norm 6.9 us, now 5.2).
+// (one channel a load, each waited for: 8 rows of 2,048 with 3 taps behind a norm 6.9 us, now 5.2), all rows' at once where a
+// thread has one such load a row (300 rows of 64 channels with 7 taps: row by row 9.1 us, so 7.5), and one channel at a time
+// beyond four rows (2,050 channels, 7 taps: 300 rows 18.4 and 17.8; with 3 taps row by row is ahead, 11.4 and 12.1, and where
+// the other taps' rows are in the state, 7.3 and 9.4).
 // FOUR: four taps, a channel's being one 16-byte read: what a thread's channels need (rows, state, weights, taps) is
 // requested before the rows' squares are summed (the same rows: 7.8 -> 4.0 us, without a norm 4.5 -> 3.2; other numbers of taps read one
 // by one with the rows were no faster, and at 300 rows slower, than where they are used).
@@ -151,32 +154,69 @@ __global__ __launch_bounds__(256) void causal_conv_kernel(ConvArgs a) {
   } else if (NORM) {
     // every block sums whole rows, whatever share of the channels it then writes
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int n_src = min(K, row - first + 1);      // rows of this step among the taps'
+    if (VEC ? n_src == 1 || C > (int)blockDim.x * 4 : n_src <= 4) {
 #pragma unroll 1
-    for (int j = 0; j < K; ++j) {
-      const int p = pos - (K - 1) + j;
-      float sum = 0.f;
-      if (p >= start) {
-        const SrcT* from = src + (size_t)(first + p - start) * a.ld_src;
-        if constexpr (VEC) {
-          for (int c0 = threadIdx.x * 4; c0 < C; c0 += blockDim.x * 16) {
-            f32x4 v[4];
+      for (int j = 0; j < K; ++j) {
+        const int p = pos - (K - 1) + j;
+        float sum = 0.f;
+        if (p >= start) {
+          const SrcT* from = src + (size_t)(first + p - start) * a.ld_src;
+          if constexpr (VEC) {
+            for (int c0 = threadIdx.x * 4; c0 < C; c0 += blockDim.x * 16) {
+              f32x4 v[4];
 #pragma unroll
-            for (int u = 0; u < 4; ++u) v[u] = conv_load4(from + min(c0 + u * (int)blockDim.x * 4, C - 4));
+              for (int u = 0; u < 4; ++u) v[u] = conv_load4(from + min(c0 + u * (int)blockDim.x * 4, C - 4));
 #pragma unroll
-            for (int u = 0; u < 4; ++u) {
-              const float t = v[u][0] * v[u][0] + v[u][1] * v[u][1] + v[u][2] * v[u][2] + v[u][3] * v[u][3];
-              sum += c0 + u * (int)blockDim.x * 4 < C ? t : 0.f;
+              for (int u = 0; u < 4; ++u) {
+                const float t = v[u][0] * v[u][0] + v[u][1] * v[u][1] + v[u][2] * v[u][2] + v[u][3] * v[u][3];
+                sum += c0 + u * (int)blockDim.x * 4 < C ? t : 0.f;
+              }
             }
-          }
-        } else {
-          for (int c = threadIdx.x; c < C; c += blockDim.x) {
-            const float v = tw_to_float(from[c]);
-            sum += v * v;
+          } else {
+            for (int c = threadIdx.x; c < C; c += blockDim.x) {
+              const float v = tw_to_float(from[c]);
+              sum += v * v;
+            }
           }
         }
         sum = tw_wave_sum(sum);
+        if (lane == 0) red[j][wave] = sum;
       }
-      if (lane == 0) red[j][wave] = sum;
+    } else {
+      // several rows of few channels, or many one channel at a time: all rows' loads of a round are requested together
+      float sums[TW_CONV_MAX_TAPS];
+#pragma unroll
+      for (int j = 0; j < TW_CONV_MAX_TAPS; ++j) sums[j] = 0.f;
+      if constexpr (VEC) {
+        const int c = threadIdx.x * 4;
+        if (c < C) {
+          f32x4 v[TW_CONV_MAX_TAPS];
+#pragma unroll
+          for (int j = 0; j < TW_CONV_MAX_TAPS; ++j) {
+            v[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+            if (from_src[j]) v[j] = conv_load4(from_src[j] + c);
+          }
+#pragma unroll
+          for (int j = 0; j < TW_CONV_MAX_TAPS; ++j) sums[j] = v[j][0] * v[j][0] + v[j][1] * v[j][1] + v[j][2] * v[j][2] + v[j][3] * v[j][3];
+        }
+      } else {
+        for (int c = threadIdx.x; c < C; c += blockDim.x) {
+#pragma unroll
+          for (int j = 0; j < TW_CONV_MAX_TAPS; ++j)
+            if (from_src[j]) {
+              const float v = tw_to_float(from_src[j][c]);
+              sums[j] += v * v;
+            }
+        }
+      }
+#pragma unroll
+      for (int j = 0; j < TW_CONV_MAX_TAPS; ++j) {
+        if (j < K) {
+          const float t = from_src[j] ? tw_wave_sum(sums[j]) : 0.f;
+          if (lane == 0) red[j][wave] = t;
+        }
+      }
     }
     __syncthreads();
     if (threadIdx.x < K) {
