@@ -56,10 +56,10 @@ __device__ __forceinline__ void tw_tiled_epilogue(f32x16 (&acc)[WM][WN], char* l
   float* bias_stage = reinterpret_cast<float*>(lds) + 4 * 32 * EROW + wave * WCOLS;
   auto swz = [](int row) { return SWIZZLED ? ((row & 1) | ((row & 2) << 1)) : 0; };
 
-  // A residual that is added to a whole tile: all of a row block's values of it are requested in front of the copy into LDS
+  // A residual that is added to whole rows: all of a row block's values of it are requested in front of the copy into LDS
   // (in the loop every round would wait for its own: C may be the residual, so no load passes a store).
   constexpr int ROUNDS = 32 * CPR / 64;
-  const bool ahead = !GLU && residual != nullptr && vec_ok && m0 + 64 * WM <= M && n0 + 64 * WN <= N;
+  auto whole = [&](int i) { return vec_ok && m0 + wm0 + i * 32 + 32 <= M && n0 + wn0 + WCOLS <= N; };   // (row block i of the wave)
   f32x4 res[GLU ? 1 : ROUNDS][2];
   auto request = [&](int i) {
 #pragma unroll
@@ -96,8 +96,41 @@ __device__ __forceinline__ void tw_tiled_epilogue(f32x16 (&acc)[WM][WN], char* l
       }
     }
   };
-  // rows i * 32 .. + 31 of any other plain product
+  // The same without a residual or an activation, for 128x128 tiles: their four rounds fit the instruction cache side by side (as a
+  // loop each round waits for its own reads of LDS: 1,024 x 4,096 x 896 in bfloat16 15.3 us, so 13.7; with the activations in it,
+  // too, the kernel takes so many registers that a CU holds one workgroup instead of two: 20 % slower).
+  constexpr bool SMALL = !GLU && WM * WN <= 4;
   const long act = residual == nullptr ? ldr : 0;             // (no residual: the stride names an activation, see tw_act)
+  auto finish_at_once = [&](int i) {
+    float v[ROUNDS][8];
+#pragma unroll
+    for (int t = 0; t < ROUNDS; ++t) {
+      const int q = lane + 64 * t;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v[t][e] = stage[(q / CPR) * EROW + (q % CPR) * 8 + e];
+    }
+    if (bias) {
+#pragma unroll
+      for (int t = 0; t < ROUNDS; ++t)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[t][e] += bias_stage[((lane + 64 * t) % CPR) * 8 + e];
+    }
+#pragma unroll
+    for (int t = 0; t < ROUNDS; ++t) {
+      const int q = lane + 64 * t;
+      OutT* dst = C + (size_t)(m0 + wm0 + i * 32 + q / CPR) * ldc + n0 + wn0 + (q % CPR) * 8;
+      if (sizeof(OutT) == 4) {
+        *reinterpret_cast<f32x4*>(dst) = f32x4{v[t][0], v[t][1], v[t][2], v[t][3]};
+        *reinterpret_cast<f32x4*>(dst + 4) = f32x4{v[t][4], v[t][5], v[t][6], v[t][7]};
+      } else {
+        bf16x8 o;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) o[e] = (bf16_t)v[t][e];
+        *reinterpret_cast<bf16x8*>(dst) = o;
+      }
+    }
+  };
+  // rows i * 32 .. + 31 of any other plain product
   auto finish = [&](int i) {
 #pragma unroll 1
     for (int q = lane; q < 32 * CPR; q += 64) {
@@ -204,7 +237,7 @@ __device__ __forceinline__ void tw_tiled_epilogue(f32x16 (&acc)[WM][WN], char* l
 #pragma unroll
   for (int i = 0; i < WM; ++i) {
     if constexpr (!GLU) {
-      if (ahead) request(i);
+      if (residual != nullptr && whole(i)) request(i);
     }
     tw_wave_lds_fence();                                      // (the last round's reads come first)
 #pragma unroll
@@ -218,7 +251,8 @@ __device__ __forceinline__ void tw_tiled_epilogue(f32x16 (&acc)[WM][WN], char* l
     if constexpr (GLU) {
       finish_glu(i);
     } else {
-      if (ahead) finish_ahead(i);
+      if (residual != nullptr && whole(i)) finish_ahead(i);
+      else if (SMALL && residual == nullptr && act == 0 && whole(i)) finish_at_once(i);
       else finish(i);
     }
   }
@@ -788,8 +822,11 @@ static int launch_dma(const bf16_t* A, long lda, const bf16_t* W, long ldw, cons
 // measured on the projections of 7B-class models from 256 to 16,384 rows. Larger tiles move fewer
 // bytes per MFMA through the 64 B/clk vector-memory path and LDS; smaller ones waste less in the
 // last round.
+// (with the present epilogue, 8,192 x 37,888 x 3,584 in bfloat16, TFLOP/s plain / gated: 128x128 906 / 891, 128x256
+// 1,027 / 1,037, 256x256 1,195 / 1,179, 256x192 1,146 / 1,121)
 #ifndef TW_DMA_SHAPES
-#define TW_DMA_SHAPES 0xC      /* bit s: shape s uses the direct-to-LDS kernel (at 128x128 it gains nothing) */
+#define TW_DMA_SHAPES 0xC      /* bit s: shape s uses the direct-to-LDS kernel (at 128x128, 1 to 10 % ahead with the present */
+                               /* epilogue and nothing with the one before it, it has not been fitted into the rule above) */
 #endif
 static const int kTileM[5] = {0, 128, 128, 256, 256}, kTileN[5] = {0, 128, 256, 256, 192};
 static const double kTileRate[5] = {0, 0.76, 0.90, 1.05, 1.00};
