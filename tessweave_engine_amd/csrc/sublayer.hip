@@ -39,6 +39,20 @@ __device__ __forceinline__ f32x4 sub_partial_sums(const float* p, int splits, si
   return sum;
 }
 
+// tw_block_sum with the waves' sums added in pairs: one after the other the sixteen of a long row are off by more than the four
+// of a smaller workgroup (3,001 squares: 1.14 times the error in the normed row).
+__device__ __forceinline__ float sub_block_sum(float v, float* lds /* 16 floats at 16 bytes */) {
+  v = tw_wave_sum(v);
+  const int wave = threadIdx.x / TW_WAVE, waves = blockDim.x / TW_WAVE;
+  __syncthreads();
+  if (threadIdx.x % TW_WAVE == 0) lds[wave] = v;
+  if (threadIdx.x < 16 && threadIdx.x >= waves) lds[threadIdx.x] = 0.f;
+  __syncthreads();
+  const f32x4* four = reinterpret_cast<const f32x4*>(lds);
+  const f32x4 t = (four[0] + four[1]) + (four[2] + four[3]);
+  return (t[0] + t[1]) + (t[2] + t[3]);
+}
+
 // Rows up to which a row's kernel requests its weights with the row (EARLY): with few rows its time is a chain of trips to
 // memory; with more than a CU has at a time, the registers that hold them are rows that are not there. 300 rows, weights with
 // the row / where they are used, us: layer_norm (two norms) of 5,120 11.5 / 8.5, 8,192 14.1 / 10.9; residual_norm of 8,192 8.7 / 7.7;
@@ -245,7 +259,7 @@ struct AddNormedArgs {
 // (in a decode step's graph 10.6 -> 4.2), 2,048 rows 23.6 -> 17.6, without partial sums 16.1 -> 10.5.)
 template <typename T, int PER>
 __global__ __launch_bounds__(1024) void add_normed_vec4_kernel(AddNormedArgs a) {
-  __shared__ float lds[16];
+  __shared__ __attribute__((aligned(16))) float lds[16];
   const int row = blockIdx.x;
   const int chunks = a.hidden / 4;
   float* x = a.x + (size_t)row * a.hidden;
@@ -267,7 +281,7 @@ __global__ __launch_bounds__(1024) void add_normed_vec4_kernel(AddNormedArgs a) 
       for (int e = 0; e < 4; ++e) ss = __fmaf_rn(v[i][e], v[i][e], ss);
     }
   }
-  const float total = tw_block_sum(ss, lds);
+  const float total = sub_block_sum(ss, lds);
   const float f = a.mult / sqrtf(total / (float)a.hidden + a.eps);
 #pragma unroll
   for (int i = 0; i < PER; ++i) {
@@ -287,7 +301,7 @@ __global__ __launch_bounds__(1024) void add_normed_vec4_kernel(AddNormedArgs a) 
 // 2,048 such rows 128 and 363, now 91 and 174; 8 rows of 3,001 6.3 and 14.7, now 3.8 and 4.7.)
 template <typename T, int W>
 __global__ __launch_bounds__(1024) void add_normed_kernel(AddNormedArgs a) {
-  __shared__ float lds[16];
+  __shared__ __attribute__((aligned(16))) float lds[16];
   constexpr int KEEP = 4;
   const int row = blockIdx.x, units = a.hidden / W;
   float* x = a.x + (size_t)row * a.hidden;
@@ -320,7 +334,7 @@ __global__ __launch_bounds__(1024) void add_normed_kernel(AddNormedArgs a) {
 #pragma unroll
     for (int e = 0; e < W; ++e) ss = __fmaf_rn(v[e], v[e], ss);
   }
-  const float total = tw_block_sum(ss, lds);
+  const float total = sub_block_sum(ss, lds);
   const float f = a.mult / sqrtf(total / (float)a.hidden + a.eps);
   T* out = a.out ? (T*)a.out + (size_t)row * a.hidden : nullptr;
   const bool whole = W == 4 && (uintptr_t)a.x % 16 == 0 && (uintptr_t)a.w % 16 == 0;
