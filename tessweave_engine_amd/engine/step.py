@@ -22,6 +22,7 @@ from __future__ import annotations
 from collections import OrderedDict
 import ctypes
 from dataclasses import dataclass, field
+import threading
 
 import numpy as np
 import torch
@@ -71,6 +72,18 @@ class _Graph:
                 lib.tw_graph_destroy(handle)
 
 
+_capturing = threading.local()           # .now: this thread is capturing a step
+_let_go_late = []                        # (buffers, readers) of stagings that were collected on a capturing thread
+
+
+def _wait_for_late():
+    while _let_go_late:
+        _, readers = _let_go_late.pop()
+        for event in readers:
+            if event is not None:
+                event.synchronize()
+
+
 class _Staging:
     """Pinned buffers in which steps' metadata waits for the device, taken in turn.
 
@@ -98,7 +111,10 @@ class _Staging:
 
     def __del__(self):
         try:
-            self.wait()
+            if getattr(_capturing, "now", False):
+                _let_go_late.append((self.buffers, self.readers))    # (a wait would end another stepper's capture)
+            else:
+                self.wait()
         except Exception:       # noqa: BLE001  (half made, or the interpreter is going down)
             pass
 
@@ -439,21 +455,26 @@ class Stepper:
                 check(end_segment(), "graph capture end")
                 check(lib.tw_graph_begin(stream), "graph capture begin")
 
-        with torch.cuda.stream(self.stream):
-            check(lib.tw_graph_begin(stream), "graph capture begin")
-            ctx.segment_end = segment_end
-            self.workspace.touched = touched = set()
-            try:
-                logits = self.model.forward(ctx)
-            except BaseException:
-                end_segment()
-                for handle in handles:
-                    lib.tw_graph_destroy(handle)
-                raise
-            finally:
-                ctx.segment_end = None
-                self.workspace.touched = None
-            check(end_segment(), "graph capture end")
+        _capturing.now = True
+        try:
+            with torch.cuda.stream(self.stream):
+                check(lib.tw_graph_begin(stream), "graph capture begin")
+                ctx.segment_end = segment_end
+                self.workspace.touched = touched = set()
+                try:
+                    logits = self.model.forward(ctx)
+                except BaseException:
+                    end_segment()
+                    for handle in handles:
+                        lib.tw_graph_destroy(handle)
+                    raise
+                finally:
+                    ctx.segment_end = None
+                    self.workspace.touched = None
+                check(end_segment(), "graph capture end")
+        finally:
+            _capturing.now = False
+            _wait_for_late()
         if self.workspace.generation != generation:
             for handle in handles:
                 lib.tw_graph_destroy(handle)

@@ -682,3 +682,33 @@ def test_staging_memory_outlives_its_readers():
     done.clear()
     del stepper, staging
     assert len(done) == 2
+
+
+def test_staging_collected_during_a_capture_waits_behind_it(monkeypatch):
+    """A dropped stepper can be collected while another one's step is being captured on the same thread, where a wait for an event
+    ends the capture: its staging is waited for, and its memory kept, until the capture is over."""
+    import gc
+    from contextlib import nullcontext
+    from types import SimpleNamespace
+    from tessweave_engine_amd.engine import step as module
+
+    log, staging = [], module._Staging.__new__(module._Staging)
+    staging.buffers, staging.next = ["memory"], 0
+    staging.readers = [SimpleNamespace(synchronize=lambda: log.append("waited"))]
+    staging.itself = staging                                     # (only the collector lets it go)
+    staging = [staging]
+
+    def forward(ctx):
+        staging.clear()
+        gc.collect()
+        log.append(module._let_go_late[0][0][0])
+
+    lib = SimpleNamespace(tw_graph_begin=lambda stream: 0, tw_graph_end=lambda stream, handle: log.append("ended") or 0)
+    monkeypatch.setattr(module, "library", lambda: lib)
+    monkeypatch.setattr(module.torch.cuda, "stream", lambda stream: nullcontext())
+    stepper = module.Stepper.__new__(module.Stepper)
+    stepper._graphs, stepper.stream = {}, SimpleNamespace(cuda_stream=0)
+    stepper.workspace = SimpleNamespace(generation=0, touched=None, versions={})
+    stepper.model = SimpleNamespace(schedule=[], forward=forward)
+    stepper._capture(SimpleNamespace(segment_end=None), False)
+    assert log == ["memory", "ended", "waited"] and not module._let_go_late
