@@ -379,7 +379,8 @@ __global__ __launch_bounds__(256) void latent_decode_kernel(LatentDecodeArgs a) 
   // one before) and, in bfloat16, the next tile's while this one is worked on: its keys behind the scores, its values behind the
   // products that free their registers, its page numbers a tile earlier still (float32 fragments are twice as many registers:
   // ahead they would halve the waves). 8 requests of 150
-  // tokens 17.7 -> 12.3 us, one of 2,048 22.6 -> 12.7 (kernel traces, where one that does nothing takes 4). A key past the end stands in for by the last one; masked below.
+  // tokens 17.7 -> 12.3 us, one of 2,048 22.6 -> 12.7 (kernel traces).
+  // A key past the end is the last one again; masked below.
   constexpr bool AHEAD = EPF == 8;
   auto key_of = [&](int t) { return min(t * 16 + r, len - 1); };
   auto value_of = [&](int t) { return min(t * 16 + 4 * g, (len - 1) / 4 * 4); };      // 4 keys: one page (multiples of 4)
