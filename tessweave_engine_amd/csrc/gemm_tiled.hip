@@ -1,6 +1,7 @@
 // Linear layers for many rows (prompt portions): LDS-staged MFMA tiles. See gemm.hip for the
 // weight layouts and the GLU form; this file holds the kernel, its epilogue and its launcher.
 #include "gemm_shared.h"
+#include <math.h>
 
 // f(integral_constant<int, 0>), ..., f(integral_constant<int, N - 1>): a loop whose index is a constant
 // expression in the body (the scheduler's group barriers take constants only)
@@ -23,7 +24,7 @@ __device__ __forceinline__ void tw_wave_lds_fence() {
 // Epilogue of the tiled kernels: each wave passes its tile through LDS (32 rows at a time) so
 // that a lane stores 8 consecutive columns of one row, whole cache lines instead of 2- or 4-byte
 // pieces; bias, residual, the output type and the SiLU-multiply of GLU pairs are applied here.
-// `lds` must hold 4 waves x (32 rows x (32 * WN + 4) + 32 * WN) floats and no wave may still read its old contents
+// `lds` must hold WAVES x (32 rows x (32 * WN + 4) + 32 * WN) floats and no wave may still read its old contents
 // (the __syncthreads below sees to that; afterwards every wave works in its own part).
 //
 // What bounds it is the instruction cache (64 KB, shared by two CUs). Unrolled over the row blocks, the rounds and the
@@ -32,7 +33,7 @@ __device__ __forceinline__ void tw_wave_lds_fence() {
 // (the copy of the accumulators into LDS must name its registers), a round is a loop of a few hundred instructions, and the
 // activation is asked for once a round. 256x256 tiles, K = 3,584, bfloat16: the gated projection of 2,048 rows x 37,888
 // columns 653 -> 491 us, of 8,192 rows 2,479 -> 1,832 us (898 -> 1,215 TFLOP/s); plain products 2 to 5 %.
-template <typename OutT, int WM, int WN, bool GLU>
+template <typename OutT, int WM, int WN, bool GLU, int WAVES = 4>
 __device__ __forceinline__ void tw_tiled_epilogue(f32x16 (&acc)[WM][WN], char* lds, const float* __restrict__ bias,
                                                   const float* residual, long ldr, OutT* C, long ldc, int M, int N,
                                                   int m0, int n0, int wm0, int wn0, int wave, int lane) {
@@ -53,7 +54,7 @@ __device__ __forceinline__ void tw_tiled_epilogue(f32x16 (&acc)[WM][WN], char* l
   float* stage = reinterpret_cast<float*>(lds) + wave * 32 * SROW;
   // A plain product's bias: the wave's columns of it go to LDS once, behind all waves' rows (read from memory in front of
   // every store it cost a fifth of a qkv projection's time at 2,048 rows; in registers a lane needs up to three groups of it).
-  float* bias_stage = reinterpret_cast<float*>(lds) + 4 * 32 * EROW + wave * WCOLS;
+  float* bias_stage = reinterpret_cast<float*>(lds) + WAVES * 32 * EROW + wave * WCOLS;
   auto swz = [](int row) { return SWIZZLED ? ((row & 1) | ((row & 2) << 1)) : 0; };
 
   // A residual that is added to whole rows: all of a row block's values of it are requested in front of the copy into LDS
@@ -485,7 +486,8 @@ __global__ __launch_bounds__(256) void gemm_tiled_kernel(const T* __restrict__ A
 }
 
 // =====================================================================================
-// bfloat16, shuffled weights, K a multiple of 32: tiles whose operands are copied from global
+// bfloat16, shuffled weights, K an odd multiple of 32 (or rows of the result that are no multiple of 16 bytes: all else goes
+// to gemm_turns_kernel below): tiles whose operands are copied from global
 // memory straight into LDS (`global_load_lds_dwordx4`: lane l's 16 bytes land at the wave's LDS
 // base + 16 l, from any address the lane names). No staging registers, no LDS write instructions.
 // Workgroup = 4 waves in a 2x2 grid, wave tile (32*WM) x (32*WN): 128x128 (two workgroups a CU),
@@ -507,6 +509,17 @@ __global__ __launch_bounds__(256) void gemm_tiled_kernel(const T* __restrict__ A
 // splits > 1: as in gemm_tiled_kernel (a split's k-tiles begin at an even one).
 // =====================================================================================
 typedef __attribute__((address_space(3))) void* tw_lds_ptr;
+// Copies of 16 bytes a lane from global memory straight into LDS, as BUFFER loads: base + lane's offset + the wave's offset, so
+// that a copy takes no address arithmetic. As global loads, with a 64-bit address a lane, four waves of a CU issued them at 30 bytes
+// a clock, and with two waves a SIMD taking turns (below) a k-tile of 256x256x64 took 2,540 clocks of which the MFMAs are 2,048;
+// as buffer loads it takes 2,080. Offsets within a tile's operands are 32-bit (checked where the kernels are launched).
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t tw_buffer(const void* base) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, 0x7fffffff, 0x00020000);
+}
+template <int AHEAD = 0>                                     // (bytes further on, in both memories)
+__device__ __forceinline__ void tw_copy_to_lds(__amdgpu_buffer_rsrc_t from, char* to, int lane_offset, int wave_offset) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(from, (tw_lds_ptr)to, 16, lane_offset, wave_offset, AHEAD, 0);
+}
 #define TW_DMA_STAGES 4       /* of W, one k-tile each */
 #define TW_DMA_A_SLOTS 3      /* of A, a pair of k-tiles each */
 
@@ -566,9 +579,10 @@ __global__ __launch_bounds__(256) void gemm_dma_kernel(const bf16_t* __restrict_
   // (A: byte offsets from the tile's first row, for group 0 and from group 0 to group 1; which group a
   // copy belongs to is not known where it is compiled, and a choice between two pointers would put them
   // into memory)
-  const char* const a_base = reinterpret_cast<const char*>(A + (size_t)m0 * lda + (size_t)kt0 * 32);
+  const auto a_buffer = tw_buffer(A + (size_t)m0 * lda + (size_t)kt0 * 32);
+  const auto w_buffer = tw_buffer(W + ((size_t)(n0 / 16) * k_steps + kt0) * 512);
   int a_off[WM], a_step[WM];
-  const bf16_t* w_src[WN];
+  int w_off[WN];
 #pragma unroll
   for (int b = 0; b < WM; ++b) {
     int off[2];
@@ -583,8 +597,8 @@ __global__ __launch_bounds__(256) void gemm_dma_kernel(const bf16_t* __restrict_
   }
 #pragma unroll
   for (int b = 0; b < WN; ++b) {
-    const int blk = min(n0 / 16 + WN * wave + b, n_blocks_w - 1);
-    w_src[b] = W + ((size_t)blk * k_steps + kt0) * 512 + lane * 8;
+    const int block = min(n0 / 16 + WN * wave + b, n_blocks_w - 1) - n0 / 16;
+    w_off[b] = block * (int)k_steps * 1024 + lane * 16;
   }
   // In a last pair that has its even k-tile only, the lanes that would fetch chunks 4..7 (past the end of
   // the row, and for the last row perhaps of the matrix) fetch chunks 0..3 again. Whether a lane's chunk
@@ -595,13 +609,12 @@ __global__ __launch_bounds__(256) void gemm_dma_kernel(const bf16_t* __restrict_
     const int tail = (half_pair && pair == pairs - 1) ? -1 : 0;
     char* slot = lds + (pair_v % TW_DMA_A_SLOTS) * A_SLOT;
     const int off = a_off[b] + (a_step[b] & -grp) + (tail_back[b & 1] & tail);
-    __builtin_amdgcn_global_load_lds((const void*)(a_base + (size_t)pair * 128 + (long)off),
-                                     (tw_lds_ptr)(slot + ((2 * WM) * wave + grp * WM + b) * 1024), 16, 0, 0);
+    tw_copy_to_lds(a_buffer, slot + ((2 * WM) * wave + grp * WM + b) * 1024, off, pair * 128);
   };
   auto copy_w_one = [&](int t_v, int b) {
     const int t = min(t_v, k_tiles - 1);
     char* stage = lds + W_RING + (t_v % TW_DMA_STAGES) * W_STAGE;
-    __builtin_amdgcn_global_load_lds((const void*)(w_src[b] + (size_t)t * 512), (tw_lds_ptr)(stage + (WN * wave + b) * 1024), 16, 0, 0);
+    tw_copy_to_lds(w_buffer, stage + (WN * wave + b) * 1024, w_off[b], t * 1024);
   };
   // this lane's fragment offsets: A in slot 0 for the k-chunk pairs of an even k-tile (an odd one's
   // chunks are 4 further on: bit 6 of the offset flipped), W in stage 0
@@ -712,6 +725,367 @@ __global__ __launch_bounds__(256) void gemm_dma_kernel(const bf16_t* __restrict_
 }
 
 // =====================================================================================
+// The same product with EIGHT waves, two a SIMD, that take turns: while one wave of a SIMD multiplies, the other reads its
+// next fragments from LDS and issues copies. K a multiple of 64, 16-byte rows of the result.
+//
+// The waves form a grid of ROWS x 8 / ROWS, each holds 64 x 32 Q of the tile: 256 x 64 Q (ROWS 4) or 128 x 128 Q (ROWS 2).
+// A k-tile is 64 elements of K, and a PHASE is 32 columns of a wave's tile in one k-tile: 16 MFMAs (256 clocks) between two
+// barriers, behind the reads of those columns of W and, in a k-tile's first phase, of the wave's rows of A. Waves 4..7 pass one
+// barrier more at the start, so that each wave's reads, copies and waits fall into the time in which the other wave of its
+// SIMD multiplies (with one wave a SIMD a copy that misses the vector cache held up the MFMAs behind it: a fifth of the
+// matrix unit's time).
+//
+// LDS holds STAGES k-tiles, filled piece by piece: what phase p read (columns p of W; A, in two halves: p = 0) is replaced by
+// the k-tile STAGES further on from phase p + 1 on (A's second half p + 2): a wave waits for its reads of phase p in front of the
+// barrier behind which it multiplies, for waves 4..7 the one behind which waves 0..3 issue the first copy of phase p + 1. In
+// phase p a wave waits until its copies of what phase p + 1 reads have landed; waves 4..7 do so right before the barrier behind
+// which waves 0..3 read it. Copies land in order, so the wait is a count of the younger ones (Turns::wait).
+//
+// One workgroup a CU takes tile after tile, and the stream of copies runs on from one tile into the next, so that a tile begins
+// with its operands in LDS and its result is stored while more arrive. The MFMAs take W as their row operand: a lane then holds
+// 4 neighbouring columns of one row of the result, and of a gated product the gate next to its up column, and stores them
+// without a trip through LDS (16 bytes a lane of bfloat16 after an exchange with the lane 16 further on). Stores count as
+// accesses in flight like copies do, in order: the first phases of a tile allow for the STORES of the one before, which is why
+// every wave issues all of them (rows and columns outside the result have an offset outside the buffer, which the memory unit
+// drops).
+//
+// What bounds it, 256x256 tiles: power. The loop keeps the matrix units busy for 98 % of its clocks at 8,192 x 8,192 and larger, and
+// the clock falls to 1.5 GHz (1.65 with the four-wave kernel below, whose loop kept them busy for 80 %); so what costs energy
+// costs time. 16x16x32 MFMAs run 10 % faster than 32x32x16 here (they read and write their accumulators half as often). Smaller
+// tiles copy more per MFMA (128x128: 32 KB a 512 clocks) and are bound by that: four waves issue buffer copies at some 33 bytes a
+// clock and CU, eight at more, so 128x128 tiles issue half of a phase's copies between its MFMAs (2,048 x 2,048 x 2,048 23.9 ->
+// 22.1 us; 256x256 tiles get 2 % slower by it).
+// bfloat16, the four-wave kernels -> this one, us (one card, weights from HBM; the same shapes by torch's library in parentheses):
+//   2,048 x 4,608 x 3,584    75.5 -> 64.4 (66)      2,048 x 37,888 x 3,584 gated    527 -> 455
+//   2,048 x 3,584 x 3,584    59.4 -> 54.2 (55)      8,192 x 37,888 x 3,584 gated  1,878 -> 1,571
+//   2,048 x 3,584 x 18,944    268 -> 240 (350)        536 x 27,648 x 5,120 gated    217 -> 188
+//   2,048 x 2,048 x 2,048    27.4 -> 22.2 (22)      2,048 x 11,264 x 2,048 gated    104 -> 88
+//   1,200 x 2,048 x 2,048    30.3 -> 18.8 (20)        536 x 5,120 x 5,120          55.8 -> 46.1
+// =====================================================================================
+__device__ __forceinline__ u32x2 tw_pack4(const float (&v)[4]) {
+  const bf16x4 o = {(bf16_t)v[0], (bf16_t)v[1], (bf16_t)v[2], (bf16_t)v[3]};
+  return __builtin_bit_cast(u32x2, o);
+}
+// 16 bytes to the buffer; bytes behind its end are dropped
+__device__ __forceinline__ void tw_buffer_store16(u32x4 v, __amdgpu_buffer_rsrc_t to, int offset) {
+  __builtin_amdgcn_raw_buffer_store_b128(v, to, offset, 0, 0);
+}
+__device__ __forceinline__ f32x4 tw_buffer_load16(__amdgpu_buffer_rsrc_t from, int offset) {
+  return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(from, offset, 0, 0));
+}
+#define TW_OUTSIDE ((int)0x80000000)   /* an offset that no buffer of tw_buffer holds */
+
+// The shape of a tile and the order of its copies.
+template <int ROWS, int Q>
+struct Turns {
+  static constexpr int COLS = 8 / ROWS, BM = 64 * ROWS, BN = 32 * Q * COLS;
+  static constexpr int A_STAGE = BM * 128, W_STAGE = BN * 128;
+  static constexpr int STAGES = 144 * 1024 / (A_STAGE + W_STAGE) > 4 ? 4 : 144 * 1024 / (A_STAGE + W_STAGE);
+  static constexpr int LDS = STAGES * (A_STAGE + W_STAGE) + 2 * BN * 4;    // (behind the stages the bias of two tiles)
+  static constexpr int A_COPIES = BM / 64, W_COPIES = COLS / 2;            // of 1 KB, a wave's share of A and of a phase's W
+  static constexpr int LEAD = STAGES * Q - 1;                              // phases from a copy's to the one that reads it
+  static constexpr int A_LATE = Q > 1 ? A_COPIES / 2 : 0;                  // A's copies that go out one phase later
+  // phase p's copies: A's late half, A's first half, W, in this order
+  static constexpr int piece(int p) { return (p + LEAD) % Q; }             // (the columns of W that it copies)
+  static constexpr bool late(int p) { return Q > 1 && piece(p) == 1; }
+  static constexpr bool first(int p) { return piece(p) == 0; }
+  static constexpr int a_copies(int p) { return (late(p) ? A_LATE : 0) + (first(p) ? A_COPIES - A_LATE : 0); }
+  static constexpr int copies(int p) { return a_copies(p) + W_COPIES; }
+  static constexpr int behind(int p) { return Q == 1 ? copies(p) / 2 : 0; }              // of them between the phase's MFMAs, behind its wait
+  // The wait of phase p: how many copies are younger than the youngest that phase p + 1 needs. Its W went out LEAD - 1 phases
+  // ago as that phase's last, A's late half one phase later in front of that phase's W.
+  static constexpr int wait(int p) {
+    int younger = 0;
+    const bool a = (p + 1) % Q == 0 && A_LATE > 0;
+    for (int k = 0; k < LEAD - 1 - (a ? 1 : 0); ++k) younger += copies((p - k + 8 * Q) % Q);
+    return younger + (a ? W_COPIES : 0) - behind(p);
+  }
+  static constexpr int CALM = LEAD - 1 - (A_LATE > 0 ? 1 : 0);             // phases of a tile that wait for copies older than the stores
+};
+template <int N>
+__device__ __forceinline__ void tw_wait_accesses() {
+  static_assert(N >= 0 && N < 64, "vmcnt has six bits");
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+}
+
+template <typename OutT, int ROWS, int Q, bool GLU>
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2)))
+void gemm_turns_kernel(const bf16_t* __restrict__ A, long lda, const bf16_t* __restrict__ W, long k_steps, const float* __restrict__ bias,
+                       const float* residual, long ldr, OutT* C, long ldc, int M, int N, int k_tiles_all, int tiles_m, int n_blocks,
+                       int splits, int per_split, float* __restrict__ partial) {
+  typedef Turns<ROWS, Q> S;
+  constexpr int BM = S::BM, BN = S::BN, BAND = 2048 / BM;            // (bands of rows as above)
+  constexpr int STORES = sizeof(OutT) == 4 ? 8 * Q : GLU ? 2 * Q : 4 * Q;   // a tile's, of every wave
+  constexpr int W_RING = S::STAGES * S::A_STAGE, BIAS = W_RING + S::STAGES * S::W_STAGE;
+  extern __shared__ __attribute__((aligned(16))) char lds[];
+  // Workgroup x of the 8 XCDs' 32 takes tiles x / 8, x / 8 + 32, ... of its XCD's run of neighbouring tiles.
+  const int per_xcd = (n_blocks + 7) / 8;
+  const int run_end = min(n_blocks, (int)(blockIdx.x % 8 + 1) * per_xcd);
+  int logical = (blockIdx.x % 8) * per_xcd + blockIdx.x / 8;
+  if (logical >= run_end) return;
+  const int n_tiles = n_blocks / splits, tiles_n = n_tiles / tiles_m;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = wave / S::COLS, wn = wave % S::COLS;                // (waves 0..3: the upper half of the rows)
+  const int turn = wave >> 2;
+
+  f32x4 acc[4][2 * Q];
+  auto clear = [&]() {
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int j = 0; j < 2 * Q; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  };
+  auto aim = [&](int block, int& m0, int& n0, int& split) {
+    const int tile = block % n_tiles;
+    split = block / n_tiles;
+    const int band = tile / (BAND * tiles_n), in_band = tile - band * BAND * tiles_n;
+    const int band_rows = min(BAND, tiles_m - band * BAND);
+    m0 = (band * BAND + in_band % band_rows) * BM;
+    n0 = in_band / band_rows * BN;
+  };
+
+  // The copies: of k-tile copy_t of block copy_block, into stage copy_stage. A copy of A is 8 rows x 128 bytes, place l % 8 of row
+  // u holds the chunk l % 8 ^ (u / 2 % 8) (fragment reads then meet no bank conflict); one of W is half a block of 16 columns x
+  // 64 of K, as it lies in memory. Rows past M and blocks past N are clamped to the last valid one (their products are never
+  // stored); behind the last tile the copies go on with its operands, which nobody reads.
+  __amdgpu_buffer_rsrc_t a_buffer, w_buffer;
+  int a_off[S::A_COPIES], copy_block = logical, copy_t = -1, copy_tiles, copy_stage = S::STAGES - 1, w_blocks;
+  auto aim_copies = [&]() {
+    int m0, n0, split;
+    aim(copy_block, m0, n0, split);
+    const int kt0 = split * per_split;
+    copy_tiles = min(k_tiles_all - kt0, per_split);
+    a_buffer = tw_buffer(A + (size_t)m0 * lda + (size_t)kt0 * 64);
+    w_buffer = tw_buffer(W + ((size_t)(n0 / 16) * k_steps + (size_t)kt0 * 2) * 512);
+    w_blocks = (N + 15) / 16 - n0 / 16;
+#pragma unroll
+    for (int b = 0; b < S::A_COPIES; ++b) {
+      const int row = (wave * S::A_COPIES + b) * 8 + (lane >> 3);
+      a_off[b] = min(row, M - 1 - m0) * (int)lda * 2 + ((lane & 7) ^ ((row >> 1) & 7)) * 16;
+    }
+  };
+  auto copy_a = [&](int b) {
+    tw_copy_to_lds(a_buffer, lds + copy_stage * S::A_STAGE + (wave * S::A_COPIES + b) * 1024, a_off[b], copy_t * 128);
+  };
+  auto copy_w = [&](int piece, bool second) {
+    // block 2 piece + j of wave column c; a wave copies both halves of one (four wave columns) or one half (two)
+    const int c = S::COLS == 4 ? wave >> 1 : wave >> 2, j = S::COLS == 4 ? wave & 1 : (wave >> 1) & 1, half = S::COLS == 4 ? 0 : wave & 1;
+    const int block = c * 2 * Q + 2 * piece + j;
+    const int at = min(block, w_blocks - 1) * (int)k_steps * 1024 + copy_t * 2048 + half * 1024;
+    char* dst = lds + W_RING + copy_stage * S::W_STAGE + block * 2048 + half * 1024;
+    if (second) tw_copy_to_lds<1024>(w_buffer, dst, lane * 16, at);
+    else tw_copy_to_lds(w_buffer, dst, lane * 16, at);
+  };
+  auto copy = [&](auto index, auto which) {                          // copy k of phase P
+    constexpr int P = decltype(index)::value, k = decltype(which)::value, of_a = S::a_copies(P);
+    if constexpr (k == 0 && S::first(P)) {
+      copy_stage = copy_stage + 1 == S::STAGES ? 0 : copy_stage + 1;
+      if (++copy_t == copy_tiles) {
+        if (copy_block + 32 < run_end) copy_block += 32;
+        aim_copies();
+        copy_t = 0;
+      }
+    }
+    if constexpr (k < of_a) copy_a(S::late(P) ? S::A_COPIES - S::A_LATE + k : k);
+    else copy_w(S::piece(P), k > of_a);
+  };
+
+  // this lane's fragments in a stage: of A chunk 4 c + g of row 64 wm + 16 i + r, of W the same chunk of column 16 j + r of a block
+  bf16x8 af[4][2], wf[2][2];
+  const int r0 = lane & 15, g0 = lane >> 4;
+  int a_frag[2];
+#pragma unroll
+  for (int c = 0; c < 2; ++c) a_frag[c] = (wm * 64 + r0) * 128 + (((4 * c + g0) ^ ((r0 >> 1) & 7)) * 16);
+  const int w_frag = W_RING + wn * 4096 * Q + lane * 16;
+  int stage = 0, phases = 0;                                         // the k-tile's stage; the tile's phases before it
+  bool behind_stores = false;                                        // a tile was stored before this one
+  auto phase = [&](auto index) {
+    constexpr int P = decltype(index)::value;
+    if constexpr (P == 0) {
+#pragma unroll
+      for (int c = 0; c < 2; ++c)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) af[i][c] = *reinterpret_cast<const bf16x8*>(lds + a_frag[c] + stage * S::A_STAGE + i * 2048);
+    }
+#pragma unroll
+    for (int c = 0; c < 2; ++c)
+#pragma unroll
+      for (int j = 0; j < 2; ++j) wf[j][c] = *reinterpret_cast<const bf16x8*>(lds + w_frag + stage * S::W_STAGE + P * 4096 + j * 2048 + c * 1024);
+    __builtin_amdgcn_sched_barrier(0);
+    tw_unroll<S::copies(P) - S::behind(P)>([&](auto which) { copy(index, which); });
+    if (behind_stores && phases + P < S::CALM) tw_wait_accesses<S::wait(P) + STORES>();
+    else tw_wait_accesses<S::wait(P)>();
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+    tw_unroll<16>([&](auto which) {
+      constexpr int m = decltype(which)::value, c = m / 8, i = m / 2 % 4, j = m % 2;
+      tw_mma16(acc[i][2 * P + j], wf[j][c], af[i][c]);
+      constexpr int b = S::behind(P), gap = 16 / (b + 1);
+      if constexpr (b > 0 && (m + 1) % gap == 0 && (m + 1) / gap <= b) {
+        __builtin_amdgcn_sched_barrier(0);
+        copy(index, std::integral_constant<int, S::copies(P) - b + (m + 1) / gap - 1>{});
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    });
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+  };
+
+  // The result of a tile. Element e of acc[i][j] is row 16 i + r, column 16 j + 4 g + e of the wave's tile.
+  // (r and g pass through an empty asm in front of a tile's stores: the compiler would else work the stores' offsets out in front
+  // of the tile loop and keep them in registers that the loop does not have)
+  int bias_at = 0;
+  auto bias_of = [&](int j, int g) { return *reinterpret_cast<const f32x4*>(lds + BIAS + bias_at + (wn * 32 * Q + j * 16 + 4 * g) * 4); };
+  auto store_f32 = [&](auto adds_residual, __amdgpu_buffer_rsrc_t to, int ld, __amdgpu_buffer_rsrc_t add, int ld_add, bool biased,
+                       int m0, int n0, auto act_of, int r, int g) {
+    constexpr bool adds = decltype(adds_residual)::value;
+    tw_unroll<4>([&](auto index) {
+      constexpr int i = decltype(index)::value;
+      const int row = wm * 64 + i * 16 + r;
+      f32x4 res[2 * Q];
+      if constexpr (adds) {
+#pragma unroll
+        for (int j = 0; j < 2 * Q; ++j) {
+          const int col = wn * 32 * Q + j * 16 + 4 * g;
+          res[j] = tw_buffer_load16(add, row < M - m0 && col < N - n0 ? row * ld_add * 4 + col * 4 : TW_OUTSIDE);
+        }
+      }
+#pragma unroll
+      for (int j = 0; j < 2 * Q; ++j) {
+        const int col = wn * 32 * Q + j * 16 + 4 * g;
+        f32x4 v = acc[i][j];
+        if (biased) v = v + bias_of(j, g);
+        if constexpr (adds) v = v + res[j];
+        else {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) v[e] = tw_act(v[e], act_of());
+        }
+        tw_buffer_store16(__builtin_bit_cast(u32x4, v), to, row < M - m0 && col < N - n0 ? row * ld * 4 + col * 4 : TW_OUTSIDE);
+      }
+    });
+  };
+  // (an activation is asked for once a tile)
+  auto with_act = [&](auto&& store) {
+    const long act = residual == nullptr ? ldr : 0;          // (no residual: the stride names an activation, see tw_act)
+    if (act == 0) store([]() { return 0L; });
+    else if (act == TW_ACT_RELU_SQUARED) store([]() { return (long)TW_ACT_RELU_SQUARED; });
+    else store([]() { return (long)TW_ACT_GELU_ERF; });
+  };
+  // 16 bytes a lane from two tiles a and b of 16 x 16 in bfloat16: after the exchange between rows of 16 lanes the lanes of
+  // g = 0, 1, 2, 3 hold columns 0..7 of a, 0..7 of b, 8..15 of a, 8..15 of b
+  auto store_pair = [&](__amdgpu_buffer_rsrc_t to, u32x2 a, u32x2 b, int offset) {
+    const auto x = __builtin_amdgcn_permlane16_swap(a[0], b[0], false, false);
+    const auto y = __builtin_amdgcn_permlane16_swap(a[1], b[1], false, false);
+    tw_buffer_store16(u32x4{x[0], y[0], x[1], y[1]}, to, offset);
+  };
+  auto store_tile = [&](int m0, int n0, int split) {
+    int r = lane & 15, g = lane >> 4;
+    asm volatile("" : "+v"(r), "+v"(g));
+    if constexpr (!GLU) {
+      if (splits > 1) {
+        store_f32(std::false_type{}, tw_buffer(partial + ((size_t)split * M + m0) * N + n0), N, a_buffer, 0, false, m0, n0, []() { return 0L; }, r, g);
+        return;
+      }
+    }
+    if constexpr (sizeof(OutT) == 4) {
+      const auto to = tw_buffer(C + (size_t)m0 * ldc + n0);
+      if (residual) store_f32(std::true_type{}, to, (int)ldc, tw_buffer(residual + (size_t)m0 * ldr + n0), (int)ldr, bias != nullptr, m0, n0, []() { return 0L; }, r, g);
+      else with_act([&](auto act_of) { store_f32(std::false_type{}, to, (int)ldc, a_buffer, 0, bias != nullptr, m0, n0, act_of, r, g); });
+    } else if constexpr (GLU) {
+      const auto to = tw_buffer(C + (size_t)m0 * ldc + n0 / 2);
+      auto gated = [&](auto code_of) {
+        auto form = [&](int i, int p) {                      // column tiles 2 p and 2 p + 1: gate and up of 16 columns
+          f32x4 gate = acc[i][2 * p], up = acc[i][2 * p + 1];
+          if (bias) {
+            gate = gate + bias_of(2 * p, g);
+            up = up + bias_of(2 * p + 1, g);
+          }
+          float v[4];
+#pragma unroll
+          for (int e = 0; e < 4; ++e) v[e] = tw_glu(gate[e], up[e], code_of());
+          return tw_pack4(v);
+        };
+        auto offset = [&](int row, int col) {                // (columns of the result)
+          return row < M - m0 && 2 * col < N - n0 ? row * (int)ldc * 2 + col * 2 : TW_OUTSIDE;
+        };
+        tw_unroll<4>([&](auto index) {                       // two neighbouring column groups of a row tile together
+          constexpr int i = decltype(index)::value;
+#pragma unroll
+          for (int p = 0; p + 1 < Q; p += 2)
+            store_pair(to, form(i, p), form(i, p + 1), offset(wm * 64 + i * 16 + r, wn * 16 * Q + p * 16 + (g & 1) * 16 + (g >> 1) * 8));
+          if constexpr (Q % 2 == 1 && i % 2 == 0)            // the last of an odd number: two row tiles
+            store_pair(to, form(i, Q - 1), form(i + 1, Q - 1), offset(wm * 64 + (i + (g & 1)) * 16 + r, wn * 16 * Q + (Q - 1) * 16 + (g >> 1) * 8));
+        });
+      };
+      if (ldr == 0) gated([]() { return 0L; });
+      else gated([&]() { return ldr; });
+    } else {
+      const auto to = tw_buffer(C + (size_t)m0 * ldc + n0);
+      with_act([&](auto act_of) {
+        tw_unroll<4>([&](auto index) {
+          constexpr int i = decltype(index)::value;
+          const int row = wm * 64 + i * 16 + r;
+#pragma unroll
+          for (int p = 0; p < Q; ++p) {
+            u32x2 half[2];
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+              f32x4 x = acc[i][2 * p + j];
+              if (bias) x = x + bias_of(2 * p + j, g);
+              float v[4];
+#pragma unroll
+              for (int e = 0; e < 4; ++e) v[e] = tw_act(x[e], act_of());
+              half[j] = tw_pack4(v);
+            }
+            const int col = wn * 32 * Q + p * 32 + (g & 1) * 16 + (g >> 1) * 8;
+            store_pair(to, half[0], half[1], row < M - m0 && col < N - n0 ? row * (int)ldc * 2 + col * 2 : TW_OUTSIDE);
+          }
+        });
+      });
+    }
+  };
+
+  // what the phases before the first would have copied, then the wait of the last of them
+  aim_copies();
+  tw_unroll<S::LEAD>([&](auto index) {
+    constexpr int T = decltype(index)::value - S::LEAD;
+    constexpr int P = (T + 8 * S::LEAD * Q) % Q;
+    tw_unroll<S::copies(P)>([&](auto which) { copy(std::integral_constant<int, P>{}, which); });
+  });
+  clear();
+  tw_wait_accesses<S::wait(Q - 1) + S::behind(Q - 1)>();
+  __builtin_amdgcn_s_barrier();
+  if (turn == 1) __builtin_amdgcn_s_barrier();                       // waves 4..7: half a phase behind
+  asm volatile("" ::: "memory");
+  for (;;) {
+    int m0, n0, split;
+    aim(logical, m0, n0, split);
+    if (bias && wave * 64 < BN) {
+      // this tile's bias, 64 columns a wave: read behind its last phase, by when it has long landed. (Two places in turn: waves
+      // 4..7 may still be at the tile before.)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(tw_buffer(bias + n0), (tw_lds_ptr)(lds + BIAS + bias_at + wave * 256), 4,
+                                               min(wave * 64 + lane, N - 1 - n0) * 4, 0, 0, 0);
+    }
+    const int k_tiles = min(k_tiles_all - split * per_split, per_split);
+    for (phases = 0; phases < k_tiles * Q; phases += Q) {
+      tw_unroll<Q>(phase);
+      stage = stage + 1 == S::STAGES ? 0 : stage + 1;
+    }
+    store_tile(m0, n0, split);
+    logical += 32;
+    if (logical >= run_end) break;
+    behind_stores = true;
+    bias_at = BN * 4 - bias_at;
+    clear();
+  }
+  if (turn == 0) __builtin_amdgcn_s_barrier();
+  tw_wait_accesses<0>();                                             // (no copy may land behind the workgroup's end)
+}
+
+// =====================================================================================
 // Host side
 // =====================================================================================
 // How many K ranges the tiled kernel uses: with fewer tiles than the chip has room for (a prompt
@@ -778,6 +1152,48 @@ static int launch_tiled(const T* A, long lda, const T* W, long ldw, const float*
 }
 
 
+// Does gemm_turns_kernel take this product? No K range is empty; a tile's bias lands within the tile, so that K is as long as its
+// stages; the result is stored 16 bytes at a time.
+static int turns_per_split(int K, int splits) { return tw_div_up(K / 64, splits); }
+static bool turns_takes(int stages, int out_bytes, long lda, const float* bias, const float* residual, long ldr, const void* C, long ldc,
+                        int N, int K) {
+  return K % 64 == 0 && K >= 64 && (bias == nullptr || K / 64 >= stages) && lda % 8 == 0 && N % 8 == 0 && ldc % (16 / out_bytes) == 0 &&
+         (uintptr_t)C % 16 == 0 && (residual == nullptr || (ldr % 4 == 0 && (uintptr_t)residual % 16 == 0)) &&
+         256 * ldc * out_bytes < (1L << 31) && (residual == nullptr || 256 * ldr * 4 < (1L << 31)) && 256L * N * 4 < (1L << 31);
+}
+
+template <typename OutT, int ROWS, int Q, bool GLU>
+static int launch_turns(const bf16_t* A, long lda, const bf16_t* W, long ldw, const float* bias, const float* residual, long ldr,
+                        OutT* C, long ldc, float* partial, long partial_bytes, int M, int N, int K, int want_splits,
+                        hipStream_t stream, TiledMode* mode = nullptr) {
+  typedef Turns<ROWS, Q> S;
+  const int tiles_m = tw_div_up(M, S::BM), tiles_n = tw_div_up(N, S::BN);
+  int splits = GLU ? 1 : (want_splits > 0 ? want_splits : tiled_splits(M, N, K, 8, S::BM, S::BN));
+  while ((splits - 1) * turns_per_split(K, splits) >= K / 64) --splits;
+  if (mode && mode->dry) {
+    mode->splits = splits;
+    return 0;
+  }
+  if (splits > 1 && (partial == nullptr || partial_bytes < (long)splits * M * N * 4 || (uintptr_t)partial % 16 != 0)) splits = 1;
+  if (mode) mode->splits = splits;
+  const long n_blocks = (long)tiles_m * tiles_n * splits;
+  TW_REQUIRE(n_blocks < (1L << 30));
+  TW_REQUIRE(S::BM * lda * 2 < (1L << 31) && S::BN / 16 * ldw * 1024 < (1L << 31));   // offsets within a tile's operands are 32-bit
+  const int grid = (int)(n_blocks > 256 ? 256 : (n_blocks + 7) / 8 * 8);
+  auto kernel = gemm_turns_kernel<OutT, ROWS, Q, GLU>;
+  static bool attribute_set = false;   // per instantiation
+  if (!attribute_set) {
+    hipError_t e = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, S::LDS);
+    if (e != hipSuccess) return (int)e;
+    attribute_set = true;
+  }
+  kernel<<<grid, 512, S::LDS, stream>>>(A, lda, W, ldw, bias, residual, ldr, C, ldc, M, N, K / 64, tiles_m, (int)n_blocks, splits,
+                                        turns_per_split(K, splits), partial);
+  int err = TW_LAUNCH_RESULT();
+  if (err || splits == 1 || (mode && mode->leave)) return err;
+  return launch_splitk_reduce<OutT>(partial, splits, bias, residual, ldr, C, ldc, M, N, stream);
+}
+
 template <typename OutT, int WM, int WN, bool GLU>
 static int launch_dma(const bf16_t* A, long lda, const bf16_t* W, long ldw, const float* bias,
                       const float* residual, long ldr, OutT* C, long ldc, float* partial, long partial_bytes,
@@ -824,10 +1240,6 @@ static int launch_dma(const bf16_t* A, long lda, const bf16_t* W, long ldw, cons
 // last round.
 // (with the present epilogue, 8,192 x 37,888 x 3,584 in bfloat16, TFLOP/s plain / gated: 128x128 906 / 891, 128x256
 // 1,027 / 1,037, 256x256 1,195 / 1,179, 256x192 1,146 / 1,121)
-#ifndef TW_DMA_SHAPES
-#define TW_DMA_SHAPES 0xC      /* bit s: shape s uses the direct-to-LDS kernel (at 128x128, 1 to 10 % ahead with the present */
-                               /* epilogue and nothing with the one before it, it has not been fitted into the rule above) */
-#endif
 static const int kTileM[5] = {0, 128, 128, 256, 256}, kTileN[5] = {0, 128, 256, 256, 192};
 static const double kTileRate[5] = {0, 0.76, 0.90, 1.05, 1.00};
 
@@ -864,7 +1276,40 @@ static double plan_seconds(int shape, int splits, int M, int N, int K) {
 // prompt (N = 3,584, K = 18,944) has 224 tiles of 128x256 or 112 of 256x256; two K ranges of the latter
 // run at the large tile's rate on 224 CUs (295 -> 265 us with the reduction).
 struct TilePlan { int shape, splits; };
+
+// The same for gemm_turns_kernel, in microseconds: a launch, then rounds of tiles over 256 CUs, each with the tile's begin and end and
+// its k-tiles. A k-tile takes `alone` where the chip is mostly idle (copies and barriers) and rounds x `full` x the share of the
+// chip in use where it is not (power: the clock falls with the matrix units in use); between the two the fourth powers add up.
+// Fitted to 126 products (100 to 8,192 rows, 512 to 11,264 columns, K 512 to 5,632, each at all four shapes: 4 to 6 % off, root mean
+// square), and K ranges to 280 with 2 or 4: the choice was the fastest of all shapes and ranges or, in the mean, 0.2 % behind it (one of
+// 126 more than 4 %).
+struct TurnsCost { double launch, tile, alone, full; };
+static const TurnsCost kTurnsCost[5] = {{}, {3.8, 1.45, 0.351, 0.482}, {4.3, 2.27, 0.589, 0.815}, {3.5, 5.29, 0.960, 1.363}, {3.2, 4.42, 0.759, 1.060}};
+static double turns_us(int shape, int splits, int M, int N, int K) {
+  const TurnsCost& c = kTurnsCost[shape];
+  const long blocks = (long)tw_div_up(M, kTileM[shape]) * tw_div_up(N, kTileN[shape]) * splits;
+  const double rounds = tw_div_up(blocks, 256), alone = rounds * c.alone, full = blocks / 256.0 * c.full;
+  double t = c.launch + rounds * c.tile + tw_div_up(K / 64, splits) * sqrt(sqrt(alone * alone * alone * alone + full * full * full * full));
+  if (splits > 1) t += 3.5 + 0.24e-6 * 4.0 * splits * M * N;       // the ranges' sums written and added up
+  return t;
+}
+static TilePlan choose_turns(bool glu, int M, int N, int K) {
+  TilePlan plan = {1, 1};
+  double best = 0;
+  for (int shape = 1; shape <= 4; ++shape)
+    for (int splits = 1; splits <= (glu ? 1 : 8); ++splits) {
+      if (splits > 1 && K / splits < 512) break;
+      const double t = turns_us(shape, splits, M, N, K);
+      if (best == 0 || t < best) {
+        best = t;
+        plan = {shape, splits};
+      }
+    }
+  return plan;
+}
+
 static TilePlan choose_plan(bool big_ok, bool glu, int M, int N, int K, int epf) {
+  if (big_ok && K % 64 == 0) return choose_turns(glu, M, N, K);
   TilePlan plan = {choose_shape(big_ok, M, N), 0};
   if (!big_ok || glu || K % 32 != 0) return plan;
   const int own = tiled_splits(M, N, K, epf, kTileM[plan.shape], kTileN[plan.shape]);
@@ -895,15 +1340,16 @@ static int tiled_by_shape(int shape, const T* A, long lda, const T* W, long ldw,
     splits = plan.splits;
   }
   if constexpr (BIG) {
-    // bfloat16 and shuffled weights: the kernels that copy straight into LDS, if K allows
+    // bfloat16 and shuffled weights: the kernels that copy straight into LDS, if K and the strides allow
+    auto takes = [&](int stages) { return turns_takes(stages, sizeof(OutT), lda, bias, residual, ldr, C, ldc, N, K); };
+    if (shape == 4 && takes(Turns<4, 3>::STAGES)) return launch_turns<OutT, 4, 3, GLU>(A, lda, W, ldw, bias, residual, ldr, C, ldc, partial, partial_bytes, M, N, K, splits, stream, mode);
+    if (shape == 3 && takes(Turns<4, 4>::STAGES)) return launch_turns<OutT, 4, 4, GLU>(A, lda, W, ldw, bias, residual, ldr, C, ldc, partial, partial_bytes, M, N, K, splits, stream, mode);
+    if (shape == 2 && takes(Turns<2, 2>::STAGES)) return launch_turns<OutT, 2, 2, GLU>(A, lda, W, ldw, bias, residual, ldr, C, ldc, partial, partial_bytes, M, N, K, splits, stream, mode);
+    if (shape == 1 && takes(Turns<2, 1>::STAGES)) return launch_turns<OutT, 2, 1, GLU>(A, lda, W, ldw, bias, residual, ldr, C, ldc, partial, partial_bytes, M, N, K, splits, stream, mode);
     if (K % 32 == 0 && K >= 32 && lda % 8 == 0) {
       if (shape == 4) return launch_dma<OutT, 4, 3, GLU>(A, lda, W, ldw, bias, residual, ldr, C, ldc, partial, partial_bytes, M, N, K, splits, stream, mode);
-      if constexpr ((TW_DMA_SHAPES & 8) != 0)
-        if (shape == 3) return launch_dma<OutT, 4, 4, GLU>(A, lda, W, ldw, bias, residual, ldr, C, ldc, partial, partial_bytes, M, N, K, splits, stream, mode);
-      if constexpr ((TW_DMA_SHAPES & 4) != 0)
-        if (shape == 2) return launch_dma<OutT, 2, 4, GLU>(A, lda, W, ldw, bias, residual, ldr, C, ldc, partial, partial_bytes, M, N, K, splits, stream, mode);
-      if constexpr ((TW_DMA_SHAPES & 2) != 0)
-        if (shape == 1) return launch_dma<OutT, 2, 2, GLU>(A, lda, W, ldw, bias, residual, ldr, C, ldc, partial, partial_bytes, M, N, K, splits, stream, mode);
+      if (shape == 3) return launch_dma<OutT, 4, 4, GLU>(A, lda, W, ldw, bias, residual, ldr, C, ldc, partial, partial_bytes, M, N, K, splits, stream, mode);
+      if (shape == 2) return launch_dma<OutT, 2, 4, GLU>(A, lda, W, ldw, bias, residual, ldr, C, ldc, partial, partial_bytes, M, N, K, splits, stream, mode);
     }
     if (shape == 3 || shape == 4)             // (K no multiple of 32: the register-staged 256x256 tile for both)
       return launch_tiled<T, OutT, 4, 4, SHUF, GLU>(A, lda, W, ldw, bias, residual, ldr, C, ldc, partial, partial_bytes, M, N, K, splits, stream, mode);

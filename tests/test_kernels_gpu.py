@@ -353,6 +353,55 @@ def test_linear_epilogues_at_tile_edges(ops, device, dtype, m, n):
         torch.testing.assert_close(out.double().cpu(), act(want + bias.double().cpu()), **tol(dtype, (1e-5, 1e-5), (1e-2, 1e-2)))
 
 
+@pytest.mark.parametrize("m,n,k", [(65, 8, 64), (256, 256, 128), (257, 264, 320), (129, 1000, 448), (2100, 8200, 128), (4200, 2600, 192), (4099, 4104, 256),
+                                   (300, 264, 2304)])
+def test_linear_of_waves_in_turns(ops, device, m, n, k):
+    """bfloat16 tiles of every shape: one k-tile, fewer and as many as a stage ring holds and no multiple of it; rows and columns
+    that end inside a tile, a wave's tile and a group of 16 columns; more tiles than CUs (a workgroup's second and third tile: its
+    first waits allow for the stores before it, its bias lies in the other place); K ranges of unequal lengths; plain, float32 with
+    a bias and a residual in place, activations, gated. A float32 sum of K exact products, in any order, is off by at most K 2^-24
+    of the sum of their sizes, and a bfloat16 result by another 2^-8 of itself."""
+    x = rand((m, k), torch.bfloat16, device, 1.0, seed=1)
+    w = rand((n, k), torch.bfloat16, device, 0.05, seed=2)
+    bias = rand((n,), torch.float32, device, 0.5, seed=3)
+    res = rand((m, n), torch.float32, device, 1.0, seed=4)
+    shuffled = ops.shuffle_weight(w)
+    want, sizes = x.double() @ w.double().T, x.double().abs() @ w.double().abs().T
+
+    def check(out, value, bound):
+        off = (out.double() - value).abs()
+        assert bool((off <= bound + (2.0 ** -8 * value.abs() if out.dtype == torch.bfloat16 else 0)).all()), float((off / bound).max())
+
+    near = (k + 4) * 2.0 ** -24 * (sizes + 4.0)
+    space = torch.empty(8 * m * n + 4, dtype=torch.float32, device=device) if m * n < 1 << 20 else None   # (room for every number of K ranges)
+    for force in (ops.GEMM_AUTO, ops.GEMM_TILED, ops.GEMM_TILED_WIDE, ops.GEMM_TILED_256, ops.GEMM_TILED_256X192):
+        for work in (None, space):
+            guarded = torch.full((m + 2, n), float("nan"), dtype=torch.bfloat16, device=device)
+            ops.linear(x, shuffled, guarded[:m], bias=bias, workspace=work, force=force)
+            check(guarded[:m], want + bias, near)
+            assert bool(guarded[m:].isnan().all())
+            acc = res.clone()
+            ops.linear(x, shuffled, acc, bias=bias, residual=acc, workspace=work, force=force)
+            check(acc, want + bias.double() + res.double(), near + 2.0 ** -22 * (want.abs() + 5.0))
+            out = torch.full((m, n), float("nan"), device=device)
+            ops.linear(x, shuffled, out, workspace=work, force=force)
+            check(out, want, near)
+        if n % 32 == 0:
+            gated = torch.full((m, n // 2), float("nan"), dtype=torch.bfloat16, device=device)
+            ops.linear_glu(x, shuffled, gated, bias=bias, force=force)
+            g, u = (want + bias).view(m, n // 32, 2, 16).unbind(2)
+            value = (torch.nn.functional.silu(g) * u).reshape(m, n // 2)
+            g_near, u_near = near.view(m, n // 32, 2, 16).unbind(2)
+            # silu has a slope of at most 1.1; its exponential and quotient are off by a few units of 2^-24 more
+            check(gated, value, (1.1 * g_near * (u.abs() + u_near) + g.abs() * u_near + 2.0 ** -20 * (g * u).abs()).reshape(m, n // 2))
+    for name, act in (("relu_squared", lambda z: torch.relu(z) ** 2), ("gelu", torch.nn.functional.gelu)):
+        out = torch.full((m, n), float("nan"), dtype=torch.bfloat16, device=device)
+        ops.linear_act(x, shuffled, out, activation=name, bias=bias)
+        value = want + bias
+        slope = 2 * value.abs() + 1.2                          # (of either; the square of what the sum is off by is in the 0.1)
+        check(out, act(value), near * slope + 2.0 ** -20 * (1 + value.abs()))
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("m,n,k", [(1, 16, 8), (16, 15, 40), (3, 33, 1536), (8, 389, 1576), (16, 256, 3104), (5, 96, 4096), (16, 64, 8200)])
 def test_linear_of_few_rows_over_whole_k(ops, device, dtype, m, n, k):
