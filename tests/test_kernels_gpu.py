@@ -353,6 +353,30 @@ def test_linear_epilogues_at_tile_edges(ops, device, dtype, m, n):
         torch.testing.assert_close(out.double().cpu(), act(want + bias.double().cpu()), **tol(dtype, (1e-5, 1e-5), (1e-2, 1e-2)))
 
 
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("m,n", [(17, 48), (40, 50), (64, 4100)])
+def test_linear_of_a_streaming_workgroup_a_cu_stores_groups(ops, device, dtype, m, n):
+    """Results, residuals and biases that allow 16-byte accesses and ones that do not (a column off, an odd stride), columns that end
+    inside a group of four: the same values. K = 128: a float32 sum is off by at most 128 x 2^-24 of the sum of its sizes."""
+    k = 128
+    x = rand((m, k), dtype, device, 1.0, seed=1)
+    w = rand((n, k), dtype, device, 0.05, seed=2)
+    bias = rand((n + 1,), torch.float32, device, 0.5, seed=3)
+    res = rand((m, n + 4), torch.float32, device, 1.0, seed=4)
+    shuffled = ops.shuffle_weight(w)
+    near = 132 * 2.0 ** -24 * (x.double().abs() @ w.double().abs().T + 8.0)
+    for b in (bias[:n], bias[1:]):
+        want = x.double() @ w.double().T + b
+        for r in (None, res[:, :n], res[:, 1:n + 1]):
+            value = want if r is None else want + r
+            for out in (torch.full((m, n), float("nan"), device=device), torch.full((m, n + 1), float("nan"), device=device)[:, 1:]):
+                ops.linear(x, shuffled, out, bias=b, residual=r, force=ops.GEMM_STREAM_CU)
+                assert bool(((out.double() - value).abs() <= near).all())
+        out = torch.full((m, n), float("nan"), dtype=dtype, device=device)
+        ops.linear(x, shuffled, out, bias=b, force=ops.GEMM_STREAM_CU)
+        assert bool(((out.double() - want).abs() <= near + (2.0 ** -8 * want.abs() if dtype == torch.bfloat16 else 0)).all())
+
+
 @pytest.mark.parametrize("m,n,k", [(65, 8, 64), (256, 256, 128), (257, 264, 320), (129, 1000, 448), (2100, 8200, 128), (4200, 2600, 192), (4099, 4104, 256),
                                    (300, 264, 2304)])
 def test_linear_of_waves_in_turns(ops, device, m, n, k):
