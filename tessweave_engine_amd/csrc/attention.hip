@@ -118,30 +118,46 @@ struct RowTile {
     l = 0.f;
   }
 
-  // One tile of 16 keys starting at position p0 (a multiple of 16).
-  // t_row: position of this lane's row (-1: no such row). lo_load: keys below it are never loaded.
+  // What a lane loads of one tile of 16 keys from position p0 (a multiple of 16) on: key p0 + r's fragments, values
+  // d = 16 dt + r of keys p0 + 4g .. + 3.
+  struct Keys {
+    Frag k[NSMAX];
+    Quad v[DTMAX];
+  };
+  // All of a tile's loads go out together and without predicates: keys outside [lo_load, kv_len) are replaced by the
+  // nearest one inside, whose page is held. (Key by key under a predicate, and the values behind the softmax, a wave waited
+  // for one load after another.)
+  __device__ __forceinline__ static void load(const AttnArgs& a, const int* table, int kvh, int p0, int kv_len, int lo_load, int r, int g,
+                                              Keys& L) {
+    const int D = a.head_dim, P = a.page_size;
+    const int chunks = D / EPF, dts = D / 16;
+    const int p = min(max(p0 + r, lo_load), kv_len - 1);
+    const int pv = min(max(p0 + 4 * g, lo_load & ~3), (kv_len - 1) & ~3);      // (a group of four keys lies in one page)
+    const T* k_row = (const T*)a.keys + (((size_t)table[p / P] * a.kv_heads + kvh) * P + p % P) * D;
+    const T* v_base = (const T*)a.values + ((size_t)table[pv / P] * a.kv_heads + kvh) * D * P + pv % P;
+#pragma unroll
+    for (int st = 0; st < NSMAX; ++st)
+      if (st * 4 < chunks) L.k[st] = tw_load_frag(k_row + min(st * 4 + g, chunks - 1) * EPF);
+#pragma unroll
+    for (int dt = 0; dt < DTMAX; ++dt)
+      if (dt < dts) L.v[dt] = *reinterpret_cast<const Quad*>(v_base + (size_t)(dt * 16 + r) * P);
+  }
   __device__ __forceinline__ void key_tile(const AttnArgs& a, const int* table, int kvh, int p0, int kv_len,
                                            int t_row, int lo_load, int r, int g) {
-    const T* keys = (const T*)a.keys;
-    const T* values = (const T*)a.values;
-    const int D = a.head_dim, P = a.page_size;
+    Keys L;
+    load(a, table, kvh, p0, kv_len, lo_load, r, g, L);
+    multiply(a, p0, kv_len, t_row, lo_load, g, L);
+  }
+
+  // t_row: position of this lane's row (-1: no such row). lo_load: values of keys below it are not used.
+  __device__ __forceinline__ void multiply(const AttnArgs& a, int p0, int kv_len, int t_row, int lo_load, int g, const Keys& L) {
+    const int D = a.head_dim;
     const int chunks = D / EPF, dts = D / 16;
     // ---- S^T = K Q^T ------------------------------------------------------
     f32x4 s = {0.f, 0.f, 0.f, 0.f};
-    {
-      const int p = p0 + r;                       // this lane loads key p's fragments
-      int page = -1;
-      if (p < kv_len && p >= lo_load) page = table[p / P];
-      const T* k_row = keys + (((size_t)(page < 0 ? 0 : page) * a.kv_heads + kvh) * P + p % P) * D;
 #pragma unroll
-      for (int st = 0; st < NSMAX; ++st) {
-        const int chunk = st * 4 + g;
-        if (st * 4 < chunks) {
-          const Frag kf = (page >= 0 && chunk < chunks) ? tw_load_frag(k_row + chunk * EPF) : Elem<T>::zero();
-          tw_mma16(s, kf, qf[st]);
-        }
-      }
-    }
+    for (int st = 0; st < NSMAX; ++st)
+      if (st * 4 < chunks) tw_mma16(s, st * 4 + g < chunks ? L.k[st] : Elem<T>::zero(), qf[st]);
     // ---- mask, online softmax (this lane: row r, keys p0 + 4g + j) ------------
     const int lo_row = attn_first_seen(a, t_row);
     float mx = -INFINITY;
@@ -168,24 +184,15 @@ struct RowTile {
     sum = tw_rows_sum(sum);
     l = l * alpha + sum;
     m = m_new;
-    // ---- O^T += V^T P^T (this lane loads d = 16 dt + r, keys p0 + 4g .. + 3) ----
+    // ---- O^T += V^T P^T ----
     const int pv = p0 + 4 * g;
-    int vpage = -1;
-    if (pv < kv_len && pv + 3 >= lo_load) vpage = table[pv / P];
-    const T* v_base = values + ((size_t)(vpage < 0 ? 0 : vpage) * a.kv_heads + kvh) * D * P + pv % P;
 #pragma unroll
     for (int dt = 0; dt < DTMAX; ++dt) {
       if (dt < dts) {
-        Quad vq;
-        if (vpage >= 0) {
-          vq = *reinterpret_cast<const Quad*>(v_base + (size_t)(dt * 16 + r) * P);
+        Quad vq = L.v[dt];
 #pragma unroll
-          for (int j = 0; j < 4; ++j)
-            if (pv + j >= kv_len || pv + j < lo_load) vq[j] = tw_from_float<T>(0.f);
-        } else {
-#pragma unroll
-          for (int j = 0; j < 4; ++j) vq[j] = tw_from_float<T>(0.f);
-        }
+        for (int j = 0; j < 4; ++j)
+          if (pv + j >= kv_len || pv + j < lo_load) vq[j] = tw_from_float<T>(0.f);
 #pragma unroll
         for (int j = 0; j < 4; ++j) acc[dt][j] *= alpha;
         tw_mma16_k4(acc[dt], vq, pr);
@@ -215,12 +222,16 @@ __device__ __forceinline__ void attn_store_row(const AttnArgs& a, int row, int h
 }
 
 // =====================================================================================
-// Decode: one token per sequence. grid = (splits, kv_heads * row_tiles, n_seqs).
+// Decode: one token per sequence. grid = (splits, kv_heads * row_tiles, n_seqs). The waves of a workgroup take key tiles in turn,
+// each with the next one's loads in flight while it multiplies. What bounds it at few and short sequences is that chain: a
+// float32 tile of head size 128 is 64 MFMAs of 32 clocks behind two rounds of latency (the page, the keys), hence eight waves
+// where their results fit LDS. float32, with a step's host work in both figures: 8 sequences of 1,500 keys, 16 heads of 128 over
+// 4: 34.9 -> 23.4 us; 64 of 1,200, 14 heads of 64 over 2: 44.9 -> 27.0 (four waves, one load after another).
 // =====================================================================================
-template <typename T, int DTMAX>
-__global__ __launch_bounds__(256) void attn_decode_kernel(AttnArgs a) {
-  __shared__ __attribute__((aligned(16))) float lds_o[3][16][DTMAX * 16 + 8];   // (rows of 32 bytes more than a multiple of 256: see tw_lds_swz4)
-  __shared__ float lds_ml[3][16][2];
+template <typename T, int DTMAX, int WAVES>
+__global__ __launch_bounds__(WAVES * 64) void attn_decode_kernel(AttnArgs a) {
+  __shared__ __attribute__((aligned(16))) float lds_o[WAVES - 1][16][DTMAX * 16 + 8];   // (rows of 32 bytes more than a multiple of 256: see tw_lds_swz4)
+  __shared__ float lds_ml[WAVES - 1][16][2];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int r = lane & 15, g = lane >> 4;
   const int G = a.q_heads / a.kv_heads;
@@ -245,10 +256,19 @@ __global__ __launch_bounds__(256) void attn_decode_kernel(AttnArgs a) {
   const int per_split = (tile_hi - tile_lo + a.splits - 1) / a.splits;
   const int begin = tile_lo + split * per_split;
   const int end = min(tile_hi, begin + per_split);
-  for (int kt = begin + wave; kt < end; kt += 4)
-    tile.key_tile(a, table, kvh, kt * 16, kv_len, row_ok ? t : -1, lo, r, g);
+  if constexpr (DTMAX > 8) {                        // (two tiles of keys would not fit the registers)
+    for (int kt = begin + wave; kt < end; kt += WAVES) tile.key_tile(a, table, kvh, kt * 16, kv_len, row_ok ? t : -1, lo, r, g);
+  } else {
+    typename RowTile<T, DTMAX>::Keys now, next;
+    if (begin + wave < end) tile.load(a, table, kvh, (begin + wave) * 16, kv_len, lo, r, g, now);
+    for (int kt = begin + wave; kt < end; kt += WAVES) {
+      if (kt + WAVES < end) tile.load(a, table, kvh, (kt + WAVES) * 16, kv_len, lo, r, g, next);
+      tile.multiply(a, kt * 16, kv_len, row_ok ? t : -1, lo, g, now);
+      now = next;
+    }
+  }
 
-  // ---- merge the 4 waves (fixed order: wave 0 absorbs 1, 2, 3) -------------------
+  // ---- merge the waves (fixed order: wave 0 absorbs 1, 2, 3, ...) -------------------
   if (wave > 0) {
 #pragma unroll
     for (int dt = 0; dt < DTMAX; ++dt)
@@ -264,7 +284,7 @@ __global__ __launch_bounds__(256) void attn_decode_kernel(AttnArgs a) {
   if (wave > 0) return;
   float m = tile.m, l = tile.l;
 #pragma unroll
-  for (int w = 0; w < 3; ++w) m = fmaxf(m, lds_ml[w][r][0]);
+  for (int w = 0; w < WAVES - 1; ++w) m = fmaxf(m, lds_ml[w][r][0]);
   const float m_use = m == -INFINITY ? 0.f : m;
   const float own = tw_exp<T>(tile.m - m_use);
   l *= own;
@@ -273,7 +293,7 @@ __global__ __launch_bounds__(256) void attn_decode_kernel(AttnArgs a) {
 #pragma unroll
     for (int j = 0; j < 4; ++j) tile.acc[dt][j] *= own;
 #pragma unroll
-  for (int w = 0; w < 3; ++w) {
+  for (int w = 0; w < WAVES - 1; ++w) {
     const float f = tw_exp<T>(lds_ml[w][r][0] - m_use);
     l += lds_ml[w][r][1] * f;
 #pragma unroll
@@ -1594,11 +1614,11 @@ static int decode_launch(AttnArgs a, int n_seqs, int generic, hipStream_t stream
     else TW_DECODE_CASE(16, false);
 #undef TW_DECODE_CASE
   } else if (a.head_dim <= 64)
-    attn_decode_kernel<T, 4><<<grid, 256, 0, stream>>>(a);
+    attn_decode_kernel<T, 4, 8><<<grid, 512, 0, stream>>>(a);
   else if (a.head_dim <= 128)
-    attn_decode_kernel<T, 8><<<grid, 256, 0, stream>>>(a);
+    attn_decode_kernel<T, 8, 8><<<grid, 512, 0, stream>>>(a);
   else
-    attn_decode_kernel<T, 16><<<grid, 256, 0, stream>>>(a);
+    attn_decode_kernel<T, 16, 4><<<grid, 256, 0, stream>>>(a);
   int err = TW_LAUNCH_RESULT();
   if (err || a.splits == 1) return err;
   const dim3 rgrid(a.q_heads, n_seqs);
