@@ -39,6 +39,11 @@
 #define TW_MOE_MAX_EXPERTS 1024
 #define TW_MOE_TILE 16
 #define TW_MOE_WIDE 4                 /* tiles a workgroup takes at once in steps of many rows */
+/* in steps of many rows, up to this many units of TW_MOE_WIDE tiles the waves of a workgroup split K (every expert streams its
+   matrices for one or two units; a range of columns a wave leaves a wave a SIMD, 125 us of float32 MFMAs at K = 2,048). 16 experts of
+   2,048 x 1,408 gated, two a token, all launches of the experts, us: 300 tokens float32 476 -> 317, bfloat16 128 -> 92; 480
+   tokens 476 -> 425 and 130 -> 117; 800 tokens (41 units) 539 -> 519 and 153 -> 188: not there */
+#define TW_MOE_SPLITK_UNITS 32
 #define TW_MOE_SPLITK_TILES 64        /* up to this many tiles a step, the waves of a workgroup split K */
 
 // ---- route ---------------------------------------------------------------------------------------------------
@@ -324,7 +329,7 @@ __global__ __launch_bounds__(256) void moe_gather_kernel(const T* __restrict__ h
 // One workgroup: a tile of 16 rows against 4 waves x NT x 16 columns of its expert's matrix W[ex] ([N][K], K a multiple
 // of 32). GLU: W and W2 are gate and up, the result glu(gate, up) goes out in the compute type; otherwise the float32
 // product. Operands go from memory straight into fragments (lane = 16 * piece + row reads 16 bytes).
-// SPLITK (steps of few rows, where the tiles in use are too few to fill the chip and every one streams its expert's whole
+// SPLITK (steps of few rows, and of many with few units, where the tiles in use are too few to fill the chip and every one streams its expert's whole
 // matrix): the four waves share one range of NT x 16 columns and take every fourth step over K each; their sums meet in
 // LDS and are added in the order of the waves.
 // MT > 1 (steps of many rows, whose experts' shares are padded to MT tiles): a workgroup takes MT tiles of one expert
@@ -417,57 +422,96 @@ __global__ __launch_bounds__(256) void moe_grouped_kernel(const T* __restrict__ 
   for (int m = 0; m < MT; ++m)
 #pragma unroll
     for (int t = 0; t < NT; ++t) acc[m][t] = acc2[m][t] = f32x4{0.f, 0.f, 0.f, 0.f};
-  // U steps' operands are on their way before the first is used: what bounds this loop is the latency of memory
-  auto steps = [&](int k, auto count) {
-    constexpr int U = decltype(count)::value;
-    typename Elem<T>::Frag a[U][MT], b[U][NT], b2[U][NT];
+  // U steps' operands are on their way before the first is used, where waves share columns of many rows those of the U steps
+  // behind them too: what bounds this loop is the latency of memory (few rows are not faster by it: their workgroups, two and
+  // more a CU, cover each other's)
+  constexpr int U = MT > 1 ? 2 : GLU ? 4 : (NT > 2 ? 4 : 8);
+  struct Operands {
+    typename Elem<T>::Frag a[U][MT], b[U][NT], b2[GLU ? U : 1][NT];
+  };
+  auto load = [&](int k, auto count, Operands& o) {
+    constexpr int UN = decltype(count)::value;
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
+    for (int u = 0; u < UN; ++u) {
 #pragma unroll
-      for (int m = 0; m < MT; ++m) a[u][m] = tw_load_frag(PLAN ? a_ptr + (k + u * k_stride) / TW_MOE_TILE
+      for (int m = 0; m < MT; ++m) o.a[u][m] = tw_load_frag(PLAN ? a_ptr + (k + u * k_stride) / TW_MOE_TILE
                                                                           : a_ptr + (size_t)m * tile_elems + k + u * k_stride);
 #pragma unroll
       for (int t = 0; t < NT; ++t) {
         // (few rows: an expert's matrices are read once a step)
-        b[u][t] = SPLITK ? tw_load_frag_stream(w_ptr[t] + k + u * k_stride) : tw_load_frag(w_ptr[t] + k + u * k_stride);
-        if (GLU) b2[u][t] = SPLITK ? tw_load_frag_stream(w2_ptr[t] + k + u * k_stride) : tw_load_frag(w2_ptr[t] + k + u * k_stride);
+        o.b[u][t] = SPLITK ? tw_load_frag_stream(w_ptr[t] + k + u * k_stride) : tw_load_frag(w_ptr[t] + k + u * k_stride);
+        if (GLU) o.b2[GLU ? u : 0][t] = SPLITK ? tw_load_frag_stream(w2_ptr[t] + k + u * k_stride) : tw_load_frag(w2_ptr[t] + k + u * k_stride);
       }
     }
     __builtin_amdgcn_sched_barrier(0);               // (the scheduler would put each load in front of its use to save registers)
+  };
+  auto multiply = [&](auto count, const Operands& o) {
+    constexpr int UN = decltype(count)::value;
 #pragma unroll
-    for (int u = 0; u < U; ++u)
+    for (int u = 0; u < UN; ++u)
 #pragma unroll
       for (int t = 0; t < NT; ++t)
 #pragma unroll
         for (int m = 0; m < MT; ++m) {
-          tw_mma16(acc[m][t], a[u][m], b[u][t]);
-          if (GLU) tw_mma16(acc2[m][t], a[u][m], b2[u][t]);
+          tw_mma16(acc[m][t], o.a[u][m], o.b[u][t]);
+          if (GLU) tw_mma16(acc2[m][t], o.a[u][m], o.b2[GLU ? u : 0][t]);
         }
+    if constexpr (SPLITK && MT > 1) __builtin_amdgcn_sched_barrier(0);
   };
-  constexpr int U = MT > 1 ? 2 : GLU ? 4 : (NT > 2 ? 4 : 8);
   int k = k_first;
   const int k_end = (int)tile_elems;
-  for (; k + (U - 1) * k_stride < k_end; k += U * k_stride) steps(k, MoeCount<U>());
-  for (; k < k_end; k += k_stride) steps(k, MoeCount<1>());
-  static_assert(!SPLITK || MT == 1);
+  if constexpr (SPLITK && MT > 1) {
+    constexpr int BATCH = U * k_stride;
+    const int last = k_end - (U - 1) * k_stride;     // a batch that begins before it is whole
+    Operands even, odd;
+    if (k < last) load(k, MoeCount<U>(), even);
+    for (; k < last; k += 2 * BATCH) {
+      if (k + BATCH < last) load(k + BATCH, MoeCount<U>(), odd);
+      multiply(MoeCount<U>(), even);
+      if (k + BATCH >= last) {
+        k += BATCH;
+        break;
+      }
+      if (k + 2 * BATCH < last) load(k + 2 * BATCH, MoeCount<U>(), even);
+      multiply(MoeCount<U>(), odd);
+    }
+    for (; k < k_end; k += k_stride) {
+      load(k, MoeCount<1>(), even);
+      multiply(MoeCount<1>(), even);
+    }
+  } else {
+    Operands now;
+    for (; k + (U - 1) * k_stride < k_end; k += U * k_stride) {
+      load(k, MoeCount<U>(), now);
+      multiply(MoeCount<U>(), now);
+    }
+    for (; k < k_end; k += k_stride) {
+      load(k, MoeCount<1>(), now);
+      multiply(MoeCount<1>(), now);
+    }
+  }
   if constexpr (SPLITK) {
-    __shared__ f32x4 part[GLU ? 2 : 1][3][NT][64];
+    __shared__ f32x4 part[GLU ? 2 : 1][3][MT][NT][64];
     if (wave > 0) {
 #pragma unroll
-      for (int t = 0; t < NT; ++t) {
-        part[0][wave - 1][t][lane] = acc[0][t];
-        if (GLU) part[GLU ? 1 : 0][wave - 1][t][lane] = acc2[0][t];
-      }
+      for (int m = 0; m < MT; ++m)
+#pragma unroll
+        for (int t = 0; t < NT; ++t) {
+          part[0][wave - 1][m][t][lane] = acc[m][t];
+          if (GLU) part[GLU ? 1 : 0][wave - 1][m][t][lane] = acc2[m][t];
+        }
     }
     __syncthreads();
     if (wave > 0) return;
 #pragma unroll
     for (int w = 0; w < 3; ++w)
 #pragma unroll
-      for (int t = 0; t < NT; ++t) {
-        acc[0][t] += part[0][w][t][lane];
-        if (GLU) acc2[0][t] += part[GLU ? 1 : 0][w][t][lane];
-      }
+      for (int m = 0; m < MT; ++m)
+#pragma unroll
+        for (int t = 0; t < NT; ++t) {
+          acc[m][t] += part[0][w][m][t][lane];
+          if (GLU) acc2[m][t] += part[GLU ? 1 : 0][w][m][t][lane];
+        }
   }
 #pragma unroll
   for (int m = 0; m < MT; ++m)
@@ -551,6 +595,12 @@ static void moe_products(const T* xs, const T* gate, const T* up, const T* down,
     moe_grouped_kernel<T, ACT, 2, true><<<dim3(tiles, tw_div_up(Fd, 16 * 2)), 256, 0, stream>>>(
         xs, Cd, first, second, tile_expert, act, Fd, Fd, Cd, limit);
     moe_grouped_kernel<T, 0, 2, true><<<dim3(tiles, tw_div_up(C, 16 * 2)), 256, 0, stream>>>(
+        act, Fd, down, nullptr, tile_expert, ys, C, C, Fd, 0.f);
+  } else if (wide && tiles <= TW_MOE_WIDE * TW_MOE_SPLITK_UNITS) {
+    // an expert's rows make one or two units, too few to fill the chip with a range of columns a wave: the waves split K
+    moe_grouped_kernel<T, ACT, 2, true, TW_MOE_WIDE><<<dim3(tiles / TW_MOE_WIDE, tw_div_up(Fd, 16 * 2)), 256, 0, stream>>>(
+        xs, Cd, first, second, tile_expert, act, Fd, Fd, Cd, limit);
+    moe_grouped_kernel<T, 0, 2, true, TW_MOE_WIDE><<<dim3(tiles / TW_MOE_WIDE, tw_div_up(C, 16 * 2)), 256, 0, stream>>>(
         act, Fd, down, nullptr, tile_expert, ys, C, C, Fd, 0.f);
   } else if (wide) {
     moe_grouped_kernel<T, ACT, 2, false, TW_MOE_WIDE><<<dim3(tiles / TW_MOE_WIDE, tw_div_up(Fd, 4 * 16 * 2)), 256, 0, stream>>>(
