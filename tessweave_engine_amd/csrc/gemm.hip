@@ -498,7 +498,8 @@ __global__ __launch_bounds__(TW_CU_WAVES * 64) void gemm_stream_cu_kernel(
 // Bound by the weights' latency and bytes, and by the activations that every workgroup reads from L2 (with K
 // above 4096 these cost more than they save).
 // =====================================================================================
-template <typename T, typename OutT, int WAVES, bool GLU>
+// ACT: the residual's stride names an activation (a form of its own: its code in the plain form cost that 0.15 us a launch).
+template <typename T, typename OutT, int WAVES, bool GLU, bool ACT = false>
 __global__ __launch_bounds__(WAVES * 64) void gemm_narrow_kernel(const T* __restrict__ A, long lda,
                                                                  const T* __restrict__ W, long ldw,
                                                                  const float* __restrict__ bias,
@@ -578,7 +579,8 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_narrow_kernel(const T* __rest
   if constexpr (GLU) {
     C[(size_t)row * ldc + col] = tw_from_float<OutT>(tw_glu(v[0], v[1], ldr));
   } else {
-    if (residual) v[0] += res;
+    if constexpr (ACT) v[0] = tw_act(v[0], ldr);
+    else if (residual) v[0] += res;
     C[(size_t)row * ldc + col] = tw_from_float<OutT>(v[0]);
   }
 }
@@ -826,28 +828,46 @@ static int launch_skinny_lds_m(const T* A, long lda, const T* W, long ldw, const
 // With more workgroups every one reads the activations again: only where the other kernel's waves sit through a chain
 // of stages and the weights outweigh the activations. Gated, between one and two a CU, the second round is nearly empty
 // and up to 8 rows (in float32 fewer k-steps too) are the most that pays.
-// `sums`: float32 sums for the caller's next kernel, no reduction saved: only where the other kernel has one range too
-// (bf16, 1 and 16 rows: 256 x 512 2.9 / 2.2, 3.2 / 2.9; 4096 x 896 5.4 / 3.4, 6.1 / 4.1; float32 4096 x 448 6.3 / 3.9, 6.9 / 4.4).
+// `sums`: float32 sums for the caller's next kernel, no reduction saved: where the other kernel has one range too
+// (bf16, 1 and 16 rows: 256 x 512 2.9 / 2.2, 3.2 / 2.9; 4096 x 896 5.4 / 3.4, 6.1 / 4.1; float32 4096 x 448 6.3 / 3.9, 6.9 / 4.4),
+// and up to 8 rows with enough columns to fill the chip, where the next kernel reads one sum instead of 3 to 10. In a captured
+// graph, with a norm that adds the sums up behind it, cold weights (K ranges / whole K), 1, 8 and 16 rows:
+//    bf16 1024 x 2048  6.6 / 6.3, 7.1 / 7.0, 7.2 / 7.6      2048 x 2048  7.1 / 6.4, 7.5 / 7.3, 7.8 / 8.1
+//         3072 x 3072  9.7 / 8.0, 10.2 / 9.2, 11.0 / 10.3   3584 x 3584  10.6 / 9.4, 11.2 / 10.4, 12.1 / 11.8
+//         4096 x 2048  8.7 / 7.7, 9.1 / 8.1, 9.6 / 8.8      2048 x 4096  8.6 / 8.1, 9.2 / 9.4, 9.6 / 10.9
+//    float32 896 x 896  7.7 / 6.6, 8.2 / 7.3, 8.6 / 8.0     2560 x 2048  10.9 / 9.1, 11.7 / 10.3, 12.2 / 11.6
+//         2048 x 2048  9.2 / 8.7, 9.7 / 9.8, 10.2 / 11.2    3584 x 3584  17.6 / 15.0, 17.8 / 16.3, 18.8 / 18.9
 static bool narrow_pays(int M, int N, int K, int epf, bool glu, bool sums) {
   const int steps = tw_div_up(K / epf, 4), groups = glu ? N / 32 : tw_div_up(N, 16);
-  if (sums) return groups <= 256 && steps >= 16 && steps < 32;
+  if (sums) {
+    if (groups > 256 || steps < 16) return false;
+    if (steps < 32 || (epf == 4 && steps <= 64 && groups >= 48)) return true;
+    return M <= 8 && groups >= (epf == 4 ? 160 : 128) && steps <= (epf == 4 ? 224 : 112);
+  }
   if (groups <= 256) return steps <= (M > 8 && groups < 96 && !glu ? 96 : 128);
   if (glu) return steps >= 28 && steps <= (groups < 512 && epf == 4 ? 32 : 64) && (M <= 8 || groups >= 512);
   return groups <= 512 && steps >= 16 && steps <= 64;
 }
 
+// A plain product with an activation behind it, against the K ranges' sums and a kernel that adds them up and applies it (bf16, in a
+// captured graph, cold weights): 4096 x 2048 1 / 8 / 16 rows 7.6 / 4.2, 7.9 / 4.6, 8.5 / 5.2; 5632 x 2048 9.0 / 5.8, 9.5 / 6.6, 10.4 / 7.9;
+// 8192 x 3072 12.5 / 9.1, 12.9 / 10.1, 13.6 / 12.3; 11264 x 2048 12.5 / 8.7, 13.1 / 9.3, 14.2 / 11.5.
+static bool narrow_act_pays(int M, int N, int K, int epf) {
+  return M <= 16 && (narrow_pays(M, N, K, epf, false, false) || (epf == 8 && tw_div_up(N, 16) <= 704 && tw_div_up(K / epf, 4) <= 96));
+}
+
 // Waves a workgroup: as few as have a wave's whole share of K in flight at once (8 k-steps), up to 16. (2048 x 1024, 8
 // rows: 4 / 8 / 16 waves 3.5 / 4.0 / 5.6 us; 2048 x 2048: 5.2 / 4.4 / 5.9; 2048 x 4096: 8.1 / 6.7 / 6.5)
-template <typename T, typename OutT, bool GLU>
+template <typename T, typename OutT, bool GLU, bool ACT = false>
 static int launch_narrow(const T* A, long lda, const T* W, long ldw, const float* bias, const float* residual, long ldr,
                          OutT* C, long ldc, int M, int N, int K, hipStream_t stream) {
   const int steps = tw_div_up(K / Elem<T>::kPerFrag, 4), groups = GLU ? N / 32 : tw_div_up(N, 16);
   if (steps <= 48)
-    gemm_narrow_kernel<T, OutT, 4, GLU><<<groups, 256, 0, stream>>>(A, lda, W, ldw, bias, residual, ldr, C, ldc, M, N, K);
+    gemm_narrow_kernel<T, OutT, 4, GLU, ACT><<<groups, 256, 0, stream>>>(A, lda, W, ldw, bias, residual, ldr, C, ldc, M, N, K);
   else if (steps <= 96)
-    gemm_narrow_kernel<T, OutT, 8, GLU><<<groups, 512, 0, stream>>>(A, lda, W, ldw, bias, residual, ldr, C, ldc, M, N, K);
+    gemm_narrow_kernel<T, OutT, 8, GLU, ACT><<<groups, 512, 0, stream>>>(A, lda, W, ldw, bias, residual, ldr, C, ldc, M, N, K);
   else
-    gemm_narrow_kernel<T, OutT, 16, GLU><<<groups, 1024, 0, stream>>>(A, lda, W, ldw, bias, residual, ldr, C, ldc, M, N, K);
+    gemm_narrow_kernel<T, OutT, 16, GLU, ACT><<<groups, 1024, 0, stream>>>(A, lda, W, ldw, bias, residual, ldr, C, ldc, M, N, K);
   return TW_LAUNCH_RESULT();
 }
 
@@ -944,6 +964,24 @@ extern "C" int tw_linear_act(int dtype, const void* A, long lda, const void* W, 
                          partial, partial_bytes, M, N, K, stream);
 }
 
+// The same for up to 16 rows of shuffled weights where a workgroup with the whole of K pays (tw_linear_act_few_pays): the
+// activation in that kernel's epilogue.
+extern "C" int tw_linear_act_few_pays(int dtype, int M, int N, int K) {
+  const int epf = dtype == TW_DTYPE_F32 ? 4 : 8;
+  return M >= 1 && N > 0 && K > 0 && K % epf == 0 && narrow_act_pays(M, N, K, epf) ? 1 : 0;
+}
+extern "C" int tw_linear_act_few(int dtype, const void* A, long lda, const void* W, long ldw, const float* bias, void* C, long ldc,
+                                 int M, int N, int K, int act, hipStream_t stream) {
+  TW_REQUIRE(act == TW_ACT_RELU_SQUARED || act == TW_ACT_GELU_ERF);
+  TW_REQUIRE(dtype == TW_DTYPE_F32 || dtype == TW_DTYPE_BF16);
+  const int epf = dtype == TW_DTYPE_F32 ? 4 : 8;
+  TW_REQUIRE(M >= 1 && M <= 16 && N > 0 && K > 0 && lda >= K && ldc >= N && K % epf == 0 && lda % epf == 0);
+  TW_REQUIRE(weight_layout_ok(dtype, 1, ldw, K) && (uintptr_t)A % 16 == 0 && (uintptr_t)W % 16 == 0);
+  if (dtype == TW_DTYPE_F32)
+    return launch_narrow<float, float, false, true>((const float*)A, lda, (const float*)W, ldw, bias, nullptr, act, (float*)C, ldc, M, N, K, stream);
+  return launch_narrow<bf16_t, bf16_t, false, true>((const bf16_t*)A, lda, (const bf16_t*)W, ldw, bias, nullptr, act, (bf16_t*)C, ldc, M, N, K, stream);
+}
+
 template <typename T>
 static int glu_layout(int shuffled, const T* A, long lda, const T* W, long ldw, const float* bias, T* C, long ldc,
                       int M, int N, int K, int force, long code, hipStream_t stream) {
@@ -986,6 +1024,7 @@ extern "C" int tw_linear_partial_splits_rows(int dtype, int shuffled, int M, int
   const int epf = dtype == TW_DTYPE_F32 ? 4 : 8;
   if (M <= 64 && shuffled && M > TW_CU_ABOVE_ROWS && K % epf == 0)
     return cu_plan(tw_div_up(M, 16), N, K, epf, false, true).splits;
+  if (M <= 16 && shuffled && K % epf == 0 && narrow_pays(M, N, K, epf, false, true)) return 1;
   if (M <= 64) return tw_linear_partial_splits(dtype, N, K);
   if (K % epf || lda < K) return 0;
   const int splits = tw_tiled_partial_splits(dtype, shuffled, lda, M, N, K);

@@ -372,6 +372,31 @@ def linear_act(x, weight, out, activation="relu_squared", bias=None, workspace=N
     return out
 
 
+def linear_act_few_pays(x, weight):
+    """Is `linear_act_few` there for these operands, and faster than the product's split-K sums with the activation behind
+    them? (up to 16 rows, shuffled weights, a workgroup with the whole of K)"""
+    rows = x.shape[0]
+    return (isinstance(weight, ShuffledWeight) and 0 < rows <= 16 and x.data_ptr() % 16 == 0
+            and (rows == 1 or x.stride(0) % (16 // x.element_size()) == 0)
+            and bool(library().tw_linear_act_few_pays(dtype_id(x.dtype), rows, *weight.shape)))
+
+
+def linear_act_few(x, weight, out, activation="relu_squared", bias=None):
+    """`linear_act` for up to 16 rows of a shuffled weight: the kernel that gives a workgroup 16 columns over the whole of K."""
+    _need(activation in LINEAR_ACTIVATIONS, f"activation must be one of {sorted(LINEAR_ACTIVATIONS)}")
+    m, k, lda = _rows(x, "x")
+    n, k2, w_ptr, ldw, shuffled, w_dtype = _weight_args(weight)
+    mo, no, ldc = _rows(out, "out")
+    _need(k == k2 and mo == m and no == n, f"linear_act_few shapes do not agree: x {tuple(x.shape)}, weight {(n, k2)}, out {tuple(out.shape)}")
+    _need(x.dtype == w_dtype == out.dtype and shuffled and 0 < m <= 16, "linear_act_few takes up to 16 rows of a shuffled weight's type")
+    if bias is not None:
+        _need(bias.numel() == n and bias.is_contiguous(), "bias has the wrong size")
+    check(library().tw_linear_act_few(dtype_id(x.dtype), _dev(x), lda, w_ptr, ldw,
+                                      _dev(bias, torch.float32, "bias") if bias is not None else None, _dev(out), ldc, m, n, k,
+                                      LINEAR_ACTIVATIONS[activation], _stream()), "linear_act_few")
+    return out
+
+
 def attn_decode_splits(n_seqs, q_heads, kv_heads, max_kv_len):
     return int(library().tw_attn_decode_splits(n_seqs, q_heads, kv_heads, max_kv_len))
 

@@ -128,10 +128,12 @@ class PlainFeedForward(FeedForward):
     def forward(self, ctx, h, x, accumulate=True):
         n = h.shape[0]
         act = ctx.scratch("ffn.act", (n, self.intermediate))
-        if n <= 64 and self.up.deferrable(n):
-            # few rows: the product leaves its split-K sums, and the activation's kernel adds them up
+        if self.up.forward_act(ctx, h, act, self.activation):             # in the product's epilogue
+            pass
+        elif n <= 64 and self.up.deferrable(n):
+            # the product leaves its split-K sums, and the activation's kernel adds them up
             ops.activation(act, self.activation, partial=self.up.forward_partials(ctx, h, "up"))
-        elif not self.up.forward_act(ctx, h, act, self.activation):       # many rows: in the product's epilogue
+        else:
             self.up.forward(ctx, h, act)
             ops.activation(act, self.activation)
         if self.defer and ctx.defer_sums and self.down.deferrable(n):

@@ -159,10 +159,16 @@ class Linear(Part):
 
     def forward_act(self, ctx, x, out, activation):
         """out = act(x @ W.T (+ bias)) in x's type, the activation in the matrix kernel's epilogue; True if it ran
-        (one packed matrix, more than 64 rows, K a multiple of 16 bytes), else nothing was written."""
-        if len(self.weights) != 1 or self.gated or not ops.can_linear_act(x, self.weights[0]):
+        (one packed matrix; more than 64 rows, K a multiple of 16 bytes, or up to 16 rows where that is faster than split-K
+        sums), else nothing was written."""
+        if len(self.weights) != 1 or self.gated:
             return False
         w = self.weights[0]
+        if ops.linear_act_few_pays(x, w):
+            ops.linear_act_few(x, w, out, activation, bias=self.biases[0] if self.biases else None)
+            return True
+        if not ops.can_linear_act(x, w):
+            return False
         floats = ops.linear_workspace_bytes(w.dtype, x.shape[0], w.shape[0], w.shape[1]) // 4
         ws = ctx.workspace.get("linear.splitk.rows", (floats,), torch.float32) if floats else None
         ops.linear_act(x, w, out, activation, bias=self.biases[0] if self.biases else None, workspace=ws)
@@ -200,10 +206,10 @@ class Linear(Part):
     # ---- leave the split-K sums to the next kernel -------------------------------------------
     def _partial_splits(self, n_rows, lda=None):
         """K ranges of `forward_partials` for N_ROWS rows, LDA elements apart (default: contiguous); 0: none.
-        Up to 64 rows the streaming kernels' ranges depend on the matrix and on how many tiles of 16 rows
-        there are; above, the tiled kernels choose them per row count and stride."""
+        From 17 to 64 rows the streaming kernels' ranges depend on the matrix and on how many tiles of 16 rows
+        there are; up to 16 and above 64 rows the count (and above, the stride) decides too."""
         lda = self.weights[0].shape[1] if lda is None else int(lda)
-        tile = (n_rows + 15) // 16 * 16 if n_rows <= 64 else n_rows       # up to 64 rows: the same for a tile of 16 rows
+        tile = (n_rows + 15) // 16 * 16 if 16 < n_rows <= 64 else n_rows  # from 17 to 64 rows: the same for a tile of 16 rows
         key = ("splits", tile, lda)
         if key not in self._ws_floats:
             self._ws_floats[key] = ops.linear_partial_splits_rows(self.weights[0], tile, lda)

@@ -354,6 +354,31 @@ def test_linear_epilogues_at_tile_edges(ops, device, dtype, m, n):
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("m,n,k", [(1, 2048, 2048), (8, 2047, 1024), (9, 2048, 2048), (8, 4096, 3584), (3, 4100, 2048), (8, 2560, 3592), (16, 896, 896)])
+def test_linear_sums_and_activations_of_few_rows(ops, device, dtype, m, n, k):
+    """Both sides of the rules for sums over the whole of K (rows, columns, k-steps) and the activation behind such a sum: as many
+    sums as are named, each of its share; act(x @ W.T + bias) rounded once. A sum of K exact products is off by at most K 2^-24 of
+    the sum of their sizes."""
+    x = rand((m, k), dtype, device, 1.0, seed=1)
+    w = rand((n, k), dtype, device, 0.05, seed=2)
+    bias = rand((n,), torch.float32, device, 0.5, seed=3)
+    shuffled = ops.shuffle_weight(w)
+    want = x.double() @ w.double().T
+    near = (k + 4) * 2.0 ** -24 * (x.double().abs() @ w.double().abs().T + 1.0)
+    splits = ops.linear_partial_splits_rows(shuffled, m)
+    part = torch.full((splits, m, n), float("nan"), device=device)
+    ops.linear_partials(x, shuffled, part)
+    assert bool(((part.double().sum(0) - want).abs() <= near).all())
+    for name, act in (("relu_squared", lambda z: torch.relu(z) ** 2), ("gelu", torch.nn.functional.gelu)):
+        for b in (None, bias):
+            z = want if b is None else want + b
+            out = torch.full((m, n), float("nan"), dtype=dtype, device=device)
+            ops.linear_act_few(x, shuffled, out, activation=name, bias=b)
+            bound = near * (2 * z.abs() + 1.2) + 2.0 ** -20 * (1 + z.abs()) + (2.0 ** -8 * act(z).abs() if dtype == torch.bfloat16 else 0)
+            assert bool(((out.double() - act(z)).abs() <= bound).all())
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("m,n", [(17, 48), (40, 50), (64, 4100)])
 def test_linear_of_a_streaming_workgroup_a_cu_stores_groups(ops, device, dtype, m, n):
     """Results, residuals and biases that allow 16-byte accesses and ones that do not (a column off, an odd stride), columns that end
