@@ -5,8 +5,11 @@
 
 // ---- embedding: x[n, :] = float(E[ids[n], :]) ------------------------------------
 // A negative id -1 - k stands for feed[k]: a token that an earlier kernel on this stream wrote
-// (the sampler's output of the step before), which the host has not read yet.
-template <typename T>
+// the sampler's output of the step before), which the host has not read yet.
+// VEC: rows of whole 16-byte pieces, a thread one piece of a row (grid.y covers a row): behind its id a row is one trip to memory.
+// Element by element, a workgroup a row, it was a chain of them: 64 rows of 3,584 in bfloat16 9.2 us in a trace, 8 of 2,048 6.5;
+// now 4.7 and 3.4.
+template <typename T, bool VEC>
 __global__ void embed_gather_kernel(const int* __restrict__ ids, const T* __restrict__ table,
                                     float* __restrict__ out, int hidden, int vocab,
                                     const int* __restrict__ feed, int feed_count) {
@@ -16,7 +19,28 @@ __global__ void embed_gather_kernel(const int* __restrict__ ids, const T* __rest
   id = id < 0 ? 0 : (id >= vocab ? vocab - 1 : id);   // ids are validated on the host; never read outside
   const T* row = table + (size_t)id * hidden;
   float* dst = out + (size_t)n * hidden;
-  for (int h = threadIdx.x; h < hidden; h += blockDim.x) dst[h] = tw_to_float(row[h]);
+  if constexpr (VEC) {
+    constexpr int EPF = Elem<T>::kPerFrag;
+    const int h = (blockIdx.y * blockDim.x + threadIdx.x) * EPF;
+    if (h >= hidden) return;
+    const auto v = tw_load_frag(row + h);
+#pragma unroll
+    for (int k = 0; k < EPF; k += 4)
+      *reinterpret_cast<f32x4*>(dst + h + k) = f32x4{tw_to_float(v[k]), tw_to_float(v[k + 1]), tw_to_float(v[k + 2]), tw_to_float(v[k + 3])};
+  } else {
+    for (int h = threadIdx.x; h < hidden; h += blockDim.x) dst[h] = tw_to_float(row[h]);
+  }
+}
+
+template <typename T>
+static void launch_embed_gather(const int* ids, const void* table, float* out, int n, int hidden, int vocab, const int* feed,
+                                int feed_count, hipStream_t stream) {
+  constexpr int EPF = Elem<T>::kPerFrag;
+  const int shares = tw_div_up(hidden / EPF, 256);
+  if (hidden % EPF == 0 && shares <= 65535 && (((uintptr_t)table | (uintptr_t)out) & 15) == 0)
+    embed_gather_kernel<T, true><<<dim3(n, shares), 256, 0, stream>>>(ids, (const T*)table, out, hidden, vocab, feed, feed_count);
+  else
+    embed_gather_kernel<T, false><<<n, 256, 0, stream>>>(ids, (const T*)table, out, hidden, vocab, feed, feed_count);
 }
 
 extern "C" int tw_embed_gather(int dtype, const int* ids, const void* table, float* out, int n,
@@ -24,9 +48,9 @@ extern "C" int tw_embed_gather(int dtype, const int* ids, const void* table, flo
   TW_REQUIRE(n >= 0 && hidden > 0 && vocab > 0 && feed_count >= 0);
   if (n == 0) return 0;
   if (dtype == TW_DTYPE_F32)
-    embed_gather_kernel<float><<<n, 256, 0, stream>>>(ids, (const float*)table, out, hidden, vocab, feed, feed_count);
+    launch_embed_gather<float>(ids, table, out, n, hidden, vocab, feed, feed_count, stream);
   else if (dtype == TW_DTYPE_BF16)
-    embed_gather_kernel<bf16_t><<<n, 256, 0, stream>>>(ids, (const bf16_t*)table, out, hidden, vocab, feed, feed_count);
+    launch_embed_gather<bf16_t>(ids, table, out, n, hidden, vocab, feed, feed_count, stream);
   else
     return TW_ERR_BAD_ARGUMENT;
   return TW_LAUNCH_RESULT();

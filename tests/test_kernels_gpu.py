@@ -37,6 +37,18 @@ def test_embed_gather(ops, device, dtype):
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("hidden", [1, 8, 70, 2048, 2056, 8200])
+def test_embed_gather_of_every_width(ops, device, dtype, hidden):
+    """Rows of whole 16-byte pieces, in one workgroup and several, and rows that are not."""
+    table = rand((50, hidden), dtype, device)
+    ids = torch.tensor([0, 49, -2, 5], dtype=torch.int32, device=device)
+    feed = torch.tensor([3, 17], dtype=torch.int32, device=device)
+    out = torch.full((4, hidden), float("nan"), device=device)
+    ops.embed_gather(ids, table, out, feed=feed)
+    torch.testing.assert_close(out, table.float()[torch.tensor([0, 49, 17, 5], device=device)], atol=0, rtol=0)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("hidden,eps", [(64, 1e-6), (200, 1e-5), (3000, 1e-2), (5120, 1e-5), (8196, 1e-6), (16384, 1e-6),
                                         (16390, 1e-6)])       # one, two and four groups per thread; the generic kernel
 def test_rmsnorm(ops, device, dtype, hidden, eps):
