@@ -24,7 +24,7 @@ __device__ __forceinline__ void tw_wave_lds_fence() {
 // Epilogue of the tiled kernels: each wave passes its tile through LDS (32 rows at a time) so
 // that a lane stores 8 consecutive columns of one row, whole cache lines instead of 2- or 4-byte
 // pieces; bias, residual, the output type and the SiLU-multiply of GLU pairs are applied here.
-// `lds` must hold WAVES x (32 rows x (32 * WN + 4) + 32 * WN) floats and no wave may still read its old contents
+// `lds` must hold 4 waves x (32 rows x (32 * WN + 4) + 32 * WN) floats and no wave may still read its old contents
 // (the __syncthreads below sees to that; afterwards every wave works in its own part).
 //
 // What bounds it is the instruction cache (64 KB, shared by two CUs). Unrolled over the row blocks, the rounds and the
@@ -33,7 +33,7 @@ __device__ __forceinline__ void tw_wave_lds_fence() {
 // (the copy of the accumulators into LDS must name its registers), a round is a loop of a few hundred instructions, and the
 // activation is asked for once a round. 256x256 tiles, K = 3,584, bfloat16: the gated projection of 2,048 rows x 37,888
 // columns 653 -> 491 us, of 8,192 rows 2,479 -> 1,832 us (898 -> 1,215 TFLOP/s); plain products 2 to 5 %.
-template <typename OutT, int WM, int WN, bool GLU, int WAVES = 4>
+template <typename OutT, int WM, int WN, bool GLU>
 __device__ __forceinline__ void tw_tiled_epilogue(f32x16 (&acc)[WM][WN], char* lds, const float* __restrict__ bias,
                                                   const float* residual, long ldr, OutT* C, long ldc, int M, int N,
                                                   int m0, int n0, int wm0, int wn0, int wave, int lane) {
@@ -54,7 +54,7 @@ __device__ __forceinline__ void tw_tiled_epilogue(f32x16 (&acc)[WM][WN], char* l
   float* stage = reinterpret_cast<float*>(lds) + wave * 32 * SROW;
   // A plain product's bias: the wave's columns of it go to LDS once, behind all waves' rows (read from memory in front of
   // every store it cost a fifth of a qkv projection's time at 2,048 rows; in registers a lane needs up to three groups of it).
-  float* bias_stage = reinterpret_cast<float*>(lds) + WAVES * 32 * EROW + wave * WCOLS;
+  float* bias_stage = reinterpret_cast<float*>(lds) + 4 * 32 * EROW + wave * WCOLS;
   auto swz = [](int row) { return SWIZZLED ? ((row & 1) | ((row & 2) << 1)) : 0; };
 
   // A residual that is added to whole rows: all of a row block's values of it are requested in front of the copy into LDS
