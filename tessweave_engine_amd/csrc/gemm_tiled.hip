@@ -750,7 +750,7 @@ __global__ __launch_bounds__(256) void gemm_dma_kernel(const bf16_t* __restrict_
 // drops).
 //
 // What bounds it, 256x256 tiles: power. The loop keeps the matrix units busy for 98 % of its clocks at 8,192 x 8,192 and larger, and
-// the clock falls to 1.5 GHz (1.65 with the four-wave kernel below, whose loop kept them busy for 80 %); so what costs energy
+// the clock falls to 1.5 GHz (1.65 with copies as global loads, where they are busy for 80 %); so what costs energy
 // costs time. 16x16x32 MFMAs run 10 % faster than 32x32x16 here (they read and write their accumulators half as often). Smaller
 // tiles copy more per MFMA (128x128: 32 KB a 512 clocks) and are bound by that: four waves issue buffer copies at some 33 bytes a
 // clock and CU, eight at more, so 128x128 tiles issue half of a phase's copies between its MFMAs (2,048 x 2,048 x 2,048 23.9 ->
