@@ -760,7 +760,12 @@ __global__ __launch_bounds__(256) void gemm_dma_kernel(const bf16_t* __restrict_
 //   2,048 x 3,584 x 3,584    59.4 -> 54.2 (55)      8,192 x 37,888 x 3,584 gated  1,878 -> 1,571
 //   2,048 x 3,584 x 18,944    268 -> 240 (350)        536 x 27,648 x 5,120 gated    217 -> 188
 //   2,048 x 2,048 x 2,048    27.4 -> 22.2 (22)      2,048 x 11,264 x 2,048 gated    104 -> 88
-//   1,200 x 2,048 x 2,048    30.3 -> 18.8 (20)        536 x 5,120 x 5,120          55.8 -> 46.1
+//   1,200 x 2,048 x 2,048    30.3 -> 19.0 (20)        536 x 5,120 x 5,120          55.8 -> 46.1
+//
+// PIECES (tiles of 128 rows, which leave registers for a second set of sums): every `piece` k-tiles a wave adds its sums to the set of
+// those before and begins anew, behind a phase's reads and copies. What a float32 sum is off by grows with its additions: see
+// choose_turns for where a product needs that. (It costs some 0.8 us a product, whatever the number of pieces: code that runs
+// once or twice has to be fetched. More of it costs more: 16 rows at a time, or MFMAs that start from zero, 2 to 4 us.)
 // =====================================================================================
 __device__ __forceinline__ u32x2 tw_pack4(const float (&v)[4]) {
   const bf16x4 o = {(bf16_t)v[0], (bf16_t)v[1], (bf16_t)v[2], (bf16_t)v[3]};
@@ -808,12 +813,13 @@ __device__ __forceinline__ void tw_wait_accesses() {
   asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
 }
 
-template <typename OutT, int ROWS, int Q, bool GLU>
+template <typename OutT, int ROWS, int Q, bool GLU, bool PIECES>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void gemm_turns_kernel(const bf16_t* __restrict__ A, long lda, const bf16_t* __restrict__ W, long k_steps, const float* __restrict__ bias,
                        const float* residual, long ldr, OutT* C, long ldc, int M, int N, int k_tiles_all, int tiles_m, int n_blocks,
-                       int splits, int per_split, float* __restrict__ partial) {
+                       int splits, int per_split, int piece, float* __restrict__ partial) {
   typedef Turns<ROWS, Q> S;
+  static_assert(!PIECES || (ROWS == 2 && !GLU));
   constexpr int BM = S::BM, BN = S::BN, BAND = 2048 / BM;            // (bands of rows as above)
   constexpr int STORES = sizeof(OutT) == 4 ? 8 * Q : GLU ? 2 * Q : 4 * Q;   // a tile's, of every wave
   constexpr int W_RING = S::STAGES * S::A_STAGE, BIAS = W_RING + S::STAGES * S::W_STAGE;
@@ -829,12 +835,17 @@ void gemm_turns_kernel(const bf16_t* __restrict__ A, long lda, const bf16_t* __r
   const int wm = wave / S::COLS, wn = wave % S::COLS;                // (waves 0..3: the upper half of the rows)
   const int turn = wave >> 2;
 
-  f32x4 acc[4][2 * Q];
+  f32x4 acc[4][2 * Q], before[PIECES ? 4 : 1][PIECES ? 2 * Q : 1];   // (of this piece of K; of those before it)
+  int left;                                                          // k-tiles until a piece ends
   auto clear = [&]() {
 #pragma unroll
     for (int i = 0; i < 4; ++i)
 #pragma unroll
-      for (int j = 0; j < 2 * Q; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+      for (int j = 0; j < 2 * Q; ++j) {
+        acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+        if constexpr (PIECES) before[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+      }
+    left = piece;
   };
   auto aim = [&](int block, int& m0, int& n0, int& split) {
     const int tile = block % n_tiles;
@@ -914,6 +925,19 @@ void gemm_turns_kernel(const bf16_t* __restrict__ A, long lda, const bf16_t* __r
       for (int j = 0; j < 2; ++j) wf[j][c] = *reinterpret_cast<const bf16x8*>(lds + w_frag + stage * S::W_STAGE + P * 4096 + j * 2048 + c * 1024);
     __builtin_amdgcn_sched_barrier(0);
     tw_unroll<S::copies(P) - S::behind(P)>([&](auto which) { copy(index, which); });
+    if constexpr (PIECES && P == 0) {
+      if (left == 0) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+          for (int j = 0; j < 2 * Q; ++j) {
+            before[i][j] = before[i][j] + acc[i][j];
+            acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+          }
+        left = piece;
+      }
+      --left;
+    }
     if (behind_stores && phases + P < S::CALM) tw_wait_accesses<S::wait(P) + STORES>();
     else tw_wait_accesses<S::wait(P)>();
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
@@ -1074,6 +1098,12 @@ void gemm_turns_kernel(const bf16_t* __restrict__ A, long lda, const bf16_t* __r
       tw_unroll<Q>(phase);
       stage = stage + 1 == S::STAGES ? 0 : stage + 1;
     }
+    if constexpr (PIECES) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int j = 0; j < 2 * Q; ++j) acc[i][j] = before[i][j] + acc[i][j];
+    }
     store_tile(m0, n0, split);
     logical += 32;
     if (logical >= run_end) break;
@@ -1164,7 +1194,7 @@ static bool turns_takes(int stages, int out_bytes, long lda, const float* bias, 
 
 template <typename OutT, int ROWS, int Q, bool GLU>
 static int launch_turns(const bf16_t* A, long lda, const bf16_t* W, long ldw, const float* bias, const float* residual, long ldr,
-                        OutT* C, long ldc, float* partial, long partial_bytes, int M, int N, int K, int want_splits,
+                        OutT* C, long ldc, float* partial, long partial_bytes, int M, int N, int K, int want_splits, int piece,
                         hipStream_t stream, TiledMode* mode = nullptr) {
   typedef Turns<ROWS, Q> S;
   const int tiles_m = tw_div_up(M, S::BM), tiles_n = tw_div_up(N, S::BN);
@@ -1180,16 +1210,22 @@ static int launch_turns(const bf16_t* A, long lda, const bf16_t* W, long ldw, co
   TW_REQUIRE(n_blocks < (1L << 30));
   TW_REQUIRE(S::BM * lda * 2 < (1L << 31) && S::BN / 16 * ldw * 1024 < (1L << 31));   // offsets within a tile's operands are 32-bit
   const int grid = (int)(n_blocks > 256 ? 256 : (n_blocks + 7) / 8 * 8);
-  auto kernel = gemm_turns_kernel<OutT, ROWS, Q, GLU>;
-  static bool attribute_set = false;   // per instantiation
-  if (!attribute_set) {
-    hipError_t e = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, S::LDS);
-    if (e != hipSuccess) return (int)e;
-    attribute_set = true;
-  }
-  kernel<<<grid, 512, S::LDS, stream>>>(A, lda, W, ldw, bias, residual, ldr, C, ldc, M, N, K / 64, tiles_m, (int)n_blocks, splits,
-                                        turns_per_split(K, splits), partial);
-  int err = TW_LAUNCH_RESULT();
+  const int per_split = turns_per_split(K, splits);
+  auto run = [&](auto in_pieces) {
+    auto kernel = gemm_turns_kernel<OutT, ROWS, Q, GLU, decltype(in_pieces)::value>;
+    static bool attribute_set = false;   // per instantiation
+    if (!attribute_set) {
+      hipError_t e = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, S::LDS);
+      if (e != hipSuccess) return (int)e;
+      attribute_set = true;
+    }
+    kernel<<<grid, 512, S::LDS, stream>>>(A, lda, W, ldw, bias, residual, ldr, C, ldc, M, N, K / 64, tiles_m, (int)n_blocks, splits,
+                                          per_split, piece, partial);
+    return TW_LAUNCH_RESULT();
+  };
+  int err;
+  if constexpr (ROWS == 2 && !GLU) err = piece > 0 && piece < per_split ? run(std::true_type{}) : run(std::false_type{});
+  else err = run(std::false_type{});
   if (err || splits == 1 || (mode && mode->leave)) return err;
   return launch_splitk_reduce<OutT>(partial, splits, bias, residual, ldr, C, ldc, M, N, stream);
 }
@@ -1275,7 +1311,26 @@ static double plan_seconds(int shape, int splits, int M, int N, int K) {
 // leave partly idle and K is long enough to pay for the reduction: the down projection of a 2,048-token
 // prompt (N = 3,584, K = 18,944) has 224 tiles of 128x256 or 112 of 256x256; two K ranges of the latter
 // run at the large tile's rate on 224 CUs (295 -> 265 us with the reduction).
-struct TilePlan { int shape, splits; };
+struct TilePlan { int shape, splits, piece; };        // piece: of gemm_turns_kernel, 0: the whole of K
+
+static TilePlan choose_staged(bool big_ok, bool glu, int M, int N, int K, int epf) {
+  TilePlan plan = {choose_shape(big_ok, M, N), 0, 0};
+  if (!big_ok || glu || K % 32 != 0) return plan;
+  const int own = tiled_splits(M, N, K, epf, kTileM[plan.shape], kTileN[plan.shape]);
+  double best = plan_seconds(plan.shape, own, M, N, K) * 0.95;
+  for (int shape = 2; shape <= 3; ++shape) {               // 128x256 and 256x256: one workgroup a CU
+    const long tiles = (long)tw_div_up(M, kTileM[shape]) * tw_div_up(N, kTileN[shape]);
+    for (int splits = 2; splits <= 8; ++splits) {
+      if (tiles * splits > 256 || K / splits < 2048) continue;
+      const double t = plan_seconds(shape, splits, M, N, K);
+      if (t < best) {
+        best = t;
+        plan = {shape, splits, 0};
+      }
+    }
+  }
+  return plan;
+}
 
 // The same for gemm_turns_kernel, in microseconds: a launch, then rounds of tiles over 256 CUs, each with the tile's begin and end and
 // its k-tiles. A k-tile takes `alone` where the chip is mostly idle (copies and barriers) and rounds x `full` x the share of the
@@ -1283,6 +1338,9 @@ struct TilePlan { int shape, splits; };
 // Fitted to 126 products (100 to 8,192 rows, 512 to 11,264 columns, K 512 to 5,632, each at all four shapes: 4 to 6 % off, root mean
 // square), and K ranges to 280 with 2 or 4: the choice was the fastest of all shapes and ranges or, in the mean, 0.2 % behind it (one of
 // 126 more than 4 %).
+// Its sums are no longer than those of the kernels above: where these would take more K ranges, tiles of 128 rows add up K in
+// pieces as long as those ranges, in the ranges' order, and larger tiles, whose registers are full, take as many ranges. (1,200 x
+// 2,048 x 2,048 in one sum instead of three ranges was off by 2.7e-7 of the result instead of 1.5e-7.)
 struct TurnsCost { double launch, tile, alone, full; };
 static const TurnsCost kTurnsCost[5] = {{}, {3.8, 1.45, 0.351, 0.482}, {4.3, 2.27, 0.589, 0.815}, {3.5, 5.29, 0.960, 1.363}, {3.2, 4.42, 0.759, 1.060}};
 static double turns_us(int shape, int splits, int M, int N, int K) {
@@ -1304,15 +1362,17 @@ static TilePlan choose_turns(bool glu, int M, int N, int K) {
   static thread_local Known known[64] = {};                  // (M = 0: none)
   Known& at = known[((unsigned)M * 2654435761u ^ (unsigned)N * 40503u ^ (unsigned)K * 2246822519u ^ (unsigned)glu) >> 26];
   if (at.M == M && at.N == N && at.K == K && at.glu == (int)glu) return at.plan;
-  TilePlan plan = {1, 1};
+  TilePlan plan = {1, 1, 0};
+  const TilePlan staged = choose_staged(true, glu, M, N, K, 8);
+  const int ranges = glu ? 1 : staged.splits > 0 ? staged.splits : tiled_splits(M, N, K, 8, kTileM[staged.shape], kTileN[staged.shape]);
   double best = 0;
   for (int shape = 1; shape <= 4; ++shape)
-    for (int splits = 1; splits <= (glu ? 1 : 8); ++splits) {
-      if (splits > 1 && K / splits < 512) break;
+    for (int splits = kTileM[shape] > 128 ? ranges : 1; splits <= (glu ? 1 : 8); ++splits) {
+      if (splits > 1 && splits > ranges && K / splits < 512) break;
       const double t = turns_us(shape, splits, M, N, K);
       if (best == 0 || t < best) {
         best = t;
-        plan = {shape, splits};
+        plan = {shape, splits, splits < ranges ? turns_per_split(K, ranges) : 0};
       }
     }
   at = {M, N, K, (int)glu, plan};
@@ -1320,23 +1380,7 @@ static TilePlan choose_turns(bool glu, int M, int N, int K) {
 }
 
 static TilePlan choose_plan(bool big_ok, bool glu, int M, int N, int K, int epf) {
-  if (big_ok && K % 64 == 0) return choose_turns(glu, M, N, K);
-  TilePlan plan = {choose_shape(big_ok, M, N), 0};
-  if (!big_ok || glu || K % 32 != 0) return plan;
-  const int own = tiled_splits(M, N, K, epf, kTileM[plan.shape], kTileN[plan.shape]);
-  double best = plan_seconds(plan.shape, own, M, N, K) * 0.95;
-  for (int shape = 2; shape <= 3; ++shape) {               // 128x256 and 256x256: one workgroup a CU
-    const long tiles = (long)tw_div_up(M, kTileM[shape]) * tw_div_up(N, kTileN[shape]);
-    for (int splits = 2; splits <= 8; ++splits) {
-      if (tiles * splits > 256 || K / splits < 2048) continue;
-      const double t = plan_seconds(shape, splits, M, N, K);
-      if (t < best) {
-        best = t;
-        plan = {shape, splits};
-      }
-    }
-  }
-  return plan;
+  return big_ok && K % 64 == 0 ? choose_turns(glu, M, N, K) : choose_staged(big_ok, glu, M, N, K, epf);
 }
 
 template <typename T, typename OutT, bool SHUF, bool GLU>
@@ -1344,19 +1388,17 @@ static int tiled_by_shape(int shape, const T* A, long lda, const T* W, long ldw,
                           const float* residual, long ldr, OutT* C, long ldc, float* partial,
                           long partial_bytes, int M, int N, int K, hipStream_t stream, TiledMode* mode = nullptr) {
   constexpr bool BIG = sizeof(T) == 2 && SHUF;
-  int splits = 0;                                   // a forced shape keeps the launcher's own rule
-  if (shape == 0) {
-    const TilePlan plan = choose_plan(BIG, GLU, M, N, K, Elem<T>::kPerFrag);
-    shape = plan.shape;
-    splits = plan.splits;
-  }
+  TilePlan plan = {shape, 0, 0};                    // a forced shape keeps the launcher's own rule
+  if (shape == 0) plan = choose_plan(BIG, GLU, M, N, K, Elem<T>::kPerFrag);
+  shape = plan.shape;
+  const int splits = plan.splits;
   if constexpr (BIG) {
     // bfloat16 and shuffled weights: the kernels that copy straight into LDS, if K and the strides allow
     auto takes = [&](int stages) { return turns_takes(stages, sizeof(OutT), lda, bias, residual, ldr, C, ldc, N, K); };
-    if (shape == 4 && takes(Turns<4, 3>::STAGES)) return launch_turns<OutT, 4, 3, GLU>(A, lda, W, ldw, bias, residual, ldr, C, ldc, partial, partial_bytes, M, N, K, splits, stream, mode);
-    if (shape == 3 && takes(Turns<4, 4>::STAGES)) return launch_turns<OutT, 4, 4, GLU>(A, lda, W, ldw, bias, residual, ldr, C, ldc, partial, partial_bytes, M, N, K, splits, stream, mode);
-    if (shape == 2 && takes(Turns<2, 2>::STAGES)) return launch_turns<OutT, 2, 2, GLU>(A, lda, W, ldw, bias, residual, ldr, C, ldc, partial, partial_bytes, M, N, K, splits, stream, mode);
-    if (shape == 1 && takes(Turns<2, 1>::STAGES)) return launch_turns<OutT, 2, 1, GLU>(A, lda, W, ldw, bias, residual, ldr, C, ldc, partial, partial_bytes, M, N, K, splits, stream, mode);
+    if (shape == 4 && takes(Turns<4, 3>::STAGES)) return launch_turns<OutT, 4, 3, GLU>(A, lda, W, ldw, bias, residual, ldr, C, ldc, partial, partial_bytes, M, N, K, splits, plan.piece, stream, mode);
+    if (shape == 3 && takes(Turns<4, 4>::STAGES)) return launch_turns<OutT, 4, 4, GLU>(A, lda, W, ldw, bias, residual, ldr, C, ldc, partial, partial_bytes, M, N, K, splits, plan.piece, stream, mode);
+    if (shape == 2 && takes(Turns<2, 2>::STAGES)) return launch_turns<OutT, 2, 2, GLU>(A, lda, W, ldw, bias, residual, ldr, C, ldc, partial, partial_bytes, M, N, K, splits, plan.piece, stream, mode);
+    if (shape == 1 && takes(Turns<2, 1>::STAGES)) return launch_turns<OutT, 2, 1, GLU>(A, lda, W, ldw, bias, residual, ldr, C, ldc, partial, partial_bytes, M, N, K, splits, plan.piece, stream, mode);
     if (K % 32 == 0 && K >= 32 && lda % 8 == 0) {
       if (shape == 4) return launch_dma<OutT, 4, 3, GLU>(A, lda, W, ldw, bias, residual, ldr, C, ldc, partial, partial_bytes, M, N, K, splits, stream, mode);
       if (shape == 3) return launch_dma<OutT, 4, 4, GLU>(A, lda, W, ldw, bias, residual, ldr, C, ldc, partial, partial_bytes, M, N, K, splits, stream, mode);
