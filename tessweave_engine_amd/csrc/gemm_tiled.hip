@@ -1182,14 +1182,16 @@ static int launch_tiled(const T* A, long lda, const T* W, long ldw, const float*
 }
 
 
-// Does gemm_turns_kernel take this product? No K range is empty; a tile's bias lands within the tile, so that K is as long as its
-// stages; the result is stored 16 bytes at a time.
+// Does gemm_turns_kernel take this product in tiles of S? No K range is empty; a tile's bias lands within the tile, so that K is as long
+// as its stages; operands are copied and results stored 16 bytes at a time; offsets within a tile are 32-bit.
 static int turns_per_split(int K, int splits) { return tw_div_up(K / 64, splits); }
-static bool turns_takes(int stages, int out_bytes, long lda, const float* bias, const float* residual, long ldr, const void* C, long ldc,
-                        int N, int K) {
-  return K % 64 == 0 && K >= 64 && (bias == nullptr || K / 64 >= stages) && lda % 8 == 0 && N % 8 == 0 && ldc % (16 / out_bytes) == 0 &&
-         (uintptr_t)C % 16 == 0 && (residual == nullptr || (ldr % 4 == 0 && (uintptr_t)residual % 16 == 0)) &&
-         256 * ldc * out_bytes < (1L << 31) && (residual == nullptr || 256 * ldr * 4 < (1L << 31)) && 256L * N * 4 < (1L << 31);
+template <typename S>
+static bool turns_takes(int out_bytes, const void* A, long lda, long ldw, const float* bias, const float* residual, long ldr, const void* C,
+                        long ldc, int N, int K) {
+  return K % 64 == 0 && K >= 64 && (bias == nullptr || K / 64 >= S::STAGES) && lda % 8 == 0 && (uintptr_t)A % 16 == 0 && N % 8 == 0 &&
+         ldc % (16 / out_bytes) == 0 && (uintptr_t)C % 16 == 0 && (residual == nullptr || (ldr % 4 == 0 && (uintptr_t)residual % 16 == 0)) &&
+         S::BM * lda * 2 < (1L << 31) && S::BN / 16 * ldw * 1024 < (1L << 31) && S::BM * ldc * out_bytes < (1L << 31) &&
+         (residual == nullptr || S::BM * ldr * 4 < (1L << 31)) && (long)S::BM * N * 4 < (1L << 31);
 }
 
 template <typename OutT, int ROWS, int Q, bool GLU>
@@ -1208,7 +1210,6 @@ static int launch_turns(const bf16_t* A, long lda, const bf16_t* W, long ldw, co
   if (mode) mode->splits = splits;
   const long n_blocks = (long)tiles_m * tiles_n * splits;
   TW_REQUIRE(n_blocks < (1L << 30));
-  TW_REQUIRE(S::BM * lda * 2 < (1L << 31) && S::BN / 16 * ldw * 1024 < (1L << 31));   // offsets within a tile's operands are 32-bit
   const int grid = (int)(n_blocks > 256 ? 256 : (n_blocks + 7) / 8 * 8);
   const int per_split = turns_per_split(K, splits);
   auto run = [&](auto in_pieces) {
@@ -1394,11 +1395,11 @@ static int tiled_by_shape(int shape, const T* A, long lda, const T* W, long ldw,
   const int splits = plan.splits;
   if constexpr (BIG) {
     // bfloat16 and shuffled weights: the kernels that copy straight into LDS, if K and the strides allow
-    auto takes = [&](int stages) { return turns_takes(stages, sizeof(OutT), lda, bias, residual, ldr, C, ldc, N, K); };
-    if (shape == 4 && takes(Turns<4, 3>::STAGES)) return launch_turns<OutT, 4, 3, GLU>(A, lda, W, ldw, bias, residual, ldr, C, ldc, partial, partial_bytes, M, N, K, splits, plan.piece, stream, mode);
-    if (shape == 3 && takes(Turns<4, 4>::STAGES)) return launch_turns<OutT, 4, 4, GLU>(A, lda, W, ldw, bias, residual, ldr, C, ldc, partial, partial_bytes, M, N, K, splits, plan.piece, stream, mode);
-    if (shape == 2 && takes(Turns<2, 2>::STAGES)) return launch_turns<OutT, 2, 2, GLU>(A, lda, W, ldw, bias, residual, ldr, C, ldc, partial, partial_bytes, M, N, K, splits, plan.piece, stream, mode);
-    if (shape == 1 && takes(Turns<2, 1>::STAGES)) return launch_turns<OutT, 2, 1, GLU>(A, lda, W, ldw, bias, residual, ldr, C, ldc, partial, partial_bytes, M, N, K, splits, plan.piece, stream, mode);
+    auto takes = [&](auto tile) { return turns_takes<decltype(tile)>(sizeof(OutT), A, lda, ldw, bias, residual, ldr, C, ldc, N, K); };
+    if (shape == 4 && takes(Turns<4, 3>{})) return launch_turns<OutT, 4, 3, GLU>(A, lda, W, ldw, bias, residual, ldr, C, ldc, partial, partial_bytes, M, N, K, splits, plan.piece, stream, mode);
+    if (shape == 3 && takes(Turns<4, 4>{})) return launch_turns<OutT, 4, 4, GLU>(A, lda, W, ldw, bias, residual, ldr, C, ldc, partial, partial_bytes, M, N, K, splits, plan.piece, stream, mode);
+    if (shape == 2 && takes(Turns<2, 2>{})) return launch_turns<OutT, 2, 2, GLU>(A, lda, W, ldw, bias, residual, ldr, C, ldc, partial, partial_bytes, M, N, K, splits, plan.piece, stream, mode);
+    if (shape == 1 && takes(Turns<2, 1>{})) return launch_turns<OutT, 2, 1, GLU>(A, lda, W, ldw, bias, residual, ldr, C, ldc, partial, partial_bytes, M, N, K, splits, plan.piece, stream, mode);
     if (K % 32 == 0 && K >= 32 && lda % 8 == 0) {
       if (shape == 4) return launch_dma<OutT, 4, 3, GLU>(A, lda, W, ldw, bias, residual, ldr, C, ldc, partial, partial_bytes, M, N, K, splits, stream, mode);
       if (shape == 3) return launch_dma<OutT, 4, 4, GLU>(A, lda, W, ldw, bias, residual, ldr, C, ldc, partial, partial_bytes, M, N, K, splits, stream, mode);
@@ -1449,10 +1450,11 @@ int tw_tiled_partial_splits(int dtype, int shuffled, long lda, int M, int N, int
   TiledMode mode;
   mode.dry = true;
   int err;
+  const long ldw = shuffled ? tw_div_up(K, dtype == TW_DTYPE_F32 ? 16 : 32) : K;
   if (dtype == TW_DTYPE_F32)
-    err = tiled_by_layout<float, float>(shuffled, 0, 0, nullptr, lda, nullptr, K, nullptr, nullptr, 0, nullptr, N, nullptr, 0, M, N, K, nullptr, &mode);
+    err = tiled_by_layout<float, float>(shuffled, 0, 0, nullptr, lda, nullptr, ldw, nullptr, nullptr, 0, nullptr, N, nullptr, 0, M, N, K, nullptr, &mode);
   else if (dtype == TW_DTYPE_BF16)
-    err = tiled_by_layout<bf16_t, float>(shuffled, 0, 0, nullptr, lda, nullptr, K, nullptr, nullptr, 0, nullptr, N, nullptr, 0, M, N, K, nullptr, &mode);
+    err = tiled_by_layout<bf16_t, float>(shuffled, 0, 0, nullptr, lda, nullptr, ldw, nullptr, nullptr, 0, nullptr, N, nullptr, 0, M, N, K, nullptr, &mode);
   else
     return 0;
   return err ? 0 : mode.splits;

@@ -463,6 +463,20 @@ def test_linear_of_waves_in_turns(ops, device, m, n, k):
         check(out, act(value), near * slope + 2.0 ** -20 * (1 + value.abs()))
 
 
+@pytest.mark.parametrize("ld", [1 << 20, 1 << 22, 1 << 23])
+def test_linear_of_rows_far_apart(ops, device, ld):
+    """Rows whose offsets within a tile still fit 31 bits, and rows whose do not in the kernels that copy into LDS: the other
+    tiles take those. A float32 sum of 512 exact products is off by at most 512 x 2^-24 of the sum of their sizes."""
+    m, n, k = 65, 256, 512
+    x = torch.empty((m - 1) * ld + k, dtype=torch.bfloat16, device=device).as_strided((m, k), (ld, 1))
+    x.copy_(rand((m, k), torch.bfloat16, device, 1.0, seed=1))
+    w = rand((n, k), torch.bfloat16, device, 0.05, seed=2)
+    out = torch.empty(m, n, device=device)
+    ops.linear(x, ops.shuffle_weight(w), out)
+    near = (k + 4) * 2.0 ** -24 * (x.double().abs() @ w.double().abs().T + 1.0)
+    assert bool(((out.double() - x.double() @ w.double().T).abs() <= near).all())
+
+
 @pytest.mark.parametrize("m,n,k,ranges", [(1200, 2048, 2048, 3), (146, 8040, 1920, 3), (489, 5496, 4736, 2), (392, 1856, 3264, 6), (1915, 1040, 18688, 6),
                                           (448, 1680, 14528, 7)])
 def test_linear_sums_in_pieces_of_k(ops, device, m, n, k, ranges):
