@@ -1380,26 +1380,26 @@ static TilePlan choose_turns(bool glu, int M, int N, int K) {
   return plan;
 }
 
-static TilePlan choose_plan(bool big_ok, bool glu, int M, int N, int K, int epf) {
-  return big_ok && K % 64 == 0 ? choose_turns(glu, M, N, K) : choose_staged(big_ok, glu, M, N, K, epf);
-}
-
 template <typename T, typename OutT, bool SHUF, bool GLU>
 static int tiled_by_shape(int shape, const T* A, long lda, const T* W, long ldw, const float* bias,
                           const float* residual, long ldr, OutT* C, long ldc, float* partial,
                           long partial_bytes, int M, int N, int K, hipStream_t stream, TiledMode* mode = nullptr) {
   constexpr bool BIG = sizeof(T) == 2 && SHUF;
+  auto takes = [&](auto tile) { return turns_takes<decltype(tile)>(sizeof(OutT), A, lda, ldw, bias, residual, ldr, C, ldc, N, K); };
   TilePlan plan = {shape, 0, 0};                    // a forced shape keeps the launcher's own rule
-  if (shape == 0) plan = choose_plan(BIG, GLU, M, N, K, Elem<T>::kPerFrag);
+  bool turns = BIG;                                 // (each plan is for its own kernels: choose_turns for a product all of whose tiles they take)
+  if (shape == 0) {
+    turns = BIG && takes(Turns<4, 3>{}) && takes(Turns<4, 4>{}) && takes(Turns<2, 2>{}) && takes(Turns<2, 1>{});
+    plan = turns ? choose_turns(GLU, M, N, K) : choose_staged(BIG, GLU, M, N, K, Elem<T>::kPerFrag);
+  }
   shape = plan.shape;
   const int splits = plan.splits;
   if constexpr (BIG) {
     // bfloat16 and shuffled weights: the kernels that copy straight into LDS, if K and the strides allow
-    auto takes = [&](auto tile) { return turns_takes<decltype(tile)>(sizeof(OutT), A, lda, ldw, bias, residual, ldr, C, ldc, N, K); };
-    if (shape == 4 && takes(Turns<4, 3>{})) return launch_turns<OutT, 4, 3, GLU>(A, lda, W, ldw, bias, residual, ldr, C, ldc, partial, partial_bytes, M, N, K, splits, plan.piece, stream, mode);
-    if (shape == 3 && takes(Turns<4, 4>{})) return launch_turns<OutT, 4, 4, GLU>(A, lda, W, ldw, bias, residual, ldr, C, ldc, partial, partial_bytes, M, N, K, splits, plan.piece, stream, mode);
-    if (shape == 2 && takes(Turns<2, 2>{})) return launch_turns<OutT, 2, 2, GLU>(A, lda, W, ldw, bias, residual, ldr, C, ldc, partial, partial_bytes, M, N, K, splits, plan.piece, stream, mode);
-    if (shape == 1 && takes(Turns<2, 1>{})) return launch_turns<OutT, 2, 1, GLU>(A, lda, W, ldw, bias, residual, ldr, C, ldc, partial, partial_bytes, M, N, K, splits, plan.piece, stream, mode);
+    if (turns && shape == 4 && takes(Turns<4, 3>{})) return launch_turns<OutT, 4, 3, GLU>(A, lda, W, ldw, bias, residual, ldr, C, ldc, partial, partial_bytes, M, N, K, splits, plan.piece, stream, mode);
+    if (turns && shape == 3 && takes(Turns<4, 4>{})) return launch_turns<OutT, 4, 4, GLU>(A, lda, W, ldw, bias, residual, ldr, C, ldc, partial, partial_bytes, M, N, K, splits, plan.piece, stream, mode);
+    if (turns && shape == 2 && takes(Turns<2, 2>{})) return launch_turns<OutT, 2, 2, GLU>(A, lda, W, ldw, bias, residual, ldr, C, ldc, partial, partial_bytes, M, N, K, splits, plan.piece, stream, mode);
+    if (turns && shape == 1 && takes(Turns<2, 1>{})) return launch_turns<OutT, 2, 1, GLU>(A, lda, W, ldw, bias, residual, ldr, C, ldc, partial, partial_bytes, M, N, K, splits, plan.piece, stream, mode);
     if (K % 32 == 0 && K >= 32 && lda % 8 == 0) {
       if (shape == 4) return launch_dma<OutT, 4, 3, GLU>(A, lda, W, ldw, bias, residual, ldr, C, ldc, partial, partial_bytes, M, N, K, splits, stream, mode);
       if (shape == 3) return launch_dma<OutT, 4, 4, GLU>(A, lda, W, ldw, bias, residual, ldr, C, ldc, partial, partial_bytes, M, N, K, splits, stream, mode);
@@ -1480,13 +1480,15 @@ int tw_tiled_partials(int dtype, int shuffled, const void* A, long lda, const vo
 
 long tw_tiled_workspace_bytes(int dtype, int rows, int N, int K) {
   const int epf = dtype == TW_DTYPE_F32 ? 4 : 8;
-  // enough for whichever kernel runs: the 128x128 tiles' own rule, or the plan for shuffled bfloat16 weights
-  const int splits = tiled_splits(rows, N, K, epf, 128, 128);
-  long bytes = splits > 1 ? (long)splits * rows * N * 4 : 0;
-  if (dtype == TW_DTYPE_BF16) {
-    const TilePlan plan = choose_plan(true, false, rows, N, K, epf);
+  // enough for whichever kernel runs: the 128x128 tiles' own rule, or either plan for shuffled bfloat16 weights
+  int most = tiled_splits(rows, N, K, epf, 128, 128);
+  auto ask = [&](const TilePlan& plan) {
     const int s = plan.splits > 0 ? plan.splits : tiled_splits(rows, N, K, epf, kTileM[plan.shape], kTileN[plan.shape]);
-    if (s > 1 && (long)s * rows * N * 4 > bytes) bytes = (long)s * rows * N * 4;
+    if (s > most) most = s;
+  };
+  if (dtype == TW_DTYPE_BF16) {
+    ask(choose_staged(true, false, rows, N, K, epf));
+    if (K % 64 == 0) ask(choose_turns(false, rows, N, K));
   }
-  return bytes;
+  return most > 1 ? (long)most * rows * N * 4 : 0;
 }
