@@ -760,7 +760,7 @@ __global__ __launch_bounds__(256) void gemm_dma_kernel(const bf16_t* __restrict_
 //   2,048 x 3,584 x 3,584    59.4 -> 54.2 (55)      8,192 x 37,888 x 3,584 gated  1,878 -> 1,571
 //   2,048 x 3,584 x 18,944    268 -> 240 (350)        536 x 27,648 x 5,120 gated    217 -> 188
 //   2,048 x 2,048 x 2,048    27.4 -> 22.2 (22)      2,048 x 11,264 x 2,048 gated    104 -> 88
-//   1,200 x 2,048 x 2,048    30.3 -> 19.0 (20)        536 x 5,120 x 5,120          55.8 -> 46.1
+//   1,200 x 2,048 x 2,048    30.3 -> 18.4 (20)        536 x 5,120 x 5,120          55.8 -> 46.1
 //
 // PIECES (tiles of 128 rows, which leave registers for a second set of sums): every `piece` k-tiles a wave adds its sums to the set of
 // those before and begins anew, behind a phase's reads and copies. What a float32 sum is off by grows with its additions: see
@@ -966,23 +966,27 @@ void gemm_turns_kernel(const bf16_t* __restrict__ A, long lda, const bf16_t* __r
   auto store_f32 = [&](auto adds_residual, __amdgpu_buffer_rsrc_t to, int ld, __amdgpu_buffer_rsrc_t add, int ld_add, bool biased,
                        int m0, int n0, auto act_of, int r, int g) {
     constexpr bool adds = decltype(adds_residual)::value;
+    // the residual of RT row tiles of 16 at a time (all four where the sums leave registers for it)
+    constexpr int RT = ROWS == 2 ? 4 : 1;
+    f32x4 res[RT][2 * Q];
     tw_unroll<4>([&](auto index) {
       constexpr int i = decltype(index)::value;
-      const int row = wm * 64 + i * 16 + r;
-      f32x4 res[2 * Q];
-      if constexpr (adds) {
+      if constexpr (adds && i % RT == 0) {
 #pragma unroll
-        for (int j = 0; j < 2 * Q; ++j) {
-          const int col = wn * 32 * Q + j * 16 + 4 * g;
-          res[j] = tw_buffer_load16(add, row < M - m0 && col < N - n0 ? row * ld_add * 4 + col * 4 : TW_OUTSIDE);
-        }
+        for (int k = 0; k < RT; ++k)
+#pragma unroll
+          for (int j = 0; j < 2 * Q; ++j) {
+            const int row = wm * 64 + (i + k) * 16 + r, col = wn * 32 * Q + j * 16 + 4 * g;
+            res[k][j] = tw_buffer_load16(add, row < M - m0 && col < N - n0 ? row * ld_add * 4 + col * 4 : TW_OUTSIDE);
+          }
       }
+      const int row = wm * 64 + i * 16 + r;
 #pragma unroll
       for (int j = 0; j < 2 * Q; ++j) {
         const int col = wn * 32 * Q + j * 16 + 4 * g;
         f32x4 v = acc[i][j];
         if (biased) v = v + bias_of(j, g);
-        if constexpr (adds) v = v + res[j];
+        if constexpr (adds) v = v + res[i % RT][j];
         else {
 #pragma unroll
           for (int e = 0; e < 4; ++e) v[e] = tw_act(v[e], act_of());
@@ -1370,7 +1374,9 @@ static TilePlan choose_turns(bool glu, int M, int N, int K) {
   for (int shape = 1; shape <= 4; ++shape)
     for (int splits = kTileM[shape] > 128 ? ranges : 1; splits <= (glu ? 1 : 8); ++splits) {
       if (splits > 1 && splits > ranges && K / splits < 512) break;
-      const double t = turns_us(shape, splits, M, N, K);
+      // (pieces against as many ranges, 13 products of 8 to 128 tiles: level at 30 to 50 tiles of 1,024 of K, 10 % behind at 10
+      // tiles and 20 to 40 % ahead at 80 and more)
+      const double t = turns_us(shape, splits, M, N, K) + (splits < ranges ? 1.8 : 0.0);
       if (best == 0 || t < best) {
         best = t;
         plan = {shape, splits, splits < ranges ? turns_per_split(K, ranges) : 0};
@@ -1378,6 +1384,18 @@ static TilePlan choose_turns(bool glu, int M, int N, int K) {
     }
   at = {M, N, K, (int)glu, plan};
   return plan;
+}
+
+// Where gemm_turns_kernel takes a product: is it the faster one? Its workgroup of 144 KB begins and ends more slowly, alone on its CU,
+// than two small ones, which shows where there is little between: up to 256 tiles of 128x128, K of 64 and 128. It ends most slowly
+// with a residual, which arrives while nothing else runs. (The others / this one, us; with a residual: 100 x 1,024 x 64 5.7 / 7.7, x 256
+// 7.5 / 7.8, 300 x 2,048 x 64 6.1 / 8.3, x 256 7.9 / 8.7, 2,048 x 2,048 x 128 8.6 / 7.4, 300 x 11,264 x 128 10.9 / 14.7, x 512 15.0 / 18.1,
+// x 1,024 20.5 / 22.8, 536 x 11,264 x 512 18.8 / 19.9, 1,024 x 11,264 x 128 17.9 / 14.6; without: 300 x 2,048 x 64 5.4 / 6.3,
+// 1,024 x 2,048 x 128 6.4 / 6.7, 2,048 x 4,096 x 64 9.0 / 7.5; gated 300 x 2,048 x 64 7.0 / 7.3.)
+static bool turns_pay(bool glu, bool adds, int M, int N, int K) {
+  const long tiles = (long)tw_div_up(M, 128) * tw_div_up(N, 128);
+  if (adds) return K > (tiles <= 128 ? 320 : tiles <= 256 ? 64 : tiles <= 600 ? 512 : 0);
+  return tiles > 256 || K > (glu ? 64 : 128);
 }
 
 template <typename T, typename OutT, bool SHUF, bool GLU>
@@ -1389,7 +1407,7 @@ static int tiled_by_shape(int shape, const T* A, long lda, const T* W, long ldw,
   TilePlan plan = {shape, 0, 0};                    // a forced shape keeps the launcher's own rule
   bool turns = BIG;                                 // (each plan is for its own kernels: choose_turns for a product all of whose tiles they take)
   if (shape == 0) {
-    turns = BIG && takes(Turns<4, 3>{}) && takes(Turns<4, 4>{}) && takes(Turns<2, 2>{}) && takes(Turns<2, 1>{});
+    turns = BIG && turns_pay(GLU, residual != nullptr, M, N, K) && takes(Turns<4, 3>{}) && takes(Turns<4, 4>{}) && takes(Turns<2, 2>{}) && takes(Turns<2, 1>{});
     plan = turns ? choose_turns(GLU, M, N, K) : choose_staged(BIG, GLU, M, N, K, Elem<T>::kPerFrag);
   }
   shape = plan.shape;

@@ -463,6 +463,34 @@ def test_linear_of_waves_in_turns(ops, device, m, n, k):
         check(out, act(value), near * slope + 2.0 ** -20 * (1 + value.abs()))
 
 
+@pytest.mark.parametrize("k", [64, 128, 192, 320, 384, 512, 576])
+@pytest.mark.parametrize("m,n", [(65, 264), (300, 7200), (400, 11008)])
+def test_linear_of_short_k(ops, device, m, n, k):
+    """Both sides of the rule that leaves short products to the four-wave tiles (K, up to 128, 256, 600 tiles and more, with a residual
+    and without, gated). Bounds as in test_linear_of_waves_in_turns."""
+    x = rand((m, k), torch.bfloat16, device, 1.0, seed=1)
+    w = rand((n, k), torch.bfloat16, device, 0.05, seed=2)
+    res = rand((m, n), torch.float32, device, 1.0, seed=3)
+    shuffled = ops.shuffle_weight(w)
+    want, sizes = x.double() @ w.double().T, x.double().abs() @ w.double().abs().T
+    near = (k + 4) * 2.0 ** -24 * (sizes + 4.0)
+    out = torch.full((m, n), float("nan"), device=device)
+    ops.linear(x, shuffled, out)
+    assert bool(((out.double() - want).abs() <= near).all())
+    ops.linear(x, shuffled, res, residual=res)
+    assert bool(((res.double() - want - rand((m, n), torch.float32, device, 1.0, seed=3).double()).abs() <= near + 2.0 ** -22 * (want.abs() + 5.0)).all())
+    half = torch.full((m, n), float("nan"), dtype=torch.bfloat16, device=device)
+    ops.linear(x, shuffled, half)
+    assert bool(((half.double() - want).abs() <= near + 2.0 ** -8 * want.abs()).all())
+    if n % 32 == 0:
+        gated = torch.full((m, n // 2), float("nan"), dtype=torch.bfloat16, device=device)
+        ops.linear_glu(x, shuffled, gated)
+        (g, u), (g_near, u_near) = want.view(m, n // 32, 2, 16).unbind(2), near.view(m, n // 32, 2, 16).unbind(2)
+        value = torch.nn.functional.silu(g) * u
+        bound = 1.1 * g_near * (u.abs() + u_near) + g.abs() * u_near + 2.0 ** -20 * (g * u).abs() + 2.0 ** -8 * value.abs()
+        assert bool(((gated.double().view(m, n // 32, 16) - value).abs() <= bound).all())
+
+
 @pytest.mark.parametrize("ld", [1 << 20, 1 << 22, 1 << 23])
 def test_linear_of_rows_far_apart(ops, device, ld):
     """Rows whose offsets within a tile still fit 31 bits, and rows whose do not in the kernels that copy into LDS: the other
