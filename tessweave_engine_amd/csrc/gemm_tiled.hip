@@ -1342,7 +1342,9 @@ static TilePlan choose_staged(bool big_ok, bool glu, int M, int N, int K, int ep
 // chip in use where it is not (power: the clock falls with the matrix units in use); between the two the fourth powers add up.
 // Fitted to 126 products (100 to 8,192 rows, 512 to 11,264 columns, K 512 to 5,632, each at all four shapes: 4 to 6 % off, root mean
 // square), and K ranges to 280 with 2 or 4: the choice was the fastest of all shapes and ranges or, in the mean, 0.2 % behind it (one of
-// 126 more than 4 %).
+// 126 more than 4 %). Asked about 764 more (65 to 5,800 rows, 256 to 152,064 columns, K 64 to 15,040; plain, float32 with a residual
+// and gated) it is 0.4 % behind, 27 of them more than 5 %, if a round counts whole for few rows of a matrix that comes from HBM
+// (its workgroups wait for memory however few they are: 384 x 32,000 x 4,096 by 128x256 124 us, by 256x256 99).
 // Its sums are no longer than those of the kernels above: where these would take more K ranges, tiles of 128 rows add up K in
 // pieces as long as those ranges, in the ranges' order, and larger tiles, whose registers are full, take as many ranges. (1,200 x
 // 2,048 x 2,048 in one sum instead of three ranges was off by 2.7e-7 of the result instead of 1.5e-7.)
@@ -1351,7 +1353,8 @@ static const TurnsCost kTurnsCost[5] = {{}, {3.8, 1.45, 0.351, 0.482}, {4.3, 2.2
 static double turns_us(int shape, int splits, int M, int N, int K) {
   const TurnsCost& c = kTurnsCost[shape];
   const long blocks = (long)tw_div_up(M, kTileM[shape]) * tw_div_up(N, kTileN[shape]) * splits;
-  const double rounds = tw_div_up(blocks, 256), alone = rounds * c.alone, full = blocks / 256.0 * c.full;
+  const double rounds = tw_div_up(blocks, 256), alone = rounds * c.alone;
+  const double full = (M <= 512 && (double)N * K >= 5e7 ? rounds : blocks / 256.0) * c.full;
   double t = c.launch + rounds * c.tile + tw_div_up(K / 64, splits) * sqrt(sqrt(alone * alone * alone * alone + full * full * full * full));
   if (splits > 1) t += 3.5 + 0.24e-6 * 4.0 * splits * M * N;       // the ranges' sums written and added up
   return t;
@@ -1365,7 +1368,7 @@ static TilePlan choose_turns(bool glu, int M, int N, int K) {
     TilePlan plan;
   };
   static thread_local Known known[64] = {};                  // (M = 0: none)
-  Known& at = known[((unsigned)M * 2654435761u ^ (unsigned)N * 40503u ^ (unsigned)K * 2246822519u ^ (unsigned)glu) >> 26];
+  Known& at = known[((unsigned)M * 2654435761u ^ (unsigned)N * 40503u ^ (unsigned)K * 2246822519u ^ (glu ? 0x80000000u : 0u)) >> 26];
   if (at.M == M && at.N == N && at.K == K && at.glu == (int)glu) return at.plan;
   TilePlan plan = {1, 1, 0};
   const TilePlan staged = choose_staged(true, glu, M, N, K, 8);
@@ -1374,9 +1377,9 @@ static TilePlan choose_turns(bool glu, int M, int N, int K) {
   for (int shape = 1; shape <= 4; ++shape)
     for (int splits = kTileM[shape] > 128 ? ranges : 1; splits <= (glu ? 1 : 8); ++splits) {
       if (splits > 1 && splits > ranges && K / splits < 512) break;
-      // (pieces against as many ranges, 13 products of 8 to 128 tiles: level at 30 to 50 tiles of 1,024 of K, 10 % behind at 10
+      // (pieces against as many ranges, 23 products of 8 to 128 tiles: level at 30 to 50 tiles and 1,024 of K, 10 % behind at 10
       // tiles and 20 to 40 % ahead at 80 and more)
-      const double t = turns_us(shape, splits, M, N, K) + (splits < ranges ? 1.8 : 0.0);
+      const double t = turns_us(shape, splits, M, N, K) + (splits < ranges ? 1.2 : 0.0);
       if (best == 0 || t < best) {
         best = t;
         plan = {shape, splits, splits < ranges ? turns_per_split(K, ranges) : 0};
@@ -1391,8 +1394,10 @@ static TilePlan choose_turns(bool glu, int M, int N, int K) {
 // with a residual, which arrives while nothing else runs. (The others / this one, us; with a residual: 100 x 1,024 x 64 5.7 / 7.7, x 256
 // 7.5 / 7.8, 300 x 2,048 x 64 6.1 / 8.3, x 256 7.9 / 8.7, 2,048 x 2,048 x 128 8.6 / 7.4, 300 x 11,264 x 128 10.9 / 14.7, x 512 15.0 / 18.1,
 // x 1,024 20.5 / 22.8, 536 x 11,264 x 512 18.8 / 19.9, 1,024 x 11,264 x 128 17.9 / 14.6; without: 300 x 2,048 x 64 5.4 / 6.3,
-// 1,024 x 2,048 x 128 6.4 / 6.7, 2,048 x 4,096 x 64 9.0 / 7.5; gated 300 x 2,048 x 64 7.0 / 7.3.)
+// 1,024 x 2,048 x 128 6.4 / 6.7, 2,048 x 4,096 x 64 9.0 / 7.5; gated 300 x 2,048 x 64 7.0 / 7.3. Tiles that N does not fill are where the
+// others end slowly: 320 x 344 x 128 7.1 / 6.1, with a residual 7,450 x 608 x 128 16.3 / 13.7.)
 static bool turns_pay(bool glu, bool adds, int M, int N, int K) {
+  if (N % 64 != 0) return true;
   const long tiles = (long)tw_div_up(M, 128) * tw_div_up(N, 128);
   if (adds) return K > (tiles <= 128 ? 320 : tiles <= 256 ? 64 : tiles <= 600 ? 512 : 0);
   return tiles > 256 || K > (glu ? 64 : 128);

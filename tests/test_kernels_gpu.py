@@ -464,7 +464,7 @@ def test_linear_of_waves_in_turns(ops, device, m, n, k):
 
 
 @pytest.mark.parametrize("k", [64, 128, 192, 320, 384, 512, 576])
-@pytest.mark.parametrize("m,n", [(65, 264), (300, 7200), (400, 11008)])
+@pytest.mark.parametrize("m,n", [(65, 264), (65, 256), (300, 7232), (400, 11008)])
 def test_linear_of_short_k(ops, device, m, n, k):
     """Both sides of the rule that leaves short products to the four-wave tiles (K, up to 128, 256, 600 tiles and more, with a residual
     and without, gated). Bounds as in test_linear_of_waves_in_turns."""
