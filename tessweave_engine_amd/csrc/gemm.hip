@@ -248,11 +248,15 @@ __device__ __attribute__((aligned(16))) const uint32_t tw_zero_chunk[4] = {0u, 0
 
 typedef __attribute__((address_space(3))) void* tw_lds_dst;
 
-template <typename T, typename OutT, int MT, bool PARTIAL, bool GLU>
+// PARTIAL: the K ranges' sums go to `partial` (always so with more than one range), otherwise the finished rows to C. WIDE: 16 bytes at a
+// time, to partial or to C, where the launcher finds that columns, strides and addresses allow it. (Forms of their own: with all
+// stores in one kernel, chosen as it runs, four row tiles spilled ten registers: 64 rows x 152,064 x 3,584 208 us instead of 185,
+// x 3,584 x 18,944 37.9 instead of 34.5, x 2,048 x 2,048 13.0 instead of 10.2.)
+template <typename T, typename OutT, int MT, bool PARTIAL, bool GLU, bool WIDE>
 __global__ __launch_bounds__(TW_CU_WAVES * 64) void gemm_stream_cu_kernel(
     const T* __restrict__ A, long lda, const T* __restrict__ W, long ldw, const float* __restrict__ bias,
     const float* residual, long ldr, OutT* C, long ldc, float* __restrict__ partial, int M, int N, int K,
-    int splits, int wgs_per_split, int compute_waves, int steps_per_split, int vec) {
+    int splits, int wgs_per_split, int compute_waves, int steps_per_split) {
   typedef typename Elem<T>::Frag Frag;
   constexpr int EPF = Elem<T>::kPerFrag, U = TW_CU_U, NBUF = TW_CU_NBUF, WAVES = TW_CU_WAVES;
   constexpr int BLOCKS = MT * U;                       // 1 KB blocks of activations per stage
@@ -448,18 +452,18 @@ __global__ __launch_bounds__(TW_CU_WAVES * 64) void gemm_stream_cu_kernel(
       for (int mt = 0; mt < MT; ++mt) {
         const int row = mt * 16 + r;
         if (row >= M || col0 >= N) continue;
-        if (PARTIAL || splits > 1) {
+        if constexpr (PARTIAL) {
           float* dst = partial + ((size_t)split * M + row) * N + col0;
-          if (vec & 1) {
+          if constexpr (WIDE) {
             *reinterpret_cast<f32x4*>(dst) = acc[mt];
           } else {
 #pragma unroll
             for (int e = 0; e < 4; ++e)
               if (col0 + e < N) dst[e] = acc[mt][e];
           }
-        } else if (vec & 2) {
-          // (whole groups of four columns, 64 bytes a row together: stored one by one, the float32 logits of a head of 152,064 x
-          // 3,584 at 64 rows took 232 us, so 223; at 32 rows 197 -> 190)
+        } else if constexpr (WIDE) {
+          // (whole groups of four columns, 64 bytes a row together: the float32 logits of a head of 152,064 x 3,584 at 64 rows
+          // 185 us, stored one by one 196; at 32 rows 174 and 177)
           f32x4 v = acc[mt];
           if (bias) v = v + *reinterpret_cast<const f32x4*>(bias + col0);
           if (residual) v = v + *reinterpret_cast<const f32x4*>(residual + (size_t)row * ldr + col0);
@@ -763,24 +767,37 @@ static int launch_stream_cu_mt(const T* A, long lda, const T* W, long ldw, const
     plan = cu_plan(MT, N, K, EPF, GLU, false);
   }
   TW_REQUIRE(!GLU || N % 32 == 0);
-  // 16-byte accesses: bit 0 to the partial sums, bit 1 to C (and of bias and residual)
-  const int vec = (N % 4 == 0 && (partial == nullptr || (uintptr_t)partial % 16 == 0) ? 1 : 0) |
-                  (N % 4 == 0 && ldc % 4 == 0 && (uintptr_t)C % (4 * sizeof(OutT)) == 0 && (uintptr_t)bias % 16 == 0 &&
-                           (residual == nullptr || (ldr % 4 == 0 && (uintptr_t)residual % 16 == 0)) ? 2 : 0);
-  auto kernel = gemm_stream_cu_kernel<T, OutT, MT, PARTIAL, GLU>;
-  static bool attribute_set = false;   // per instantiation
-  if (!attribute_set) {
-    hipError_t e = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, TW_CU_LDS_BYTES);
-    if (e != hipSuccess) return (int)e;
-    attribute_set = true;
+  auto run = [&](auto sums, auto wide) {
+    constexpr bool SUMS = decltype(sums)::value;
+    typedef std::conditional_t<SUMS, float, OutT> Out;
+    auto kernel = gemm_stream_cu_kernel<T, Out, MT, SUMS, GLU, decltype(wide)::value>;
+    static bool attribute_set = false;   // per instantiation
+    if (!attribute_set) {
+      hipError_t e = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, TW_CU_LDS_BYTES);
+      if (e != hipSuccess) return (int)e;
+      attribute_set = true;
+    }
+    kernel<<<plan.splits * plan.wgs_per_split, TW_CU_WAVES * 64, TW_CU_LDS_BYTES, stream>>>(
+        A, lda, W, ldw, bias, residual, ldr, (Out*)C, ldc, partial, M, N, K, plan.splits, plan.wgs_per_split, plan.compute_waves,
+        plan.steps_per_split);
+    return TW_LAUNCH_RESULT();
+  };
+  if constexpr (GLU) {
+    return run(std::false_type{}, std::false_type{});
+  } else {
+    if (PARTIAL || plan.splits > 1) {
+      const bool wide = N % 4 == 0 && (uintptr_t)partial % 16 == 0;
+      const int err = wide ? run(std::true_type{}, std::true_type{}) : run(std::true_type{}, std::false_type{});
+      if (err || PARTIAL) return err;
+      return launch_splitk_reduce<OutT>(partial, plan.splits, bias, residual, ldr, C, ldc, M, N, stream);
+    }
+    if constexpr (!PARTIAL) {
+      const bool wide = N % 4 == 0 && ldc % 4 == 0 && (uintptr_t)C % (4 * sizeof(OutT)) == 0 && (uintptr_t)bias % 16 == 0 &&
+                        (residual == nullptr || (ldr % 4 == 0 && (uintptr_t)residual % 16 == 0));
+      return wide ? run(std::false_type{}, std::true_type{}) : run(std::false_type{}, std::false_type{});
+    }
+    return TW_ERR_BAD_ARGUMENT;
   }
-  const int threads = TW_CU_WAVES * 64;
-  kernel<<<plan.splits * plan.wgs_per_split, threads, TW_CU_LDS_BYTES, stream>>>(
-      A, lda, W, ldw, bias, residual, ldr, C, ldc, partial, M, N, K, plan.splits, plan.wgs_per_split, plan.compute_waves,
-      plan.steps_per_split, vec);
-  int err = TW_LAUNCH_RESULT();
-  if (err || plan.splits == 1 || PARTIAL) return err;
-  return launch_splitk_reduce<OutT>(partial, plan.splits, bias, residual, ldr, C, ldc, M, N, stream);
 }
 
 template <typename T, typename OutT, bool PARTIAL, bool GLU>

@@ -414,6 +414,31 @@ def test_linear_of_a_streaming_workgroup_a_cu_stores_groups(ops, device, dtype, 
         assert bool(((out.double() - want).abs() <= near + (2.0 ** -8 * want.abs() if dtype == torch.bfloat16 else 0)).all())
 
 
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("m,n", [(17, 48), (33, 50), (64, 260)])
+def test_linear_of_a_streaming_workgroup_a_cu_adds_ranges_up(ops, device, dtype, m, n):
+    """The same with K ranges, whose sums go to scratch 16 bytes at a time where columns and scratch allow it: scratch that does and
+    that does not, results in float32 with a bias and a residual and in the operands' type."""
+    k = 2048
+    x = rand((m, k), dtype, device, 1.0, seed=1)
+    w = rand((n, k), dtype, device, 0.05, seed=2)
+    bias = rand((n,), torch.float32, device, 0.5, seed=3)
+    res = rand((m, n), torch.float32, device, 1.0, seed=4)
+    shuffled = ops.shuffle_weight(w)
+    floats = ops.linear_workspace_bytes(dtype, m, n, k) // 4
+    assert ops.linear_partial_splits_rows(shuffled, m) > 1 and floats
+    want = x.double() @ w.double().T
+    near = (k + 8) * 2.0 ** -24 * (x.double().abs() @ w.double().abs().T + 8.0)
+    for at in (0, 1):
+        space = torch.full((floats + 4,), float("nan"), device=device)[at:]
+        out = torch.full((m, n), float("nan"), device=device)
+        ops.linear(x, shuffled, out, bias=bias, residual=res, workspace=space)
+        assert bool(((out.double() - want - bias - res).abs() <= near).all())
+        out = torch.full((m, n), float("nan"), dtype=dtype, device=device)
+        ops.linear(x, shuffled, out, workspace=space)
+        assert bool(((out.double() - want).abs() <= near + (2.0 ** -8 * want.abs() if dtype == torch.bfloat16 else 0)).all())
+
+
 @pytest.mark.parametrize("m,n,k", [(65, 8, 64), (256, 256, 128), (257, 264, 320), (129, 1000, 448), (2100, 8200, 128), (4200, 2600, 192), (4099, 4104, 256),
                                    (300, 264, 2304)])
 def test_linear_of_waves_in_turns(ops, device, m, n, k):
