@@ -39,11 +39,6 @@
 #define TW_MOE_MAX_EXPERTS 1024
 #define TW_MOE_TILE 16
 #define TW_MOE_WIDE 4                 /* tiles a workgroup takes at once in steps of many rows */
-/* in steps of many rows, up to this many units of TW_MOE_WIDE tiles the waves of a workgroup split K (every expert streams its
-   matrices for one or two units; a range of columns a wave leaves a wave a SIMD, 125 us of float32 MFMAs at K = 2,048). 16 experts of
-   2,048 x 1,408 gated, two a token, all launches of the experts, us: 300 tokens float32 476 -> 317, bfloat16 128 -> 92; 480
-   tokens 476 -> 425 and 130 -> 117; 800 tokens (41 units) 539 -> 519 and 153 -> 188: not there */
-#define TW_MOE_SPLITK_UNITS 32
 #define TW_MOE_SPLITK_TILES 64        /* up to this many tiles a step, the waves of a workgroup split K */
 
 // ---- route ---------------------------------------------------------------------------------------------------
@@ -329,9 +324,9 @@ __global__ __launch_bounds__(256) void moe_gather_kernel(const T* __restrict__ h
 // One workgroup: a tile of 16 rows against 4 waves x NT x 16 columns of its expert's matrix W[ex] ([N][K], K a multiple
 // of 32). GLU: W and W2 are gate and up, the result glu(gate, up) goes out in the compute type; otherwise the float32
 // product. Operands go from memory straight into fragments (lane = 16 * piece + row reads 16 bytes).
-// SPLITK (steps of few rows, and of many with few units, where the tiles in use are too few to fill the chip and every one streams its expert's whole
-// matrix): the four waves share one range of NT x 16 columns and take every fourth step over K each; their sums meet in
-// LDS and are added in the order of the waves.
+// SPLITK (steps of few rows, where the tiles in use are too few to fill the chip and every one streams its expert's whole
+// matrix; some of many rows, see moe_splits_k): the four waves share one range of NT x 16 columns and take every
+// fourth step over K each; their sums meet in LDS and are added in the order of the waves.
 // MT > 1 (steps of many rows, whose experts' shares are padded to MT tiles): a workgroup takes MT tiles of one expert
 // against every fragment of the expert's matrices it reads.
 template <int N> struct MoeCount { static constexpr int value = N; };
@@ -479,7 +474,9 @@ __global__ __launch_bounds__(256) void moe_grouped_kernel(const T* __restrict__ 
       load(k, MoeCount<1>(), even);
       multiply(MoeCount<1>(), even);
     }
-  } else {
+  } else if constexpr (sizeof(T) == 4 && !GLU && (SPLITK || ACT != 0)) {
+    // (operands that outlive a step: other code, ten registers less than below; faster in float32 without a gate, 8 experts of 4,096 x
+    // 2,048, 80 tokens 585 -> 540 us, but in bfloat16, with a gate and in the last product of many rows up to 6 % slower)
     Operands now;
     for (; k + (U - 1) * k_stride < k_end; k += U * k_stride) {
       load(k, MoeCount<U>(), now);
@@ -489,6 +486,35 @@ __global__ __launch_bounds__(256) void moe_grouped_kernel(const T* __restrict__ 
       load(k, MoeCount<1>(), now);
       multiply(MoeCount<1>(), now);
     }
+  } else {
+    auto steps = [&](int k, auto count) {
+      constexpr int U = decltype(count)::value;
+      typename Elem<T>::Frag a[U][MT], b[U][NT], b2[U][NT];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+#pragma unroll
+        for (int m = 0; m < MT; ++m) a[u][m] = tw_load_frag(PLAN ? a_ptr + (k + u * k_stride) / TW_MOE_TILE
+                                                                            : a_ptr + (size_t)m * tile_elems + k + u * k_stride);
+#pragma unroll
+        for (int t = 0; t < NT; ++t) {
+          // (few rows: an expert's matrices are read once a step)
+          b[u][t] = SPLITK ? tw_load_frag_stream(w_ptr[t] + k + u * k_stride) : tw_load_frag(w_ptr[t] + k + u * k_stride);
+          if (GLU) b2[u][t] = SPLITK ? tw_load_frag_stream(w2_ptr[t] + k + u * k_stride) : tw_load_frag(w2_ptr[t] + k + u * k_stride);
+        }
+      }
+      __builtin_amdgcn_sched_barrier(0);               // (the scheduler would put each load in front of its use to save registers)
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+#pragma unroll
+        for (int t = 0; t < NT; ++t)
+#pragma unroll
+          for (int m = 0; m < MT; ++m) {
+            tw_mma16(acc[m][t], a[u][m], b[u][t]);
+            if (GLU) tw_mma16(acc2[m][t], a[u][m], b2[u][t]);
+          }
+    };
+    for (; k + (U - 1) * k_stride < k_end; k += U * k_stride) steps(k, MoeCount<U>());
+    for (; k < k_end; k += k_stride) steps(k, MoeCount<1>());
   }
   if constexpr (SPLITK) {
     __shared__ f32x4 part[GLU ? 2 : 1][3][MT][NT][64];
@@ -582,11 +608,34 @@ __global__ __launch_bounds__(256) void moe_combine_kernel(float* __restrict__ x,
   }
 }
 
+// Steps of many rows: do the waves of a workgroup better split K than the columns? (float32, 16 experts of 2,048 x 1,408 gated, two a
+// token, all launches of the experts, us, columns / K: 134 to 256 tokens 305 / 310, 268 to 440 tokens 473 / 315, 500 tokens 473 / 420; 8
+// experts, 300 tokens 298 / 299, 500 tokens 425 / 384; 4 experts, 600 tokens 278 / 355.) A range of columns a wave leaves a CU that
+// holds one workgroup a wave a SIMD, 125 us of MFMAs at K = 2,048, so what counts are the rounds of workgroups on the 256 CUs (8
+// more are still one: units without rows end at once). With K split there are four times as many, a quarter as long and 1.4
+// times as dear, every wave reading rows of its own. Where experts have one unit each, half of the units are empty, which
+// costs whole columns' rounds and next to nothing with K split. Of 222 steps of 17 to 32 units (1 to 64 experts, 256 to 4,096 x 96 to
+// 5,632) the rule is 0.8 % behind the better of the two in the mean; 6 are 4 to 11 % slower than by columns.
+// In bfloat16, whose MFMAs take a tenth of the time, K split is 17 % slower in the mean and up to 2.2 times; there only gated
+// products of long sums with one unit an expert have it (16 experts of 2,048 x 1,408, 268 to 440 tokens 121 / 93; of 4,096 x 1,408, 300
+// tokens 234 / 154; but of 1,024 x 1,408 53 / 60, and without a gate 70 / 73).
+#define TW_MOE_SPLITK_UNITS 32
+static bool moe_splits_k(bool f32, int units, long items, int X, int C, int Cd, int Fd, bool gated) {
+  if (units > TW_MOE_SPLITK_UNITS) return false;
+  const int up = units * tw_div_up(Fd, 4 * 16 * 2), down = units * tw_div_up(C, 4 * 16 * 2);
+  if (items <= 60L * X && up > 264 && (f32 || (gated && Cd >= 2048))) return true;
+  if (!f32) return false;
+  const double first = (gated ? 2.0 : 1.0) * Cd;
+  const double columns = first * tw_div_up(up, 264) + (double)Fd * tw_div_up(down, 264);
+  const double ranges = first * tw_div_up(units * tw_div_up(Fd, 16 * 2), 256) + (double)Fd * tw_div_up(units * tw_div_up(C, 16 * 2), 256);
+  return 1.4 * ranges / 4 < columns;
+}
+
 // The two grouped products of a step: kind 0 gated with the limited swish, 1 up alone with gelu, 2 gated with SiLU, 3 up alone
 // with the square of relu.
 template <typename T, int ACT>
 static void moe_products(const T* xs, const T* gate, const T* up, const T* down, const int* tile_expert, T* act, float* ys, int C,
-                         int Cd, int Fd, float limit, int tiles, bool wide, hipStream_t stream) {
+                         int Cd, int Fd, float limit, int tiles, bool wide, long items, int X, hipStream_t stream) {
   constexpr bool PLAIN = ACT == 2 || ACT == 4;
   const T* first = PLAIN ? up : gate;
   const T* second = PLAIN ? nullptr : up;
@@ -596,8 +645,7 @@ static void moe_products(const T* xs, const T* gate, const T* up, const T* down,
         xs, Cd, first, second, tile_expert, act, Fd, Fd, Cd, limit);
     moe_grouped_kernel<T, 0, 2, true><<<dim3(tiles, tw_div_up(C, 16 * 2)), 256, 0, stream>>>(
         act, Fd, down, nullptr, tile_expert, ys, C, C, Fd, 0.f);
-  } else if (wide && tiles <= TW_MOE_WIDE * TW_MOE_SPLITK_UNITS) {
-    // an expert's rows make one or two units, too few to fill the chip with a range of columns a wave: the waves split K
+  } else if (wide && moe_splits_k(sizeof(T) == 4, tiles / TW_MOE_WIDE, items, X, C, Cd, Fd, !PLAIN)) {
     moe_grouped_kernel<T, ACT, 2, true, TW_MOE_WIDE><<<dim3(tiles / TW_MOE_WIDE, tw_div_up(Fd, 16 * 2)), 256, 0, stream>>>(
         xs, Cd, first, second, tile_expert, act, Fd, Fd, Cd, limit);
     moe_grouped_kernel<T, 0, 2, true, TW_MOE_WIDE><<<dim3(tiles / TW_MOE_WIDE, tw_div_up(C, 16 * 2)), 256, 0, stream>>>(
@@ -660,7 +708,7 @@ static void moe_run(const MoeStep& s, hipStream_t stream) {
     const int tiles = s.capacity / TW_MOE_TILE;
 #define TW_MOE_PRODUCTS(ACT)                                                                                            \
     moe_products<T, ACT>((const T*)s.xs, (const T*)s.gate, (const T*)s.up, (const T*)s.down, s.tile_expert, (T*)s.act,    \
-                         s.ys, s.C, s.Cd, s.Fd, s.limit, tiles, s.wide, stream)
+                         s.ys, s.C, s.Cd, s.Fd, s.limit, tiles, s.wide, (long)s.n * s.top, s.X, stream)
     if (s.kind == 0) TW_MOE_PRODUCTS(1);
     else if (s.kind == 1) TW_MOE_PRODUCTS(2);
     else if (s.kind == 2) TW_MOE_PRODUCTS(3);

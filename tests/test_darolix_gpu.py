@@ -411,6 +411,45 @@ def test_grouped_experts_with_identities(device, dtype, n, C, X, identity, top, 
     assert torch.allclose(x.double().cpu() - base, want, atol=2e-5 if dtype == "float32" else 4e-2)
 
 
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("kind", ["silu", "gelu", "swish_limited"])
+@pytest.mark.parametrize("n,X,top,C,F", [(270, 8, 2, 800, 544), (300, 8, 2, 1056, 288), (400, 8, 2, 100, 1184), (150, 16, 2, 544, 2240), (440, 4, 2, 416, 672)])
+def test_grouped_experts_of_many_rows_and_long_sums(device, dtype, kind, n, X, top, C, F):
+    """Units of 64 rows, few enough that float32 splits K over a workgroup's waves, and one step that does not: sums whose steps fill
+    the waves' two batches of loads several times over, none, and end in the first, the second and the tail; columns that are no
+    multiple of a workgroup's. A float32 result is two sums of at most 2,240 products of terms of size 1 over the square root of
+    their number, off by some 2^-24 times 50 in the mean; bfloat16 rounds what lies between them, 2^-9 of itself."""
+    from tessweave_engine_amd.kernels import ops
+    dt = tdtype(dtype)
+    g = torch.Generator().manual_seed(n + X + C)
+    h = torch.randn(n, C, generator=g).to(device).to(dt)
+    gates, ups = ((torch.randn(X, F, C, generator=g) / math.sqrt(C)).to(dt).to(device) for _ in range(2))
+    downs = (torch.randn(X, C, F, generator=g) / math.sqrt(F)).to(dt).to(device)
+    ids = torch.stack([torch.randperm(X, generator=g)[:top] for _ in range(n)]).to(torch.int32).to(device)
+    weights = torch.softmax(torch.randn(n, top, generator=g), -1).to(device)
+    Cd, Fd = ops.moe_pad(C), ops.moe_pad(F)
+    gate, up = (torch.zeros(X, Fd, Cd, dtype=dt, device=device) for _ in range(2))
+    down = torch.zeros(X, (C + 15) // 16 * 16, Fd, dtype=dt, device=device)
+    gate[:, :F, :C], up[:, :F, :C], down[:, :C, :F] = gates, ups, downs
+    want = torch.zeros(n, C, dtype=torch.float64, device=device)
+    for e in range(X):
+        rows, choice = (ids == e).nonzero(as_tuple=True)
+        w = weights[rows, choice].double()[:, None]
+        if kind == "swish_limited":                       # (its weights are on the inputs, which are rounded)
+            y = (weights[rows, choice][:, None] * h[rows].float()).to(dt).double()
+            a, b = (y @ gates[e].double().T).clamp(max=1.5), (y @ ups[e].double().T).clamp(-1.5, 1.5)
+            mid, w = a * torch.sigmoid(1.702 * a) * (b + 1), 1.0
+        elif kind == "silu":
+            mid = torch.nn.functional.silu(h[rows].double() @ gates[e].double().T) * (h[rows].double() @ ups[e].double().T)
+        else:
+            mid = torch.nn.functional.gelu(h[rows].double() @ ups[e].double().T)
+        want.index_add_(0, rows, w * (mid @ downs[e].double().T))
+    x = torch.zeros(n, C, device=device)
+    ops.moe_experts(h, ids, weights, None if kind == "gelu" else ops.moe_blocked(gate), ops.moe_blocked(up), ops.moe_blocked(down), 1.5, x,
+                    lambda tag, shape, kind_: torch.empty(shape, dtype=kind_, device=device), kind=kind)
+    assert torch.allclose(x.double(), want, atol=2e-5 if dtype == "float32" else 4e-2)
+
+
 # ---------------------------------------------------------------------------------------------------------
 # whole models
 
