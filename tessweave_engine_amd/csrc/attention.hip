@@ -8,9 +8,10 @@
 // p iff p <= t, p < kv_len and (window == 0 or p > t - window) and (chunk == 0 or
 // p / chunk == t / chunk: chunks are counted from the sequence's start). Scores are
 // q.k * scale; softmax statistics, probabilities and the output sum are float32.
-// Masked scores are SELECTED to -inf and keys outside the sequence are loaded
-// as zeros, so whatever an unowned or reused page holds (NaN included) never
-// reaches a result.
+// Masked scores are SELECTED to -inf, and keys outside the sequence are not loaded
+// (the fast kernels put zeros in their place, the general ones the nearest key
+// inside and zeros for its value), so whatever an unowned or reused page holds
+// (NaN included) never reaches a result.
 //
 // The unit of work is a wave with a tile of 16 query ROWS that share one kv
 // head; a row is a (token, query head of the group) pair. Per 16 keys the wave
@@ -21,8 +22,8 @@
 // that the A operand of that product is one aligned load of 4 consecutive keys.
 //
 //   attn_decode_kernel   rows = the group's heads of ONE token; the sequence's
-//                        keys are split over workgroups (and over the 4 waves
-//                        of each); partial results are merged in a fixed order.
+//                        keys are split over workgroups (and over the 4 or 8
+//                        waves of each); partial results are merged in a fixed order.
 //   attn_prefill_kernel  rows = (token, head) pairs of a prompt portion; each
 //                        wave walks the keys its rows can see.
 #include "tw_common.h"
@@ -225,8 +226,9 @@ __device__ __forceinline__ void attn_store_row(const AttnArgs& a, int row, int h
 // Decode: one token per sequence. grid = (splits, kv_heads * row_tiles, n_seqs). The waves of a workgroup take key tiles in turn,
 // each with the next one's loads in flight while it multiplies. What bounds it at few and short sequences is that chain: a
 // float32 tile of head size 128 is 64 MFMAs of 32 clocks behind two rounds of latency (the page, the keys), hence eight waves
-// where their results fit LDS. float32, with a step's host work in both figures: 8 sequences of 1,500 keys, 16 heads of 128 over
-// 4: 34.9 -> 23.4 us; 64 of 1,200, 14 heads of 64 over 2: 44.9 -> 27.0 (four waves, one load after another).
+// where their results fit LDS. float32, in a captured graph, four waves with one load after another / now: 8 sequences of 1,500 keys, 16
+// heads of 128 over 4 35.5 / 24.6 us; 64 of 1,200, 14 heads of 64 over 2 44.9 / 27.6, 16 heads of 256 over 4 (a tile's loads together, no
+// tile ahead) 354 / 158; bfloat16, 8 of 1,500, heads of 256 45.4 / 27.6.
 // =====================================================================================
 template <typename T, int DTMAX, int WAVES>
 __global__ __launch_bounds__(WAVES * 64) void attn_decode_kernel(AttnArgs a) {
@@ -245,17 +247,23 @@ __global__ __launch_bounds__(WAVES * 64) void attn_decode_kernel(AttnArgs a) {
   const int* table = a.block_table + (size_t)seq * a.table_stride;
   const int D = a.head_dim, dts = D / 16;
 
-  const int hig = rt * 16 + r;                      // head within the group
-  const bool row_ok = hig < G;
-  const int head = kvh * G + hig;
-  RowTile<T, DTMAX> tile;
-  tile.init(row_ok ? (const T*)a.q + (size_t)token * a.ldq + (size_t)head * D : nullptr, D, g);
-
   const int lo = attn_first_seen(a, t);
   const int tile_lo = lo / 16, tile_hi = (kv_len + 15) / 16;     // key tiles [tile_lo, tile_hi)
   const int per_split = (tile_hi - tile_lo + a.splits - 1) / a.splits;
   const int begin = tile_lo + split * per_split;
   const int end = min(tile_hi, begin + per_split);
+  // up to four key tiles: four waves, of whose sums fewer are merged (64 keys, head size 128, 8 sequences: 10.2 -> 8.9 us)
+  const bool few = WAVES > 4 && end - begin <= 4;
+  if (few && wave >= 4) {
+    __syncthreads();
+    return;
+  }
+
+  const int hig = rt * 16 + r;                      // head within the group
+  const bool row_ok = hig < G;
+  const int head = kvh * G + hig;
+  RowTile<T, DTMAX> tile;
+  tile.init(row_ok ? (const T*)a.q + (size_t)token * a.ldq + (size_t)head * D : nullptr, D, g);
   if constexpr (DTMAX > 8) {                        // (two tiles of keys would not fit the registers)
     for (int kt = begin + wave; kt < end; kt += WAVES) tile.key_tile(a, table, kvh, kt * 16, kv_len, row_ok ? t : -1, lo, r, g);
   } else {
@@ -284,7 +292,11 @@ __global__ __launch_bounds__(WAVES * 64) void attn_decode_kernel(AttnArgs a) {
   if (wave > 0) return;
   float m = tile.m, l = tile.l;
 #pragma unroll
-  for (int w = 0; w < WAVES - 1; ++w) m = fmaxf(m, lds_ml[w][r][0]);
+  for (int w = 0; w < 3; ++w) m = fmaxf(m, lds_ml[w][r][0]);
+  if (!few) {
+#pragma unroll
+    for (int w = 3; w < WAVES - 1; ++w) m = fmaxf(m, lds_ml[w][r][0]);
+  }
   const float m_use = m == -INFINITY ? 0.f : m;
   const float own = tw_exp<T>(tile.m - m_use);
   l *= own;
@@ -294,6 +306,7 @@ __global__ __launch_bounds__(WAVES * 64) void attn_decode_kernel(AttnArgs a) {
     for (int j = 0; j < 4; ++j) tile.acc[dt][j] *= own;
 #pragma unroll
   for (int w = 0; w < WAVES - 1; ++w) {
+    if (w == 3 && few) break;
     const float f = tw_exp<T>(lds_ml[w][r][0] - m_use);
     l += lds_ml[w][r][1] * f;
 #pragma unroll
@@ -641,7 +654,10 @@ __global__ __launch_bounds__(TW_REDUCE_THREADS) void attn_decode_reduce_kernel(
 
 // =====================================================================================
 // Prefill: q_len tokens of a sequence. grid = (row tiles / 4, kv_heads, n_seqs);
-// each of the 4 waves of a workgroup takes one tile of 16 (token, head) rows.
+// each of the 4 waves of a workgroup takes one tile of 16 (token, head) rows. A tile's keys and values are requested together, which
+// takes registers (float32, heads of 128: two waves a SIMD instead of three; of 256: one) and still is what this loop, bound by
+// the latency of its loads, gains most by: 512 rows of float32, 16 heads over 4, load by load / together, 64 74 / 60 us, 128 123 / 100, 256
+// 343 / 179; behind 1,536 more keys 337 / 232, 672 / 386, 1,349 / 679.
 // =====================================================================================
 template <typename T, int DTMAX>
 __global__ __launch_bounds__(256) void attn_prefill_kernel(AttnArgs a) {

@@ -843,6 +843,27 @@ def test_attn_decode_matrix(ops, device, dtype, head_dim, heads, kv_heads):
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("head_dim", [64, 128, 192])
+def test_attn_decode_of_few_and_many_key_tiles(ops, device, dtype, head_dim):
+    """The general kernel's workgroups of four waves and of eight: tiles of 16 keys a range up to four and more, ends inside a tile."""
+    lengths, page, heads, kv_heads = [16, 48, 49, 64, 65, 79, 81, 112, 128, 129, 144], 4, 8, 2
+    torch.manual_seed(7)
+    k = [torch.randn(n, kv_heads, head_dim).to(dtype).float() for n in lengths]
+    v = [torch.randn(n, kv_heads, head_dim).to(dtype).float() for n in lengths]
+    q = torch.randn(len(lengths), heads, head_dim).to(dtype)
+    keys, values, table = build_paged(k, v, lengths, page, 260, device, dtype)
+    want = torch.stack([plain.attention(q[i:i + 1].float(), k[i], v[i], torch.tensor([n - 1]))[0] for i, n in enumerate(lengths)])
+    q_start = torch.arange(len(lengths) + 1, dtype=torch.int32, device=device)
+    kv_len = torch.tensor(lengths, dtype=torch.int32, device=device)
+    for splits in (1, 2):
+        out = torch.full((len(lengths), heads * head_dim), float("nan"), dtype=dtype, device=device)
+        ws = torch.empty(max(1, ops.attn_decode_workspace_floats(len(lengths), heads, head_dim, splits)), device=device)
+        ops.attn_decode(q.reshape(len(lengths), -1).to(device), keys, values, table, q_start, kv_len, 0, len(lengths), out, heads, kv_heads,
+                        head_dim, head_dim ** -0.5, splits=splits, workspace=ws, generic=True)
+        torch.testing.assert_close(out.float().cpu().reshape(len(lengths), heads, head_dim), want, **ATTN_TOL[dtype])
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
 def test_attn_reference_vector_tables(ops, device, dtype):
     """tests/test_engine.py:288-307 of the reference: tables [[3,1,6],[4,7]], lengths [37,19], 8 q heads on 2."""
     torch.manual_seed(5)
