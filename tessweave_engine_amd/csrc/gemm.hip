@@ -854,12 +854,22 @@ static int launch_skinny_lds_m(const T* A, long lda, const T* W, long ldw, const
 //         4096 x 2048  8.7 / 7.7, 9.1 / 8.1, 9.6 / 8.8      2048 x 4096  8.6 / 8.1, 9.2 / 9.4, 9.6 / 10.9
 //    float32 896 x 896  7.7 / 6.6, 8.2 / 7.3, 8.6 / 8.0     2560 x 2048  10.9 / 9.1, 11.7 / 10.3, 12.2 / 11.6
 //         2048 x 2048  9.2 / 8.7, 9.7 / 9.8, 10.2 / 11.2    3584 x 3584  17.6 / 15.0, 17.8 / 16.3, 18.8 / 18.9
+// Between 2,048 and 3,584 columns the lines are the other kernel's: it gets 1.5 us slower where it has more workgroups than CUs, and
+// a microsecond for every 8 k-steps of a range that begin; this one where its 16 waves begin another batch, at 128 and 192 k-steps.
+// (8 rows: bf16 2304 x 2560, 180 workgroups of 16 k-steps, 8.3 / 9.0, x 2816, of 17.6, 9.3 / 9.1; 2560 x 3328, 240, 10.1 / 9.8, x 3584, 280, 10.5 / 9.9;
+// 2816 x 3328 11.4 / 10.0. float32 2560 x 1536, 240 workgroups, 9.6 / 9.8, x 1792, 280, 11.5 / 10.4, x 2304, 144 k-steps, 12.3 / 12.9; 3072 x 2816, 17.6 k-steps
+// a range, 15.1 / 13.7, x 3328, 208, 15.4 / 16.3.)
 static bool narrow_pays(int M, int N, int K, int epf, bool glu, bool sums) {
   const int steps = tw_div_up(K / epf, 4), groups = glu ? N / 32 : tw_div_up(N, 16);
   if (sums) {
     if (groups > 256 || steps < 16) return false;
     if (steps < 32 || (epf == 4 && steps <= 64 && groups >= 48)) return true;
-    return M <= 8 && groups >= (epf == 4 ? 160 : 128) && steps <= (epf == 4 ? 224 : 112);
+    if (M > 8) return false;
+    const int ranges = skinny_lds_splits(N, K, epf), workgroups = tw_div_up(N, 64) * ranges;
+    const bool second = workgroups > 256;                                 // more than one of the other kernel's workgroups a CU
+    if (epf == 8) return groups >= 128 && steps <= 112 && (steps <= 72 || second || steps > 16 * ranges);
+    if (groups < 160) return false;
+    return steps <= 128 ? second : steps <= 192 ? groups >= 224 || steps > 16 * ranges : steps <= 224 && (groups >= 240 || steps > 24 * ranges);
   }
   if (groups <= 256) return steps <= (M > 8 && groups < 96 && !glu ? 96 : 128);
   if (glu) return steps >= 28 && steps <= (groups < 512 && epf == 4 ? 32 : 64) && (M <= 8 || groups >= 512);

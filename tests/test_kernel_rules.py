@@ -16,3 +16,12 @@ def test_products_that_one_kernel_does_not_take_keep_the_plan_of_the_other(m, n,
     for cols in (n, n + 4):
         named = lib.tw_linear_partial_splits_rows(BF16, 1, m, cols, k, k)
         assert lib.tw_linear_workspace_bytes(BF16, m, cols, k) >= named * m * cols * 4
+
+
+@pytest.mark.parametrize("dtype,m,n,k,whole", [(BF16, 8, 2048, 2304, True), (BF16, 8, 2304, 2560, False), (BF16, 8, 2304, 2816, True), (BF16, 1, 2304, 3584, False),
+                                               (BF16, 8, 2560, 3584, True), (BF16, 9, 2560, 3584, False), (F32, 8, 2560, 1536, False), (F32, 8, 2560, 1792, True),
+                                               (F32, 1, 2560, 2304, False), (F32, 8, 3072, 2816, True), (F32, 8, 3072, 3328, False), (F32, 8, 3584, 3584, True),
+                                               (F32, 8, 3584, 3328, False), (F32, 9, 3584, 2048, False)])
+def test_sums_for_the_next_kernel_over_the_whole_of_k(dtype, m, n, k, whole):
+    """Up to 8 rows and a long K: K ranges stay where they are the faster form, one workgroup a CU of whole stages."""
+    assert (library().tw_linear_partial_splits_rows(dtype, 1, m, n, k, k) == 1) == whole
