@@ -45,8 +45,10 @@ __device__ __forceinline__ float qf_turned(const float* row, const float* w, flo
   return first ? __fmaf_rn(mine, c, -__fmul_rn(theirs, s)) : __fmaf_rn(mine, c, __fmul_rn(theirs, s));
 }
 
-// A workgroup a token, of 1,024 threads where the tokens do not fill the chip: a thread's elements are one chain of loads, of
-// divisions by the head size and of stores behind the other (one token of 16 + 4 heads of 128, in a trace: 12.7 -> 6.8 us).
+// A workgroup a token, of 1,024 threads where the tokens do not fill the chip and a row has elements for them: a thread's elements are
+// one chain of loads, of divisions by the head size and of stores behind the other. In a captured graph, 256 / 1,024 threads, 1, 64 and 256
+// tokens, us: 16 + 4 heads of 128 8.0 / 5.3, 8.4 / 5.8, 8.9 / 6.3; 8 + 2 of 64 4.6 / 4.2, 5.1 / 4.7, 5.2 / 4.9; 4 + 4 of 64 4.3 / 4.4, 4.8 / 4.9, 4.9 / 5.2; 4 + 1
+// of 32 4.0 / 4.1, 4.4 / 4.6, 4.5 / 4.8.
 template <typename T, int THREADS>
 __global__ __launch_bounds__(THREADS) void qk_finish_kernel(QkFinishArgs a) {
   __shared__ float lds[16];
@@ -95,7 +97,7 @@ extern "C" int tw_qk_finish(int dtype, const float* src, long ld, int q_col, int
   QkFinishArgs a{src, ld, q_col, k_col, wq, wk, cos_t, sin_t, q_out, ld_q, keys, values, slots, H, G, D, Dp, rot, pairing,
                  page_size, eps};
   TW_REQUIRE(dtype == TW_DTYPE_BF16 || dtype == TW_DTYPE_F32);
-  if (n <= 256) {
+  if (n <= 256 && (long)(H + G) * D > 512) {
     if (dtype == TW_DTYPE_BF16) qk_finish_kernel<bf16_t, 1024><<<n, 1024, 0, stream>>>(a);
     else qk_finish_kernel<float, 1024><<<n, 1024, 0, stream>>>(a);
   } else if (dtype == TW_DTYPE_BF16) {
