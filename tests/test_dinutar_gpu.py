@@ -71,9 +71,9 @@ def test_hashed_pair_embedding_carries_the_last_token(device, dtype):
 
 
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
-@pytest.mark.parametrize("C", [4, 70, 2048, 4096, 4104, 8192, 8200])
+@pytest.mark.parametrize("C", [4, 70, 256, 264, 2048, 4096, 4104, 8192, 8200])
 def test_hashed_pair_embedding_of_every_width(device, dtype, C):
-    """Rows of whole 16-byte pieces and not, one piece, as many as the threads keep (4,096 float32 values, 8,192 bfloat16) and more.
+    """Rows of whole 16-byte pieces and not, too few for pieces and just enough, as many as the threads keep (4,096 float32 values, 8,192 bfloat16) and more.
     float32 sums of at most 8,200 squares, off by 2^-24 of themselves a term at the very most: 5e-4 of the norm, in practice 1e-6."""
     from tessweave_engine_amd.kernels import ops
     dt = tdtype(dtype)
