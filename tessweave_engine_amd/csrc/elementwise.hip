@@ -5,10 +5,11 @@
 
 // ---- embedding: x[n, :] = float(E[ids[n], :]) ------------------------------------
 // A negative id -1 - k stands for feed[k]: a token that an earlier kernel on this stream wrote
-// the sampler's output of the step before), which the host has not read yet.
-// VEC: rows of whole 16-byte pieces, a thread one piece of a row (grid.y covers a row): behind its id a row is one trip to memory.
-// Element by element, a workgroup a row, it was a chain of them: 64 rows of 3,584 in bfloat16 9.2 us in a trace, 8 of 2,048 6.5;
-// now 4.7 and 3.4.
+// (the sampler's output of the step before), which the host has not read yet.
+// VEC: rows of whole groups of four elements, a thread one group of a row (grid.y covers a row): behind its id a row is one trip to
+// memory. Element by element, a workgroup a row, it was a chain of them. (Four and not the eight bfloat16 values of 16 bytes: the float32
+// results, twice as many bytes, then leave in one store of neighbouring lanes.) bfloat16, in a
+// captured graph, element by element / now: 64 rows of 3,584 3.6 / 2.4 us, 2,048 of 2,048 5.5 / 4.9 (in eights 6.1).
 template <typename T, bool VEC>
 __global__ void embed_gather_kernel(const int* __restrict__ ids, const T* __restrict__ table,
                                     float* __restrict__ out, int hidden, int vocab,
@@ -20,13 +21,11 @@ __global__ void embed_gather_kernel(const int* __restrict__ ids, const T* __rest
   const T* row = table + (size_t)id * hidden;
   float* dst = out + (size_t)n * hidden;
   if constexpr (VEC) {
-    constexpr int EPF = Elem<T>::kPerFrag;
-    const int h = (blockIdx.y * blockDim.x + threadIdx.x) * EPF;
+    typedef T Four __attribute__((ext_vector_type(4)));
+    const int h = (blockIdx.y * blockDim.x + threadIdx.x) * 4;
     if (h >= hidden) return;
-    const auto v = tw_load_frag(row + h);
-#pragma unroll
-    for (int k = 0; k < EPF; k += 4)
-      *reinterpret_cast<f32x4*>(dst + h + k) = f32x4{tw_to_float(v[k]), tw_to_float(v[k + 1]), tw_to_float(v[k + 2]), tw_to_float(v[k + 3])};
+    const Four v = *reinterpret_cast<const Four*>(row + h);
+    *reinterpret_cast<f32x4*>(dst + h) = f32x4{tw_to_float(v[0]), tw_to_float(v[1]), tw_to_float(v[2]), tw_to_float(v[3])};
   } else {
     for (int h = threadIdx.x; h < hidden; h += blockDim.x) dst[h] = tw_to_float(row[h]);
   }
@@ -35,9 +34,8 @@ __global__ void embed_gather_kernel(const int* __restrict__ ids, const T* __rest
 template <typename T>
 static void launch_embed_gather(const int* ids, const void* table, float* out, int n, int hidden, int vocab, const int* feed,
                                 int feed_count, hipStream_t stream) {
-  constexpr int EPF = Elem<T>::kPerFrag;
-  const int shares = tw_div_up(hidden / EPF, 256);
-  if (hidden % EPF == 0 && shares <= 65535 && (((uintptr_t)table | (uintptr_t)out) & 15) == 0)
+  const int shares = tw_div_up(hidden / 4, 256);
+  if (hidden % 4 == 0 && shares <= 65535 && (uintptr_t)table % (4 * sizeof(T)) == 0 && (uintptr_t)out % 16 == 0)
     embed_gather_kernel<T, true><<<dim3(n, shares), 256, 0, stream>>>(ids, (const T*)table, out, hidden, vocab, feed, feed_count);
   else
     embed_gather_kernel<T, false><<<n, 256, 0, stream>>>(ids, (const T*)table, out, hidden, vocab, feed, feed_count);
