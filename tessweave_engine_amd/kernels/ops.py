@@ -376,8 +376,8 @@ def linear_act_few_pays(x, weight):
     """Is `linear_act_few` there for these operands, and faster than the product's split-K sums with the activation behind
     them? (up to 16 rows, shuffled weights, a workgroup with the whole of K)"""
     rows = x.shape[0]
-    return (isinstance(weight, ShuffledWeight) and 0 < rows <= 16 and x.data_ptr() % 16 == 0
-            and (rows == 1 or x.stride(0) % (16 // x.element_size()) == 0)
+    ld = x.stride(0) if rows > 1 else max(x.stride(0), x.shape[1])
+    return (isinstance(weight, ShuffledWeight) and 0 < rows <= 16 and x.data_ptr() % 16 == 0 and ld % (16 // x.element_size()) == 0
             and bool(library().tw_linear_act_few_pays(dtype_id(x.dtype), rows, *weight.shape)))
 
 

@@ -1,6 +1,8 @@
 """The rules by which kernels are chosen, asked on the host: no GPU is needed to ask."""
 import pytest
+import torch
 
+from tessweave_engine_amd.kernels import ops
 from tessweave_engine_amd.kernels.lib import library
 
 F32, BF16 = 0, 1
@@ -25,3 +27,12 @@ def test_products_that_one_kernel_does_not_take_keep_the_plan_of_the_other(m, n,
 def test_sums_for_the_next_kernel_over_the_whole_of_k(dtype, m, n, k, whole):
     """Up to 8 rows and a long K: K ranges stay where they are the faster form, one workgroup a CU of whole stages."""
     assert (library().tw_linear_partial_splits_rows(dtype, 1, m, n, k, k) == 1) == whole
+
+
+@pytest.mark.parametrize("rows", [1, 8])
+def test_an_activation_behind_few_rows_asks_for_what_its_kernel_takes(rows):
+    """Rows 2,050 elements apart are no multiple of 16 bytes apart, which the kernel refuses of a single row too."""
+    weight = ops.shuffle_weight(torch.zeros(4096, 2048, dtype=torch.bfloat16))
+    assert ops.linear_act_few_pays(torch.zeros(rows, 2048, dtype=torch.bfloat16), weight)
+    assert ops.linear_act_few_pays(torch.zeros(rows + 1, 2056, dtype=torch.bfloat16)[:rows, :2048], weight)
+    assert not ops.linear_act_few_pays(torch.zeros(rows + 1, 2050, dtype=torch.bfloat16)[:rows, :2048], weight)
