@@ -445,7 +445,8 @@ def test_linear_of_waves_in_turns(ops, device, m, n, k):
     """bfloat16 tiles of every shape: one k-tile, fewer and as many as a stage ring holds and no multiple of it; rows and columns
     that end inside a tile, a wave's tile and a group of 16 columns; more tiles than CUs (a workgroup's second and third tile: its
     first waits allow for the stores before it, its bias lies in the other place); K ranges of unequal lengths; plain, float32 with
-    a bias and a residual in place, activations, gated. A float32 sum of K exact products, in any order, is off by at most K 2^-24
+    a bias and a residual in place, activations, a gated one of one tile. A float32 sum of K exact products, in any order, is off by
+    at most K 2^-24
     of the sum of their sizes, and a bfloat16 result by another 2^-8 of itself."""
     x = rand((m, k), torch.bfloat16, device, 1.0, seed=1)
     w = rand((n, k), torch.bfloat16, device, 0.05, seed=2)
@@ -486,6 +487,43 @@ def test_linear_of_waves_in_turns(ops, device, m, n, k):
         value = want + bias
         slope = 2 * value.abs() + 1.2                          # (of either; the square of what the sum is off by is in the 0.1)
         check(out, act(value), near * slope + 2.0 ** -20 * (1 + value.abs()))
+
+
+@pytest.mark.parametrize("biased", [False, True])
+@pytest.mark.parametrize("m,n,k", [(4200, 4128, 256), (4100, 4640, 320), (4353, 4320, 448)])
+def test_linear_glu_of_waves_in_turns_goes_on_to_more_tiles(ops, device, m, n, k, biased):
+    """Gated products of more tiles than CUs in every shape, K as long as every ring of stages and no multiple of it, rows and columns
+    that end inside a tile: a workgroup's second tile begins with copies made during the first, waits past its stores and has its
+    bias in the other place. Bounds as in test_linear_of_waves_in_turns."""
+    x = rand((m, k), torch.bfloat16, device, 1.0, seed=1)
+    w = rand((n, k), torch.bfloat16, device, 0.05, seed=2)
+    bias = rand((n,), torch.float32, device, 0.5, seed=3) if biased else None
+    shuffled = ops.shuffle_weight(w)
+    want = x.double() @ w.double().T
+    near = (k + 4) * 2.0 ** -24 * (x.double().abs() @ w.double().abs().T + 4.0)
+    (g, u), (g_near, u_near) = (want if bias is None else want + bias).view(m, n // 32, 2, 16).unbind(2), near.view(m, n // 32, 2, 16).unbind(2)
+    value = torch.nn.functional.silu(g) * u
+    bound = 1.1 * g_near * (u.abs() + u_near) + g.abs() * u_near + 2.0 ** -20 * (g * u).abs() + 2.0 ** -8 * value.abs()
+    for force in (ops.GEMM_AUTO, ops.GEMM_TILED, ops.GEMM_TILED_WIDE, ops.GEMM_TILED_256, ops.GEMM_TILED_256X192):
+        gated = torch.full((m + 1, n // 2), float("nan"), dtype=torch.bfloat16, device=device)
+        ops.linear_glu(x, shuffled, gated[:m], bias=bias, force=force)
+        assert bool(((gated[:m].double().view(m, n // 32, 16) - value).abs() <= bound).all()) and bool(gated[m:].isnan().all())
+
+
+@pytest.mark.parametrize("m,n,k", [(300, 520, 448), (1100, 2056, 1024), (2049, 264, 3584)])
+def test_linear_of_waves_in_turns_rounds_as_the_other_tiles(ops, device, m, n, k):
+    """One sum over the whole of K is the same bits in every tile: 16x16x32 MFMAs by waves in turns (a result of 16-byte rows), 32x32x16
+    ones copied into LDS or staged through registers (a result one element off that)."""
+    x = rand((m, k), torch.bfloat16, device, 1.0, seed=1)
+    shuffled = ops.shuffle_weight(rand((n, k), torch.bfloat16, device, 0.05, seed=2))
+    seen = []
+    for force in (ops.GEMM_TILED, ops.GEMM_TILED_WIDE, ops.GEMM_TILED_256, ops.GEMM_TILED_256X192):
+        for at in (0, 1):
+            out = torch.full((m, n + 4), float("nan"), device=device)[:, at:at + n]
+            ops.linear(x, shuffled, out, force=force)
+            seen.append(out)
+    for out in seen[1:]:
+        assert torch.equal(out, seen[0])
 
 
 @pytest.mark.parametrize("k", [64, 128, 192, 320, 384, 512, 576])
