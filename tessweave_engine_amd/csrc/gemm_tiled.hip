@@ -486,12 +486,11 @@ __global__ __launch_bounds__(256) void gemm_tiled_kernel(const T* __restrict__ A
 }
 
 // =====================================================================================
-// bfloat16, shuffled weights, K an odd multiple of 32 (or rows of the result that are no multiple of 16 bytes: all else goes
-// to gemm_turns_kernel below): tiles whose operands are copied from global
-// memory straight into LDS (`global_load_lds_dwordx4`: lane l's 16 bytes land at the wave's LDS
-// base + 16 l, from any address the lane names). No staging registers, no LDS write instructions.
-// Workgroup = 4 waves in a 2x2 grid, wave tile (32*WM) x (32*WN): 128x128 (two workgroups a CU),
-// 128x256, 256x256 (one a CU, the accumulators in AGPRs).
+// bfloat16, shuffled weights, K a multiple of 32, where gemm_turns_kernel below does not take the product (an odd multiple of 32, rows of
+// the result or a residual that are not 16 bytes apart, a bias over a K shorter than the stages: turns_takes) or is the slower
+// one (turns_pay): tiles whose operands are copied from global memory straight into LDS (buffer loads of 16 bytes a lane, which land at
+// the wave's LDS base + 16 l, from any 32-bit offset the lane names). No staging registers, no LDS write instructions.
+// Workgroup = 4 waves in a 2x2 grid, wave tile (32*WM) x (32*WN): 128x256, 256x192, 256x256 (one a CU).
 //
 // A k-tile is 32 elements of K (one k-step of the shuffled layout). What limits this kernel is the
 // number of 128-byte lines a CU's vector cache can have on their way from L2; a copy that takes 64 bytes
@@ -510,9 +509,8 @@ __global__ __launch_bounds__(256) void gemm_tiled_kernel(const T* __restrict__ A
 // =====================================================================================
 typedef __attribute__((address_space(3))) void* tw_lds_ptr;
 // Copies of 16 bytes a lane from global memory straight into LDS, as BUFFER loads: base + lane's offset + the wave's offset, so
-// that a copy takes no address arithmetic. As global loads, with a 64-bit address a lane, four waves of a CU issued them at 30 bytes
-// a clock, and with two waves a SIMD taking turns (below) a k-tile of 256x256x64 took 2,540 clocks of which the MFMAs are 2,048;
-// as buffer loads it takes 2,080. Offsets within a tile's operands are 32-bit (checked where the kernels are launched).
+// that a copy takes no address arithmetic (as global loads, with a 64-bit address a lane, they held up the waves that take turns
+// below). Offsets within a tile's operands are 32-bit: asked before the kernels are chosen or where they are launched.
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t tw_buffer(const void* base) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, 0x7fffffff, 0x00020000);
 }
@@ -749,13 +747,13 @@ __global__ __launch_bounds__(256) void gemm_dma_kernel(const bf16_t* __restrict_
 // every wave issues all of them (rows and columns outside the result have an offset outside the buffer, which the memory unit
 // drops).
 //
-// What bounds it, 256x256 tiles: power. The loop keeps the matrix units busy for 98 % of its clocks at 8,192 x 8,192 and larger, and
-// the clock falls to 1.5 GHz (1.65 with copies as global loads, where they are busy for 80 %); so what costs energy
-// costs time. 16x16x32 MFMAs run 10 % faster than 32x32x16 here (they read and write their accumulators half as often). Smaller
-// tiles copy more per MFMA (128x128: 32 KB a 512 clocks) and are bound by that: four waves issue buffer copies at some 33 bytes a
-// clock and CU, eight at more, so 128x128 tiles issue half of a phase's copies between its MFMAs (2,048 x 2,048 x 2,048 23.9 ->
-// 22.1 us; 256x256 tiles get 2 % slower by it).
-// bfloat16, the four-wave kernels -> this one, us (one card, weights from HBM; the same shapes by torch's library in parentheses):
+// What bounds it, 256x256 tiles: power first. From 8,192 rows on the matrix units are busy for 77 to 84 % of the waves' lifetime, and
+// the clock over it is 1.66 to 1.76 GHz of 2.4; at 2,048 rows 73 to 81 % at 1.74 to 1.92 (counters; the rest is the first tile's
+// copies, the last one's stores and a last round that is not full). So what costs energy costs time: 16x16x32 MFMAs run 6 % faster
+// than 32x32x16 here (they read and write their accumulators half as often). Smaller tiles copy more per MFMA (128x128: 32 KB a
+// 512 clocks; 128x256 63 % busy) and are bound by that, so 128x128 tiles issue half of a phase's copies between its MFMAs (2,048 x
+// 2,048 x 2,048 23.9 -> 22.1 us; 256x256 tiles get 2 % slower by it).
+// bfloat16, the four-wave kernels -> this one, us (one card, weights from HBM; torch's library on another run in parentheses):
 //   2,048 x 4,608 x 3,584    75.5 -> 64.4 (66)      2,048 x 37,888 x 3,584 gated    527 -> 455
 //   2,048 x 3,584 x 3,584    59.4 -> 54.2 (55)      8,192 x 37,888 x 3,584 gated  1,878 -> 1,571
 //   2,048 x 3,584 x 18,944    268 -> 240 (350)        536 x 27,648 x 5,120 gated    217 -> 188
