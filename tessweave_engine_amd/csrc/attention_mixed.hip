@@ -453,30 +453,303 @@ __global__ __launch_bounds__(WMAX * 64) void attn_mixed_kernel(MixedAttnArgs a) 
   }
 }
 
-// Merge the partial results of a tile's key ranges, in index order. grid (tiles, n_seqs, H).
+// One query token a sequence (a decode step): the query HEADS of a key/value head are the rows of the matrix unit's tile instead
+// of 16 tokens of which one is there, and a wave has one key/value head. Per NT key tiles it forms S = Q K^T, leaves its heads'
+// raw scores in LDS ([key][head]), and after one barrier reads all heads' scores of a key, four neighbouring heads a lane: the A
+// operand of the mixing product S^T talk^T, whose result, its own heads across and keys down, is what the softmax and
+// O^T += V^T P^T want. Nothing is shared behind the mixing, so waves keep and store their own heads' sums. Without mixing
+// S^T = K Q^T is formed directly and waves never meet. Distance slopes are mixed once (sum_g talk[h][g] slope_g) and come off the
+// mixed scores.
+// What bounds it is a wave's chain: the trips to memory (everything NT tiles read is requested together and a group ahead) and
+// its instructions, about 2 ns each with one wave a SIMD. 16-token tiles whose waves share the heads out walk a range's key
+// tiles in turn at 4 us each; one wave with all heads of a key tile (no LDS, the products with other heads' keys thrown away)
+// had five times the instructions and was as slow. With the merge, in a chain of such calls, bfloat16, heads of 128 (us, tiles of
+// tokens / here): 16 on 4, window 1,024, one sequence 26.6 / 13.4, 32 sequences 45.2 / 25.6; 24 on 4, 2,048 keys 57.0 / 14.7, 64
+// sequences of 1,500 208 / 41; without mixing 26.7 / 11.1; float32, 16 on 4, 800 keys 57.7 / 18.6. 8 heads of 64 on 8, 8 sequences
+// of 2,050: 29.9 / 21.5. Errors against 64 bits: as before in bfloat16, 0.5 to 1.0 times as large in float32.
+template <typename T, int S, int NT, bool TALK>
+__global__ __launch_bounds__(512) void attn_mixed_one_kernel(MixedAttnArgs a) {
+  typedef typename Elem<T>::Frag Frag;
+  typedef typename MxQuad<T>::Type Quad;
+  constexpr int EPF = Elem<T>::kPerFrag;
+  constexpr int KC = S / (4 * EPF), VT = S / 16;             // k-steps of a key, 16-element tiles of a value
+  extern __shared__ __attribute__((aligned(16))) unsigned char lds_raw[];
+  const int lane = threadIdx.x & 63, kv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int r = lane & 15, g = lane >> 4;
+  const int H = a.H, G = a.G, P = a.P;
+  const int seq = a.seq0 + blockIdx.y;
+  const int q0 = a.q_start[seq];
+  if (a.q_start[seq + 1] <= q0) return;
+  const int kv_len = a.kv_len[seq], pos = kv_len - 1;       // the token's own position
+  const int* table = a.block_table + (size_t)seq * a.table_stride;
+  const int per_kv = H / G, head = kv * per_kv + r;         // lane r's query head, where r < per_kv
+  const bool mine = r < per_kv;
+
+  // ---- this workgroup's key tiles, numbered without the gap between the kept first keys and the window (as in attn_mixed_kernel) ----
+  const int lo = a.window > 0 ? max(0, pos - a.window + 1) : 0;
+  const int keep = a.window > 0 ? a.keep : 0;
+  const int win_lo = lo / 16;
+  const int kept = min((keep + 15) / 16, win_lo), skip = win_lo - kept;
+  int tile_lo = 0, tile_hi = pos / 16 + 1 - skip;
+  if (a.splits > 1) {
+    const int per = (tile_hi + a.splits - 1) / a.splits;
+    tile_lo = blockIdx.z * per;
+    tile_hi = min(tile_hi, tile_lo + per);
+  }
+  auto key_tile = [&](int v) { return v < kept ? v : v + skip; };
+  // Page sizes are multiples of 16: a key tile lies in one page, whose number and addresses are the whole wave's (scalar). A
+  // tile of the range holds a key that is seen, so its page is held; what else lies in it is masked. Tiles past the range are
+  // its last one again, masked whole.
+  const uint32_t k_off = r * S + g * EPF, page_size = (uint32_t)G * P * S;
+  const uint32_t v_off = r * P + 4 * g;
+  Frag kf[NT][KC];
+  Quad vq[NT][VT];
+  int page[NT];
+  auto find_pages = [&](int v0) {
+#pragma unroll
+    for (int i = 0; i < NT; ++i) {
+      const int p = key_tile(min(v0 + i, tile_hi - 1)) * 16;
+      page[i] = max(0, table[p >> a.page_shift]);
+    }
+  };
+  auto place_of = [&](int v) { return (key_tile(min(v, tile_hi - 1)) * 16) & (P - 1); };
+  auto request_keys = [&](int v0) {
+#pragma unroll
+    for (int i = 0; i < NT; ++i) {
+      const T* base = (const T*)a.keys + ((uint64_t)(uint32_t)page[i] * page_size + (uint32_t)((kv * P + place_of(v0 + i)) * S));
+#pragma unroll
+      for (int st = 0; st < KC; ++st) kf[i][st] = tw_load_frag(base + k_off + st * 4 * EPF);
+    }
+  };
+  auto request_values = [&](int v0) {
+#pragma unroll
+    for (int i = 0; i < NT; ++i) {
+      const T* base = (const T*)a.values + ((uint64_t)(uint32_t)page[i] * page_size + (uint32_t)(kv * S * P + place_of(v0 + i)));
+#pragma unroll
+      for (int dt = 0; dt < VT; ++dt) vq[i][dt] = *reinterpret_cast<const Quad*>(base + (uint32_t)(dt * 16 * P) + v_off);
+    }
+  };
+  if (tile_lo < tile_hi) {
+    find_pages(tile_lo);
+    request_keys(tile_lo);
+    request_values(tile_lo);
+  }
+  // ---- the heads' queries, their rows of the mixing matrix, their slopes --------------------------------------------------
+  Frag qf[KC];
+#pragma unroll
+  for (int st = 0; st < KC; ++st) {
+    const Frag f = tw_load_frag((const T*)a.q + (size_t)q0 * a.ldq + (size_t)min(head, H - 1) * S + (st * 4 + g) * EPF);
+    qf[st] = mine ? f : Elem<T>::zero();
+  }
+  constexpr int CT = TALK ? 2 : 1;                           // up to 32 heads, 16 a product
+  f32x4 talk[CT];
+  float slope = 0.f;
+  if constexpr (TALK) {
+#pragma unroll
+    for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int from = ct * 16 + 4 * g + e;
+        const float w = a.talk[min(head, H - 1) * H + min(from, H - 1)];
+        talk[ct][e] = mine && from < H ? w : 0.f;
+        if (a.slopes) slope = fmaf(talk[ct][e], a.slopes[min(from, H - 1)], slope);
+      }
+    if (a.slopes) slope = tw_rows_sum(slope);
+  } else if (a.slopes) {
+    slope = a.slopes[min(head, H - 1)];
+  }
+  const bool with_sink = a.sink != nullptr && blockIdx.z == 0;
+  float m = with_sink ? a.sink[min(head, H - 1)] : -INFINITY;     // the sink: a key of score sink_h and value zero
+  float l = with_sink ? 1.f : 0.f;
+  f32x4 acc[VT];
+#pragma unroll
+  for (int dt = 0; dt < VT; ++dt) acc[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const int row_floats = (H + 3) / 4 * 4 + 4;                // (rows of whole 16-byte reads)
+  float* raw = (float*)lds_raw;
+
+  for (int t = tile_lo; t < tile_hi; t += NT) {
+    const bool more = t + NT < tile_hi;
+    // ---- scores: lane (r, g) then holds its head r against keys 4g + e of every tile -----------------------------------------
+    f32x4 s[NT];
+#pragma unroll
+    for (int i = 0; i < NT; ++i) {
+      s[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int st = 0; st < KC; ++st) {
+        if constexpr (TALK) tw_mma16(s[i], qf[st], kf[i][st]);
+        else tw_mma16(s[i], kf[i][st], qf[st]);
+      }
+    }
+    if (more) {
+      find_pages(t + NT);
+      request_keys(t + NT);
+    }
+    if constexpr (TALK) {
+      // (here lane (r, g) holds key r against the wave's heads 4g + e)
+      if (per_kv % 4 == 0) {
+        if (4 * g < per_kv) {
+#pragma unroll
+          for (int i = 0; i < NT; ++i) *reinterpret_cast<f32x4*>(raw + (i * 16 + r) * row_floats + kv * per_kv + 4 * g) = s[i];
+        }
+      } else {
+#pragma unroll
+        for (int i = 0; i < NT; ++i)
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            if (4 * g + e < per_kv) raw[(i * 16 + r) * row_floats + kv * per_kv + 4 * g + e] = s[i][e];
+      }
+      __syncthreads();
+#pragma unroll
+      for (int i = 0; i < NT; ++i) {
+        s[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+        // (heads 4g + 3 first, 4g last: the first head's product is then added to the others' sum and not rounded by itself)
+#pragma unroll
+        for (int ct = CT - 1; ct >= 0; --ct)
+          if (ct * 16 < H) {
+            f32x4 all = *reinterpret_cast<const f32x4*>(raw + (i * 16 + r) * row_floats + min(ct * 16 + 4 * g, (H - 1) / 4 * 4));
+#pragma unroll
+            for (int e = 3; e >= 0; --e)
+              s[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(ct * 16 + 4 * g + e < H ? all[e] : 0.f, talk[ct][e], s[i], 0, 0, 0);
+          }
+      }
+      raw = (float*)lds_raw + (raw == (float*)lds_raw ? NT * 16 * row_floats : 0);
+    }
+    // ---- mask, softmax ---------------------------------------------------------------------------------------------------------
+    float mx = -INFINITY;
+#pragma unroll
+    for (int i = 0; i < NT; ++i) {
+      const int p0 = key_tile(min(t + i, tile_hi - 1)) * 16;
+      // (a wave's branch: masks only where a key of the tile is not seen)
+      const bool interior = t + i < tile_hi && p0 + 15 <= pos && (p0 >= lo || p0 + 15 < keep);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) s[i][e] = s[i][e] * a.scale - slope * (float)(pos - (p0 + 4 * g + e));
+      if (!interior) {
+        bool seen[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int p = p0 + 4 * g + e;
+          seen[e] = t + i < tile_hi && p <= pos && (p >= lo || p < keep);
+          s[i][e] = seen[e] ? s[i][e] : -INFINITY;
+        }
+#pragma unroll
+        for (int dt = 0; dt < VT; ++dt) {
+          if constexpr (EPF == 8) {
+            u32x2 bits = __builtin_bit_cast(u32x2, vq[i][dt]);
+#pragma unroll
+            for (int h = 0; h < 2; ++h) bits[h] &= (seen[2 * h] ? 0x0000ffffu : 0u) | (seen[2 * h + 1] ? 0xffff0000u : 0u);
+            vq[i][dt] = __builtin_bit_cast(Quad, bits);
+          } else {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) vq[i][dt][e] = seen[e] ? vq[i][dt][e] : 0.f;
+          }
+        }
+      }
+#pragma unroll
+      for (int e = 0; e < 4; ++e) mx = fmaxf(mx, s[i][e]);
+    }
+    mx = tw_rows_max(mx);
+    const float m_new = fmaxf(m, mx);
+    const float m_use = m_new == -INFINITY ? 0.f : m_new;
+    const float alpha = mx_exp<T>(m - m_use);
+    float sum = 0.f;
+#pragma unroll
+    for (int i = 0; i < NT; ++i) {
+      float part = 0.f;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        s[i][e] = mx_exp<T>(s[i][e] - m_use);
+        part += s[i][e];
+      }
+      sum += part;
+    }
+    l = l * alpha + tw_rows_sum(sum);
+    m = m_new;
+    if (__builtin_amdgcn_ballot_w64(alpha != 1.f) != 0) {
+#pragma unroll
+      for (int dt = 0; dt < VT; ++dt)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc[dt][e] *= alpha;
+    }
+    // ---- O^T += V^T P^T ----------------------------------------------------------------------------------------------------------
+#pragma unroll
+    for (int i = 0; i < NT; ++i)
+#pragma unroll
+      for (int dt = 0; dt < VT; ++dt) tw_mma16_k4(acc[dt], vq[i][dt], s[i]);
+    if (more) request_values(t + NT);
+  }
+
+  // ---- results: lane (r, g) holds out[head r][16 dt + 4 g + e] -------------------------------------------------------------------
+  if (!mine) return;
+  if (a.splits == 1) {
+    const float inv = l > 0.f ? a.out_scale / l : 0.f;
+    T* dst = (T*)a.out + (size_t)q0 * a.ldo + (size_t)head * S + 4 * g;
+#pragma unroll
+    for (int dt = 0; dt < VT; ++dt)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) dst[dt * 16 + e] = tw_from_float<T>(acc[dt][e] * inv);
+  } else {
+    float* dst = a.part + (((size_t)blockIdx.y * a.splits + blockIdx.z) * H + head) * (S + 2);
+#pragma unroll
+    for (int dt = 0; dt < VT; ++dt)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) dst[dt * 16 + 4 * g + e] = acc[dt][e];
+    if (g == 0) {
+      dst[S] = m;
+      dst[S + 1] = l;
+    }
+  }
+}
+
+// Merge the partial results of a tile's key ranges, in index order. grid (tiles, n_seqs, H). The ranges' weights are formed
+// once a row in LDS (threads side by side: one after the other, every thread for itself, 16 ranges took 9 us of a decode step),
+// then eight ranges' sums are in flight a thread. (Ranges past the 64th, which no rule here asks for, are weighted one by one.)
+constexpr int MX_MERGE_MOST = 64;                            // weights held a row
+
 template <typename T>
 __global__ __launch_bounds__(256) void attn_mixed_merge_kernel(MixedAttnArgs a) {
+  __shared__ float weight[16 * MX_MERGE_MOST], top_row[16], inv_row[16];
   const int seq = a.seq0 + blockIdx.y, head = blockIdx.z, tile = blockIdx.x;
   const int q0 = a.q_start[seq], q_len = a.q_start[seq + 1] - q0;
   if (tile * 16 >= q_len) return;
   const int n_rows = min(min(16, q_len - tile * 16), a.rows_kept);
-  const int E = a.E;
+  const int E = a.E, S = a.splits;
   const size_t stride = (size_t)a.H * a.rows_kept * (E + 2);          // between key ranges
-  const float* tile_base = a.part + ((((size_t)blockIdx.y * gridDim.x + tile) * a.splits) * a.H + head) * a.rows_kept * (E + 2);
+  const float* tile_base = a.part + ((((size_t)blockIdx.y * gridDim.x + tile) * S) * a.H + head) * a.rows_kept * (E + 2);
+  // a wave a row: lane s the ranges s, s + 64, ...
+  const int lane = threadIdx.x & 63;
+  for (int row = threadIdx.x >> 6; row < n_rows; row += 4) {
+    const float* base = tile_base + (size_t)row * (E + 2) + E;
+    float top = -INFINITY, total = 0.f;
+    for (int s = lane; s < S; s += 64) top = fmaxf(top, base[s * stride]);
+    top = tw_wave_max(top);
+    top = top == -INFINITY ? 0.f : top;
+    for (int s = lane; s < S; s += 64) {
+      const float f = mx_exp<T>(base[s * stride] - top);
+      total += base[s * stride + 1] * f;
+      if (s < MX_MERGE_MOST) weight[row * MX_MERGE_MOST + s] = f;
+    }
+    total = tw_wave_sum(total);
+    if (lane == 0) {
+      top_row[row] = top;
+      inv_row[row] = total > 0.f ? a.out_scale / total : 0.f;
+    }
+  }
+  __syncthreads();
   for (int i = threadIdx.x; i < n_rows * E; i += blockDim.x) {
     const int row = i / E, d = i % E;
     const float* base = tile_base + (size_t)row * (E + 2);
-    float m = -INFINITY;
-    for (int s = 0; s < a.splits; ++s) m = fmaxf(m, base[s * stride + E]);
-    const float m_use = m == -INFINITY ? 0.f : m;
-    float l = 0.f, o = 0.f;
-    for (int s = 0; s < a.splits; ++s) {
-      const float f = mx_exp<T>(base[s * stride + E] - m_use);
-      l += base[s * stride + E + 1] * f;
-      o += base[s * stride + d] * f;
+    const float* w = weight + row * MX_MERGE_MOST;
+    float o = 0.f;
+    int s = 0;
+    for (; s + 8 <= min(S, MX_MERGE_MOST); s += 8) {
+      float v[8];
+#pragma unroll
+      for (int k = 0; k < 8; ++k) v[k] = base[(s + k) * stride + d];
+#pragma unroll
+      for (int k = 0; k < 8; ++k) o += v[k] * w[s + k];
     }
-    const float inv = l > 0.f ? a.out_scale / l : 0.f;
-    ((T*)a.out)[(size_t)(q0 + tile * 16 + row) * a.ldo + (size_t)head * E + d] = tw_from_float<T>(o * inv);
+    for (; s < S; ++s) o += base[s * stride + d] * (s < MX_MERGE_MOST ? w[s] : mx_exp<T>(base[s * stride + E] - top_row[row]));
+    ((T*)a.out)[(size_t)(q0 + tile * 16 + row) * a.ldo + (size_t)head * E + d] = tw_from_float<T>(o * inv_row[row]);
   }
 }
 
@@ -492,6 +765,20 @@ static int mixed_launch(MixedAttnArgs a, int n_seqs, int tiles, int waves, size_
     if (e != hipSuccess) return (int)e;
   }
   kernel<<<dim3(tiles, n_seqs, a.splits), waves * 64, lds, stream>>>(a);
+  return TW_LAUNCH_RESULT();
+}
+
+// One query token a sequence: sizes that attn_mixed_one_kernel holds (a wave a key/value head, its query heads one tile's rows,
+// a key tile in one page).
+static bool mixed_one_takes(int max_q_len, int H, int G, int D, int E, int P) {
+  return max_q_len == 1 && G <= 8 && H / G <= 16 && D == E && (D == 64 || D == 128) && P >= 16 && (P & (P - 1)) == 0;
+}
+
+template <typename T, int S, bool TALK>
+static int mixed_one_launch(const MixedAttnArgs& a, int n_seqs, hipStream_t stream) {
+  constexpr int NT = Elem<T>::kPerFrag == 8 ? 4 : 2;          // (float32 fragments are twice as many registers)
+  const size_t lds = TALK ? (size_t)2 * NT * 16 * ((a.H + 3) / 4 * 4 + 4) * sizeof(float) : 0;
+  attn_mixed_one_kernel<T, S, NT, TALK><<<dim3(1, n_seqs, a.splits), a.G * 64, lds, stream>>>(a);
   return TW_LAUNCH_RESULT();
 }
 
@@ -514,6 +801,13 @@ static int mixed_dispatch(const MixedAttnArgs& args, int n_seqs, int max_q_len, 
   const size_t lds = mx_lds_bytes<T>(a.H, a.D, a.q_in_lds != 0);
   TW_REQUIRE(waves <= 16 && lds <= 150 * 1024);
   int code;
+  if (mixed_one_takes(max_q_len, a.H, a.G, a.D, a.E, a.P)) {
+    code = a.D == 64 ? (a.talk ? mixed_one_launch<T, 64, true>(a, n_seqs, stream) : mixed_one_launch<T, 64, false>(a, n_seqs, stream))
+                     : (a.talk ? mixed_one_launch<T, 128, true>(a, n_seqs, stream) : mixed_one_launch<T, 128, false>(a, n_seqs, stream));
+    if (code != 0 || a.splits == 1) return code;
+    attn_mixed_merge_kernel<T><<<dim3(1, n_seqs, a.H), 256, 0, stream>>>(a);
+    return TW_LAUNCH_RESULT();
+  }
   // (the sizes of most models: compile-time instances for values of 128 beside keys of four MFMA steps)
   const bool exact = a.D == 16 * Elem<T>::kPerFrag && a.E == 128;
 #define TW_MIXED(HPW_, VT_, WMAX_, AHEAD_)                                                                          \
@@ -537,12 +831,13 @@ static int mixed_dispatch(const MixedAttnArgs& args, int n_seqs, int max_q_len, 
   return TW_LAUNCH_RESULT();
 }
 
-// Key ranges for one-token sequences: enough workgroups to spread over the chip, each with at least 4 key tiles.
+// Key ranges for one-token sequences of up to max_kv_len seen keys: up to two workgroups a CU, each with 4 key tiles or more:
+// what attn_mixed_one_kernel takes at once.
 extern "C" int tw_attn_mixed_splits(int n_seqs, int max_kv_len) {
   if (n_seqs <= 0) return 1;
   const int tiles = tw_div_up(max_kv_len, 16);
-  int want = 1024 / n_seqs;
-  int most = tiles / 4;
+  int want = 512 / n_seqs;
+  int most = tw_div_up(tiles, 4);
   int s = want < most ? want : most;
   if (s > 64) s = 64;
   return s < 1 ? 1 : s;

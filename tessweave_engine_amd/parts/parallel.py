@@ -128,7 +128,7 @@ class MixedHeadAttention(MixerBranch):
             longest = ctx.kv_bound if ctx.capturing else ctx.max_kv_len
             most = ctx.kv_capacity
             if window:
-                longest, most = min(longest, window), min(most, window)
+                longest, most = min(longest, window + 15), min(most, window + 15)   # (of the key tiles a window touches)
             splits = ops.attn_mixed_splits(ctx.n_decode, longest)
             ws = None
             if splits > 1:

@@ -131,6 +131,54 @@ def test_mixed_head_attention_forms(device, dtype, H, G, D, E, window, T, q_len,
     test_mixed_head_attention(device, dtype, H, G, D, E, window, T, q_len, page)
 
 
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("H,G,S,window,keep,page,lengths,splits", [
+    (16, 4, 128, 0, 0, 16, [1, 15, 16, 17, 63, 64, 65, 300], 1),       # tiles' and groups' edges, one range
+    (24, 4, 128, 60, 0, 16, [60, 61, 76, 77, 129, 200], 3),            # two products of heads; windows that begin inside a tile
+    (6, 2, 64, 40, 5, 32, [39, 41, 56, 90, 250], 4),                   # three heads a key head, kept keys, two tiles a page
+    (32, 2, 128, 33, 20, 64, [33, 53, 54, 100, 180], 2),               # sixteen heads a key head, kept keys past a tile
+    (8, 8, 64, 0, 0, 16, [5, 70, 140], 16),                            # a head each, more ranges than tiles
+    (5, 1, 128, 24, 1, 16, [24, 25, 40, 41, 99], 70),                  # one wave, ranges past the 64th
+])
+@pytest.mark.parametrize("mixed", [True, False])
+def test_mixed_head_attention_of_one_token(device, dtype, H, G, S, window, keep, page, lengths, splits, mixed):
+    """One query token a sequence, sequences of unequal lengths together, against the formula in 64 bits: pages hold NaN
+    wherever no key of the sequence lies, and pages before a window are not held."""
+    from tessweave_engine_amd.kernels import ops
+    g = torch.Generator().manual_seed(H * 100 + S + len(lengths))
+    dt, n, width = tdtype(dtype), len(lengths), max(lengths) // page + 3
+    keys = torch.full((n * width + 1, G, page, S), float("nan"))
+    values = torch.full((n * width + 1, G, S, page), float("nan"))
+    table = torch.full((n, width), -1, dtype=torch.int32)
+    order = torch.randperm(n * width, generator=g).tolist()
+    q = torch.randn(n, H, S, generator=g).to(dt).float()
+    talk = torch.eye(H) + 0.3 * torch.randn(H, H, generator=g)
+    slopes = torch.tensor([2.0 ** (-8.0 * (h + 1) / H) for h in range(H)])
+    sink, scale, want = torch.randn(H, generator=g), 0.4 * S ** -0.5, []
+    for i, T in enumerate(lengths):
+        k, v = (torch.randn(T, G, S, generator=g).to(dt).float() for _ in range(2))
+        dist = T - 1 - torch.arange(T)
+        seen = ((dist < window) | (torch.arange(T) < keep)) if window else torch.ones(T, dtype=torch.bool)
+        for b in range((T + page - 1) // page):
+            lo, hi = b * page, min(T, (b + 1) * page)
+            if seen[lo:hi].any():
+                at = table[i, b] = order.pop()
+                keys[at, :, :hi - lo], values[at, :, :, :hi - lo] = k[lo:hi].transpose(0, 1), v[lo:hi].permute(1, 2, 0)
+        k, v = (t.double().repeat_interleave(H // G, 1) for t in (k, v))
+        s = torch.einsum("hd,thd->ht", q[i].double(), k) * scale - (slopes.double().view(H, 1) * dist if mixed else 0.0)
+        s = (talk.double() @ s if mixed else s).masked_fill(~seen, -math.inf)
+        p = torch.softmax(torch.cat([s, sink.double().view(H, 1)], 1), 1)[:, :T]
+        want.append(torch.einsum("ht,the->he", p, v).reshape(H * S))
+    out = torch.full((n, H * S), float("nan"), dtype=dt, device=device)
+    ws = torch.full((ops.attn_mixed_workspace_floats(n, 1, H, S, splits),), float("nan"), device=device) if splits > 1 else None
+    ops.attn_mixed(q.view(n, H * S).to(dt).to(device), keys.to(dt).to(device), values.to(dt).to(device), table.to(device),
+                   torch.arange(n + 1, dtype=torch.int32, device=device), torch.tensor(lengths, dtype=torch.int32, device=device),
+                   0, n, 1, out, H, G, scale, window=window, talk=talk.to(device) if mixed else None, sink=sink.to(device),
+                   slopes=slopes.to(device) if mixed else None, splits=splits, workspace=ws, keep_first=keep)
+    err = row_error(out.float().cpu().numpy(), torch.stack(want).numpy()).max()
+    assert err < (1e-5 if dtype == "float32" else 2e-2), err
+
+
 def test_mixed_head_attention_does_not_round_the_first_heads_product(device):
     """Distance slopes make the first head's score the largest; its product with the mixing weight goes into the sum unrounded.
     Here w0 r0 = 2^20 (1 + 2^-12)^2 and w1 r1 = -2^20 (1 + 2^-11), both factors exact in float32: the sum is 2^-4, and nothing
