@@ -30,9 +30,7 @@ struct LatentFinishArgs {
 };
 
 template <typename T>
-__global__ __launch_bounds__(256) void latent_finish_kernel(LatentFinishArgs a) {
-  __shared__ float lds[16];
-  const int n = blockIdx.x;
+__device__ __forceinline__ void latent_finish_token(const LatentFinishArgs& a, int n, float* lds) {
   const T* row = (const T*)a.proj + (size_t)n * a.ld;
   const int half = a.rot / 2;
   const float* cs = a.cos_t + (size_t)n * half;
@@ -101,11 +99,81 @@ __global__ __launch_bounds__(256) void latent_finish_kernel(LatentFinishArgs a) 
   }
 }
 
+// ---- one small matrix per head: out[n][a * so + o] = sum_i x[n][a * sx + i] * w[a][o][i] ------------------------
+// x and out hold the heads side by side, sx and so elements apart; w [heads][No][Ni] row-major. A wave takes 16
+// rows and 16 output columns of one head; the weights are the A operand, so a lane ends with four consecutive
+// output columns of one row. Sums are float32, rounded once to the compute type. Bound by the trips to memory in a row: the
+// operands of 8 k-steps are requested together (64 columns a wave, each k-step waiting for its own: 7.6 us of a decode step's
+// layer for 16 heads of 128 x 192, 4.4 for 192 x 64).
+template <typename T>
+struct HeadLinear {
+  const T* x; long ldx; int sx;
+  const T* w;
+  T* out; long ldo; int so;
+  int n, heads, Ni, No;
+  __host__ __device__ int units() const { return heads * ((No + 15) / 16); }       // of 16 rows each
+};
+
+template <typename T>
+__device__ __forceinline__ void head_linear_unit(const HeadLinear<T>& a, int unit, int row_tile) {
+  typedef typename Elem<T>::Frag Frag;
+  constexpr int EPF = Elem<T>::kPerFrag, U = 8;
+  const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
+  const int col_tiles = (a.No + 15) / 16;
+  const int head = unit / col_tiles, col = unit % col_tiles * 16;
+  const int row = row_tile * 16 + r;
+  const int chunks = a.Ni / EPF, steps = (chunks + 3) / 4;
+  const T* x_row = a.x + (size_t)min(row, a.n - 1) * a.ldx + (size_t)head * a.sx;      // (rows and columns past the last: never stored)
+  const T* w_row = a.w + ((size_t)head * a.No + min(col + r, a.No - 1)) * a.Ni;
+  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+  for (int st0 = 0; st0 < steps; st0 += U) {
+    Frag xf[U], wf[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int chunk = min((st0 + u) * 4 + g, chunks - 1);
+      xf[u] = tw_load_frag(x_row + chunk * EPF);
+      wf[u] = tw_load_frag(w_row + chunk * EPF);
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      if (st0 + u < steps) {
+        const bool in = (st0 + u) * 4 + g < chunks;
+        tw_mma16(acc, in ? wf[u] : Elem<T>::zero(), in ? xf[u] : Elem<T>::zero());      // D[output 4g + e][row r]
+      }
+  }
+  const int o = col + 4 * g;
+  if (row < a.n && o < a.No) {
+    T* dst = a.out + (size_t)row * a.ldo + (size_t)head * a.so + o;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) dst[e] = tw_from_float<T>(acc[e]);
+  }
+}
+
+template <typename T>
+__global__ __launch_bounds__(256) void head_linear_kernel(HeadLinear<T> a) {
+  const int unit = blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (unit < a.units()) head_linear_unit(a, unit, blockIdx.y);
+}
+
+// Workgroups 0 .. n - 1 finish a token each; those behind them form the query side's products W_uk,a^T q_plain,a of the first
+// absorb.n rows, which read and write nothing the others write: one launch instead of two.
+template <typename T>
+__global__ __launch_bounds__(256) void latent_finish_kernel(LatentFinishArgs a, HeadLinear<T> absorb, int n) {
+  __shared__ float lds[16];
+  if ((int)blockIdx.x < n) {
+    latent_finish_token<T>(a, blockIdx.x, lds);
+    return;
+  }
+  const int unit = ((int)blockIdx.x - n) * 4 + (threadIdx.x >> 6), per_tile = absorb.units();
+  const int row_tile = unit / per_tile;
+  if (row_tile * 16 < absorb.n) head_linear_unit(absorb, unit - row_tile * per_tile, row_tile);
+}
+
 extern "C" int tw_latent_finish(int dtype, const void* proj, long ld, int q_col, int c_col, int kr_col,
                                 const float* cos_t, const float* sin_t, const float* norm_w, void* q_out, long ld_q,
                                 void* q_full, long ld_full, int D, int Dp, int hd, int full_from,
                                 void* keys, void* values, const int* slots, int n, int H, int L, int Lp, int Rp, int rot,
-                                int page_size, float eps, hipStream_t stream) {
+                                int page_size, float eps, const void* absorb, int absorb_rows, hipStream_t stream) {
   TW_REQUIRE(proj && cos_t && sin_t && q_out && n >= 0 && H > 0 && Rp > 0 && rot > 0 && rot % 2 == 0 && rot <= Rp);
   if (q_full) TW_REQUIRE(D > 0 && Dp >= D && hd >= D + rot && ld_full >= (long)H * hd && full_from >= 0 && q_col >= H * Dp);
   TW_REQUIRE(q_col >= 0 && ld >= q_col + (long)H * Rp && ld_q >= (long)H * (Lp + Rp) && Lp >= 0);
@@ -116,54 +184,23 @@ extern "C" int tw_latent_finish(int dtype, const void* proj, long ld, int q_col,
   if (n == 0) return 0;
   LatentFinishArgs a{proj, ld, q_col, c_col, kr_col, cos_t, sin_t, norm_w, q_out, ld_q, q_full, ld_full, D, Dp, hd, full_from,
                      keys, values, slots, H, L, Lp, Rp, rot, page_size, eps};
-  if (dtype == TW_DTYPE_BF16) latent_finish_kernel<bf16_t><<<n, 256, 0, stream>>>(a);
-  else if (dtype == TW_DTYPE_F32) latent_finish_kernel<float><<<n, 256, 0, stream>>>(a);
+  if (absorb) {            // [H][Lp][Dp]: the first absorb_rows rows' latent queries too, into columns 0 .. Lp of every head of q_out
+    const int epf = dtype == TW_DTYPE_BF16 ? 8 : 4;
+    TW_REQUIRE(absorb_rows >= 0 && absorb_rows <= n && Dp > 0 && Dp % epf == 0 && Lp % 4 == 0 && ld % epf == 0 && q_col >= H * Dp);
+    TW_REQUIRE((uintptr_t)proj % 16 == 0 && (uintptr_t)absorb % 16 == 0);
+  }
+  const int rows = absorb ? absorb_rows : 0;
+#define TW_LATENT_FINISH(T)                                                                                                    \
+  do {                                                                                                                         \
+    const HeadLinear<T> hl{(const T*)proj, ld, Dp, (const T*)absorb, (T*)q_out, ld_q, Lp + Rp, rows, H, Dp, Lp};                \
+    const int groups = rows ? tw_div_up((long)hl.units() * tw_div_up(rows, 16), 4) : 0;                                         \
+    latent_finish_kernel<T><<<n + groups, 256, 0, stream>>>(a, hl, n);                                                         \
+  } while (0)
+  if (dtype == TW_DTYPE_BF16) TW_LATENT_FINISH(bf16_t);
+  else if (dtype == TW_DTYPE_F32) TW_LATENT_FINISH(float);
   else return TW_ERR_BAD_ARGUMENT;
+#undef TW_LATENT_FINISH
   return TW_LAUNCH_RESULT();
-}
-
-// ---- one small matrix per head: out[n][a * so + o] = sum_i x[n][a * sx + i] * w[a][o][i] ------------------------
-// x and out hold the heads side by side, sx and so elements apart; w [heads][No][Ni] row-major. A wave takes 16
-// rows and 64 output columns of one head; the weights are the A operand, so a lane ends with four consecutive
-// output columns of one row. Sums are float32, rounded once to the compute type.
-template <typename T>
-__global__ __launch_bounds__(256) void head_linear_kernel(const T* __restrict__ x, long ldx, int sx, const T* __restrict__ w,
-                                                          T* __restrict__ out, long ldo, int so, int n, int heads, int Ni,
-                                                          int No, int col_groups) {
-  typedef typename Elem<T>::Frag Frag;
-  constexpr int EPF = Elem<T>::kPerFrag;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int r = lane & 15, g = lane >> 4;
-  const int unit = blockIdx.x * 4 + wave;
-  const int head = unit / col_groups, cg = unit % col_groups;
-  if (head >= heads) return;
-  const int row = blockIdx.y * 16 + r;
-  const int chunks = Ni / EPF, steps = (chunks + 3) / 4;
-  const T* x_row = x + (size_t)(row < n ? row : 0) * ldx + (size_t)head * sx;
-  f32x4 acc[4];
-#pragma unroll
-  for (int t = 0; t < 4; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-  for (int st = 0; st < steps; ++st) {
-    const int chunk = st * 4 + g;
-    const bool in = chunk < chunks;
-    const Frag xf = (in && row < n) ? tw_load_frag(x_row + chunk * EPF) : Elem<T>::zero();
-#pragma unroll
-    for (int t = 0; t < 4; ++t) {
-      const int o = cg * 64 + t * 16 + r;
-      const Frag wf = (in && o < No) ? tw_load_frag(w + ((size_t)head * No + o) * Ni + chunk * EPF) : Elem<T>::zero();
-      tw_mma16(acc[t], wf, xf);                            // D[output 4g + e][row r]
-    }
-  }
-  if (row >= n) return;
-#pragma unroll
-  for (int t = 0; t < 4; ++t) {
-    const int o = cg * 64 + t * 16 + 4 * g;
-    if (o < No) {
-      T* dst = out + (size_t)row * ldo + (size_t)head * so + o;
-#pragma unroll
-      for (int e = 0; e < 4; ++e) dst[e] = tw_from_float<T>(acc[t][e]);
-    }
-  }
 }
 
 extern "C" int tw_head_linear(int dtype, const void* x, long ldx, int sx, const void* w, void* out, long ldo, int so,
@@ -175,14 +212,14 @@ extern "C" int tw_head_linear(int dtype, const void* x, long ldx, int sx, const 
   TW_REQUIRE(ldx >= (long)(heads - 1) * sx + Ni && ldo >= (long)(heads - 1) * so + No);
   TW_REQUIRE((uintptr_t)x % 16 == 0 && (uintptr_t)w % 16 == 0);
   if (n == 0) return 0;
-  const int col_groups = tw_div_up(No, 64);
-  const dim3 grid(tw_div_up((long)heads * col_groups, 4), tw_div_up(n, 16));
-  if (dtype == TW_DTYPE_BF16)
-    head_linear_kernel<bf16_t><<<grid, 256, 0, stream>>>((const bf16_t*)x, ldx, sx, (const bf16_t*)w, (bf16_t*)out, ldo, so, n,
-                                                         heads, Ni, No, col_groups);
-  else
-    head_linear_kernel<float><<<grid, 256, 0, stream>>>((const float*)x, ldx, sx, (const float*)w, (float*)out, ldo, so, n,
-                                                        heads, Ni, No, col_groups);
+#define TW_HEAD_LINEAR(T)                                                                                                      \
+  do {                                                                                                                         \
+    const HeadLinear<T> hl{(const T*)x, ldx, sx, (const T*)w, (T*)out, ldo, so, n, heads, Ni, No};                              \
+    head_linear_kernel<T><<<dim3(tw_div_up(hl.units(), 4), tw_div_up(n, 16)), 256, 0, stream>>>(hl);                            \
+  } while (0)
+  if (dtype == TW_DTYPE_BF16) TW_HEAD_LINEAR(bf16_t);
+  else TW_HEAD_LINEAR(float);
+#undef TW_HEAD_LINEAR
   return TW_LAUNCH_RESULT();
 }
 
@@ -318,7 +355,7 @@ extern "C" int tw_latent_expand_store(int dtype, const void* up, long ld_up, con
 // keys of one element are one 8-byte load. A sequence's keys are cut into `splits` ranges for separate workgroups,
 // whose waves take the range's tiles in turn; waves are combined through LDS, ranges by a second kernel in index order.
 //
-//   part [seq][head tile][split][16][Lp + 2]: output sums relative to the range's maximum, that maximum, the sum
+//   part [seq][head tile][split][16][Lp + 4]: output sums relative to the range's maximum, that maximum, the sum
 struct LatentDecodeArgs {
   const void* q; long ldq;            // head a of sequence s at q + row(s) * ldq + a * K
   const void* keys; const void* values;
@@ -328,6 +365,8 @@ struct LatentDecodeArgs {
   float* part;
   float scale;
   int H, K, Lp, P, splits;
+  int to_part;                        // ranges' results stay in part (also that of a single range)
+  int page_shift;                     // log2(P) if P is a power of two, else -1
   const float* sink;                  // [H] or null: exp(sink_a) more in head a's denominator (no key, no value, not scaled)
 };
 
@@ -339,20 +378,22 @@ template <typename T> struct LtQuad;
 template <> struct LtQuad<float> { typedef f32x4 Type; };
 template <> struct LtQuad<bf16_t> { typedef bf16x4 Type; };
 
-template <typename T>
+// EXACT: key rows of KS and latents of LS elements, pages of a power of two and at least 16: sizes are compile-time constants
+// and a key tile's page and addresses the whole wave's (scalar).
+template <typename T, int KS = 256, int LS = 240, bool EXACT = false>
 __global__ __launch_bounds__(256) void latent_decode_kernel(LatentDecodeArgs a) {
   typedef typename Elem<T>::Frag Frag;
   typedef typename LtQuad<T>::Type Quad;
   constexpr int EPF = Elem<T>::kPerFrag;
   constexpr int STEP = 4 * EPF;                 // key elements one product consumes
-  constexpr int KC_MAX = 256 / STEP;
-  constexpr int LT_MAX = 15;                    // Lp <= 240
+  constexpr int KC_MAX = KS / STEP;
+  constexpr int LT_MAX = LS / 16;
   extern __shared__ float ld_lds[];
   const int s = blockIdx.x, split = blockIdx.y, ht = blockIdx.z;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int r = lane & 15, g = lane >> 4;
-  const int K = a.K, Lp = a.Lp, P = a.P;
-  const int KC = (K + STEP - 1) / STEP, LT = Lp / 16;
+  const int K = EXACT ? KS : a.K, Lp = EXACT ? LS : a.Lp, P = a.P;
+  const int KC = EXACT ? KC_MAX : (K + STEP - 1) / STEP, LT = EXACT ? LT_MAX : Lp / 16;
   const int len = a.kv_len[s];
   const int row = a.q_start[s];
   const int head = ht * 16 + r;
@@ -381,19 +422,36 @@ __global__ __launch_bounds__(256) void latent_decode_kernel(LatentDecodeArgs a) 
   // ahead they would halve the waves). 8 requests of 150
   // tokens 17.7 -> 12.3 us, one of 2,048 22.6 -> 12.7 (kernel traces).
   // A key past the end is the last one again; masked below.
-  constexpr bool AHEAD = EPF == 8;
+  constexpr bool AHEAD = EPF == 8 || EXACT;
   auto key_of = [&](int t) { return min(t * 16 + r, len - 1); };
   auto value_of = [&](int t) { return min(t * 16 + 4 * g, (len - 1) / 4 * 4); };      // 4 keys: one page (multiples of 4)
   Frag kf[KC_MAX];
   Quad vq[LT_MAX];
-  auto key_row = [&](int t, int page) { return keys + ((size_t)page * P + key_of(t) % P) * K; };
+  // (EXACT: places behind the sequence's end in its last page hold anything: masked like them all)
+  auto page_of = [&](int t, int key) { return EXACT ? max(0, table[(t * 16) >> a.page_shift]) : table[key / P]; };
+  auto key_row = [&](int t, int page) {
+    if constexpr (EXACT) return keys + ((uint64_t)(uint32_t)page * (uint32_t)(P * KS) + (uint32_t)(((t * 16) & (P - 1)) * KS)) + r * KS;
+    else return keys + ((size_t)page * P + key_of(t) % P) * K;
+  };
   auto request_keys = [&](int t, int page) {
     const T* krow = key_row(t, page);
+    if constexpr (EXACT) {
+#pragma unroll
+      for (int kc = 0; kc < KC_MAX; ++kc) kf[kc] = tw_load_frag(krow + kc * STEP + g * EPF);
+      return;
+    }
 #pragma unroll
     for (int kc = 0; kc < KC_MAX; ++kc)
       if (kc < KC) kf[kc] = tw_load_frag(krow + min(kc * STEP + g * EPF, K - EPF));   // (past the row: a copy)
   };
   auto request_values = [&](int t, int page) {
+    if constexpr (EXACT) {
+      const T* base = values + ((uint64_t)(uint32_t)page * (uint32_t)(P * LS) + (uint32_t)((t * 16) & (P - 1)));
+#pragma unroll
+      for (int lt = 0; lt < LT_MAX; ++lt)
+        vq[lt] = *reinterpret_cast<const Quad*>(base + (uint32_t)(lt * 16 * P) + (uint32_t)(r * P + 4 * g));
+      return;
+    }
     const T* vbase = values + (size_t)page * Lp * P + value_of(t) % P + (size_t)r * P;
 #pragma unroll
     for (int lt = 0; lt < LT_MAX; ++lt)
@@ -402,14 +460,14 @@ __global__ __launch_bounds__(256) void latent_decode_kernel(LatentDecodeArgs a) 
   int t = t_begin + wave;
   int k_page = 0, v_page = 0;                     // of the tile to be requested next
   if (t < t_end) {
-    k_page = table[key_of(t) / P];
-    v_page = table[value_of(t) / P];
+    k_page = page_of(t, key_of(t));
+    v_page = page_of(t, value_of(t));
     if (AHEAD) {
       request_keys(t, k_page);
       request_values(t, v_page);
       if (t + 4 < t_end) {
-        k_page = table[key_of(t + 4) / P];
-        v_page = table[value_of(t + 4) / P];
+        k_page = page_of(t + 4, key_of(t + 4));
+        v_page = page_of(t + 4, value_of(t + 4));
       }
     }
   }
@@ -435,8 +493,8 @@ __global__ __launch_bounds__(256) void latent_decode_kernel(LatentDecodeArgs a) 
     } else if (!AHEAD) {
       request_values(t, v_page);
       if (more) {
-        k_page = table[key_of(t + 4) / P];
-        v_page = table[value_of(t + 4) / P];
+        k_page = page_of(t + 4, key_of(t + 4));
+        v_page = page_of(t + 4, value_of(t + 4));
       }
     }
     float top = -INFINITY;
@@ -457,6 +515,7 @@ __global__ __launch_bounds__(256) void latent_decode_kernel(LatentDecodeArgs a) 
     }
     sum = sum * alpha + tw_rows_sum(part);
     m = m_new;
+    const bool rescale = __builtin_amdgcn_ballot_w64(alpha != 1.f) != 0;     // (some head's maximum has moved)
 #pragma unroll
     for (int lt = 0; lt < LT_MAX; ++lt) {
       if (lt < LT) {
@@ -466,16 +525,18 @@ __global__ __launch_bounds__(256) void latent_decode_kernel(LatentDecodeArgs a) 
           for (int j = 0; j < 4; ++j)
             if (t * 16 + 4 * g + j >= len) v[j] = tw_from_float<T>(0.f);     // whatever lies there must not reach a sum
         }
+        if (rescale) {
 #pragma unroll
-        for (int j = 0; j < 4; ++j) O[lt][j] *= alpha;
+          for (int j = 0; j < 4; ++j) O[lt][j] *= alpha;
+        }
         tw_mma16_k4(O[lt], v, Pr);               // O[lt][j]: element lt * 16 + 4 g + j of head r
       }
     }
     if (AHEAD && more) {
       request_values(t + 4, v_page);
       if (t + 8 < t_end) {
-        k_page = table[key_of(t + 8) / P];
-        v_page = table[value_of(t + 8) / P];
+        k_page = page_of(t + 8, key_of(t + 8));
+        v_page = page_of(t + 8, value_of(t + 8));
       }
     }
   }
@@ -492,29 +553,36 @@ __global__ __launch_bounds__(256) void latent_decode_kernel(LatentDecodeArgs a) 
     sw[wave * 16 + r] = sum;
   }
   __syncthreads();
-  for (int i = threadIdx.x; i < 16 * Lp; i += 256) {
-    const int hh = i / Lp, l = i - hh * Lp;
+  const int quads = Lp / 4;
+  for (int i = threadIdx.x; i < 16 * quads; i += 256) {
+    const int hh = i / quads, l = (i - hh * quads) * 4;
     if (ht * 16 + hh >= a.H) continue;
-    float top = fmaxf(fmaxf(mw[hh], mw[16 + hh]), fmaxf(mw[32 + hh], mw[48 + hh]));
-    float o = 0.f, total = 0.f;
+    const float top = fmaxf(fmaxf(mw[hh], mw[16 + hh]), fmaxf(mw[32 + hh], mw[48 + hh]));
+    f32x4 o = {0.f, 0.f, 0.f, 0.f};
+    float total = 0.f;
 #pragma unroll
     for (int w = 0; w < 4; ++w) {
       const float f = mw[w * 16 + hh] == -INFINITY ? 0.f : lt_exp<T>(mw[w * 16 + hh] - top);
-      o += f * Ow[((size_t)w * 16 + hh) * OS + l];
+      const f32x4 v = *reinterpret_cast<const f32x4*>(Ow + ((size_t)w * 16 + hh) * OS + l);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) o[e] += f * v[e];
       total += f * sw[w * 16 + hh];
     }
-    if (a.splits == 1) {
+    if (!a.to_part) {
+      float scale = 1.f;
       if (a.sink) {
         const float sk = a.sink[ht * 16 + hh];
         const float both = fmaxf(top, sk);
         const float f = top == -INFINITY ? 0.f : lt_exp<T>(top - both);
-        o *= f;
+        scale = f;
         total = total * f + lt_exp<T>(sk - both);
       }
-      ((T*)a.out)[(size_t)row * a.ldo + (size_t)(ht * 16 + hh) * Lp + l] = tw_from_float<T>(o / total);
+      T* dst = (T*)a.out + (size_t)row * a.ldo + (size_t)(ht * 16 + hh) * Lp + l;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) dst[e] = tw_from_float<T>(o[e] * scale / total);
     } else {
-      float* dst = a.part + ((((size_t)s * gridDim.z + ht) * a.splits + split) * 16 + hh) * (Lp + 2);
-      dst[l] = o;
+      float* dst = a.part + ((((size_t)s * gridDim.z + ht) * a.splits + split) * 16 + hh) * (Lp + 4);
+      *reinterpret_cast<f32x4*>(dst + l) = o;
       if (l == 0) {
         dst[Lp] = top;
         dst[Lp + 1] = total;
@@ -533,8 +601,8 @@ __global__ __launch_bounds__(256) void latent_decode_merge_kernel(LatentDecodeAr
   const int Lp = a.Lp;
   const int row = a.q_start[s];
   const int head_tiles = (a.H + 15) / 16;
-  const float* base = a.part + ((((size_t)s * head_tiles + ht) * a.splits) * 16 + hh) * (Lp + 2);
-  const size_t stride = (size_t)16 * (Lp + 2);                  // from one range to the next
+  const float* base = a.part + ((((size_t)s * head_tiles + ht) * a.splits) * 16 + hh) * (Lp + 4);
+  const size_t stride = (size_t)16 * (Lp + 4);                  // from one range to the next
   if (threadIdx.x < 64) {
     const int sp = threadIdx.x;
     const float m = sp < a.splits ? base[sp * stride + Lp] : -INFINITY;
@@ -555,45 +623,196 @@ __global__ __launch_bounds__(256) void latent_decode_merge_kernel(LatentDecodeAr
   }
 }
 
-// Key ranges a sequence: enough workgroups for the chip, each range at least 8 tiles of 16 keys.
+// The same with what follows it in a layer: the ranges' results of 16 rows of one head are added up, rounded to the compute type and
+// multiplied with the head's W_uv ([No][Lp]); gate (or null): the result times sigmoid(gate). One workgroup a (head, 16 rows). Its
+// waves' fragments of W_uv are requested first and the ranges' sums before their weights are known, so that three trips to memory
+// lie in a row; with few rows several threads share a row's element and take every P-th range each. From the projections to the
+// gated heads, 16 heads, latents of 192, in a chain of such calls (us; five or six launches, 64-column products, run-time sizes and
+// ranges of 8 tiles / three launches): 8 requests of 190 keys bfloat16 29.6 / 15.5, float32 48.7 / 21.8; one of 2,050 keys 31.7 / 16.1;
+// 64 of 500 36.0 / 25.2; 24 heads, 64 of 4,000 88.2 / 80.2. The results are off by 0.8 times as much against 64 bits (the gate
+// multiplies the float32 product).
+struct LatentLeave {
+  const void* w;                      // [H][No][Lp]
+  void* out; long ldo; int so;        // head a's results at out + row(s) * ldo + a * so
+  const void* gate; long ldg;         // or null: head a's gate at gate + row(s) * ldg + a * so
+  int No, n;
+};
+
+template <typename T>
+__global__ __launch_bounds__(512) void latent_leave_kernel(LatentDecodeArgs a, LatentLeave b) {
+  typedef typename Elem<T>::Frag Frag;
+  constexpr int EPF = Elem<T>::kPerFrag, U = 8, AHEAD = 4;
+  extern __shared__ __attribute__((aligned(16))) unsigned char lt_lds[];
+  const int head = blockIdx.x, s0 = blockIdx.y * 16, n = min(16, b.n - s0);
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int r = lane & 15, g = lane >> 4;
+  const int Lp = a.Lp, S = a.splits, quads = Lp / 4, OS = Lp + 4;
+  const int chunks = Lp / EPF, steps = (chunks + 3) / 4;
+  const int xrow = Lp + 32 / (int)sizeof(T);
+  float* weight = (float*)lt_lds;                            // [16][64]
+  float* inv = weight + 16 * 64;                             // [16]
+  f32x4* sums = (f32x4*)(inv + 16);                          // [P][items], P x items <= 512
+  T* xs = (T*)(sums + 512);                                  // [16][xrow]
+  const int ht = head >> 4, hh = head & 15, head_tiles = (a.H + 15) / 16;
+  const size_t stride = (size_t)16 * OS;                     // from one range to the next
+  auto row_part = [&](int row) { return a.part + ((((size_t)(s0 + row) * head_tiles + ht) * S) * 16 + hh) * OS; };
+  // ---- requested first: W_uv's fragments of the wave's first 16 columns, the sums of the thread's first ranges ----------------
+  auto load_w = [&](int col, int st0, Frag (&f)[U]) {
+    const T* w_row = (const T*)b.w + ((size_t)head * b.No + min(col + r, b.No - 1)) * Lp;
+#pragma unroll
+    for (int u = 0; u < U; ++u) f[u] = tw_load_frag(w_row + min((st0 + u) * 4 + g, chunks - 1) * EPF);
+  };
+  Frag wf[U];
+  if (wave * 16 < b.No) load_w(wave * 16, 0, wf);
+  const int items = n * quads;
+  const int P = items >= 512 ? 1 : min(S, 512 / items);      // threads that share an element
+  const int item = P == 1 ? threadIdx.x : threadIdx.x % items, p = P == 1 ? 0 : threadIdx.x / items;
+  f32x4 first[AHEAD];
+  const bool active = item < items && p < P;
+  if (active) {
+    const float* base = row_part(item / quads) + item % quads * 4;
+#pragma unroll
+    for (int k = 0; k < AHEAD; ++k) first[k] = *reinterpret_cast<const f32x4*>(base + min(p + k * P, S - 1) * stride);
+  }
+  // ---- the ranges' weights, a wave a row, lane s the range s ----------------------------------------------------------------
+  for (int row = wave; row < n; row += 8) {
+    const float* base = row_part(row) + Lp;
+    const float m = lane < S ? base[lane * stride] : -INFINITY;
+    const float l = lane < S ? base[lane * stride + 1] : 0.f;
+    const float sk = a.sink ? a.sink[head] : -INFINITY;
+    const float top = fmaxf(tw_wave_max(m), sk);
+    const float f = m == -INFINITY ? 0.f : lt_exp<T>(m - top);
+    const float total = tw_wave_sum(f * l);
+    weight[row * 64 + lane] = f;
+    if (lane == 0) inv[row] = 1.f / (total + (a.sink ? lt_exp<T>(sk - top) : 0.f));
+  }
+  __syncthreads();
+  // ---- the rows, in index order of the ranges within a thread ----------------------------------------------------------------
+  auto finish = [&](int i, f32x4 o) {
+    const int row = i / quads;
+    T* dst = xs + row * xrow + i % quads * 4;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) dst[e] = tw_from_float<T>(o[e] * inv[row]);
+  };
+  for (int i = item; i < items; i += 512) {                  // (more than once only where P is 1)
+    if (!active) break;
+    const int row = i / quads;
+    const float* base = row_part(row) + i % quads * 4;
+    f32x4 o = {0.f, 0.f, 0.f, 0.f};
+    int k = p;
+    if (i == item) {
+#pragma unroll
+      for (int j = 0; j < AHEAD; ++j)
+        if (p + j * P < S) {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) o[e] += weight[row * 64 + p + j * P] * first[j][e];
+        }
+      k = p + AHEAD * P;
+    }
+    for (; k < S; k += 4 * P) {
+      f32x4 v[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) v[j] = *reinterpret_cast<const f32x4*>(base + min(k + j * P, S - 1) * stride);
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        if (k + j * P < S) {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) o[e] += weight[row * 64 + k + j * P] * v[j][e];
+        }
+    }
+    if (P == 1) finish(i, o);
+    else sums[p * items + i] = o;
+  }
+  __syncthreads();
+  if (P > 1) {
+    if (threadIdx.x < items) {
+      f32x4 o = sums[threadIdx.x];
+      for (int q = 1; q < P; ++q) o += sums[q * items + threadIdx.x];
+      finish(threadIdx.x, o);
+    }
+    __syncthreads();
+  }
+  // ---- times W_uv: D[output 4g + e][row r] --------------------------------------------------------------------------------------
+  const int at_row = a.q_start[s0 + min(r, n - 1)];
+  for (int col = wave * 16; col < b.No; col += 128) {
+    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+    for (int st0 = 0; st0 < steps; st0 += U) {
+      if (st0 > 0 || col != wave * 16) load_w(col, st0, wf);
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+        if (st0 + u < steps) {
+          const int chunk = (st0 + u) * 4 + g;
+          const bool in = chunk < chunks;
+          const Frag x = *reinterpret_cast<const Frag*>(xs + min(r, n - 1) * xrow + min(chunk, chunks - 1) * EPF);
+          tw_mma16(acc, in ? wf[u] : Elem<T>::zero(), in ? x : Elem<T>::zero());
+        }
+    }
+    const int o = col + 4 * g;
+    if (r < n && o < b.No) {
+      T* dst = (T*)b.out + (size_t)at_row * b.ldo + (size_t)head * b.so + o;
+      const T* gate = (const T*)b.gate + (size_t)at_row * b.ldg + (size_t)head * b.so + o;
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        dst[e] = tw_from_float<T>(b.gate ? acc[e] / (1.f + expf(-tw_to_float(gate[e]))) : acc[e]);
+    }
+  }
+}
+
+// Key ranges a sequence: up to two workgroups a CU, each range 4 tiles of 16 keys or more, one a wave. (Against ranges of 8 tiles and
+// sizes known at run time, with the merge: 8 requests of 190 keys 15.2 -> 8.0 us, one of 2,050 17.7 -> 10.8, float32 25.8 -> 11.6.)
 extern "C" int tw_latent_decode_splits(int n_seqs, int heads, int max_kv_len) {
   if (n_seqs <= 0) return 1;
   const int tiles = tw_div_up(max_kv_len, 16);
   int want = 512 / (n_seqs * tw_div_up(heads, 16));
-  if (want > tiles / 8) want = tiles / 8;
+  if (want > tw_div_up(tiles, 4)) want = tw_div_up(tiles, 4);
   if (want > 64) want = 64;
   return want < 1 ? 1 : want;
 }
 
 extern "C" long tw_latent_decode_workspace_floats(int n_seqs, int heads, int Lp, int splits) {
-  return splits > 1 ? (long)n_seqs * tw_div_up(heads, 16) * splits * 16 * (Lp + 2) : 0;
+  return (long)n_seqs * tw_div_up(heads, 16) * splits * 16 * (Lp + 4);
 }
 
 extern "C" int tw_latent_decode(int dtype, const void* q, long ldq, const void* keys, const void* values,
                                 const int* block_table, int table_stride, const int* q_start, const int* kv_len,
                                 int n_seqs, void* out, long ldo, float* workspace, long workspace_floats, int heads,
-                                int K, int Lp, int page_size, float scale, int splits, const float* sink, hipStream_t stream) {
+                                int K, int Lp, int page_size, float scale, int splits, const float* sink, const void* expand,
+                                int expand_out, int out_stride, const void* gate, long ldg, hipStream_t stream) {
   TW_REQUIRE(q && keys && values && block_table && q_start && kv_len && out && n_seqs >= 0 && splits >= 1 && splits <= 64);
   TW_REQUIRE(heads >= 1 && K % 16 == 0 && K <= 256 && Lp % 16 == 0 && Lp >= 16 && Lp <= 240 && Lp <= K);
   TW_REQUIRE(page_size > 0 && page_size % 4 == 0);
-  TW_REQUIRE(ldq >= (long)heads * K && ldo >= (long)heads * Lp);
+  TW_REQUIRE(ldq >= (long)heads * K && (expand || ldo >= (long)heads * Lp));
   const int esize = dtype == TW_DTYPE_BF16 ? 2 : 4;
   TW_REQUIRE((uintptr_t)q % 16 == 0 && (uintptr_t)keys % 16 == 0 && (uintptr_t)values % 16 == 0 && (ldq * esize) % 16 == 0);
-  if (splits > 1) TW_REQUIRE(workspace && workspace_floats >= tw_latent_decode_workspace_floats(n_seqs, heads, Lp, splits));
+  if (splits > 1 || expand)
+    TW_REQUIRE(workspace && (uintptr_t)workspace % 16 == 0 && workspace_floats >= tw_latent_decode_workspace_floats(n_seqs, heads, Lp, splits));
+  if (expand) {            // [heads][expand_out][Lp]: out takes the heads' results times their matrices, times sigmoid(gate)
+    TW_REQUIRE((uintptr_t)expand % 16 == 0 && expand_out > 0 && expand_out % 4 == 0 && out_stride >= expand_out);
+    TW_REQUIRE(ldo >= (long)(heads - 1) * out_stride + expand_out && (!gate || ldg >= (long)(heads - 1) * out_stride + expand_out));
+  }
+  TW_REQUIRE(expand || !gate);
   if (n_seqs == 0) return 0;
+  const bool pow2 = (page_size & (page_size - 1)) == 0;
   LatentDecodeArgs a{q, ldq, keys, values, block_table, table_stride, q_start, kv_len, out, ldo, workspace, scale,
-                     heads, K, Lp, page_size, splits, sink};
+                     heads, K, Lp, page_size, splits, splits > 1 || expand, pow2 ? __builtin_ctz(page_size) : -1, sink};
+  const LatentLeave b{expand, out, ldo, out_stride, gate, ldg, expand_out, n_seqs};
   const int head_tiles = tw_div_up(heads, 16);
   const dim3 grid(n_seqs, splits, head_tiles);
   const size_t lds = ((size_t)4 * 16 * (Lp + 4) + 128) * sizeof(float);
-  if (dtype == TW_DTYPE_BF16) {
-    latent_decode_kernel<bf16_t><<<grid, 256, lds, stream>>>(a);
-    if (splits > 1) latent_decode_merge_kernel<bf16_t><<<dim3(n_seqs, heads), 256, 0, stream>>>(a);
-  } else if (dtype == TW_DTYPE_F32) {
-    latent_decode_kernel<float><<<grid, 256, lds, stream>>>(a);
-    if (splits > 1) latent_decode_merge_kernel<float><<<dim3(n_seqs, heads), 256, 0, stream>>>(a);
-  } else {
-    return TW_ERR_BAD_ARGUMENT;
-  }
+#define TW_LATENT_DECODE(T)                                                                                                     \
+  do {                                                                                                                         \
+    if (K == 256 && Lp == 192 && pow2 && page_size >= 16) latent_decode_kernel<T, 256, 192, true><<<grid, 256, lds, stream>>>(a); \
+    else latent_decode_kernel<T><<<grid, 256, lds, stream>>>(a);                                                                 \
+    if (expand) {                                                                                                              \
+      const size_t leave = (16 * 64 + 16) * 4 + 512 * 16 + (size_t)16 * (Lp + 32 / sizeof(T)) * sizeof(T);                       \
+      latent_leave_kernel<T><<<dim3(heads, tw_div_up(n_seqs, 16)), 512, leave, stream>>>(a, b);                                  \
+    } else if (splits > 1) {                                                                                                   \
+      latent_decode_merge_kernel<T><<<dim3(n_seqs, heads), 256, 0, stream>>>(a);                                                 \
+    }                                                                                                                          \
+  } while (0)
+  if (dtype == TW_DTYPE_BF16) TW_LATENT_DECODE(bf16_t);
+  else if (dtype == TW_DTYPE_F32) TW_LATENT_DECODE(float);
+  else return TW_ERR_BAD_ARGUMENT;
+#undef TW_LATENT_DECODE
   return TW_LAUNCH_RESULT();
 }

@@ -896,13 +896,15 @@ def embed_hashed(ids, table, pairs, norm_weight, q_start, kv_len, state_slots, p
 # ---- attention over a cached latent: finishing a token's projections, one small matrix per head -----------------------
 
 def latent_finish(proj, q_col, c_col, kr_col, cos, sin, norm_weight, q_out, heads, latent, latent_dev, rot_dev, eps,
-                  keys=None, values=None, slots=None, q_full=None, dim=0, dim_dev=0, full_from=0):
+                  keys=None, values=None, slots=None, q_full=None, dim=0, dim_dev=0, full_from=0, absorb=None, absorb_rows=0):
     """Rotates the heads' rotated query parts proj[n, q_col + a * rot_dev ...] into q_out[n, a, latent_dev:], and,
     with keys/values, stores the token's key row [unit(proj[n, c_col : c_col + latent]) * norm_weight | zeros |
     rotated proj[n, kr_col ...] | zeros] and its value (the normed latent) into page slot slots[n] (-1: not stored).
     keys [pages, 1, page, latent_dev + rot_dev]; values [pages, 1, latent_dev, page]; q_out [n, heads * (latent_dev + rot_dev)].
     q_full [n, heads * hd]: rows from full_from on also get whole query heads [the head's dim unrotated elements (which lie
-    first in proj, dim_dev apart) | its rotated part | zeros], for attention against keys expanded per head."""
+    first in proj, dim_dev apart) | its rotated part | zeros], for attention against keys expanded per head.
+    absorb [heads, latent_dev, dim_dev] of proj's type: the first absorb_rows rows' unrotated parts times their head's matrix
+    as well, into q_out[n, a, :latent_dev]."""
     n, width, ld = _rows(proj, "proj")
     rot = 2 * cos.shape[1]
     _need(tuple(cos.shape) == (n, rot // 2) and tuple(sin.shape) == (n, rot // 2) and cos.is_contiguous() and sin.is_contiguous()
@@ -926,12 +928,19 @@ def latent_finish(proj, q_col, c_col, kr_col, cos, sin, norm_weight, q_out, head
         hd = wf // heads
         _need(nf == n and wf == heads * hd and q_full.dtype == proj.dtype and hd >= dim + rot and dim_dev >= dim > 0
               and q_col >= heads * dim_dev, "q_full must be [n, heads * hd] with hd >= dim + rot")
+    if absorb is not None:
+        epf = 16 // proj.element_size()
+        _need(absorb.is_contiguous() and absorb.dtype == proj.dtype and tuple(absorb.shape) == (heads, latent_dev, dim_dev)
+              and 0 <= absorb_rows <= n and q_col >= heads * dim_dev, "absorb must be [heads, latent_dev, dim_dev] of proj's type")
+        _need(dim_dev % epf == 0 and latent_dev % 4 == 0 and ld % epf == 0 and proj.data_ptr() % 16 == 0,
+              "absorb needs 16-byte rows and heads")
     check(library().tw_latent_finish(dtype_id(proj.dtype), _dev(proj), ld, int(q_col), int(c_col), int(kr_col), _dev(cos), _dev(sin),
                                      _dev(norm_weight) if keys is not None else None, _dev(q_out), ldq,
                                      _dev(q_full) if q_full is not None else None, ld_full, int(dim), int(dim_dev), int(hd),
                                      int(full_from), _dev(keys) if keys is not None else None, _dev(values) if keys is not None else None,
                                      _dev(slots, torch.int32, "slots") if keys is not None else None, n, heads, int(latent),
-                                     int(latent_dev), int(rot_dev), rot, page, float(eps), _stream()), "latent_finish")
+                                     int(latent_dev), int(rot_dev), rot, page, float(eps),
+                                     _dev(absorb) if absorb is not None else None, int(absorb_rows), _stream()), "latent_finish")
 
 
 def latent_decode_splits(n_seqs, heads, max_kv_len):
@@ -942,19 +951,31 @@ def latent_decode_workspace_floats(n_seqs, heads, latent_dev, splits):
     return int(library().tw_latent_decode_workspace_floats(int(n_seqs), int(heads), int(latent_dev), int(splits)))
 
 
-def latent_decode(q, keys, values, block_table, q_start, kv_len, n_seqs, out, heads, scale, splits=1, workspace=None, sink=None):
+def latent_decode(q, keys, values, block_table, q_start, kv_len, n_seqs, out, heads, scale, splits=1, workspace=None, sink=None,
+                  expand=None, out_stride=0, gate=None):
     """Attention of sequences 0 .. n_seqs - 1, ONE query token each, all heads against the one cached head: softmax of
     scale * q_a . key over the sequence's keys, times the values (the first latent_dev elements of the key rows).
     q [rows, heads * K] (head a at a * K), keys [pages, 1, page, K], values [pages, 1, latent_dev, page] (the same
     elements, transposed inside a page), out [rows, heads * latent_dev]. splits > 1 cuts every sequence's keys into
     ranges for separate workgroups; needs a float32 workspace of `latent_decode_workspace_floats` floats. sink float32
-    [heads]: exp(sink_a) more in head a's denominator (no key, no value, not scaled)."""
+    [heads]: exp(sink_a) more in head a's denominator (no key, no value, not scaled).
+    expand [heads, size, latent_dev] of q's type: out [rows, heads * out_stride] takes every head's result (rounded to that type)
+    times its matrix instead, head a at a * out_stride; gate (laid out like out): times sigmoid(gate). Needs the workspace
+    for one range too."""
     _need(sink is None or (sink.dtype == torch.float32 and sink.is_contiguous() and sink.numel() == heads), "sink must be float32 [heads]")
     page, K = keys.shape[2], keys.shape[3]
     Lp = values.shape[2]
     nq, wq, ldq = _rows(q, "q")
     no, wo, ldo = _rows(out, "out")
-    _need(wq == heads * K and wo == heads * Lp and no >= n_seqs and nq >= n_seqs, "latent_decode q/out shapes do not agree")
+    _need(wq == heads * K and (expand is not None or wo == heads * Lp) and no >= n_seqs and nq >= n_seqs, "latent_decode q/out shapes do not agree")
+    size = ldg = 0
+    if expand is not None:
+        size = expand.shape[1]
+        _need(expand.is_contiguous() and expand.dtype == q.dtype and tuple(expand.shape) == (heads, size, Lp) and size % 4 == 0
+              and out_stride >= size and (heads - 1) * out_stride + size <= wo, "expand must be [heads, size, latent_dev] of q's type, out as wide")
+    if gate is not None:
+        ng, wg, ldg = _rows(gate, "gate")
+        _need(expand is not None and ng >= n_seqs and (heads - 1) * out_stride + size <= wg and gate.dtype == q.dtype, "gate must be laid out like out")
     _need(out.dtype == q.dtype == keys.dtype == values.dtype, "attention operand types differ")
     _need(keys.dim() == 4 and keys.shape[1] == 1 and keys.is_contiguous() and values.is_contiguous()
           and tuple(values.shape) == (keys.shape[0], 1, Lp, page), "keys [pages, 1, page, K], values [pages, 1, latent_dev, page]")
@@ -962,14 +983,15 @@ def latent_decode(q, keys, values, block_table, q_start, kv_len, n_seqs, out, he
     _need(block_table.dim() == 2 and block_table.stride(1) == 1 and block_table.shape[0] >= n_seqs, "block_table must be 2-D")
     _need(q_start.numel() >= n_seqs + 1 and kv_len.numel() >= n_seqs, "sequence metadata is too short")
     ws_ptr, ws_floats = None, 0
-    if splits > 1:
+    if splits > 1 or expand is not None:
         _need(workspace is not None and workspace.dtype == torch.float32, "split attention needs a float32 workspace")
         ws_ptr, ws_floats = _dev(workspace), workspace.numel()
     check(library().tw_latent_decode(dtype_id(q.dtype), _dev(q), ldq, _dev(keys), _dev(values),
                                      _dev(block_table, torch.int32, "block_table"), block_table.stride(0),
                                      _dev(q_start, torch.int32, "q_start"), _dev(kv_len, torch.int32, "kv_len"), int(n_seqs),
                                      _dev(out), ldo, ws_ptr, ws_floats, int(heads), K, Lp, page, float(scale), int(splits),
-                                     _dev(sink) if sink is not None else None, _stream()), "latent_decode")
+                                     _dev(sink) if sink is not None else None, _dev(expand) if expand is not None else None, size,
+                                     int(out_stride), _dev(gate) if gate is not None else None, ldg, _stream()), "latent_decode")
     return out
 
 

@@ -163,22 +163,19 @@ class LatentAttention(Mixer):
         q_full = ctx.scratch("latent.q_full", (n, H * hd)) if portions else None
         store = dict(keys=keys, values=values, slots=group.slot_mapping) if self.own_latent else {}
         ops.latent_finish(proj, self.q_col, self.c_col, self.kr_col, cos, sin, self.latent_norm, q, H, self.latent, Lp, Rp,
-                          self.eps, q_full=q_full, dim=self.dim, dim_dev=self.dim_dev, full_from=nd, **store)
+                          self.eps, q_full=q_full, dim=self.dim, dim_dev=self.dim_dev, full_from=nd,
+                          absorb=self.absorb if nd else None, absorb_rows=nd, **store)
         out = ctx.scratch("latent.out", (n, H * hd))
+        gate = proj[:, self.g_col:self.g_col + H * hd] if self.gate_name else None
         if nd:
-            # one-token sequences: all heads over the one cached head, W_uk on the query side, W_uv on the output side
-            ops.head_linear(proj[:nd], self.dim_dev, self.absorb, q[:nd], K)
-            mixed = ctx.scratch("latent.mixed", (n, H * Lp))[:nd]
+            # one-token sequences: all heads over the one cached head, W_uk on the query side (above), W_uv and the gate behind
             longest = ctx.kv_bound if ctx.capturing else ctx.max_kv_len
             splits = ops.latent_decode_splits(nd, H, longest)
-            ws = None
-            if splits > 1:
-                # sized for the most splits any length class can ask for, so that it never grows under a capture
-                floats = ops.latent_decode_workspace_floats(nd, H, Lp, max(splits, ops.latent_decode_splits(nd, H, ctx.kv_capacity)))
-                ws = ctx.workspace.get("latent.split", (floats,), torch.float32)
-            ops.latent_decode(q[:nd], keys, values, group.block_table, ctx.q_start, ctx.kv_len, nd, mixed, H, self.scale,
-                              splits=splits, workspace=ws, sink=self.sink)
-            ops.head_linear(mixed, Lp, self.expand, out[:nd], hd)
+            # sized for the most splits any length class can ask for, so that it never grows under a capture
+            floats = ops.latent_decode_workspace_floats(nd, H, Lp, max(splits, ops.latent_decode_splits(nd, H, ctx.kv_capacity)))
+            ws = ctx.workspace.get("latent.split", (floats,), torch.float32)
+            ops.latent_decode(q[:nd], keys, values, group.block_table, ctx.q_start, ctx.kv_len, nd, out, H, self.scale,
+                              splits=splits, workspace=ws, sink=self.sink, expand=self.expand, out_stride=hd, gate=gate)
         if portions:
             # prompt portions: their sequences' cached latents expanded per head into pages of this step's own
             own_pages = ctx.h_kv_page_start[ctx.n_seqs] - ctx.h_kv_page_start[nd]
@@ -196,8 +193,8 @@ class LatentAttention(Mixer):
                 ws = ctx.workspace.get("attn.prefill_split", (ops.attn_prefill_workspace_floats(n, H, hd, split[0]),), torch.float32)
             ops.attn_prefill(q_full, own_keys, own_values, own_table, ctx.q_start, ctx.kv_len, nd,
                              portions, longest_portion, out, H, H, hd, self.scale, split=split, workspace=ws, sink=self.sink)
-        if self.gate_name:
-            ops.sigmoid_gate(out, proj[:, self.g_col:self.g_col + H * hd])
+            if gate is not None:
+                ops.sigmoid_gate(out[nd:], gate[nd:])
         if ctx.defer_sums and self.o.deferrable(n):
             return self.o.forward_partials(ctx, out, "o")          # whoever norms next adds them up
         self.o.forward(ctx, out, x, residual=x if accumulate else None)

@@ -202,6 +202,61 @@ def test_one_token_attention_over_the_cached_latent(device, dtype, H, L, R, page
         assert err < (3e-2 if dtype == "bfloat16" else 2e-5), (s, err)
 
 
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("H,L,R,D,E,page,lengths,splits,gated", [
+    (16, 192, 64, 64, 128, 16, [1, 16, 17, 64, 65, 200], 0, True),        # the sizes with compile-time loops; tile and group edges
+    (17, 192, 64, 64, 144, 32, [300], 64, False),                         # one row, most ranges, a second tile of heads
+    (3, 192, 64, 8, 16, 16, list(range(1, 18)), 2, True),                 # a second tile of rows; threads with several elements each
+    (5, 48, 16, 24, 20, 4, [40, 7], 3, True),                             # the last k-step ends inside itself, columns inside a tile
+    (2, 240, 16, 16, 64, 12, [5, 130], 1, True),                          # a page size that is no power of two
+])
+def test_one_token_latent_attention_between_its_products(device, dtype, H, L, R, D, E, page, lengths, splits, gated):
+    """W_uk on the query side, attention over the cached latent, W_uv and the gate behind it, against the same in 64 bits: the
+    two launches in front of and behind the attention hold what four separate ones would."""
+    from tessweave_engine_amd.kernels import ops
+    dt, n, K = tdtype(dtype), len(lengths), L + R
+    g = torch.Generator().manual_seed(H * 10 + L + n)
+    blocks = [(T + page - 1) // page for T in lengths]
+    keys = torch.full((sum(blocks) + 1, 1, page, K), float("nan"), dtype=dt)
+    values = torch.full((sum(blocks) + 1, 1, L, page), float("nan"), dtype=dt)
+    table = torch.full((n, max(blocks)), -1, dtype=torch.int32)
+    q_col, g_col = H * D, H * (D + R)
+    proj = torch.randn(n, (g_col + H * (E + 4) + 7) // 8 * 8, generator=g).to(dt)         # (rows of whole 16 bytes)
+    absorb = (torch.randn(H, L, D, generator=g) / D ** 0.5).to(dt)
+    expand = (torch.randn(H, E, L, generator=g) / L ** 0.5).to(dt)
+    sink, scale, want, free = torch.randn(H, generator=g), 0.4 * K ** -0.5, [], list(range(sum(blocks)))
+    gate = proj[:, g_col:g_col + H * (E + 4)].reshape(n, H, E + 4)[..., :E].double()
+    for s, T in enumerate(lengths):
+        rows = torch.randn(T, K, generator=g).to(dt)
+        for b in range(blocks[s]):
+            pg = table[s, b] = free.pop()
+            part = rows[b * page:(b + 1) * page]
+            keys[pg, 0, :len(part)], values[pg, 0, :, :len(part)] = part, part[:, :L].T
+        plain_part = torch.einsum("ald,ad->al", absorb.double(), proj[s, :q_col].view(H, D).double())
+        turned = proj[s, q_col:g_col].view(H, R).double()
+        sc = torch.cat([plain_part, turned], 1) @ rows.double().T * scale
+        p = torch.softmax(torch.cat([sc, sink.double().view(H, 1)], 1), 1)[:, :T]
+        o = torch.einsum("ael,al->ae", expand.double(), p @ rows[:, :L].double())
+        want.append(o * torch.sigmoid(gate[s]) if gated else o)
+    q = torch.full((n, H * K), float("nan"), dtype=dt, device=device)
+    dev = proj.to(device)
+    none = torch.ones(n, R // 2, device=device)                           # an angle of zero: the rotated parts pass
+    ops.latent_finish(dev, q_col, 0, 0, none, torch.zeros_like(none), None, q, H, L, L, R, 1e-6, dim=D, dim_dev=D,
+                      absorb=absorb.to(device), absorb_rows=n)
+    splits = splits or ops.latent_decode_splits(n, H, max(lengths))
+    ws = torch.full((ops.latent_decode_workspace_floats(n, H, L, splits),), float("nan"), device=device)
+    out = torch.full((n, H * (E + 4)), 7.0, dtype=dt, device=device)
+    ops.latent_decode(q, keys.to(device), values.to(device), table.to(device), ints(list(range(n + 1)), device), ints(lengths, device),
+                      n, out, H, scale, splits=splits, workspace=ws, sink=sink.to(device), expand=expand.to(device), out_stride=E + 4,
+                      gate=dev[:, g_col:] if gated else None)
+    got = out.cpu().double().view(n, H, E + 4)
+    assert (got[..., E:] == 7.0).all()
+    want = torch.stack(want)
+    # bfloat16 rounds the latent queries, the probabilities, the mixed latents and the results, 2^-9 each: 4 x 2^-9 of values around 1
+    err = ((got[..., :E] - want).abs().amax() / want.abs().amax()).item()
+    assert err < (2e-2 if dtype == "bfloat16" else 1e-5), err
+
+
 def retention_case(H, D, E, rot_dims, decay, lengths, seed):
     """Raw projections [T, 2 H D + 2 H E] of several sequences and what the mechanism gives for each (float64)."""
     g = torch.Generator().manual_seed(seed)
