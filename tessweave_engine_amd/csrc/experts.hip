@@ -325,8 +325,10 @@ __global__ __launch_bounds__(256) void moe_gather_kernel(const T* __restrict__ h
 // of 32). GLU: W and W2 are gate and up, the result glu(gate, up) goes out in the compute type; otherwise the float32
 // product. Operands go from memory straight into fragments (lane = 16 * piece + row reads 16 bytes).
 // SPLITK (steps of few rows, where the tiles in use are too few to fill the chip and every one streams its expert's whole
-// matrix; some of many rows, see moe_splits_k): the four waves share one range of NT x 16 columns and take every
-// fourth step over K each; their sums meet in LDS and are added in the order of the waves.
+// matrix; some of many rows, see moe_splits_k): the waves share one range of NT x 16 columns and take every WAVES-th
+// step over K each; their sums meet in LDS and are added in the order of the waves. The ranges are the grid's first dimension there:
+// workgroups go round the 8 XCDs in that order, and with the tiles first all ranges of a tile met on one XCD, so that five tiles
+// kept five eighths of the chip busy and ten one eighth for twice as long (see moe_few_form).
 // MT > 1 (steps of many rows, whose experts' shares are padded to MT tiles): a workgroup takes MT tiles of one expert
 // against every fragment of the expert's matrices it reads.
 template <int N> struct MoeCount { static constexpr int value = N; };
@@ -343,14 +345,14 @@ struct MoePairs {
   int* tile_expert;
   int* pos;
 };
-template <typename T, int ACT, int NT, bool SPLITK = false, int MT = 1, bool PLAN = false>
-__global__ __launch_bounds__(256) void moe_grouped_kernel(const T* __restrict__ A, long lda, const T* __restrict__ W,
+template <typename T, int ACT, int NT, bool SPLITK = false, int MT = 1, bool PLAN = false, int WAVES = 4, int STEPS = 4, bool AHEAD = false>
+__global__ __launch_bounds__(WAVES * 64) void moe_grouped_kernel(const T* __restrict__ A, long lda, const T* __restrict__ W,
                                                           const T* __restrict__ W2, const int* __restrict__ tile_expert,
                                                           void* __restrict__ out, long ldo, int N, int K, float limit,
                                                           MoePairs pairs = {}) {
   constexpr int EPF = Elem<T>::kPerFrag;
   constexpr bool GLU = ACT == 1 || ACT == 3;
-  const int tile = blockIdx.x * MT;
+  const int tile = (SPLITK ? blockIdx.y : blockIdx.x) * MT, range = SPLITK ? blockIdx.x : blockIdx.y;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int r = lane & 15, g = lane >> 4;
   int ex, row_of_lane = 0;                           // PLAN: the row of h that lane's row r of the tile is
@@ -369,7 +371,7 @@ __global__ __launch_bounds__(256) void moe_grouped_kernel(const T* __restrict__ 
       for (int i = 0; i < tile && left; ++i) left &= left - 1;
       if (left) opener = __ffsll((unsigned long long)left) - 1;
     }
-    const bool leads = blockIdx.y == 0 && wave == 0;
+    const bool leads = range == 0 && wave == 0;
     if (leads && tile == 0 && lane < pairs.items && !real) pairs.pos[lane] = -1;
     if (opener < 0) {
       if (leads && lane == 0) pairs.tile_expert[tile] = -1;
@@ -395,11 +397,11 @@ __global__ __launch_bounds__(256) void moe_grouped_kernel(const T* __restrict__ 
     ex = tile_expert[tile];
     if (ex < 0) return;
   }
-  const int col0 = (SPLITK ? blockIdx.y : blockIdx.y * 4 + wave) * 16 * NT;
+  const int col0 = (SPLITK ? range : range * 4 + wave) * 16 * NT;
   if (col0 >= N) return;
   constexpr int KSTEP = 4 * EPF;
   constexpr int BLK = 64 * EPF;                      // elements of one step's fragment of a tile: lane l's at l * EPF
-  constexpr int k_stride = (SPLITK ? 4 : 1) * BLK;    // (k counts the elements of a tile's fragments, step after step)
+  constexpr int k_stride = (SPLITK ? WAVES : 1) * BLK;    // (k counts the elements of a tile's fragments, step after step)
   const int k_first = SPLITK ? wave * BLK : 0;
   const size_t tile_elems = (size_t)K * TW_MOE_TILE;  // all steps of one tile of 16 rows
   const int n_blocks = (N + 15) / 16;
@@ -417,10 +419,9 @@ __global__ __launch_bounds__(256) void moe_grouped_kernel(const T* __restrict__ 
   for (int m = 0; m < MT; ++m)
 #pragma unroll
     for (int t = 0; t < NT; ++t) acc[m][t] = acc2[m][t] = f32x4{0.f, 0.f, 0.f, 0.f};
-  // U steps' operands are on their way before the first is used, where waves share columns of many rows those of the U steps
-  // behind them too: what bounds this loop is the latency of memory (few rows are not faster by it: their workgroups, two and
-  // more a CU, cover each other's)
-  constexpr int U = MT > 1 ? 2 : GLU ? 4 : (NT > 2 ? 4 : 8);
+  // U steps' operands are on their way before the first is used, where waves share columns of many rows (and in AHEAD) those of
+  // the U steps behind them too: what bounds this loop is the latency of memory
+  constexpr int U = MT > 1 ? 2 : GLU ? STEPS : (NT > 2 ? STEPS : 2 * STEPS);
   struct Operands {
     typename Elem<T>::Frag a[U][MT], b[U][NT], b2[GLU ? U : 1][NT];
   };
@@ -451,11 +452,11 @@ __global__ __launch_bounds__(256) void moe_grouped_kernel(const T* __restrict__ 
           tw_mma16(acc[m][t], o.a[u][m], o.b[u][t]);
           if (GLU) tw_mma16(acc2[m][t], o.a[u][m], o.b2[GLU ? u : 0][t]);
         }
-    if constexpr (SPLITK && MT > 1) __builtin_amdgcn_sched_barrier(0);
+    if constexpr (SPLITK && (MT > 1 || AHEAD)) __builtin_amdgcn_sched_barrier(0);
   };
   int k = k_first;
   const int k_end = (int)tile_elems;
-  if constexpr (SPLITK && MT > 1) {
+  if constexpr (SPLITK && (MT > 1 || AHEAD)) {
     constexpr int BATCH = U * k_stride;
     const int last = k_end - (U - 1) * k_stride;     // a batch that begins before it is whole
     Operands even, odd;
@@ -517,7 +518,7 @@ __global__ __launch_bounds__(256) void moe_grouped_kernel(const T* __restrict__ 
     for (; k < k_end; k += k_stride) steps(k, MoeCount<1>());
   }
   if constexpr (SPLITK) {
-    __shared__ f32x4 part[GLU ? 2 : 1][3][MT][NT][64];
+    __shared__ f32x4 part[GLU ? 2 : 1][WAVES - 1][MT][NT][64];
     if (wave > 0) {
 #pragma unroll
       for (int m = 0; m < MT; ++m)
@@ -530,7 +531,7 @@ __global__ __launch_bounds__(256) void moe_grouped_kernel(const T* __restrict__ 
     __syncthreads();
     if (wave > 0) return;
 #pragma unroll
-    for (int w = 0; w < 3; ++w)
+    for (int w = 0; w < WAVES - 1; ++w)
 #pragma unroll
       for (int m = 0; m < MT; ++m)
 #pragma unroll
@@ -631,6 +632,40 @@ static bool moe_splits_k(bool f32, int units, long items, int X, int C, int Cd, 
   return 1.4 * ranges / 4 < columns;
 }
 
+// Steps of few rows: columns a workgroup (NT x 16), waves and k-steps a request, by how many tiles can be in use. What bounds
+// them is the tail of the last workgroups and a wave's chain of requests, so the fewer tiles the smaller the pieces. float32
+// (whose MFMAs take as long as the loads) has 16 columns: 16 waves of 2 steps up to 16 tiles, 8 of 4 above; bfloat16 32 columns
+// and 4 waves of 4 steps, but up to 16 tiles of gated experts, 4 of plain ones, 16 columns and 8 waves with 2 steps on their way
+// behind 2. 16 experts of 2,048 x 1,408, two a token, gated, all launches of the experts, us (32 columns and 4 waves with the tiles
+// first in the grid / the same with the ranges first / this): float32 1 token 29.7 / 29.8 / 20.5, 2 33.1 / 33.8 / 33.6, 4 59.6 / 61.4 /
+// 51.0, 8 90.3 / 73.7 / 67.9, 32 120 / 101 / 99; bfloat16 1 token 18.0 / 18.1 / 13.4, 4 30.4 / 30.8 / 28.1, 8 42.8 / 38.0 / 37.5, 32
+// 57.6 / 52.1; plain bfloat16 1 token 14.2 / 14.4 / 11.6, 8 31.7 / 28.4; 128 experts of 2,048 x 768, 8 of them, 8 tokens: float32 187 /
+// 173 / 180, bfloat16 94.0 / 90.5.
+template <typename T, int ACT, bool PLAN, int NT, int WAVES, int STEPS, bool AHEAD>
+static void moe_few_form(const T* rows, const T* first, const T* second, const T* down, const int* tile_expert, T* act, float* ys, int C,
+                         int Cd, int Fd, float limit, int tiles, const MoePairs& pairs, hipStream_t stream) {
+  moe_grouped_kernel<T, ACT, NT, true, 1, PLAN, WAVES, STEPS, AHEAD><<<dim3(tw_div_up(Fd, 16 * NT), tiles), WAVES * 64, 0, stream>>>(
+      rows, Cd, first, second, tile_expert, act, Fd, Fd, Cd, limit, pairs);
+  moe_grouped_kernel<T, 0, NT, true, 1, false, WAVES, STEPS, AHEAD><<<dim3(tw_div_up(C, 16 * NT), tiles), WAVES * 64, 0, stream>>>(
+      act, Fd, down, nullptr, tile_expert, ys, C, C, Fd, 0.f, MoePairs{});
+}
+
+// tiles: of the launch; in_use: the most of them that can hold rows
+template <typename T, int ACT, bool PLAN>
+static void moe_few_products(const T* rows, const T* first, const T* second, const T* down, const int* tile_expert, T* act, float* ys,
+                             int C, int Cd, int Fd, float limit, int tiles, int in_use, const MoePairs& pairs, hipStream_t stream) {
+#define TW_MOE_FEW(...)                                                                                                           \
+  moe_few_form<T, ACT, PLAN, __VA_ARGS__>(rows, first, second, down, tile_expert, act, ys, C, Cd, Fd, limit, tiles, pairs, stream)
+  if constexpr (sizeof(T) == 4) {
+    if (in_use <= 16) TW_MOE_FEW(1, 16, 2, false);
+    else TW_MOE_FEW(1, 8, 4, false);
+  } else {
+    if (in_use <= (ACT == 1 || ACT == 3 ? 16 : 4)) TW_MOE_FEW(1, 8, 2, true);
+    else TW_MOE_FEW(2, 4, 4, false);
+  }
+#undef TW_MOE_FEW
+}
+
 // The two grouped products of a step: kind 0 gated with the limited swish, 1 up alone with gelu, 2 gated with SiLU, 3 up alone
 // with the square of relu.
 template <typename T, int ACT>
@@ -641,14 +676,12 @@ static void moe_products(const T* xs, const T* gate, const T* up, const T* down,
   const T* second = PLAIN ? nullptr : up;
   if (tiles <= TW_MOE_SPLITK_TILES) {
     // few rows: most tiles hold one or two rows and each streams its expert's matrices once; the waves then split K
-    moe_grouped_kernel<T, ACT, 2, true><<<dim3(tiles, tw_div_up(Fd, 16 * 2)), 256, 0, stream>>>(
-        xs, Cd, first, second, tile_expert, act, Fd, Fd, Cd, limit);
-    moe_grouped_kernel<T, 0, 2, true><<<dim3(tiles, tw_div_up(C, 16 * 2)), 256, 0, stream>>>(
-        act, Fd, down, nullptr, tile_expert, ys, C, C, Fd, 0.f);
+    moe_few_products<T, ACT, false>(xs, first, second, down, tile_expert, act, ys, C, Cd, Fd, limit, tiles,
+                                    items < tiles ? (int)items : tiles, MoePairs{}, stream);
   } else if (wide && moe_splits_k(sizeof(T) == 4, tiles / TW_MOE_WIDE, items, X, C, Cd, Fd, !PLAIN)) {
-    moe_grouped_kernel<T, ACT, 2, true, TW_MOE_WIDE><<<dim3(tiles / TW_MOE_WIDE, tw_div_up(Fd, 16 * 2)), 256, 0, stream>>>(
+    moe_grouped_kernel<T, ACT, 2, true, TW_MOE_WIDE><<<dim3(tw_div_up(Fd, 16 * 2), tiles / TW_MOE_WIDE), 256, 0, stream>>>(
         xs, Cd, first, second, tile_expert, act, Fd, Fd, Cd, limit);
-    moe_grouped_kernel<T, 0, 2, true, TW_MOE_WIDE><<<dim3(tiles / TW_MOE_WIDE, tw_div_up(C, 16 * 2)), 256, 0, stream>>>(
+    moe_grouped_kernel<T, 0, 2, true, TW_MOE_WIDE><<<dim3(tw_div_up(C, 16 * 2), tiles / TW_MOE_WIDE), 256, 0, stream>>>(
         act, Fd, down, nullptr, tile_expert, ys, C, C, Fd, 0.f);
   } else if (wide) {
     moe_grouped_kernel<T, ACT, 2, false, TW_MOE_WIDE><<<dim3(tiles / TW_MOE_WIDE, tw_div_up(Fd, 4 * 16 * 2)), 256, 0, stream>>>(
@@ -682,11 +715,8 @@ static void moe_products_few(const MoeStep& s, hipStream_t stream) {
   // (every tile is opened by a pair of its own, and the tiles in use never exceed what a plan could need)
   const int tiles = s.n * s.top < s.capacity / TW_MOE_TILE ? s.n * s.top : s.capacity / TW_MOE_TILE;
   const MoePairs pairs{s.ids, s.n * s.top, s.top, s.X, s.ld_h, const_cast<int*>(s.tile_expert), const_cast<int*>(s.pos)};
-  moe_grouped_kernel<T, ACT, 2, true, 1, true><<<dim3(tiles, tw_div_up(s.Fd, 16 * 2)), 256, 0, stream>>>(
-      (const T*)s.h, s.Cd, (const T*)(PLAIN ? s.up : s.gate), (const T*)(PLAIN ? nullptr : s.up), nullptr, s.act, s.Fd, s.Fd,
-      s.Cd, s.limit, pairs);
-  moe_grouped_kernel<T, 0, 2, true><<<dim3(tiles, tw_div_up(s.C, 16 * 2)), 256, 0, stream>>>(
-      (const T*)s.act, s.Fd, (const T*)s.down, nullptr, s.tile_expert, s.ys, s.C, s.C, s.Fd, 0.f);
+  moe_few_products<T, ACT, true>((const T*)s.h, (const T*)(PLAIN ? s.up : s.gate), (const T*)(PLAIN ? nullptr : s.up), (const T*)s.down,
+                                 s.tile_expert, (T*)s.act, s.ys, s.C, s.Cd, s.Fd, s.limit, tiles, tiles, pairs, stream);
 }
 
 // Can the first product find its tiles and rows itself? (few pairs, rows of h that are whole fragments)

@@ -450,6 +450,16 @@ def test_grouped_experts_of_many_rows_and_long_sums(device, dtype, kind, n, X, t
     assert torch.allclose(x.double(), want, atol=2e-5 if dtype == "float32" else 4e-2)
 
 
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("kind", ["silu", "gelu", "swish_limited"])
+@pytest.mark.parametrize("n,X,top,C,F", [(1, 4, 2, 32, 32), (8, 32, 2, 544, 96), (2, 24, 2, 288, 1088), (17, 40, 1, 800, 144), (16, 20, 4, 256, 288),
+                                         (13, 30, 5, 64, 80)])
+def test_grouped_experts_of_few_rows(device, dtype, kind, n, X, top, C, F):
+    """Up to and past 4, 16 and 64 tiles and 64 pairs, K from less than a step a wave to several requests and a tail, columns that end
+    inside a workgroup's. The oracle and the bars of the steps of many rows; sums are shorter."""
+    test_grouped_experts_of_many_rows_and_long_sums(device, dtype, kind, n, X, top, C, F)
+
+
 # ---------------------------------------------------------------------------------------------------------
 # whole models
 
