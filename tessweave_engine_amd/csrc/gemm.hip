@@ -900,13 +900,13 @@ static int launch_narrow(const T* A, long lda, const T* W, long ldw, const float
 
 // force: 0 = choose, 1 = generic, 3 = tiled 128x128, 4 = tiled 128x256, 5 = skinny, 6 = tiled 256x256,
 // 7 = tiled 256x192, 8 = streaming with one workgroup per CU (shuffled weights, up to 64 rows),
-// 9 = whole K per workgroup (shuffled weights, up to 16 rows)
+// 9 = whole K per workgroup (shuffled weights, up to 16 rows), 10 to 14 = tiled 192x128, 192x192, 192x256, 192x384, 256x320 (shuffled bfloat16)
 template <typename T, typename OutT, bool SHUF, bool GLU>
 static int linear_dispatch(const T* A, long lda, const T* W, long ldw, const float* bias,
                            const float* residual, long ldr, OutT* C, long ldc, float* partial,
                            long partial_bytes, int M, int N, int K, int force, hipStream_t stream) {
   constexpr int EPF = Elem<T>::kPerFrag;
-  TW_REQUIRE(force == 0 || force == 1 || (force >= 3 && force <= 9));
+  TW_REQUIRE(force == 0 || force == 1 || (force >= 3 && force <= 14));
   // the shuffled layout exists only for K that is a multiple of 16 bytes and is always aligned
   const bool aligned = K % EPF == 0 && lda % EPF == 0 && ((uintptr_t)A % 16 == 0) && ((uintptr_t)W % 16 == 0) &&
                        (SHUF || ldw % EPF == 0);
@@ -933,7 +933,7 @@ static int linear_dispatch(const T* A, long lda, const T* W, long ldw, const flo
     TW_REQUIRE(M <= 64);
     return launch_skinny_lds_m<T, OutT, false, SHUF, GLU>(A, lda, W, ldw, bias, residual, ldr, C, ldc, partial, partial_bytes, M, N, K, stream);
   }
-  const int shape = force == 3 ? 1 : (force == 4 ? 2 : (force == 6 ? 3 : (force == 7 ? 4 : 0)));
+  const int shape = force >= 10 ? force - 5 : force == 3 ? 1 : (force == 4 ? 2 : (force == 6 ? 3 : (force == 7 ? 4 : 0)));
   return tw_tiled_linear(sizeof(T) == 4 ? TW_DTYPE_F32 : TW_DTYPE_BF16, sizeof(OutT) == 4 ? 1 : 0, SHUF ? 1 : 0,
                          GLU ? 1 : 0, shape, A, lda, W, ldw, bias, residual, ldr, C, ldc, partial, partial_bytes,
                          M, N, K, stream);

@@ -726,8 +726,9 @@ __global__ __launch_bounds__(256) void gemm_dma_kernel(const bf16_t* __restrict_
 // The same product with EIGHT waves, two a SIMD, that take turns: while one wave of a SIMD multiplies, the other reads its
 // next fragments from LDS and issues copies. K a multiple of 64, 16-byte rows of the result.
 //
-// The waves form a grid of ROWS x 8 / ROWS, each holds 64 x 32 Q of the tile: 256 x 64 Q (ROWS 4) or 128 x 128 Q (ROWS 2).
-// A k-tile is 64 elements of K, and a PHASE is 32 columns of a wave's tile in one k-tile: 16 MFMAs (256 clocks) between two
+// The waves form a grid of ROWS x 8 / ROWS, each holds 16 RT x 32 Q of the tile: with RT of 4 256 x 64 Q (ROWS 4) or 128 x 128 Q
+// (ROWS 2), with 3 192 x 64 Q (for rows that would leave a third of 256 empty).
+// A k-tile is 64 elements of K, and a PHASE is 32 columns of a wave's tile in one k-tile: 4 RT MFMAs (256 clocks at 4) between two
 // barriers, behind the reads of those columns of W and, in a k-tile's first phase, of the wave's rows of A. Waves 4..7 pass one
 // barrier more at the start, so that each wave's reads, copies and waits fall into the time in which the other wave of its
 // SIMD multiplies (with one wave a SIMD a copy that misses the vector cache held up the MFMAs behind it: a fifth of the
@@ -779,9 +780,9 @@ __device__ __forceinline__ f32x4 tw_buffer_load16(__amdgpu_buffer_rsrc_t from, i
 #define TW_OUTSIDE ((int)0x80000000)   /* an offset that no buffer of tw_buffer holds */
 
 // The shape of a tile and the order of its copies.
-template <int ROWS, int Q>
+template <int ROWS, int Q, int RT = 4>
 struct Turns {
-  static constexpr int COLS = 8 / ROWS, BM = 64 * ROWS, BN = 32 * Q * COLS;
+  static constexpr int COLS = 8 / ROWS, BM = 16 * RT * ROWS, BN = 32 * Q * COLS;
   static constexpr int A_STAGE = BM * 128, W_STAGE = BN * 128;
   static constexpr int STAGES = 144 * 1024 / (A_STAGE + W_STAGE) > 4 ? 4 : 144 * 1024 / (A_STAGE + W_STAGE);
   static constexpr int LDS = STAGES * (A_STAGE + W_STAGE) + 2 * BN * 4;    // (behind the stages the bias of two tiles)
@@ -811,15 +812,15 @@ __device__ __forceinline__ void tw_wait_accesses() {
   asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
 }
 
-template <typename OutT, int ROWS, int Q, bool GLU, bool PIECES>
+template <typename OutT, int ROWS, int Q, int RT, bool GLU, bool PIECES>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void gemm_turns_kernel(const bf16_t* __restrict__ A, long lda, const bf16_t* __restrict__ W, long k_steps, const float* __restrict__ bias,
                        const float* residual, long ldr, OutT* C, long ldc, int M, int N, int k_tiles_all, int tiles_m, int n_blocks,
                        int splits, int per_split, int piece, float* __restrict__ partial) {
-  typedef Turns<ROWS, Q> S;
+  typedef Turns<ROWS, Q, RT> S;
   static_assert(!PIECES || (ROWS == 2 && !GLU));
   constexpr int BM = S::BM, BN = S::BN, BAND = 2048 / BM;            // (bands of rows as above)
-  constexpr int STORES = sizeof(OutT) == 4 ? 8 * Q : GLU ? 2 * Q : 4 * Q;   // a tile's, of every wave
+  constexpr int STORES = sizeof(OutT) == 4 ? 2 * RT * Q : GLU ? RT * (Q / 2) + Q % 2 * ((RT + 1) / 2) : RT * Q;   // a tile's, of every wave
   constexpr int W_RING = S::STAGES * S::A_STAGE, BIAS = W_RING + S::STAGES * S::W_STAGE;
   extern __shared__ __attribute__((aligned(16))) char lds[];
   // Workgroup x of the 8 XCDs' 32 takes tiles x / 8, x / 8 + 32, ... of its XCD's run of neighbouring tiles.
@@ -833,11 +834,11 @@ void gemm_turns_kernel(const bf16_t* __restrict__ A, long lda, const bf16_t* __r
   const int wm = wave / S::COLS, wn = wave % S::COLS;                // (waves 0..3: the upper half of the rows)
   const int turn = wave >> 2;
 
-  f32x4 acc[4][2 * Q], before[PIECES ? 4 : 1][PIECES ? 2 * Q : 1];   // (of this piece of K; of those before it)
+  f32x4 acc[RT][2 * Q], before[PIECES ? RT : 1][PIECES ? 2 * Q : 1];   // (of this piece of K; of those before it)
   int left;                                                          // k-tiles until a piece ends
   auto clear = [&]() {
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+    for (int i = 0; i < RT; ++i)
 #pragma unroll
       for (int j = 0; j < 2 * Q; ++j) {
         acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -900,12 +901,12 @@ void gemm_turns_kernel(const bf16_t* __restrict__ A, long lda, const bf16_t* __r
     else copy_w(S::piece(P), k > of_a);
   };
 
-  // this lane's fragments in a stage: of A chunk 4 c + g of row 64 wm + 16 i + r, of W the same chunk of column 16 j + r of a block
-  bf16x8 af[4][2], wf[2][2];
+  // this lane's fragments in a stage: of A chunk 4 c + g of row 16 RT wm + 16 i + r, of W the same chunk of column 16 j + r of a block
+  bf16x8 af[RT][2], wf[2][2];
   const int r0 = lane & 15, g0 = lane >> 4;
   int a_frag[2];
 #pragma unroll
-  for (int c = 0; c < 2; ++c) a_frag[c] = (wm * 64 + r0) * 128 + (((4 * c + g0) ^ ((r0 >> 1) & 7)) * 16);
+  for (int c = 0; c < 2; ++c) a_frag[c] = (wm * 16 * RT + r0) * 128 + (((4 * c + g0) ^ ((r0 >> 1) & 7)) * 16);
   const int w_frag = W_RING + wn * 4096 * Q + lane * 16;
   int stage = 0, phases = 0;                                         // the k-tile's stage; the tile's phases before it
   bool behind_stores = false;                                        // a tile was stored before this one
@@ -915,7 +916,7 @@ void gemm_turns_kernel(const bf16_t* __restrict__ A, long lda, const bf16_t* __r
 #pragma unroll
       for (int c = 0; c < 2; ++c)
 #pragma unroll
-        for (int i = 0; i < 4; ++i) af[i][c] = *reinterpret_cast<const bf16x8*>(lds + a_frag[c] + stage * S::A_STAGE + i * 2048);
+        for (int i = 0; i < RT; ++i) af[i][c] = *reinterpret_cast<const bf16x8*>(lds + a_frag[c] + stage * S::A_STAGE + i * 2048);
     }
 #pragma unroll
     for (int c = 0; c < 2; ++c)
@@ -926,7 +927,7 @@ void gemm_turns_kernel(const bf16_t* __restrict__ A, long lda, const bf16_t* __r
     if constexpr (PIECES && P == 0) {
       if (left == 0) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
+        for (int i = 0; i < RT; ++i)
 #pragma unroll
           for (int j = 0; j < 2 * Q; ++j) {
             before[i][j] = before[i][j] + acc[i][j];
@@ -941,10 +942,10 @@ void gemm_turns_kernel(const bf16_t* __restrict__ A, long lda, const bf16_t* __r
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     __builtin_amdgcn_s_barrier();
     __builtin_amdgcn_sched_barrier(0);
-    tw_unroll<16>([&](auto which) {
-      constexpr int m = decltype(which)::value, c = m / 8, i = m / 2 % 4, j = m % 2;
+    tw_unroll<4 * RT>([&](auto which) {
+      constexpr int m = decltype(which)::value, c = m / (2 * RT), i = m / 2 % RT, j = m % 2;
       tw_mma16(acc[i][2 * P + j], wf[j][c], af[i][c]);
-      constexpr int b = S::behind(P), gap = 16 / (b + 1);
+      constexpr int b = S::behind(P), gap = 4 * RT / (b + 1);
       if constexpr (b > 0 && (m + 1) % gap == 0 && (m + 1) / gap <= b) {
         __builtin_amdgcn_sched_barrier(0);
         copy(index, std::integral_constant<int, S::copies(P) - b + (m + 1) / gap - 1>{});
@@ -964,27 +965,27 @@ void gemm_turns_kernel(const bf16_t* __restrict__ A, long lda, const bf16_t* __r
   auto store_f32 = [&](auto adds_residual, __amdgpu_buffer_rsrc_t to, int ld, __amdgpu_buffer_rsrc_t add, int ld_add, bool biased,
                        int m0, int n0, auto act_of, int r, int g) {
     constexpr bool adds = decltype(adds_residual)::value;
-    // the residual of RT row tiles of 16 at a time (all four where the sums leave registers for it)
-    constexpr int RT = ROWS == 2 ? 4 : 1;
-    f32x4 res[RT][2 * Q];
-    tw_unroll<4>([&](auto index) {
+    // the residual of AT row tiles of 16 at a time (all four where the sums leave registers for it)
+    constexpr int AT = ROWS == 2 ? 4 : 1;
+    f32x4 res[AT][2 * Q];
+    tw_unroll<RT>([&](auto index) {
       constexpr int i = decltype(index)::value;
-      if constexpr (adds && i % RT == 0) {
+      if constexpr (adds && i % AT == 0) {
 #pragma unroll
-        for (int k = 0; k < RT; ++k)
+        for (int k = 0; k < AT; ++k)
 #pragma unroll
           for (int j = 0; j < 2 * Q; ++j) {
-            const int row = wm * 64 + (i + k) * 16 + r, col = wn * 32 * Q + j * 16 + 4 * g;
+            const int row = wm * 16 * RT + (i + k) * 16 + r, col = wn * 32 * Q + j * 16 + 4 * g;
             res[k][j] = tw_buffer_load16(add, row < M - m0 && col < N - n0 ? row * ld_add * 4 + col * 4 : TW_OUTSIDE);
           }
       }
-      const int row = wm * 64 + i * 16 + r;
+      const int row = wm * 16 * RT + i * 16 + r;
 #pragma unroll
       for (int j = 0; j < 2 * Q; ++j) {
         const int col = wn * 32 * Q + j * 16 + 4 * g;
         f32x4 v = acc[i][j];
         if (biased) v = v + bias_of(j, g);
-        if constexpr (adds) v = v + res[i % RT][j];
+        if constexpr (adds) v = v + res[i % AT][j];
         else {
 #pragma unroll
           for (int e = 0; e < 4; ++e) v[e] = tw_act(v[e], act_of());
@@ -1037,13 +1038,17 @@ void gemm_turns_kernel(const bf16_t* __restrict__ A, long lda, const bf16_t* __r
         auto offset = [&](int row, int col) {                // (columns of the result)
           return row < M - m0 && 2 * col < N - n0 ? row * (int)ldc * 2 + col * 2 : TW_OUTSIDE;
         };
-        tw_unroll<4>([&](auto index) {                       // two neighbouring column groups of a row tile together
+        tw_unroll<RT>([&](auto index) {                      // two neighbouring column groups of a row tile together
           constexpr int i = decltype(index)::value;
 #pragma unroll
           for (int p = 0; p + 1 < Q; p += 2)
-            store_pair(to, form(i, p), form(i, p + 1), offset(wm * 64 + i * 16 + r, wn * 16 * Q + p * 16 + (g & 1) * 16 + (g >> 1) * 8));
-          if constexpr (Q % 2 == 1 && i % 2 == 0)            // the last of an odd number: two row tiles
-            store_pair(to, form(i, Q - 1), form(i + 1, Q - 1), offset(wm * 64 + (i + (g & 1)) * 16 + r, wn * 16 * Q + (Q - 1) * 16 + (g >> 1) * 8));
+            store_pair(to, form(i, p), form(i, p + 1), offset(wm * 16 * RT + i * 16 + r, wn * 16 * Q + p * 16 + (g & 1) * 16 + (g >> 1) * 8));
+          if constexpr (Q % 2 == 1 && i % 2 == 0) {          // the last of an odd number: two row tiles, or the last one alone
+            const u32x2 first = form(i, Q - 1);
+            const int at = offset(wm * 16 * RT + (i + (g & 1)) * 16 + r, wn * 16 * Q + (Q - 1) * 16 + (g >> 1) * 8);
+            if constexpr (i + 1 < RT) store_pair(to, first, form(i + 1, Q - 1), at);
+            else store_pair(to, first, first, g & 1 ? TW_OUTSIDE : at);
+          }
         });
       };
       if (ldr == 0) gated([]() { return 0L; });
@@ -1051,9 +1056,9 @@ void gemm_turns_kernel(const bf16_t* __restrict__ A, long lda, const bf16_t* __r
     } else {
       const auto to = tw_buffer(C + (size_t)m0 * ldc + n0);
       with_act([&](auto act_of) {
-        tw_unroll<4>([&](auto index) {
+        tw_unroll<RT>([&](auto index) {
           constexpr int i = decltype(index)::value;
-          const int row = wm * 64 + i * 16 + r;
+          const int row = wm * 16 * RT + i * 16 + r;
 #pragma unroll
           for (int p = 0; p < Q; ++p) {
             u32x2 half[2];
@@ -1102,7 +1107,7 @@ void gemm_turns_kernel(const bf16_t* __restrict__ A, long lda, const bf16_t* __r
     }
     if constexpr (PIECES) {
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
+      for (int i = 0; i < RT; ++i)
 #pragma unroll
         for (int j = 0; j < 2 * Q; ++j) acc[i][j] = before[i][j] + acc[i][j];
     }
@@ -1196,11 +1201,11 @@ static bool turns_takes(int out_bytes, const void* A, long lda, long ldw, const 
          (residual == nullptr || S::BM * ldr * 4 < (1L << 31)) && (long)S::BM * N * 4 < (1L << 31);
 }
 
-template <typename OutT, int ROWS, int Q, bool GLU>
+template <typename OutT, int ROWS, int Q, int RT, bool GLU>
 static int launch_turns(const bf16_t* A, long lda, const bf16_t* W, long ldw, const float* bias, const float* residual, long ldr,
                         OutT* C, long ldc, float* partial, long partial_bytes, int M, int N, int K, int want_splits, int piece,
                         hipStream_t stream, TiledMode* mode = nullptr) {
-  typedef Turns<ROWS, Q> S;
+  typedef Turns<ROWS, Q, RT> S;
   const int tiles_m = tw_div_up(M, S::BM), tiles_n = tw_div_up(N, S::BN);
   int splits = GLU ? 1 : (want_splits > 0 ? want_splits : tiled_splits(M, N, K, 8, S::BM, S::BN));
   while ((splits - 1) * turns_per_split(K, splits) >= K / 64) --splits;
@@ -1215,7 +1220,7 @@ static int launch_turns(const bf16_t* A, long lda, const bf16_t* W, long ldw, co
   const int grid = (int)(n_blocks > 256 ? 256 : (n_blocks + 7) / 8 * 8);
   const int per_split = turns_per_split(K, splits);
   auto run = [&](auto in_pieces) {
-    auto kernel = gemm_turns_kernel<OutT, ROWS, Q, GLU, decltype(in_pieces)::value>;
+    auto kernel = gemm_turns_kernel<OutT, ROWS, Q, RT, GLU, decltype(in_pieces)::value>;
     static bool attribute_set = false;   // per instantiation
     if (!attribute_set) {
       hipError_t e = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, S::LDS);
@@ -1279,7 +1284,8 @@ static int launch_dma(const bf16_t* A, long lda, const bf16_t* W, long ldw, cons
 // last round.
 // (with the present epilogue, 8,192 x 37,888 x 3,584 in bfloat16, TFLOP/s plain / gated: 128x128 906 / 891, 128x256
 // 1,027 / 1,037, 256x256 1,195 / 1,179, 256x192 1,146 / 1,121)
-static const int kTileM[5] = {0, 128, 128, 256, 256}, kTileN[5] = {0, 128, 256, 256, 192};
+// (1 to 4: of every kernel; 5 to 9: of gemm_turns_kernel alone)
+static const int kTileM[10] = {0, 128, 128, 256, 256, 192, 192, 192, 192, 256}, kTileN[10] = {0, 128, 256, 256, 192, 128, 192, 256, 384, 320};
 static const double kTileRate[5] = {0, 0.76, 0.90, 1.05, 1.00};
 
 static int choose_shape(bool big_ok, int M, int N) {
@@ -1348,8 +1354,15 @@ static TilePlan choose_staged(bool big_ok, bool glu, int M, int N, int K, int ep
 // 2,048 x 2,048 in one sum instead of three ranges was off by 2.7e-7 of the result instead of 1.5e-7.)
 struct TurnsCost { double launch, tile, alone, full; };
 static const TurnsCost kTurnsCost[5] = {{}, {3.8, 1.45, 0.351, 0.482}, {4.3, 2.27, 0.589, 0.815}, {3.5, 5.29, 0.960, 1.363}, {3.2, 4.42, 0.759, 1.060}};
-static double turns_us(int shape, int splits, int M, int N, int K) {
-  const TurnsCost& c = kTurnsCost[shape];
+// Tiles of 192 rows, and of 320 columns, come after: they take a product where they are expected to be 3 % faster than the choice among
+// the four, all nine estimated from another 402 products in one sum (65 to 4,700 rows, 896 to 37,888 columns, K 512 to 8,192; 5 to 7 %
+// off). Over these the choice is then 1.8 % faster in the mean than among the four, none more than 1 % slower, and 0.4 % behind the
+// best of the nine. (With K ranges, which no product of that fit had, 8 %: products of 129 to 167 rows were 3 to 7 % slower at 3.) They fill what 128 and 256 rows leave (536 x 27,648 x 5,120 183 -> 145 us by 192x384, 521 x 22,016 x 2,048 59 -> 49 by 192x256,
+// 536 x 7,168 x 5,120 58.6 -> 54.8 by 192x128), and 256x320 has a tenth less to copy and to read a product than 256x256
+// (8,192 x 37,888 x 3,584 1,605 -> 1,549).
+static const TurnsCost kNineCost[10] = {{}, {4.1, 1.71, 0.361, 0.504}, {4.5, 2.95, 0.596, 0.819}, {1.0, 8.67, 0.982, 1.136}, {2.7, 5.83, 0.776, 0.955},
+                                        {4.2, 2.50, 0.535, 0.608}, {4.1, 3.97, 0.663, 0.808}, {3.1, 5.44, 0.843, 0.989}, {1.0, 9.36, 1.179, 1.298}, {1.0, 9.78, 1.194, 1.316}};
+static double turns_us(const TurnsCost& c, int shape, int splits, int M, int N, int K) {
   const long blocks = (long)tw_div_up(M, kTileM[shape]) * tw_div_up(N, kTileN[shape]) * splits;
   const double rounds = tw_div_up(blocks, 256), alone = rounds * c.alone;
   const double full = (M <= 512 && (double)N * K >= 5e7 ? rounds : blocks / 256.0) * c.full;
@@ -1372,17 +1385,21 @@ static TilePlan choose_turns(bool glu, int M, int N, int K) {
   const TilePlan staged = choose_staged(true, glu, M, N, K, 8);
   const int ranges = glu ? 1 : staged.splits > 0 ? staged.splits : tiled_splits(M, N, K, 8, kTileM[staged.shape], kTileN[staged.shape]);
   double best = 0;
-  for (int shape = 1; shape <= 4; ++shape)
+  auto ask = [&](const TurnsCost& cost, int shape, double of_ranges) {
     for (int splits = kTileM[shape] > 128 ? ranges : 1; splits <= (glu ? 1 : 8); ++splits) {
       if (splits > 1 && splits > ranges && K / splits < 512) break;
       // (pieces against as many ranges, 23 products of 8 to 128 tiles: level at 30 to 50 tiles and 1,024 of K, 10 % behind at 10
       // tiles and 20 to 40 % ahead at 80 and more)
-      const double t = turns_us(shape, splits, M, N, K) + (splits < ranges ? 1.2 : 0.0);
+      const double t = turns_us(cost, shape, splits, M, N, K) * (splits > 1 ? of_ranges : 1.0) + (splits < ranges ? 1.2 : 0.0);
       if (best == 0 || t < best) {
         best = t;
         plan = {shape, splits, splits < ranges ? turns_per_split(K, ranges) : 0};
       }
     }
+  };
+  for (int shape = 1; shape <= 4; ++shape) ask(kTurnsCost[shape], shape, 1.0);
+  best = 0.97 * turns_us(kNineCost[plan.shape], plan.shape, plan.splits, M, N, K) + (plan.piece ? 1.2 : 0.0);
+  for (int shape = 5; shape <= 9; ++shape) ask(kNineCost[shape], shape, 1.05);
   at = {M, N, K, (int)glu, plan};
   return plan;
 }
@@ -1410,17 +1427,26 @@ static int tiled_by_shape(int shape, const T* A, long lda, const T* W, long ldw,
   TilePlan plan = {shape, 0, 0};                    // a forced shape keeps the launcher's own rule
   bool turns = BIG;                                 // (each plan is for its own kernels: choose_turns for a product all of whose tiles they take)
   if (shape == 0) {
-    turns = BIG && turns_pay(GLU, residual != nullptr, M, N, K) && takes(Turns<4, 3>{}) && takes(Turns<4, 4>{}) && takes(Turns<2, 2>{}) && takes(Turns<2, 1>{});
+    turns = BIG && turns_pay(GLU, residual != nullptr, M, N, K) && takes(Turns<4, 3>{}) && takes(Turns<4, 4>{}) && takes(Turns<2, 2>{}) && takes(Turns<2, 1>{}) && takes(Turns<4, 6, 3>{}) && takes(Turns<4, 5, 4>{});
     plan = turns ? choose_turns(GLU, M, N, K) : choose_staged(BIG, GLU, M, N, K, Elem<T>::kPerFrag);
   }
   shape = plan.shape;
   const int splits = plan.splits;
   if constexpr (BIG) {
     // bfloat16 and shuffled weights: the kernels that copy straight into LDS, if K and the strides allow
-    if (turns && shape == 4 && takes(Turns<4, 3>{})) return launch_turns<OutT, 4, 3, GLU>(A, lda, W, ldw, bias, residual, ldr, C, ldc, partial, partial_bytes, M, N, K, splits, plan.piece, stream, mode);
-    if (turns && shape == 3 && takes(Turns<4, 4>{})) return launch_turns<OutT, 4, 4, GLU>(A, lda, W, ldw, bias, residual, ldr, C, ldc, partial, partial_bytes, M, N, K, splits, plan.piece, stream, mode);
-    if (turns && shape == 2 && takes(Turns<2, 2>{})) return launch_turns<OutT, 2, 2, GLU>(A, lda, W, ldw, bias, residual, ldr, C, ldc, partial, partial_bytes, M, N, K, splits, plan.piece, stream, mode);
-    if (turns && shape == 1 && takes(Turns<2, 1>{})) return launch_turns<OutT, 2, 1, GLU>(A, lda, W, ldw, bias, residual, ldr, C, ldc, partial, partial_bytes, M, N, K, splits, plan.piece, stream, mode);
+#define TW_TURNS(SHAPE, ROWS, Q, RT)                                                                                              \
+    if (turns && shape == SHAPE && takes(Turns<ROWS, Q, RT>{}))                                                                     \
+      return launch_turns<OutT, ROWS, Q, RT, GLU>(A, lda, W, ldw, bias, residual, ldr, C, ldc, partial, partial_bytes, M, N, K, splits, plan.piece, stream, mode)
+    TW_TURNS(1, 2, 1, 4);
+    TW_TURNS(2, 2, 2, 4);
+    TW_TURNS(3, 4, 4, 4);
+    TW_TURNS(4, 4, 3, 4);
+    TW_TURNS(5, 4, 2, 3);
+    TW_TURNS(6, 4, 3, 3);
+    TW_TURNS(7, 4, 4, 3);
+    TW_TURNS(8, 4, 6, 3);
+    TW_TURNS(9, 4, 5, 4);
+#undef TW_TURNS
     if (K % 32 == 0 && K >= 32 && lda % 8 == 0) {
       if (shape == 4) return launch_dma<OutT, 4, 3, GLU>(A, lda, W, ldw, bias, residual, ldr, C, ldc, partial, partial_bytes, M, N, K, splits, stream, mode);
       if (shape == 3) return launch_dma<OutT, 4, 4, GLU>(A, lda, W, ldw, bias, residual, ldr, C, ldc, partial, partial_bytes, M, N, K, splits, stream, mode);
@@ -1429,7 +1455,7 @@ static int tiled_by_shape(int shape, const T* A, long lda, const T* W, long ldw,
     if (shape == 3 || shape == 4)             // (K no multiple of 32: the register-staged 256x256 tile for both)
       return launch_tiled<T, OutT, 4, 4, SHUF, GLU>(A, lda, W, ldw, bias, residual, ldr, C, ldc, partial, partial_bytes, M, N, K, splits, stream, mode);
   }
-  if (shape == 3 || shape == 4) return TW_ERR_BAD_ARGUMENT;
+  if (shape >= 3) return TW_ERR_BAD_ARGUMENT;
   if (shape == 2)
     return launch_tiled<T, OutT, 2, 4, SHUF, GLU>(A, lda, W, ldw, bias, residual, ldr, C, ldc, partial, partial_bytes, M, N, K, splits, stream, mode);
   return launch_tiled<T, OutT, 2, 2, SHUF, GLU>(A, lda, W, ldw, bias, residual, ldr, C, ldc, partial, partial_bytes, M, N, K, splits, stream, mode);
@@ -1457,7 +1483,7 @@ static int tiled_by_layout(int shuffled, int glu, int shape, const void* A, long
 int tw_tiled_linear(int dtype, int out_f32, int shuffled, int glu, int shape, const void* A, long lda,
                     const void* W, long ldw, const float* bias, const float* residual, long ldr, void* C,
                     long ldc, float* partial, long partial_bytes, int M, int N, int K, hipStream_t stream) {
-  TW_REQUIRE(shape >= 0 && shape <= 4);
+  TW_REQUIRE(shape >= 0 && shape <= 9);
   if (dtype == TW_DTYPE_F32)
     return tiled_by_layout<float, float>(shuffled, glu, shape, A, lda, W, ldw, bias, residual, ldr, C, ldc, partial, partial_bytes, M, N, K, stream);
   if (dtype != TW_DTYPE_BF16) return TW_ERR_BAD_ARGUMENT;

@@ -310,6 +310,7 @@ def linear_glu(x, weight, out, bias=None, force=0, activation="silu", factor=1.0
 
 
 GEMM_AUTO, GEMM_GENERIC, GEMM_TILED, GEMM_TILED_WIDE, GEMM_SKINNY, GEMM_TILED_256, GEMM_TILED_256X192, GEMM_STREAM_CU, GEMM_NARROW = 0, 1, 3, 4, 5, 6, 7, 8, 9
+GEMM_TILED_192X128, GEMM_TILED_192X192, GEMM_TILED_192X256, GEMM_TILED_192X384, GEMM_TILED_256X320 = 10, 11, 12, 13, 14
 
 
 def linear(x, weight, out, bias=None, residual=None, workspace=None, force=GEMM_AUTO):

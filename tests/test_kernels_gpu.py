@@ -510,6 +510,46 @@ def test_linear_glu_of_waves_in_turns_goes_on_to_more_tiles(ops, device, m, n, k
         assert bool(((gated[:m].double().view(m, n // 32, 16) - value).abs() <= bound).all()) and bool(gated[m:].isnan().all())
 
 
+@pytest.mark.parametrize("shape", ["192X128", "192X192", "192X256", "192X384", "256X320"])
+@pytest.mark.parametrize("m,n,k", [(65, 32, 64), (193, 416, 192), (383, 1000, 448), (4200, 4128, 256), (4353, 6240, 320), (300, 264, 2304)])
+def test_linear_of_waves_in_turns_in_192_rows_and_320_columns(ops, device, shape, m, n, k):
+    """The same in the tiles whose waves hold three row tiles or five pairs of column tiles: one k-tile, rings of two and three
+    stages, rows and columns that end inside a wave's tile, a workgroup's second and third tile, K ranges; one sum over the whole of
+    K is the bits of the 128x128 tiles. Bounds as in test_linear_of_waves_in_turns."""
+    force = getattr(ops, "GEMM_TILED_" + shape)
+    x = rand((m, k), torch.bfloat16, device, 1.0, seed=1)
+    w = rand((n, k), torch.bfloat16, device, 0.05, seed=2)
+    bias = rand((n,), torch.float32, device, 0.5, seed=3) if k >= 192 else None        # (a bias lands within three k-tiles)
+    res = rand((m, n), torch.float32, device, 1.0, seed=4)
+    shuffled = ops.shuffle_weight(w)
+    want = x.double() @ w.double().T
+    near = (k + 4) * 2.0 ** -24 * (x.double().abs() @ w.double().abs().T + 4.0)
+    out, first = (torch.full((m + 2, n), float("nan"), device=device) for _ in range(2))
+    ops.linear(x, shuffled, out[:m], force=force)
+    ops.linear(x, shuffled, first[:m], force=ops.GEMM_TILED)
+    assert torch.equal(out[:m], first[:m]) and bool(out[m:].isnan().all())
+    if bias is not None:
+        want = want + bias
+    space = torch.empty(8 * m * n + 4, dtype=torch.float32, device=device) if m * n < 1 << 20 else None
+    for work in (None, space):
+        half = torch.full((m + 2, n), float("nan"), dtype=torch.bfloat16, device=device)
+        ops.linear(x, shuffled, half[:m], bias=bias, workspace=work, force=force)
+        assert bool(((half[:m].double() - want).abs() <= near + 2.0 ** -8 * want.abs()).all()) and bool(half[m:].isnan().all())
+        acc = res.clone()
+        ops.linear(x, shuffled, acc, bias=bias, residual=acc, workspace=work, force=force)
+        assert bool(((acc.double() - want - res).abs() <= near + 2.0 ** -22 * (want.abs() + 5.0)).all())
+    if n % 32 == 0:
+        gated = torch.full((m + 1, n // 2), float("nan"), dtype=torch.bfloat16, device=device)
+        ops.linear_glu(x, shuffled, gated[:m], bias=bias, force=force)
+        (g, u), (g_near, u_near) = want.view(m, n // 32, 2, 16).unbind(2), near.view(m, n // 32, 2, 16).unbind(2)
+        value = torch.nn.functional.silu(g) * u
+        bound = 1.1 * g_near * (u.abs() + u_near) + g.abs() * u_near + 2.0 ** -20 * (g * u).abs() + 2.0 ** -8 * value.abs()
+        assert bool(((gated[:m].double().view(m, n // 32, 16) - value).abs() <= bound).all()) and bool(gated[m:].isnan().all())
+    else:
+        with pytest.raises(Exception):
+            ops.linear(x, w, torch.empty(m, n, device=device), force=force)            # (row-major weights have no such tiles)
+
+
 @pytest.mark.parametrize("m,n,k", [(300, 520, 448), (1100, 2056, 1024), (2049, 264, 3584)])
 def test_linear_of_waves_in_turns_rounds_as_the_other_tiles(ops, device, m, n, k):
     """One sum over the whole of K is the same bits in every tile: 16x16x32 MFMAs by waves in turns (a result of 16-byte rows), 32x32x16
