@@ -21,6 +21,8 @@
 // C[M, N/2][.., 16j + i] = silu(gate_j[i]) * up_j[i] in their epilogues, in float32 from the
 // accumulators, so the [M, N] intermediate never reaches memory.
 #include <type_traits>
+#include <math.h>
+
 #include "tw_common.h"
 #include "gemm_shared.h"
 
@@ -859,6 +861,33 @@ static int launch_skinny_lds_m(const T* A, long lda, const T* W, long ldw, const
 // (8 rows: bf16 2304 x 2560, 180 workgroups of 16 k-steps, 8.3 / 9.0, x 2816, of 17.6, 9.3 / 9.1; 2560 x 3328, 240, 10.1 / 9.8, x 3584, 280, 10.5 / 9.9;
 // 2816 x 3328 11.4 / 10.0. float32 2560 x 1536, 240 workgroups, 9.6 / 9.8, x 1792, 280, 11.5 / 10.4, x 2304, 144 k-steps, 12.3 / 12.9; 3072 x 2816, 17.6 k-steps
 // a range, 15.1 / 13.7, x 3328, 208, 15.4 / 16.3.)
+//
+// An eighth and more beyond those lines both are estimated, and this kernel taken where it is expected to be 10 % (float32: 7) faster. What a workgroup reads goes at
+// a CU's own rate (its weights, and the activations in whole batches of four k-steps a wave), rounds of workgroups one after the
+// other, all together no faster than memory; the other kernel's time is that of its k-steps, of memory and of the reduction. Fitted to
+// 3,952 products of 1 to 16 rows (256 to 32,000 x 256 to 11,008, both types, plain with a residual and gated; 3 to 7 % off): plain ones
+// come out 3 % faster in the mean than by the lines alone, gated ones 9 % in bfloat16 and 17 in float32, one of them 2 % slower, and are 1
+// and 0.4 % behind the better of the two. (us, K ranges or two waves a column / whole K, at 1 and 8 rows: bf16 9216 x 2048 11.3 / 8.2, 11.6 /
+// 8.9, 12288 x 2048 13.0 / 9.9, 13.4 / 9.9; 2048 x 5632 with a residual 9.4 / 7.1, 9.7 / 9.0; float32 8192 x 2048 18.8 / 13.9, 19.4 / 14.3, 10304 x
+// 2048 21.3 / 18.0, 22.2 / 19.2, 2048 x 4096 13.2 / 11.2, 13.2 / 12.3.)
+static double narrow_us(int M, int N, int K, int epf, bool glu) {
+  const int size = 16 / epf, steps = tw_div_up(K / epf, 4), groups = glu ? N / 32 : tw_div_up(N, 16);
+  const int waves = steps <= 48 ? 4 : steps <= 96 ? 8 : 16;            // (see launch_narrow)
+  const double covered = (double)tw_div_up(tw_div_up(steps, waves), 4) * 4 * waves * 64;      // bytes of a row
+  const double cu = 1e-3 * (size == 2 ? (glu ? 0.0187 : 0.0195) : 0.0254) * ((glu ? 32 : 16) + (size == 2 ? 1.33 : glu ? 0.73 : 0.87) * M) * covered * tw_div_up(groups, 256);
+  const double memory = 1e-6 * N * (double)K * size / (size == 2 ? 6.57 : 6.14);
+  return (size == 2 ? (glu ? 2.66 : 2.80) : glu ? 2.81 : 2.97) + sqrt(sqrt(cu * cu * cu * cu + memory * memory * memory * memory));
+}
+static double skinny_us(int M, int N, int K, int epf, bool glu) {
+  const int size = 16 / epf, steps = tw_div_up(K / epf, 4), splits = glu ? 1 : skinny_lds_splits(N, K, epf);
+  const double fill = tw_div_up(N, 64) * splits / 512.0;
+  const double step = size == 2 ? (glu ? 0.0918 + 0.0005 * M : 0.0715 + 0.0014 * M) : glu ? 0.1101 + 0.0002 * M : 0.0589 + 0.0017 * M;
+  const double cu = tw_div_up(steps, splits) * step * (fill > 1 ? fill : 1.0);
+  const double memory = 1e-6 * N * (double)K * size / (size == 2 ? 6.57 : 6.4);
+  return (size == 2 ? (glu ? 2.99 : 3.62) : glu ? 3.29 : 4.31) + (splits > 1 ? (size == 2 ? 1.95 + 0.74e-6 * 4 * splits * M * N : 2.22 + 0.67e-6 * 4 * splits * M * N) : 0.0) +
+         sqrt(sqrt(cu * cu * cu * cu + memory * memory * memory * memory));
+}
+
 static bool narrow_pays(int M, int N, int K, int epf, bool glu, bool sums) {
   const int steps = tw_div_up(K / epf, 4), groups = glu ? N / 32 : tw_div_up(N, 16);
   if (sums) {
@@ -871,9 +900,11 @@ static bool narrow_pays(int M, int N, int K, int epf, bool glu, bool sums) {
     if (groups < 160) return false;
     return steps <= 128 ? second : steps <= 192 ? groups >= 224 || steps > 16 * ranges : steps <= 224 && (groups >= 240 || steps > 24 * ranges);
   }
-  if (groups <= 256) return steps <= (M > 8 && groups < 96 && !glu ? 96 : 128);
-  if (glu) return steps >= 28 && steps <= (groups < 512 && epf == 4 ? 32 : 64) && (M <= 8 || groups >= 512);
-  return groups <= 512 && steps >= 16 && steps <= 64;
+  if (groups <= 256 ? steps <= (M > 8 && groups < 96 && !glu ? 96 : 128)
+      : glu ? steps >= 28 && steps <= (groups < 512 && epf == 4 ? 32 : 64) && (M <= 8 || groups >= 512)
+            : groups <= 512 && steps >= 16 && steps <= 64) return true;
+  const bool beyond = groups >= 576 || steps > (groups <= 256 ? 144 : 72);      // (by an eighth: what lies at the lines stays where it is)
+  return beyond && steps >= 28 && narrow_us(M, N, K, epf, glu) < (epf == 4 ? 0.93 : 0.9) * skinny_us(M, N, K, epf, glu);
 }
 
 // A plain product with an activation behind it, against the K ranges' sums and a kernel that adds them up and applies it (bf16, in a

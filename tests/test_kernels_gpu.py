@@ -784,6 +784,25 @@ def test_linear_glu_of_few_rows_chooses_by_rows_and_type(ops, device, dtype, m, 
     assert torch.equal(got[ops.GEMM_AUTO], got[ops.GEMM_NARROW if narrow else ops.GEMM_SKINNY])
 
 
+@pytest.mark.parametrize("dtype,glu,m,n,k,narrow", [
+    (torch.bfloat16, False, 1, 2048, 5632, True), (torch.bfloat16, False, 16, 2048, 5632, False), (torch.bfloat16, False, 4, 9216, 2048, True),
+    (torch.bfloat16, False, 1, 9216, 512, False), (torch.bfloat16, False, 8, 16384, 5632, False), (torch.float32, False, 4, 10304, 2048, True),
+    (torch.float32, False, 16, 10304, 2048, False), (torch.float32, False, 1, 2048, 4096, True), (torch.float32, False, 8, 896, 4864, False),
+    (torch.bfloat16, True, 1, 4096, 8192, True), (torch.bfloat16, True, 16, 9216, 8192, False), (torch.float32, True, 8, 1024, 2560, True)])
+def test_linear_of_few_rows_chooses_by_estimate(ops, device, dtype, glu, m, n, k, narrow):
+    """Both sides of the estimated times, where the measured ones lie a tenth and more apart: the bits tell which kernel ran."""
+    x, w = rand((m, k), dtype, device, 1.0, seed=1), ops.shuffle_weight(rand((n, k), dtype, device, 0.05, seed=2))
+    workspace = torch.empty(max(4, ops.linear_workspace_bytes(dtype, 64, n, k) // 4), device=device)
+    got = {}
+    for force in (ops.GEMM_AUTO, ops.GEMM_SKINNY, ops.GEMM_NARROW):
+        if glu:
+            got[force] = ops.linear_glu(x, w, torch.empty(m, n // 2, dtype=dtype, device=device), force=force)
+        else:
+            got[force] = ops.linear(x, w, torch.empty(m, n, device=device), workspace=workspace, force=force)
+    assert not torch.equal(got[ops.GEMM_SKINNY], got[ops.GEMM_NARROW])
+    assert torch.equal(got[ops.GEMM_AUTO], got[ops.GEMM_NARROW if narrow else ops.GEMM_SKINNY])
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("m,n,k", [(300, 256, 4096), (1024, 512, 8192), (2048, 896, 9472), (520, 130, 2056),
                                    (2048, 4096, 512)])
