@@ -122,7 +122,7 @@ static inline int launch_splitk_reduce(const float* partial, int splits, const f
 }
 
 // The tiled kernels (gemm_tiled.hip). shape: 0 = choose, 1 = tiles of 128x128, 2 = 128x256,
-// 3 = 256x256 (bfloat16 with shuffled weights only). Returns 0 or an error code.
+// 3 = 256x256 (bfloat16 with shuffled weights only; float32's second is 64x128). Returns 0 or an error code.
 int tw_tiled_linear(int dtype, int out_f32, int shuffled, int glu, int shape, const void* A, long lda,
                     const void* W, long ldw, const float* bias, const float* residual, long ldr, void* C,
                     long ldc, float* partial, long partial_bytes, int M, int N, int K, hipStream_t stream);

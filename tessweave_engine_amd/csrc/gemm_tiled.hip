@@ -2,6 +2,7 @@
 // weight layouts and the GLU form; this file holds the kernel, its epilogue and its launcher.
 #include "gemm_shared.h"
 #include <math.h>
+#include <algorithm>
 
 // f(integral_constant<int, 0>), ..., f(integral_constant<int, N - 1>): a loop whose index is a constant
 // expression in the body (the scheduler's group barriers take constants only)
@@ -261,8 +262,8 @@ __device__ __forceinline__ void tw_tiled_epilogue(f32x16 (&acc)[WM][WN], char* l
 
 // =====================================================================================
 // Tiled kernel. Workgroup = 4 waves in a 2x2 grid, wave tile (32*WM) x (32*WN): tiles of 128x128
-// (two workgroups per CU), 128x256 and 256x256 (one per CU, the accumulators in AGPRs).
-// One stage holds 128 bytes of K per row (64 bf16 / 32 f32), rows padded to 144
+// (two workgroups per CU), 128x256 and 256x256 (one per CU, the accumulators in AGPRs). bfloat16; float32: gemm_parts_kernel below.
+// One stage holds 128 bytes of K per row (64 elements), rows padded to 144
 // bytes in LDS so that 16-byte fragment reads of 8 consecutive lanes hit
 // distinct banks. Two stages: the next stage's global loads are in flight
 // while the current one is multiplied.
@@ -483,6 +484,246 @@ __global__ __launch_bounds__(256) void gemm_tiled_kernel(const T* __restrict__ A
     return;
   }
   tw_tiled_epilogue<OutT, WM, WN, GLU>(acc, lds, bias, residual, ldr, C, ldc, M, N, m0, n0, wm0, wn0, wave, lane);
+}
+
+// =====================================================================================
+// float32: every operand as the sum of three bfloat16 numbers, on the bfloat16 matrix unit.
+//
+// x = h + m + l: h holds the first 8 bits of x's mantissa (x with its low 16 bits cleared), m the next 8, l the last 8. The three are
+// exact (x - h and x - h - m are representable, nothing is rounded), and a product of two of them is exact in the matrix unit, which
+// adds in float32. Of the nine products m l, l m and l l are below 2^-22 of the whole one and left out; the other six are added with the
+// smallest first. What is left out is smaller than what rounding the sum costs, and the sum is rounded less often than by the float32
+// MFMA, which adds two products at a time.
+//
+// Why: the float32 MFMA takes 64 cycles for 32x32x2, the bfloat16 one 32 for 32x32x16, so six of these are 2.7 times as fast. Workgroup =
+// 4 waves in a 2x2 grid, wave tile (32*WM) x (32*WN): 128x128, 64x128 and 64x64. A k-tile is 32 elements of K; it is split once, on its way
+// from registers to LDS (5.5 vector instructions an element), while the next one is on its way from memory, and two to five workgroups
+// share a CU, so that one splits while another multiplies. A row of a part is 64 bytes of LDS, four pieces of 16, piece p at
+// p ^ (row / 4 % 4): the 16 rows that a pass of a fragment read takes, and the 8 lanes of a write, are in different banks. The products
+// with a part m or l have sums of their own, which costs 1 to 3 % and keeps their roundings away from the large sums.
+//
+// Against the float32 MFMA (128x128 tiles, two LDS stages, the K ranges of tiled_splits): 478 x 10,432 x 2,048 271 -> 147 us, 478 x 2,048 x
+// 4,096 108 -> 64, 4,096 x 32,000 x 2,048 4,303 -> 2,938 (183 TFLOP/s, so 1.1 PFLOP/s in bfloat16, where power is the bound), 65 x 896 x 4,864
+// 47 -> 21; 109 random products (65 to 3,000 rows) take 0.49 of the time, the slowest 0.86. Their error against 64 bits is 0.41 of what it
+// was in the mean and 0.81 at the most (short K, with a residual).
+//
+// A value that is not finite has no such parts (inf - inf), and every result that it enters is then not finite either. So a tile with such
+// a result is formed again by the float32 MFMA from the operands themselves, and infinities, NaN and sums that overflow are what they are there.
+// (Parts below 2^-126 may be lost: of values below 2^-110.)
+// =====================================================================================
+#define TW_PART_ROW 64
+
+__device__ __forceinline__ void tw_three_parts(f32x4 lo, f32x4 hi, bf16x8& h, bf16x8& m, bf16x8& l) {
+  u32x4 ph, pm, pl;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const float x0 = e < 2 ? lo[2 * e] : hi[2 * e - 4], x1 = e < 2 ? lo[2 * e + 1] : hi[2 * e - 3];
+    const unsigned a0 = __float_as_uint(x0), a1 = __float_as_uint(x1);
+    const float y0 = x0 - __uint_as_float(a0 & 0xffff0000u), y1 = x1 - __uint_as_float(a1 & 0xffff0000u);
+    const unsigned b0 = __float_as_uint(y0), b1 = __float_as_uint(y1);
+    const float z0 = y0 - __uint_as_float(b0 & 0xffff0000u), z1 = y1 - __uint_as_float(b1 & 0xffff0000u);
+    ph[e] = __builtin_amdgcn_perm(a1, a0, 0x07060302);        // the upper halves side by side
+    pm[e] = __builtin_amdgcn_perm(b1, b0, 0x07060302);
+    pl[e] = __builtin_amdgcn_perm(__float_as_uint(z1), __float_as_uint(z0), 0x07060302);
+  }
+  h = __builtin_bit_cast(bf16x8, ph);
+  m = __builtin_bit_cast(bf16x8, pm);
+  l = __builtin_bit_cast(bf16x8, pl);
+}
+
+template <int WM, int WN, bool SHUF, bool GLU>
+__global__ __launch_bounds__(256, WN <= 2 ? 2 : 1) void gemm_parts_kernel(const float* __restrict__ A, long lda, const float* __restrict__ W, long ldw,
+                                                            const float* __restrict__ bias, const float* residual, long ldr, float* C,
+                                                            long ldc, int M, int N, int K, int tiles_m, int n_blocks, int splits,
+                                                            float* __restrict__ partial) {
+  constexpr int BM = 64 * WM, BN = 64 * WN, BK = 32;
+  constexpr int A_PIECES = BM * 4 / 256, W_PIECES = BN * 4 / 256;       // of 8 elements of K, a thread's
+  constexpr int PART = (BM + BN) * TW_PART_ROW;
+  extern __shared__ __attribute__((aligned(16))) char lds[];
+
+  // (workgroups, K ranges and bands as in gemm_tiled_kernel)
+  const int per_xcd = gridDim.x / 8;
+  const int logical = (blockIdx.x % 8) * per_xcd + blockIdx.x / 8;
+  if (logical >= n_blocks) return;
+  const int n_tiles = n_blocks / splits;
+  const int split = logical / n_tiles, tile = logical % n_tiles;
+  constexpr int BAND = 2048 / BM;
+  const int tiles_n = n_tiles / tiles_m;
+  const int band = tile / (BAND * tiles_n), in_band = tile - band * BAND * tiles_n;
+  const int band_rows = min(BAND, tiles_m - band * BAND);
+  const int tile_m = band * BAND + in_band % band_rows, tile_n = in_band / band_rows;
+  const int m0 = tile_m * BM, n0 = tile_n * BN;
+
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int wm0 = (wave >> 1) * 32 * WM, wn0 = (wave & 1) * 32 * WN;
+  const int r = lane & 31, g = lane >> 5;
+
+  f32x16 acc[WM][WN], small[WM][WN];                           // the sums of h h, and of the other products
+#pragma unroll
+  for (int i = 0; i < WM; ++i)
+#pragma unroll
+    for (int j = 0; j < WN; ++j)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) acc[i][j][e] = small[i][j][e] = 0.f;
+
+  // A thread's pieces: a base that is the same for every lane and offsets fixed for the whole of K. Rows past the end are clamped to
+  // the last one (what they produce is never stored).
+  const float* a_tile = A + (size_t)m0 * lda;
+  const float* w_tile = SHUF ? W + (size_t)(n0 / 16) * ldw * 256 : W + (size_t)n0 * ldw;
+  const int n_blocks_w = (N + 15) / 16;
+  unsigned a_off[A_PIECES], w_off[W_PIECES];
+  int a_st[A_PIECES], w_st[W_PIECES], w_k[W_PIECES];          // the piece's place in LDS; its first k (chunks of 4 that begin past K are zeros)
+  auto place = [](int row, int p) { return row * TW_PART_ROW + ((p ^ (row >> 2)) & 3) * 16; };
+#pragma unroll
+  for (int i = 0; i < A_PIECES; ++i) {
+    const int c = tid + i * 256, row = c >> 2, p = c & 3;
+    a_off[i] = (unsigned)(min(m0 + row, M - 1) - m0) * (unsigned)lda + p * 8;
+    a_st[i] = place(row, p);
+  }
+#pragma unroll
+  for (int i = 0; i < W_PIECES; ++i) {
+    const int c = tid + i * 256;
+    if (SHUF) {                                                // 16 rows of a block, then the pieces of its two k-steps
+      const int row = (c >> 6) * 16 + (c & 15), p = (c >> 4) & 3;
+      const int gblk = min(n0 / 16 + (c >> 6), n_blocks_w - 1);
+      w_off[i] = (unsigned)(gblk - n0 / 16) * (unsigned)ldw * 256 + (p >> 1) * 256 + (p & 1) * 128 + (c & 15) * 4;
+      w_st[i] = BM * TW_PART_ROW + place(row, p);
+      w_k[i] = p * 8;
+    } else {
+      const int row = c >> 2, p = c & 3;
+      w_off[i] = (unsigned)(min(n0 + row, N - 1) - n0) * (unsigned)ldw + p * 8;
+      w_st[i] = BM * TW_PART_ROW + place(row, p);
+      w_k[i] = p * 8;
+    }
+  }
+  const int a_k = (tid & 3) * 8;
+  constexpr int W_NEXT = SHUF ? 64 : 4;                        // floats to the piece's second chunk
+
+  f32x4 a_reg[A_PIECES][2], w_reg[W_PIECES][2];
+  const int k_tiles_all = (K + BK - 1) / BK;
+  const int per_split = (k_tiles_all + splits - 1) / splits;
+  const int kt0 = split * per_split;
+  const int k_end = min(k_tiles_all, kt0 + per_split);
+  const int whole_tiles = K / BK;
+
+  auto load = [&](int kt) {
+    const float* ab = a_tile + (size_t)kt * BK;
+    const float* wb = SHUF ? w_tile + (size_t)kt * 512 : w_tile + (size_t)kt * BK;
+    if (kt < whole_tiles) {
+#pragma unroll
+      for (int i = 0; i < A_PIECES; ++i) {
+        a_reg[i][0] = tw_load_frag(ab + a_off[i]);
+        a_reg[i][1] = tw_load_frag(ab + a_off[i] + 4);
+      }
+#pragma unroll
+      for (int i = 0; i < W_PIECES; ++i) {
+        w_reg[i][0] = tw_load_frag(wb + w_off[i]);
+        w_reg[i][1] = tw_load_frag(wb + w_off[i] + W_NEXT);
+      }
+    } else {                                                   // (the shuffled layout ends at a k-step: its chunks past K are zeros)
+      const int left = K - kt * BK, w_left = SHUF ? (left + 15) / 16 * 16 : left;
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+#pragma unroll
+        for (int i = 0; i < A_PIECES; ++i)
+          a_reg[i][h] = a_k + 4 * h < left ? tw_load_frag(ab + a_off[i] + 4 * h) : Elem<float>::zero();
+#pragma unroll
+        for (int i = 0; i < W_PIECES; ++i)
+          w_reg[i][h] = w_k[i] + 4 * h < w_left ? tw_load_frag(wb + w_off[i] + W_NEXT * h) : Elem<float>::zero();
+      }
+    }
+  };
+  auto split_store = [&]() {
+    auto put = [&](int at, const f32x4 (&x)[2]) {
+      bf16x8 h, m, l;
+      tw_three_parts(x[0], x[1], h, m, l);
+      *reinterpret_cast<bf16x8*>(lds + at) = h;
+      *reinterpret_cast<bf16x8*>(lds + PART + at) = m;
+      *reinterpret_cast<bf16x8*>(lds + 2 * PART + at) = l;
+    };
+#pragma unroll
+    for (int i = 0; i < A_PIECES; ++i) put(a_st[i], a_reg[i]);
+#pragma unroll
+    for (int i = 0; i < W_PIECES; ++i) put(w_st[i], w_reg[i]);
+  };
+  const int swz = (r >> 2) & 3;                                // (every fragment's rows begin at a multiple of 16)
+  auto multiply = [&]() {
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+      const int at = ((2 * s + g) ^ swz) * 16;
+      bf16x8 af[3][WM], wf[3][WN];
+#pragma unroll
+      for (int p = 2; p >= 0; --p) {
+#pragma unroll
+        for (int i = 0; i < WM; ++i) af[p][i] = *reinterpret_cast<const bf16x8*>(lds + p * PART + (wm0 + i * 32 + r) * TW_PART_ROW + at);
+#pragma unroll
+        for (int j = 0; j < WN; ++j) wf[p][j] = *reinterpret_cast<const bf16x8*>(lds + p * PART + (BM + wn0 + j * 32 + r) * TW_PART_ROW + at);
+      }
+      auto product = [&](f32x16 (&sum)[WM][WN], int p, int q) {
+#pragma unroll
+        for (int i = 0; i < WM; ++i)
+#pragma unroll
+          for (int j = 0; j < WN; ++j) tw_mma32(sum[i][j], af[p][i], wf[q][j]);
+      };
+      product(small, 2, 0);
+      product(small, 0, 2);
+      product(small, 1, 1);
+      product(small, 1, 0);
+      product(small, 0, 1);
+      product(acc, 0, 0);
+    }
+  };
+
+  if (kt0 < k_end) load(kt0);
+  for (int kt = kt0; kt < k_end; ++kt) {
+    __syncthreads();                                           // (the reads of the k-tile before)
+    split_store();
+    if (kt + 1 < k_end) load(kt + 1);
+    __syncthreads();
+    multiply();
+  }
+
+  float odd = 0.f;                                             // NaN as soon as one of them is not finite
+#pragma unroll
+  for (int i = 0; i < WM; ++i)
+#pragma unroll
+    for (int j = 0; j < WN; ++j)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) {
+        acc[i][j][e] += small[i][j][e];
+        odd = __fmaf_rn(acc[i][j][e], 0.f, odd);
+      }
+  if (__syncthreads_or(odd != odd)) {
+#pragma unroll
+    for (int i = 0; i < WM; ++i)
+#pragma unroll
+      for (int j = 0; j < WN; ++j)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
+    const int k_from = kt0 * BK, k_to = min(K, k_end * BK);
+    for (int k = k_from; k < k_to; k += 8) {
+      f32x4 af[WM], wf[WN];
+      const int mine = k + 4 * g;
+#pragma unroll
+      for (int i = 0; i < WM; ++i) af[i] = mine < K ? tw_load_frag(A + (size_t)min(m0 + wm0 + i * 32 + r, M - 1) * lda + mine) : Elem<float>::zero();
+#pragma unroll
+      for (int j = 0; j < WN; ++j) {
+        const int n = min(n0 + wn0 + j * 32 + r, N - 1);
+        const float* w = SHUF ? W + ((size_t)(n >> 4) * ldw + (mine >> 4)) * 256 + ((mine >> 2) & 3) * 64 + (n & 15) * 4 : W + (size_t)n * ldw + mine;
+        wf[j] = mine < K ? tw_load_frag(w) : Elem<float>::zero();
+      }
+#pragma unroll
+      for (int i = 0; i < WM; ++i)
+#pragma unroll
+        for (int j = 0; j < WN; ++j) tw_mma32(acc[i][j], af[i], wf[j]);
+    }
+  }
+
+  if (splits > 1)
+    tw_tiled_epilogue<float, WM, WN, false>(acc, lds, nullptr, nullptr, 0, partial + (size_t)split * M * N, (long)N, M, N, m0, n0, wm0, wn0,
+                                            wave, lane);
+  else
+    tw_tiled_epilogue<float, WM, WN, GLU>(acc, lds, bias, residual, ldr, C, ldc, M, N, m0, n0, wm0, wn0, wave, lane);
 }
 
 // =====================================================================================
@@ -1170,10 +1411,13 @@ static int launch_tiled(const T* A, long lda, const T* W, long ldw, const float*
   TW_REQUIRE((long)BM * lda < (1L << 31));
   TW_REQUIRE(SHUF ? (long)(BN / 16) * ldw * 64 * EPF < (1L << 31) : (long)BN * ldw < (1L << 31));
   const int grid = (int)((n_blocks + 7) / 8 * 8);
-  const size_t pipeline_bytes = 2 * (size_t)(BM + BN) * (KCH * 16 + 16);
+  const size_t pipeline_bytes = sizeof(T) == 4 ? 3 * (size_t)(BM + BN) * TW_PART_ROW : 2 * (size_t)(BM + BN) * (KCH * 16 + 16);
   const size_t epilogue_bytes = 4 * (32 * (size_t)(32 * WN + 4) + 32 * WN) * 4;
   const size_t lds_bytes = pipeline_bytes > epilogue_bytes ? pipeline_bytes : epilogue_bytes;
-  auto kernel = gemm_tiled_kernel<T, OutT, WM, WN, SHUF, GLU>;
+  auto kernel = [] {
+    if constexpr (sizeof(T) == 4) return gemm_parts_kernel<WM, WN, SHUF, GLU>;
+    else return gemm_tiled_kernel<T, OutT, WM, WN, SHUF, GLU>;
+  }();
   static bool attribute_set = false;   // per instantiation
   if (!attribute_set) {
     hipError_t e = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
@@ -1418,11 +1662,53 @@ static bool turns_pay(bool glu, bool adds, int M, int N, int K) {
   return tiles > 256 || K > (glu ? 64 : 128);
 }
 
+// float32 (gemm_parts_kernel): 1 is 128x128, 2 64x128, 3 64x64, with K ranges, the least estimated time in microseconds. A launch, rounds of
+// the workgroups that a CU holds, and k-tiles of 32, which take `alone` a round where a CU has little else and n x `full` where its n
+// workgroups share the matrix unit; the fourth powers of the two add up. Fitted to 1,586 forms of 142 products (65 to 3,000 rows, 512 to
+// 32,000 columns, K 256 to 4,864, 1 to 8 ranges): 5 to 6 % off, the choice 0.4 % behind the fastest of all, 4 of 142 more than 5 %.
+static const struct { int m, n, held; double launch, tile, alone, full, sums; } kParts[4] = {
+    {}, {128, 128, 2, 3.1, 1.73, 1.429, 1.170, 0.32}, {64, 128, 3, 4.2, 0.0, 0.966, 0.723, 0.30}, {64, 64, 5, 3.1, 0.0, 0.686, 0.426, 0.34}};
+static TilePlan choose_parts(bool glu, int M, int N, int K) {
+  static const int kRanges[6] = {1, 2, 3, 4, 6, 8};
+  TilePlan plan = {1, 1, 0};
+  double best = 0;
+  for (int shape = 1; shape <= 3; ++shape) {
+    const auto& c = kParts[shape];
+    const long tiles = (long)tw_div_up(M, c.m) * tw_div_up(N, c.n);
+    for (int splits : kRanges) {
+      if (splits > 1 && (glu || tiles >= 512 || tiles * splits > 1536 || K / splits < 128)) break;
+      const long blocks = tiles * splits, n = (blocks + 255) / 256, rounds = (n + c.held - 1) / c.held;
+      const double alone = rounds * c.alone, full = (n <= 2 * c.held ? n : blocks / 256.0 + 0.5) * c.full;
+      double t = c.launch + rounds * c.tile + tw_div_up(tw_div_up(K, 32), splits) * sqrt(sqrt(alone * alone * alone * alone + full * full * full * full));
+      if (splits > 1) t += 3.0 + c.sums * 4e-6 * splits * M * N;
+      if (best == 0 || t < best) {
+        best = t;
+        plan = {shape, splits, 0};
+      }
+    }
+  }
+  return plan;
+}
+
 template <typename T, typename OutT, bool SHUF, bool GLU>
-static int tiled_by_shape(int shape, const T* A, long lda, const T* W, long ldw, const float* bias,
+static std::enable_if_t<sizeof(T) == 4, int> tiled_by_shape(int shape, const T* A, long lda, const T* W, long ldw, const float* bias,
                           const float* residual, long ldr, OutT* C, long ldc, float* partial,
                           long partial_bytes, int M, int N, int K, hipStream_t stream, TiledMode* mode = nullptr) {
-  constexpr bool BIG = sizeof(T) == 2 && SHUF;
+  if (shape >= 3) return TW_ERR_BAD_ARGUMENT;      // (forced shapes 1 and 2: float32's first and second)
+  const TilePlan plan = shape ? TilePlan{shape, 0, 0} : choose_parts(GLU, M, N, K);
+  auto run = [&](auto wm, auto wn) {
+    return launch_tiled<T, OutT, wm.value, wn.value, SHUF, GLU>(A, lda, W, ldw, bias, residual, ldr, C, ldc, partial, partial_bytes, M, N, K, plan.splits, stream, mode);
+  };
+  constexpr std::integral_constant<int, 1> one;
+  constexpr std::integral_constant<int, 2> two;
+  return plan.shape == 1 ? run(two, two) : plan.shape == 2 ? run(one, two) : run(one, one);
+}
+
+template <typename T, typename OutT, bool SHUF, bool GLU>
+static std::enable_if_t<sizeof(T) == 2, int> tiled_by_shape(int shape, const T* A, long lda, const T* W, long ldw, const float* bias,
+                          const float* residual, long ldr, OutT* C, long ldc, float* partial,
+                          long partial_bytes, int M, int N, int K, hipStream_t stream, TiledMode* mode = nullptr) {
+  constexpr bool BIG = SHUF;
   auto takes = [&](auto tile) { return turns_takes<decltype(tile)>(sizeof(OutT), A, lda, ldw, bias, residual, ldr, C, ldc, N, K); };
   TilePlan plan = {shape, 0, 0};                    // a forced shape keeps the launcher's own rule
   bool turns = BIG;                                 // (each plan is for its own kernels: choose_turns for a product all of whose tiles they take)
@@ -1527,8 +1813,9 @@ int tw_tiled_partials(int dtype, int shuffled, const void* A, long lda, const vo
 
 long tw_tiled_workspace_bytes(int dtype, int rows, int N, int K) {
   const int epf = dtype == TW_DTYPE_F32 ? 4 : 8;
-  // enough for whichever kernel runs: the 128x128 tiles' own rule, or either plan for shuffled bfloat16 weights
+  // enough for whichever kernel runs: the 128x128 tiles' own rule, float32's plan, or either plan for shuffled bfloat16 weights
   int most = tiled_splits(rows, N, K, epf, 128, 128);
+  if (dtype == TW_DTYPE_F32) most = std::max(most, choose_parts(false, rows, N, K).splits);
   auto ask = [&](const TilePlan& plan) {
     const int s = plan.splits > 0 ? plan.splits : tiled_splits(rows, N, K, epf, kTileM[plan.shape], kTileN[plan.shape]);
     if (s > most) most = s;

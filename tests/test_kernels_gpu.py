@@ -631,6 +631,44 @@ def test_linear_sums_in_pieces_of_k(ops, device, m, n, k, ranges):
     assert off <= 1.03 * parts_off, off / parts_off
 
 
+@pytest.mark.parametrize("m,n,k", [(65, 33, 4), (66, 130, 36), (129, 300, 76), (200, 1024, 512), (478, 2080, 1040), (640, 4096, 96)])
+def test_float32_linear_in_three_parts(ops, device, m, n, k):
+    """float32 products of many rows are six bfloat16 ones: all tiles, rows, columns and K that end inside one, K ranges, magnitudes
+    2^24 apart, all of one sign. The sum of the leading parts is rounded no more than twice in 16 elements of K, the others' sum is
+    2^-7 of it and less, and the three products left out and the last additions come to less than 4 x 2^-24 of the sum of sizes."""
+    x = rand((m, k), torch.float32, device, 1.0, seed=1) * torch.exp2(rand((k,), torch.float32, device, 6.0, seed=3).round().clamp(-12, 12))
+    for x, w in ((x, rand((n, k), torch.float32, device, 0.05, seed=2)), (x.abs(), rand((n, k), torch.float32, device, 0.05, seed=2).abs())):
+        want, near = x.double() @ w.double().T, (k / 8 + 4) * 2.0 ** -24 * (x.double().abs() @ w.double().abs().T)
+        space = torch.empty(ops.linear_workspace_bytes(torch.float32, m, n, k) // 4 + 4, device=device)
+        for weight in (w, ops.shuffle_weight(w)):
+            for force in (ops.GEMM_AUTO, ops.GEMM_TILED, ops.GEMM_TILED_WIDE):
+                out = torch.full((m, n), float("nan"), device=device)
+                ops.linear(x, weight, out, workspace=space, force=force)
+                assert bool(((out.double() - want).abs() <= near).all())
+
+
+@pytest.mark.parametrize("shuffled", [False, True])
+def test_float32_linear_of_values_without_parts(ops, device, shuffled):
+    """Infinities, NaN (also one whose upper half is an infinity's) and sums that overflow come out as they do of float32 products,
+    and what is beside them in their tiles is off by no more than a float32 sum of K products is."""
+    m, n, k = 130, 260, 72
+    x, w = rand((m, k), torch.float32, device, 1.0, seed=1), rand((n, k), torch.float32, device, 0.05, seed=2)
+    x[3, 5] = float("inf")
+    x[70, 71] = float("-inf")
+    x.view(torch.int32)[129, 40] = 0x7F800001
+    x[9, 0] = 3.4e38
+    w[8, 0] = 100.0
+    w[200, 33] = float("inf")
+    out = torch.zeros(m, n, device=device)
+    ops.linear(x, ops.shuffle_weight(w) if shuffled else w, out)
+    want = x.double() @ w.double().T
+    rounded = want.float()
+    assert bool((out.isnan() == rounded.isnan()).all()) and bool((out[rounded.isinf()] == rounded[rounded.isinf()]).all())
+    sound = rounded.isfinite()
+    near = (k + 4) * 2.0 ** -24 * (x.double().abs() @ w.double().abs().T)
+    assert bool(((out.double() - want).abs() <= near)[sound].all())
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("m,n,k", [(1, 16, 8), (16, 15, 40), (3, 33, 1536), (8, 389, 1576), (16, 256, 3104), (5, 96, 4096), (16, 64, 8200)])
 def test_linear_of_few_rows_over_whole_k(ops, device, dtype, m, n, k):
