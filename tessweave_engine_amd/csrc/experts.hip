@@ -563,6 +563,147 @@ __global__ __launch_bounds__(WAVES * 64) void moe_grouped_kernel(const T* __rest
     }
 }
 
+// float32, steps of many rows: the same products from three bfloat16 parts an operand (gemm_parts_kernel says why and how exact). One
+// workgroup: a unit's 64 rows against 64 * WN rows of its expert's matrices (GLU: half of gate, half of up, of the same columns), waves in
+// a 2x2 grid, wave tile 32 x (32 * WN). A k-tile is two k-steps; rows and matrices are read in fragment order, split and laid into LDS, two
+// k-tiles are on their way (the matrices come from HBM) and three workgroups share a CU. What is not finite is formed again from the
+// operands themselves. All launches of the experts, us, the float32 MFMA / this: 16 experts of 2,048 x 1,408, two a token, gated, 128 tokens
+// 303 / 163, 478 349 / 221, 2,000 954 / 594; 8 of 4,096 x 2,048, 300 tokens 714 / 413; 64 of 1,024 x 512, four a token, 300 tokens 274 / 147.
+// (With one k-tile on its way the first takes 181 us; at two workgroups a CU 179, and 478 tokens 257.)
+template <int ACT, int WN>
+__global__ __launch_bounds__(256, WN == 2 ? 3 : 4) void moe_parts_kernel(const float* __restrict__ A, const float* __restrict__ W, const float* __restrict__ W2,
+                                                           const int* __restrict__ tile_expert, float* __restrict__ out, long ldo, int N, int K,
+                                                           float limit) {
+  constexpr bool GLU = ACT == 1 || ACT == 3;
+  static_assert(!GLU || WN == 2, "a wave holds gate and up");
+  constexpr int ROWS = 64 + 64 * WN, PART = ROWS * TW_PART_ROW, COLS = GLU ? 64 : 64 * WN;
+  __shared__ __attribute__((aligned(16))) char lds[3 * PART];
+  const int tile = blockIdx.x * TW_MOE_WIDE;
+  const int ex = tile_expert[tile];
+  if (ex < 0) return;
+  const int col0 = blockIdx.y * COLS;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int r = lane & 31, g = lane >> 5;
+  const int wm0 = (wave >> 1) * 32;
+  const size_t tile_elems = (size_t)K * TW_MOE_TILE;
+  const int n_blocks = (N + 15) / 16;
+  // the matrix row of LDS row `row` behind the unit's 64, and where its block of 16 begins
+  auto block_of = [&](int row) {
+    const bool second = GLU && row >= 64;
+    const int block = min((col0 + (second ? row - 64 : row)) / 16, n_blocks - 1);
+    return (second ? W2 : W) + ((size_t)ex * n_blocks + block) * tile_elems;
+  };
+  auto wave_row = [&](int j) { return GLU ? 64 * j + (wave & 1) * 32 : (wave & 1) * 32 * WN + 32 * j; };
+
+  f32x16 acc[WN], small[WN];
+#pragma unroll
+  for (int j = 0; j < WN; ++j)
+#pragma unroll
+    for (int e = 0; e < 16; ++e) acc[j][e] = small[j][e] = 0.f;
+
+  const float* src[1 + WN];                                    // a thread's pieces: one of the rows, WN of the matrices
+  int at[1 + WN];
+  {
+    const int row = tid & 15, p = (tid >> 4) & 3, in_block = (p >> 1) * 256 + (p & 1) * 128 + row * 4;
+    src[0] = A + (size_t)(tile + wave) * tile_elems + in_block;
+    at[0] = tw_part_place(wave * 16 + row, p);
+#pragma unroll
+    for (int i = 0; i < WN; ++i) {
+      src[1 + i] = block_of(i * 64 + wave * 16) + in_block;
+      at[1 + i] = tw_part_place(64 + i * 64 + wave * 16 + row, p);
+    }
+  }
+  // (two k-tiles on their way: the experts' matrices come from HBM)
+  f32x4 regs[2][1 + WN][2];
+  auto load = [&](int kt, f32x4 (&reg)[1 + WN][2]) {
+#pragma unroll
+    for (int i = 0; i <= WN; ++i) {
+      reg[i][0] = tw_load_frag(src[i] + (size_t)kt * 512);
+      reg[i][1] = tw_load_frag(src[i] + (size_t)kt * 512 + 64);
+    }
+  };
+  const int swz = (r >> 2) & 3;
+  const int k_tiles = K / 32;
+  auto k_tile = [&](int kt, f32x4 (&reg)[1 + WN][2]) {
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i <= WN; ++i) {
+      bf16x8 h, m, l;
+      tw_three_parts(reg[i][0], reg[i][1], h, m, l);
+      *reinterpret_cast<bf16x8*>(lds + at[i]) = h;
+      *reinterpret_cast<bf16x8*>(lds + PART + at[i]) = m;
+      *reinterpret_cast<bf16x8*>(lds + 2 * PART + at[i]) = l;
+    }
+    load(min(kt + 2, k_tiles - 1), reg);                       // (unconditional: the last one again behind the end)
+    __syncthreads();
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+      const int piece = ((2 * s + g) ^ swz) * 16;
+      bf16x8 af[3], wf[3][WN];
+#pragma unroll
+      for (int p = 2; p >= 0; --p) {
+        af[p] = *reinterpret_cast<const bf16x8*>(lds + p * PART + (wm0 + r) * TW_PART_ROW + piece);
+#pragma unroll
+        for (int j = 0; j < WN; ++j) wf[p][j] = *reinterpret_cast<const bf16x8*>(lds + p * PART + (64 + wave_row(j) + r) * TW_PART_ROW + piece);
+      }
+      auto product = [&](f32x16 (&sum)[WN], int p, int q) {
+#pragma unroll
+        for (int j = 0; j < WN; ++j) tw_mma32(sum[j], af[p], wf[q][j]);
+      };
+      TW_PART_PRODUCTS(product);
+    }
+  };
+  load(0, regs[0]);
+  load(min(1, k_tiles - 1), regs[1]);
+  int kt = 0;
+  for (; kt + 1 < k_tiles; kt += 2) {
+    k_tile(kt, regs[0]);
+    k_tile(kt + 1, regs[1]);
+  }
+  if (kt < k_tiles) k_tile(kt, regs[0]);
+
+  float odd = 0.f;                                             // NaN as soon as one of them is not finite
+#pragma unroll
+  for (int j = 0; j < WN; ++j)
+#pragma unroll
+    for (int e = 0; e < 16; ++e) {
+      acc[j][e] += small[j][e];
+      odd = __fmaf_rn(acc[j][e], 0.f, odd);
+    }
+  if (__syncthreads_or(odd != odd)) {
+#pragma unroll
+    for (int j = 0; j < WN; ++j)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) acc[j][e] = 0.f;
+    const int in_block = g * 64 + (r & 15) * 4;
+    const float* a = A + (size_t)(tile + (wm0 + r) / 16) * tile_elems + in_block;
+    const float* w[WN];
+#pragma unroll
+    for (int j = 0; j < WN; ++j) w[j] = block_of(wave_row(j) + r) + in_block;
+    for (int k = 0; k < K; k += 8)                             // (8 elements of K are 128 floats of a block)
+#pragma unroll
+      for (int j = 0; j < WN; ++j) tw_mma32(acc[j], tw_load_frag(a + (size_t)k * 16), tw_load_frag(w[j] + (size_t)k * 16));
+  }
+
+#pragma unroll
+  for (int j = 0; j < (GLU ? 1 : WN); ++j) {
+    const int col = col0 + (GLU ? (wave & 1) * 32 : wave_row(j)) + r;
+    if (col >= N) continue;
+#pragma unroll
+    for (int e = 0; e < 16; ++e) {
+      const int row = wm0 + 8 * (e / 4) + 4 * g + e % 4;
+      const float z = acc[j][e];
+      if (ACT == 0) {
+        out[(size_t)(tile * TW_MOE_TILE + row) * ldo + col] = z;
+      } else {
+        const float y = ACT == 1 ? tw_swish_limited(z, acc[WN - 1][e], limit) : ACT == 3 ? tw_silu(z) * acc[WN - 1][e]
+                        : ACT == 4 ? fmaxf(z, 0.f) * fmaxf(z, 0.f) : 0.5f * z * (1.f + erff(z * 0.70710678118654752f));
+        out[(size_t)(tile + row / 16) * ldo * TW_MOE_TILE + ((size_t)(col / 4) * TW_MOE_TILE + row % 16) * 4 + col % 4] = y;
+      }
+    }
+  }
+}
+
 // ---- combine: x[token] += its experts' rows, in the order of its choices ------------------------------------------
 // A workgroup takes 1,024 columns of a row, four a thread where rows and addresses allow 16-byte accesses.
 // weights (or null): a factor on each of the token's rows; accumulate 0: x is written, not added to. more (or null):
@@ -666,6 +807,22 @@ static void moe_few_products(const T* rows, const T* first, const T* second, con
 #undef TW_MOE_FEW
 }
 
+// Where moe_parts_kernel takes a float32 step of many rows: where the first product has 140 workgroups of 64 columns and 256 of K. (Fewer
+// of either begin and end for longer than they multiply: 8 experts of 2,368 x 320, 848 tokens, 110 workgroups 96 -> 110 us; 16 of 160 x
+// 1,440, 128 tokens 41 -> 49.) A tile has 128 columns where they make more than 320 workgroups: 64 for 16 experts of 2,048 x 1,408 without a
+// gate, 128 tokens 148 -> 134 us, 1,000 tokens 232 -> 271.
+static bool moe_parts_pay(int units, int C, int Fd) { return units * tw_div_up(Fd, 64) > 140 && C >= 256; }
+template <int ACT>
+static void moe_parts(const float* rows, const float* W, const float* W2, const int* tile_expert, float* out, long ldo, int N, int K, float limit,
+                      int units, hipStream_t stream) {
+  if constexpr (ACT == 1 || ACT == 3)
+    moe_parts_kernel<ACT, 2><<<dim3(units, tw_div_up(N, 64)), 256, 0, stream>>>(rows, W, W2, tile_expert, out, ldo, N, K, limit);
+  else if (units * tw_div_up(N, 128) > 320)
+    moe_parts_kernel<ACT, 2><<<dim3(units, tw_div_up(N, 128)), 256, 0, stream>>>(rows, W, W2, tile_expert, out, ldo, N, K, limit);
+  else
+    moe_parts_kernel<ACT, 1><<<dim3(units, tw_div_up(N, 64)), 256, 0, stream>>>(rows, W, W2, tile_expert, out, ldo, N, K, limit);
+}
+
 // The two grouped products of a step: kind 0 gated with the limited swish, 1 up alone with gelu, 2 gated with SiLU, 3 up alone
 // with the square of relu.
 template <typename T, int ACT>
@@ -674,6 +831,13 @@ static void moe_products(const T* xs, const T* gate, const T* up, const T* down,
   constexpr bool PLAIN = ACT == 2 || ACT == 4;
   const T* first = PLAIN ? up : gate;
   const T* second = PLAIN ? nullptr : up;
+  if constexpr (sizeof(T) == 4) {
+    if (tiles > TW_MOE_SPLITK_TILES && wide && moe_parts_pay(tiles / TW_MOE_WIDE, C, Fd)) {
+      moe_parts<ACT>(xs, first, second, tile_expert, act, Fd, Fd, Cd, limit, tiles / TW_MOE_WIDE, stream);
+      moe_parts<0>(act, down, nullptr, tile_expert, ys, C, C, Fd, 0.f, tiles / TW_MOE_WIDE, stream);
+      return;
+    }
+  }
   if (tiles <= TW_MOE_SPLITK_TILES) {
     // few rows: most tiles hold one or two rows and each streams its expert's matrices once; the waves then split K
     moe_few_products<T, ACT, false>(xs, first, second, down, tile_expert, act, ys, C, Cd, Fd, limit, tiles,

@@ -511,28 +511,8 @@ __global__ __launch_bounds__(256) void gemm_tiled_kernel(const T* __restrict__ A
 // a result is formed again by the float32 MFMA from the operands themselves, and infinities, NaN and sums that overflow are what they are there.
 // (Parts below 2^-126 may be lost: of values below 2^-110.)
 // =====================================================================================
-#define TW_PART_ROW 64
-
-__device__ __forceinline__ void tw_three_parts(f32x4 lo, f32x4 hi, bf16x8& h, bf16x8& m, bf16x8& l) {
-  u32x4 ph, pm, pl;
-#pragma unroll
-  for (int e = 0; e < 4; ++e) {
-    const float x0 = e < 2 ? lo[2 * e] : hi[2 * e - 4], x1 = e < 2 ? lo[2 * e + 1] : hi[2 * e - 3];
-    const unsigned a0 = __float_as_uint(x0), a1 = __float_as_uint(x1);
-    const float y0 = x0 - __uint_as_float(a0 & 0xffff0000u), y1 = x1 - __uint_as_float(a1 & 0xffff0000u);
-    const unsigned b0 = __float_as_uint(y0), b1 = __float_as_uint(y1);
-    const float z0 = y0 - __uint_as_float(b0 & 0xffff0000u), z1 = y1 - __uint_as_float(b1 & 0xffff0000u);
-    ph[e] = __builtin_amdgcn_perm(a1, a0, 0x07060302);        // the upper halves side by side
-    pm[e] = __builtin_amdgcn_perm(b1, b0, 0x07060302);
-    pl[e] = __builtin_amdgcn_perm(__float_as_uint(z1), __float_as_uint(z0), 0x07060302);
-  }
-  h = __builtin_bit_cast(bf16x8, ph);
-  m = __builtin_bit_cast(bf16x8, pm);
-  l = __builtin_bit_cast(bf16x8, pl);
-}
-
 template <int WM, int WN, bool SHUF, bool GLU>
-__global__ __launch_bounds__(256, WN <= 2 ? 2 : 1) void gemm_parts_kernel(const float* __restrict__ A, long lda, const float* __restrict__ W, long ldw,
+__global__ __launch_bounds__(256, 2) void gemm_parts_kernel(const float* __restrict__ A, long lda, const float* __restrict__ W, long ldw,
                                                             const float* __restrict__ bias, const float* residual, long ldr, float* C,
                                                             long ldc, int M, int N, int K, int tiles_m, int n_blocks, int splits,
                                                             float* __restrict__ partial) {
@@ -573,12 +553,11 @@ __global__ __launch_bounds__(256, WN <= 2 ? 2 : 1) void gemm_parts_kernel(const 
   const int n_blocks_w = (N + 15) / 16;
   unsigned a_off[A_PIECES], w_off[W_PIECES];
   int a_st[A_PIECES], w_st[W_PIECES], w_k[W_PIECES];          // the piece's place in LDS; its first k (chunks of 4 that begin past K are zeros)
-  auto place = [](int row, int p) { return row * TW_PART_ROW + ((p ^ (row >> 2)) & 3) * 16; };
 #pragma unroll
   for (int i = 0; i < A_PIECES; ++i) {
     const int c = tid + i * 256, row = c >> 2, p = c & 3;
     a_off[i] = (unsigned)(min(m0 + row, M - 1) - m0) * (unsigned)lda + p * 8;
-    a_st[i] = place(row, p);
+    a_st[i] = tw_part_place(row, p);
   }
 #pragma unroll
   for (int i = 0; i < W_PIECES; ++i) {
@@ -587,12 +566,12 @@ __global__ __launch_bounds__(256, WN <= 2 ? 2 : 1) void gemm_parts_kernel(const 
       const int row = (c >> 6) * 16 + (c & 15), p = (c >> 4) & 3;
       const int gblk = min(n0 / 16 + (c >> 6), n_blocks_w - 1);
       w_off[i] = (unsigned)(gblk - n0 / 16) * (unsigned)ldw * 256 + (p >> 1) * 256 + (p & 1) * 128 + (c & 15) * 4;
-      w_st[i] = BM * TW_PART_ROW + place(row, p);
+      w_st[i] = BM * TW_PART_ROW + tw_part_place(row, p);
       w_k[i] = p * 8;
     } else {
       const int row = c >> 2, p = c & 3;
       w_off[i] = (unsigned)(min(n0 + row, N - 1) - n0) * (unsigned)ldw + p * 8;
-      w_st[i] = BM * TW_PART_ROW + place(row, p);
+      w_st[i] = BM * TW_PART_ROW + tw_part_place(row, p);
       w_k[i] = p * 8;
     }
   }
@@ -665,12 +644,7 @@ __global__ __launch_bounds__(256, WN <= 2 ? 2 : 1) void gemm_parts_kernel(const 
 #pragma unroll
           for (int j = 0; j < WN; ++j) tw_mma32(sum[i][j], af[p][i], wf[q][j]);
       };
-      product(small, 2, 0);
-      product(small, 0, 2);
-      product(small, 1, 1);
-      product(small, 1, 0);
-      product(small, 0, 1);
-      product(acc, 0, 0);
+      TW_PART_PRODUCTS(product);
     }
   };
 

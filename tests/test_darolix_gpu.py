@@ -450,6 +450,37 @@ def test_grouped_experts_of_many_rows_and_long_sums(device, dtype, kind, n, X, t
     assert torch.allclose(x.double(), want, atol=2e-5 if dtype == "float32" else 4e-2)
 
 
+@pytest.mark.parametrize("kind", ["silu", "gelu", "swish_limited"])
+@pytest.mark.parametrize("n,X,top,C,F", [(600, 16, 2, 288, 544), (1100, 8, 2, 330, 1600), (600, 16, 2, 1190, 416), (500, 64, 4, 256, 160)])
+def test_float32_grouped_experts_in_three_parts(device, kind, n, X, top, C, F):
+    """Products of bfloat16 parts: tiles of 64 and 128 columns that the columns end inside, an odd and an even number of k-tiles,
+    units with and without rows. The oracle and the bars of the other forms; the sums are rounded less often."""
+    test_grouped_experts_of_many_rows_and_long_sums(device, "float32", kind, n, X, top, C, F)
+
+
+def test_float32_grouped_experts_of_values_without_parts(device):
+    """A token with an infinity and one with a NaN, their experts' other tokens beside them in the same tiles."""
+    from tessweave_engine_amd.kernels import ops
+    g = torch.Generator().manual_seed(5)
+    n, X, C, F = 400, 4, 256, 512
+    h = torch.randn(n, C, generator=g).to(device)
+    gate, up = (torch.randn(X, F, C, generator=g).to(device) / 16 for _ in range(2))
+    down = torch.randn(X, C, F, generator=g).to(device) / 16
+    ids = torch.randint(0, X, (n, 1), generator=g).to(torch.int32).to(device)
+    results = []
+    for odd in (False, True):
+        if odd:
+            h[17, 3], h[300, 255] = float("inf"), float("nan")
+        x = torch.zeros(n, C, device=device)
+        ops.moe_experts(h, ids, torch.ones(n, 1, device=device), ops.moe_blocked(gate), ops.moe_blocked(up), ops.moe_blocked(down), 0.0, x,
+                        lambda tag, shape, kind_: torch.empty(shape, dtype=kind_, device=device), kind="silu")
+        results.append(x)
+    rows = torch.tensor([i for i in range(n) if i not in (17, 300)], device=device)
+    assert not bool(results[1][[17, 300]].isfinite().any())
+    # (float32 sums of 256 and 512 products of terms of size 1 over the square root of their number, by either way)
+    assert torch.allclose(results[0][rows], results[1][rows], atol=1e-5, rtol=1e-5)
+
+
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 @pytest.mark.parametrize("kind", ["silu", "gelu", "swish_limited"])
 @pytest.mark.parametrize("n,X,top,C,F", [(1, 4, 2, 32, 32), (8, 32, 2, 544, 96), (2, 24, 2, 288, 1088), (17, 40, 1, 800, 144), (16, 20, 4, 256, 288),
