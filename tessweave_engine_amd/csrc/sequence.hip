@@ -625,10 +625,13 @@ extern "C" int tw_gated_recurrence(int dtype, const float* gates, long ld_gates,
 
 // ---- block-diagonal product: out[n][b * No + o] = sum_i x[n][b * Ni + i] * w[b][o][i] + bias[b * No + o] ---------
 // `blocks` square-ish matrices [No][Ni] side by side along the diagonal (the gates of a recurrence read only
-// their own block of channels). One wave takes 16 rows and 64 output columns of one block: the weights are the
+// their own block of channels). One wave takes 16 rows and 16 * TILES output columns of one block: the weights are the
 // A operand (so a lane ends with 4 consecutive output columns of one row), the rows the B operand, both read
-// straight from memory in 16-byte fragments. Ni must be a multiple of 16 bytes, No of 16.
-template <typename T>
+// straight from memory in 16-byte fragments, STEPS steps over Ni on their way at once. Ni must be a multiple of 16 bytes, No of 16.
+// Many rows: 64 columns, so that a row is read a quarter as often. Up to 64 rows a wave's trips to memory are its time: 16 columns and
+// eight steps at once; up to 128, 32 and four. (8 blocks of 512 x 256 in bfloat16, us, 16 / 32 / 64 columns: one row 3.0 / - / 7.0, 64 4.0 /
+// 5.1 / 7.4, 100 5.8 / 5.3 / 7.3, 200 9.1 / 8.0 / 7.6, 2,047 60 / 47 / 41; float32, one row 4.9 / - / 15.0.)
+template <typename T, int TILES, int STEPS>
 __global__ __launch_bounds__(256) void block_diagonal_kernel(const T* __restrict__ x, long ldx, const T* __restrict__ w,
                                                              const float* __restrict__ bias, float* __restrict__ out,
                                                              long ldo, int n, int blocks, int Ni, int No, int col_groups) {
@@ -636,31 +639,38 @@ __global__ __launch_bounds__(256) void block_diagonal_kernel(const T* __restrict
   constexpr int EPF = Elem<T>::kPerFrag;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int r = lane & 15, g = lane >> 4;
-  const int unit = blockIdx.x * 4 + wave;                  // (block, group of 64 columns)
+  const int unit = blockIdx.x * 4 + wave;                  // (block, group of columns)
   const int b = unit / col_groups, cg = unit % col_groups;
   if (b >= blocks) return;
   const int row0 = blockIdx.y * 16;
   const int chunks = Ni / EPF, steps = (chunks + 3) / 4;
   const int row = row0 + r;
   const T* x_row = x + (size_t)(row < n ? row : 0) * ldx + (size_t)b * Ni;
-  f32x4 acc[4];
+  f32x4 acc[TILES];
 #pragma unroll
-  for (int t = 0; t < 4; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-  for (int st = 0; st < steps; ++st) {
-    const int chunk = st * 4 + g;
-    const bool in = chunk < chunks;
-    const Frag xf = (in && row < n) ? tw_load_frag(x_row + chunk * EPF) : Elem<T>::zero();
+  for (int t = 0; t < TILES; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int st = 0; st < steps; st += STEPS) {
+    Frag xf[STEPS], wf[STEPS][TILES];
 #pragma unroll
-    for (int t = 0; t < 4; ++t) {
-      const int o = cg * 64 + t * 16 + r;
-      const Frag wf = (in && o < No) ? tw_load_frag(w + ((size_t)b * No + o) * Ni + chunk * EPF) : Elem<T>::zero();
-      tw_mma16(acc[t], wf, xf);                            // D[output 4g + e][row r]
+    for (int u = 0; u < STEPS; ++u) {
+      const int chunk = (st + u) * 4 + g;
+      const bool in = chunk < chunks;
+      xf[u] = (in && row < n) ? tw_load_frag(x_row + chunk * EPF) : Elem<T>::zero();
+#pragma unroll
+      for (int t = 0; t < TILES; ++t) {
+        const int o = (cg * TILES + t) * 16 + r;
+        wf[u][t] = (in && o < No) ? tw_load_frag(w + ((size_t)b * No + o) * Ni + chunk * EPF) : Elem<T>::zero();
+      }
     }
+#pragma unroll
+    for (int u = 0; u < STEPS; ++u)
+#pragma unroll
+      for (int t = 0; t < TILES; ++t) tw_mma16(acc[t], wf[u][t], xf[u]);   // D[output 4g + e][row r]
   }
   if (row >= n) return;
 #pragma unroll
-  for (int t = 0; t < 4; ++t) {
-    const int o = cg * 64 + t * 16 + 4 * g;
+  for (int t = 0; t < TILES; ++t) {
+    const int o = (cg * TILES + t) * 16 + 4 * g;
     if (o < No) {
       f32x4 v = acc[t];
 #pragma unroll
@@ -668,6 +678,14 @@ __global__ __launch_bounds__(256) void block_diagonal_kernel(const T* __restrict
       *reinterpret_cast<f32x4*>(out + (size_t)row * ldo + (size_t)b * No + o) = v;
     }
   }
+}
+
+template <typename T, int TILES, int STEPS>
+static void block_diagonal_launch(const void* x, long ldx, const void* w, const float* bias, float* out, long ldo, int n, int blocks, int Ni,
+                                  int No, hipStream_t stream) {
+  const int col_groups = tw_div_up(No, 16 * TILES);
+  block_diagonal_kernel<T, TILES, STEPS><<<dim3(tw_div_up((long)blocks * col_groups, 4), tw_div_up(n, 16)), 256, 0, stream>>>(
+      (const T*)x, ldx, (const T*)w, bias, out, ldo, n, blocks, Ni, No, col_groups);
 }
 
 extern "C" int tw_block_diagonal(int dtype, const void* x, long ldx, const void* w, const float* bias, float* out,
@@ -678,12 +696,15 @@ extern "C" int tw_block_diagonal(int dtype, const void* x, long ldx, const void*
   TW_REQUIRE(Ni % epf == 0 && No % 16 == 0 && ldx % epf == 0 && ldx >= (long)blocks * Ni && ldo % 4 == 0 && ldo >= (long)blocks * No);
   TW_REQUIRE((uintptr_t)x % 16 == 0 && (uintptr_t)w % 16 == 0 && (uintptr_t)out % 16 == 0);
   if (n == 0) return 0;
-  const int col_groups = tw_div_up(No, 64);
-  const dim3 grid(tw_div_up((long)blocks * col_groups, 4), tw_div_up(n, 16));
-  if (dtype == TW_DTYPE_BF16)
-    block_diagonal_kernel<bf16_t><<<grid, 256, 0, stream>>>((const bf16_t*)x, ldx, (const bf16_t*)w, bias, out, ldo, n, blocks, Ni, No, col_groups);
-  else
-    block_diagonal_kernel<float><<<grid, 256, 0, stream>>>((const float*)x, ldx, (const float*)w, bias, out, ldo, n, blocks, Ni, No, col_groups);
+  if (dtype == TW_DTYPE_BF16) {
+    if (n <= 64) block_diagonal_launch<bf16_t, 1, 8>(x, ldx, w, bias, out, ldo, n, blocks, Ni, No, stream);
+    else if (n <= 128) block_diagonal_launch<bf16_t, 2, 4>(x, ldx, w, bias, out, ldo, n, blocks, Ni, No, stream);
+    else block_diagonal_launch<bf16_t, 4, 1>(x, ldx, w, bias, out, ldo, n, blocks, Ni, No, stream);
+  } else {
+    if (n <= 64) block_diagonal_launch<float, 1, 8>(x, ldx, w, bias, out, ldo, n, blocks, Ni, No, stream);
+    else if (n <= 128) block_diagonal_launch<float, 2, 4>(x, ldx, w, bias, out, ldo, n, blocks, Ni, No, stream);
+    else block_diagonal_launch<float, 4, 1>(x, ldx, w, bias, out, ldo, n, blocks, Ni, No, stream);
+  }
   return TW_LAUNCH_RESULT();
 }
 
@@ -796,11 +817,65 @@ __global__ __launch_bounds__(256) void layer_end_kernel(float* __restrict__ x, c
   }
 }
 
+// The same for few rows, four columns a thread: what bounds it is a row's trips to memory, so everything a thread needs (the whole
+// row of y for the sum of squares, PER pieces of it, and its own columns of x, w and up to eight earlier results) is on its way
+// at once. A block has 1,024 columns. (In a chain of its like, a row of 2,048 and four results 3.8 -> 2.6 us, of 4,096 4.6 -> 2.7.)
+template <int PER>
+__global__ __launch_bounds__(256) void layer_end_few_kernel(float* __restrict__ x, const float* __restrict__ y, const float* __restrict__ w,
+                                                            float eps, float mult, float* __restrict__ history, long history_stride,
+                                                            int layer, const float* __restrict__ mix, int width) {
+  constexpr int HELD = 8;
+  __shared__ float red[16];
+  const size_t row = (size_t)blockIdx.x * width;
+  const int own = (blockIdx.y * 256 + threadIdx.x) * 4;
+  const int at = min(own, width - 4);                        // (a thread without columns reads the last ones)
+  f32x4 yv[PER], yo, wv, held[HELD];
+  f32x4 v = *reinterpret_cast<const f32x4*>(x + row + at);
+  if (y) {
+    yo = *reinterpret_cast<const f32x4*>(y + row + at);
+    wv = *reinterpret_cast<const f32x4*>(w + at);
+#pragma unroll
+    for (int i = 0; i < PER; ++i) yv[i] = *reinterpret_cast<const f32x4*>(y + row + min((int)(i * 256 + threadIdx.x) * 4, width - 4));
+  }
+  const float* past = history + row + at;
+  if (mix) {
+#pragma unroll
+    for (int j = 0; j < HELD; ++j) held[j] = *reinterpret_cast<const f32x4*>(past + (size_t)min(j, layer) * history_stride);
+  }
+  if (y) {
+    float sum = 0.f;
+#pragma unroll
+    for (int i = 0; i < PER; ++i)
+      if ((int)(i * 256 + threadIdx.x) * 4 < width) sum += ((yv[i][0] * yv[i][0] + yv[i][1] * yv[i][1]) + yv[i][2] * yv[i][2]) + yv[i][3] * yv[i][3];
+    const float scale = mult * rsqrtf(tw_block_sum(sum, red) / (float)width + eps);
+    v += scale * yo * wv;
+  }
+  if (own >= width) return;
+  if (history) *reinterpret_cast<f32x4*>(history + (size_t)(layer + 1) * history_stride + row + own) = v;
+  if (mix) {
+    v = mix[layer + 1] * v;
+#pragma unroll
+    for (int j = 0; j < HELD; ++j)
+      if (j <= layer) v += mix[j] * held[j];
+    for (int j = HELD; j <= layer; ++j) v += mix[j] * *reinterpret_cast<const f32x4*>(past + (size_t)j * history_stride);
+  }
+  *reinterpret_cast<f32x4*>(x + row + own) = v;
+}
+
 extern "C" int tw_layer_end(float* x, const float* y, const float* w, float eps, float mult, float* history,
                             long history_stride, int layer, const float* mix, int n, int width, hipStream_t stream) {
   TW_REQUIRE(x && n >= 0 && width > 0 && layer >= 0 && (!y || w) && (!mix || history));
   TW_REQUIRE(!history || history_stride >= (long)n * width);
   if (n == 0) return 0;
+  // (rows in whole pieces; from 512 rows on the chip is full of rows and memory is what bounds it)
+  const bool pieces = width % 4 == 0 && history_stride % 4 == 0 && (uintptr_t)x % 16 == 0 && (uintptr_t)y % 16 == 0 && (uintptr_t)w % 16 == 0 &&
+                      (uintptr_t)history % 16 == 0;
+  if (n < 512 && pieces && width <= 4096) {
+    const dim3 grid(n, tw_div_up(width, 1024));
+    if (width <= 2048) layer_end_few_kernel<2><<<grid, 256, 0, stream>>>(x, y, w, eps, mult, history, history_stride, layer, mix, width);
+    else layer_end_few_kernel<4><<<grid, 256, 0, stream>>>(x, y, w, eps, mult, history, history_stride, layer, mix, width);
+    return TW_LAUNCH_RESULT();
+  }
   int shares = n >= 512 ? 1 : tw_div_up(width, 512);
   if (shares > 8) shares = 8;
   layer_end_kernel<<<dim3(n, shares), 256, 0, stream>>>(x, y, w, eps, mult, history, history_stride, layer, mix, width);

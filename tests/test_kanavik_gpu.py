@@ -401,6 +401,34 @@ def test_block_diagonal_product(device, dtype, n, blocks, n_in, n_out):
 
 
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("n,blocks,n_in,n_out", [(1, 3, 264, 48), (64, 2, 256, 80), (65, 5, 128, 32), (128, 3, 136, 112), (129, 1, 40, 16)])
+def test_block_diagonal_product_by_rows(device, dtype, n, blocks, n_in, n_out):
+    """Rows at the edges of the three forms; steps that fill a form's requests, are one more, and end inside one; columns that end
+    inside a wave's."""
+    test_block_diagonal_product(device, dtype, n, blocks, n_in, n_out)
+
+
+@pytest.mark.parametrize("n,width,layer", [(1, 4, 0), (3, 1028, 2), (511, 2048, 7), (2, 2052, 8), (5, 4096, 11), (512, 2048, 3), (2, 4100, 2), (3, 1030, 1)])
+@pytest.mark.parametrize("branch", [True, False])
+def test_layer_end_of_few_rows(device, n, width, layer, branch):
+    """Rows shorter than a block, of whole blocks, a piece longer; up to and past the results held at once; and the sizes that the other
+    form takes. Sums of twelve products of sizes below 5 x 4: off by less than 16 x 2^-24 of 240."""
+    from tessweave_engine_amd.kernels import ops
+    g = torch.Generator().manual_seed(n + width)
+    x, y = torch.randn(n, width, generator=g), torch.randn(n, width, generator=g)
+    w, mix = torch.randn(width, generator=g), torch.randn(layer + 2, generator=g)
+    hist = torch.randn(layer + 3, n, width, generator=g)
+    hist[layer + 1:] = float("nan")
+    xd, hd = x.to(device), hist.to(device)
+    ops.layer_end(xd, layer, branch=y.to(device) if branch else None, branch_weight=w.to(device) if branch else None, eps=1e-5, mult=0.4,
+                  history=hd, mix=mix.to(device))
+    result = x.double() + (0.4 * plain.rms_unit(y.double(), 1e-5) * w.double() if branch else 0.0)
+    mixed = sum(mix[j].double() * hist[j].double() for j in range(layer + 1)) + mix[layer + 1].double() * result
+    assert torch.allclose(hd[layer + 1].cpu().double(), result, atol=2e-5) and bool(hd[layer + 2:].isnan().all())
+    assert torch.allclose(xd.cpu().double(), mixed, atol=2.5e-4)
+
+
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 @pytest.mark.parametrize("rows", [3, 40, 300])
 def test_gated_product_with_gelu_and_a_factor(device, dtype, rows):
     """The matrix kernels' gated epilogue with the tanh form of gelu (few rows, 17-64 rows, tiled) and shuffled weights."""
