@@ -565,7 +565,20 @@ __global__ __launch_bounds__(256) void gated_recurrence_kernel(RecurrenceArgs a)
     S = *st;
   } else {
     S = part[2 * (size_t)a.C];
-    for (int j = 0; j < z; ++j) S = part[((size_t)j * 3 + 0) * a.C] * S + part[((size_t)j * 3 + 1) * a.C];
+    // (sixteen chunks' pairs requested together: one after the other, the last of 64 chunks waited for memory 63
+    // times: 2,047 tokens of 2,048 channels 39 -> 27 us)
+    for (int j = 0; j < z; j += 16) {
+      float P[16], Q[16];
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        const size_t at = (size_t)min(j + i, z - 1) * 3;
+        P[i] = part[at * a.C];
+        Q[i] = part[(at + 1) * a.C];
+      }
+#pragma unroll
+      for (int i = 0; i < 16; ++i)
+        if (j + i < z) S = P[i] * S + Q[i];
+    }
   }
   const T* branch = (const T*)a.branch;
   int t = t0;

@@ -381,6 +381,24 @@ def test_gated_recurrence_carries_its_state(device, dtype):
     assert torch.allclose(state[1].cpu().double(), S[-1], atol=1e-5, rtol=1e-5)
 
 
+@pytest.mark.parametrize("n", [512, 513, 544, 545, 1088])
+def test_gated_recurrence_of_many_chunks(device, n):
+    """A last chunk with 15, 16, 17 and 33 before it, whose states it adds up sixteen at a time. The bar of the portions."""
+    from tessweave_engine_amd.kernels import ops
+    g = torch.Generator().manual_seed(n)
+    R = 16
+    u, ga, gi, branch = (torch.randn(n, R, generator=g) for _ in range(4))
+    lam = torch.randn(R, generator=g) - 4                  # (slow decays: the first chunks still count in the last)
+    S = plain.gated_recurrence(u.double(), torch.sigmoid(ga.double()), torch.sigmoid(gi.double()), lam.double())
+    state, out = torch.zeros(1, R, device=device), torch.empty(n, R, device=device)
+    ws = torch.full((ops.gated_recurrence_workspace_floats(1, n, R),), float("nan"), device=device)
+    ops.gated_recurrence(torch.cat([ga, gi], 1).to(device), u.to(device), branch.to(device), lam.to(device), state,
+                         torch.tensor([0, n], dtype=torch.int32, device=device), torch.zeros(1, dtype=torch.int32, device=device), 1, n, out,
+                         1, 8.0, workspace=ws)
+    assert torch.allclose(state[0].cpu().double(), S[-1], atol=1e-4, rtol=1e-4)
+    assert torch.allclose(out.cpu().double(), S * plain.gelu_tanh(branch.double()), atol=1e-4, rtol=1e-4)
+
+
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 @pytest.mark.parametrize("n,blocks,n_in,n_out", [(1, 3, 8, 16), (37, 2, 40, 80), (130, 16, 128, 256)])
 def test_block_diagonal_product(device, dtype, n, blocks, n_in, n_out):
