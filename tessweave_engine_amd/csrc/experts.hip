@@ -570,8 +570,8 @@ __global__ __launch_bounds__(WAVES * 64) void moe_grouped_kernel(const T* __rest
 // a 2x2 grid, wave tile 32 x (32 * WN). A k-tile is two k-steps; rows and matrices are read in fragment order, split and laid into LDS, two
 // k-tiles are on their way (the matrices come from HBM) and three workgroups share a CU. What is not finite is formed again from the
 // operands themselves. All launches of the experts, us, the float32 MFMA / this: 16 experts of 2,048 x 1,408, two a token, gated, 128 tokens
-// 303 / 163, 478 349 / 221, 2,000 954 / 594; 8 of 4,096 x 2,048, 300 tokens 714 / 413; 64 of 1,024 x 512, four a token, 300 tokens 274 / 147.
-// (With one k-tile on its way the first takes 181 us; at two workgroups a CU 179, and 478 tokens 257.)
+// 303 / 193, 478 423 / 257, 2,000 956 / 661; 8 of 4,096 x 2,048, 300 tokens 751 / 487; 64 of 1,024 x 512, four a token, 300 tokens 274 / 153.
+// (With six products and one k-tile on its way the first took 181 us against 163; at two workgroups a CU 179, and 478 tokens 257 against 221.)
 template <int ACT, int WN>
 __global__ __launch_bounds__(256, WN == 2 ? 3 : 4) void moe_parts_kernel(const float* __restrict__ A, const float* __restrict__ W, const float* __restrict__ W2,
                                                            const int* __restrict__ tile_expert, float* __restrict__ out, long ldo, int N, int K,

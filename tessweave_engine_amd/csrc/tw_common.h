@@ -131,32 +131,34 @@ __device__ __forceinline__ void tw_mma32(f32x16& acc, f32x4 a, f32x4 b) {
 }
 
 // ---- float32 as three bfloat16 parts ------------------------------------------------
-// x = h + m + l: h is x with its low 16 bits cleared, m the same of x - h, l the rest; nothing is rounded (a finite x above 2^-110).
-// Of eight values of a row, for the bfloat16 MFMAs of gemm_parts_kernel and moe_parts_kernel.
+// x = h + m + l, as is well known: h is x rounded to bfloat16, m what is left rounded to bfloat16, l what is then left. x - h is a multiple
+// of x's last place and below 2^-8 of x, x - h - m below 2^-17, so that l has six bits and the three parts are x (a finite x above
+// 2^-110). They are rounded to the nearest, so m and l have either sign: parts cut off have x's own, and what is left out of a sum
+// of products then always makes it smaller. Of eight values of a row, for the bfloat16 MFMAs of gemm_parts_kernel and moe_parts_kernel.
 __device__ __forceinline__ void tw_three_parts(f32x4 lo, f32x4 hi, bf16x8& h, bf16x8& m, bf16x8& l) {
   u32x4 ph, pm, pl;
+  auto two = [](float a, float b) { return __builtin_bit_cast(unsigned, bf16x2{(bf16_t)a, (bf16_t)b}); };
 #pragma unroll
   for (int e = 0; e < 4; ++e) {
     const float x0 = e < 2 ? lo[2 * e] : hi[2 * e - 4], x1 = e < 2 ? lo[2 * e + 1] : hi[2 * e - 3];
-    const unsigned a0 = __float_as_uint(x0), a1 = __float_as_uint(x1);
-    const float y0 = x0 - __uint_as_float(a0 & 0xffff0000u), y1 = x1 - __uint_as_float(a1 & 0xffff0000u);
-    const unsigned b0 = __float_as_uint(y0), b1 = __float_as_uint(y1);
-    const float z0 = y0 - __uint_as_float(b0 & 0xffff0000u), z1 = y1 - __uint_as_float(b1 & 0xffff0000u);
-    ph[e] = __builtin_amdgcn_perm(a1, a0, 0x07060302);        // the upper halves side by side
-    pm[e] = __builtin_amdgcn_perm(b1, b0, 0x07060302);
-    pl[e] = __builtin_amdgcn_perm(__float_as_uint(z1), __float_as_uint(z0), 0x07060302);
+    ph[e] = two(x0, x1);
+    const float y0 = x0 - __uint_as_float(ph[e] << 16), y1 = x1 - __uint_as_float(ph[e] & 0xffff0000u);
+    pm[e] = two(y0, y1);
+    pl[e] = two(y0 - __uint_as_float(pm[e] << 16), y1 - __uint_as_float(pm[e] & 0xffff0000u));
   }
   h = __builtin_bit_cast(bf16x8, ph);
   m = __builtin_bit_cast(bf16x8, pm);
   l = __builtin_bit_cast(bf16x8, pl);
 }
 
-// A part's rows in LDS: 64 bytes, 32 elements of K, four pieces; and the six products of the parts (0: h, 1: m, 2: l) of a 32x32 tile,
-// the smallest first. m l, l m and l l are below 2^-22 of the whole product.
+// A part's rows in LDS: 64 bytes, 32 elements of K, four pieces; and the products of the parts (0: h, 1: m, 2: l) of a 32x32 tile, the
+// smallest first. All but l l, which is below 2^-34 of the whole product: with m l and l m left out too one product is off by up to 2^-24 more
+// than its rounding.
 #define TW_PART_ROW 64
 __device__ __forceinline__ constexpr int tw_part_place(int row, int piece) { return row * TW_PART_ROW + ((piece ^ (row >> 2)) & 3) * 16; }
-#define TW_PART_PRODUCTS(product)                                                       \
-  product(small, 2, 0); product(small, 0, 2); product(small, 1, 1); product(small, 1, 0); product(small, 0, 1); product(acc, 0, 0)
+#define TW_PART_PRODUCTS(product)                                                                                   \
+  product(small, 2, 1); product(small, 1, 2); product(small, 2, 0); product(small, 0, 2); product(small, 1, 1);       \
+  product(small, 1, 0); product(small, 0, 1); product(acc, 0, 0)
 
 // ---- reductions ------------------------------------------------------------------
 // A value combined over lanes l, l ^ 16, l ^ 32, l ^ 48 (the four 16-lane rows of a wave) with gfx950's

@@ -458,6 +458,38 @@ def test_float32_grouped_experts_in_three_parts(device, kind, n, X, top, C, F):
     test_grouped_experts_of_many_rows_and_long_sums(device, "float32", kind, n, X, top, C, F)
 
 
+def _experts_that_select(device, kind, h, first, up=None):
+    """x of routed experts of many float32 rows (43 units: tiles of 128 columns in front, of 64 behind) whose down matrix passes the first C
+    inner elements on, one expert a token, and which token has which."""
+    from tessweave_engine_amd.kernels import ops
+    (n, C), (X, F, _) = h.shape, first.shape
+    ids = (torch.arange(n, device=device) * 5 % X).to(torch.int32)[:, None].contiguous()
+    down = torch.zeros(X, C, F, device=device)
+    down[:, torch.arange(C), torch.arange(C)] = 1.0
+    x = torch.zeros(n, C, device=device)
+    ops.moe_experts(h, ids, torch.ones(n, 1, device=device), ops.moe_blocked(first) if up is not None else None,
+                    ops.moe_blocked(first if up is None else up), ops.moe_blocked(down), 0.0, x,
+                    lambda tag, shape, kind_: torch.empty(shape, dtype=kind_, device=device), kind=kind)
+    return x, ids[:, 0].long()
+
+
+@pytest.mark.parametrize("kind", ["silu", "relu_squared"])
+def test_float32_grouped_experts_keep_the_bits_of_a_product(device, kind):
+    """Rows of one element that is not zero: a product is rounded once (and by less than 2^-6 of that in its smaller parts' sums), the
+    product of the two, or the square, once more, and the other matrix passes it on. The gate's results are past 40, where silu(z) is z."""
+    n, X, C, F = 2200, 8, 288, 1600
+    g = torch.Generator().manual_seed(6)
+    col, value = torch.arange(n) * 7 % C, torch.rand(n, generator=g) + 0.5
+    h = torch.zeros(n, C)
+    h[torch.arange(n), col] = value
+    first, up = 100 * torch.rand(X, F, C, generator=g) + 100, torch.randn(X, F, C, generator=g)
+    h, first, up, col, value = (t.to(device) for t in (h, first, up, col, value))
+    x, ex = _experts_that_select(device, kind, h, *((first, up) if kind == "silu" else (up,)))
+    u = up.double()[ex, :C, col] * value.double()[:, None]
+    want = u * first.double()[ex, :C, col] * value.double()[:, None] if kind == "silu" else u.clamp(min=0) ** 2
+    assert bool(((x.double() - want).abs() <= (3 + 2.0 ** -4) * 2.0 ** -24 * want.abs()).all())
+
+
 def test_float32_grouped_experts_of_values_without_parts(device):
     """A token with an infinity and one with a NaN, their experts' other tokens beside them in the same tiles."""
     from tessweave_engine_amd.kernels import ops

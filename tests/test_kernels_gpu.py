@@ -633,13 +633,32 @@ def test_linear_sums_in_pieces_of_k(ops, device, m, n, k, ranges):
 
 @pytest.mark.parametrize("m,n,k", [(65, 33, 4), (66, 130, 36), (129, 300, 76), (200, 1024, 512), (478, 2080, 1040), (640, 4096, 96)])
 def test_float32_linear_in_three_parts(ops, device, m, n, k):
-    """float32 products of many rows are six bfloat16 ones: all tiles, rows, columns and K that end inside one, K ranges, magnitudes
+    """float32 products of many rows are eight bfloat16 ones: all tiles, rows, columns and K that end inside one, K ranges, magnitudes
     2^24 apart, all of one sign. The sum of the leading parts is rounded no more than twice in 16 elements of K, the others' sum is
-    2^-7 of it and less, and the three products left out and the last additions come to less than 4 x 2^-24 of the sum of sizes."""
+    2^-7 of it and less, and the product left out and the last additions come to less than 4 x 2^-24 of the sum of sizes."""
     x = rand((m, k), torch.float32, device, 1.0, seed=1) * torch.exp2(rand((k,), torch.float32, device, 6.0, seed=3).round().clamp(-12, 12))
     for x, w in ((x, rand((n, k), torch.float32, device, 0.05, seed=2)), (x.abs(), rand((n, k), torch.float32, device, 0.05, seed=2).abs())):
         want, near = x.double() @ w.double().T, (k / 8 + 4) * 2.0 ** -24 * (x.double().abs() @ w.double().abs().T)
         space = torch.empty(ops.linear_workspace_bytes(torch.float32, m, n, k) // 4 + 4, device=device)
+        for weight in (w, ops.shuffle_weight(w)):
+            for force in (ops.GEMM_AUTO, ops.GEMM_TILED, ops.GEMM_TILED_WIDE):
+                out = torch.full((m, n), float("nan"), device=device)
+                ops.linear(x, weight, out, workspace=space, force=force)
+                assert bool(((out.double() - want).abs() <= near).all())
+
+
+@pytest.mark.parametrize("k", [4, 36, 256])
+def test_float32_linear_keeps_the_bits_of_a_product(ops, device, k):
+    """Rows of one element that is not zero: a product is rounded once to float32, 2^-24 of it, and what its smaller parts' sums are rounded
+    by is below 2^-6 of that. And operands of whose parts everything left out would have one sign: K equal products in sums of 16,
+    which are rounded no more than twice each, and at the end."""
+    m, n = 130, 260
+    one, w = torch.zeros(m, k, device=device), rand((n, k), torch.float32, device, 0.05, seed=2)
+    one[torch.arange(m), torch.arange(m) * 7 % k] = rand((m,), torch.float32, device, 1.0, seed=1)
+    worst = torch.full((m + n, k), 0x3F80FFFF, dtype=torch.int32, device=device).view(torch.float32)
+    space = torch.empty(ops.linear_workspace_bytes(torch.float32, m, n, k) // 4 + 4, device=device)
+    for x, w, most in ((one, w, 1 + 2.0 ** -6), (worst[:m], worst[m:], k / 8 + 1)):
+        want, near = x.double() @ w.double().T, most * 2.0 ** -24 * (x.double().abs() @ w.double().abs().T)
         for weight in (w, ops.shuffle_weight(w)):
             for force in (ops.GEMM_AUTO, ops.GEMM_TILED, ops.GEMM_TILED_WIDE):
                 out = torch.full((m, n), float("nan"), device=device)
