@@ -570,7 +570,7 @@ __global__ __launch_bounds__(WAVES * 64) void moe_grouped_kernel(const T* __rest
 // a 2x2 grid, wave tile 32 x (32 * WN). A k-tile is two k-steps; rows and matrices are read in fragment order, split and laid into LDS, two
 // k-tiles are on their way (the matrices come from HBM) and three workgroups share a CU. What is not finite is formed again from the
 // operands themselves. All launches of the experts, us, the float32 MFMA / this: 16 experts of 2,048 x 1,408, two a token, gated, 128 tokens
-// 303 / 193, 478 423 / 257, 2,000 956 / 661; 8 of 4,096 x 2,048, 300 tokens 751 / 487; 64 of 1,024 x 512, four a token, 300 tokens 274 / 153.
+// 303 / 198, 478 423 / 266, 2,000 956 / 673; 8 of 4,096 x 2,048, 300 tokens 751 / 497; 64 of 1,024 x 512, four a token, 300 tokens 274 / 154.
 // (With six products and one k-tile on its way the first took 181 us against 163; at two workgroups a CU 179, and 478 tokens 257 against 221.)
 template <int ACT, int WN>
 __global__ __launch_bounds__(256, WN == 2 ? 3 : 4) void moe_parts_kernel(const float* __restrict__ A, const float* __restrict__ W, const float* __restrict__ W2,
@@ -685,6 +685,11 @@ __global__ __launch_bounds__(256, WN == 2 ? 3 : 4) void moe_parts_kernel(const f
     for (int k = 0; k < K; k += 8)                             // (8 elements of K are 128 floats of a block)
 #pragma unroll
       for (int j = 0; j < WN; ++j) tw_mma32(acc[j], tw_load_frag(a + (size_t)k * 16), tw_load_frag(w[j] + (size_t)k * 16));
+  } else {
+#pragma unroll
+    for (int j = 0; j < WN; ++j)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) acc[j][e] *= TW_PART_BACK;
   }
 
 #pragma unroll

@@ -489,7 +489,7 @@ __global__ __launch_bounds__(256) void gemm_tiled_kernel(const T* __restrict__ A
 // =====================================================================================
 // float32: every operand as the sum of three bfloat16 numbers, on the bfloat16 matrix unit.
 //
-// x = h + m + l exactly (tw_three_parts; a known method), and a product of two parts is exact in the matrix unit, which adds in float32. Of
+// x = 2^-24 (h + m + l) exactly (tw_three_parts; a known method), and a product of two parts is exact in the matrix unit, which adds in float32. Of
 // the nine products l l alone, below 2^-34 of the whole, is left out; the other eight are added with the smallest first, all but h h into
 // sums of their own, which keeps their roundings away from the large sums. So a product by itself is as good as float32's own
 // (one element of a row not zero: off by 0.995 x 2^-24 at the most and 0.426 in the mean square, by the float32 MFMA 0.994 and 0.426; with m l and
@@ -498,22 +498,22 @@ __global__ __launch_bounds__(256) void gemm_tiled_kernel(const T* __restrict__ A
 //
 // Why: the float32 MFMA takes 64 cycles for 32x32x2, the bfloat16 one 32 for 32x32x16, so eight of these are twice as fast. Workgroup =
 // 4 waves in a 2x2 grid, wave tile (32*WM) x (32*WN): 128x128, 64x128 and 64x64. A k-tile is 32 elements of K; it is split once, on its way
-// from registers to LDS (5.5 vector instructions an element), while the next one is on its way from memory, and two to five workgroups
+// from registers to LDS (6.5 vector instructions an element), while the next one is on its way from memory, and two to five workgroups
 // share a CU, so that one splits while another multiplies. A row of a part is 64 bytes of LDS, four pieces of 16, piece p at
 // p ^ (row / 4 % 4): the 16 rows that a pass of a fragment read takes, and the 8 lanes of a write, are in different banks.
 //
-// Against the float32 MFMA (128x128 tiles, two LDS stages, the K ranges of tiled_splits): 478 x 10,432 x 2,048 271 -> 161 us, 478 x 2,048 x
-// 4,096 108 -> 67, 4,096 x 32,000 x 2,048 4,314 -> 3,375 (159 TFLOP/s, so 1.27 PFLOP/s in bfloat16, where power is the bound), 65 x 896 x 4,864
-// 46 -> 21; 109 random products (65 to 3,000 rows) take 0.52 of the time, the slowest 0.92. (With six products 137, 57, 2,817 and 20;
-// 0.49.) Their error against 64 bits is 0.35 of what it was in the mean and 0.77 at the most. Rows of 4 to 2,048 elements, of 2^-24 of the sum of
+// Against the float32 MFMA (128x128 tiles, two LDS stages, the K ranges of tiled_splits): 478 x 10,432 x 2,048 271 -> 163 us, 478 x 2,048 x
+// 4,096 108 -> 67, 4,096 x 32,000 x 2,048 4,314 -> 3,430 (157 TFLOP/s, so 1.25 PFLOP/s in bfloat16, where power is the bound), 65 x 896 x 4,864
+// 46 -> 22; 109 random products (65 to 3,000 rows) take 0.54 of the time, the slowest 0.92. (With six products 137, 57, 2,817 and 20;
+// 0.49. The factor of 2^24 costs 0 to 4 %.) Their error against 64 bits is 0.35 of what it was in the mean and 0.77 at the most. Rows of 4 to 2,048 elements, of 2^-24 of the sum of
 // sizes, largest and mean square (float32 MFMA / this): dense 2.4 to 4.3 and 0.45 to 0.47 / 1.5 to 2.2 and 0.15 to 0.30, all of one sign 58 and
 // 11.8 / 18 and 4.2, four elements not zero 2.7 and 0.45 / 2.1 and 0.34, the first element 2^14 times the others 103 and 14.6 / 30 and 5.2.
 // What the float32 MFMA does better is a row whose LAST element is 2^14 times the others, 3.0 and 0.42 / 5.0 and 0.95: 16 products meet
 // in one instruction, which lines them all up with the largest.
 //
-// A value that is not finite has no such parts (inf - inf), and every result that it enters is then not finite either. So a tile with such
-// a result is formed again by the float32 MFMA from the operands themselves, and infinities, NaN and sums that overflow are what they are there.
-// (Parts below 2^-126 may be lost: of values below 2^-110.)
+// A value of 2^104 and more, an infinity or NaN has no such parts, and every result that it enters is then not finite (nor is a result of 2^79
+// and more, 2^48 of whose products are summed). So a tile with such a result is formed again by the float32 MFMA from the operands
+// themselves, and infinities, NaN and sums that overflow are what they are there.
 // =====================================================================================
 template <int WM, int WN, bool SHUF, bool GLU>
 __global__ __launch_bounds__(256, WM * WN == 1 ? 5 : 2) void gemm_parts_kernel(const float* __restrict__ A, long lda, const float* __restrict__ W, long ldw,
@@ -695,6 +695,13 @@ __global__ __launch_bounds__(256, WM * WN == 1 ? 5 : 2) void gemm_parts_kernel(c
 #pragma unroll
         for (int j = 0; j < WN; ++j) tw_mma32(acc[i][j], af[i], wf[j]);
     }
+  } else {
+#pragma unroll
+    for (int i = 0; i < WM; ++i)
+#pragma unroll
+      for (int j = 0; j < WN; ++j)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) acc[i][j][e] *= TW_PART_BACK;
   }
 
   if (splits > 1)

@@ -131,16 +131,20 @@ __device__ __forceinline__ void tw_mma32(f32x16& acc, f32x4 a, f32x4 b) {
 }
 
 // ---- float32 as three bfloat16 parts ------------------------------------------------
-// x = h + m + l, as is well known: h is x rounded to bfloat16, m what is left rounded to bfloat16, l what is then left. x - h is a multiple
-// of x's last place and below 2^-8 of x, x - h - m below 2^-17, so that l has six bits and the three parts are x (a finite x above
-// 2^-110). They are rounded to the nearest, so m and l have either sign: parts cut off have x's own, and what is left out of a sum
-// of products then always makes it smaller. Of eight values of a row, for the bfloat16 MFMAs of gemm_parts_kernel and moe_parts_kernel.
+// x * 2^24 = h + m + l, as is well known: h is the left side rounded to bfloat16, m what is left rounded to bfloat16, l what is then left.
+// What h leaves is a multiple of x's last place and below 2^-8 of x, what m leaves below 2^-17, so that l has six bits and the three parts
+// are exact. They are rounded to the nearest, so m and l have either sign: parts cut off have x's own, and what is left out of a sum
+// of products then always makes it smaller. The factor keeps the parts of every x down to the smallest one normal (of an x below 2^-110 l,
+// below 2^-118 m too would be lost without it, and 8 bits of x left); sums of products take TW_PART_BACK. An x of 2^104 and more has no
+// such parts (nor has an infinity or NaN): its h is infinite. Of eight values of a row, for gemm_parts_kernel and moe_parts_kernel.
+#define TW_PART_SCALE 0x1p24f
+#define TW_PART_BACK 0x1p-48f
 __device__ __forceinline__ void tw_three_parts(f32x4 lo, f32x4 hi, bf16x8& h, bf16x8& m, bf16x8& l) {
   u32x4 ph, pm, pl;
   auto two = [](float a, float b) { return __builtin_bit_cast(unsigned, bf16x2{(bf16_t)a, (bf16_t)b}); };
 #pragma unroll
   for (int e = 0; e < 4; ++e) {
-    const float x0 = e < 2 ? lo[2 * e] : hi[2 * e - 4], x1 = e < 2 ? lo[2 * e + 1] : hi[2 * e - 3];
+    const float x0 = TW_PART_SCALE * (e < 2 ? lo[2 * e] : hi[2 * e - 4]), x1 = TW_PART_SCALE * (e < 2 ? lo[2 * e + 1] : hi[2 * e - 3]);
     ph[e] = two(x0, x1);
     const float y0 = x0 - __uint_as_float(ph[e] << 16), y1 = x1 - __uint_as_float(ph[e] & 0xffff0000u);
     pm[e] = two(y0, y1);

@@ -490,6 +490,19 @@ def test_float32_grouped_experts_keep_the_bits_of_a_product(device, kind):
     assert bool(((x.double() - want).abs() <= (3 + 2.0 ** -4) * 2.0 ** -24 * want.abs()).all())
 
 
+def test_float32_grouped_experts_of_small_values(device):
+    """Rows of 2^-119 beside matrices of 2^60, whose squared sums are of 2^-118 again: off by what sums of C products of that size are, twice
+    for the square."""
+    n, X, C, F = 2200, 8, 288, 1600
+    g = torch.Generator().manual_seed(7)
+    h, up = torch.ldexp(torch.randn(n, C, generator=g), torch.tensor(-119)).to(device), torch.ldexp(torch.randn(X, F, C, generator=g), torch.tensor(56)).to(device)
+    x, ex = _experts_that_select(device, "relu_squared", h, up)
+    for e in range(X):
+        rows, m = h[ex == e].double(), up[e, :C].double()
+        z, off = (rows @ m.T).clamp(min=0), (C / 8 + 4) * 2.0 ** -24 * (rows.abs() @ m.abs().T)
+        assert bool(((x[ex == e].double() - z * z).abs() <= (2 * z + off) * off + 2.0 ** -23 * z * z + 2.0 ** -148).all())
+
+
 def test_float32_grouped_experts_of_values_without_parts(device):
     """A token with an infinity and one with a NaN, their experts' other tokens beside them in the same tiles."""
     from tessweave_engine_amd.kernels import ops

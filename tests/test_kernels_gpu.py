@@ -666,6 +666,21 @@ def test_float32_linear_keeps_the_bits_of_a_product(ops, device, k):
                 assert bool(((out.double() - want).abs() <= near).all())
 
 
+@pytest.mark.parametrize("k", [36, 256])
+@pytest.mark.parametrize("x_exp,w_exp", [(-119, 0), (0, -121), (-130, 40), (-60, -60)])
+def test_float32_linear_of_small_values(ops, device, k, x_exp, w_exp):
+    """Values whose last bits lie below the smallest normal number, subnormal ones beside large weights, and products that are nearly
+    subnormal are as exact as others (the bar of test_float32_linear_in_three_parts), down to the smallest number."""
+    m, n = 130, 260
+    x, w = torch.ldexp(rand((m, k), torch.float32, device, 1.0, seed=1), torch.tensor(x_exp)), torch.ldexp(rand((n, k), torch.float32, device, 1.0, seed=2), torch.tensor(w_exp))
+    assert bool((x != 0).all() and (w != 0).all())
+    want, near = x.double() @ w.double().T, (k / 8 + 4) * 2.0 ** -24 * (x.double().abs() @ w.double().abs().T) + 2.0 ** -149
+    for weight in (w, ops.shuffle_weight(w)):
+        out = torch.full((m, n), float("nan"), device=device)
+        ops.linear(x, weight, out)
+        assert bool(((out.double() - want).abs() <= near).all())
+
+
 @pytest.mark.parametrize("shuffled", [False, True])
 def test_float32_linear_of_values_without_parts(ops, device, shuffled):
     """Infinities, NaN (also one whose upper half is an infinity's) and sums that overflow come out as they do of float32 products,
