@@ -568,8 +568,8 @@ __global__ __launch_bounds__(WAVES * 64) void moe_grouped_kernel(const T* __rest
 // float32, steps of many rows: the same products from three bfloat16 parts an operand (gemm_parts_kernel says why and how exact). One
 // workgroup: a unit's 64 rows against 64 * WN rows of its expert's matrices (GLU: half of gate, half of up, of the same columns), waves in
 // a 2x2 grid, wave tile 32 x (32 * WN). A k-tile is two k-steps; rows and matrices are read in fragment order, split and laid into LDS, two
-// k-tiles are on their way (the matrices come from HBM) and three workgroups share a CU. What is not finite is formed again from the
-// operands themselves. All launches of the experts, us, the float32 MFMA / this: 16 experts of 2,048 x 1,408, two a token, gated, 128 tokens
+// k-tiles are on their way (the matrices come from HBM) and three workgroups share a CU. What is not finite, and nothing beside it, is
+// formed again from the operands themselves. All launches of the experts, us, the float32 MFMA / this: 16 experts of 2,048 x 1,408, two a token, gated, 128 tokens
 // 303 / 198, 478 423 / 266, 2,000 956 / 673; 8 of 4,096 x 2,048, 300 tokens 751 / 497; 64 of 1,024 x 512, four a token, 300 tokens 274 / 154.
 // (With six products and one k-tile on its way the first took 181 us against 163; at two workgroups a CU 179, and 478 tokens 257 against 221.)
 template <int ACT, int WN>
@@ -676,7 +676,7 @@ __global__ __launch_bounds__(256, WN == 2 ? 3 : 4) void moe_parts_kernel(const f
 #pragma unroll
     for (int j = 0; j < WN; ++j)
 #pragma unroll
-      for (int e = 0; e < 16; ++e) acc[j][e] = 0.f;
+      for (int e = 0; e < 16; ++e) small[j][e] = 0.f;
     const int in_block = g * 64 + (r & 15) * 4;
     const float* a = A + (size_t)(tile + (wm0 + r) / 16) * tile_elems + in_block;
     const float* w[WN];
@@ -684,7 +684,11 @@ __global__ __launch_bounds__(256, WN == 2 ? 3 : 4) void moe_parts_kernel(const f
     for (int j = 0; j < WN; ++j) w[j] = block_of(wave_row(j) + r) + in_block;
     for (int k = 0; k < K; k += 8)                             // (8 elements of K are 128 floats of a block)
 #pragma unroll
-      for (int j = 0; j < WN; ++j) tw_mma32(acc[j], tw_load_frag(a + (size_t)k * 16), tw_load_frag(w[j] + (size_t)k * 16));
+      for (int j = 0; j < WN; ++j) tw_mma32(small[j], tw_load_frag(a + (size_t)k * 16), tw_load_frag(w[j] + (size_t)k * 16));
+#pragma unroll
+    for (int j = 0; j < WN; ++j)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) acc[j][e] = acc[j][e] * 0.f == 0.f ? acc[j][e] * TW_PART_BACK : small[j][e];
   } else {
 #pragma unroll
     for (int j = 0; j < WN; ++j)

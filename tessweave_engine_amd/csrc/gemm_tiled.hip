@@ -513,7 +513,8 @@ __global__ __launch_bounds__(256) void gemm_tiled_kernel(const T* __restrict__ A
 //
 // A value of 2^104 and more, an infinity or NaN has no such parts, and every result that it enters is then not finite (nor is a result of 2^79
 // and more, 2^48 of whose products are summed). So a tile with such a result is formed again by the float32 MFMA from the operands
-// themselves, and infinities, NaN and sums that overflow are what they are there.
+// themselves, and infinities, NaN and sums that overflow are what they are there. The tile's other results stay the parts' sums: a row's
+// bits do not depend on what its neighbours hold.
 // =====================================================================================
 template <int WM, int WN, bool SHUF, bool GLU>
 __global__ __launch_bounds__(256, WM * WN == 1 ? 5 : 2) void gemm_parts_kernel(const float* __restrict__ A, long lda, const float* __restrict__ W, long ldw,
@@ -677,7 +678,7 @@ __global__ __launch_bounds__(256, WM * WN == 1 ? 5 : 2) void gemm_parts_kernel(c
 #pragma unroll
       for (int j = 0; j < WN; ++j)
 #pragma unroll
-        for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
+        for (int e = 0; e < 16; ++e) small[i][j][e] = 0.f;
     const int k_from = kt0 * BK, k_to = min(K, k_end * BK);
     for (int k = k_from; k < k_to; k += 8) {
       f32x4 af[WM], wf[WN];
@@ -693,8 +694,14 @@ __global__ __launch_bounds__(256, WM * WN == 1 ? 5 : 2) void gemm_parts_kernel(c
 #pragma unroll
       for (int i = 0; i < WM; ++i)
 #pragma unroll
-        for (int j = 0; j < WN; ++j) tw_mma32(acc[i][j], af[i], wf[j]);
+        for (int j = 0; j < WN; ++j) tw_mma32(small[i][j], af[i], wf[j]);
     }
+#pragma unroll
+    for (int i = 0; i < WM; ++i)
+#pragma unroll
+      for (int j = 0; j < WN; ++j)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) acc[i][j][e] = acc[i][j][e] * 0.f == 0.f ? acc[i][j][e] * TW_PART_BACK : small[i][j][e];
   } else {
 #pragma unroll
     for (int i = 0; i < WM; ++i)

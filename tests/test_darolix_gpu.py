@@ -473,16 +473,19 @@ def _experts_that_select(device, kind, h, first, up=None):
     return x, ids[:, 0].long()
 
 
+@pytest.mark.parametrize("exp", [0, 110])
 @pytest.mark.parametrize("kind", ["silu", "relu_squared"])
-def test_float32_grouped_experts_keep_the_bits_of_a_product(device, kind):
+def test_float32_grouped_experts_keep_the_bits_of_a_product(device, kind, exp):
     """Rows of one element that is not zero: a product is rounded once (and by less than 2^-6 of that in its smaller parts' sums), the
-    product of the two, or the square, once more, and the other matrix passes it on. The gate's results are past 40, where silu(z) is z."""
+    product of the two, or the square, once more, and the other matrix passes it on. The gate's results are past 40, where silu(z) is z.
+    Also of rows too large for parts beside small matrices."""
     n, X, C, F = 2200, 8, 288, 1600
     g = torch.Generator().manual_seed(6)
     col, value = torch.arange(n) * 7 % C, torch.rand(n, generator=g) + 0.5
     h = torch.zeros(n, C)
     h[torch.arange(n), col] = value
     first, up = 100 * torch.rand(X, F, C, generator=g) + 100, torch.randn(X, F, C, generator=g)
+    h, value, first, up = h * 2.0 ** exp, value * 2.0 ** exp, first * 2.0 ** -exp, up * 2.0 ** -exp
     h, first, up, col, value = (t.to(device) for t in (h, first, up, col, value))
     x, ex = _experts_that_select(device, kind, h, *((first, up) if kind == "silu" else (up,)))
     u = up.double()[ex, :C, col] * value.double()[:, None]
@@ -503,11 +506,38 @@ def test_float32_grouped_experts_of_small_values(device):
         assert bool(((x[ex == e].double() - z * z).abs() <= (2 * z + off) * off + 2.0 ** -23 * z * z + 2.0 ** -148).all())
 
 
-def test_float32_grouped_experts_of_values_without_parts(device):
-    """A token with an infinity and one with a NaN, their experts' other tokens beside them in the same tiles."""
+@pytest.mark.parametrize("kind", ["silu", "relu_squared"])
+def test_float32_grouped_experts_rows_do_not_depend_on_their_neighbours(device, kind):
+    """A token with an infinity, one with a NaN, one whose sums overflow and a weight that is infinite leave the bits of the other rows of
+    their tiles, and of the other columns, as they are. (43 units, tiles of 128 columns in front and of 64 behind.)"""
+    from tessweave_engine_amd.kernels import ops
+    n, X, C, F = 2200, 8, 288, 1600
+    g = torch.Generator().manual_seed(8)
+    h = torch.randn(n, C, generator=g).to(device)
+    first, up = (torch.randn(X, F, C, generator=g).to(device) / 16 for _ in range(2))
+    down = torch.randn(X, C, F, generator=g).to(device) / 40
+    ids = (torch.arange(n, device=device) * 5 % X).to(torch.int32)[:, None].contiguous()
+    results = []
+    for odd in (False, True):
+        if odd:
+            h[17, 3], h[300, 255], h[41, 9], down[2, 100, 7] = float("inf"), float("nan"), 3e38, float("inf")
+        x = torch.zeros(n, C, device=device)
+        ops.moe_experts(h, ids, torch.ones(n, 1, device=device), ops.moe_blocked(first) if kind == "silu" else None, ops.moe_blocked(up),
+                        ops.moe_blocked(down), 0.0, x, lambda tag, shape, kind_: torch.empty(shape, dtype=kind_, device=device), kind=kind)
+        results.append(x)
+    same = torch.ones(n, C, dtype=torch.bool, device=device)
+    same[[17, 41, 300]] = False
+    same[ids[:, 0] == 2, 100] = False
+    assert bool((results[0] == results[1])[same].all()) and bool(results[0].isfinite().all())
+    assert not bool(results[1][17].isfinite().any())           # (relu drops a NaN)
+
+
+@pytest.mark.parametrize("n,X,C,F", [(400, 4, 256, 512), (2200, 8, 288, 1600)])
+def test_float32_grouped_experts_of_values_without_parts(device, n, X, C, F):
+    """A token with an infinity and one with a NaN, their experts' other tokens beside them in the same tiles: steps of 44 tiles (few rows)
+    and of 43 units (parts)."""
     from tessweave_engine_amd.kernels import ops
     g = torch.Generator().manual_seed(5)
-    n, X, C, F = 400, 4, 256, 512
     h = torch.randn(n, C, generator=g).to(device)
     gate, up = (torch.randn(X, F, C, generator=g).to(device) / 16 for _ in range(2))
     down = torch.randn(X, C, F, generator=g).to(device) / 16
@@ -522,7 +552,7 @@ def test_float32_grouped_experts_of_values_without_parts(device):
         results.append(x)
     rows = torch.tensor([i for i in range(n) if i not in (17, 300)], device=device)
     assert not bool(results[1][[17, 300]].isfinite().any())
-    # (float32 sums of 256 and 512 products of terms of size 1 over the square root of their number, by either way)
+    # (float32 sums of 256 to 1,600 products of terms of size 1 over the square root of their number, by either way)
     assert torch.allclose(results[0][rows], results[1][rows], atol=1e-5, rtol=1e-5)
 
 

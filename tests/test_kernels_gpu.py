@@ -682,6 +682,26 @@ def test_float32_linear_of_small_values(ops, device, k, x_exp, w_exp):
 
 
 @pytest.mark.parametrize("shuffled", [False, True])
+@pytest.mark.parametrize("m,n,k", [(130, 260, 72), (300, 64, 2048)])
+def test_float32_linear_rows_do_not_depend_on_their_neighbours(ops, device, shuffled, m, n, k):
+    """A row with an infinity or a NaN, and a column of such weights, leave the bits of the other rows and columns of their tiles as they are."""
+    x, w = rand((m, k), torch.float32, device, 1.0, seed=1), rand((n, k), torch.float32, device, 0.05, seed=2)
+    space = torch.empty(ops.linear_workspace_bytes(torch.float32, m, n, k) // 4 + 4, device=device)
+    results = []
+    for odd in (False, True):
+        if odd:
+            x[3, 5], x[70, 71], w[33, 40], x[100, 9] = float("inf"), float("nan"), float("inf"), 2.0 ** 120
+        out = torch.full((m, n), 7.0, device=device)
+        ops.linear(x, ops.shuffle_weight(w) if shuffled else w, out, workspace=space)
+        results.append(out)
+    rows, cols = (torch.tensor([i for i in range(size) if i not in odd], device=device) for size, odd in ((m, (3, 70, 100)), (n, (33,))))
+    assert bool((results[0][rows][:, cols] == results[1][rows][:, cols]).all())
+    assert not bool(results[1][[3, 70]].isfinite().any()) and not bool(results[1][:, 33].isfinite().any())
+    want, size = x[100].double() @ w[cols].double().T, x[100].double().abs() @ w[cols].double().abs().T
+    assert bool(((results[1][100, cols].double() - want).abs() <= (k + 4) * 2.0 ** -24 * size).all())
+
+
+@pytest.mark.parametrize("shuffled", [False, True])
 def test_float32_linear_of_values_without_parts(ops, device, shuffled):
     """Infinities, NaN (also one whose upper half is an infinity's) and sums that overflow come out as they do of float32 products,
     and what is beside them in their tiles is off by no more than a float32 sum of K products is."""
