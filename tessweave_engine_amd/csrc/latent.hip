@@ -378,22 +378,27 @@ template <typename T> struct LtQuad;
 template <> struct LtQuad<float> { typedef f32x4 Type; };
 template <> struct LtQuad<bf16_t> { typedef bf16x4 Type; };
 
-// EXACT: key rows of KS and latents of LS elements, pages of a power of two and at least 16: sizes are compile-time constants
-// and a key tile's page and addresses the whole wave's (scalar).
-template <typename T, int KS = 256, int LS = 240, bool EXACT = false>
-__global__ __launch_bounds__(256) void latent_decode_kernel(LatentDecodeArgs a) {
+// TILES > 0: latents of 16 TILES elements, key rows of up to 64 more (WHOLE: of 64 more), pages of a power of two and at least 16: loops
+// have no branches, and a key tile's page and addresses are the whole wave's (scalar). 0: sizes known at run time. With what
+// follows in latent_leave_kernel, in a chain of such calls (us, 0 / TILES; bfloat16, then float32): latents of 64 with 32 rotated, 8 requests
+// of 190 keys 10.3 / 8.6, 12.2 / 10.9, 64 of 2,000 19.0 / 16.2, 36.2 / 26.5; 128 with 64 11.5 / 9.9, 14.9 / 13.5 and 29.4 / 25.5, 59.7 / 43.9; 192 with 64 12.5 / 11.0, 18.3 / 17.1 and 37.8 / 35.2, 79.9 / 59.9;
+// 224 with 32 12.7 / 11.2, 20.0 / 19.6 and 39.7 / 36.5, 83.0 / 80.7.
+template <typename T, int TILES, bool WHOLE = false>
+__global__ __launch_bounds__(256, TILES ? 2 : 1) void latent_decode_kernel(LatentDecodeArgs a) {
   typedef typename Elem<T>::Frag Frag;
   typedef typename LtQuad<T>::Type Quad;
   constexpr int EPF = Elem<T>::kPerFrag;
   constexpr int STEP = 4 * EPF;                 // key elements one product consumes
-  constexpr int KC_MAX = KS / STEP;
-  constexpr int LT_MAX = LS / 16;
+  constexpr bool SIZED = TILES > 0;
+  constexpr int KC_MAX = ((SIZED && 16 * TILES + 64 < 256 ? 16 * TILES + 64 : 256) + STEP - 1) / STEP;
+  constexpr int KC_SURE = WHOLE ? KC_MAX : SIZED ? 16 * TILES / STEP : 0;       // products whose elements are all there, whatever K is
+  constexpr int LT_MAX = SIZED ? TILES : 15;    // Lp <= 240
   extern __shared__ float ld_lds[];
   const int s = blockIdx.x, split = blockIdx.y, ht = blockIdx.z;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int r = lane & 15, g = lane >> 4;
-  const int K = EXACT ? KS : a.K, Lp = EXACT ? LS : a.Lp, P = a.P;
-  const int KC = EXACT ? KC_MAX : (K + STEP - 1) / STEP, LT = EXACT ? LT_MAX : Lp / 16;
+  const int K = WHOLE ? 16 * TILES + 64 : a.K, Lp = SIZED ? 16 * TILES : a.Lp, P = a.P;
+  const int KC = SIZED ? KC_MAX : (K + STEP - 1) / STEP, LT = SIZED ? LT_MAX : Lp / 16;
   const int len = a.kv_len[s];
   const int row = a.q_start[s];
   const int head = ht * 16 + r;
@@ -418,35 +423,33 @@ __global__ __launch_bounds__(256) void latent_decode_kernel(LatentDecodeArgs a) 
   // What bounds it is the trips to memory in a row: a decode step's wave has one tile or two. Everything a tile reads is
   // requested together (with `col < K ? load : zero` in front of every product each of a tile's eight key loads waited for the
   // one before) and, in bfloat16, the next tile's while this one is worked on: its keys behind the scores, its values behind the
-  // products that free their registers, its page numbers a tile earlier still (float32 fragments are twice as many registers:
-  // ahead they would halve the waves). 8 requests of 150
+  // products that free their registers, its page numbers a tile earlier still (float32 with sizes known at run time: the most
+  // registers that they can need, twice as many, would halve the waves). 8 requests of 150
   // tokens 17.7 -> 12.3 us, one of 2,048 22.6 -> 12.7 (kernel traces).
   // A key past the end is the last one again; masked below.
-  constexpr bool AHEAD = EPF == 8 || EXACT;
+  constexpr bool AHEAD = EPF == 8 || SIZED;
   auto key_of = [&](int t) { return min(t * 16 + r, len - 1); };
   auto value_of = [&](int t) { return min(t * 16 + 4 * g, (len - 1) / 4 * 4); };      // 4 keys: one page (multiples of 4)
   Frag kf[KC_MAX];
   Quad vq[LT_MAX];
-  // (EXACT: places behind the sequence's end in its last page hold anything: masked like them all)
-  auto page_of = [&](int t, int key) { return EXACT ? max(0, table[(t * 16) >> a.page_shift]) : table[key / P]; };
+  // (SIZED: places behind the sequence's end in its last page hold anything: masked like them all)
+  auto page_of = [&](int t, int key) { return SIZED ? max(0, table[(t * 16) >> a.page_shift]) : table[key / P]; };
   auto key_row = [&](int t, int page) {
-    if constexpr (EXACT) return keys + ((uint64_t)(uint32_t)page * (uint32_t)(P * KS) + (uint32_t)(((t * 16) & (P - 1)) * KS)) + r * KS;
+    if constexpr (SIZED) return keys + ((uint64_t)(uint32_t)page * (uint32_t)(P * K) + (uint32_t)(((t * 16) & (P - 1)) * K)) + r * K;
     else return keys + ((size_t)page * P + key_of(t) % P) * K;
   };
   auto request_keys = [&](int t, int page) {
     const T* krow = key_row(t, page);
-    if constexpr (EXACT) {
-#pragma unroll
-      for (int kc = 0; kc < KC_MAX; ++kc) kf[kc] = tw_load_frag(krow + kc * STEP + g * EPF);
-      return;
-    }
 #pragma unroll
     for (int kc = 0; kc < KC_MAX; ++kc)
-      if (kc < KC) kf[kc] = tw_load_frag(krow + min(kc * STEP + g * EPF, K - EPF));   // (past the row: a copy)
+      if (kc < KC) {                              // (past the row: a copy)
+        const int col = kc * STEP + g * EPF;
+        kf[kc] = tw_load_frag(krow + (kc < KC_SURE ? col : min(col, K - EPF)));
+      }
   };
   auto request_values = [&](int t, int page) {
-    if constexpr (EXACT) {
-      const T* base = values + ((uint64_t)(uint32_t)page * (uint32_t)(P * LS) + (uint32_t)((t * 16) & (P - 1)));
+    if constexpr (SIZED) {
+      const T* base = values + ((uint64_t)(uint32_t)page * (uint32_t)(P * Lp) + (uint32_t)((t * 16) & (P - 1)));
 #pragma unroll
       for (int lt = 0; lt < LT_MAX; ++lt)
         vq[lt] = *reinterpret_cast<const Quad*>(base + (uint32_t)(lt * 16 * P) + (uint32_t)(r * P + 4 * g));
@@ -481,7 +484,7 @@ __global__ __launch_bounds__(256) void latent_decode_kernel(LatentDecodeArgs a) 
       if (kc < KC) {
         const int col = kc * STEP + g * EPF;
         if constexpr (AHEAD) {
-          if (K % STEP != 0 && col >= K) kf[kc] = Elem<T>::zero();
+          if (kc >= KC_SURE && (SIZED || K % STEP != 0) && col >= K) kf[kc] = Elem<T>::zero();
           tw_mma16(S, kf[kc], qf[kc]);            // S[j]: key t * 16 + 4 g + j against head r
         } else {
           const Frag one = col < K ? tw_load_frag(krow + col) : Elem<T>::zero();
@@ -799,10 +802,21 @@ extern "C" int tw_latent_decode(int dtype, const void* q, long ldq, const void* 
   const int head_tiles = tw_div_up(heads, 16);
   const dim3 grid(n_seqs, splits, head_tiles);
   const size_t lds = ((size_t)4 * 16 * (Lp + 4) + 128) * sizeof(float);
+  // (latents of whole 32s from 64 on have an instance each; pages that are no power of two, or rotated parts of more than 64, have none)
+  const int sized = pow2 && page_size >= 16 && K <= Lp + 64 && Lp >= 64 && Lp % 32 == 0 ? Lp / 16 : 0;
+  const bool whole = K == Lp + 64;
 #define TW_LATENT_DECODE(T)                                                                                                     \
   do {                                                                                                                         \
-    if (K == 256 && Lp == 192 && pow2 && page_size >= 16) latent_decode_kernel<T, 256, 192, true><<<grid, 256, lds, stream>>>(a); \
-    else latent_decode_kernel<T><<<grid, 256, lds, stream>>>(a);                                                                 \
+    auto attend = [&](auto kernel) { kernel<<<grid, 256, lds, stream>>>(a); };                                                  \
+    switch (sized) {                                                                                                           \
+      case 4: whole ? attend(latent_decode_kernel<T, 4, true>) : attend(latent_decode_kernel<T, 4>); break;                    \
+      case 6: whole ? attend(latent_decode_kernel<T, 6, true>) : attend(latent_decode_kernel<T, 6>); break;                    \
+      case 8: whole ? attend(latent_decode_kernel<T, 8, true>) : attend(latent_decode_kernel<T, 8>); break;                    \
+      case 10: whole ? attend(latent_decode_kernel<T, 10, true>) : attend(latent_decode_kernel<T, 10>); break;                 \
+      case 12: whole ? attend(latent_decode_kernel<T, 12, true>) : attend(latent_decode_kernel<T, 12>); break;                 \
+      case 14: attend(latent_decode_kernel<T, 14>); break;                                                                     \
+      default: attend(latent_decode_kernel<T, 0>);                                                                             \
+    }                                                                                                                          \
     if (expand) {                                                                                                              \
       const size_t leave = (16 * 64 + 16) * 4 + 512 * 16 + (size_t)16 * (Lp + 32 / sizeof(T)) * sizeof(T);                       \
       latent_leave_kernel<T><<<dim3(heads, tw_div_up(n_seqs, 16)), 512, leave, stream>>>(a, b);                                  \

@@ -204,7 +204,16 @@ def test_one_token_attention_over_the_cached_latent(device, dtype, H, L, R, page
 
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 @pytest.mark.parametrize("H,L,R,D,E,page,lengths,splits,gated", [
-    (16, 192, 64, 64, 128, 16, [1, 16, 17, 64, 65, 200], 0, True),        # the sizes with compile-time loops; tile and group edges
+    (16, 192, 64, 64, 128, 16, [1, 16, 17, 64, 65, 200], 0, True),        # sizes with compile-time loops; tile and group edges
+    (4, 64, 16, 16, 32, 16, [1, 15, 33, 129], 2, True),                   # every other one of them: the smallest; a last k-step that ends inside
+    (4, 96, 48, 16, 32, 64, [90, 7], 1, False),                           # itself; pages of several tiles;
+    (4, 128, 64, 16, 32, 16, [260, 31], 3, True),
+    (4, 160, 32, 16, 32, 32, [17, 48], 1, False),
+    (4, 64, 64, 16, 32, 16, [33], 1, False),
+    (4, 96, 64, 16, 32, 16, [50, 64], 2, False),
+    (4, 160, 64, 16, 32, 16, [18], 1, True),
+    (4, 224, 32, 16, 32, 16, [100, 1], 2, True),                          # the most registers
+    (4, 64, 80, 16, 32, 16, [40], 1, False),                              # rotated parts that they do not hold
     (17, 192, 64, 64, 144, 32, [300], 64, False),                         # one row, most ranges, a second tile of heads
     (3, 192, 64, 8, 16, 16, list(range(1, 18)), 2, True),                 # a second tile of rows; threads with several elements each
     (5, 48, 16, 24, 20, 4, [40, 7], 3, True),                             # the last k-step ends inside itself, columns inside a tile
