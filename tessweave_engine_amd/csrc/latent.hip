@@ -149,12 +149,6 @@ __device__ __forceinline__ void head_linear_unit(const HeadLinear<T>& a, int uni
   }
 }
 
-template <typename T>
-__global__ __launch_bounds__(256) void head_linear_kernel(HeadLinear<T> a) {
-  const int unit = blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (unit < a.units()) head_linear_unit(a, unit, blockIdx.y);
-}
-
 // Workgroups 0 .. n - 1 finish a token each; those behind them form the query side's products W_uk,a^T q_plain,a of the first
 // absorb.n rows, which read and write nothing the others write: one launch instead of two.
 template <typename T>
@@ -203,6 +197,7 @@ extern "C" int tw_latent_finish(int dtype, const void* proj, long ld, int q_col,
   return TW_LAUNCH_RESULT();
 }
 
+// (the products alone: no token is finished)
 extern "C" int tw_head_linear(int dtype, const void* x, long ldx, int sx, const void* w, void* out, long ldo, int so,
                               int n, int heads, int Ni, int No, hipStream_t stream) {
   const int epf = dtype == TW_DTYPE_BF16 ? 8 : 4;
@@ -215,7 +210,7 @@ extern "C" int tw_head_linear(int dtype, const void* x, long ldx, int sx, const 
 #define TW_HEAD_LINEAR(T)                                                                                                      \
   do {                                                                                                                         \
     const HeadLinear<T> hl{(const T*)x, ldx, sx, (const T*)w, (T*)out, ldo, so, n, heads, Ni, No};                              \
-    head_linear_kernel<T><<<dim3(tw_div_up(hl.units(), 4), tw_div_up(n, 16)), 256, 0, stream>>>(hl);                            \
+    latent_finish_kernel<T><<<tw_div_up((long)hl.units() * tw_div_up(n, 16), 4), 256, 0, stream>>>(LatentFinishArgs{}, hl, 0);    \
   } while (0)
   if (dtype == TW_DTYPE_BF16) TW_HEAD_LINEAR(bf16_t);
   else TW_HEAD_LINEAR(float);
@@ -353,7 +348,7 @@ extern "C" int tw_latent_expand_store(int dtype, const void* up, long ld_up, con
 // layout the next one, O^T += V^T P^T, wants as its operand, and a key row is read once for 16 heads. Values are the
 // first Lp elements of the key rows, kept a second time transposed inside a page ([Lp][P]) so that four consecutive
 // keys of one element are one 8-byte load. A sequence's keys are cut into `splits` ranges for separate workgroups,
-// whose waves take the range's tiles in turn; waves are combined through LDS, ranges by a second kernel in index order.
+// whose waves take the range's tiles in turn; waves are combined through LDS, ranges by latent_leave_kernel.
 //
 //   part [seq][head tile][split][16][Lp + 4]: output sums relative to the range's maximum, that maximum, the sum
 struct LatentDecodeArgs {
@@ -361,11 +356,9 @@ struct LatentDecodeArgs {
   const void* keys; const void* values;
   const int* block_table; int table_stride;
   const int* q_start; const int* kv_len;
-  void* out; long ldo;                // head a at out + row(s) * ldo + a * Lp
   float* part;
   float scale;
   int H, K, Lp, P, splits;
-  int to_part;                        // ranges' results stay in part (also that of a single range)
   int page_shift;                     // log2(P) if P is a power of two, else -1
   const float* sink;                  // [H] or null: exp(sink_a) more in head a's denominator (no key, no value, not scaled)
 };
@@ -571,63 +564,17 @@ __global__ __launch_bounds__(256, TILES ? 2 : 1) void latent_decode_kernel(Laten
       for (int e = 0; e < 4; ++e) o[e] += f * v[e];
       total += f * sw[w * 16 + hh];
     }
-    if (!a.to_part) {
-      float scale = 1.f;
-      if (a.sink) {
-        const float sk = a.sink[ht * 16 + hh];
-        const float both = fmaxf(top, sk);
-        const float f = top == -INFINITY ? 0.f : lt_exp<T>(top - both);
-        scale = f;
-        total = total * f + lt_exp<T>(sk - both);
-      }
-      T* dst = (T*)a.out + (size_t)row * a.ldo + (size_t)(ht * 16 + hh) * Lp + l;
-#pragma unroll
-      for (int e = 0; e < 4; ++e) dst[e] = tw_from_float<T>(o[e] * scale / total);
-    } else {
-      float* dst = a.part + ((((size_t)s * gridDim.z + ht) * a.splits + split) * 16 + hh) * (Lp + 4);
-      *reinterpret_cast<f32x4*>(dst + l) = o;
-      if (l == 0) {
-        dst[Lp] = top;
-        dst[Lp + 1] = total;
-      }
+    float* dst = a.part + ((((size_t)s * gridDim.z + ht) * a.splits + split) * 16 + hh) * (Lp + 4);
+    *reinterpret_cast<f32x4*>(dst + l) = o;
+    if (l == 0) {
+      dst[Lp] = top;
+      dst[Lp + 1] = total;
     }
   }
 }
 
-// One workgroup a (sequence, head): the ranges' maxima and sums first (one thread a range), then a thread an element.
-template <typename T>
-__global__ __launch_bounds__(256) void latent_decode_merge_kernel(LatentDecodeArgs a) {
-  __shared__ float weight[64];
-  __shared__ float total_s;
-  const int s = blockIdx.x, head = blockIdx.y;
-  const int ht = head >> 4, hh = head & 15;
-  const int Lp = a.Lp;
-  const int row = a.q_start[s];
-  const int head_tiles = (a.H + 15) / 16;
-  const float* base = a.part + ((((size_t)s * head_tiles + ht) * a.splits) * 16 + hh) * (Lp + 4);
-  const size_t stride = (size_t)16 * (Lp + 4);                  // from one range to the next
-  if (threadIdx.x < 64) {
-    const int sp = threadIdx.x;
-    const float m = sp < a.splits ? base[sp * stride + Lp] : -INFINITY;
-    float top = tw_wave_max(m);
-    const float sk = a.sink ? a.sink[head] : -INFINITY;
-    top = fmaxf(top, sk);
-    const float f = m == -INFINITY ? 0.f : lt_exp<T>(m - top);
-    weight[sp] = f;
-    const float total = tw_wave_sum(sp < a.splits ? f * base[sp * stride + Lp + 1] : 0.f);
-    if (sp == 0) total_s = total + (a.sink ? lt_exp<T>(sk - top) : 0.f);
-  }
-  __syncthreads();
-  const float inv = 1.f / total_s;
-  for (int l = threadIdx.x; l < Lp; l += 256) {
-    float o = 0.f;
-    for (int sp = 0; sp < a.splits; ++sp) o += weight[sp] * base[sp * stride + l];
-    ((T*)a.out)[(size_t)row * a.ldo + (size_t)head * Lp + l] = tw_from_float<T>(o * inv);
-  }
-}
-
-// The same with what follows it in a layer: the ranges' results of 16 rows of one head are added up, rounded to the compute type and
-// multiplied with the head's W_uv ([No][Lp]); gate (or null): the result times sigmoid(gate). One workgroup a (head, 16 rows). Its
+// What follows it in a layer: the ranges' results of 16 rows of one head are added up, rounded to the compute type and multiplied
+// with the head's W_uv ([No][Lp]; null: they go out as they are); gate (or null): the result times sigmoid(gate). One workgroup a (head, 16 rows). Its
 // waves' fragments of W_uv are requested first and the ranges' sums before their weights are known, so that three trips to memory
 // lie in a row; with few rows several threads share a row's element and take every P-th range each. From the projections to the
 // gated heads, 16 heads, latents of 192, in a chain of such calls (us; five or six launches, 64-column products, run-time sizes and
@@ -635,7 +582,7 @@ __global__ __launch_bounds__(256) void latent_decode_merge_kernel(LatentDecodeAr
 // 64 of 500 36.0 / 25.2; 24 heads, 64 of 4,000 88.2 / 80.2. The results are off by 0.8 times as much against 64 bits (the gate
 // multiplies the float32 product).
 struct LatentLeave {
-  const void* w;                      // [H][No][Lp]
+  const void* w;                      // [H][No][Lp] or null
   void* out; long ldo; int so;        // head a's results at out + row(s) * ldo + a * so
   const void* gate; long ldg;         // or null: head a's gate at gate + row(s) * ldg + a * so
   int No, n;
@@ -666,7 +613,7 @@ __global__ __launch_bounds__(512) void latent_leave_kernel(LatentDecodeArgs a, L
     for (int u = 0; u < U; ++u) f[u] = tw_load_frag(w_row + min((st0 + u) * 4 + g, chunks - 1) * EPF);
   };
   Frag wf[U];
-  if (wave * 16 < b.No) load_w(wave * 16, 0, wf);
+  if (b.w && wave * 16 < b.No) load_w(wave * 16, 0, wf);
   const int items = n * quads;
   const int P = items >= 512 ? 1 : min(S, 512 / items);      // threads that share an element
   const int item = P == 1 ? threadIdx.x : threadIdx.x % items, p = P == 1 ? 0 : threadIdx.x / items;
@@ -693,7 +640,7 @@ __global__ __launch_bounds__(512) void latent_leave_kernel(LatentDecodeArgs a, L
   // ---- the rows, in index order of the ranges within a thread ----------------------------------------------------------------
   auto finish = [&](int i, f32x4 o) {
     const int row = i / quads;
-    T* dst = xs + row * xrow + i % quads * 4;
+    T* dst = b.w ? xs + row * xrow + i % quads * 4 : (T*)b.out + (size_t)a.q_start[s0 + row] * b.ldo + (size_t)head * b.so + i % quads * 4;
 #pragma unroll
     for (int e = 0; e < 4; ++e) dst[e] = tw_from_float<T>(o[e] * inv[row]);
   };
@@ -735,6 +682,7 @@ __global__ __launch_bounds__(512) void latent_leave_kernel(LatentDecodeArgs a, L
     }
     __syncthreads();
   }
+  if (!b.w) return;
   // ---- times W_uv: D[output 4g + e][row r] --------------------------------------------------------------------------------------
   const int at_row = a.q_start[s0 + min(r, n - 1)];
   for (int col = wave * 16; col < b.No; col += 128) {
@@ -787,8 +735,7 @@ extern "C" int tw_latent_decode(int dtype, const void* q, long ldq, const void* 
   TW_REQUIRE(ldq >= (long)heads * K && (expand || ldo >= (long)heads * Lp));
   const int esize = dtype == TW_DTYPE_BF16 ? 2 : 4;
   TW_REQUIRE((uintptr_t)q % 16 == 0 && (uintptr_t)keys % 16 == 0 && (uintptr_t)values % 16 == 0 && (ldq * esize) % 16 == 0);
-  if (splits > 1 || expand)
-    TW_REQUIRE(workspace && (uintptr_t)workspace % 16 == 0 && workspace_floats >= tw_latent_decode_workspace_floats(n_seqs, heads, Lp, splits));
+  TW_REQUIRE(n_seqs == 0 || (workspace && (uintptr_t)workspace % 16 == 0 && workspace_floats >= tw_latent_decode_workspace_floats(n_seqs, heads, Lp, splits)));
   if (expand) {            // [heads][expand_out][Lp]: out takes the heads' results times their matrices, times sigmoid(gate)
     TW_REQUIRE((uintptr_t)expand % 16 == 0 && expand_out > 0 && expand_out % 4 == 0 && out_stride >= expand_out);
     TW_REQUIRE(ldo >= (long)(heads - 1) * out_stride + expand_out && (!gate || ldg >= (long)(heads - 1) * out_stride + expand_out));
@@ -796,9 +743,9 @@ extern "C" int tw_latent_decode(int dtype, const void* q, long ldq, const void* 
   TW_REQUIRE(expand || !gate);
   if (n_seqs == 0) return 0;
   const bool pow2 = (page_size & (page_size - 1)) == 0;
-  LatentDecodeArgs a{q, ldq, keys, values, block_table, table_stride, q_start, kv_len, out, ldo, workspace, scale,
-                     heads, K, Lp, page_size, splits, splits > 1 || expand, pow2 ? __builtin_ctz(page_size) : -1, sink};
-  const LatentLeave b{expand, out, ldo, out_stride, gate, ldg, expand_out, n_seqs};
+  LatentDecodeArgs a{q, ldq, keys, values, block_table, table_stride, q_start, kv_len, workspace, scale,
+                     heads, K, Lp, page_size, splits, pow2 ? __builtin_ctz(page_size) : -1, sink};
+  const LatentLeave b{expand, out, ldo, expand ? out_stride : Lp, gate, ldg, expand_out, n_seqs};
   const int head_tiles = tw_div_up(heads, 16);
   const dim3 grid(n_seqs, splits, head_tiles);
   const size_t lds = ((size_t)4 * 16 * (Lp + 4) + 128) * sizeof(float);
@@ -817,12 +764,8 @@ extern "C" int tw_latent_decode(int dtype, const void* q, long ldq, const void* 
       case 14: attend(latent_decode_kernel<T, 14>); break;                                                                     \
       default: attend(latent_decode_kernel<T, 0>);                                                                             \
     }                                                                                                                          \
-    if (expand) {                                                                                                              \
-      const size_t leave = (16 * 64 + 16) * 4 + 512 * 16 + (size_t)16 * (Lp + 32 / sizeof(T)) * sizeof(T);                       \
-      latent_leave_kernel<T><<<dim3(heads, tw_div_up(n_seqs, 16)), 512, leave, stream>>>(a, b);                                  \
-    } else if (splits > 1) {                                                                                                   \
-      latent_decode_merge_kernel<T><<<dim3(n_seqs, heads), 256, 0, stream>>>(a);                                                 \
-    }                                                                                                                          \
+    const size_t leave = (16 * 64 + 16) * 4 + 512 * 16 + (size_t)16 * (Lp + 32 / sizeof(T)) * sizeof(T);                         \
+    latent_leave_kernel<T><<<dim3(heads, tw_div_up(n_seqs, 16)), 512, leave, stream>>>(a, b);                                    \
   } while (0)
   if (dtype == TW_DTYPE_BF16) TW_LATENT_DECODE(bf16_t);
   else if (dtype == TW_DTYPE_F32) TW_LATENT_DECODE(float);

@@ -958,11 +958,11 @@ def latent_decode(q, keys, values, block_table, q_start, kv_len, n_seqs, out, he
     scale * q_a . key over the sequence's keys, times the values (the first latent_dev elements of the key rows).
     q [rows, heads * K] (head a at a * K), keys [pages, 1, page, K], values [pages, 1, latent_dev, page] (the same
     elements, transposed inside a page), out [rows, heads * latent_dev]. splits > 1 cuts every sequence's keys into
-    ranges for separate workgroups; needs a float32 workspace of `latent_decode_workspace_floats` floats. sink float32
+    ranges for separate workgroups. workspace: float32, `latent_decode_workspace_floats` floats. sink float32
     [heads]: exp(sink_a) more in head a's denominator (no key, no value, not scaled).
     expand [heads, size, latent_dev] of q's type: out [rows, heads * out_stride] takes every head's result (rounded to that type)
-    times its matrix instead, head a at a * out_stride; gate (laid out like out): times sigmoid(gate). Needs the workspace
-    for one range too."""
+    times its matrix instead, head a at a * out_stride; gate (laid out like out): times sigmoid(gate). (One range without EXPAND makes
+    a workspace of its own if it gets none.)"""
     _need(sink is None or (sink.dtype == torch.float32 and sink.is_contiguous() and sink.numel() == heads), "sink must be float32 [heads]")
     page, K = keys.shape[2], keys.shape[3]
     Lp = values.shape[2]
@@ -983,10 +983,10 @@ def latent_decode(q, keys, values, block_table, q_start, kv_len, n_seqs, out, he
     _need(K % 16 == 0 and K <= 256 and Lp % 16 == 0 and 16 <= Lp <= 240 and Lp <= K and page % 4 == 0, "unsupported sizes")
     _need(block_table.dim() == 2 and block_table.stride(1) == 1 and block_table.shape[0] >= n_seqs, "block_table must be 2-D")
     _need(q_start.numel() >= n_seqs + 1 and kv_len.numel() >= n_seqs, "sequence metadata is too short")
-    ws_ptr, ws_floats = None, 0
-    if splits > 1 or expand is not None:
-        _need(workspace is not None and workspace.dtype == torch.float32, "split attention needs a float32 workspace")
-        ws_ptr, ws_floats = _dev(workspace), workspace.numel()
+    if workspace is None and splits == 1 and expand is None:
+        workspace = torch.empty(latent_decode_workspace_floats(n_seqs, heads, Lp, 1), dtype=torch.float32, device=q.device)
+    _need(workspace is not None and workspace.dtype == torch.float32, "split attention needs a float32 workspace")
+    ws_ptr, ws_floats = _dev(workspace), workspace.numel()
     check(library().tw_latent_decode(dtype_id(q.dtype), _dev(q), ldq, _dev(keys), _dev(values),
                                      _dev(block_table, torch.int32, "block_table"), block_table.stride(0),
                                      _dev(q_start, torch.int32, "q_start"), _dev(kv_len, torch.int32, "kv_len"), int(n_seqs),

@@ -8,8 +8,9 @@ head a's key is [W_uk,a c | kr], its value W_uv,a c, its query [D unrotated | R 
 Only c and kr are cached; the engine's paged cache holds them like any other group (one key/value head whose key row
 is [c | kr] and whose value is c). One-token sequences run the attention over that one head directly, for all query
 heads at once: the products with W_uk and W_uv are moved to the query side and the output side (one small matrix per
-head each, `ops.head_linear`), so a step reads every cached token once, at the latent's size. Prompt portions, with
-many query rows against the same keys, go the other way round: the cached latents of their sequences are expanded
+head each, in the launches of `ops.latent_finish` and `ops.latent_decode`), so a step reads every cached token once, at
+the latent's size. Prompt portions, with many query rows against the same keys, go the other way round: the cached
+latents of their sequences are expanded
 once a step (one product with [W_uk; W_uv] over the gathered key rows) into keys and values per head in scratch pages
 of their own, and the engine's ordinary prompt attention runs on those. A layer may read the cache slot of another
 layer (`LayerRun(writes_cache=False)`): it then has no down-projection of its own (`own_latent=False`) and uses that
