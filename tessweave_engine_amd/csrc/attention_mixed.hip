@@ -831,12 +831,16 @@ static int mixed_dispatch(const MixedAttnArgs& args, int n_seqs, int max_q_len, 
   return TW_LAUNCH_RESULT();
 }
 
-// Key ranges for one-token sequences of up to max_kv_len seen keys: up to two workgroups a CU, each with 4 key tiles or more:
-// what attn_mixed_one_kernel takes at once.
-extern "C" int tw_attn_mixed_splits(int n_seqs, int max_kv_len) {
+// Key ranges for one-token sequences of up to max_kv_len seen keys, each of 4 key tiles or more: up to two workgroups a CU where
+// attn_mixed_one_kernel takes the sizes (H 0: taken to be so), which reads 4 tiles at once; one a CU for attn_mixed_kernel, whose workgroups
+// walk their tiles one by one and gain nothing from a second one beside them. (That kernel, bfloat16 / float32, us, four / two / one a CU: 20 heads of
+// 128 on 10, 8 sequences of 2,050 keys 51.8, 104 / 57.6, 106 / 51.8, 104, 16 of 2,050 95, 198 / 95, 198 / 81, 176, 64 of 600 97, 202 / 96, 201
+// / 90, 196, 64 of 2,050 299, 670 / 271, 626 / 259, 604; values of 256 on 4 134, 244 / 134, 244 / 114, 213 for 16 of 2,050. With ranges of 5 tiles
+// instead of 4, one sequence of 300 keys 39.0, 75.9 instead of 33.8, 63.0.)
+extern "C" int tw_attn_mixed_splits(int n_seqs, int max_kv_len, int H, int G, int D, int E, int page_size) {
   if (n_seqs <= 0) return 1;
   const int tiles = tw_div_up(max_kv_len, 16);
-  int want = 512 / n_seqs;
+  int want = (H == 0 || mixed_one_takes(1, H, G, D, E, page_size) ? 512 : 256) / n_seqs;
   int most = tw_div_up(tiles, 4);
   int s = want < most ? want : most;
   if (s > 64) s = 64;

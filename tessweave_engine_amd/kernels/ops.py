@@ -753,8 +753,13 @@ def layer_end(x, layer, branch=None, branch_weight=None, eps=0.0, mult=1.0, hist
 
 # ---- attention with scores mixed across heads ------------------------------------------------------------------------
 
-def attn_mixed_splits(n_seqs, max_kv_len):
-    return int(library().tw_attn_mixed_splits(int(n_seqs), int(max_kv_len)))
+def attn_mixed_splits(n_seqs, max_kv_len, q_heads=0, keys=None, values=None):
+    """Key ranges for n_seqs one-token sequences that see up to max_kv_len keys (a window: and the 15 that its first tile may hold
+    more); the query heads and the paged keys and values, if given, say which kernel will run."""
+    if keys is None:
+        return int(library().tw_attn_mixed_splits(int(n_seqs), int(max_kv_len), 0, 1, 0, 0, 0))
+    return int(library().tw_attn_mixed_splits(int(n_seqs), int(max_kv_len), int(q_heads), keys.shape[1], keys.shape[3],
+                                              values.shape[2], keys.shape[2]))
 
 
 def attn_mixed_prefill_splits(n_tokens, n_seqs, max_kv_len):

@@ -129,11 +129,12 @@ class MixedHeadAttention(MixerBranch):
             most = ctx.kv_capacity
             if window:
                 longest, most = min(longest, window + 15), min(most, window + 15)   # (of the key tiles a window touches)
-            splits = ops.attn_mixed_splits(ctx.n_decode, longest)
+            splits = ops.attn_mixed_splits(ctx.n_decode, longest, H, keys, values)
             ws = None
             if splits > 1:
                 # sized for the most splits any length class can ask for, so that it never grows under a capture
-                floats = ops.attn_mixed_workspace_floats(ctx.n_decode, 1, H, E, max(splits, ops.attn_mixed_splits(ctx.n_decode, most)))
+                floats = ops.attn_mixed_workspace_floats(ctx.n_decode, 1, H, E,
+                                                         max(splits, ops.attn_mixed_splits(ctx.n_decode, most, H, keys, values)))
                 ws = ctx.workspace.get("attn.mixed.split", (floats,), torch.float32)
             ops.attn_mixed(proj, keys, values, group.block_table, ctx.q_start, ctx.kv_len, 0, ctx.n_decode, 1, out,
                            H, G, self.scale, splits=splits, workspace=ws, **common)

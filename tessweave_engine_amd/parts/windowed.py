@@ -44,13 +44,13 @@ def mixed_attention(ctx, q, keys, values, group, out, q_heads, kv_heads, value_d
         longest = ctx.kv_bound if ctx.capturing else ctx.max_kv_len
         most = ctx.kv_capacity
         if window:
-            longest, most = min(longest, span), min(most, span)
-        splits = ops.attn_mixed_splits(ctx.n_decode, longest)
+            longest, most = min(longest, span + 15), min(most, span + 15)     # (of the key tiles a window touches)
+        splits = ops.attn_mixed_splits(ctx.n_decode, longest, q_heads, keys, values)
         ws = None
         if splits > 1:
             # sized for the most splits any length class can ask for, so that it never grows under a capture
             floats = ops.attn_mixed_workspace_floats(ctx.n_decode, 1, q_heads, value_dev,
-                                                     max(splits, ops.attn_mixed_splits(ctx.n_decode, most)))
+                                                     max(splits, ops.attn_mixed_splits(ctx.n_decode, most, q_heads, keys, values)))
             ws = ctx.workspace.get(tag + ".split", (floats,), torch.float32)
         ops.attn_mixed(q, keys, values, group.block_table, ctx.q_start, ctx.kv_len, 0, ctx.n_decode, 1, out, q_heads,
                        kv_heads, scale, splits=splits, workspace=ws, **common)

@@ -36,3 +36,29 @@ def test_an_activation_behind_few_rows_asks_for_what_its_kernel_takes(rows):
     assert ops.linear_act_few_pays(torch.zeros(rows, 2048, dtype=torch.bfloat16), weight)
     assert ops.linear_act_few_pays(torch.zeros(rows + 1, 2056, dtype=torch.bfloat16)[:rows, :2048], weight)
     assert not ops.linear_act_few_pays(torch.zeros(rows + 1, 2050, dtype=torch.bfloat16)[:rows, :2048], weight)
+
+
+@pytest.mark.parametrize("heads,kv_heads,dim,value_dim,page,one", [(16, 4, 128, 128, 16, True), (20, 10, 128, 128, 16, False), (16, 4, 128, 256, 16, False),
+                                                                   (16, 8, 192, 128, 16, False), (16, 4, 128, 128, 24, False)])
+def test_key_ranges_of_mixed_heads_follow_the_kernel(heads, kv_heads, dim, value_dim, page, one):
+    """Two workgroups a CU for the kernel whose waves have a key head each, one for the other, ranges of four tiles or more."""
+    keys, values = torch.empty(1, kv_heads, page, dim), torch.empty(1, kv_heads, value_dim, page)
+    for n in (1, 4, 8, 16, 32, 64, 512):
+        assert ops.attn_mixed_splits(n, 4096, heads, keys, values) == max(1, min((512 if one else 256) // n, 64))
+        assert ops.attn_mixed_splits(n, 65, heads, keys, values) == (2 if n <= (256 if one else 128) else 1)
+
+
+@pytest.mark.parametrize("window,keep_first", [(1024, 0), (1024, 8), (50, 0)])
+def test_key_ranges_of_a_window_hold_the_tiles_that_it_touches(monkeypatch, window, keep_first):
+    """A window that ends inside a tile touches one tile more than a window of whole tiles: no range of the step has a fifth."""
+    from types import SimpleNamespace
+    from tessweave_engine_amd.parts.windowed import mixed_attention
+    seen = []
+    monkeypatch.setattr(ops, "attn_mixed", lambda *a, **k: seen.append(k["splits"]))
+    keys = torch.empty(1, 4, 16, 128)
+    ctx = SimpleNamespace(n_decode=1, n_seqs=1, capturing=False, kv_bound=4096, max_kv_len=4000, kv_capacity=4096, q_start=None, kv_len=None,
+                          workspace=SimpleNamespace(get=lambda tag, shape, dtype: torch.empty(shape, dtype=dtype)))
+    mixed_attention(ctx, None, keys, torch.empty(1, 4, 128, 16), SimpleNamespace(block_table=None), None, 16, 4, 128, 0.1, window=window,
+                    keep_first=keep_first)
+    tiles = max(len({j // 16 for j in range(p - window + 1, p + 1)} | {j // 16 for j in range(keep_first)}) for p in range(3900, 3950))
+    assert -(-tiles // seen[0]) <= 4
