@@ -784,15 +784,23 @@ static bool moe_splits_k(bool f32, int units, long items, int X, int C, int Cd, 
   return 1.4 * ranges / 4 < columns;
 }
 
-// Steps of few rows: columns a workgroup (NT x 16), waves and k-steps a request, by how many tiles can be in use. What bounds
-// them is the tail of the last workgroups and a wave's chain of requests, so the fewer tiles the smaller the pieces. float32
-// (whose MFMAs take as long as the loads) has 16 columns: 16 waves of 2 steps up to 16 tiles, 8 of 4 above; bfloat16 32 columns
-// and 4 waves of 4 steps, but up to 16 tiles of gated experts, 4 of plain ones, 16 columns and 8 waves with 2 steps on their way
-// behind 2. 16 experts of 2,048 x 1,408, two a token, gated, all launches of the experts, us (32 columns and 4 waves with the tiles
-// first in the grid / the same with the ranges first / this): float32 1 token 29.7 / 29.8 / 20.5, 2 33.1 / 33.8 / 33.6, 4 59.6 / 61.4 /
-// 51.0, 8 90.3 / 73.7 / 67.9, 32 120 / 101 / 99; bfloat16 1 token 18.0 / 18.1 / 13.4, 4 30.4 / 30.8 / 28.1, 8 42.8 / 38.0 / 37.5, 32
-// 57.6 / 52.1; plain bfloat16 1 token 14.2 / 14.4 / 11.6, 8 31.7 / 28.4; 128 experts of 2,048 x 768, 8 of them, 8 tokens: float32 187 /
-// 173 / 180, bfloat16 94.0 / 90.5.
+// Steps of few rows: columns a workgroup (NT x 16), waves and k-steps a request. What bounds few tiles is the tail of the last workgroups
+// and a wave's chain of requests, so the pieces are small: 16 columns, in float32 (whose MFMAs take as long as the loads) 16 waves of
+// 2 steps, in bfloat16 8 waves with 2 steps on their way behind 2. Many tiles fill the chip whatever the pieces are, and what each
+// workgroup costs by itself counts: the rows that it reads once more, its sums' meeting in LDS. Then float32 has 32 columns and 8 waves of
+// 2 steps, without a gate from 16 tiles and 512 elements of K on, behind one from 32 tiles and 1,536 on; shorter sums 16 columns and waves
+// of 4 steps, 8 of them, behind a gate from 32 tiles on 4. bfloat16 has 32 columns and 4 waves of 4, behind a gate from 17 tiles on, without
+// one from 20,000 columns of all tiles' two products on. All launches of the experts, their matrices from
+// HBM, us (32 columns and 4 waves / 16 and 16 (bfloat16: 8) / float32: 16 and 8 / 16 and 4 / 32 and 8; C x F, experts, tiles):
+//   float32, gated: 2,048 x 1,408, 16, 2 tiles 31.4 / 22.1 / 22.7 / 24.8 / 32.3, 8 61.8 / 51.8 / 52.5 / 53.7 / 60.6, 17 95.3 / 90.8 / 89.7 / 92.0 / 91.8;
+//   2,048 x 768, 128, 8 39.6 / 41.7 / 42.0 / 40.5 / 38.9, 64 169 / 190 / 176 / 169 / 166; 1,024 x 512, 64, 4 19.1 / 16.4 / 16.5 / 15.7 / 20.0, 32 42.6 / 46.2 / 43.7
+//   / 41.3 / 41.6, 62 57.5 / 76.5 / 63.3 / 54.3 / 58.8; 4,096 x 2,048, 8, 44 514 / 524 / 534 / 535 / 451
+//   float32, plain: 2,048 x 1,408, 16, 2 25.0 / 18.5 / 19.1 / 20.7 / 24.5, 8 44.8 / 39.7 / 40.8 / 41.4 / 42.8, 16 55.0 / 54.8 / 55.6 / 55.6 / 52.3; 1,536 x 2,816,
+//   16, 18 105 / 119 / 124 / 108 / 98; 2,048 x 768, 128, 64 123 / 151 / 147 / 126 / 118; 1,024 x 512, 64, 16 22.2 / 24.0 / 23.6 / 23.0 / 21.7, 62 44.5 / 68.4 / 59.0 /
+//   46.4 / 44.2; 256 x 96, 8, 64 18.4 / 17.9 / 16.7 / 17.5 / 17.3
+//   bfloat16, gated: 2,048 x 1,408, 16, 2 19.7 / 14.8, 8 31.8 / 28.7, 16 39.3 / 39.4; 2,048 x 768, 128, 32 56.7 / 60.3, 64 89 / 100
+//   bfloat16, plain: 2,048 x 1,408, 16, 2 15.8 / 13.0, 8 24.1 / 24.1, 16 29.8 / 32.9; 768 x 256, 32, 8 12.7 / 10.9, 16 13.9 / 12.6, 32 15.3 / 15.3; 512 x 1,024, 4, 5 11.5 /
+//   10.4; 1,536 x 2,816, 16, 8 33.2 / 34.7; 2,048 x 768, 128, 8 19.6 / 20.0
 template <typename T, int ACT, bool PLAN, int NT, int WAVES, int STEPS, bool AHEAD>
 static void moe_few_form(const T* rows, const T* first, const T* second, const T* down, const int* tile_expert, T* act, float* ys, int C,
                          int Cd, int Fd, float limit, int tiles, const MoePairs& pairs, hipStream_t stream) {
@@ -808,11 +816,14 @@ static void moe_few_products(const T* rows, const T* first, const T* second, con
                              int C, int Cd, int Fd, float limit, int tiles, int in_use, const MoePairs& pairs, hipStream_t stream) {
 #define TW_MOE_FEW(...)                                                                                                           \
   moe_few_form<T, ACT, PLAN, __VA_ARGS__>(rows, first, second, down, tile_expert, act, ys, C, Cd, Fd, limit, tiles, pairs, stream)
+  constexpr bool GLU = ACT == 1 || ACT == 3;
   if constexpr (sizeof(T) == 4) {
-    if (in_use <= 16) TW_MOE_FEW(1, 16, 2, false);
-    else TW_MOE_FEW(1, 8, 4, false);
+    if (GLU ? in_use >= 32 && Cd >= 1536 : in_use >= 16 && Cd >= 512) TW_MOE_FEW(2, 8, 2, false);
+    else if (in_use <= 16) TW_MOE_FEW(1, 16, 2, false);
+    else if (!GLU || in_use < 32) TW_MOE_FEW(1, 8, 4, false);
+    else if constexpr (GLU) TW_MOE_FEW(1, 4, 4, false);
   } else {
-    if (in_use <= (ACT == 1 || ACT == 3 ? 16 : 4)) TW_MOE_FEW(1, 8, 2, true);
+    if (GLU ? in_use <= 16 : (long)in_use * (Fd + C) <= 20000) TW_MOE_FEW(1, 8, 2, true);
     else TW_MOE_FEW(2, 4, 4, false);
   }
 #undef TW_MOE_FEW
