@@ -504,7 +504,7 @@ __global__ __launch_bounds__(256) void gemm_tiled_kernel(const T* __restrict__ A
 //
 // Against the float32 MFMA (128x128 tiles, two LDS stages, the K ranges of tiled_splits): 478 x 10,432 x 2,048 271 -> 163 us, 478 x 2,048 x
 // 4,096 108 -> 67, 4,096 x 32,000 x 2,048 4,314 -> 3,430 (157 TFLOP/s, so 1.25 PFLOP/s in bfloat16, where power is the bound), 65 x 896 x 4,864
-// 46 -> 22; 109 random products (65 to 3,000 rows) take 0.54 of the time, the slowest 0.92. (With six products 137, 57, 2,817 and 20;
+// 46 -> 22; 109 random products (65 to 3,000 rows) take 0.55 of the time, the slowest 0.92. (With six products 137, 57, 2,817 and 20;
 // 0.49. The factor of 2^24 costs 0 to 4 %.) Their error against 64 bits is 0.35 of what it was in the mean and 0.77 at the most. Rows of 4 to 2,048 elements, of 2^-24 of the sum of
 // sizes, largest and mean square (float32 MFMA / this): dense 2.4 to 4.3 and 0.45 to 0.47 / 1.5 to 2.2 and 0.15 to 0.30, all of one sign 58 and
 // 11.8 / 18 and 4.2, four elements not zero 2.7 and 0.45 / 2.1 and 0.34, the first element 2^14 times the others 103 and 14.6 / 30 and 5.2.
@@ -1595,7 +1595,7 @@ static const TurnsCost kTurnsCost[5] = {{}, {3.8, 1.45, 0.351, 0.482}, {4.3, 2.2
 // off). Over these the choice is then 1.8 % faster in the mean than among the four, none more than 1 % slower, and 0.4 % behind the
 // best of the nine. (With K ranges, which no product of that fit had, 8 %: products of 129 to 167 rows were 3 to 7 % slower at 3.) They fill what 128 and 256 rows leave (536 x 27,648 x 5,120 183 -> 145 us by 192x384, 521 x 22,016 x 2,048 59 -> 49 by 192x256,
 // 536 x 7,168 x 5,120 58.6 -> 54.8 by 192x128), and 256x320 has a tenth less to copy and to read a product than 256x256
-// (8,192 x 37,888 x 3,584 1,605 -> 1,549).
+// (37,888 x 3,584, gated: 2,048 rows 416 to 434 -> 405 to 410, 8,192 rows 1,535 -> 1,502 to 1,519).
 static const TurnsCost kNineCost[10] = {{}, {4.1, 1.71, 0.361, 0.504}, {4.5, 2.95, 0.596, 0.819}, {1.0, 8.67, 0.982, 1.136}, {2.7, 5.83, 0.776, 0.955},
                                         {4.2, 2.50, 0.535, 0.608}, {4.1, 3.97, 0.663, 0.808}, {3.1, 5.44, 0.843, 0.989}, {1.0, 9.36, 1.179, 1.298}, {1.0, 9.78, 1.194, 1.316}};
 static double turns_us(const TurnsCost& c, int shape, int splits, int M, int N, int K) {
@@ -1657,7 +1657,9 @@ static bool turns_pay(bool glu, bool adds, int M, int N, int K) {
 // float32 (gemm_parts_kernel): 1 is 128x128, 2 64x128, 3 64x64, with K ranges, the least estimated time in microseconds. A launch, rounds of
 // the workgroups that a CU holds, and k-tiles of 32, which take `alone` a round where a CU has little else and n x `full` where its n
 // workgroups share the matrix unit; the fourth powers of the two add up. Fitted to 1,586 forms of 142 products (65 to 3,000 rows, 512 to
-// 32,000 columns, K 256 to 4,864, 1 to 8 ranges): 5 to 6 % off, the choice 0.4 % behind the fastest of all, 4 of 142 more than 5 %.
+// 32,000 columns, K 256 to 4,864, 1 to 8 ranges) when the kernel formed six products of parts: 5 to 6 % off, the choice 0.4 % behind the
+// fastest of all. With eight every form takes some 15 % longer and the choice stays good: of 159 other products it is 0.6 % behind the fastest form,
+// 8 of them more than 5 %, the same as by constants fitted anew to their 1,327 forms. (An estimate takes 0.3 us: it is not kept.)
 static const struct { int m, n, held; double launch, tile, alone, full, sums; } kParts[4] = {
     {}, {128, 128, 2, 3.1, 1.73, 1.429, 1.170, 0.32}, {64, 128, 3, 4.2, 0.0, 0.966, 0.723, 0.30}, {64, 64, 5, 3.1, 0.0, 0.686, 0.426, 0.34}};
 static TilePlan choose_parts(bool glu, int M, int N, int K) {
