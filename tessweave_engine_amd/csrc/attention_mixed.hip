@@ -24,6 +24,8 @@
 // A tile's keys can be cut into `splits` ranges for separate workgroups (one-token sequences, whose only tile
 // would otherwise walk all keys alone; prompt portions with fewer tiles than the chip has CUs); a second kernel
 // merges the partial results in index order.
+#include <algorithm>
+
 #include "tw_common.h"
 
 template <typename T> __device__ __forceinline__ float mx_exp(float v);
@@ -831,20 +833,36 @@ static int mixed_dispatch(const MixedAttnArgs& args, int n_seqs, int max_q_len, 
   return TW_LAUNCH_RESULT();
 }
 
-// Key ranges for one-token sequences of up to max_kv_len seen keys, each of 4 key tiles or more: up to two workgroups a CU where
-// attn_mixed_one_kernel takes the sizes (H 0: taken to be so), which reads 4 tiles at once; one a CU for attn_mixed_kernel, whose workgroups
-// walk their tiles one by one and gain nothing from a second one beside them. (That kernel, bfloat16 / float32, us, four / two / one a CU: 20 heads of
-// 128 on 10, 8 sequences of 2,050 keys 51.8, 104 / 57.6, 106 / 51.8, 104, 16 of 2,050 95, 198 / 95, 198 / 81, 176, 64 of 600 97, 202 / 96, 201
-// / 90, 196, 64 of 2,050 299, 670 / 271, 626 / 259, 604; values of 256 on 4 134, 244 / 134, 244 / 114, 213 for 16 of 2,050. With ranges of 5 tiles
-// instead of 4, one sequence of 300 keys 39.0, 75.9 instead of 33.8, 63.0.)
-extern "C" int tw_attn_mixed_splits(int n_seqs, int max_kv_len, int H, int G, int D, int E, int page_size) {
+// Key ranges for one-token sequences of up to max_kv_len seen keys: the least estimated time, in steps of a workgroup over its key tiles
+// (attn_mixed_one_kernel takes 4 tiles a step in bfloat16, 2 in float32, attn_mixed_kernel one): rounds of as many workgroups as the
+// CUs work on at once, each a begin and its steps, and for more than one range the merge. A CU works on four of the one's waves (one a SIMD),
+// eight of the other's. Of 1,189 calls of 15 forms (1 to 32 heads on 1 to 16, 1 to 300 sequences of 48 to 4,000 keys, both types) whose ranges
+// were measured beside one another the choice is 1.4 % behind the fastest, by rules without rounds (256 or 512 workgroups, ranges of four tiles or
+// more) 10 and 21 %: bfloat16, 30 heads of 64 on 10, 93 sequences of 645 keys 2 ranges 144 us, 5 132; 20 of 128 on 10, one of 80 keys 2 ranges 1.6
+// times as long as 5; 24 on 4, 200 of 100 keys 2 ranges 1.9 times as long as one.
+// No call gets more ranges than tw_attn_mixed_most_splits: the merge holds 64, and from 1,024 workgroups on more only cost.
+extern "C" int tw_attn_mixed_most_splits(int n_seqs, int max_kv_len) {
   if (n_seqs <= 0) return 1;
-  const int tiles = tw_div_up(max_kv_len, 16);
-  int want = (H == 0 || mixed_one_takes(1, H, G, D, E, page_size) ? 512 : 256) / n_seqs;
-  int most = tw_div_up(tiles, 4);
-  int s = want < most ? want : most;
-  if (s > 64) s = 64;
-  return s < 1 ? 1 : s;
+  return std::max(1, std::min({MX_MERGE_MOST, tw_div_up(max_kv_len, 16), 1024 / n_seqs}));
+}
+
+extern "C" int tw_attn_mixed_splits(int dtype, int n_seqs, int max_kv_len, int H, int G, int D, int E, int page_size) {
+  const int tiles = tw_div_up(max_kv_len, 16), most = tw_attn_mixed_most_splits(n_seqs, max_kv_len);
+  const bool one = mixed_one_takes(1, H, G, D, E, page_size);
+  const int step = !one ? 1 : dtype == TW_DTYPE_BF16 ? 4 : 2, waves = one ? G : H <= 8 ? H : tw_div_up(H, 2);
+  const int at_once = 256 * std::max(1, (one ? 4 : 8) / waves);
+  int best = 1;
+  double least = 0;
+  for (int s = 1; s <= most; ++s) {
+    const int blocks = n_seqs * s, steps = tw_div_up(tw_div_up(tiles, s), step);
+    double t = tw_div_up(blocks, at_once) * ((one ? 0.3 : 0.6) + steps);
+    if (s > 1) t += one ? 1.5 + 0.002 * blocks * H / 16 : 0.3 + 0.001 * blocks;
+    if (s == 1 || t < least) {
+      least = t;
+      best = s;
+    }
+  }
+  return best;
 }
 
 // Key ranges for prompt portions: only where the row tiles alone would leave most of the chip idle and a tile

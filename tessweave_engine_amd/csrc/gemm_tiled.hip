@@ -1607,7 +1607,7 @@ static double turns_us(const TurnsCost& c, int shape, int splits, int M, int N, 
   return t;
 }
 // (A product asks for its plan up to three times, for its scratch, its ranges and its launch, and a model's steps ask for the
-// same few: the last 64 are kept, a thread's own. Estimating 32 candidates takes some microseconds, which a step that is issued launch by
+// same few: the last 64 are kept, a thread's own. Estimating 32 candidates takes a microsecond, which a step that is issued launch by
 // launch, a prompt's portion, would spend in front of each product.)
 static TilePlan choose_turns(bool glu, int M, int N, int K) {
   struct Known {

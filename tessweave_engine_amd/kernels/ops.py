@@ -753,13 +753,18 @@ def layer_end(x, layer, branch=None, branch_weight=None, eps=0.0, mult=1.0, hist
 
 # ---- attention with scores mixed across heads ------------------------------------------------------------------------
 
-def attn_mixed_splits(n_seqs, max_kv_len, q_heads=0, keys=None, values=None):
+def attn_mixed_splits(n_seqs, max_kv_len, q_heads=16, keys=None, values=None):
     """Key ranges for n_seqs one-token sequences that see up to max_kv_len keys (a window: and the 15 that its first tile may hold
-    more); the query heads and the paged keys and values, if given, say which kernel will run."""
+    more); the query heads and the paged keys and values say which kernel will run (none: bfloat16, 4 heads of 128 in pages of 16)."""
     if keys is None:
-        return int(library().tw_attn_mixed_splits(int(n_seqs), int(max_kv_len), 0, 1, 0, 0, 0))
-    return int(library().tw_attn_mixed_splits(int(n_seqs), int(max_kv_len), int(q_heads), keys.shape[1], keys.shape[3],
-                                              values.shape[2], keys.shape[2]))
+        return int(library().tw_attn_mixed_splits(dtype_id(torch.bfloat16), int(n_seqs), int(max_kv_len), int(q_heads), 4, 128, 128, 16))
+    return int(library().tw_attn_mixed_splits(dtype_id(keys.dtype), int(n_seqs), int(max_kv_len), int(q_heads), keys.shape[1],
+                                              keys.shape[3], values.shape[2], keys.shape[2]))
+
+
+def attn_mixed_most_splits(n_seqs, max_kv_len):
+    """The most that `attn_mixed_splits` gives for up to max_kv_len keys: what a workspace that may not grow is sized for."""
+    return int(library().tw_attn_mixed_most_splits(int(n_seqs), int(max_kv_len)))
 
 
 def attn_mixed_prefill_splits(n_tokens, n_seqs, max_kv_len):

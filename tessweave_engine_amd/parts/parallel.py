@@ -133,8 +133,7 @@ class MixedHeadAttention(MixerBranch):
             ws = None
             if splits > 1:
                 # sized for the most splits any length class can ask for, so that it never grows under a capture
-                floats = ops.attn_mixed_workspace_floats(ctx.n_decode, 1, H, E,
-                                                         max(splits, ops.attn_mixed_splits(ctx.n_decode, most, H, keys, values)))
+                floats = ops.attn_mixed_workspace_floats(ctx.n_decode, 1, H, E, max(splits, ops.attn_mixed_most_splits(ctx.n_decode, most)))
                 ws = ctx.workspace.get("attn.mixed.split", (floats,), torch.float32)
             ops.attn_mixed(proj, keys, values, group.block_table, ctx.q_start, ctx.kv_len, 0, ctx.n_decode, 1, out,
                            H, G, self.scale, splits=splits, workspace=ws, **common)

@@ -50,7 +50,7 @@ def mixed_attention(ctx, q, keys, values, group, out, q_heads, kv_heads, value_d
         if splits > 1:
             # sized for the most splits any length class can ask for, so that it never grows under a capture
             floats = ops.attn_mixed_workspace_floats(ctx.n_decode, 1, q_heads, value_dev,
-                                                     max(splits, ops.attn_mixed_splits(ctx.n_decode, most, q_heads, keys, values)))
+                                                     max(splits, ops.attn_mixed_most_splits(ctx.n_decode, most)))
             ws = ctx.workspace.get(tag + ".split", (floats,), torch.float32)
         ops.attn_mixed(q, keys, values, group.block_table, ctx.q_start, ctx.kv_len, 0, ctx.n_decode, 1, out, q_heads,
                        kv_heads, scale, splits=splits, workspace=ws, **common)

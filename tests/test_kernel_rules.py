@@ -38,14 +38,27 @@ def test_an_activation_behind_few_rows_asks_for_what_its_kernel_takes(rows):
     assert not ops.linear_act_few_pays(torch.zeros(rows + 1, 2050, dtype=torch.bfloat16)[:rows, :2048], weight)
 
 
-@pytest.mark.parametrize("heads,kv_heads,dim,value_dim,page,one", [(16, 4, 128, 128, 16, True), (20, 10, 128, 128, 16, False), (16, 4, 128, 256, 16, False),
-                                                                   (16, 8, 192, 128, 16, False), (16, 4, 128, 128, 24, False)])
-def test_key_ranges_of_mixed_heads_follow_the_kernel(heads, kv_heads, dim, value_dim, page, one):
-    """Two workgroups a CU for the kernel whose waves have a key head each, one for the other, ranges of four tiles or more."""
-    keys, values = torch.empty(1, kv_heads, page, dim), torch.empty(1, kv_heads, value_dim, page)
-    for n in (1, 4, 8, 16, 32, 64, 512):
-        assert ops.attn_mixed_splits(n, 4096, heads, keys, values) == max(1, min((512 if one else 256) // n, 64))
-        assert ops.attn_mixed_splits(n, 65, heads, keys, values) == (2 if n <= (256 if one else 128) else 1)
+@pytest.mark.parametrize("dtype,heads,kv_heads,dim,value_dim,n,keys,good", [
+    ("bfloat16", 16, 4, 128, 128, 1, 320, {5}), ("bfloat16", 16, 4, 128, 128, 16, 48, {1}), ("bfloat16", 1, 1, 128, 128, 2, 68, {1}),
+    ("bfloat16", 24, 4, 128, 128, 200, 100, {1}), ("float32", 16, 4, 128, 128, 1, 128, {4}), ("bfloat16", 30, 10, 64, 64, 93, 645, {5, 11}),
+    ("bfloat16", 20, 10, 128, 128, 64, 600, {4}), ("float32", 20, 10, 128, 128, 1, 80, {5}), ("bfloat16", 16, 4, 128, 256, 130, 400, {4, 5}),
+    ("float32", 24, 12, 128, 128, 24, 700, {9, 10}), ("bfloat16", 16, 4, 192, 128, 4, 3000, set(range(47, 65)))])
+def test_key_ranges_of_mixed_heads_fill_whole_rounds(dtype, heads, kv_heads, dim, value_dim, n, keys, good):
+    """Where the ranges measured beside one another lie 3 % apart and more: the fastest, for the kernel whose waves have a key head each and
+    for the other."""
+    kind = getattr(torch, dtype)
+    k, v = torch.empty(1, kv_heads, 16, dim, dtype=kind), torch.empty(1, kv_heads, value_dim, 16, dtype=kind)
+    assert ops.attn_mixed_splits(n, keys, heads, k, v) in good
+
+
+@pytest.mark.parametrize("heads,kv_heads,dim,value_dim,page", [(16, 4, 128, 128, 16), (1, 1, 64, 64, 32), (20, 10, 128, 128, 16), (16, 4, 128, 128, 24)])
+def test_no_length_has_more_key_ranges_than_a_workspace_is_sized_for(heads, kv_heads, dim, value_dim, page):
+    """A captured step's workspace is sized once for all lengths up to the cache's."""
+    k, v = torch.empty(1, kv_heads, page, dim), torch.empty(1, kv_heads, value_dim, page)
+    for n in (1, 3, 16, 100, 1024, 2000):
+        most = [ops.attn_mixed_most_splits(n, length) for length in (1, 100, 1000, 8000)]
+        assert most == sorted(most) and most[-1] <= 64
+        assert all(1 <= ops.attn_mixed_splits(n, length, heads, k, v) <= most[-1] for length in range(1, 8000, 37))
 
 
 @pytest.mark.parametrize("window,keep_first", [(1024, 0), (1024, 8), (50, 0)])
