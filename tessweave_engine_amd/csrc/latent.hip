@@ -7,6 +7,8 @@
 // so the attention itself runs over ONE key/value head whose key row is [c | kr] and whose value is c, and only
 // c and kr are ever stored. Here: the kernel that finishes a token's projections (norm of c, rotation of kr and
 // of the queries' rotated parts, cache write), and the per-head matrix product both sides use.
+#include <algorithm>
+
 #include "tw_common.h"
 
 // One rotated pair, products and sums spelled out (a*b - c*d left to the compiler becomes one fused form or the other).
@@ -709,15 +711,38 @@ __global__ __launch_bounds__(512) void latent_leave_kernel(LatentDecodeArgs a, L
   }
 }
 
-// Key ranges a sequence: up to two workgroups a CU, each range 4 tiles of 16 keys or more, one a wave. (Against ranges of 8 tiles and
-// sizes known at run time, with the merge: 8 requests of 190 keys 15.2 -> 8.0 us, one of 2,050 17.7 -> 10.8, float32 25.8 -> 11.6.)
-extern "C" int tw_latent_decode_splits(int n_seqs, int heads, int max_kv_len) {
+// Latents of whole 32s from 64 on have an instance each; pages that are no power of two, or rotated parts of more than 64, have none.
+static int latent_sized(int K, int Lp, int page_size) {
+  return (page_size & (page_size - 1)) == 0 && page_size >= 16 && K <= Lp + 64 && Lp >= 64 && Lp <= 224 && Lp % 32 == 0 ? Lp / 16 : 0;
+}
+
+// Key ranges a sequence: the least estimated time, in tiles that a wave takes one after the other: rounds of the workgroups that the CUs
+// work on at once, each a begin and its waves' tiles, and the ranges' sums that latent_leave_kernel reads. A CU works on one workgroup where the
+// sizes are known at compile time, on two of the general kernel's, which wait longer. Of 150 calls (4 to 32 heads, nine latents, 1 to 174
+// sequences of 20 to 5,400 keys, both types) whose ranges were measured beside one another the choice is 1.6 % behind the fastest; 512 workgroups
+// with ranges of four tiles or more were 3.8 (192 + 64, 16 heads, 28 sequences of 1,092 keys 18 ranges 23.2 us, 9 17.9; 112 + 48, 10 of 3,651
+// 51 ranges 25.7, 25 19.9). (8 requests of 190 keys, latents of 192: with ranges of 8 tiles and sizes known at run time 15.2 us, now 8.0.)
+// No call gets more ranges than tw_latent_decode_most_splits.
+extern "C" int tw_latent_decode_most_splits(int n_seqs, int heads, int max_kv_len) {
   if (n_seqs <= 0) return 1;
-  const int tiles = tw_div_up(max_kv_len, 16);
-  int want = 512 / (n_seqs * tw_div_up(heads, 16));
-  if (want > tw_div_up(tiles, 4)) want = tw_div_up(tiles, 4);
-  if (want > 64) want = 64;
-  return want < 1 ? 1 : want;
+  return std::max(1, std::min({64, tw_div_up(max_kv_len, 16), 1024 / (n_seqs * tw_div_up(heads, 16))}));
+}
+
+extern "C" int tw_latent_decode_splits(int n_seqs, int heads, int max_kv_len, int K, int Lp, int page_size) {
+  const int tiles = tw_div_up(max_kv_len, 16), most = tw_latent_decode_most_splits(n_seqs, heads, max_kv_len);
+  const bool sized = latent_sized(K, Lp, page_size) != 0;
+  const int groups = n_seqs * tw_div_up(heads, 16), at_once = sized ? 256 : 512;
+  const double begin = sized ? 0.6 : 0.3, sums = sized ? 4e-4 : 1e-4;
+  int best = 1;
+  double least = 0;
+  for (int s = 1; s <= most; ++s) {
+    const double t = tw_div_up(groups * s, at_once) * (begin + tw_div_up(tw_div_up(tiles, s), 4)) + sums * n_seqs * heads * s;
+    if (s == 1 || t < least) {
+      least = t;
+      best = s;
+    }
+  }
+  return best;
 }
 
 extern "C" long tw_latent_decode_workspace_floats(int n_seqs, int heads, int Lp, int splits) {
@@ -749,8 +774,7 @@ extern "C" int tw_latent_decode(int dtype, const void* q, long ldq, const void* 
   const int head_tiles = tw_div_up(heads, 16);
   const dim3 grid(n_seqs, splits, head_tiles);
   const size_t lds = ((size_t)4 * 16 * (Lp + 4) + 128) * sizeof(float);
-  // (latents of whole 32s from 64 on have an instance each; pages that are no power of two, or rotated parts of more than 64, have none)
-  const int sized = pow2 && page_size >= 16 && K <= Lp + 64 && Lp >= 64 && Lp % 32 == 0 ? Lp / 16 : 0;
+  const int sized = latent_sized(K, Lp, page_size);
   const bool whole = K == Lp + 64;
 #define TW_LATENT_DECODE(T)                                                                                                     \
   do {                                                                                                                         \

@@ -954,8 +954,16 @@ def latent_finish(proj, q_col, c_col, kr_col, cos, sin, norm_weight, q_out, head
                                      _dev(absorb) if absorb is not None else None, int(absorb_rows), _stream()), "latent_finish")
 
 
-def latent_decode_splits(n_seqs, heads, max_kv_len):
-    return int(library().tw_latent_decode_splits(int(n_seqs), int(heads), int(max_kv_len)))
+def latent_decode_splits(n_seqs, heads, max_kv_len, keys=None, values=None):
+    """Key ranges for n_seqs one-token sequences of up to max_kv_len keys; the paged keys and values say which kernel will run (none:
+    latents of 192 with 64 rotated elements in pages of 16)."""
+    K, latent_dev, page = (256, 192, 16) if keys is None else (keys.shape[3], values.shape[2], keys.shape[2])
+    return int(library().tw_latent_decode_splits(int(n_seqs), int(heads), int(max_kv_len), K, latent_dev, page))
+
+
+def latent_decode_most_splits(n_seqs, heads, max_kv_len):
+    """The most that `latent_decode_splits` gives for up to max_kv_len keys: what a workspace that may not grow is sized for."""
+    return int(library().tw_latent_decode_most_splits(int(n_seqs), int(heads), int(max_kv_len)))
 
 
 def latent_decode_workspace_floats(n_seqs, heads, latent_dev, splits):

@@ -171,9 +171,9 @@ class LatentAttention(Mixer):
         if nd:
             # one-token sequences: all heads over the one cached head, W_uk on the query side (above), W_uv and the gate behind
             longest = ctx.kv_bound if ctx.capturing else ctx.max_kv_len
-            splits = ops.latent_decode_splits(nd, H, longest)
+            splits = ops.latent_decode_splits(nd, H, longest, keys, values)
             # sized for the most splits any length class can ask for, so that it never grows under a capture
-            floats = ops.latent_decode_workspace_floats(nd, H, Lp, max(splits, ops.latent_decode_splits(nd, H, ctx.kv_capacity)))
+            floats = ops.latent_decode_workspace_floats(nd, H, Lp, max(splits, ops.latent_decode_most_splits(nd, H, ctx.kv_capacity)))
             ws = ctx.workspace.get("latent.split", (floats,), torch.float32)
             ops.latent_decode(q[:nd], keys, values, group.block_table, ctx.q_start, ctx.kv_len, nd, out, H, self.scale,
                               splits=splits, workspace=ws, sink=self.sink, expand=self.expand, out_stride=hd, gate=gate)

@@ -61,6 +61,17 @@ def test_no_length_has_more_key_ranges_than_a_workspace_is_sized_for(heads, kv_h
         assert all(1 <= ops.attn_mixed_splits(n, length, heads, k, v) <= most[-1] for length in range(1, 8000, 37))
 
 
+@pytest.mark.parametrize("latent,rotated,heads,n,length,good", [(192, 64, 16, 28, 1092, {6, 7, 8, 9}), (128, 64, 32, 10, 1590, set(range(9, 13))), (192, 64, 16, 8, 190, {3}),
+                                                                (192, 64, 16, 1, 2050, {33}), (192, 64, 24, 9, 1733, {14}), (128, 64, 16, 174, 1149, {1}),
+                                                                (240, 16, 32, 92, 633, {2}), (112, 48, 16, 175, 1142, {2}), (240, 16, 16, 21, 4764, set(range(19, 25)))])
+def test_key_ranges_of_a_cached_latent_fill_whole_rounds(latent, rotated, heads, n, length, good):
+    """Where the ranges measured beside one another lie 3 % apart and more: the fastest. And no length has more than a workspace is sized for."""
+    keys, values = torch.empty(1, 1, 16, latent + rotated), torch.empty(1, 1, latent, 16)
+    assert ops.latent_decode_splits(n, heads, length, keys, values) in good
+    most = ops.latent_decode_most_splits(n, heads, length)
+    assert most <= 64 and all(1 <= ops.latent_decode_splits(n, heads, t, keys, values) <= most for t in range(1, length, 13))
+
+
 @pytest.mark.parametrize("window,keep_first", [(1024, 0), (1024, 8), (50, 0)])
 def test_key_ranges_of_a_window_hold_the_tiles_that_it_touches(monkeypatch, window, keep_first):
     """A window that ends inside a tile touches one tile more than a window of whole tiles: no range of the step has a fifth."""
