@@ -784,14 +784,15 @@ static bool moe_splits_k(bool f32, int units, long items, int X, int C, int Cd, 
   return 1.4 * ranges / 4 < columns;
 }
 
-// Steps of few rows: columns a workgroup (NT x 16), waves and k-steps a request. What bounds few tiles is the tail of the last workgroups
-// and a wave's chain of requests, so the pieces are small: 16 columns, in float32 (whose MFMAs take as long as the loads) 16 waves of
-// 2 steps, in bfloat16 8 waves with 2 steps on their way behind 2. Many tiles fill the chip whatever the pieces are, and what each
-// workgroup costs by itself counts: the rows that it reads once more, its sums' meeting in LDS. Then float32 has 32 columns and 8 waves of
-// 2 steps, without a gate from 16 tiles and 512 elements of K on, behind one from 32 tiles and 1,536 on; shorter sums 16 columns and waves
-// of 4 steps, 8 of them, behind a gate from 32 tiles on 4. bfloat16 has 32 columns and 4 waves of 4, behind a gate from 17 tiles on, without
-// one from 20,000 columns of all tiles' two products on. All launches of the experts, their matrices from
-// HBM, us (32 columns and 4 waves / 16 and 16 (bfloat16: 8) / float32: 16 and 8 / 16 and 4 / 32 and 8; C x F, experts, tiles):
+// Steps of few rows: columns a workgroup (NT x 16), waves and k-steps a request, for either product by itself. What bounds few workgroups
+// is the tail of the last ones and a wave's chain of requests, so the pieces are small: 16 columns, in float32 (whose MFMAs take as long as the
+// loads) 16 waves of 2 steps, in bfloat16 8 waves with 2 steps on their way behind 2. Many fill the chip whatever the pieces are, and what each
+// costs by itself counts, the rows that it reads once more and its sums' meeting in LDS: then float32 has 32 columns and 8 waves of 2 steps, or with
+// a gate and 17 to 31 tiles 16 and 8 waves of 4, bfloat16 32 columns and 4 waves of 4. Sums too short for the waves have 16 columns and 4 waves of 4.
+// Where the lines lie: 156 calls (2 to 128 experts, 96 to 4,096 x 64 to 4,096, 1 to 100 tokens) with either product in each form; the choice is 1.2 to 2.3 %
+// behind the fastest form of a product, none more than 14 % of a call (by tiles alone, for both products, 2.3 to 3.6 and 43; 4 experts of 128 x
+// 1,632, 31 tokens 24.8 us, now 16.5). All launches of the experts with both products in one form, matrices from HBM,
+// us (32 columns and 4 waves / 16 and 16 (bfloat16: 8) / float32: 16 and 8 / 16 and 4 / 32 and 8; C x F, experts, tiles):
 //   float32, gated: 2,048 x 1,408, 16, 2 tiles 31.4 / 22.1 / 22.7 / 24.8 / 32.3, 8 61.8 / 51.8 / 52.5 / 53.7 / 60.6, 17 95.3 / 90.8 / 89.7 / 92.0 / 91.8;
 //   2,048 x 768, 128, 8 39.6 / 41.7 / 42.0 / 40.5 / 38.9, 64 169 / 190 / 176 / 169 / 166; 1,024 x 512, 64, 4 19.1 / 16.4 / 16.5 / 15.7 / 20.0, 32 42.6 / 46.2 / 43.7
 //   / 41.3 / 41.6, 62 57.5 / 76.5 / 63.3 / 54.3 / 58.8; 4,096 x 2,048, 8, 44 514 / 524 / 534 / 535 / 451
@@ -801,32 +802,41 @@ static bool moe_splits_k(bool f32, int units, long items, int X, int C, int Cd, 
 //   bfloat16, gated: 2,048 x 1,408, 16, 2 19.7 / 14.8, 8 31.8 / 28.7, 16 39.3 / 39.4; 2,048 x 768, 128, 32 56.7 / 60.3, 64 89 / 100
 //   bfloat16, plain: 2,048 x 1,408, 16, 2 15.8 / 13.0, 8 24.1 / 24.1, 16 29.8 / 32.9; 768 x 256, 32, 8 12.7 / 10.9, 16 13.9 / 12.6, 32 15.3 / 15.3; 512 x 1,024, 4, 5 11.5 /
 //   10.4; 1,536 x 2,816, 16, 8 33.2 / 34.7; 2,048 x 768, 128, 8 19.6 / 20.0
-template <typename T, int ACT, bool PLAN, int NT, int WAVES, int STEPS, bool AHEAD>
-static void moe_few_form(const T* rows, const T* first, const T* second, const T* down, const int* tile_expert, T* act, float* ys, int C,
-                         int Cd, int Fd, float limit, int tiles, const MoePairs& pairs, hipStream_t stream) {
-  moe_grouped_kernel<T, ACT, NT, true, 1, PLAN, WAVES, STEPS, AHEAD><<<dim3(tw_div_up(Fd, 16 * NT), tiles), WAVES * 64, 0, stream>>>(
-      rows, Cd, first, second, tile_expert, act, Fd, Fd, Cd, limit, pairs);
-  moe_grouped_kernel<T, 0, NT, true, 1, false, WAVES, STEPS, AHEAD><<<dim3(tw_div_up(C, 16 * NT), tiles), WAVES * 64, 0, stream>>>(
-      act, Fd, down, nullptr, tile_expert, ys, C, C, Fd, 0.f, MoePairs{});
-}
-
 // tiles: of the launch; in_use: the most of them that can hold rows
 template <typename T, int ACT, bool PLAN>
-static void moe_few_products(const T* rows, const T* first, const T* second, const T* down, const int* tile_expert, T* act, float* ys,
-                             int C, int Cd, int Fd, float limit, int tiles, int in_use, const MoePairs& pairs, hipStream_t stream) {
-#define TW_MOE_FEW(...)                                                                                                           \
-  moe_few_form<T, ACT, PLAN, __VA_ARGS__>(rows, first, second, down, tile_expert, act, ys, C, Cd, Fd, limit, tiles, pairs, stream)
+static void moe_few_product(const T* rows, const T* W, const T* W2, const int* tile_expert, void* out, int N, int K, float limit, int tiles, int in_use,
+                            const MoePairs& pairs, hipStream_t stream) {
+  auto run = [&](auto kernel, int nt, int waves) {
+    kernel<<<dim3(tw_div_up(N, 16 * nt), tiles), waves * 64, 0, stream>>>(rows, K, W, W2, tile_expert, out, N, N, K, limit, pairs);
+  };
+#define TW_MOE_FEW(NT, WAVES, STEPS, AHEAD) run(moe_grouped_kernel<T, ACT, NT, true, 1, PLAN, WAVES, STEPS, AHEAD>, NT, WAVES)
   constexpr bool GLU = ACT == 1 || ACT == 3;
-  if constexpr (sizeof(T) == 4) {
-    if (GLU ? in_use >= 32 && Cd >= 1536 : in_use >= 16 && Cd >= 512) TW_MOE_FEW(2, 8, 2, false);
+  const int pieces = in_use * tw_div_up(N, 16);                // of 16 columns
+  if constexpr (sizeof(T) == 4 && GLU) {
+    if (K < 448 || (in_use >= 32 && K < 1536)) TW_MOE_FEW(1, 4, 4, false);
+    else if (in_use >= 32) TW_MOE_FEW(2, 8, 2, false);
     else if (in_use <= 16) TW_MOE_FEW(1, 16, 2, false);
-    else if (!GLU || in_use < 32) TW_MOE_FEW(1, 8, 4, false);
-    else if constexpr (GLU) TW_MOE_FEW(1, 4, 4, false);
+    else TW_MOE_FEW(1, 8, 4, false);
+  } else if constexpr (sizeof(T) == 4) {
+    if (K < (ACT == 0 ? 160 : 256)) TW_MOE_FEW(1, 4, 4, false);
+    else if (pieces <= 360 || (in_use < 16 && K > 1200)) TW_MOE_FEW(1, 16, 2, false);
+    else TW_MOE_FEW(2, 8, 2, false);
+  } else if constexpr (GLU) {
+    if (K < 256) TW_MOE_FEW(1, 4, 4, false);
+    else if (in_use <= 16) TW_MOE_FEW(1, 8, 2, true);
+    else TW_MOE_FEW(2, 4, 4, false);
   } else {
-    if (GLU ? in_use <= 16 : (long)in_use * (Fd + C) <= 20000) TW_MOE_FEW(1, 8, 2, true);
+    if (pieces <= (ACT == 0 ? 800 : 400)) TW_MOE_FEW(1, 8, 2, true);
     else TW_MOE_FEW(2, 4, 4, false);
   }
 #undef TW_MOE_FEW
+}
+
+template <typename T, int ACT, bool PLAN>
+static void moe_few_products(const T* rows, const T* first, const T* second, const T* down, const int* tile_expert, T* act, float* ys,
+                             int C, int Cd, int Fd, float limit, int tiles, int in_use, const MoePairs& pairs, hipStream_t stream) {
+  moe_few_product<T, ACT, PLAN>(rows, first, second, tile_expert, act, Fd, Cd, limit, tiles, in_use, pairs, stream);
+  moe_few_product<T, 0, false>(act, down, nullptr, tile_expert, ys, C, Fd, 0.f, tiles, in_use, MoePairs{}, stream);
 }
 
 // Where moe_parts_kernel takes a float32 step of many rows: where the first product has 140 workgroups of 64 columns and 256 of K. (Fewer

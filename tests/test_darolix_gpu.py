@@ -559,9 +559,10 @@ def test_float32_grouped_experts_of_values_without_parts(device, n, X, C, F):
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 @pytest.mark.parametrize("kind", ["silu", "gelu", "swish_limited"])
 @pytest.mark.parametrize("n,X,top,C,F", [(1, 4, 2, 32, 32), (8, 32, 2, 544, 96), (2, 24, 2, 288, 1088), (17, 40, 1, 800, 144), (16, 20, 4, 256, 288),
-                                         (13, 30, 5, 64, 80), (8, 40, 4, 1568, 80), (12, 40, 3, 576, 112), (1, 6, 5, 160, 2000), (40, 20, 2, 480, 96)])
+                                         (13, 30, 5, 64, 80), (8, 40, 4, 1568, 80), (12, 40, 3, 576, 112), (1, 6, 5, 160, 2000), (40, 20, 2, 480, 96), (5, 16, 2, 1280, 640),
+                                         (8, 40, 4, 480, 448)])
 def test_grouped_experts_of_few_rows(device, dtype, kind, n, X, top, C, F):
-    """Up to and past 4, 16, 32 and 64 tiles and 64 pairs, K from less than a step a wave to several requests and a tail, columns that end
+    """Up to and past 16, 32 and 64 tiles, 64 pairs, 360, 400 and 800 pieces of 16 columns, K from less than a step a wave to several requests and a tail, columns that end
     inside a workgroup's. The oracle and the bars of the steps of many rows; sums are shorter."""
     test_grouped_experts_of_many_rows_and_long_sums(device, dtype, kind, n, X, top, C, F)
 
