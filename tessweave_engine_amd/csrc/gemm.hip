@@ -32,6 +32,43 @@ __device__ __forceinline__ size_t tw_shuffled_chunk(int n, int c, int k_steps, i
 }
 
 // =====================================================================================
+// A norm that travels with its product (decode steps of up to 16 rows). y = W (x rinv w), rinv = 1 / sqrt(mean(x^2) + eps), is
+// rinv (W (x w)): whoever forms x last (the epilogue of a product that has the whole of K, EndLeave below) leaves the rows x w
+// rounded once, as a norm rounds x rinv w, and of every 16 columns the sum of x^2; whoever multiplies those rows adds the sums up,
+// always in one order, while its first weights are on their way, and multiplies its float32 sums by rinv. No norm kernel stands
+// between two products then: such a kernel is a few rows' latency and a launch, 3 to 4 us a time.
+// =====================================================================================
+struct RowNorms {
+  const float* sums;          // [M][count]: sums of squares of 16 columns each; count a multiple of 4, up to TW_NORM_MAX_SUMS
+  int count;
+  float width, eps;
+};
+struct RowsAsTheyAre {};
+#define TW_NORM_MAX_SUMS 256
+
+// THREADS / 16 lanes a row add its sums up: `request` asks for all of them (clamped, so that no load has a predicate), `finish`
+// leaves 1 / sqrt(mean + eps) of row i in rinv[i] (a barrier must lie between it and the readers).
+template <int THREADS>
+struct RowNormLoads {
+  static constexpr int LANES = THREADS / 16, LOADS = TW_NORM_MAX_SUMS / 4 / LANES;
+  f32x4 v[LOADS];
+  __device__ __forceinline__ void request(const RowNorms& n, int M) {
+    const int row = min((int)threadIdx.x / LANES, M - 1), l = threadIdx.x % LANES, last = n.count / 4 - 1;
+#pragma unroll
+    for (int i = 0; i < LOADS; ++i) v[i] = *reinterpret_cast<const f32x4*>(n.sums + (size_t)row * n.count + min(l + i * LANES, last) * 4);
+  }
+  __device__ __forceinline__ void finish(const RowNorms& n, float* rinv) const {
+    const int l = threadIdx.x % LANES;
+    float s = 0.f;
+#pragma unroll
+    for (int i = 0; i < LOADS; ++i) s += l + i * LANES < n.count / 4 ? (v[i][0] + v[i][1]) + (v[i][2] + v[i][3]) : 0.f;
+#pragma unroll
+    for (int o = LANES / 2; o > 0; o >>= 1) s += __shfl_xor(s, o, TW_WAVE);
+    if (l == 0) rinv[threadIdx.x / LANES] = 1.0f / sqrtf(s / n.width + n.eps);
+  }
+};
+
+// =====================================================================================
 // Skinny kernel (M <= 16*MT rows), workgroup-cooperative. The WAVES (4, or 2) waves of a workgroup own
 // neighbouring tiles of 16 output columns and the SAME K range. Per stage of U
 // MFMA steps the workgroup copies the activations' K slice [16*MT rows][U*64 B]
@@ -49,14 +86,17 @@ __device__ __forceinline__ size_t tw_shuffled_chunk(int n, int c, int k_steps, i
 // GLU (splits == 1 only): the workgroup's tiles are gate, up(, gate, up); C gets half as many columns.
 // WAVES = 2 halves the workgroups' size and doubles their number: used where that spreads them more
 // evenly over the CUs (the kernel's time is that of the fullest CU).
-template <typename T, typename OutT, int MT, int U, int WAVES, bool PARTIAL, bool SHUF, bool GLU>
+// In: RowNorms (MT == 1) where A's rows are to be multiplied by their norms' factors, see above.
+template <typename T, typename OutT, int MT, int U, int WAVES, bool PARTIAL, bool SHUF, bool GLU, class In = RowsAsTheyAre>
 __global__ __launch_bounds__(WAVES * 64) void gemm_skinny_lds_kernel(const T* __restrict__ A, long lda,
                                                               const T* __restrict__ W, long ldw,
                                                               const float* __restrict__ bias,
                                                               const float* residual, long ldr, OutT* C,
                                                               long ldc, float* __restrict__ partial, int M,
-                                                              int N, int K, int n_groups, int splits) {
+                                                              int N, int K, int n_groups, int splits, In norms) {
   typedef typename Elem<T>::Frag Frag;
+  constexpr bool NORMED = std::is_same<In, RowNorms>::value;
+  static_assert(!NORMED || MT == 1, "norms travel with up to 16 rows");
   constexpr int EPF = Elem<T>::kPerFrag;
   constexpr int XROW = TW_XROW(U);
   constexpr int XSTAGE = MT * 16 * XROW;
@@ -152,10 +192,24 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_skinny_lds_kernel(const T* __
     __syncthreads();
   };
 
+  __shared__ float rinv[16];
+  RowNormLoads<THREADS> norm_sums;
+  if constexpr (NORMED) norm_sums.request(norms, M);
   if (n_stages > 0) {
     load_x(step_begin);
     load_w(0, step_begin);
+    // (of two waves, whose lanes hold 32 registers of sums, the second stage's weights go out behind the sums: with both it takes 138
+    // registers, and three waves a SIMD run instead of four)
+    if constexpr (NORMED && WAVES == 2) {
+      __builtin_amdgcn_sched_barrier(0);
+      norm_sums.finish(norms, rinv);
+      __builtin_amdgcn_sched_barrier(0);
+    }
     if (n_stages > 1) load_w(1, step_begin + U);
+    if constexpr (NORMED && WAVES != 2) {
+      __builtin_amdgcn_sched_barrier(0);
+      norm_sums.finish(norms, rinv);
+    }
     store_x(0, step_begin);
     __syncthreads();
     int i = 0;
@@ -164,6 +218,10 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_skinny_lds_kernel(const T* __
   }
 
   // acc[mt][j] = sum_k W[n0 + 4g + j][k] * A[16 mt + r][k]
+  if constexpr (NORMED) {                                      // (a workgroup without a K range has sums of zero: any factor does)
+    const float f = n_stages > 0 ? rinv[r] : 1.f;
+    acc[0] = f32x4{acc[0][0] * f, acc[0][1] * f, acc[0][2] * f, acc[0][3] * f};
+  }
   if (GLU) {
     // the waves swap their tiles through LDS (every wave is past its last LDS read: the loop
     // ends with a barrier), then each thread forms outputs from a (gate, up) pair
@@ -505,23 +563,78 @@ __global__ __launch_bounds__(TW_CU_WAVES * 64) void gemm_stream_cu_kernel(
 // above 4096 these cost more than they save).
 // =====================================================================================
 // ACT: the residual's stride names an activation (a form of its own: its code in the plain form cost that 0.15 us a launch).
-template <typename T, typename OutT, int WAVES, bool GLU, bool ACT = false>
+// In: RowNorms where A's rows are to be multiplied by their norms' factors.
+// End: what the epilogue does with a finished element.
+//   EndPlain   C = sum (+ bias) (+ residual), or act(sum + bias).
+//   EndLeave   C (float32, the residual stream) = sum + bias + residual, and beside it what a norm that travels needs: the rows times
+//              the next norm's weight in T (times a second weight too where two norms read the stream), and each 16 columns' sum of
+//              squares. AFTER: the stream itself is such a normed row, C = alpha * residual * rinv * before_weight + scale * (sum + bias).
+//   EndRotate  the packed product of queries, keys and values: q and k are rotated, q goes to C, k and v to the cache's pages. A
+//              workgroup's 16 columns are then eight of a head's first rotated half and the eight they turn with (each eight weight
+//              rows of a fragment are a cache line, so the loads are as wide as before), so that no other kernel has to bring the
+//              two halves together: it was 2.5 to 4 us behind every such product.
+struct EndPlain {};
+template <bool AFTER_NORM>
+struct EndLeave {
+  static constexpr bool AFTER = AFTER_NORM;
+  const float *weight, *weight2;       // [N]; weight2 may be null
+  void *rows, *rows2;                  // [M][N] in the input type
+  float* sums;                         // [M][N / 16]
+  RowNorms before;                     // AFTER: of the residual's rows (sums null: they are as they are)
+  const float *before_weight, *scale;  // AFTER: [N]; scale may be null
+  float alpha;
+};
+struct EndRotate {
+  const float *cos_t, *sin_t;          // [M][rot / 2]
+  const int* slots;
+  void *keys, *values;
+  int q_heads, kv_heads, head_dim, rot, page_size, write_cache, adjacent;
+};
+template <class End> struct IsLeave { static constexpr bool value = false, after = false; };
+template <bool A> struct IsLeave<EndLeave<A>> { static constexpr bool value = true, after = A; };
+
+template <typename T, typename OutT, int WAVES, bool GLU, bool ACT = false, class In = RowsAsTheyAre, class End = EndPlain>
 __global__ __launch_bounds__(WAVES * 64) void gemm_narrow_kernel(const T* __restrict__ A, long lda,
                                                                  const T* __restrict__ W, long ldw,
                                                                  const float* __restrict__ bias,
                                                                  const float* residual, long ldr, OutT* C, long ldc,
-                                                                 int M, int N, int K) {
+                                                                 int M, int N, int K, In norms, End end) {
   typedef typename Elem<T>::Frag Frag;
+  constexpr bool NORMED = std::is_same<In, RowNorms>::value, ROTATE = std::is_same<End, EndRotate>::value;
+  constexpr bool LEAVE = IsLeave<End>::value, AFTER = IsLeave<End>::after;
+  static_assert(!(GLU && (ROTATE || LEAVE)), "the gated form finishes plain outputs");
   constexpr int EPF = Elem<T>::kPerFrag, U = 4, NT = GLU ? 2 : 1;
   __shared__ float sums[NT * WAVES * 16 * 16];
+  __shared__ float rinv[16], rinv_before[16];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int r = lane & 15, g = lane >> 4;
   const int chunks = K / EPF, steps = (chunks + 3) / 4;
   const int mine = steps > wave ? (steps - wave + WAVES - 1) / WAVES : 0;      // this wave's steps
+  // the column of the workgroup's place i (of 16): consecutive, or eight and the eight that turn with them
+  int first = blockIdx.x * 16, apart = 0;
+  bool turns = false;                                                           // does this workgroup's part of a head turn?
+  if constexpr (ROTATE) {
+    const int per_head = end.head_dim / 16, head = blockIdx.x / per_head, t = blockIdx.x % per_head;
+    turns = head < end.q_heads + end.kv_heads && t < end.rot / 16;
+    if (turns && !end.adjacent) {
+      first = head * end.head_dim + 8 * t;
+      apart = end.rot / 2 - 8;
+    }
+  }
+  auto column = [&](int i) { return first + i + (i >= 8 ? apart : 0); };
   const T* w_base = W + ((size_t)blockIdx.x * NT * ldw * 64 + lane) * EPF;
+  if constexpr (ROTATE) {
+    const int n = column(r);
+    w_base = W + ((size_t)(n >> 4) * ldw * 64 + g * 16 + (n & 15)) * EPF;
+  }
   const size_t w_tile = (size_t)ldw * 64 * EPF;
   const T* x_base = A + (size_t)min(r, M - 1) * lda;                            // (rows past M: never stored)
 
+  RowNormLoads<WAVES * 64> norm_sums, before_sums;
+  if constexpr (NORMED) norm_sums.request(norms, M);
+  if constexpr (AFTER) {
+    if (end.before.sums) before_sums.request(end.before, M);
+  }
   // Loads carry no predicate: steps are clamped to the last one and chunks to the last chunk, and activations
   // past either are replaced by zeros before the product.
   Frag wf[2][NT][U], xf[2][U];
@@ -550,12 +663,41 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_narrow_kernel(const T* __rest
   load(0, 0);
   load(1, U);
   // what the epilogue adds, requested behind the first weights: thread t < 256 finishes row t / 16, column t % 16
-  const int row = tid >> 4, c = tid & 15, col = blockIdx.x * 16 + c;
+  const int row = tid >> 4, c = tid & 15, col = ROTATE ? column(c) : blockIdx.x * 16 + c;
   const bool store = row < M && col < N / NT;
   float add[NT], res = 0.f;
 #pragma unroll
-  for (int t = 0; t < NT; ++t) add[t] = store && bias ? bias[(blockIdx.x * NT + t) * 16 + c] : 0.f;
+  for (int t = 0; t < NT; ++t) add[t] = store && bias ? bias[ROTATE ? col : (blockIdx.x * NT + t) * 16 + c] : 0.f;
   if (!GLU && store && residual) res = residual[(size_t)row * ldr + col];
+  float weight = 0.f, weight2 = 0.f, before_weight = 0.f, scale = 1.f;
+  if constexpr (LEAVE) {
+    if (store) {
+      weight = end.weight[col];
+      if (end.weight2) weight2 = end.weight2[col];
+      if constexpr (AFTER) {
+        if (end.before.sums) before_weight = end.before_weight[col];
+        if (end.scale) scale = end.scale[col];
+      }
+    }
+  }
+  float turn_cos = 1.f, turn_sin = 0.f;
+  int slot = -1;
+  if constexpr (ROTATE) {
+    if (store) {
+      if (end.write_cache) slot = end.slots[row];
+      if (turns) {
+        const int in_head = (end.adjacent ? col : first + (c & 7)) % end.head_dim;
+        const int pair = end.adjacent ? in_head >> 1 : in_head;
+        turn_cos = end.cos_t[(size_t)row * (end.rot / 2) + pair];
+        turn_sin = end.sin_t[(size_t)row * (end.rot / 2) + pair];
+      }
+    }
+  }
+  if constexpr (NORMED || AFTER) __builtin_amdgcn_sched_barrier(0);
+  if constexpr (NORMED) norm_sums.finish(norms, rinv);
+  if constexpr (AFTER) {
+    if (end.before.sums) before_sums.finish(end.before, rinv_before);
+  }
   for (int i = 0; i < mine; i += 2 * U) {
     multiply(0, i);
     if (i + 2 * U < mine) load(0, i + 2 * U);
@@ -573,17 +715,54 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_narrow_kernel(const T* __rest
 #pragma unroll
     for (int j = 0; j < 4; ++j) sums[((t * WAVES + wave) * 16 + r) * 16 + ((4 * g + j) ^ r)] = acc[t][j];
   __syncthreads();
-  if (!store) return;
+  if (!store) return;                                          // (LEAVE, ROTATE: N is a multiple of 16, so a row's 16 lanes stay or go together)
   float v[NT];
 #pragma unroll
   for (int t = 0; t < NT; ++t) {
     v[t] = 0.f;
 #pragma unroll
     for (int w = 0; w < WAVES; ++w) v[t] += sums[((t * WAVES + w) * 16 + row) * 16 + (c ^ row)];
+    if constexpr (NORMED) v[t] *= rinv[row];
     v[t] += add[t];
   }
   if constexpr (GLU) {
     C[(size_t)row * ldc + col] = tw_from_float<OutT>(tw_glu(v[0], v[1], ldr));
+  } else if constexpr (LEAVE) {
+    if constexpr (AFTER) {
+      v[0] *= scale;
+      if (end.before.sums) res = res * rinv_before[row] * before_weight;
+      res *= end.alpha;
+    }
+    const float x = v[0] + res;
+    C[(size_t)row * ldc + col] = x;
+    static_cast<T*>(end.rows)[(size_t)row * N + col] = tw_from_float<T>(x * weight);
+    if (end.weight2) static_cast<T*>(end.rows2)[(size_t)row * N + col] = tw_from_float<T>(x * weight2);
+    float sq = x * x;                                          // over the row's 16 lanes
+    sq += tw_dpp<TW_ROTATE_8>(sq);
+    sq += tw_dpp<TW_ROTATE_4>(sq);
+    sq += tw_dpp<TW_SWAP_2>(sq);
+    sq += tw_dpp<TW_SWAP_1>(sq);
+    if (c == 0) end.sums[(size_t)row * (N / 16) + blockIdx.x] = sq;
+  } else if constexpr (ROTATE) {
+    T out = tw_from_float<T>(v[0]);                            // what the product would have stored
+    if (turns) {
+      const float self = tw_to_float(out), other = end.adjacent ? tw_dpp<TW_SWAP_1>(self) : tw_dpp<TW_ROTATE_8>(self);
+      const bool high = end.adjacent ? c & 1 : c >= 8;
+      // (the products and sums of tw_rotate_pair in elementwise.hip, which round alike)
+      const float a = __fmaf_rn(self, turn_cos, -__fmul_rn(other, turn_sin)), b = __fmaf_rn(self, turn_cos, __fmul_rn(other, turn_sin));
+      out = tw_from_float<T>(high ? b : a);
+    }
+    const int head = blockIdx.x / (end.head_dim / 16), d = col - head * end.head_dim;
+    if (head < end.q_heads) {
+      C[(size_t)row * ldc + col] = out;
+    } else if (slot >= 0) {
+      const size_t page = slot / end.page_size;
+      const int off = slot % end.page_size, kh = (head - end.q_heads) % end.kv_heads;
+      if (head < end.q_heads + end.kv_heads)
+        static_cast<T*>(end.keys)[((page * end.kv_heads + kh) * end.page_size + off) * end.head_dim + d] = out;
+      else
+        static_cast<T*>(end.values)[((page * end.kv_heads + kh) * end.head_dim + d) * end.page_size + off] = out;
+    }
   } else {
     if constexpr (ACT) v[0] = tw_act(v[0], ldr);
     else if (residual) v[0] += res;
@@ -724,10 +903,10 @@ static double cu_imbalance(long workgroups) {
   return workgroups <= 256 ? 1.0 : (double)tw_div_up(workgroups, 256) * 256.0 / (double)workgroups;
 }
 
-template <typename T, typename OutT, int MT, bool PARTIAL, bool SHUF, bool GLU>
+template <typename T, typename OutT, int MT, bool PARTIAL, bool SHUF, bool GLU, class In = RowsAsTheyAre>
 static int launch_skinny_lds(const T* A, long lda, const T* W, long ldw, const float* bias,
                              const float* residual, long ldr, OutT* C, long ldc, float* partial,
-                             long partial_bytes, int M, int N, int K, hipStream_t stream) {
+                             long partial_bytes, int M, int N, int K, hipStream_t stream, In norms = In{}) {
   constexpr int EPF = Elem<T>::kPerFrag;
   constexpr int U = MT == 1 ? 8 : 4;
   int splits = GLU ? 1 : skinny_lds_splits(N, K, EPF);
@@ -743,14 +922,14 @@ static int launch_skinny_lds(const T* A, long lda, const T* W, long ldw, const f
   if constexpr (MT == 1 && !PARTIAL) {
     if (splits == 1 && cu_imbalance(tw_div_up(N, 32)) < cu_imbalance(tw_div_up(N, 64)) - 0.03) {
       const int groups = tw_div_up(N, 32);
-      gemm_skinny_lds_kernel<T, OutT, MT, U, 2, PARTIAL, SHUF, GLU><<<groups, 128, 0, stream>>>(
-          A, lda, W, ldw, bias, residual, ldr, C, ldc, partial, M, N, K, groups, 1);
+      gemm_skinny_lds_kernel<T, OutT, MT, U, 2, PARTIAL, SHUF, GLU, In><<<groups, 128, 0, stream>>>(
+          A, lda, W, ldw, bias, residual, ldr, C, ldc, partial, M, N, K, groups, 1, norms);
       return TW_LAUNCH_RESULT();
     }
   }
   const int groups = tw_div_up(N, 64);
-  gemm_skinny_lds_kernel<T, OutT, MT, U, 4, PARTIAL, SHUF, GLU><<<groups * splits, 256, 0, stream>>>(
-      A, lda, W, ldw, bias, residual, ldr, C, ldc, partial, M, N, K, groups, splits);
+  gemm_skinny_lds_kernel<T, OutT, MT, U, 4, PARTIAL, SHUF, GLU, In><<<groups * splits, 256, 0, stream>>>(
+      A, lda, W, ldw, bias, residual, ldr, C, ldc, partial, M, N, K, groups, splits, norms);
   int err = TW_LAUNCH_RESULT();
   if (err || splits == 1 || PARTIAL) return err;
   return launch_splitk_reduce<OutT>(partial, splits, bias, residual, ldr, C, ldc, M, N, stream);
@@ -878,13 +1057,13 @@ static double narrow_us(int M, int N, int K, int epf, bool glu) {
   const double memory = 1e-6 * N * (double)K * size / (size == 2 ? 6.57 : 6.14);
   return (size == 2 ? (glu ? 2.66 : 2.80) : glu ? 2.81 : 2.97) + sqrt(sqrt(cu * cu * cu * cu + memory * memory * memory * memory));
 }
-static double skinny_us(int M, int N, int K, int epf, bool glu) {
+static double skinny_us(int M, int N, int K, int epf, bool glu, bool reduced = true) {
   const int size = 16 / epf, steps = tw_div_up(K / epf, 4), splits = glu ? 1 : skinny_lds_splits(N, K, epf);
   const double fill = tw_div_up(N, 64) * splits / 512.0;
   const double step = size == 2 ? (glu ? 0.0918 + 0.0005 * M : 0.0715 + 0.0014 * M) : glu ? 0.1101 + 0.0002 * M : 0.0589 + 0.0017 * M;
   const double cu = tw_div_up(steps, splits) * step * (fill > 1 ? fill : 1.0);
   const double memory = 1e-6 * N * (double)K * size / (size == 2 ? 6.57 : 6.4);
-  return (size == 2 ? (glu ? 2.99 : 3.62) : glu ? 3.29 : 4.31) + (splits > 1 ? (size == 2 ? 1.95 + 0.74e-6 * 4 * splits * M * N : 2.22 + 0.67e-6 * 4 * splits * M * N) : 0.0) +
+  return (size == 2 ? (glu ? 2.99 : 3.62) : glu ? 3.29 : 4.31) + (splits > 1 && reduced ? (size == 2 ? 1.95 + 0.74e-6 * 4 * splits * M * N : 2.22 + 0.67e-6 * 4 * splits * M * N) : 0.0) +
          sqrt(sqrt(cu * cu * cu * cu + memory * memory * memory * memory));
 }
 
@@ -907,6 +1086,17 @@ static bool narrow_pays(int M, int N, int K, int epf, bool glu, bool sums) {
   return beyond && steps >= 28 && narrow_us(M, N, K, epf, glu) < (epf == 4 ? 0.93 : 0.9) * skinny_us(M, N, K, epf, glu);
 }
 
+// Whole K a workgroup where its epilogue spares the kernel that would add the K ranges' sums up anyway: a norm (EndLeave) or the
+// rotation and cache write (EndRotate), LAUNCH microseconds as a node of a captured step. (Four layers and a head, captured steps, us:
+// neither / norms that travel / rotation too, at 1, 8 and 16 rows: 896 wide with down products of 4,864 174 / 162 / 155, 188 / 180 / 172, 203 / 195 / 187;
+// 2,048 wide, 11,008: 318 / 303 / 295, 338 / 326 / 316, 363 / 351 / 342; 3,584 wide, 18,944, 1 and 8 rows: 584 / 559 / 561, 629 / 618 / 618. The
+// down products of the last at 8 rows, 3.4 us behind by estimate, gain 6 us a step; those of 2,048 x 11,008 at 4, 3 behind, 2.)
+static bool narrow_end_pays(int M, int N, int K, int epf, double launch) {
+  return M >= 1 && M <= 16 && N % 64 == 0 && K % epf == 0 && narrow_us(M, N, K, epf, false) < skinny_us(M, N, K, epf, false, false) + launch;
+}
+#define TW_LEAVE_SPARES_US 3.5
+#define TW_ROTATE_SPARES_US 1.5
+
 // A plain product with an activation behind it, against the K ranges' sums and a kernel that adds them up and applies it (bf16, in a
 // captured graph, cold weights): 4096 x 2048 1 / 8 / 16 rows 7.6 / 4.2, 7.9 / 4.6, 8.5 / 5.2; 5632 x 2048 9.0 / 5.8, 9.5 / 6.6, 10.4 / 7.9;
 // 8192 x 3072 12.5 / 9.1, 12.9 / 10.1, 13.6 / 12.3; 11264 x 2048 12.5 / 8.7, 13.1 / 9.3, 14.2 / 11.5.
@@ -916,16 +1106,16 @@ static bool narrow_act_pays(int M, int N, int K, int epf) {
 
 // Waves a workgroup: as few as have a wave's whole share of K in flight at once (8 k-steps), up to 16. (2048 x 1024, 8
 // rows: 4 / 8 / 16 waves 3.5 / 4.0 / 5.6 us; 2048 x 2048: 5.2 / 4.4 / 5.9; 2048 x 4096: 8.1 / 6.7 / 6.5)
-template <typename T, typename OutT, bool GLU, bool ACT = false>
+template <typename T, typename OutT, bool GLU, bool ACT = false, class In = RowsAsTheyAre, class End = EndPlain>
 static int launch_narrow(const T* A, long lda, const T* W, long ldw, const float* bias, const float* residual, long ldr,
-                         OutT* C, long ldc, int M, int N, int K, hipStream_t stream) {
+                         OutT* C, long ldc, int M, int N, int K, hipStream_t stream, In norms = In{}, End end = End{}) {
   const int steps = tw_div_up(K / Elem<T>::kPerFrag, 4), groups = GLU ? N / 32 : tw_div_up(N, 16);
   if (steps <= 48)
-    gemm_narrow_kernel<T, OutT, 4, GLU, ACT><<<groups, 256, 0, stream>>>(A, lda, W, ldw, bias, residual, ldr, C, ldc, M, N, K);
+    gemm_narrow_kernel<T, OutT, 4, GLU, ACT, In, End><<<groups, 256, 0, stream>>>(A, lda, W, ldw, bias, residual, ldr, C, ldc, M, N, K, norms, end);
   else if (steps <= 96)
-    gemm_narrow_kernel<T, OutT, 8, GLU, ACT><<<groups, 512, 0, stream>>>(A, lda, W, ldw, bias, residual, ldr, C, ldc, M, N, K);
+    gemm_narrow_kernel<T, OutT, 8, GLU, ACT, In, End><<<groups, 512, 0, stream>>>(A, lda, W, ldw, bias, residual, ldr, C, ldc, M, N, K, norms, end);
   else
-    gemm_narrow_kernel<T, OutT, 16, GLU, ACT><<<groups, 1024, 0, stream>>>(A, lda, W, ldw, bias, residual, ldr, C, ldc, M, N, K);
+    gemm_narrow_kernel<T, OutT, 16, GLU, ACT, In, End><<<groups, 1024, 0, stream>>>(A, lda, W, ldw, bias, residual, ldr, C, ldc, M, N, K, norms, end);
   return TW_LAUNCH_RESULT();
 }
 
@@ -1126,4 +1316,117 @@ extern "C" int tw_linear_partials(int dtype, const void* A, long lda, const void
   if (dtype == TW_DTYPE_BF16)
     return partials_layout<bf16_t>(shuffled, (const bf16_t*)A, lda, (const bf16_t*)W, ldw, partial, partial_bytes, M, N, K, stream);
   return TW_ERR_BAD_ARGUMENT;
+}
+
+// ---- up to 16 rows of shuffled weights, norms that travel ----------------------------------------------------------
+static bool few_rows_ok(int dtype, const void* A, long lda, const void* W, long ldw, int M, int N, int K) {
+  const int epf = dtype == TW_DTYPE_F32 ? 4 : 8;
+  return (dtype == TW_DTYPE_F32 || dtype == TW_DTYPE_BF16) && M >= 1 && M <= 16 && N > 0 && K > 0 && lda >= K && K % epf == 0 && lda % epf == 0 &&
+         weight_layout_ok(dtype, 1, ldw, K) && (uintptr_t)A % 16 == 0 && (uintptr_t)W % 16 == 0;
+}
+static bool norms_ok(const float* sums, int count, float eps) {
+  return sums != nullptr && (uintptr_t)sums % 16 == 0 && count > 0 && count % 4 == 0 && count <= TW_NORM_MAX_SUMS && eps > 0.f;
+}
+
+template <typename T>
+static int linear_normed(int mode, int out_f32, const T* A, long lda, RowNorms norms, const T* W, long ldw, const float* bias, void* C,
+                         long ldc, float* partial, long partial_bytes, int M, int N, int K, long code, hipStream_t stream) {
+  constexpr int EPF = Elem<T>::kPerFrag;
+  if (mode == 1) {                                             // K ranges' sums, as tw_linear_partials
+    if (narrow_pays(M, N, K, EPF, false, true)) {
+      TW_REQUIRE(partial != nullptr && partial_bytes >= (long)M * N * 4);
+      return launch_narrow<T, float, false, false, RowNorms>(A, lda, W, ldw, nullptr, nullptr, 0, partial, N, M, N, K, stream, norms);
+    }
+    return launch_skinny_lds<T, float, 1, true, true, false, RowNorms>(A, lda, W, ldw, nullptr, nullptr, 0, (float*)nullptr, N, partial,
+                                                                      partial_bytes, M, N, K, stream, norms);
+  }
+  if (mode == 2) {                                             // gated, as tw_linear_glu
+    TW_REQUIRE(N % 32 == 0);
+    if (narrow_pays(M, N, K, EPF, true, false))
+      return launch_narrow<T, T, true, false, RowNorms>(A, lda, W, ldw, bias, nullptr, code, (T*)C, ldc, M, N, K, stream, norms);
+    return launch_skinny_lds<T, T, 1, false, true, true, RowNorms>(A, lda, W, ldw, bias, nullptr, code, (T*)C, ldc, nullptr, 0, M, N, K, stream, norms);
+  }
+  if (mode == 3)                                               // with an activation, as tw_linear_act_few
+    return launch_narrow<T, T, false, true, RowNorms>(A, lda, W, ldw, bias, nullptr, code, (T*)C, ldc, M, N, K, stream, norms);
+  const bool narrow = narrow_pays(M, N, K, EPF, false, false);
+  auto plain = [&](auto* out) {
+    typedef std::remove_reference_t<decltype(*out)> OutT;
+    if (narrow) return launch_narrow<T, OutT, false, false, RowNorms>(A, lda, W, ldw, bias, nullptr, 0, out, ldc, M, N, K, stream, norms);
+    return launch_skinny_lds<T, OutT, 1, false, true, false, RowNorms>(A, lda, W, ldw, bias, nullptr, 0, out, ldc, partial, partial_bytes, M, N, K,
+                                                                      stream, norms);
+  };
+  return out_f32 ? plain((float*)C) : plain((T*)C);
+}
+
+// The products of up to 16 rows whose norms travel (see RowNorms): A holds x * w rounded, sums [M][count] their sums of squares over
+// `width` elements. mode 0: C = product (+ bias), float32 or the input type; 1: partial = the K ranges' sums, as tw_linear_partials;
+// 2: the gated form, act and factor as tw_linear_glu; 3: C = act(product + bias), as tw_linear_act_few.
+extern "C" int tw_linear_normed(int dtype, int mode, int out_f32, const void* A, long lda, const float* sums, int count, int width, float eps,
+                                const void* W, long ldw, const float* bias, void* C, long ldc, float* partial, long partial_bytes, int M,
+                                int N, int K, int act, float factor, hipStream_t stream) {
+  TW_REQUIRE(mode >= 0 && mode <= 3 && few_rows_ok(dtype, A, lda, W, ldw, M, N, K) && norms_ok(sums, count, eps) && width > 0);
+  TW_REQUIRE(mode == 1 || (C != nullptr && ldc >= (mode == 2 ? N / 2 : N)));
+  TW_REQUIRE(mode != 2 || act == TW_GLU_SILU || act == TW_GLU_GELU_TANH || act == TW_GLU_SWISH_LIMITED);
+  TW_REQUIRE(mode != 3 || act == TW_ACT_RELU_SQUARED || act == TW_ACT_GELU_ERF);
+  const long code = mode == 2 ? tw_glu_code(act, factor) : act;
+  const RowNorms norms = {sums, count, (float)width, eps};
+  if (dtype == TW_DTYPE_F32)
+    return linear_normed<float>(mode, 1, (const float*)A, lda, norms, (const float*)W, ldw, bias, C, ldc, partial, partial_bytes, M, N, K, code, stream);
+  return linear_normed<bf16_t>(mode, out_f32, (const bf16_t*)A, lda, norms, (const bf16_t*)W, ldw, bias, C, ldc, partial, partial_bytes, M, N, K, code, stream);
+}
+
+extern "C" int tw_linear_leave_pays(int dtype, int M, int N, int K) {
+  const int epf = dtype == TW_DTYPE_F32 ? 4 : 8;
+  return N > 0 && K > 0 && N / 16 <= TW_NORM_MAX_SUMS && narrow_end_pays(M, N, K, epf, TW_LEAVE_SPARES_US) ? 1 : 0;
+}
+
+// C [M][N] (float32) += A W^T (+ bias), and what a norm of the new rows needs to travel: rows = C * weight (rows2 = C * weight2, or null)
+// in the input type, sums [M][N / 16]. after != 0: C <- alpha * (C * rinv * before_weight) + scale * (A W^T + bias), the old rows' rinv from
+// before_sums [M][N / 16] over N elements (null: C as it is); these must not be `sums`.
+extern "C" int tw_linear_leave(int dtype, const void* A, long lda, const void* W, long ldw, const float* bias, float* C, long ldc, int M, int N,
+                               int K, const float* weight, void* rows, const float* weight2, void* rows2, float* sums, int after,
+                               const float* before_sums, const float* before_weight, const float* scale, float alpha, float eps,
+                               hipStream_t stream) {
+  TW_REQUIRE(few_rows_ok(dtype, A, lda, W, ldw, M, N, K) && C != nullptr && ldc >= N && N % 64 == 0 && N / 16 <= TW_NORM_MAX_SUMS);
+  TW_REQUIRE(weight && rows && sums && (weight2 == nullptr) == (rows2 == nullptr));
+  TW_REQUIRE(before_sums == nullptr || (after && before_weight && before_sums != sums && norms_ok(before_sums, N / 16, eps)));
+  auto run = [&](auto t, auto end) {
+    typedef decltype(t) T;
+    return launch_narrow<T, float, false, false, RowsAsTheyAre>((const T*)A, lda, (const T*)W, ldw, bias, C, ldc, C, ldc, M, N, K, stream,
+                                                                RowsAsTheyAre{}, end);
+  };
+  const RowNorms before = {before_sums, N / 16, (float)N, eps};
+  const EndLeave<true> with = {weight, weight2, rows, rows2, sums, before, before_weight, scale, alpha};
+  const EndLeave<false> without = {weight, weight2, rows, rows2, sums, before, nullptr, nullptr, 1.f};
+  if (dtype == TW_DTYPE_F32) return after ? run(float{}, with) : run(float{}, without);
+  return after ? run(bf16_t{}, with) : run(bf16_t{}, without);
+}
+
+extern "C" int tw_linear_rotate_pays(int dtype, int M, int N, int K) {
+  const int epf = dtype == TW_DTYPE_F32 ? 4 : 8;
+  return N > 0 && K > 0 && narrow_end_pays(M, N, K, epf, TW_ROTATE_SPARES_US) ? 1 : 0;
+}
+
+// The packed product of queries, keys and values of up to 16 rows, finished as tw_rope_kv_write finishes it: qkv [M][ld] = round(A W^T +
+// bias), q rotated in place; rotated k and v to the pages of the rows' slots (write_cache; the k and v columns of qkv are not written).
+// sums: null, or the rows' norms as tw_linear_normed. rot: a multiple of 16.
+extern "C" int tw_linear_rotate(int dtype, const void* A, long lda, const float* sums, int count, int width, float eps, const void* W, long ldw,
+                                const float* bias, void* qkv, long ld, int M, int K, const float* cos_t, const float* sin_t, const int* slots,
+                                void* keys, void* values, int q_heads, int kv_heads, int head_dim, int rot, int page_size, int write_cache,
+                                int adjacent, hipStream_t stream) {
+  TW_REQUIRE(q_heads > 0 && kv_heads > 0 && head_dim > 0 && head_dim % 16 == 0 && page_size > 0);
+  const int N = (q_heads + 2 * kv_heads) * head_dim;
+  TW_REQUIRE(few_rows_ok(dtype, A, lda, W, ldw, M, N, K) && qkv != nullptr && ld >= N && rot >= 0 && rot % 16 == 0 && rot <= head_dim);
+  TW_REQUIRE(rot == 0 || (cos_t && sin_t));
+  TW_REQUIRE(!write_cache || (slots && keys && values));
+  TW_REQUIRE(sums == nullptr || (norms_ok(sums, count, eps) && width > 0));
+  const EndRotate end = {cos_t, sin_t, slots, keys, values, q_heads, kv_heads, head_dim, rot, page_size, write_cache, adjacent};
+  auto run = [&](auto t, auto norms) {
+    typedef decltype(t) T;
+    return launch_narrow<T, T, false, false, decltype(norms)>((const T*)A, lda, (const T*)W, ldw, bias, nullptr, 0, (T*)qkv, ld, M, N, K, stream,
+                                                              norms, end);
+  };
+  const RowNorms norms = {sums, count, (float)width, eps};
+  if (dtype == TW_DTYPE_F32) return sums ? run(float{}, norms) : run(float{}, RowsAsTheyAre{});
+  return sums ? run(bf16_t{}, norms) : run(bf16_t{}, RowsAsTheyAre{});
 }

@@ -17,6 +17,7 @@ struct ResidualNormArgs {
   void* out;                // [n][hidden], compute type, or null
   int hidden;
   float alpha, eps;
+  const float* before;      // [hidden] or null: x stands for before * unit(x) (few rows: the kernel of four consecutive elements)
 };
 
 // Four columns of split-K partial sums, `stride` apart, requested up to eight at a time and added in index order. (Four, two and
@@ -94,6 +95,21 @@ __global__ __launch_bounds__(1024) void residual_norm_vec4_kernel(ResidualNormAr
     if (EARLY && a.scale) sv[i] = *reinterpret_cast<const f32x4*>(a.scale + 4 * c);
   }
   float ss = 0.f;
+  if (EARLY && a.before) {
+    f32x4 bv[PER];
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+      bv[i] = *reinterpret_cast<const f32x4*>(a.before + 4 * min((int)(threadIdx.x + i * blockDim.x), chunks - 1));
+      if (threadIdx.x + i * blockDim.x < chunks) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) ss = __fmaf_rn(xv[i][e], xv[i][e], ss);
+      }
+    }
+    const float unit = 1.f / sqrtf(tw_block_sum(ss, lds) / (float)a.hidden + a.eps);
+#pragma unroll
+    for (int i = 0; i < PER; ++i) xv[i] = f32x4{xv[i][0] * unit * bv[i][0], xv[i][1] * unit * bv[i][1], xv[i][2] * unit * bv[i][2], xv[i][3] * unit * bv[i][3]};
+    ss = 0.f;
+  }
 #pragma unroll
   for (int i = 0; i < PER; ++i) {
     const int c = min((int)(threadIdx.x + i * blockDim.x), chunks - 1);
@@ -155,12 +171,16 @@ __global__ void residual_norm_kernel(ResidualNormArgs a) {
   }
 }
 
+static bool residual_rows_aligned(const ResidualNormArgs& a) {
+  return a.hidden % 4 == 0 && (uintptr_t)a.x % 16 == 0 && (uintptr_t)a.w % 16 == 0 &&
+         (!a.y || ((uintptr_t)a.y % 16 == 0 && a.ldy % 4 == 0)) &&
+         (!a.add || ((uintptr_t)a.add % 16 == 0 && a.add_stride % 4 == 0)) &&
+         (!a.scale || (uintptr_t)a.scale % 16 == 0);
+}
+
 template <typename T>
 static void residual_norm_launch(const ResidualNormArgs& a, int n, hipStream_t stream) {
-  const bool aligned = a.hidden % 4 == 0 && (uintptr_t)a.x % 16 == 0 && (uintptr_t)a.w % 16 == 0 &&
-                       (!a.y || ((uintptr_t)a.y % 16 == 0 && a.ldy % 4 == 0)) &&
-                       (!a.add || ((uintptr_t)a.add % 16 == 0 && a.add_stride % 4 == 0)) &&
-                       (!a.scale || (uintptr_t)a.scale % 16 == 0);
+  const bool aligned = residual_rows_aligned(a);
   const int chunks = a.hidden / 4;
   if (aligned && chunks <= 4096) {
     const int per = chunks <= 1024 ? 1 : (chunks <= 2048 ? 2 : 4);
@@ -180,12 +200,13 @@ static void residual_norm_launch(const ResidualNormArgs& a, int n, hipStream_t s
 
 extern "C" int tw_residual_norm(int out_dtype, float* x, const float* y, long ldy, const float* add, int splits,
                                 long add_stride, const float* scale, const float* w, void* out, int n, int hidden,
-                                float alpha, float eps, hipStream_t stream) {
+                                float alpha, float eps, const float* before, hipStream_t stream) {
   TW_REQUIRE(x && w && n >= 0 && hidden > 0 && eps > 0.f);
   TW_REQUIRE(add == nullptr || (splits > 0 && add_stride >= (long)n * hidden));
   TW_REQUIRE(y == nullptr || ldy >= hidden);
   if (n == 0) return 0;
-  ResidualNormArgs a{x, add ? nullptr : y, ldy, add, splits, (size_t)add_stride, scale, w, out, hidden, alpha, eps};
+  ResidualNormArgs a{x, add ? nullptr : y, ldy, add, splits, (size_t)add_stride, scale, w, out, hidden, alpha, eps, before};
+  TW_REQUIRE(!before || (n <= TW_EARLY_ROWS && residual_rows_aligned(a) && (uintptr_t)before % 16 == 0 && hidden <= 4 * 4096));
   if (out_dtype == TW_DTYPE_BF16) residual_norm_launch<bf16_t>(a, n, stream);
   else if (out_dtype == TW_DTYPE_F32) residual_norm_launch<float>(a, n, stream);
   else return TW_ERR_BAD_ARGUMENT;

@@ -33,6 +33,11 @@ _SIGNATURES = {
     "tw_linear_act": (I, [I, P, L, P, L, I, P, P, L, P, L, I, I, I, I, P]),
     "tw_linear_act_few_pays": (I, [I, I, I, I]),
     "tw_linear_act_few": (I, [I, P, L, P, L, P, P, L, I, I, I, I, P]),
+    "tw_linear_normed": (I, [I, I, I, P, L, P, I, I, F, P, L, P, P, L, P, L, I, I, I, I, F, P]),
+    "tw_linear_leave_pays": (I, [I, I, I, I]),
+    "tw_linear_leave": (I, [I, P, L, P, L, P, P, L, I, I, I, P, P, P, P, P, I, P, P, P, F, F, P]),
+    "tw_linear_rotate_pays": (I, [I, I, I, I]),
+    "tw_linear_rotate": (I, [I, P, L, P, I, I, F, P, L, P, P, L, I, I, P, P, P, P, P, I, I, I, I, I, I, I, P]),
     "tw_attn_decode_splits": (I, [I, I, I, I]),
     "tw_attn_decode_workspace_floats": (L, [I, I, I, I]),
     "tw_attn_decode": (I, [I, P, L, P, P, P, I, P, P, I, I, P, L, P, L, I, I, I, I, I, I, F, F, I, I, P, P, I, P]),
@@ -55,7 +60,7 @@ _SIGNATURES = {
     "tw_attn_mixed_workspace_floats": (L, [I, I, I, I, I]),
     "tw_attn_mixed": (I, [I, P, L, P, P, P, I, P, P, I, I, I, P, L, P, P, P, P, L, I, I, I, I, I, I, I, F, F, I, P]),
     "tw_kv_store": (I, [I, P, L, I, I, P, P, P, I, I, I, I, I, P]),
-    "tw_residual_norm": (I, [I, P, P, L, P, I, L, P, P, P, I, I, F, F, P]),
+    "tw_residual_norm": (I, [I, P, P, L, P, I, L, P, P, P, I, I, F, F, P, P]),
     "tw_relu_squared": (I, [I, P, L, I, I, P, I, P]),
     "tw_embed_hashed": (I, [I, P, P, I, P, P, P, P, P, P, P, P, I, I, I, I, L, L, L, F, F, P, P, P]),
     "tw_latent_finish": (I, [I, P, L, I, I, I, P, P, P, P, L, P, L, I, I, I, I, P, P, P, I, I, I, I, I, I, I, F, P, I, P]),

@@ -398,6 +398,136 @@ def linear_act_few(x, weight, out, activation="relu_squared", bias=None):
     return out
 
 
+class NormedRows:
+    """Rows whose norm travels: rows [n, k] = x * w rounded to the compute type, sums float32 [n, k / 16] the sums of squares of x
+    over 16 columns each. norm(x) is a row times 1 / sqrt(sum / k + eps), a factor that the products of up to 16 rows
+    (`linear_normed`) apply to their float32 sums. norm: the part whose norm this is; second: the same stream behind another norm."""
+
+    def __init__(self, rows, sums, eps, norm=None, second=None):
+        self.rows, self.sums, self.eps, self.norm, self.second = rows, sums, float(eps), norm, second
+
+    @property
+    def shape(self):
+        return self.rows.shape
+
+
+def can_leave_norms(n, width):
+    """Can a norm over WIDTH columns of N rows travel with a product?"""
+    return 0 < n <= 16 and width % 64 == 0 and width <= 4096
+
+
+def _normed_args(x, k):
+    _need(isinstance(x, NormedRows) and x.sums.is_contiguous() and can_leave_norms(x.rows.shape[0], k)
+          and tuple(x.sums.shape) == (x.rows.shape[0], k // 16), "the rows' sums of squares must be [n, k / 16], n up to 16, k up to 4,096")
+    return _dev(x.sums, torch.float32, "sums"), k // 16, k, x.eps
+
+
+def linear_normed(x, weight, out=None, bias=None, partial=None, activation=None, factor=1.0, workspace=None):
+    """A product of `NormedRows` x with a shuffled weight: out = x @ weight.T (+ bias), float32 or x's type; with a gated `activation`
+    (GLU_ACTIVATIONS) as `linear_glu`, with another (LINEAR_ACTIVATIONS) as `linear_act_few`; with `partial` instead of
+    out the K ranges' sums, as `linear_partials`."""
+    m, k, lda = _rows(x.rows, "x")
+    n, k2, w_ptr, ldw, shuffled, w_dtype = _weight_args(weight)
+    _need(k == k2 and shuffled and x.rows.dtype == w_dtype, "linear_normed takes rows of a shuffled weight's type and width")
+    norms = _normed_args(x, k)
+    mode = 1 if partial is not None else 2 if activation in GLU_ACTIVATIONS else 3 if activation is not None else 0
+    act, ldc, out_ptr, out_f32, part_ptr, part_bytes = 0, 0, None, 0, None, 0
+    if mode == 1:
+        splits = linear_partial_splits_rows(weight, m, lda)
+        _need(partial.is_contiguous() and tuple(partial.shape) == (splits, m, n), f"partial must be [{splits}, {m}, {n}]")
+        part_ptr, part_bytes = _dev(partial, torch.float32, "partial"), partial.numel() * 4
+    else:
+        mo, no, ldc = _rows(out, "out")
+        _need(mo == m and no == (n // 2 if mode == 2 else n) and (mode != 2 or n % 32 == 0), "linear_normed shapes do not agree")
+        out_ptr, out_f32 = _dev(out), 1 if out.dtype == torch.float32 else 0
+        _need(out.dtype == w_dtype or (mode == 0 and out_f32), "out must be float32 (a plain product) or the input type")
+        if mode:
+            names = GLU_ACTIVATIONS if mode == 2 else LINEAR_ACTIVATIONS
+            _need(activation in names, f"activation must be one of {sorted(names)}")
+            act = names[activation]
+        if workspace is not None:
+            part_ptr, part_bytes = _dev(workspace), workspace.numel() * workspace.element_size()
+    _need(bias is None or (mode != 1 and bias.numel() == n and bias.is_contiguous()), "bias has the wrong size")
+    check(library().tw_linear_normed(dtype_id(w_dtype), mode, out_f32, _dev(x.rows), lda, *norms, w_ptr, ldw,
+                                     _dev(bias, torch.float32, "bias") if bias is not None else None, out_ptr, ldc, part_ptr, part_bytes,
+                                     m, n, k, act, float(factor), _stream()), "linear_normed")
+    return partial if mode == 1 else out
+
+
+def _few_rows_of_shuffled(x, weight):
+    rows = x.shape[0]
+    ld = x.stride(0) if rows > 1 else max(x.stride(0), x.shape[1])
+    return isinstance(weight, ShuffledWeight) and 0 < rows <= 16 and x.data_ptr() % 16 == 0 and ld % (16 // x.element_size()) == 0
+
+
+def linear_leave_pays(x, weight):
+    """Is `linear_leave` there for these operands, and faster than split-K sums with a norm kernel behind them?"""
+    return (_few_rows_of_shuffled(x, weight) and can_leave_norms(x.shape[0], weight.shape[0])
+            and bool(library().tw_linear_leave_pays(dtype_id(x.dtype), x.shape[0], *weight.shape)))
+
+
+def linear_leave(x, weight, stream, norm_weight, eps, rows, sums, bias=None, second=None, after=None):
+    """stream (float32 [m, n]) += x @ weight.T (+ bias), and what its norm needs to travel: rows = stream * norm_weight in x's
+    type, sums; returns the `NormedRows`. second = (weight, rows): a second norm of the same stream. after = (before, before_weight, alpha,
+    scale): the stream itself is the rows of a norm not yet applied (before: `NormedRows`, or None: it is as it is) and becomes
+    alpha * norm(stream) + scale * (x @ weight.T + bias)."""
+    m, k, lda = _rows(x, "x")
+    n, k2, w_ptr, ldw, shuffled, w_dtype = _weight_args(weight)
+    ms, ns, lds = _rows(stream, "stream")
+    _need(k == k2 and shuffled and x.dtype == w_dtype and (ms, ns) == (m, n) and can_leave_norms(m, n), "linear_leave shapes do not agree")
+    for r, w in [(rows, norm_weight)] + ([(second[1], second[0])] if second is not None else []):
+        _need(r.is_contiguous() and tuple(r.shape) == (m, n) and r.dtype == w_dtype and w.numel() == n and w.is_contiguous(), "the rows left must be [m, n] in x's type")
+    _need(sums.is_contiguous() and tuple(sums.shape) == (m, n // 16), "the sums of squares must be [m, n / 16]")
+    _need(bias is None or (bias.numel() == n and bias.is_contiguous()), "bias has the wrong size")
+    before, before_weight, alpha, scale = after if after is not None else (None, None, 1.0, None)
+    _need(scale is None or (scale.numel() == n and scale.is_contiguous()), "scale has the wrong size")
+    _need(before is None or (tuple(before.sums.shape) == (m, n // 16) and before.sums.is_contiguous() and before_weight.numel() == n
+                             and before.sums.data_ptr() != sums.data_ptr()), "the stream's own norm needs sums apart from those left")
+    f32 = torch.float32
+    check(library().tw_linear_leave(
+        dtype_id(w_dtype), _dev(x), lda, w_ptr, ldw, _dev(bias, f32, "bias") if bias is not None else None, _dev(stream, f32, "stream"), lds, m, n, k,
+        _dev(norm_weight, f32, "norm_weight"), _dev(rows), _dev(second[0], f32, "weight") if second is not None else None,
+        _dev(second[1]) if second is not None else None, _dev(sums, f32, "sums"), 1 if after is not None else 0,
+        _dev(before.sums, f32, "sums") if before is not None else None, _dev(before_weight, f32, "weight") if before is not None else None,
+        _dev(scale, f32, "scale") if scale is not None else None, float(alpha), before.eps if before is not None else float(eps), _stream()), "linear_leave")
+    return NormedRows(rows, sums, eps, second=NormedRows(second[1], sums, eps) if second is not None else None)
+
+
+def linear_rotate_pays(x, weight, rot):
+    """Is `linear_rotate` there for these operands, and faster than split-K sums that `rope_kv_write` finishes?"""
+    rows = x.rows if isinstance(x, NormedRows) else x
+    return (rot % 16 == 0 and _few_rows_of_shuffled(rows, weight)
+            and bool(library().tw_linear_rotate_pays(dtype_id(rows.dtype), rows.shape[0], *weight.shape)))
+
+
+def linear_rotate(x, weight, qkv, cos, sin, slots, keys, values, q_heads, kv_heads, head_dim, page_size, write_cache=True, bias=None, adjacent=False):
+    """The packed product of queries, keys and values of up to 16 rows (`NormedRows` or plain ones), with what `rope_kv_write` does behind it
+    in its epilogue: the q columns of qkv are written rotated, k and v go to the pages only."""
+    rows = x.rows if isinstance(x, NormedRows) else x
+    m, k, lda = _rows(rows, "x")
+    n, k2, w_ptr, ldw, shuffled, w_dtype = _weight_args(weight)
+    mo, no, ld = _rows(qkv, "qkv")
+    _need(k == k2 and shuffled and rows.dtype == w_dtype == qkv.dtype and (mo, no) == (m, n) and m <= 16, "linear_rotate takes up to 16 rows of a shuffled weight's type")
+    _need(n == (q_heads + 2 * kv_heads) * head_dim and head_dim % 16 == 0, "qkv width does not match the head counts")
+    half = cos.shape[1] if cos is not None else 0
+    _need(2 * half <= head_dim and half % 8 == 0, "linear_rotate turns multiples of 16 elements of a head")
+    if half:
+        _need(tuple(cos.shape) == (m, half) and tuple(sin.shape) == (m, half) and cos.is_contiguous() and sin.is_contiguous(), "rotary tables must be [n, rot/2]")
+    if write_cache:
+        _need(keys.dtype == qkv.dtype and values.dtype == qkv.dtype and keys.is_contiguous() and values.is_contiguous(), "cache tensors must be contiguous, of qkv's type")
+        _need(tuple(keys.shape[1:]) == (kv_heads, page_size, head_dim) and values.numel() == keys.numel(), "keys must be [pages, kv_heads, page_size, head_dim]")
+        _need(slots.numel() == m, "one cache slot per token is needed")
+    _need(bias is None or (bias.numel() == n and bias.is_contiguous()), "bias has the wrong size")
+    norms = _normed_args(x, k) if isinstance(x, NormedRows) else (None, 0, 0, 0.0)
+    f32 = torch.float32
+    check(library().tw_linear_rotate(
+        dtype_id(w_dtype), _dev(rows), lda, *norms, w_ptr, ldw, _dev(bias, f32, "bias") if bias is not None else None, _dev(qkv), ld, m, k,
+        _dev(cos, f32, "cos") if half else None, _dev(sin, f32, "sin") if half else None, _dev(slots, torch.int32, "slots") if write_cache else None,
+        _dev(keys) if write_cache else None, _dev(values) if write_cache else None, q_heads, kv_heads, head_dim, 2 * half, page_size,
+        1 if write_cache else 0, 1 if adjacent else 0, _stream()), "linear_rotate")
+    return qkv
+
+
 def attn_decode_splits(n_seqs, q_heads, kv_heads, max_kv_len):
     return int(library().tw_attn_decode_splits(n_seqs, q_heads, kv_heads, max_kv_len))
 
@@ -831,8 +961,9 @@ def attn_mixed(q, keys, values, block_table, q_start, kv_len, seq0, n_seqs, max_
 
 # ---- norm after the sum, relu squared, hashed pair embedding ----------------------------------------------------------
 
-def residual_norm(x, weight, eps, out=None, y=None, add=None, scale=None, alpha=1.0):
+def residual_norm(x, weight, eps, out=None, y=None, add=None, scale=None, alpha=1.0, before=None):
     """x <- weight * unit(alpha * x + scale * y), unit(v) = v / sqrt(mean(v^2) + eps); x float32 [n, hidden] in place.
+    before (float32 [hidden], for `can_leave_norms` rows): before * unit(x) takes the place of x.
 
     y: float32 [n, hidden] (rows may be strided), or add: float32 [splits, n, hidden] partial sums added up here;
     scale: float32 [hidden] or None; out: the normed rows once more, rounded to its type (the compute type)."""
@@ -851,6 +982,8 @@ def residual_norm(x, weight, eps, out=None, y=None, add=None, scale=None, alpha=
         splits, stride = add.shape[0], n * hidden
     if scale is not None:
         _need(scale.numel() == hidden and scale.dtype == torch.float32 and scale.is_contiguous(), "scale must be float32 [hidden]")
+    if before is not None:
+        _need(can_leave_norms(n, hidden) and before.numel() == hidden and before.is_contiguous(), "before must be [hidden], of rows whose norms can travel")
     out_dtype = F32
     if out is not None:
         _need(out.is_contiguous() and tuple(out.shape) == (n, hidden), "out must be contiguous [n, hidden]")
@@ -858,7 +991,8 @@ def residual_norm(x, weight, eps, out=None, y=None, add=None, scale=None, alpha=
     check(library().tw_residual_norm(out_dtype, _dev(x), _dev(y) if y is not None else None, ldy,
                                      _dev(add) if add is not None else None, splits, stride,
                                      _dev(scale) if scale is not None else None, _dev(weight),
-                                     _dev(out) if out is not None else None, n, hidden, float(alpha), float(eps), _stream()),
+                                     _dev(out) if out is not None else None, n, hidden, float(alpha), float(eps),
+                                     _dev(before, torch.float32, "before") if before is not None else None, _stream()),
           "residual_norm")
     return x
 

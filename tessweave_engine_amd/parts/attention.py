@@ -63,6 +63,8 @@ def paged_attention(ctx, q, keys, values, group, out, q_heads, kv_heads, head_di
 
 
 class GroupedQueryAttention(Mixer):
+    leaves_normed = True
+
     def __init__(self, prefix, hidden, q_heads, kv_heads, head_dim, position, qkv_bias=True,
                  o_bias=False, window=None, scale=None, packed=True, head_hook=None, softcap=None, value_dim=None,
                  names=("q_proj", "k_proj", "v_proj", "o_proj"), suffixes=(".weight", ".bias")):
@@ -121,6 +123,10 @@ class GroupedQueryAttention(Mixer):
     def cache_need(self):
         return CacheNeed(paged=PagedKV(self.kv_heads, self.head_dim, self.window))
 
+    @property
+    def takes_normed(self):
+        return self.qkv.takes_normed
+
     def forward(self, ctx, run, h, x, accumulate=True):
         n = ctx.n_tokens
         width = (self.q_heads + 2 * self.kv_heads) * self.head_dim
@@ -129,7 +135,11 @@ class GroupedQueryAttention(Mixer):
         adjacent = self.position.pairing == "adjacent"
         keys, values, g = ctx.cache.keys_values(run.cache_slot)
         group = ctx.groups[g]
-        if n <= 64 and self.head_hook is None and self.qkv.deferrable(n):
+        if n <= 16 and self.head_hook is None and self.qkv.takes_normed and ops.linear_rotate_pays(h, self.qkv.weights[0], self.position.rotary_dim):
+            ops.linear_rotate(h, self.qkv.weights[0], qkv, cos, sin, group.slot_mapping, keys, values, self.q_heads, self.kv_heads, self.head_dim,
+                              ctx.cache.page_size, write_cache=run.writes_cache, bias=self.qkv.biases[0] if self.qkv.biases else None,
+                              adjacent=adjacent)
+        elif n <= 64 and self.head_hook is None and self.qkv.deferrable(n):
             # few rows: the projection leaves split-K sums; bias, rotation and cache write finish them
             partial = self.qkv.forward_partials(ctx, h, "qkv")
             ops.rope_kv_write(qkv, cos, sin, group.slot_mapping, keys, values, self.q_heads, self.kv_heads,
@@ -145,6 +155,9 @@ class GroupedQueryAttention(Mixer):
         out = ctx.scratch("attn.out", (n, self.q_heads * self.head_dim))
         paged_attention(ctx, qkv, keys, values, group, out, self.q_heads, self.kv_heads, self.head_dim, self.scale,
                         window=self.window or 0, softcap=self.softcap)
+        left = self.o.forward_left(ctx, out)
+        if left is not None:
+            return left
         if ctx.defer_sums and not self.o.biases and self.o.deferrable(n):
             return self.o.forward_partials(ctx, out, "o")          # the next norm adds them into x
         self.o.forward(ctx, out, x, residual=x if accumulate else None)

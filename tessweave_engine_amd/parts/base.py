@@ -15,6 +15,7 @@ import math
 
 import torch
 
+from ..kernels import ops
 
 #: key of `StepContext.shared` under which a part that has just written the residual stream may leave the same rows
 #: rounded to the compute type (in float32 runs: the stream itself), for a sublayer that reads the stream as it is
@@ -27,6 +28,9 @@ NORMED_STREAM = "stream.normed"
 #: key of `StepContext.shared` under which an embedding that is asked to keeps its output (float32 [n, hidden]) for layer
 #: runs that add it to the stream again (`LayerRun.adds_embedding`)
 EMBEDDING_OUTPUT = "embedding.output"
+
+#: key of `StepContext.shared`: which of the two buffers took the last sums of squares that travel (see `NormAhead`)
+SUMS_TURN = "left.sums.turn"
 
 
 @dataclass(frozen=True)
@@ -51,6 +55,14 @@ class Part:
     #: stream: no host synchronisation, no allocation once buffers exist. Only
     #: models whose parts all say so are replayed from HIP graphs.
     graph_safe = True
+
+    #: may the rows a sublayer or a head is given be `ops.NormedRows` (see `NormAhead`)? Only parts whose first use of them is a
+    #: product say so.
+    takes_normed = False
+
+    #: does a sublayer's `forward` end in ONE product into the stream that looks at `ctx.norm_ahead` (`Linear.forward_left`)? A part
+    #: that runs another one and adds more to the stream behind it must leave this False.
+    leaves_normed = False
 
     def tensor_specs(self):
         return []
@@ -151,6 +163,11 @@ class FeedForward(Part):
 class Block(Part):
     mixer: Mixer
 
+    def entry(self):
+        """(norms, readers): the norms that the block starts with (none: it reads the stream as it is) and the parts that read the
+        rows, if the block takes `ops.NormedRows` for them in place of pending sums; None if not."""
+        return None
+
     def cache_need(self):
         """What the block keeps per request in its cache slot: its mixer's need, unless the block itself
         carries something more from token to token."""
@@ -167,6 +184,28 @@ def fold_pending(x, pending):
     if pending is not None:
         x += pending.sum(0)
     return None
+
+
+class NormAhead:
+    """In steps of up to 16 one-token rows a sublayer's last product may leave the residual stream's rows for the norms that read
+    them next, so that no norm kernel runs: `ctx.norm_ahead` tells it which. norms: one `RMSNorm` part, or two of the same eps
+    side by side; stream: the float32 residual stream; after: None, or (before, weight, alpha, scale) where the sublayer's result meets a
+    stream that is itself behind a norm (see `ops.linear_leave`). A part that leaves them (`Linear.forward_left`) returns `ops.NormedRows` in
+    place of pending sums, and the stream is complete. It is set only for parts that say `leaves_normed`."""
+    __slots__ = ("norms", "stream", "after")
+
+    def __init__(self, norms, stream, after=None):
+        self.norms, self.stream, self.after = tuple(norms), stream, after
+
+
+def norm_ahead(ctx, stream, norms, readers, after=None):
+    """A `NormAhead` if NORMS (each read by one of READERS) can travel in this step, else None."""
+    n, width = stream.shape
+    if not ctx.capturing or not ops.can_leave_norms(n, width) or len({norm.eps for norm in norms}) != 1:       # (none: not here either)
+        return None
+    if not all(getattr(norm, "travels", False) and norm.size == width for norm in norms) or not all(r.takes_normed for r in readers):
+        return None
+    return NormAhead(norms, stream, after)
 
 
 class Workspace:
@@ -253,6 +292,8 @@ class StepContext:
         self.token_feed = None       # int32 device tensor: a token id -1 - k in token_ids stands for token_feed[k]
         self.defer_sums = True       # may a mixer or feed-forward leave partial sums pending for the next norm?
         self.capturing = False       # launches may depend on kv_bound and capacities, not on this step's lengths
+        self.norm_ahead = None       # NormAhead for the sublayer that runs now: the norms that read the stream behind it
+        self.entry_behind = None     # (norms, readers) of what runs behind the block that runs now, or None (see Block.entry)
         self.segment_end = None      # while a step is captured: called with the index of each finished layer run
         self.max_tokens = 0          # row capacity of per-token scratch buffers
         self.cache = None            # cache.CacheManager

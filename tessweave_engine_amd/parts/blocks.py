@@ -4,12 +4,14 @@
 """
 from __future__ import annotations
 
+from contextlib import contextmanager
+
 import torch
 
 from ..cache.spec import CacheNeed
 from ..kernels import ops
 from ..weights.spec import AVERAGE, ONE_PLUS_NORMAL, VECTOR, TensorSpec
-from .base import NORMED_STREAM, ROUNDED_STREAM, Block, fold_pending
+from .base import NORMED_STREAM, ROUNDED_STREAM, Block, fold_pending, norm_ahead
 
 
 class PreNormBlock(Block):
@@ -26,16 +28,35 @@ class PreNormBlock(Block):
         for p in self.parts():
             p.bind(tensors, dtype, device)
 
+    def entry(self):
+        return (self.mixer_norm,), (self.mixer,)
+
     def forward(self, ctx, run, x, pending=None):
         h = normalise(self.mixer_norm, ctx, x, pending)
-        pending = self.mixer.forward(ctx, run, h, x)
+        with leaving(ctx, x, self.mixer, ((self.ffn_norm,), (self.ffn,))):
+            pending = self.mixer.forward(ctx, run, h, x)
         h = normalise(self.ffn_norm, ctx, x, pending)
-        return self.ffn.forward(ctx, h, x)
+        with leaving(ctx, x, self.ffn, ctx.entry_behind):
+            return self.ffn.forward(ctx, h, x)
+
+
+@contextmanager
+def leaving(ctx, x, sublayer, entry):
+    """While SUBLAYER runs, whose last product may leave the stream X for the norms of ENTRY ((norms, readers), or None)."""
+    ctx.norm_ahead = norm_ahead(ctx, x, *entry) if entry is not None and sublayer.leaves_normed else None
+    try:
+        yield
+    finally:
+        ctx.norm_ahead = None
 
 
 def normalise(norm, ctx, x, pending=None, rows=None):
     """NORM of X; PENDING partial sums go to a norm that folds them, and are folded here for one that does not
     (which only happens when parts are driven by hand: a model defers sums only if all its norms fold them)."""
+    if isinstance(pending, ops.NormedRows):
+        if pending.norm is not norm or (rows is not None and rows.numel() != pending.shape[0]):
+            raise RuntimeError("the rows left by the product before are another norm's")
+        return pending
     if pending is not None and not norm.folds_pending:
         pending = fold_pending(x, pending)
     if pending is not None:
@@ -90,20 +111,34 @@ class ParallelBlock(Block):
                 return self.ffn.forward(ctx, h, x, more=left)
             fold_pending(x, left)
             return self.ffn.forward(ctx, h, x)
-        pending = fold_pending(x, pending)
-        n = ctx.n_tokens
-        h1 = ctx.scratch("norm.out", (n, self.hidden))
-        h2 = ctx.scratch("norm.out.second", (n, self.hidden)) if self.ffn is not None else None
-        ops.rmsnorm_pair(x, self.mixer_norm.weight, self.mixer_norm.eps, h1,
-                         self.ffn_norm.weight if self.ffn is not None else None, h2)
-        left = self.mixer.forward(ctx, run, h1, x)
-        if left is not None:
+        if isinstance(pending, ops.NormedRows):
+            h1, h2 = pending, pending.second
+            if h1.norm is not self.mixer_norm or (h2.norm if h2 is not None else None) is not self.ffn_norm:
+                raise RuntimeError("the rows left by the product before are other norms'")
+        else:
+            pending = fold_pending(x, pending)
+            n = ctx.n_tokens
+            h1 = ctx.scratch("norm.out", (n, self.hidden))
+            h2 = ctx.scratch("norm.out.second", (n, self.hidden)) if self.ffn is not None else None
+            ops.rmsnorm_pair(x, self.mixer_norm.weight, self.mixer_norm.eps, h1,
+                             self.ffn_norm.weight if self.ffn is not None else None, h2)
+        with leaving(ctx, x, self.mixer, ctx.entry_behind if self.ffn is None else None):
+            left = self.mixer.forward(ctx, run, h1, x)
+        if left is not None and (self.ffn is not None or not isinstance(left, ops.NormedRows)):
             raise RuntimeError("a parallel block's mixer must add into the stream itself")
         if self.ffn is not None:
-            left = self.ffn.forward(ctx, h2, x)
-            if left is not None:
+            with leaving(ctx, x, self.ffn, ctx.entry_behind):
+                left = self.ffn.forward(ctx, h2, x)
+            if left is not None and not isinstance(left, ops.NormedRows):
                 raise RuntimeError("a parallel block's feed-forward must add into the stream itself")
-        return None
+        return left
+
+    def entry(self):
+        if self.shared_norm:
+            return None
+        if self.ffn is None:
+            return (self.mixer_norm,), (self.mixer,)
+        return (self.mixer_norm, self.ffn_norm), (self.mixer, self.ffn)
 
 
 class PostNormBlock(Block):
@@ -155,22 +190,34 @@ class PostNormBlock(Block):
             h = ops.round_rows(x, ctx.scratch("stream.rounded", (ctx.n_tokens, self.hidden)))
         return h
 
-    def _sublayer(self, ctx, x, norm, scale, result, pending):
+    def entry(self):
+        return (), (self.mixer,)
+
+    def _sublayer(self, ctx, x, part, args, norm, scale, readers, behind):
+        """x <- norm(alpha * x + scale * PART(rows)), ARGS what the part takes before its rows. BEHIND: `ops.NormedRows` where x is still
+        the rows of a norm that travels (None: x is the stream). Returns the same of the new stream."""
+        result = ctx.scratch("sublayer.result", (ctx.n_tokens, self.hidden), torch.float32)
+        if readers and part.leaves_normed:
+            ctx.norm_ahead = norm_ahead(ctx, x, (norm,), readers, (behind, behind.norm.weight if behind is not None else None, self.alpha, scale))
+        try:
+            left = part.forward(ctx, *args, behind if behind is not None else self._rounded(ctx, x), result, accumulate=False)
+        finally:
+            ctx.norm_ahead = None
+        if isinstance(left, ops.NormedRows):
+            return left
         rounded = ctx.scratch("stream.rounded", (ctx.n_tokens, self.hidden)) if ctx.dtype != torch.float32 else None
-        ops.residual_norm(x, norm.weight, norm.eps, out=rounded, y=result if pending is None else None, add=pending,
-                          scale=scale, alpha=self.alpha)
+        ops.residual_norm(x, norm.weight, norm.eps, out=rounded, y=result if left is None else None, add=left, scale=scale, alpha=self.alpha,
+                          before=behind.norm.weight if behind is not None else None)
         ctx.shared[ROUNDED_STREAM] = rounded if rounded is not None else x
+        return None
 
     def forward(self, ctx, run, x, pending=None):
-        pending = fold_pending(x, pending)
-        n = ctx.n_tokens
-        result = ctx.scratch("sublayer.result", (n, self.hidden), torch.float32)
-        left = self.mixer.forward(ctx, run, self._rounded(ctx, x), result, accumulate=False)
-        self._sublayer(ctx, x, self.mixer_norm, self.mixer_scale, result, left)
+        behind = pending if isinstance(pending, ops.NormedRows) else fold_pending(x, pending)
+        follows = ctx.entry_behind[1] if ctx.entry_behind is not None and not ctx.entry_behind[0] else ()      # (a block that reads the stream as it is)
+        behind = self._sublayer(ctx, x, self.mixer, (run,), self.mixer_norm, self.mixer_scale, (self.ffn,) if self.ffn is not None else follows, behind)
         if self.ffn is not None:
-            left = self.ffn.forward(ctx, self._rounded(ctx, x), result, accumulate=False)
-            self._sublayer(ctx, x, self.ffn_norm, self.ffn_scale, result, left)
-        return None
+            behind = self._sublayer(ctx, x, self.ffn, (), self.ffn_norm, self.ffn_scale, follows, behind)
+        return behind
 
 
 class ResultNormBlock(Block):

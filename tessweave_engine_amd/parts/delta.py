@@ -38,6 +38,7 @@ class StackedTaps(CausalConv):
 
 
 class GatedDeltaRule(Mixer):
+    leaves_normed = True
     STATE = "delta.s"
     CONV_STATE = "delta.conv"
 
@@ -89,6 +90,10 @@ class GatedDeltaRule(Mixer):
         state = FixedState((self.heads, self.value_dim, ops.delta_key_extent(self.dim)), "float32")
         return CacheNeed(states=((self.STATE, state), self.conv.state_need()))
 
+    @property
+    def takes_normed(self):
+        return self.proj.takes_normed
+
     def forward(self, ctx, run, h, x, accumulate=True):
         n, H, G, D, E = ctx.n_tokens, self.heads, self.key_heads, self.dim, self.value_dim
         col = self.columns
@@ -111,5 +116,8 @@ class GatedDeltaRule(Mixer):
         ops.delta_rule(*common, apart, sequences, result, G, D, D ** -0.5, max_q_len=ctx.max_q_len, workspace=ws, rows=rows)
         act = ctx.scratch("delta.act", (n, H * E))
         ops.head_norm_gate(result, proj[:, col["g"]:col["g"] + H * E], self.norm_weight, act, H, E, self.eps)
+        left = self.o.forward_left(ctx, act)
+        if left is not None:
+            return left
         self.o.forward(ctx, act, x, residual=x if accumulate else None)
         return None

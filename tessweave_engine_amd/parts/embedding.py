@@ -177,10 +177,14 @@ class OutputHead(Part):
     def weight_tensors(self):
         return [self.weight]          # (the embedding's table is not listed by its part: a step gathers a few rows of it)
 
+    @property
+    def takes_normed(self):
+        return isinstance(self.weight, ops.ShuffledWeight)
+
     def forward(self, ctx, h):
         # The logits live in a shared scratch buffer: they are valid until the next step.
         logits = ctx.workspace.get("logits", (h.shape[0], self.vocab), torch.float32)
-        ops.linear(h, self.matrix(), logits)
+        (ops.linear_normed if isinstance(h, ops.NormedRows) else ops.linear)(h, self.matrix(), logits)
         if self.scale != 1.0:
             ops.scale_values(logits, self.scale)
         if self.softcap:

@@ -11,6 +11,8 @@ from .linear import Linear
 
 
 class SwiGLU(FeedForward):
+    leaves_normed = True
+
     def __init__(self, prefix, hidden, intermediate, packed=True):
         self.hidden, self.intermediate = int(hidden), int(intermediate)
         self.gate_up = Linear([prefix + "gate_proj", prefix + "up_proj"], hidden, [intermediate, intermediate],
@@ -27,6 +29,10 @@ class SwiGLU(FeedForward):
         self.gate_up.bind(tensors, dtype, device)
         self.down.bind(tensors, dtype, device)
 
+    @property
+    def takes_normed(self):
+        return self.gate_up.takes_normed
+
     def forward(self, ctx, h, x, accumulate=True):
         n = h.shape[0]
         act = ctx.scratch("ffn.act", (n, self.intermediate))
@@ -37,6 +43,9 @@ class SwiGLU(FeedForward):
             gu = ctx.scratch("ffn.gate_up", (n, 2 * self.intermediate))
             self.gate_up.forward(ctx, h, gu)
             ops.silu_mul(gu, act)
+        left = self.down.forward_left(ctx, act)
+        if left is not None:
+            return left
         if ctx.defer_sums and not self.down.biases and self.down.deferrable(n):
             # where the down projection splits K (few rows; many rows against its long K), the sums are left to the next norm
             return self.down.forward_partials(ctx, act, "down")
@@ -53,6 +62,8 @@ class GatedFeedForward(FeedForward):
     folded into that multiplication, before the rounding to the compute type, so the down projection adds straight
     into the residual stream.
     """
+
+    leaves_normed = True
 
     def __init__(self, names, hidden, intermediate, activation="gelu_tanh", out_scale=1.0, suffix=".weight", limit=None):
         """activation: "gelu_tanh", "silu", or "swish_limited", which needs `limit` L and computes
@@ -78,6 +89,10 @@ class GatedFeedForward(FeedForward):
         self.gate_up.bind(tensors, dtype, device)
         self.down.bind(tensors, dtype, device)
 
+    @property
+    def takes_normed(self):
+        return self.gate_up.takes_normed
+
     def forward(self, ctx, h, x, accumulate=True):
         n = h.shape[0]
         act = ctx.scratch("ffn.act", (n, self.intermediate))
@@ -95,6 +110,9 @@ class GatedFeedForward(FeedForward):
                 raise ValueError("silu with an output scale needs an intermediate size that is a multiple of 16")
             else:
                 ops.gelu_mul(gu, act, self.out_scale)
+        left = self.down.forward_left(ctx, act)
+        if left is not None:
+            return left
         if not accumulate and ctx.defer_sums and self.down.deferrable(n):
             return self.down.forward_partials(ctx, act, "down")          # the caller's norm adds them up
         self.down.forward(ctx, act, x, residual=x if accumulate else None)
@@ -105,6 +123,8 @@ class PlainFeedForward(FeedForward):
     """x += down( act(up(h)) ): no gate, no biases; act "relu_squared" (max(z, 0)^2) or "gelu" (the exact one, z Phi(z)).
     names = (up, down), the checkpoint prefixes of the two matrices. defer=False: the down projection always finishes
     its sums itself (for a part that adds more to the same result)."""
+
+    leaves_normed = True
 
     def __init__(self, names, hidden, intermediate, suffix=".weight", activation="relu_squared", defer=True):
         up, down = names
@@ -125,6 +145,10 @@ class PlainFeedForward(FeedForward):
         self.up.bind(tensors, dtype, device)
         self.down.bind(tensors, dtype, device)
 
+    @property
+    def takes_normed(self):
+        return self.up.takes_normed
+
     def forward(self, ctx, h, x, accumulate=True):
         n = h.shape[0]
         act = ctx.scratch("ffn.act", (n, self.intermediate))
@@ -136,6 +160,9 @@ class PlainFeedForward(FeedForward):
         else:
             self.up.forward(ctx, h, act)
             ops.activation(act, self.activation)
+        left = self.down.forward_left(ctx, act)
+        if left is not None:
+            return left
         if self.defer and ctx.defer_sums and self.down.deferrable(n):
             return self.down.forward_partials(ctx, act, "down")          # whoever norms next adds them up
         self.down.forward(ctx, act, x, residual=x if accumulate else None)

@@ -38,6 +38,8 @@ def _round_up(v, m):
 
 
 class LatentAttention(Mixer):
+    leaves_normed = True
+
     def __init__(self, prefix, hidden, heads, dim, rot_dim, value_dim, latent, scale, position, eps, own_latent=True,
                  names=("q", "dkv", "dkv.norm", "uk", "uv", "o"), sink_name=None, gate_name=None):
         """position: a rotary encoding over `rot_dim` elements (its `rotary_dim` may be smaller: the rest of the
@@ -145,6 +147,10 @@ class LatentAttention(Mixer):
     def cache_need(self):
         return CacheNeed(paged=PagedKV(1, self.key_dev, None, self.latent_dev))
 
+    @property
+    def takes_normed(self):
+        return self.proj.takes_normed
+
     def forward(self, ctx, run, h, x, accumulate=True):
         if run.writes_cache != self.own_latent:
             raise RuntimeError("a layer with a latent of its own writes its cache slot; one without reads another layer's")
@@ -196,6 +202,9 @@ class LatentAttention(Mixer):
                              portions, longest_portion, out, H, H, hd, self.scale, split=split, workspace=ws, sink=self.sink)
             if gate is not None:
                 ops.sigmoid_gate(out[nd:], gate[nd:])
+        left = self.o.forward_left(ctx, out)
+        if left is not None:
+            return left
         if ctx.defer_sums and self.o.deferrable(n):
             return self.o.forward_partials(ctx, out, "o")          # whoever norms next adds them up
         self.o.forward(ctx, out, x, residual=x if accumulate else None)

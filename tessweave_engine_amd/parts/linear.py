@@ -11,7 +11,7 @@ import torch
 
 from ..kernels import ops
 from ..weights.spec import MATRIX, VECTOR, NORMAL, TensorSpec
-from .base import Part
+from .base import SUMS_TURN, Part
 
 
 def pad_groups(t, dim, unit, to):
@@ -154,6 +154,8 @@ class Linear(Part):
 
     def forward_glu(self, ctx, x, out, activation="silu", factor=1.0):
         """out [n, rows of one matrix] = factor * act(x @ gate.T + b) * (x @ up.T + b), in x's type (needs `gated`)."""
+        if isinstance(x, ops.NormedRows):
+            return ops.linear_normed(x, self.weights[0], out, bias=self.biases[0] if self.biases else None, activation=activation, factor=factor)
         return ops.linear_glu(x, self.weights[0], out, bias=self.biases[0] if self.biases else None,
                               activation=activation, factor=factor)
 
@@ -164,6 +166,11 @@ class Linear(Part):
         if len(self.weights) != 1 or self.gated:
             return False
         w = self.weights[0]
+        if isinstance(x, ops.NormedRows):
+            if ops.linear_act_few_pays(x.rows, w):
+                ops.linear_normed(x, w, out, bias=self.biases[0] if self.biases else None, activation=activation)
+                return True
+            return False
         if ops.linear_act_few_pays(x, w):
             ops.linear_act_few(x, w, out, activation, bias=self.biases[0] if self.biases else None)
             return True
@@ -178,6 +185,9 @@ class Linear(Part):
         """out[:, columns] = x @ W.T (+ bias) (+ residual); out may be float32 or x's type."""
         if self.gated:
             raise RuntimeError("a gated pair of matrices has interleaved rows; use forward_glu")
+        normed = isinstance(x, ops.NormedRows)
+        if normed and (residual is not None or not self.takes_normed):
+            raise RuntimeError("rows whose norm travels meet one packed matrix, without a residual")
         col = 0
         for i, w in enumerate(self.weights):
             rows = w.shape[0]
@@ -199,7 +209,10 @@ class Linear(Part):
                 floats = ops.linear_workspace_bytes(w.dtype, x.shape[0], rows, w.shape[1]) // 4
                 if floats:
                     ws = ctx.workspace.get("linear.splitk.rows", (floats,), torch.float32)
-            ops.linear(x, w, target, bias=self.biases[i] if self.biases else None, residual=res, workspace=ws)
+            if normed:
+                ops.linear_normed(x, w, target, bias=self.biases[i] if self.biases else None, workspace=ws)
+            else:
+                ops.linear(x, w, target, bias=self.biases[i] if self.biases else None, residual=res, workspace=ws)
             col += rows
         return out
 
@@ -227,14 +240,40 @@ class Linear(Part):
         """float32 [splits, n, out] partial sums of x @ W.T (bias NOT added); see ops.linear_partials."""
         w = self.weights[0]
         n = x.shape[0]
-        splits = self._partial_splits(n, x.stride(0) if n > 1 else None)
+        normed = isinstance(x, ops.NormedRows)
+        splits = self._partial_splits(n, x.stride(0) if n > 1 and not normed else None)
         if n <= 64:     # sized once for the largest such batch, so that it never regrows under a captured graph
             most = max(self._partial_splits(rows) for rows in (16, 32, 48, 64))
             buf = ctx.workspace.get("linear.partial." + tag, (most, 64, w.shape[0]), torch.float32)
         else:
             buf = ctx.workspace.get("linear.partial.rows." + tag, (splits, n, w.shape[0]), torch.float32)
         partial = buf.view(-1)[:splits * n * w.shape[0]].view(splits, n, w.shape[0])
-        return ops.linear_partials(x, w, partial)
+        return ops.linear_normed(x, w, partial=partial) if normed else ops.linear_partials(x, w, partial)
+
+    # ---- norms that travel with the product ---------------------------------------------------
+    @property
+    def takes_normed(self):
+        """May the input be `ops.NormedRows`? (one packed matrix in the kernels' layout)"""
+        return len(self.weights) == 1 and isinstance(self.weights[0], ops.ShuffledWeight)
+
+    def forward_left(self, ctx, x):
+        """Add x @ W.T (+ bias) into the stream of `ctx.norm_ahead` and leave the rows for the norms that read it next, as
+        `ops.NormedRows`; None, and nothing done, where nobody asked for that or a norm kernel is no slower."""
+        ahead = getattr(ctx, "norm_ahead", None)
+        if ahead is None or not self.takes_normed or self.gated or not ops.linear_leave_pays(x, self.weights[0]):
+            return None
+        n, width = x.shape[0], self.weights[0].shape[0]
+        rows = [ctx.workspace.get(f"left.rows{i}", (16, width), x.dtype)[:n] for i in range(len(ahead.norms))]
+        # (two buffers in turn: the product that leaves sums may read those left before)
+        ctx.shared[SUMS_TURN] = turn = ctx.shared.get(SUMS_TURN, 0) ^ 1
+        sums = ctx.workspace.get(f"left.sums{turn}", (16 * width // 16,), torch.float32)[:n * width // 16].view(n, width // 16)
+        first, second = ahead.norms[0], ahead.norms[1] if len(ahead.norms) > 1 else None
+        left = ops.linear_leave(x, self.weights[0], ahead.stream, first.weight, first.eps, rows[0], sums, bias=self.biases[0] if self.biases else None,
+                                second=(second.weight, rows[1]) if second is not None else None, after=ahead.after)
+        left.norm = first
+        if second is not None:
+            left.second.norm = second
+        return left
 
 
 class JoinedLinear(Linear):

@@ -113,6 +113,14 @@ class DecoderModel(Part):
             self._layout = CacheLayout(needs)
         return self._layout
 
+    def _entry_behind(self, i):
+        """What norms read the stream behind run I (see `Block.entry`): the next block's, or the model's last one (a captured step
+        wants every row's logits, in order)."""
+        if i + 1 == len(self.schedule):
+            return (self.final_norm,), (self.head,)
+        following = self.schedule[i + 1]
+        return None if following.adds_embedding else self.blocks[following.block].entry()
+
     # ---- one step -----------------------------------------------------------------
     def forward(self, ctx):
         """Run the step's tokens; float32 logits [n_logits, vocab] at ctx.logit_rows."""
@@ -125,6 +133,7 @@ class DecoderModel(Part):
                     pending = first.unsqueeze(0)          # the run's first norm adds it, like any pending sum
                 else:
                     ops.add_values(x, first)
+            ctx.entry_behind = self._entry_behind(i) if ctx.capturing else None
             pending = self.blocks[run.block].forward(ctx, run, x, pending)
             if ctx.segment_end is not None:
                 ctx.segment_end(i)

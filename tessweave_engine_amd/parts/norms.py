@@ -13,6 +13,7 @@ from .base import Norm
 
 class RMSNorm(Norm):
     folds_pending = True
+    travels = True            # (see `NormAhead`)
 
     def __init__(self, name, size, eps, suffix=".weight", offset=0.0):
         """offset: what the stored weight is to be increased by (1.0 for checkpoints that keep their norm weights

@@ -23,6 +23,7 @@ def _round_up(v, m):
 
 
 class Retention(Mixer):
+    leaves_normed = True
     STATE = "retention.s"
 
     def __init__(self, prefix, hidden, heads, dim, value_dim, decay, position, eps, names=("q", "k", "v", "g", "o"),
@@ -63,6 +64,10 @@ class Retention(Mixer):
     def cache_need(self):
         return CacheNeed(states=((self.STATE, FixedState((self.heads, self.dim_dev, self.value_dev), "float32")),))
 
+    @property
+    def takes_normed(self):
+        return self.proj.takes_normed
+
     def forward(self, ctx, run, h, x, accumulate=True):
         n, H, Dp, Ep = ctx.n_tokens, self.heads, self.dim_dev, self.value_dev
         proj = ctx.scratch("retention.proj", (n, 2 * H * (Dp + Ep)))
@@ -80,6 +85,9 @@ class Retention(Mixer):
             ops.retention(*common, ctx.n_decode, portions, result, self.dim ** -0.5, max_q_len=ctx.max_q_len, workspace=ws)
         act = ctx.scratch("retention.act", (n, H * Ep))
         ops.unit_gate(result, proj[:, 2 * H * Dp + H * Ep:], act, H, self.value_dim, Ep, self.eps)
+        left = self.o.forward_left(ctx, act)
+        if left is not None:
+            return left
         if ctx.defer_sums and self.o.deferrable(n):
             return self.o.forward_partials(ctx, act, "o")          # whoever norms next adds them up
         self.o.forward(ctx, act, x, residual=x if accumulate else None)

@@ -1,0 +1,152 @@
+"""Norms that travel with the products of up to 16 rows, and the packed product that rotates and fills the cache, against float64."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+DTYPES = [torch.float32, torch.bfloat16]
+BITS = {torch.float32: 2.0 ** -24, torch.bfloat16: 2.0 ** -8}       # half a last place: 24 and 8 bits of significand
+
+
+@pytest.fixture(scope="module")
+def ops(device):
+    from tessweave_engine_amd.kernels import ops
+    return ops
+
+
+def rand(shape, dtype, device, scale=1.0, seed=0):
+    g = torch.Generator().manual_seed(seed)
+    return (torch.randn(shape, generator=g) * scale).to(dtype).to(device)
+
+
+def close(got, want, sizes, dtype, rounded=True):
+    """SIZES: the sum of the products' magnitudes behind each element. float32 sums of products of K are off by less than 2^-18 of it here
+    (K up to 8,192 in any order: the errors' random walk, not its bound); what is rounded once more by half a last place."""
+    bound = 2.0 ** -18 * sizes + (BITS[dtype] * want.abs() if rounded else 0)
+    assert torch.isfinite(got.float()).all()
+    assert ((got.double() - want).abs() <= 1.01 * bound + 1e-30).all(), float(((got.double() - want).abs() / (bound + 1e-30)).max())
+
+
+# rows, columns, K: one and all rows of a tile; the fewest columns, sums that fill a lane's share exactly and not; K of four, eight and sixteen waves, and ragged
+LEAVES = [(1, 64, 64), (16, 64, 72), (3, 896, 4864), (8, 2048, 5632), (5, 2112, 3000), (16, 4096, 1024), (1, 4096, 8192)]
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("m,n,k", LEAVES)
+@pytest.mark.parametrize("form", ["plain", "two norms", "after a norm", "after rows as they are"])
+def test_rows_left(ops, device, dtype, m, n, k, form):
+    x, w = rand((m, k), dtype, device), rand((n, k), dtype, device, k ** -0.5, 1)
+    bias, stream = rand((n,), torch.float32, device, 0.1, 2), rand((m, n), torch.float32, device, 1.0, 3)
+    weight, second = 1 + rand((n,), torch.float32, device, 0.1, 4), 1 + rand((n,), torch.float32, device, 0.1, 5)
+    before_weight, scale = 1 + rand((n,), torch.float32, device, 0.1, 6), 1 + rand((n,), torch.float32, device, 0.1, 7)
+    rows, rows2 = (torch.full((m, n), float("nan"), dtype=dtype, device=device) for _ in range(2))
+    sums, old = torch.full((m, n // 16), float("nan"), device=device), stream.double()
+    product = x.double() @ w.double().T + bias.double()
+    size = x.double().abs() @ w.double().abs().T + bias.abs().double()
+    after = None
+    if form.startswith("after"):
+        before = None
+        if form == "after a norm":
+            before = ops.NormedRows(None, (old ** 2).view(m, n // 16, 16).sum(-1).float().contiguous(), 1e-6)
+            old = old / torch.sqrt((old ** 2).mean(-1, keepdim=True) + 1e-6) * before_weight.double()
+        after = (before, before_weight if before is not None else None, 0.7, scale)
+        want, size = 0.7 * old + scale.double() * product, scale.abs().double() * size + old.abs()
+    else:
+        want, size = old + product, size + old.abs()
+    left = ops.linear_leave(x, ops.shuffle_weight(w), stream, weight, 1e-6, rows, sums, bias=bias,
+                            second=(second, rows2) if form == "two norms" else None, after=after)
+    close(stream, want, size, torch.float32)
+    close(rows, stream.double() * weight.double(), stream.abs().double(), dtype)         # of the stream as it was written
+    assert left.rows is rows and (left.second is not None) == (form == "two norms")
+    if left.second is not None:
+        close(left.second.rows, stream.double() * second.double(), stream.abs().double(), dtype)
+    else:
+        assert torch.isnan(rows2.float()).all()
+    torch.testing.assert_close(sums.double(), (stream.double() ** 2).view(m, n // 16, 16).sum(-1), rtol=2.0 ** -21, atol=0)
+
+
+def normed(ops, m, k, dtype, device, seed=0):
+    """`NormedRows` of float32 rows, and the rows behind the norm as the product meets them, in float64."""
+    x = rand((m, k), torch.float32, device, 2.0, seed)
+    rows = (x * (1 + rand((k,), torch.float32, device, 0.1, seed + 1))).to(dtype)
+    sums = (x.double() ** 2).view(m, k // 16, 16).sum(-1).float().contiguous()
+    return ops.NormedRows(rows, sums, 1e-5), rows.double() / torch.sqrt((x.double() ** 2).mean(-1, keepdim=True) + 1e-5)
+
+
+# products of whole K and of K ranges, of two waves (more than a round of workgroups) and four, gated ones of either kernel
+TAKES = [(1, 64, 64), (16, 1152, 896), (3, 9472, 3584), (8, 8192, 2048), (16, 4608, 3584), (2, 20000, 896), (5, 37888, 3584)]
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("m,n,k", TAKES)
+@pytest.mark.parametrize("form", ["plain", "float32", "sums", "gated", "activation"])
+def test_rows_taken(ops, device, dtype, m, n, k, form):
+    if form == "gated":
+        n = n // 32 * 32
+    x, rows = normed(ops, m, k, dtype, device)
+    w, bias = rand((n, k), dtype, device, k ** -0.5, 2), rand((n,), torch.float32, device, 0.1, 3)
+    want, size = rows @ w.double().T, rows.abs() @ w.double().abs().T
+    weight = ops.shuffle_weight(w)
+    if form == "sums":
+        splits = ops.linear_partial_splits_rows(weight, m)
+        got = ops.linear_normed(x, weight, partial=torch.full((splits, m, n), float("nan"), device=device))
+        return close(got.double().sum(0), want, size, torch.float32)
+    want, size = want + bias.double(), size + bias.abs().double()
+    if form == "gated":
+        got = ops.linear_normed(x, weight, torch.empty(m, n // 2, dtype=dtype, device=device), bias=bias, activation="silu")
+        gate, up = (v.view(m, n // 32, 2, 16)[:, :, i].reshape(m, -1) for v in (want,) for i in (0, 1))
+        gs, us = (v.view(m, n // 32, 2, 16)[:, :, i].reshape(m, -1) for v in (size,) for i in (0, 1))
+        # (silu's slope is below 1.1)
+        return close(got, gate * torch.sigmoid(gate) * up, 1.1 * gs * up.abs() + us * gate.abs() + 2.0 ** -4 * (gate * up).abs(), dtype)
+    if form == "activation":
+        got = ops.linear_normed(x, weight, torch.empty(m, n, dtype=dtype, device=device), bias=bias, activation="relu_squared")
+        return close(got, want.clamp(min=0) ** 2, 2 * size * want.abs() + 2.0 ** -18 * size ** 2, dtype)
+    workspace = torch.empty(ops.linear_workspace_bytes(dtype, m, n, k) // 4 + 4, device=device)
+    out = torch.empty(m, n, dtype=torch.float32 if form == "float32" else dtype, device=device)
+    close(ops.linear_normed(x, weight, out, bias=bias, workspace=workspace), want, size, out.dtype)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("with_norms", [False, True])
+@pytest.mark.parametrize("m,q_heads,kv_heads,dim,rot,adjacent,k", [(1, 14, 2, 64, 64, False, 896), (16, 2, 1, 128, 64, False, 256), (7, 4, 4, 48, 32, True, 320),
+                                                                 (9, 3, 1, 16, 16, False, 2048), (2, 1, 1, 80, 0, False, 128), (16, 16, 4, 256, 256, True, 64)])
+def test_rotated_product(ops, device, dtype, with_norms, m, q_heads, kv_heads, dim, rot, adjacent, k):
+    """Against the product, then `rope_kv_write`: the same values but for the product's float32 order."""
+    width, page = (q_heads + 2 * kv_heads) * dim, 16
+    x, rows = normed(ops, m, k, dtype, device)
+    w, bias = rand((width, k), dtype, device, k ** -0.5, 2), rand((width,), torch.float32, device, 0.1, 3)
+    angle = torch.arange(m * max(rot // 2, 1), device=device).view(m, -1)[:, :rot // 2].float() * 0.37
+    cos, sin = (angle.cos(), angle.sin()) if rot else (None, None)
+    slots = torch.tensor([(5 * i + 3) % (4 * page) if i != 4 else -1 for i in range(m)], dtype=torch.int32, device=device)
+    keys, values = (torch.full((4, kv_heads, page, dim), -9.0, dtype=dtype, device=device) for _ in range(2))
+    want_keys, want_values = keys.clone(), values.clone()
+    if not with_norms:
+        x, rows = x.rows, x.rows.double()
+    qkv = torch.full((m, width), -9.0, dtype=dtype, device=device)
+    ops.linear_rotate(x, ops.shuffle_weight(w), qkv, cos, sin, slots, keys, values, q_heads, kv_heads, dim, page, bias=bias, adjacent=adjacent)
+    product = rows @ w.double().T + bias.double()
+    size = rows.abs() @ w.double().abs().T + bias.abs().double()
+    want = product.to(dtype)
+    ops.rope_kv_write(want, cos, sin, slots, want_keys, want_values, q_heads, kv_heads, dim, page, adjacent=adjacent)
+    # the product's own error, a rounding of either element of a pair that falls the other way, and the rotated one's: at most a pair's sizes
+    slack = 2.0 ** -18 * float(size.max()) + 6 * BITS[dtype] * float(product.abs().max())
+    torch.testing.assert_close(qkv[:, :q_heads * dim].float(), want[:, :q_heads * dim].float(), atol=slack, rtol=0)
+    torch.testing.assert_close(keys.float(), want_keys.float(), atol=slack, rtol=0)
+    torch.testing.assert_close(values.float(), want_values.float(), atol=slack, rtol=0)
+    assert (keys == want_keys).float().mean() > (0.9 if dtype == torch.bfloat16 else 0.1) and ((keys == -9) == (want_keys == -9)).all()
+    before = keys.clone()
+    ops.linear_rotate(x, ops.shuffle_weight(w), qkv, cos, sin, None, None, None, q_heads, kv_heads, dim, page, write_cache=False, bias=bias, adjacent=adjacent)
+    assert torch.equal(before, keys)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("hidden", [64, 2048, 4096])
+def test_residual_norm_of_rows_behind_a_norm(ops, device, dtype, hidden):
+    x, y = rand((16, hidden), torch.float32, device, 3.0), rand((3, 16, hidden), torch.float32, device, 1.0, 1)
+    w, before, scale = (1 + rand((hidden,), torch.float32, device, 0.1, s) for s in (2, 3, 4))
+    out = torch.empty(16, hidden, dtype=dtype, device=device)
+    unit = lambda v: v / torch.sqrt((v ** 2).mean(-1, keepdim=True) + 1e-6)       # noqa: E731
+    want = unit(0.7 * unit(x.double()) * before.double() + scale.double() * y.double().sum(0)) * w.double()
+    ops.residual_norm(x, w, 1e-6, out=out, add=y, scale=scale, alpha=0.7, before=before)
+    torch.testing.assert_close(x.double(), want, atol=3e-6, rtol=3e-6)             # (as this kernel's other forms)
+    torch.testing.assert_close(out, x.to(dtype), atol=0, rtol=0)
