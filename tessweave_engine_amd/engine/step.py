@@ -53,6 +53,8 @@ SECOND_FORM_MISSES = 16      # a captured step's other form (cut into segments o
 MAX_GRAPHS = 96              # captured steps kept (one per batch size and length class met); the least recently
                              # replayed one goes first
 
+MAX_VIEWS = 128              # cuts of the metadata buffer kept (see Stepper._cut)
+
 
 class _Graph:
     """A captured decode step in one or both of two forms, {cut into segments?: (graphs launched one after the other, the
@@ -90,9 +92,10 @@ class _Staging:
     The kernel that fetches a step's metadata reads its buffer when it runs. The allocator of pinned memory does not know
     of it and would hand the memory to its next taker at once, so the buffers are let go only once their readers are done."""
 
-    def __init__(self, words, count=4):
+    def __init__(self, words, device_words, count=4):
         self.buffers = [torch.zeros(words, dtype=torch.int32, pin_memory=True) for _ in range(count)]
         self.arrays = [t.numpy() for t in self.buffers]
+        self.uploads = [ops.WordUpload(t, device_words) for t in self.buffers]
         self.readers = [None] * count        # per buffer: an event behind its last reader
         self.next = 0
 
@@ -179,7 +182,9 @@ class Stepper:
         self._sections, self._meta_ints = sections, offset
         self._meta_dev = torch.zeros(offset, dtype=torch.int32, device=self.device)
         self._staging = None                 # (the old buffers go first)
-        self._staging = _Staging(offset)
+        self._staging = _Staging(offset, self._meta_dev)
+        self._views = OrderedDict()          # (tokens, requests, wanted rows) -> the buffer's sections cut to them, least recently used first
+        self._counting = np.arange(max(max_tokens, max_seqs) + 1)
         # a first step on another stream comes behind this stream's work: the clearing of the new buffers, and the model's and
         # the cache's initialisation if they were made here
         self._mark(stream)
@@ -187,6 +192,25 @@ class Stepper:
     def _dev(self, name, count=None):
         off, cap = self._sections[name]
         return self._meta_dev[off:off + (cap if count is None else count)]
+
+    def _cut(self, n_tokens, n_seqs, n_logits):
+        """The metadata buffer's sections as a step of these counts sees them. (They are the same tensors whenever the counts are: a
+        decode step's are made once, 25 us of host time.)"""
+        key = (n_tokens, n_seqs, n_logits)
+        hit = self._views.get(key)
+        if hit is None:
+            width, axes = self.cache.table_width, self.position_axes
+            hit = self._views[key] = (
+                self._dev("token_ids", n_tokens), self._dev("positions", axes * n_tokens).view(axes, n_tokens), self._dev("q_start", n_seqs + 1),
+                self._dev("kv_len", n_seqs), self._dev("state_slots", n_seqs), self._dev("state_phase", n_seqs),
+                self._dev("kv_page_start", n_seqs + 1), self._dev("logit_rows", n_logits),
+                [GroupStep(self._dev(f"table{g}", n_seqs * width).view(n_seqs, width), self._dev(f"slots{g}", n_tokens))
+                 for g in range(len(self.cache.pools))])
+            while len(self._views) > MAX_VIEWS:
+                self._views.popitem(last=False)
+        else:
+            self._views.move_to_end(key)
+        return hit
 
     def _drop_graphs(self):
         if self._graphs:
@@ -298,7 +322,7 @@ class Stepper:
     def _upload(self, ctx):
         k = ctx.staging_index
         if ctx.staging_segments is not None and len(ctx.staging_segments) <= 16:
-            ops.upload_words(self._staging.buffers[k], self._meta_dev, ctx.staging_segments)
+            self._staging.uploads[k].run(ctx.staging_segments)
         else:
             self._meta_dev.copy_(self._staging.buffers[k], non_blocking=True)
 
@@ -317,7 +341,7 @@ class Stepper:
             seen.add(id(e.seq))
             if e.seq.closed:
                 raise ValueError(f"request {e.seq.id!r} is closed")
-            if any(type(t) is not int or t >= vocab or t < -feed for t in e.tokens):
+            if set(map(type, e.tokens)) != {int} or max(e.tokens) >= vocab or min(e.tokens) < -feed:
                 raise ValueError(f"request {e.seq.id!r}: token ids must be integers in [0, {vocab})")
             if any(type(w) is not int or w < 0 or w >= len(e.tokens) for w in e.want):
                 raise ValueError(f"request {e.seq.id!r}: wanted places must index this step's tokens")
@@ -331,24 +355,29 @@ class Stepper:
             self.cache.ensure(e.seq, e.seq.computed + len(e.tokens))
 
         # decode entries (one token) first, then prompt portions; stable
-        order = sorted(range(len(entries)), key=lambda i: len(entries[i].tokens) != 1)
-        ordered = [entries[i] for i in order]
-        n_seqs = len(ordered)
-        q_lens = np.fromiter((len(e.tokens) for e in ordered), dtype=np.int64, count=n_seqs)
-        n_decode = int((q_lens == 1).sum())
-        computed = np.fromiter((e.seq.computed for e in ordered), dtype=np.int64, count=n_seqs)
-        slots_of = np.fromiter((e.seq.state_slot for e in ordered), dtype=np.int64, count=n_seqs)
-        q_start = np.zeros(n_seqs + 1, dtype=np.int64)
-        np.cumsum(q_lens, out=q_start[1:])
-        kv_len = computed + q_lens
-        seq_of_token = np.repeat(np.arange(n_seqs), q_lens)
-        positions = np.arange(n_tokens) - np.repeat(q_start[:-1] - computed, q_lens)
-        if n_decode == n_seqs:
-            token_ids = np.fromiter((e.tokens[0] for e in ordered), dtype=np.int64, count=n_seqs)
+        n_seqs = len(entries)
+        n_decode = sum(len(e.tokens) == 1 for e in entries)
+        if n_decode == n_seqs:               # (a step that only decodes: everything below counts requests)
+            ordered = entries
+            q_lens, q_start, seq_of_token = self._counting[1:2].repeat(n_seqs), self._counting[:n_seqs + 1], self._counting[:n_seqs]
+            positions = computed = np.array([e.seq.computed for e in ordered], dtype=np.int64)
+            kv_len = computed + 1
+            token_ids = [e.tokens[0] for e in ordered]
+            rows = [i for i, e in enumerate(entries) for _ in e.want]
         else:
+            order = sorted(range(n_seqs), key=lambda i: len(entries[i].tokens) != 1)
+            ordered = [entries[i] for i in order]
+            q_lens = np.array([len(e.tokens) for e in ordered], dtype=np.int64)
+            computed = np.array([e.seq.computed for e in ordered], dtype=np.int64)
+            q_start = np.zeros(n_seqs + 1, dtype=np.int64)
+            np.cumsum(q_lens, out=q_start[1:])
+            kv_len = computed + q_lens
+            seq_of_token = np.repeat(self._counting[:n_seqs], q_lens)
+            positions = self._counting[:n_tokens] - np.repeat(q_start[:-1] - computed, q_lens)
             token_ids = np.concatenate([np.asarray(e.tokens, dtype=np.int64) for e in ordered])
-        position_in_order = {orig: pos for pos, orig in enumerate(order)}
-        rows = [int(q_start[position_in_order[i]]) + w for i, e in enumerate(entries) for w in e.want]
+            position_in_order = {orig: pos for pos, orig in enumerate(order)}
+            rows = [int(q_start[position_in_order[i]]) + w for i, e in enumerate(entries) for w in e.want]
+        state_slots = [e.seq.state_slot for e in ordered]
         n_logits = len(rows)
 
         # pack the metadata into a pinned buffer and upload it once
@@ -364,29 +393,36 @@ class Stepper:
 
         put("token_ids", token_ids)
         axes = self.position_axes
-        ids = np.tile(positions, (axes, 1))                      # [axes, n_tokens]; `positions` stays the token order
-        for s_index, e in enumerate(ordered):
-            if e.positions is not None:
-                ids[:, q_start[s_index]:q_start[s_index + 1]] = np.asarray(e.positions, dtype=np.int64)
-        put("positions", ids.reshape(-1))
+        if axes == 1 and not any(e.positions is not None for e in ordered):
+            put("positions", positions)
+        else:
+            ids = np.tile(positions, (axes, 1))                  # [axes, n_tokens]; `positions` stays the token order
+            for s_index, e in enumerate(ordered):
+                if e.positions is not None:
+                    ids[:, q_start[s_index]:q_start[s_index + 1]] = np.asarray(e.positions, dtype=np.int64)
+            put("positions", ids.reshape(-1))
         put("q_start", q_start)
         put("kv_len", kv_len)
-        put("state_slots", slots_of)
-        put("state_phase", np.fromiter((e.seq.steps & 1 for e in ordered), dtype=np.int64, count=n_seqs))
-        put("logit_rows", np.asarray(rows, dtype=np.int64))
+        put("state_slots", state_slots)
+        put("state_phase", [e.seq.steps & 1 for e in ordered])
+        put("logit_rows", rows)
         page = self.cache.page_size
         kv_page_start = np.zeros(n_seqs + 1, dtype=np.int64)
         np.cumsum((kv_len + page - 1) // page, out=kv_page_start[1:])
         put("kv_page_start", kv_page_start)
         width = self.cache.table_width
+        page_of, place = np.divmod(positions, page)
         for g in range(len(self.cache.pools)):
-            tables = self.cache.table_rows[g][slots_of]                       # [n_seqs, width]
-            pages = tables[seq_of_token, positions // page]
-            first = self._first_positions(g, computed)
-            live = positions >= np.repeat(first, q_lens)
-            if (pages[live] < 0).any():
-                raise RuntimeError("a token's page is not held; the cache manager and the step disagree")
-            put(f"slots{g}", np.where(pages >= 0, pages * page + positions % page, -1))
+            tables = self.cache.table_rows[g][state_slots]                    # [n_seqs, width]
+            pages = tables[seq_of_token, page_of]
+            missing = pages < 0
+            if missing.any():                # (only behind a window may they be)
+                live = positions >= np.repeat(self._first_positions(g, computed), q_lens)
+                if missing[live].any():
+                    raise RuntimeError("a token's page is not held; the cache manager and the step disagree")
+                put(f"slots{g}", np.where(missing, -1, pages * page + place))
+            else:
+                put(f"slots{g}", pages * page + place)
             off, _ = self._sections[f"table{g}"]
             host[off:off + n_seqs * width] = tables.reshape(-1)
             segments.append((off, n_seqs * width))
@@ -394,20 +430,12 @@ class Stepper:
         ctx = StepContext()
         ctx.device, ctx.dtype = self.device, self.dtype
         ctx.n_tokens, ctx.n_seqs, ctx.n_decode, ctx.n_logits = n_tokens, n_seqs, n_decode, n_logits
-        ctx.token_ids = self._dev("token_ids", n_tokens)
-        ctx.positions = self._dev("positions", axes * n_tokens).view(axes, n_tokens)
-        ctx.q_start = self._dev("q_start", n_seqs + 1)
-        ctx.kv_len = self._dev("kv_len", n_seqs)
-        ctx.state_slots = self._dev("state_slots", n_seqs)
-        ctx.state_phase = self._dev("state_phase", n_seqs)
-        ctx.kv_page_start = self._dev("kv_page_start", n_seqs + 1)
+        (ctx.token_ids, ctx.positions, ctx.q_start, ctx.kv_len, ctx.state_slots, ctx.state_phase, ctx.kv_page_start, ctx.logit_rows,
+         ctx.groups) = self._cut(n_tokens, n_seqs, n_logits)
         ctx.h_kv_page_start = kv_page_start.tolist()
-        ctx.logit_rows = self._dev("logit_rows", n_logits)
-        ctx.groups = [GroupStep(self._dev(f"table{g}", n_seqs * width).view(n_seqs, width),
-                                self._dev(f"slots{g}", n_tokens)) for g in range(len(self.cache.pools))]
         ctx.h_q_start = q_start.tolist()
         ctx.h_kv_len = kv_len.tolist()
-        ctx.h_state_slots = slots_of.tolist()
+        ctx.h_state_slots = state_slots
         ctx.max_q_len = int(q_lens[n_decode:].max()) if n_decode < n_seqs else 0
         ctx.max_kv_len = int(kv_len.max())
         ctx.kv_capacity = width * page
