@@ -223,10 +223,15 @@ __global__ void rmsnorm_vec4_kernel(float* __restrict__ x, const float* __restri
   }
 }
 
-// Many rows: one WAVE per row (4 rows per workgroup), a row of up to 256 * NG elements in registers as
+// Many rows of up to 4,096 elements: one WAVE per row (4 rows per workgroup), a row in registers as
 // up to NG groups of 4, every load of a pass issued at once, and no barrier: the sum of squares is a wave
-// reduction. (With one workgroup of 896 threads per row, 2,048 rows of 3,584 took 15 us.) With ADD the
-// row is (sum_s add[s]) + x, added in that order as everywhere, and written back to x.
+// reduction. With ADD the row is (sum_s add[s]) + x, added in that order as everywhere, and written back to x.
+// Rows whose workgroups of the kernel above are all there at once (2,048 threads a CU) are that kernel's, and so are longer rows, of
+// which a wave's registers hold half at a time: the loads of many waves cover each other's latency. (us, two partial sums, a wave a row / a
+// workgroup a row: 2,048 wide, 256, 536, 1,024 and 2,048 rows 5.5 / 3.5, 6.1 / 4.9, 6.9 / 6.2, 13.8 / 14.3; 3,584 wide, 256, 536, 800, 2,048 rows 7.1 / 4.4,
+// 8.6 / 7.7, 10.7 / 10.9, 20.9 / 23.7; 5,120 wide, 256, 536, 1,024, 2,048 rows 10.8 / 5.4, 13.9 / 10.5, 19.4 / 17.4, 36.6 / 31.5; 8,192 wide 18.1 / 6.6 and, 4,096
+// rows, 126 / 112.)
+#define TW_THREADS_AT_ONCE (2048 * 256)
 template <typename T, int NG, bool ADD>
 __global__ __launch_bounds__(256) void rmsnorm_wave_kernel(float* __restrict__ x, const float* __restrict__ w,
                                                            T* __restrict__ out, int n_rows, int hidden, float eps,
@@ -239,35 +244,30 @@ __global__ __launch_bounds__(256) void rmsnorm_wave_kernel(float* __restrict__ x
   f32x4 v[NG];
   float ss = 0.f;
   if (ADD) {
-    // CH groups at a time (a whole row of up to 4,096 elements, half of a longer one): the row's own
-    // values and one split's sums are in flight together
-    constexpr int CH = NG <= 16 ? NG : 16;
+    // the row's own values and one split's sums are in flight together
     const float* p = add + (size_t)row * hidden;
+    f32x4 xv[NG], acc[NG];
 #pragma unroll
-    for (int c = 0; c < NG; c += CH) {
-      f32x4 xv[CH], acc[CH];
+    for (int j = 0; j < NG; ++j) {
+      const int h = (j * 64 + lane) * 4;
+      xv[j] = h < hidden ? *reinterpret_cast<const f32x4*>(src + h) : f32x4{0.f, 0.f, 0.f, 0.f};
+      acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+    for (int s = 0; s < add_splits; ++s) {
+      f32x4 a[NG];
 #pragma unroll
-      for (int j = 0; j < CH; ++j) {
-        const int h = ((c + j) * 64 + lane) * 4;
-        xv[j] = h < hidden ? *reinterpret_cast<const f32x4*>(src + h) : f32x4{0.f, 0.f, 0.f, 0.f};
-        acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
-      }
-      for (int s = 0; s < add_splits; ++s) {
-        f32x4 a[CH];
-#pragma unroll
-        for (int j = 0; j < CH; ++j) {
-          const int h = ((c + j) * 64 + lane) * 4;
-          a[j] = h < hidden ? *reinterpret_cast<const f32x4*>(p + s * add_stride + h) : f32x4{0.f, 0.f, 0.f, 0.f};
-        }
-#pragma unroll
-        for (int j = 0; j < CH; ++j) acc[j] = acc[j] + a[j];
+      for (int j = 0; j < NG; ++j) {
+        const int h = (j * 64 + lane) * 4;
+        a[j] = h < hidden ? *reinterpret_cast<const f32x4*>(p + s * add_stride + h) : f32x4{0.f, 0.f, 0.f, 0.f};
       }
 #pragma unroll
-      for (int j = 0; j < CH; ++j) {
-        const int h = ((c + j) * 64 + lane) * 4;
-        v[c + j] = acc[j] + xv[j];
-        if (h < hidden) *reinterpret_cast<f32x4*>(src + h) = v[c + j];
-      }
+      for (int j = 0; j < NG; ++j) acc[j] = acc[j] + a[j];
+    }
+#pragma unroll
+    for (int j = 0; j < NG; ++j) {
+      const int h = (j * 64 + lane) * 4;
+      v[j] = acc[j] + xv[j];
+      if (h < hidden) *reinterpret_cast<f32x4*>(src + h) = v[j];
     }
   } else {
 #pragma unroll
@@ -312,13 +312,8 @@ template <typename T>
 static void launch_rmsnorm_wave(int n_out, hipStream_t stream, float* x, const float* w, T* out, int hidden,
                                 float eps, const float* add, int add_splits, size_t add_stride) {
   const int grid = (n_out + 3) / 4;
-  if (hidden <= 4096) {
-    if (add) rmsnorm_wave_kernel<T, 16, true><<<grid, 256, 0, stream>>>(x, w, out, n_out, hidden, eps, add, add_splits, add_stride);
-    else rmsnorm_wave_kernel<T, 16, false><<<grid, 256, 0, stream>>>(x, w, out, n_out, hidden, eps, nullptr, 0, 0);
-  } else {
-    if (add) rmsnorm_wave_kernel<T, 32, true><<<grid, 256, 0, stream>>>(x, w, out, n_out, hidden, eps, add, add_splits, add_stride);
-    else rmsnorm_wave_kernel<T, 32, false><<<grid, 256, 0, stream>>>(x, w, out, n_out, hidden, eps, nullptr, 0, 0);
-  }
+  if (add) rmsnorm_wave_kernel<T, 16, true><<<grid, 256, 0, stream>>>(x, w, out, n_out, hidden, eps, add, add_splits, add_stride);
+  else rmsnorm_wave_kernel<T, 16, false><<<grid, 256, 0, stream>>>(x, w, out, n_out, hidden, eps, nullptr, 0, 0);
 }
 
 extern "C" int tw_rmsnorm(int out_dtype, float* x, const float* w, void* out, const int* rows,
@@ -328,7 +323,7 @@ extern "C" int tw_rmsnorm(int out_dtype, float* x, const float* w, void* out, co
   TW_REQUIRE(add == nullptr || (add_splits > 0 && (rows == nullptr || row_scratch != nullptr)));
   if (n_out == 0) return 0;
   if (out_dtype != TW_DTYPE_F32 && out_dtype != TW_DTYPE_BF16) return TW_ERR_BAD_ARGUMENT;
-  if (rows == nullptr && n_out >= 256 && hidden % 4 == 0 && hidden <= 8192 &&
+  if (rows == nullptr && n_out >= 256 && hidden % 4 == 0 && hidden <= 4096 && (long)n_out * (hidden / 4) > TW_THREADS_AT_ONCE &&
       (uintptr_t)x % 16 == 0 && (uintptr_t)w % 16 == 0 && (uintptr_t)out % 16 == 0 &&
       (add == nullptr || ((uintptr_t)add % 16 == 0 && add_stride % 4 == 0))) {
     if (out_dtype == TW_DTYPE_F32)

@@ -99,6 +99,22 @@ def test_rmsnorm(ops, device, dtype, hidden, eps):
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("n,hidden", [(513, 4096), (512, 4096), (2101, 1000), (8200, 256), (700, 5120)])
+def test_rmsnorm_of_so_many_rows_that_a_wave_takes_each(ops, device, dtype, n, hidden):
+    """Beyond 2,048 threads a CU of row workgroups (and, for comparison, just not and for longer rows): with and without partial sums."""
+    x, w = rand((n, hidden), torch.float32, device, 3.0), 1 + rand((hidden,), torch.float32, device, 0.1, seed=1)
+    out = torch.full((n, hidden), float("nan"), dtype=dtype, device=device)
+    ops.rmsnorm(x, w, 1e-6, out)
+    unit = lambda v: (v / torch.sqrt((v ** 2).mean(-1, keepdim=True) + 1e-6) * w.double()).float()      # noqa: E731
+    torch.testing.assert_close(out.float(), unit(x.double()), **tol(dtype, (3e-6, 3e-6), (1e-2, 1e-2)))
+    add = rand((2, n, hidden), torch.float32, device, 1.0, seed=2)
+    total = x.double() + add.double().sum(0)
+    ops.rmsnorm(x, w, 1e-6, out, add=add)
+    torch.testing.assert_close(x, total.float(), atol=1e-5, rtol=1e-6)
+    torch.testing.assert_close(out.float(), unit(total), **tol(dtype, (3e-6, 3e-6), (1e-2, 1e-2)))
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("q_heads,kv_heads,head_dim,page,theta", [(4, 2, 16, 16, 1e4), (6, 1, 32, 8, 1e6), (5, 5, 48, 4, 5e5),
                                                                  (3, 1, 20, 8, 1e4), (28, 4, 128, 16, 1e6),
                                                                  (4, 2, 32, 12, 1e4), (2, 1, 64, 24, 1e6), (3, 3, 16, 48, 1e4)])
