@@ -38,7 +38,8 @@ _SIGNATURES = {
     "tw_linear_leave": (I, [I, P, L, P, L, P, P, L, I, I, I, P, P, P, P, P, I, P, P, P, F, F, P]),
     "tw_linear_rotate_pays": (I, [I, I, I, I]),
     "tw_linear_rotate": (I, [I, P, L, P, I, I, F, P, L, P, P, L, I, I, P, P, P, P, P, I, I, I, I, I, I, I, P]),
-    "tw_attn_decode_splits": (I, [I, I, I, I]),
+    "tw_attn_decode_splits": (I, [I, I, I, I, I, I]),
+    "tw_attn_decode_most_splits": (I, [I, I, I, I, I, I, I]),
     "tw_attn_decode_workspace_floats": (L, [I, I, I, I]),
     "tw_attn_decode": (I, [I, P, L, P, P, P, I, P, P, I, I, P, L, P, L, I, I, I, I, I, I, F, F, I, I, P, P, I, P]),
     "tw_attn_prefill_split": (I, [I, I, I, I, I, I, ctypes.POINTER(c_int), ctypes.POINTER(c_int)]),

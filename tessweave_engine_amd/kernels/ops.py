@@ -544,8 +544,17 @@ def linear_rotate(x, weight, qkv, cos, sin, slots, keys, values, q_heads, kv_hea
     return qkv
 
 
-def attn_decode_splits(n_seqs, q_heads, kv_heads, max_kv_len):
-    return int(library().tw_attn_decode_splits(n_seqs, q_heads, kv_heads, max_kv_len))
+def attn_decode_splits(n_seqs, q_heads, kv_heads, max_kv_len, head_dim=128, dtype=torch.bfloat16):
+    """Key ranges for `attn_decode`."""
+    return int(library().tw_attn_decode_splits(dtype_id(dtype), n_seqs, q_heads, kv_heads, head_dim, max_kv_len))
+
+
+def attn_decode_class_splits(n_seqs, q_heads, kv_heads, bound, capacity, span, head_dim, dtype):
+    """(key ranges for steps whose longest sequence lies in the class up to BOUND keys, the most that any class up to CAPACITY asks for):
+    of a class the middle is taken, of which a query sees at most SPAN keys (0: all)."""
+    span, shape = span or 1 << 30, (dtype_id(dtype), n_seqs, q_heads, kv_heads, head_dim)
+    splits = int(library().tw_attn_decode_splits(*shape, min(max(1, bound * 3 // 4), span)))
+    return splits, max(splits, int(library().tw_attn_decode_most_splits(*shape, capacity, span)))
 
 
 def attn_decode_workspace_floats(n_seqs, q_heads, head_dim, splits):

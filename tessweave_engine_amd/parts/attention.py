@@ -29,17 +29,12 @@ def paged_attention(ctx, q, keys, values, group, out, q_heads, kv_heads, head_di
     extras = dict(chunk=chunk, sink=sink, gate=gate)
     span = window or chunk                                 # most keys a query sees (0: all before it)
     if ctx.n_decode:
-        # A captured step is replayed for other lengths: its split count follows the step's length
-        # class (the kernel itself cuts each sequence's own keys into that many ranges).
-        longest = ctx.kv_bound if ctx.capturing else ctx.max_kv_len
-        if span:
-            longest = min(longest, span)
-        splits = ops.attn_decode_splits(ctx.n_decode, q_heads, kv_heads, longest)
+        # A captured step is replayed for other lengths: the split count follows the step's length class (the kernel itself cuts
+        # each sequence's own keys into that many ranges), and the scratch memory the most that any class asks for, so that it never
+        # grows under a capture.
+        splits, most = ops.attn_decode_class_splits(ctx.n_decode, q_heads, kv_heads, ctx.kv_bound, ctx.kv_capacity, span, head_dim, q.dtype)
         ws = None
         if splits > 1:
-            # sized for the most splits any length class can ask for, so that it never grows under a capture
-            most = max(splits, ops.attn_decode_splits(ctx.n_decode, q_heads, kv_heads,
-                                                      min(ctx.kv_capacity, span) if span else ctx.kv_capacity))
             floats = ops.attn_decode_workspace_floats(ctx.n_decode, q_heads, head_dim, most)
             ws = ctx.workspace.get("attn.split", (floats,), torch.float32)
         ops.attn_decode(q, keys, values, group.block_table, ctx.q_start, ctx.kv_len, 0, ctx.n_decode, out,
