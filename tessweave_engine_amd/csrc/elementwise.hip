@@ -2,6 +2,7 @@
 // write, SiLU-multiply. Statistics, angles and products are float32; storage
 // is float32 or bfloat16. The residual stream is float32 in both precisions.
 #include "tw_common.h"
+#include "rope_tables.h"
 
 // ---- embedding: x[n, :] = float(E[ids[n], :]) ------------------------------------
 // A negative id -1 - k stands for feed[k]: a token that an earlier kernel on this stream wrote
@@ -51,6 +52,67 @@ extern "C" int tw_embed_gather(int dtype, const int* ids, const void* table, flo
     launch_embed_gather<bf16_t>(ids, table, out, n, hidden, vocab, feed, feed_count, stream);
   else
     return TW_ERR_BAD_ARGUMENT;
+  return TW_LAUNCH_RESULT();
+}
+
+// ---- what a decode step begins with, in one launch: token rows, what their first reader wants, and the rotary tables ------------
+// x[n] = float(table[ids[n]]) as above, a thread four elements; beside it either the rows for a norm that travels (rows = x * weight
+// rounded, a second norm's, sums of squares of 16 columns: see RowNorms in gemm.hip) or the rows rounded as they are. The
+// workgroups behind the rows' form the tables, which need nothing of the rows. (Each of these was a launch of its own in front of the
+// first product, 2 us in a captured step.)
+struct EmbedBegin {
+  const int *ids, *feed;
+  const void* table;
+  float* x;
+  const float *weight, *weight2;      // [hidden] or null
+  void *rows, *rows2;                 // [n][hidden] in the table's type, or null; without `weight`: rows is x rounded
+  float* sums;                        // [n][hidden / 16], with `weight`
+  int n_feed, hidden, vocab, shares, row_blocks;
+};
+
+template <typename T>
+__global__ __launch_bounds__(256) void embed_begin_kernel(EmbedBegin a, RopeTables tables) {
+  if ((int)blockIdx.x >= a.row_blocks) return tw_rope_block(tables, blockIdx.x - a.row_blocks);
+  const int n = blockIdx.x / a.shares, h = ((blockIdx.x % a.shares) * 256 + threadIdx.x) * 4;
+  if (h >= a.hidden) return;                                            // (hidden % 16 == 0: four lanes of 16 columns stay or go together)
+  int id = a.ids[n];
+  f32x4 w = {0.f, 0.f, 0.f, 0.f}, w2 = w;
+  if (a.weight) w = *reinterpret_cast<const f32x4*>(a.weight + h);
+  if (a.weight2) w2 = *reinterpret_cast<const f32x4*>(a.weight2 + h);
+  if (id < 0 && a.feed != nullptr && -1 - id < a.n_feed) id = a.feed[-1 - id];
+  id = id < 0 ? 0 : (id >= a.vocab ? a.vocab - 1 : id);                // ids are validated on the host; never read outside
+  typedef T Four __attribute__((ext_vector_type(4)));
+  const Four v = *reinterpret_cast<const Four*>((const T*)a.table + (size_t)id * a.hidden + h);
+  const f32x4 x = {tw_to_float(v[0]), tw_to_float(v[1]), tw_to_float(v[2]), tw_to_float(v[3])};
+  const size_t at = (size_t)n * a.hidden + h;
+  *reinterpret_cast<f32x4*>(a.x + at) = x;
+  auto four = [](f32x4 r) { return Four{tw_from_float<T>(r[0]), tw_from_float<T>(r[1]), tw_from_float<T>(r[2]), tw_from_float<T>(r[3])}; };
+  if (a.weight) {
+    *reinterpret_cast<Four*>((T*)a.rows + at) = four(f32x4{x[0] * w[0], x[1] * w[1], x[2] * w[2], x[3] * w[3]});
+    if (a.weight2) *reinterpret_cast<Four*>((T*)a.rows2 + at) = four(f32x4{x[0] * w2[0], x[1] * w2[1], x[2] * w2[2], x[3] * w2[3]});
+    float sq = (x[0] * x[0] + x[1] * x[1]) + (x[2] * x[2] + x[3] * x[3]);
+    sq += tw_dpp<TW_SWAP_2>(sq);
+    sq += tw_dpp<TW_SWAP_1>(sq);
+    if (h % 16 == 0) a.sums[(size_t)n * (a.hidden / 16) + h / 16] = sq;
+  } else if (a.rows) {
+    *reinterpret_cast<Four*>((T*)a.rows + at) = v;
+  }
+}
+
+extern "C" int tw_embed_begin(int dtype, const int* ids, const void* table, float* x, int n, int hidden, int vocab, const int* feed, int n_feed,
+                              const float* weight, void* rows, const float* weight2, void* rows2, float* sums, const RopeTables* tables,
+                              hipStream_t stream) {
+  TW_REQUIRE(ids && table && x && n >= 0 && hidden > 0 && hidden % 16 == 0 && vocab > 0 && n_feed >= 0 && tables && tw_rope_tables_ok(*tables, n));
+  TW_REQUIRE((weight == nullptr || (rows && sums)) && (weight2 == nullptr || (weight && rows2)));
+  TW_REQUIRE((((uintptr_t)table | (uintptr_t)x | (uintptr_t)weight | (uintptr_t)weight2 | (uintptr_t)rows | (uintptr_t)rows2) & 15) == 0);
+  if (n == 0) return 0;
+  const int shares = tw_div_up(hidden / 4, 256);
+  TW_REQUIRE((long)n * shares < (1L << 30));
+  const EmbedBegin a = {ids, feed, table, x, weight, weight2, rows, rows2, sums, n_feed, hidden, vocab, shares, n * shares};
+  const int grid = a.row_blocks + tw_rope_blocks(*tables);
+  if (dtype == TW_DTYPE_BF16) embed_begin_kernel<bf16_t><<<grid, 256, 0, stream>>>(a, *tables);
+  else if (dtype == TW_DTYPE_F32) embed_begin_kernel<float><<<grid, 256, 0, stream>>>(a, *tables);
+  else return TW_ERR_BAD_ARGUMENT;
   return TW_LAUNCH_RESULT();
 }
 
@@ -355,37 +417,17 @@ extern "C" int tw_rmsnorm(int out_dtype, float* x, const float* w, void* out, co
   return TW_LAUNCH_RESULT();
 }
 
-// ---- rotary tables: cos/sin[n, j] of angle = float(position[n]) * inv_freq[j], times `magnitude` -----
-// (1 for the plain encoding; encodings that stretch their frequencies for longer contexts also scale both tables)
-// rest (or null): what float32 rounded off the frequencies; the angle then carries the product's rounding error and this
-// one beside it (at position 1,000 a float32 product alone is off by up to 3e-5).
-__global__ void rope_table_kernel(const int* __restrict__ positions, const float* __restrict__ inv_freq, const float* __restrict__ rest,
-                                  float* __restrict__ cos_out, float* __restrict__ sin_out, int n, int half,
-                                  float magnitude) {
+// ---- rotary tables (see rope_tables.h) -----------------------------------------------------------------
+__global__ void rope_table_kernel(RopeTable a, const int* __restrict__ positions, int entries) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n * half) return;
-  const int t = i / half, j = i % half;
-  const float p = (float)positions[t], f = inv_freq[j];
-  const float angle = __fmul_rn(p, f);
-  float c = cosf(angle), s = sinf(angle);
-  if (rest) {
-    const float off = __fmaf_rn(p, rest[j], __fmaf_rn(p, f, -angle));      // (a few hundredths at most)
-    const float off2 = off * off;
-    const float so = off * __fmaf_rn(-off2, 1.f / 6.f, 1.f), co = -0.5f * off2;
-    const float sine = __fmaf_rn(so, c, __fmaf_rn(co, s, s));
-    c = __fmaf_rn(-so, s, __fmaf_rn(co, c, c));
-    s = sine;
-  }
-  cos_out[i] = c * magnitude;
-  sin_out[i] = s * magnitude;
+  if (i < entries) tw_rope_entry(a, positions, i);
 }
 
 extern "C" int tw_rope_table(const int* positions, const float* inv_freq, const float* rest, float* cos_out, float* sin_out,
                              int n, int half, float magnitude, hipStream_t stream) {
   TW_REQUIRE(n >= 0 && half > 0);
   if (n == 0) return 0;
-  rope_table_kernel<<<tw_div_up((long)n * half, 256), 256, 0, stream>>>(positions, inv_freq, rest, cos_out,
-                                                                       sin_out, n, half, magnitude);
+  rope_table_kernel<<<tw_div_up((long)n * half, 256), 256, 0, stream>>>(RopeTable{inv_freq, rest, cos_out, sin_out, half, magnitude}, positions, n * half);
   return TW_LAUNCH_RESULT();
 }
 

@@ -8,6 +8,7 @@
 // state slot. Everything here is float32 arithmetic; only inputs that come from a projection and outputs
 // that feed one have the compute type.
 #include "tw_common.h"
+#include "rope_tables.h"
 #include <type_traits>
 
 __device__ __forceinline__ float tw_gelu_tanh(float z) {
@@ -901,6 +902,7 @@ extern "C" int tw_layer_end(float* x, const float* y, const float* w, float eps,
 // token of a sequence is part of the request's state: int32 [requests][2], copy `phase` read, the other copy
 // written by the block of the sequence's last token (so no block reads what another block of the launch writes).
 // A token id -1 - k stands for feed[k]. The normed row goes to x (float32) and, rounded, to out.
+// The workgroups behind the rows' form rotary tables (see embed_begin_kernel).
 // VEC: rows of whole 16-byte pieces, at most four a thread, and more than 256 elements (of fewer, most threads have none and the
 // others eight in a row instead of one: 64 elements, 8,192 tokens 10.1 / 12.1 us element by element / in pieces, 256 12.8 / 13.2, 384 14.5 / 13.5).
 template <typename T, bool VEC>
@@ -909,9 +911,10 @@ __global__ __launch_bounds__(256) void embed_hashed_kernel(
     const T* __restrict__ pairs, const float* __restrict__ norm_w, const int* __restrict__ q_start,
     const int* __restrict__ kv_len, const int* __restrict__ state_slots, const int* __restrict__ phase,
     int* __restrict__ state, int n_seqs, int hidden, int vocab, long buckets, long mul_prev, long mul_cur, float scale,
-    float eps, float* __restrict__ x, T* __restrict__ out) {
+    float eps, float* __restrict__ x, T* __restrict__ out, int rows, RopeTables tables) {
   __shared__ float lds[16];
   const int row = blockIdx.x;
+  if (row >= rows) return tw_rope_block(tables, row - rows);
   const int s = tw_seq_of_row(q_start, n_seqs, row);
   const int first = q_start[s], q_len = q_start[s + 1] - first;
   const int start = kv_len[s] - q_len;
@@ -997,8 +1000,8 @@ extern "C" int tw_embed_hashed(int dtype, const int* ids, const int* feed, int n
                                const void* pairs, const float* norm_w, const int* q_start, const int* kv_len,
                                const int* state_slots, const int* phase, int* state, int n, int n_seqs, int hidden,
                                int vocab, long buckets, long mul_prev, long mul_cur, float scale, float eps, float* x,
-                               void* out, hipStream_t stream) {
-  TW_REQUIRE(ids && table && pairs && norm_w && q_start && kv_len && state_slots && phase && state && x);
+                               void* out, const RopeTables* tables, hipStream_t stream) {
+  TW_REQUIRE(ids && table && pairs && norm_w && q_start && kv_len && state_slots && phase && state && x && tables && tw_rope_tables_ok(*tables, n));
   TW_REQUIRE(n >= 0 && n_seqs > 0 && hidden > 0 && vocab > 0 && buckets > 0 && mul_prev >= 0 && mul_cur >= 0 && eps > 0.f);
   if (n == 0) return 0;
   TW_REQUIRE(dtype == TW_DTYPE_BF16 || dtype == TW_DTYPE_F32);
@@ -1007,9 +1010,9 @@ extern "C" int tw_embed_hashed(int dtype, const int* ids, const int* feed, int n
                    (((uintptr_t)table | (uintptr_t)pairs | (uintptr_t)norm_w | (uintptr_t)x | (uintptr_t)out) & 15) == 0;
   auto run = [&](auto tag, auto wide) {
     typedef decltype(tag) T;
-    embed_hashed_kernel<T, decltype(wide)::value><<<n, 256, 0, stream>>>(ids, feed, n_feed, (const T*)table, (const T*)pairs, norm_w, q_start,
+    embed_hashed_kernel<T, decltype(wide)::value><<<n + tw_rope_blocks(*tables), 256, 0, stream>>>(ids, feed, n_feed, (const T*)table, (const T*)pairs, norm_w, q_start,
                                                                          kv_len, state_slots, phase, state, n_seqs, hidden, vocab,
-                                                                         buckets, mul_prev, mul_cur, scale, eps, x, (T*)out);
+                                                                         buckets, mul_prev, mul_cur, scale, eps, x, (T*)out, n, *tables);
   };
   if (dtype == TW_DTYPE_BF16) {
     if (vec) run(bf16_t{}, std::true_type{});

@@ -10,6 +10,18 @@ _lib = None
 
 P, I, L, F = c_void_p, c_int, c_long, c_float
 
+ROPE_TABLES = 4
+
+
+class RopeTable(ctypes.Structure):
+    """As in rope_tables.h."""
+    _fields_ = [("inv_freq", P), ("rest", P), ("cos_out", P), ("sin_out", P), ("half", I), ("magnitude", F)]
+
+
+class RopeTables(ctypes.Structure):
+    _fields_ = [("table", RopeTable * ROPE_TABLES), ("positions", P), ("count", I), ("n", I)]
+
+
 _SIGNATURES = {
     "tw_error_string": (ctypes.c_char_p, [I]),
     "tw_abi_version": (I, []),
@@ -20,6 +32,7 @@ _SIGNATURES = {
     "tw_probe_read": (I, [P, L, P, I, ctypes.POINTER(c_long), P]),
     "tw_upload_words": (I, [P, P, I, ctypes.POINTER(c_int), ctypes.POINTER(c_int), P]),
     "tw_embed_gather": (I, [I, P, P, P, I, I, I, P, I, P]),
+    "tw_embed_begin": (I, [I, P, P, P, I, I, I, P, I, P, P, P, P, P, ctypes.POINTER(RopeTables), P]),
     "tw_rmsnorm": (I, [I, P, P, P, P, I, I, F, P, I, L, P, P]),
     "tw_rope_table": (I, [P, P, P, P, P, I, I, F, P]),
     "tw_rope_kv_write": (I, [I, P, L, P, P, P, P, P, I, I, I, I, I, I, I, P, I, P, I, P]),
@@ -63,7 +76,7 @@ _SIGNATURES = {
     "tw_kv_store": (I, [I, P, L, I, I, P, P, P, I, I, I, I, I, P]),
     "tw_residual_norm": (I, [I, P, P, L, P, I, L, P, P, P, I, I, F, F, P, P]),
     "tw_relu_squared": (I, [I, P, L, I, I, P, I, P]),
-    "tw_embed_hashed": (I, [I, P, P, I, P, P, P, P, P, P, P, P, I, I, I, I, L, L, L, F, F, P, P, P]),
+    "tw_embed_hashed": (I, [I, P, P, I, P, P, P, P, P, P, P, P, I, I, I, I, L, L, L, F, F, P, P, ctypes.POINTER(RopeTables), P]),
     "tw_latent_finish": (I, [I, P, L, I, I, I, P, P, P, P, L, P, L, I, I, I, I, P, P, P, I, I, I, I, I, I, I, F, P, I, P]),
     "tw_latent_decode_splits": (I, [I, I, I, I, I, I]),
     "tw_latent_decode_most_splits": (I, [I, I, I]),

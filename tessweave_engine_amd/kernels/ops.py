@@ -9,7 +9,7 @@ from __future__ import annotations
 
 import torch
 
-from .lib import library, check
+from .lib import ROPE_TABLES, RopeTables, library, check
 
 F32, BF16 = 0, 1
 _DTYPE_ID = {torch.float32: F32, torch.bfloat16: BF16}
@@ -100,6 +100,51 @@ def embed_gather(ids, table, out, feed=None):
                                     feed.numel() if feed is not None else 0, _stream()),
           "embed_gather")
     return out
+
+
+def _rope_tables(positions, tables):
+    """What `embed_begin` and `embed_hashed` hand their kernels of TABLES, up to `ROPE_TABLES` of (inv_freq, rest or None, cos, sin,
+    magnitude), each as `rope_table` takes them."""
+    arg, n = RopeTables(), positions.numel() if positions is not None else 0
+    _need(len(tables) <= ROPE_TABLES and (positions is not None or not tables), "too many rotary tables")
+    for t, (inv_freq, rest, cos, sin, magnitude) in zip(arg.table, tables):
+        half = inv_freq.numel()
+        _need(cos.is_contiguous() and sin.is_contiguous() and tuple(cos.shape) == (n, half) and tuple(sin.shape) == (n, half), "rotary tables must be [n, rot/2]")
+        _need(rest is None or (rest.is_contiguous() and rest.numel() == half), "the frequencies' remainders must be as many")
+        t.inv_freq, t.rest = _dev(inv_freq, torch.float32, "inv_freq"), _dev(rest, torch.float32, "rest") if rest is not None else None
+        t.cos_out, t.sin_out, t.half, t.magnitude = _dev(cos, torch.float32, "cos"), _dev(sin, torch.float32, "sin"), half, float(magnitude)
+    if tables:
+        arg.positions, arg.count, arg.n = _dev(positions, torch.int32, "positions"), len(tables), n
+    return arg
+
+
+def can_embed_begin(table):
+    return table.shape[1] % 16 == 0 and table.is_contiguous() and table.data_ptr() % 16 == 0
+
+
+def embed_begin(ids, table, out, feed=None, norm=None, second=None, sums=None, eps=0.0, rounded=None, positions=None, tables=()):
+    """`embed_gather`, and in the same launch what a decode step's first reader wants of the rows: norm = (weight, rows) (second: another one
+    of the same stream) with sums leaves the rows for a norm that travels, as `NormedRows`; rounded receives them in the table's type.
+    tables: rotary tables of POSITIONS, (inv_freq, rest or None, cos, sin, magnitude) each (see `rope_table`)."""
+    n = ids.numel()
+    vocab, hidden = table.shape
+    _need(can_embed_begin(table) and out.is_contiguous() and tuple(out.shape) == (n, hidden), "embed_begin takes rows of a multiple of 16 elements")
+    _need(norm is None or (rounded is None and can_leave_norms(n, hidden) and sums is not None and sums.is_contiguous()
+                           and tuple(sums.shape) == (n, hidden // 16)), "the norm of these rows cannot travel")
+    for w, r in [p for p in (norm, second) if p is not None] + ([(None, rounded)] if rounded is not None else []):
+        _need(r.is_contiguous() and tuple(r.shape) == (n, hidden) and r.dtype == table.dtype, "the rows left must be [n, hidden] of the table's type")
+        _need(w is None or (w.is_contiguous() and w.numel() == hidden), "a norm weight has the wrong size")
+    _need(second is None or norm is not None, "a second norm comes with a first")
+    f32, arg = torch.float32, _rope_tables(positions, tables)
+    rows = norm[1] if norm is not None else rounded
+    check(library().tw_embed_begin(dtype_id(table.dtype), _dev(ids, torch.int32, "ids"), _dev(table), _dev(out, f32, "out"), n, hidden, vocab,
+                                   _dev(feed, torch.int32, "feed") if feed is not None else None, feed.numel() if feed is not None else 0,
+                                   _dev(norm[0], f32, "weight") if norm is not None else None, _dev(rows) if rows is not None else None,
+                                   _dev(second[0], f32, "weight") if second is not None else None, _dev(second[1]) if second is not None else None,
+                                   _dev(sums, f32, "sums") if norm is not None else None, arg, _stream()), "embed_begin")
+    if norm is None:
+        return None
+    return NormedRows(norm[1], sums, eps, second=NormedRows(second[1], sums, eps) if second is not None else None)
 
 
 def rmsnorm(x, weight, eps, out, rows=None, add=None, row_scratch=None):
@@ -1037,10 +1082,11 @@ def relu_squared(x, partial=None):
 
 
 def embed_hashed(ids, table, pairs, norm_weight, q_start, kv_len, state_slots, phase, state, n_seqs, buckets, mul_prev,
-                 mul_cur, scale, eps, x, out=None, feed=None):
+                 mul_cur, scale, eps, x, out=None, feed=None, positions=None, tables=()):
     """x[n] = norm_weight * unit(scale * table[ids[n]] + pairs[r]), r = (previous token * mul_prev + token * mul_cur) mod
     buckets, r = buckets for a sequence's first token. state int32 [requests, 2] holds the last token of every request
-    twice (copy phase[s] is read, the other written). x float32 [n, hidden]; out: the same rounded to its type."""
+    twice (copy phase[s] is read, the other written). x float32 [n, hidden]; out: the same rounded to its type.
+    positions, tables: rotary tables formed in the same launch, as for `embed_begin`."""
     n = ids.numel()
     vocab, hidden = table.shape
     _need(table.is_contiguous() and pairs.is_contiguous() and pairs.dtype == table.dtype and tuple(pairs.shape) == (buckets + 1, hidden),
@@ -1058,8 +1104,8 @@ def embed_hashed(ids, table, pairs, norm_weight, q_start, kv_len, state_slots, p
                                     _dev(q_start, torch.int32, "q_start"), _dev(kv_len, torch.int32, "kv_len"),
                                     _dev(state_slots, torch.int32, "state_slots"), _dev(phase, torch.int32, "phase"),
                                     _dev(state), n, int(n_seqs), hidden, vocab, int(buckets), int(mul_prev), int(mul_cur),
-                                    float(scale), float(eps), _dev(x), _dev(out) if out is not None else None, _stream()),
-          "embed_hashed")
+                                    float(scale), float(eps), _dev(x), _dev(out) if out is not None else None,
+                                    _rope_tables(positions, tables), _stream()), "embed_hashed")
     return x
 
 

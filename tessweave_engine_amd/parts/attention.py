@@ -59,6 +59,7 @@ def paged_attention(ctx, q, keys, values, group, out, q_heads, kv_heads, head_di
 
 class GroupedQueryAttention(Mixer):
     leaves_normed = True
+    uses_tables = True
 
     def __init__(self, prefix, hidden, q_heads, kv_heads, head_dim, position, qkv_bias=True,
                  o_bias=False, window=None, scale=None, packed=True, head_hook=None, softcap=None, value_dim=None,

@@ -29,6 +29,9 @@ NORMED_STREAM = "stream.normed"
 #: runs that add it to the stream again (`LayerRun.adds_embedding`)
 EMBEDDING_OUTPUT = "embedding.output"
 
+#: key of `StepContext.shared` under which an embedding leaves its rows for the first block's norms (`ops.NormedRows`)
+LEFT_ROWS = "left.rows"
+
 #: key of `StepContext.shared`: which of the two buffers took the last sums of squares that travel (see `NormAhead`)
 SUMS_TURN = "left.sums.turn"
 
@@ -127,6 +130,9 @@ class HeadHook(Part):
 
 
 class Mixer(Part):
+    #: does `forward` ask its `position` part for its tables in every step?
+    uses_tables = False
+
     def cache_need(self):
         """A cache.CacheNeed (paged keys/values and/or fixed-size state), or None."""
         return None
@@ -196,6 +202,20 @@ class NormAhead:
 
     def __init__(self, norms, stream, after=None):
         self.norms, self.stream, self.after = tuple(norms), stream, after
+
+    def buffers(self, ctx, dtype):
+        """([rows for each norm], sums) to leave them in. (Two buffers of sums in turn: the product that leaves some may read those left before.)"""
+        n, width = self.stream.shape
+        rows = [ctx.workspace.get(f"left.rows{i}", (16, width), dtype)[:n] for i in range(len(self.norms))]
+        ctx.shared[SUMS_TURN] = turn = ctx.shared.get(SUMS_TURN, 0) ^ 1
+        return rows, ctx.workspace.get(f"left.sums{turn}", (width,), torch.float32)[:n * width // 16].view(n, width // 16)
+
+    def named(self, left):
+        """LEFT (`ops.NormedRows`), its rows marked with the norms they are for."""
+        left.norm = self.norms[0]
+        if left.second is not None:
+            left.second.norm = self.norms[1]
+        return left
 
 
 def norm_ahead(ctx, stream, norms, readers, after=None):
@@ -293,6 +313,7 @@ class StepContext:
         self.defer_sums = True       # may a mixer or feed-forward leave partial sums pending for the next norm?
         self.capturing = False       # launches may depend on kv_bound and capacities, not on this step's lengths
         self.norm_ahead = None       # NormAhead for the sublayer that runs now: the norms that read the stream behind it
+        self.tables_wanted = ()      # rotary encodings whose tables a layer will ask for: an embedding may form them with its rows
         self.entry_behind = None     # (norms, readers) of what runs behind the block that runs now, or None (see Block.entry)
         self.segment_end = None      # while a step is captured: called with the index of each finished layer run
         self.max_tokens = 0          # row capacity of per-token scratch buffers

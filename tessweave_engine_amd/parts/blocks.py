@@ -259,6 +259,9 @@ class ResultNormBlock(Block):
             h = ops.round_rows(x, ctx.scratch("stream.rounded", (ctx.n_tokens, self.hidden)))
         return h
 
+    def entry(self):
+        return (), ()                     # (reads the stream as it is; nothing is left for it in place of sums)
+
     def _sublayer(self, ctx, x, norm, result, pending):
         rounded = ctx.scratch("stream.rounded", (ctx.n_tokens, self.hidden)) if ctx.dtype != torch.float32 else None
         ops.add_normed(x, norm.weight, norm.eps, mult=self.mult, y=result if pending is None else None, add=pending,

@@ -12,7 +12,7 @@ import torch
 from ..cache.spec import CacheNeed, FixedState
 from ..kernels import ops
 from ..weights.spec import MATRIX, NORMAL, TensorSpec
-from .base import EMBEDDING_OUTPUT, ROUNDED_STREAM, Part
+from .base import EMBEDDING_OUTPUT, LEFT_ROWS, ROUNDED_STREAM, Part, norm_ahead
 
 
 class TokenEmbedding(Part):
@@ -27,9 +27,31 @@ class TokenEmbedding(Part):
     def bind(self, tensors, dtype, device):
         self.weight = tensors.pop(self.name + self.suffix).contiguous()
 
+    def _stream(self, ctx):
+        return ctx.scratch("residual", (ctx.n_tokens, self.hidden), torch.float32)
+
+    def gather(self, ctx):
+        return ops.embed_gather(ctx.token_ids, self.weight, self._stream(ctx), feed=ctx.token_feed)
+
     def forward(self, ctx):
-        x = ctx.scratch("residual", (ctx.n_tokens, self.hidden), torch.float32)
-        return ops.embed_gather(ctx.token_ids, self.weight, x, feed=ctx.token_feed)
+        if not ctx.capturing or not ops.can_embed_begin(self.weight):
+            return self.gather(ctx)
+        # a step of one-token rows: the rotary tables, and the rows as their first reader wants them, are formed in the same launch
+        x, norms, readers = self._stream(ctx), *(ctx.entry_behind or (None, ()))
+        options, ahead = {}, norm_ahead(ctx, x, norms, readers) if norms else None
+        if ahead is not None:
+            rows, sums = ahead.buffers(ctx, self.weight.dtype)
+            pairs = [(norm.weight, r) for norm, r in zip(norms, rows)]
+            options = dict(norm=pairs[0], second=pairs[1] if len(pairs) > 1 else None, sums=sums, eps=norms[0].eps)
+        elif norms == ():
+            options = dict(rounded=ctx.scratch("stream.rounded", (ctx.n_tokens, self.hidden))) if ctx.dtype != torch.float32 else {}
+        left = ops.embed_begin(ctx.token_ids, self.weight, x, feed=ctx.token_feed, positions=ctx.positions[0],
+                               tables=[part.table_job(ctx) for part in ctx.tables_wanted[:ops.ROPE_TABLES]], **options)
+        if left is not None:
+            ctx.shared[LEFT_ROWS] = ahead.named(left)
+        elif norms == ():
+            ctx.shared[ROUNDED_STREAM] = options.get("rounded", x)
+        return x
 
 
 class PositionedEmbedding(TokenEmbedding):
@@ -53,7 +75,7 @@ class PositionedEmbedding(TokenEmbedding):
         self.positions = tensors.pop(self.position_name + self.suffix).contiguous()
 
     def forward(self, ctx):
-        x = super().forward(ctx)
+        x = self.gather(ctx)
         copy = None
         if self.keep is not None:
             tag, leading = self.keep
@@ -140,7 +162,8 @@ class HashedPairEmbedding(TokenEmbedding):
         state = ctx.cache.states[self.cache_slot][self.STATE]
         ops.embed_hashed(ctx.token_ids, self.weight, self.pairs, self.norm.weight, ctx.q_start, ctx.kv_len, ctx.state_slots,
                          ctx.state_phase, state, ctx.n_seqs, self.buckets, self.mul_prev, self.mul_cur, self.scale,
-                         self.norm.eps, x, out=rounded, feed=ctx.token_feed)
+                         self.norm.eps, x, out=rounded, feed=ctx.token_feed, positions=ctx.positions[0],
+                         tables=[part.table_job(ctx) for part in ctx.tables_wanted[:ops.ROPE_TABLES]])
         ctx.shared[ROUNDED_STREAM] = rounded if rounded is not None else x
         return x
 

@@ -39,6 +39,7 @@ def _round_up(v, m):
 
 class LatentAttention(Mixer):
     leaves_normed = True
+    uses_tables = True
 
     def __init__(self, prefix, hidden, heads, dim, rot_dim, value_dim, latent, scale, position, eps, own_latent=True,
                  names=("q", "dkv", "dkv.norm", "uk", "uv", "o"), sink_name=None, gate_name=None):

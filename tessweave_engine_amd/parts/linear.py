@@ -11,7 +11,7 @@ import torch
 
 from ..kernels import ops
 from ..weights.spec import MATRIX, VECTOR, NORMAL, TensorSpec
-from .base import SUMS_TURN, Part
+from .base import Part
 
 
 def pad_groups(t, dim, unit, to):
@@ -262,18 +262,11 @@ class Linear(Part):
         ahead = getattr(ctx, "norm_ahead", None)
         if ahead is None or not self.takes_normed or self.gated or not ops.linear_leave_pays(x, self.weights[0]):
             return None
-        n, width = x.shape[0], self.weights[0].shape[0]
-        rows = [ctx.workspace.get(f"left.rows{i}", (16, width), x.dtype)[:n] for i in range(len(ahead.norms))]
-        # (two buffers in turn: the product that leaves sums may read those left before)
-        ctx.shared[SUMS_TURN] = turn = ctx.shared.get(SUMS_TURN, 0) ^ 1
-        sums = ctx.workspace.get(f"left.sums{turn}", (16 * width // 16,), torch.float32)[:n * width // 16].view(n, width // 16)
+        rows, sums = ahead.buffers(ctx, x.dtype)
         first, second = ahead.norms[0], ahead.norms[1] if len(ahead.norms) > 1 else None
         left = ops.linear_leave(x, self.weights[0], ahead.stream, first.weight, first.eps, rows[0], sums, bias=self.biases[0] if self.biases else None,
                                 second=(second.weight, rows[1]) if second is not None else None, after=ahead.after)
-        left.norm = first
-        if second is not None:
-            left.second.norm = second
-        return left
+        return ahead.named(left)
 
 
 class JoinedLinear(Linear):

@@ -5,8 +5,9 @@ import torch
 
 from ..cache.spec import CacheLayout
 from ..kernels import ops
-from .base import EMBEDDING_OUTPUT, LayerRun, Norm, Part, PositionEncoding
+from .base import EMBEDDING_OUTPUT, LEFT_ROWS, LayerRun, Mixer, Norm, Part, PositionEncoding
 from .blocks import normalise
+from .positions import RotaryEmbedding
 
 
 def walk(part):
@@ -32,7 +33,7 @@ class DecoderModel(Part):
                 raise ValueError(f"schedule names block {run.block}, the model has {len(self.blocks)}")
         self.dtype = None
         self.device = None
-        self._layout = None
+        self._layout = self._tables = None
 
     # ---- structure ----------------------------------------------------------
     def parts(self):
@@ -113,19 +114,29 @@ class DecoderModel(Part):
             self._layout = CacheLayout(needs)
         return self._layout
 
+    def _tables_wanted(self):
+        """The rotary encodings whose tables some layer asks for in every step, each once."""
+        if self._tables is None:
+            self._tables = tuple({id(m.position): m.position for run in self.schedule for m in walk(self.blocks[run.block])
+                                  if isinstance(m, Mixer) and m.uses_tables and isinstance(m.position, RotaryEmbedding)}.values())
+        return self._tables
+
     def _entry_behind(self, i):
         """What norms read the stream behind run I (see `Block.entry`): the next block's, or the model's last one (a captured step
         wants every row's logits, in order)."""
         if i + 1 == len(self.schedule):
-            return (self.final_norm,), (self.head,)
+            return ((self.final_norm,), (self.head,)) if self.schedule else None
         following = self.schedule[i + 1]
         return None if following.adds_embedding else self.blocks[following.block].entry()
 
     # ---- one step -----------------------------------------------------------------
     def forward(self, ctx):
         """Run the step's tokens; float32 logits [n_logits, vocab] at ctx.logit_rows."""
+        if ctx.capturing:
+            ctx.entry_behind, ctx.tables_wanted = self._entry_behind(-1), self._tables_wanted()
         x = self.embedding.forward(ctx)
-        pending = None              # partial sums a block left for the next norm to add into x
+        ctx.tables_wanted = ()
+        pending = ctx.shared.pop(LEFT_ROWS, None)     # partial sums a block left for the next norm to add into x, or rows for it
         for i, run in enumerate(self.schedule):
             if run.adds_embedding:
                 first = ctx.shared[EMBEDDING_OUTPUT]

@@ -78,14 +78,21 @@ class RotaryEmbedding(PositionEncoding):
             raise ValueError("a stretched encoding scales its cosines and sines: use its tables")
         return ctx.positions[0], self.inv_freq, self.rest
 
+    def _table_buffers(self, ctx):
+        shape = (ctx.n_tokens, self.rotary_dim // 2)
+        return tuple(ctx.scratch(f"rotary.{name}.{id(self)}", shape, torch.float32) for name in ("cos", "sin"))
+
+    def table_job(self, ctx):
+        """The step's tables as something its caller will form (see `ops.embed_begin`): they count as formed from here on."""
+        cos, sin = ctx.shared["rotary", id(self)] = self._table_buffers(ctx)
+        return self.inv_freq, self.rest, cos, sin, self.magnitude
+
     def tables(self, ctx):
         """(cos, sin), float32 [n_tokens, rotary_dim / 2], computed once per step."""
         key = ("rotary", id(self))
         hit = ctx.shared.get(key)
         if hit is None:
-            half = self.rotary_dim // 2
-            cos = ctx.scratch(f"rotary.cos.{id(self)}", (ctx.n_tokens, half), torch.float32)
-            sin = ctx.scratch(f"rotary.sin.{id(self)}", (ctx.n_tokens, half), torch.float32)
+            cos, sin = self._table_buffers(ctx)
             ops.rope_table(ctx.positions[0], self.inv_freq, cos, sin, self.magnitude, rest=self.rest)
             hit = ctx.shared[key] = (cos, sin)
         return hit

@@ -24,6 +24,7 @@ def _round_up(v, m):
 
 class Retention(Mixer):
     leaves_normed = True
+    uses_tables = True
     STATE = "retention.s"
 
     def __init__(self, prefix, hidden, heads, dim, value_dim, decay, position, eps, names=("q", "k", "v", "g", "o"),

@@ -68,6 +68,7 @@ def mixed_attention(ctx, q, keys, values, group, out, q_heads, kv_heads, value_d
 
 
 class ConvolvedWindowAttention(Mixer):
+    uses_tables = True
     CONV_STATE = "attention.conv"
     MAX_HEADS = 32                  # what the attention kernel's workgroup holds
 

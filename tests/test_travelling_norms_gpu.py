@@ -150,3 +150,39 @@ def test_residual_norm_of_rows_behind_a_norm(ops, device, dtype, hidden):
     ops.residual_norm(x, w, 1e-6, out=out, add=y, scale=scale, alpha=0.7, before=before)
     torch.testing.assert_close(x.double(), want, atol=3e-6, rtol=3e-6)             # (as this kernel's other forms)
     torch.testing.assert_close(out, x.to(dtype), atol=0, rtol=0)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("n,hidden,form", [(1, 64, "norm"), (16, 896, "two norms"), (3, 4096, "norm"), (40, 2064, "rounded"), (5, 16, "rows alone"), (16, 3072, "no tables")])
+def test_embed_begin(ops, device, dtype, n, hidden, form):
+    """Against the gather, a table at a time and the sums in float64: the same bits where a value is only moved or rounded once."""
+    table = rand((50, hidden), dtype, device, 1.5)
+    ids = torch.tensor([(7 * i) % 50 for i in range(n - 1)] + [-2], dtype=torch.int32, device=device)
+    feed = torch.tensor([3, 17], dtype=torch.int32, device=device)
+    positions = torch.tensor([(311 * i) % 5000 for i in range(n)], dtype=torch.int32, device=device)
+    weights = [1 + rand((hidden,), torch.float32, device, 0.1, s) for s in (1, 2)]
+    rows = [torch.full((n, hidden), float("nan"), dtype=dtype, device=device) for _ in range(2)]
+    sums = torch.full((n, hidden // 16), float("nan"), device=device)
+    tables, want = [], []
+    for half, magnitude, rest in ((32, 1.0, False), (64, 1.25, True), (1, 1.0, True), (5, 0.5, False))[:0 if form == "no tables" else 4]:
+        freq = 10000.0 ** (-torch.arange(half, dtype=torch.float32) / half)
+        rest = (freq * 1e-8).to(device) if rest else None
+        pair = [torch.full((n, half), float("nan"), device=device) for _ in range(4)]
+        tables.append((freq.to(device), rest, pair[0], pair[1], magnitude))
+        ops.rope_table(positions, freq.to(device), pair[2], pair[3], magnitude, rest=rest)
+        want.append(pair)
+    options = {"norm": dict(norm=(weights[0], rows[0]), sums=sums), "two norms": dict(norm=(weights[0], rows[0]), second=(weights[1], rows[1]), sums=sums),
+               "rounded": dict(rounded=rows[0])}.get(form, {})
+    x = torch.full((n, hidden), float("nan"), device=device)
+    left = ops.embed_begin(ids, table, x, feed=feed, positions=positions, tables=tables, **options)
+    gathered = ops.embed_gather(ids, table, torch.empty_like(x), feed=feed)
+    assert torch.equal(x, gathered)
+    for cos, sin, want_cos, want_sin in want:
+        assert torch.equal(cos, want_cos) and torch.equal(sin, want_sin)
+    if form in ("norm", "two norms"):
+        assert torch.equal(left.rows, (x * weights[0]).to(dtype)) and (left.second is None) == (form == "norm")
+        torch.testing.assert_close(sums.double(), (x.double() ** 2).view(n, hidden // 16, 16).sum(-1), rtol=2.0 ** -21, atol=0)
+        if form == "two norms":
+            assert torch.equal(left.second.rows, (x * weights[1]).to(dtype))
+    elif form == "rounded":
+        assert left is None and torch.equal(rows[0], x.to(dtype))
