@@ -18,6 +18,7 @@
 // [H][E][Dk] (a column of S is contiguous), Dk <= KS * DPL. Tokens are staged in LDS in chunks: the waves share a
 // chunk's tokens out, norm q and k, form beta and g, then all walk the chunk.
 #include "tw_common.h"
+#include "norm_gate.h"
 
 #define TW_DELTA_CHUNK 16             /* tokens the walk stages at a time */
 #define TW_DELTA_WALK_MOST 4          /* up to this many tokens a sequence, a step walks them one by one */
@@ -907,7 +908,8 @@ extern "C" int tw_delta_rule(const float* qkv, long ld_qkv, int q_col, int k_col
 }
 
 // out[n][h * E + e] = o[n][h * E + e] / sqrt(mean_e(o^2) + eps) * weight[e] * silu(gate[n][h * E + e]), rounded to the
-// compute type: a unit norm per head with one weight vector shared by the heads, times a gate. One wave a (token, head).
+// compute type: a unit norm per head with one weight vector shared by the heads, times a gate. One wave a (token, head), element by
+// element: heads of whole groups of four are norm_gate_kernel's.
 template <typename T>
 __global__ __launch_bounds__(256) void head_norm_gate_kernel(const float* __restrict__ o, long ld_o, const float* __restrict__ gate,
                                                              long ld_g, const float* __restrict__ weight, T* __restrict__ out,
@@ -939,6 +941,12 @@ extern "C" int tw_head_norm_gate(int dtype, const float* o, long ld_o, const flo
   const int weight_stride = weight_per_head ? E : 0;
   TW_REQUIRE(ld_o >= (long)H * E && ld_g >= (long)H * E && ld_out >= (long)H * E);
   if (n == 0) return 0;
+  const NormGateArgs a{o, ld_o, gate, ld_g, weight, out, ld_out, n, H, E, E, weight_stride, eps, 1.f};
+  auto fast = [&](auto t) {
+    typedef decltype(t) T;
+    return gate_kind == 1 ? norm_gate_launch<T, float, TW_GATE_SIGMOID_BEHIND>(a, stream) : norm_gate_launch<T, float, TW_GATE_SILU_BEHIND>(a, stream);
+  };
+  if (dtype == TW_DTYPE_BF16 ? fast(bf16_t{}) : dtype == TW_DTYPE_F32 && fast(float{})) return TW_LAUNCH_RESULT();
   const int blocks = tw_div_up((long)n * H, 4);
   if (dtype == TW_DTYPE_BF16)
     head_norm_gate_kernel<bf16_t><<<blocks, 256, 0, stream>>>(o, ld_o, gate, ld_g, weight, (bf16_t*)out, ld_out, n, H, E, eps, weight_stride, gate_kind);

@@ -27,6 +27,7 @@
 // would build from zero, a scan turns those into the states the segments start from (and writes the request's new
 // state), and the main launch walks all segments at once.
 #include "tw_common.h"
+#include "norm_gate.h"
 
 #define LS_L 16
 #define LS_RANGE (-60.f)
@@ -694,7 +695,7 @@ extern "C" int tw_decay_logs(const float* low, long ld, const float* up, const f
 
 // ---- a gate, then a norm in equal parts -----------------------------------------------------------------------------
 // out[n] = [.. u_p / sqrt(mean(u_p^2) + eps) ..] * weight over `parts` equal parts u_p of u = y * silu(gate), rounded to the
-// compute type. THREADS 256: a block a (token, part); 64: a wave. AFTER: u = y, and the normed row is multiplied by
+// compute type, element by element (parts of whole groups of four, up to 2,048, are norm_gate_kernel's). THREADS 256: a block a (token, part); 64: a wave. AFTER: u = y, and the normed row is multiplied by
 // sigmoid(gate) and by `scale` before it is rounded.
 template <typename T, int THREADS, bool AFTER>
 __global__ __launch_bounds__(256) void gate_group_norm_kernel(const float* __restrict__ y, long ld_y, const float* __restrict__ gate,
@@ -743,6 +744,8 @@ __global__ __launch_bounds__(256) void gate_group_norm_kernel(const float* __res
 template <typename T, bool AFTER>
 static void gate_group_norm_launch(const float* y, long ld_y, const float* gate, long ld_g, const float* weight, void* out,
                                    long ld_out, int n, int parts, int size, float eps, float scale, hipStream_t stream) {
+  const NormGateArgs a{y, ld_y, gate, ld_g, weight, out, ld_out, n, parts, size, size, size, eps, scale};
+  if (norm_gate_launch<T, float, AFTER ? TW_GATE_SIGMOID_BEHIND : TW_GATE_SILU_BEFORE>(a, stream)) return;
   const long units = (long)n * parts;
   if (size > 512)
     gate_group_norm_kernel<T, 256, AFTER><<<(unsigned)units, 256, 0, stream>>>(y, ld_y, gate, ld_g, weight, (T*)out, ld_out, n, parts, size, eps, scale);

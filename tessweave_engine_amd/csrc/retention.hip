@@ -11,6 +11,7 @@
 // Heads are laid out with Dp = 16 * NT key elements and Ep value elements on the device (tails of zeros, which
 // add nothing to a product and leave zero columns in S).
 #include "tw_common.h"
+#include "norm_gate.h"
 
 struct RetentionArgs {
   const void* proj; long ld;          // a token's projections: q of head h at q_col + h * Dp, k at k_col + h * Dp,
@@ -468,7 +469,8 @@ extern "C" int tw_retention(int dtype, const void* proj, long ld, int q_col, int
 
 // ---- each head's result over its root mean square, times silu of a gate ------------------------------------------
 // out[n][h * Ep + e] = o[n][h * Ep + e] / sqrt(mean_e(o^2) + eps) * silu(gate[n][h * Ep + e]); the mean runs over
-// the head's E real elements (the device layout's tail is zeros and stays zeros). One wave a (token, head).
+// the head's E real elements (the device layout's tail is zeros and stays zeros). One wave a (token, head), element by element:
+// heads of whole groups of four are norm_gate_kernel's.
 template <typename T>
 __global__ __launch_bounds__(256) void unit_gate_kernel(const float* __restrict__ o, long ld_o, const T* __restrict__ gate,
                                                         long ld_g, T* __restrict__ out, long ld_out, int n, int H, int E,
@@ -499,6 +501,9 @@ extern "C" int tw_unit_gate(int dtype, const float* o, long ld_o, const void* ga
   TW_REQUIRE(o && gate && out && n >= 0 && H > 0 && E > 0 && Ep >= E && eps > 0.f);
   TW_REQUIRE(ld_o >= (long)H * Ep && ld_g >= (long)H * Ep && ld_out >= (long)H * Ep);
   if (n == 0) return 0;
+  const NormGateArgs a{o, ld_o, gate, ld_g, nullptr, out, ld_out, n, H, E, Ep, 0, eps, 1.f};
+  if (dtype == TW_DTYPE_BF16 && norm_gate_launch<bf16_t, bf16_t, TW_GATE_SILU_BEHIND>(a, stream)) return TW_LAUNCH_RESULT();
+  if (dtype == TW_DTYPE_F32 && norm_gate_launch<float, float, TW_GATE_SILU_BEHIND>(a, stream)) return TW_LAUNCH_RESULT();
   const int blocks = tw_div_up((long)n * H, 4);
   if (dtype == TW_DTYPE_BF16)
     unit_gate_kernel<bf16_t><<<blocks, 256, 0, stream>>>(o, ld_o, (const bf16_t*)gate, ld_g, (bf16_t*)out, ld_out, n, H, E, Ep, eps);

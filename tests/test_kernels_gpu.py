@@ -1378,3 +1378,37 @@ def test_sampling_greedy_ties_and_distribution(ops, device):
                     seeds=torch.tensor([12345], dtype=torch.int64, device=device),
                     counters=torch.tensor([9], dtype=torch.int32, device=device))
     assert one.item() == want
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("n,parts,size,pitch,offset", [(1, 1, 4, 4, 0), (3, 5, 128, 128, 0), (1, 3, 132, 132, 0), (3, 5, 252, 256, 0), (2, 3, 256, 256, 4), (7, 2, 260, 272, 0), (5, 1, 512, 512, 0),
+                                                       (2, 2, 516, 516, 8), (3, 1, 1024, 1024, 0), (2, 2, 1028, 1028, 0), (1, 1, 2048, 2048, 0),
+                                                       (2, 1, 2052, 2052, 0), (3, 4, 126, 128, 0), (3, 4, 128, 128, 1)])      # (the last three element by element)
+def test_units_normed_and_gated(ops, device, dtype, n, parts, size, pitch, offset):
+    """The norms with gates of retention, the delta rule, the mLSTM and the linear states: each of their forms against float64."""
+    width = parts * pitch
+    y, z = rand((n, width + offset), torch.float32, device, 2.0), rand((n, width + offset), torch.float32, device, 2.0, 1)
+    y, z = y[:, offset:], z[:, offset:]
+    cut = lambda t: t.double().reshape(n, parts, pitch)[..., :size]                     # noqa: E731
+    unit = lambda u: u / torch.sqrt((u ** 2).mean(-1, keepdim=True) + 1e-5)             # noqa: E731
+    silu = lambda u: u * torch.sigmoid(u)                                               # noqa: E731
+    close = tol(dtype, (4e-6, 4e-6), (1e-30, 2.0 ** -8))
+    bf = z.to(dtype) if offset == 0 else z.to(dtype).clone()
+    out = torch.full((n, width), float("nan"), dtype=dtype, device=device)
+    ops.unit_gate(y, bf, out, parts, size, pitch, 1e-5)
+    want = torch.zeros(n, parts, pitch, dtype=torch.float64, device=device)
+    want[..., :size] = unit(cut(y)) * silu(cut(bf))
+    torch.testing.assert_close(out.double(), want.view(n, width).to(dtype).double() if dtype == torch.bfloat16 else want.view(n, width), **close)
+    if pitch != size:
+        return
+    w = 1 + rand((width,), torch.float32, device, 0.1, 2)
+    for weight, act in ((w[:size].contiguous(), "silu"), (w, "sigmoid")):
+        ops.head_norm_gate(y, z, weight, out, parts, size, 1e-5, gate_activation=act)
+        want = unit(cut(y)) * weight.double().view(-1, size) * (silu(cut(z)) if act == "silu" else torch.sigmoid(cut(z)))
+        torch.testing.assert_close(out.double().view_as(want), want, **close)
+    ops.gate_group_norm(y, z, w, out, parts, 1e-5)
+    want = unit(cut(y) * silu(cut(z))) * w.double().view(parts, size)
+    torch.testing.assert_close(out.double().view_as(want), want, **close)
+    ops.gate_group_norm(y, z, w, out, parts, 1e-5, after=True, scale=0.6)
+    want = unit(cut(y)) * w.double().view(parts, size) * torch.sigmoid(cut(z)) * 0.6
+    torch.testing.assert_close(out.double().view_as(want), want, **close)
