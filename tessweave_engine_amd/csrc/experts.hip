@@ -51,8 +51,10 @@ __device__ __forceinline__ f32x4 moe_four(const bf16_t* p) {
 
 // A workgroup takes R rows: a wave forms two experts' logits for all of them at a time, four elements a lane and load,
 // several loads in flight before the first is used (a logit is a chain of loads from memory, and their latency is all it
-// costs: few rows get many waves each, many rows share a read of the router). Then a wave a row chooses.
-template <typename T, int R, int WAVES>
+// costs: few rows get many waves each, many rows share a read of the router; B pieces of 256 elements go out together, all of 2,048
+// where a wave has no more than its two experts). Then a wave a row chooses. (us, four pieces at a time and the choice through LDS / now: 4 rows,
+// 20 experts of 2,048, softmax 6.4 / 4.7; 1 row, 16 experts 4.9 / 4.0; 8 rows, 64 experts, eight chosen 14.2 / 9.5; 1,000 rows 9.9 / 6.9.)
+template <typename T, int R, int WAVES, int B>
 __global__ __launch_bounds__(64 * WAVES) void moe_route_kernel(const T* __restrict__ h, long ld_h, const float* __restrict__ router,
                                                                const float* __restrict__ bias, int mode, int n, int C, int X,
                                                                int top, int* __restrict__ ids, float* __restrict__ weights,
@@ -71,19 +73,27 @@ __global__ __launch_bounds__(64 * WAVES) void moe_route_kernel(const T* __restri
 #pragma unroll
     for (int r = 0; r < R; ++r) s0[r] = s1[r] = 0.f;
     if (vec) {
-#pragma unroll 4
-      for (int c = 4 * lane; c < C; c += 256) {
-        const f32x4 a = *reinterpret_cast<const f32x4*>(w0 + c);
-        const f32x4 b = *reinterpret_cast<const f32x4*>(w1 + c);
+      for (int c0 = 4 * lane; c0 < C; c0 += 256 * B) {
+        f32x4 a[B], b[B], xv[R][B];
 #pragma unroll
-        for (int r = 0; r < R; ++r) {
-          const f32x4 xv = moe_four(x[r] + c);
+        for (int j = 0; j < B; ++j) {
+          const int c = min(c0 + 256 * j, C - 4);
+          a[j] = *reinterpret_cast<const f32x4*>(w0 + c);
+          b[j] = *reinterpret_cast<const f32x4*>(w1 + c);
 #pragma unroll
-          for (int j = 0; j < 4; ++j) {
-            s0[r] = __fmaf_rn(a[j], xv[j], s0[r]);
-            s1[r] = __fmaf_rn(b[j], xv[j], s1[r]);
-          }
+          for (int r = 0; r < R; ++r) xv[r][j] = moe_four(x[r] + c);
         }
+#pragma unroll
+        for (int j = 0; j < B; ++j)
+          if (c0 + 256 * j < C) {
+#pragma unroll
+            for (int r = 0; r < R; ++r)
+#pragma unroll
+              for (int i = 0; i < 4; ++i) {
+                s0[r] = __fmaf_rn(a[j][i], xv[r][j][i], s0[r]);
+                s1[r] = __fmaf_rn(b[j][i], xv[r][j][i], s1[r]);
+              }
+          }
       }
     } else {
       for (int c = lane; c < C; c += 64) {
@@ -110,6 +120,45 @@ __global__ __launch_bounds__(64 * WAVES) void moe_route_kernel(const T* __restri
   const int row = row0 + wave;
   float* z = z_s[wave];
   float* score = score_s[wave];
+  if (X <= 64 && keep == groups) {
+    // An expert a lane, everything in registers: the largest of the wave, the lowest lane that holds it, and lane r keeps choice r.
+    float v = lane < X ? z[lane] : -INFINITY, share = 0.f;
+    if (mode == 2) {
+      const float most = tw_wave_max(v);
+      share = lane < X ? expf(v - most) : 0.f;
+      share /= tw_wave_sum(share);
+      v = lane < X ? share + (bias ? bias[lane] : 0.f) : -INFINITY;
+    }
+    int mine = 0;
+    float weight = 0.f;
+    for (int r = 0; r < top; ++r) {
+      const float best = tw_wave_max(v);
+      const unsigned long long holders = __ballot(v == best);
+      const int at = min(holders ? __ffsll((long long)holders) - 1 : X - 1, X - 1);      // (no logit compares as the largest if all are NaN)
+      const float chosen = mode == 2 ? share : best;
+      const float w = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(chosen), at));
+      if (lane == r) {
+        mine = at;
+        weight = w;
+      }
+      if (lane == at) v = -INFINITY;
+    }
+    auto of_choice = [&](float f, int r) { return __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(f), r)); };
+    if (mode == 0) {
+      weight = scale / (1.f + expf(-weight));
+    } else {
+      // the softmax over the chosen logits (the first is the largest), or the chosen shares', added up in the order of the choices
+      if (mode == 1) weight = expf(weight - of_choice(weight, 0));
+      float sum = mode == 1 ? 0.f : 1e-20f;
+      for (int r = 0; r < top; ++r) sum += of_choice(weight, r);
+      weight /= sum;
+    }
+    if (lane < top) {
+      ids[(size_t)row * top + lane] = mine;
+      weights[(size_t)row * top + lane] = weight;
+    }
+    return;
+  }
   if (mode == 2) {
     float most = -INFINITY, sum = 0.f;
     for (int e = lane; e < X; e += 64) most = fmaxf(most, z[e]);
@@ -217,9 +266,10 @@ extern "C" int tw_moe_route(int dtype, const void* h, long ld_h, const float* ro
   if (n == 0) return 0;
 #define TW_MOE_ROUTE(T)                                                                                                 \
   do {                                                                                                                  \
-    if (n <= 64) moe_route_kernel<T, 1, 16><<<n, 1024, 0, stream>>>((const T*)h, ld_h, router, bias, mode, n, C, X, top, ids, weights, groups, keep, scale); \
-    else if (n <= 512) moe_route_kernel<T, 1, 4><<<n, 256, 0, stream>>>((const T*)h, ld_h, router, bias, mode, n, C, X, top, ids, weights, groups, keep, scale); \
-    else moe_route_kernel<T, 4, 8><<<tw_div_up(n, 4), 512, 0, stream>>>((const T*)h, ld_h, router, bias, mode, n, C, X, top, ids, weights, groups, keep, scale); \
+    if (n <= 64 && X <= 32) moe_route_kernel<T, 1, 16, 8><<<n, 1024, 0, stream>>>((const T*)h, ld_h, router, bias, mode, n, C, X, top, ids, weights, groups, keep, scale); \
+    else if (n <= 64) moe_route_kernel<T, 1, 16, 4><<<n, 1024, 0, stream>>>((const T*)h, ld_h, router, bias, mode, n, C, X, top, ids, weights, groups, keep, scale); \
+    else if (n <= 512) moe_route_kernel<T, 1, 4, 8><<<n, 256, 0, stream>>>((const T*)h, ld_h, router, bias, mode, n, C, X, top, ids, weights, groups, keep, scale); \
+    else moe_route_kernel<T, 4, 8, 2><<<tw_div_up(n, 4), 512, 0, stream>>>((const T*)h, ld_h, router, bias, mode, n, C, X, top, ids, weights, groups, keep, scale); \
   } while (0)
   if (dtype == TW_DTYPE_BF16) TW_MOE_ROUTE(bf16_t);
   else if (dtype == TW_DTYPE_F32) TW_MOE_ROUTE(float);
@@ -721,44 +771,86 @@ __global__ __launch_bounds__(256, WN == 2 ? 3 : 4) void moe_parts_kernel(const f
 // float32 [splits][n][C] partial sums of something else that belongs to the same result (a shared expert's last product
 // with its K ranges not yet added up): added here, in index order, before the experts' rows.
 // A choice without a row (pos -1) is an expert that returns h itself.
+struct MoeCombineArgs {
+  float* x; long ld_x;
+  const float* ys; long ld_y;
+  const int* pos;
+  const float* weights;
+  const float* more; size_t more_stride;
+  const void* h; long ld_h;
+  int C, top, splits, accumulate;
+};
+
+// Columns c .. c + 3 of a row's sum. Of up to four choices at a time the rows' places go out together, then the rows.
+template <typename T>
+__device__ __forceinline__ f32x4 moe_combined(const MoeCombineArgs& a, int row, int c) {
+  f32x4 sum = {0.f, 0.f, 0.f, 0.f};
+  const f32x4 own = moe_four((const T*)a.h + (size_t)row * a.ld_h + c);
+  if (a.more)
+    for (int s = 0; s < a.splits; ++s) sum += *reinterpret_cast<const f32x4*>(a.more + s * a.more_stride + (size_t)row * a.C + c);
+  for (int r0 = 0; r0 < a.top; r0 += 4) {
+    int at[4];
+    float w[4];
+    f32x4 y[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const size_t item = (size_t)row * a.top + min(r0 + j, a.top - 1);
+      at[j] = a.pos[item];
+      w[j] = a.weights ? a.weights[item] : 1.f;
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) y[j] = *reinterpret_cast<const f32x4*>(a.ys + (size_t)max(at[j], 0) * a.ld_y + c);
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      if (r0 + j < a.top) sum += w[j] * (at[j] >= 0 ? y[j] : own);
+  }
+  return sum;
+}
+
 template <typename T, bool VEC>
-__global__ __launch_bounds__(256) void moe_combine_kernel(float* __restrict__ x, long ld_x, const float* __restrict__ ys,
-                                                          long ld_y, const int* __restrict__ pos, int C, int top,
-                                                          const float* __restrict__ weights, int accumulate,
-                                                          const float* __restrict__ more, int splits, size_t more_stride,
-                                                          const T* __restrict__ h, long ld_h) {
+__global__ __launch_bounds__(256) void moe_combine_kernel(MoeCombineArgs a) {
   const int row = blockIdx.x;
   const int c = blockIdx.y * 1024 + threadIdx.x * 4;
-  if (c >= C) return;
-  const T* own = h + (size_t)row * ld_h + c;
+  if (c >= a.C) return;
   if constexpr (VEC) {
-    f32x4 sum = {0.f, 0.f, 0.f, 0.f};
-    if (more)
-      for (int s = 0; s < splits; ++s) sum += *reinterpret_cast<const f32x4*>(more + s * more_stride + (size_t)row * C + c);
-    for (int r = 0; r < top; ++r) {
-      const int at = pos[(size_t)row * top + r];
-      f32x4 y;
-      if (at >= 0) y = *reinterpret_cast<const f32x4*>(ys + (size_t)at * ld_y + c);
-      else y = f32x4{tw_to_float(own[0]), tw_to_float(own[1]), tw_to_float(own[2]), tw_to_float(own[3])};
-      if (weights) sum += weights[(size_t)row * top + r] * y;
-      else sum += y;
-    }
-    f32x4* dst = reinterpret_cast<f32x4*>(x + (size_t)row * ld_x + c);
-    if (accumulate) *dst += sum;
-    else *dst = sum;
+    f32x4* dst = reinterpret_cast<f32x4*>(a.x + (size_t)row * a.ld_x + c);
+    const f32x4 before = a.accumulate ? *dst : f32x4{0.f, 0.f, 0.f, 0.f};
+    const f32x4 sum = moe_combined<T>(a, row, c);
+    *dst = a.accumulate ? before + sum : sum;
   } else {
-    for (int j = 0; j < 4 && c + j < C; ++j) {
+    const T* own = (const T*)a.h + (size_t)row * a.ld_h + c;
+    for (int j = 0; j < 4 && c + j < a.C; ++j) {
       float sum = 0.f;
-      if (more)
-        for (int s = 0; s < splits; ++s) sum += more[s * more_stride + (size_t)row * C + c + j];
-      for (int r = 0; r < top; ++r) {
-        const int at = pos[(size_t)row * top + r];
-        sum += (weights ? weights[(size_t)row * top + r] : 1.f) * (at >= 0 ? ys[(size_t)at * ld_y + c + j] : tw_to_float(own[j]));
+      if (a.more)
+        for (int s = 0; s < a.splits; ++s) sum += a.more[s * a.more_stride + (size_t)row * a.C + c + j];
+      for (int r = 0; r < a.top; ++r) {
+        const int at = a.pos[(size_t)row * a.top + r];
+        sum += (a.weights ? a.weights[(size_t)row * a.top + r] : 1.f) * (at >= 0 ? a.ys[(size_t)at * a.ld_y + c + j] : tw_to_float(own[j]));
       }
-      if (accumulate) x[(size_t)row * ld_x + c + j] += sum;
-      else x[(size_t)row * ld_x + c + j] = sum;
+      float* x = a.x + (size_t)row * a.ld_x + c + j;
+      *x = a.accumulate ? *x + sum : sum;
     }
   }
+}
+
+// The same with the RMS norm of the new rows behind it, out = round(x / sqrt(mean(x^2) + eps) * weight): rows of up to 4,096 elements, a
+// workgroup each, so that the stream's next reader needs no launch of its own in front of it (a captured step of float32 layers with
+// experts, 4 rows, 469 us with launches of their own and the routers as they were, 445 with both). out may be h.
+template <typename T>
+__global__ __launch_bounds__(1024) void moe_combine_norm_kernel(MoeCombineArgs a, const float* __restrict__ weight, float eps, T* out) {
+  __shared__ float lds[16];
+  const int row = blockIdx.x, c = min((int)threadIdx.x * 4, a.C - 4);
+  const bool mine = (int)threadIdx.x * 4 < a.C;
+  float* x = a.x + (size_t)row * a.ld_x + c;
+  const f32x4 before = *reinterpret_cast<const f32x4*>(x), w = *reinterpret_cast<const f32x4*>(weight + c);
+  const f32x4 v = before + moe_combined<T>(a, row, c);
+  const float ss = mine ? ((v[0] * v[0] + v[1] * v[1]) + v[2] * v[2]) + v[3] * v[3] : 0.f;
+  const float rinv = 1.0f / sqrtf(tw_block_sum(ss, lds) / (float)a.C + eps);       // (the barrier: every read of the row, clamped ones too, lies before)
+  if (!mine) return;
+  *reinterpret_cast<f32x4*>(x) = v;
+  T* dst = out + (size_t)row * a.C + c;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) dst[e] = tw_from_float<T>(v[e] * rinv * w[e]);
 }
 
 // Steps of many rows: do the waves of a workgroup better split K than the columns? (float32, 16 experts of 2,048 x 1,408 gated, two a
@@ -903,6 +995,9 @@ struct MoeStep {
   int n, top, X, C, Cd, Fd, capacity, kind, accumulate, more_splits;
   float limit;
   bool wide, few;
+  const float* norm_weight;
+  void* normed;
+  float norm_eps;
 };
 
 template <typename T, int ACT>
@@ -919,6 +1014,11 @@ static void moe_products_few(const MoeStep& s, hipStream_t stream) {
 static bool moe_few(int dtype, const void* h, long ld_h, int n, int top, int C, int Cd, int kind) {
   const int epf = dtype == TW_DTYPE_BF16 ? 8 : 4;
   return kind != 0 && n * top <= 64 && C == Cd && C % (4 * epf) == 0 && ld_h % epf == 0 && (uintptr_t)h % 16 == 0;
+}
+
+template <typename T>
+static bool moe_combine_wide(const MoeStep& s) {
+  return s.C % 4 == 0 && s.ld_x % 4 == 0 && s.ld_h % 4 == 0 && ((((uintptr_t)s.x | (uintptr_t)s.ys | (uintptr_t)s.more) & 15) == 0) && ((uintptr_t)s.h & (4 * sizeof(T) - 1)) == 0;
 }
 
 template <typename T>
@@ -942,27 +1042,25 @@ static void moe_run(const MoeStep& s, hipStream_t stream) {
 #undef TW_MOE_PRODUCTS
   }
   if (!s.x) return;                                  // (whoever reads ys and pos adds them up)
+  const MoeCombineArgs a{s.x, s.ld_x, s.ys, s.C, s.pos, s.kind == 0 ? nullptr : s.weights, s.more, (size_t)s.n * s.C, s.h, s.ld_h,
+                         s.C, s.top, s.more_splits, s.accumulate};
   const dim3 grid(s.n, tw_div_up(s.C, 1024));
-  const size_t more_stride = (size_t)s.n * s.C;
-  const float* weights = s.kind == 0 ? nullptr : s.weights;
-  if (s.C % 4 == 0 && s.ld_x % 4 == 0 && (uintptr_t)s.x % 16 == 0 && (uintptr_t)s.ys % 16 == 0 && (uintptr_t)s.more % 16 == 0)
-    moe_combine_kernel<T, true><<<grid, 256, 0, stream>>>(s.x, s.ld_x, s.ys, s.C, s.pos, s.C, s.top, weights, s.accumulate, s.more,
-                                                          s.more_splits, more_stride, (const T*)s.h, s.ld_h);
-  else
-    moe_combine_kernel<T, false><<<grid, 256, 0, stream>>>(s.x, s.ld_x, s.ys, s.C, s.pos, s.C, s.top, weights, s.accumulate, s.more,
-                                                           s.more_splits, more_stride, (const T*)s.h, s.ld_h);
+  if (s.norm_weight) moe_combine_norm_kernel<T><<<s.n, tw_div_up(s.C, 256) * 64, 0, stream>>>(a, s.norm_weight, s.norm_eps, (T*)s.normed);
+  else if (moe_combine_wide<T>(s)) moe_combine_kernel<T, true><<<grid, 256, 0, stream>>>(a);
+  else moe_combine_kernel<T, false><<<grid, 256, 0, stream>>>(a);
 }
 
 // h [n][C] (compute type) -> x [n][C] float32 += the routed experts' results. ids, weights [n * top] come from
 // tw_moe_route (ids of X and above, where the weights multiply outputs: experts that return h). Scratch: pos [n * top],
 // src_item [capacity], tile_expert [capacity / 16] (int32), xs [capacity][Cd], act [capacity][Fd] (compute type),
 // ys [capacity][C] (float32), capacity = tw_moe_capacity(n * top, X). x null: the experts' rows stay in ys, unweighted, pair i's
-// in row pos[i] (kinds whose weights multiply outputs).
+// in row pos[i] (kinds whose weights multiply outputs). norm_weight (or null; with accumulate, aligned rows of up to 4,096 elements): the new rows
+// of x behind an RMS norm as well, normed [n][C] in the compute type (h, if it is contiguous, will do).
 extern "C" int tw_moe_experts(int dtype, const void* h, long ld_h, const int* ids, const float* weights, int n, int top, int X,
                               const void* gate, const void* up, const void* down, int C, int Cd, int Fd, float limit,
                               int* pos, int* src_item, int* tile_expert, void* xs, void* act, float* ys, int capacity,
                               float* x, long ld_x, int kind, int accumulate, const float* more, int more_splits,
-                              hipStream_t stream) {
+                              const float* norm_weight, float norm_eps, void* normed, hipStream_t stream) {
   TW_REQUIRE(h && ids && weights && up && down && pos && src_item && tile_expert && xs && act && ys && (x || (kind != 0 && !more)));
   TW_REQUIRE(((kind == 0 || kind == 2) && gate) || kind == 1 || kind == 3);
   TW_REQUIRE(more == nullptr || more_splits > 0);
@@ -980,7 +1078,9 @@ extern "C" int tw_moe_experts(int dtype, const void* h, long ld_h, const int* id
   const bool wide = moe_unit((long)n * top, X) == TW_MOE_TILE * TW_MOE_WIDE;
   TW_REQUIRE(!wide || capacity % (TW_MOE_TILE * TW_MOE_WIDE) == 0);
   const MoeStep s{h, gate, up, down, ld_h, ld_x, weights, ids, src_item, tile_expert, pos, xs, act, ys, x, more,
-                  n, top, X, C, Cd, Fd, capacity, kind, accumulate, more_splits, limit, wide, few};
+                  n, top, X, C, Cd, Fd, capacity, kind, accumulate, more_splits, limit, wide, few, norm_weight, normed, norm_eps};
+  TW_REQUIRE(norm_weight == nullptr || (x && accumulate && normed && norm_eps > 0.f && C <= 4096 && (uintptr_t)norm_weight % 16 == 0 &&
+                                        (dtype == TW_DTYPE_BF16 ? moe_combine_wide<bf16_t>(s) : moe_combine_wide<float>(s))));
   if (dtype == TW_DTYPE_BF16) moe_run<bf16_t>(s, stream);
   else moe_run<float>(s, stream);
   return TW_LAUNCH_RESULT();

@@ -1506,7 +1506,12 @@ MOE_KINDS = {"swish_limited": 0, "gelu": 1, "silu": 2, "relu_squared": 3}
 MOE_PLAIN = ("gelu", "relu_squared")           # kinds without a gate
 
 
-def moe_experts(h, ids, weights, gate, up, down, limit, x, scratch, kind="swish_limited", accumulate=True, more=None):
+def can_moe_norm(h, x):
+    """Can `moe_experts` norm the rows it adds to? (aligned rows of up to 4,096 elements)"""
+    return (x.shape[1] <= 4096 and x.shape[1] % 4 == 0 and x.is_contiguous() and h.is_contiguous() and x.data_ptr() % 16 == 0 and h.data_ptr() % 16 == 0)
+
+
+def moe_experts(h, ids, weights, gate, up, down, limit, x, scratch, kind="swish_limited", accumulate=True, more=None, norm=None):
     """kind "gelu" (gate None): x[n] (+)= sum over a row's chosen experts e of weights_e * down_e(gelu(up_e h[n])), the exact
     gelu; accumulate=False writes x instead of adding to it; more: float32 [splits, n, C] partial sums of something that
     belongs to the same result (a shared expert's last product), added up here as well. kind "silu": the same with
@@ -1514,7 +1519,8 @@ def moe_experts(h, ids, weights, gate, up, down, limit, x, scratch, kind="swish_
     nothing is added up; returns (rows, pos), row pos[i] being what pair i's expert gives. In these kinds an id of X or above names an expert that returns h[n] itself.
     kind "swish_limited": x[n] += sum over a row's chosen experts e of down_e(glu(gate_e y, up_e y)), y = round(weights * h[n]), glu the
     limited swish with LIMIT. gate, up [X, Fd, Cd], down [X, C16, Fd] in h's type, zero padded (Fd, Cd: `moe_pad` of the
-    sizes, C16: C rounded up to 16) and laid out by `moe_blocked`. scratch(tag, shape, dtype) hands out the step's scratch tensors."""
+    sizes, C16: C rounded up to 16) and laid out by `moe_blocked`. scratch(tag, shape, dtype) hands out the step's scratch tensors.
+    norm (with accumulate, see `can_moe_norm`): (weight, eps, out), the new x behind that RMS norm as well, out [n, C] of h's type (h will do)."""
     n, C, ld_h = _rows(h, "h")
     top = ids.shape[1]
     _need(kind in MOE_KINDS and (gate is None) == (kind in MOE_PLAIN), f"experts are one of {sorted(MOE_KINDS)}, all but {MOE_PLAIN} with a gate")
@@ -1535,6 +1541,10 @@ def moe_experts(h, ids, weights, gate, up, down, limit, x, scratch, kind="swish_
     if more is not None:
         _need(more.dim() == 3 and more.is_contiguous() and tuple(more.shape[1:]) == (n, C) and more.dtype == torch.float32,
               "more must be float32 [splits, n, C]")
+    if norm is not None:
+        weight, norm_eps, normed = norm
+        _need(x is not None and accumulate and can_moe_norm(h, x) and weight.is_contiguous() and weight.numel() == C, "these rows cannot be normed here")
+        _need(normed.is_contiguous() and tuple(normed.shape) == (n, C) and normed.dtype == h.dtype, "the normed rows must be [n, C] of h's type")
     capacity = moe_capacity(n * top, X)
     pos = scratch("moe.pos", (n * top,), torch.int32)
     src_item = scratch("moe.src", (capacity,), torch.int32)
@@ -1548,7 +1558,8 @@ def moe_experts(h, ids, weights, gate, up, down, limit, x, scratch, kind="swish_
                                    float(limit), _dev(pos), _dev(src_item), _dev(tile_expert), _dev(xs), _dev(act), _dev(ys),
                                    capacity, _dev(x) if x is not None else None, ld_x, MOE_KINDS[kind], 1 if accumulate else 0,
                                    _dev(more) if more is not None else None, more.shape[0] if more is not None else 0,
-                                   _stream()), "moe_experts")
+                                   _dev(weight, torch.float32, "norm weight") if norm is not None else None, float(norm_eps) if norm is not None else 0.0,
+                                   _dev(normed) if norm is not None else None, _stream()), "moe_experts")
     return x if x is not None else (ys, pos)
 
 

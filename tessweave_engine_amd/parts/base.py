@@ -169,6 +169,11 @@ class FeedForward(Part):
 class Block(Part):
     mixer: Mixer
 
+    @property
+    def first_norm(self):
+        """The one norm through which the block reads the stream, if it takes the rows that the part before left under NORMED_STREAM; else None."""
+        return None
+
     def entry(self):
         """(norms, readers): the norms that the block starts with (none: it reads the stream as it is) and the parts that read the
         rows, if the block takes `ops.NormedRows` for them in place of pending sums; None if not."""
@@ -313,6 +318,9 @@ class StepContext:
         self.defer_sums = True       # may a mixer or feed-forward leave partial sums pending for the next norm?
         self.capturing = False       # launches may depend on kv_bound and capacities, not on this step's lengths
         self.norm_ahead = None       # NormAhead for the sublayer that runs now: the norms that read the stream behind it
+        self.norm_behind = None      # the one norm that reads the stream behind the block that runs now, if only one does (captured steps)
+        self.norm_closing = None     # the same for a sublayer whose last kernel writes the stream as that norm will read it: it may norm
+                                     # it there and leave it under NORMED_STREAM
         self.tables_wanted = ()      # rotary encodings whose tables a layer will ask for: an embedding may form them with its rows
         self.entry_behind = None     # (norms, readers) of what runs behind the block that runs now, or None (see Block.entry)
         self.segment_end = None      # while a step is captured: called with the index of each finished layer run

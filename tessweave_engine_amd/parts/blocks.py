@@ -12,6 +12,7 @@ from ..cache.spec import CacheNeed
 from ..kernels import ops
 from ..weights.spec import AVERAGE, ONE_PLUS_NORMAL, VECTOR, TensorSpec
 from .base import NORMED_STREAM, ROUNDED_STREAM, Block, fold_pending, norm_ahead
+from .norms import LayerNorm, RMSNorm
 
 
 class PreNormBlock(Block):
@@ -57,6 +58,9 @@ def normalise(norm, ctx, x, pending=None, rows=None):
         if pending.norm is not norm or (rows is not None and rows.numel() != pending.shape[0]):
             raise RuntimeError("the rows left by the product before are another norm's")
         return pending
+    held, normed = ctx.shared.pop(NORMED_STREAM, (None, None))
+    if held is norm and pending is None and (rows is None or rows.numel() == normed.shape[0] == x.shape[0]):
+        return normed
     if pending is not None and not norm.folds_pending:
         pending = fold_pending(x, pending)
     if pending is not None:
@@ -105,12 +109,14 @@ class ParallelBlock(Block):
             left = self.mixer.forward(ctx, run, h, x)
             if self.ffn is None:
                 return left
-            if left is None:
-                return self.ffn.forward(ctx, h, x)
-            if self.ffn.folds_beside:
-                return self.ffn.forward(ctx, h, x, more=left)
-            fold_pending(x, left)
-            return self.ffn.forward(ctx, h, x)
+            more = {"more": left} if left is not None and self.ffn.folds_beside else {}
+            if left is not None and not more:
+                fold_pending(x, left)
+            ctx.norm_closing = ctx.norm_behind if isinstance(ctx.norm_behind, RMSNorm) else None
+            try:
+                return self.ffn.forward(ctx, h, x, **more)
+            finally:
+                ctx.norm_closing = None
         if isinstance(pending, ops.NormedRows):
             h1, h2 = pending, pending.second
             if h1.norm is not self.mixer_norm or (h2.norm if h2 is not None else None) is not self.ffn_norm:
@@ -132,6 +138,10 @@ class ParallelBlock(Block):
             if left is not None and not isinstance(left, ops.NormedRows):
                 raise RuntimeError("a parallel block's feed-forward must add into the stream itself")
         return left
+
+    @property
+    def first_norm(self):
+        return self.mixer_norm if self.shared_norm else None
 
     def entry(self):
         if self.shared_norm:
@@ -324,17 +334,20 @@ class SandwichBlock(Block):
 
     def forward(self, ctx, run, x, pending=None):
         norm, h = ctx.shared.pop(NORMED_STREAM, (None, None))
+        follows = self.next_norm
+        if follows is None and isinstance(ctx.norm_behind, LayerNorm) and ctx.norm_behind.size == self.hidden and ctx.norm_behind.eps == self.mixer_norm.eps:
+            follows = ctx.norm_behind         # (of a captured step, which wants every row)
         if norm is not self.mixer_norm or pending is not None:
             h = normalise(self.mixer_norm, ctx, x, pending)
         result = ctx.scratch("sublayer.result", (ctx.n_tokens, self.hidden), torch.float32)
         left = self.mixer.forward(ctx, run, h, result, accumulate=False)
-        h = self._close(ctx, x, self.mixer_after, self.ffn_norm if self.ffn is not None else self.next_norm, result, left)
+        h = self._close(ctx, x, self.mixer_after, self.ffn_norm if self.ffn is not None else follows, result, left)
         if self.ffn is not None:
             options = {"apart": True} if self.ffn.leaves_apart else {}
             left = self.ffn.forward(ctx, h, result, accumulate=False, **options)
-            h = self._close(ctx, x, self.ffn_after, self.next_norm, result, left)
+            h = self._close(ctx, x, self.ffn_after, follows, result, left)
         if h is not None:
-            ctx.shared[NORMED_STREAM] = (self.next_norm, h)
+            ctx.shared[NORMED_STREAM] = (follows, h)
         return None
 
 

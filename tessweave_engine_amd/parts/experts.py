@@ -31,7 +31,7 @@ import torch
 
 from ..kernels import ops
 from ..weights.spec import MATRIX, NORMAL, VECTOR, TensorSpec
-from .base import FeedForward, fold_pending
+from .base import FeedForward, NORMED_STREAM, fold_pending
 
 
 #: a result left apart: `add` float32 [splits, n, hidden] or None, `pairs` (expert rows, places, weights), and whether a further
@@ -152,6 +152,10 @@ class RoutedExperts(FeedForward):
         if apart:
             rows, pos = ops.moe_experts(h, ids, weights, self.gate, self.up, self.down, self.limit, None, scratch, kind=self.kind)
             return ApartResult(pending, (rows, pos, weights), wrote)
+        norm, behind = None, getattr(ctx, "norm_closing", None)
+        if behind is not None and accumulate and behind.size == self.hidden and ops.can_moe_norm(h, x):
+            norm = (behind.weight, behind.eps, ctx.scratch("norm.out", (n, self.hidden)))      # (the last kernel norms what it wrote)
+            ctx.shared[NORMED_STREAM] = (behind, norm[2])
         ops.moe_experts(h, ids, weights, self.gate, self.up, self.down, self.limit, x, scratch, kind=self.kind,
-                        accumulate=accumulate or wrote, more=pending)
+                        accumulate=accumulate or wrote, more=pending, norm=norm)
         return None

@@ -129,6 +129,13 @@ class DecoderModel(Part):
         following = self.schedule[i + 1]
         return None if following.adds_embedding else self.blocks[following.block].entry()
 
+    def _norm_behind(self, i):
+        """The one norm that reads the stream behind run I, or None (see `Block.first_norm`)."""
+        if i + 1 == len(self.schedule):
+            return self.final_norm
+        following = self.schedule[i + 1]
+        return None if following.adds_embedding else self.blocks[following.block].first_norm
+
     # ---- one step -----------------------------------------------------------------
     def forward(self, ctx):
         """Run the step's tokens; float32 logits [n_logits, vocab] at ctx.logit_rows."""
@@ -144,7 +151,8 @@ class DecoderModel(Part):
                     pending = first.unsqueeze(0)          # the run's first norm adds it, like any pending sum
                 else:
                     ops.add_values(x, first)
-            ctx.entry_behind = self._entry_behind(i) if ctx.capturing else None
+            if ctx.capturing:
+                ctx.entry_behind, ctx.norm_behind = self._entry_behind(i), self._norm_behind(i)
             pending = self.blocks[run.block].forward(ctx, run, x, pending)
             if ctx.segment_end is not None:
                 ctx.segment_end(i)

@@ -186,3 +186,27 @@ def test_embed_begin(ops, device, dtype, n, hidden, form):
             assert torch.equal(left.second.rows, (x * weights[1]).to(dtype))
     elif form == "rounded":
         assert left is None and torch.equal(rows[0], x.to(dtype))
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("n,c,top,splits", [(1, 64, 1, 0), (4, 2048, 2, 3), (16, 1056, 5, 0), (3, 4096, 8, 1)])
+def test_experts_sums_behind_a_norm(ops, device, dtype, n, c, top, splits):
+    """The kernel that adds up a token's experts and norms the row, against the same sums and the norm's own kernel."""
+    experts, ff = 6, 32
+    h, x = rand((n, c), dtype, device), rand((n, c), torch.float32, device, 1.0, 1)
+    gate, up = (ops.moe_blocked(rand((experts, ff, c), dtype, device, c ** -0.5, s)) for s in (2, 3))
+    down = ops.moe_blocked(rand((experts, c, ff), dtype, device, ff ** -0.5, 4))
+    ids = torch.tensor([[(3 * i + 2 * j) % (experts + 2) for j in range(top)] for i in range(n)], dtype=torch.int32, device=device)    # (two return their input)
+    weights, norm = rand((n, top), torch.float32, device, 0.3, 5), 1 + rand((c,), torch.float32, device, 0.1, 6)
+    more = rand((splits, n, c), torch.float32, device, 1.0, 7) if splits else None
+    buffers = {}
+
+    def scratch(tag, shape, dt):
+        return buffers.setdefault((tag, dt), torch.empty(shape, dtype=dt, device=device))
+    want = x.clone()
+    ops.moe_experts(h, ids, weights, gate, up, down, 0.0, want, scratch, kind="silu", more=more)
+    wanted = ops.rmsnorm(want, norm, 1e-6, torch.empty_like(h))
+    out = h.clone()
+    ops.moe_experts(out, ids, weights, gate, up, down, 0.0, x, scratch, kind="silu", more=more, norm=(norm, 1e-6, out))
+    assert torch.equal(x, want)
+    torch.testing.assert_close(out.float(), wanted.float(), atol=0, rtol=2.0 ** -7 if dtype == torch.bfloat16 else 1e-6)     # (a last place: sums in another order)
