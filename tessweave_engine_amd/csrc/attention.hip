@@ -626,7 +626,7 @@ __global__ __launch_bounds__(TW_REDUCE_THREADS) void attn_decode_reduce_kernel(
     const float lw = tid < splits ? part_ml[(slot0 + tid) * 2 + 1] * w : 0.f;
     // fixed-order sum over the splits
     float l = 0.f;
-    for (int i = 0; i < 64; ++i) l += __shfl(lw, i, TW_WAVE);
+    for (int i = 0; i < splits; ++i) l += __shfl(lw, i, TW_WAVE);
     if (sink) l += expf(sink[head] - m_use);
     if (tid == 0) s_l = l;
   }
@@ -650,6 +650,57 @@ __global__ __launch_bounds__(TW_REDUCE_THREADS) void attn_decode_reduce_kernel(
     if (gate) total *= gate[(size_t)token * q_heads + head];
     out[(size_t)token * ldo + (size_t)head * head_dim + tid] = tw_from_float<T>(total);
   }
+}
+
+// The same where a head is two maps side by side whose difference is normed (differential attention, as map_difference_kernel):
+//   o = a1 - lambda a2,   out = o / sqrt(mean(o^2) + eps) * factor * gate,   rounded once, heads out_dim elements apart.
+// A workgroup has both maps of a (head, token), half of its threads each, so that the merged maps need not go through memory and another
+// launch. In captured steps of 8 tokens, 8 heads of 128, 1.8 us a layer of 10 (the ranges' merge, and map_difference behind it).
+struct MapsEnd {
+  const float* gate;                           // [tokens][heads], or null
+  int value_dim, out_dim;
+  float lambda, factor, eps;
+};
+template <typename T>
+__global__ __launch_bounds__(512) void attn_decode_difference_kernel(const float* __restrict__ part_o, const float* __restrict__ part_ml,
+                                                                     const int* __restrict__ q_start, int seq0, T* out, long ldo, int heads,
+                                                                     int head_dim, int splits, MapsEnd e) {
+  __shared__ float s_w[2][64], s_l[2], s_second[256], red[16];
+  const int half = blockDim.x / 2, map = threadIdx.x >= half, d = threadIdx.x - map * half;      // half: whole waves, at least head_dim
+  const int head = blockIdx.x, local = blockIdx.y;
+  const size_t slot0 = ((size_t)local * 2 * heads + 2 * head + map) * splits;
+  const int token = q_start[seq0 + local];
+  const float gate = e.gate ? e.gate[(size_t)token * heads + head] : 1.f;
+  const bool mine = d < head_dim;
+  float po[8];                                 // (on their way while the weights are formed)
+#pragma unroll
+  for (int i = 0; i < 8; ++i) po[i] = mine && i < splits ? part_o[(slot0 + i) * head_dim + d] : 0.f;
+  if (d < 64) {                                // each map's first wave
+    const float m_of = d < splits ? part_ml[(slot0 + d) * 2] : -INFINITY, l_of = d < splits ? part_ml[(slot0 + d) * 2 + 1] : 0.f;
+    const float m = tw_wave_max(m_of), m_use = m == -INFINITY ? 0.f : m;
+    const float w = d < splits ? expf(m_of - m_use) : 0.f;
+    s_w[map][d] = w;
+    const float lw = l_of * w;
+    float l = 0.f;
+    for (int i = 0; i < splits; ++i) l += __shfl(lw, i, TW_WAVE);
+    if (d == 0) s_l[map] = l;
+  }
+  __syncthreads();
+  float o = 0.f;
+#pragma unroll
+  for (int i = 0; i < 8; ++i)
+    if (i < splits) o += po[i] * s_w[map][i];
+  if (mine)
+    for (int i = 8; i < splits; ++i) o += part_o[(slot0 + i) * head_dim + d] * s_w[map][i];
+  const float l = s_l[map];
+  o = l > 0.f ? o / l : 0.f;
+  if (map && mine) s_second[d] = o;
+  __syncthreads();
+  const float v = !map && d < e.value_dim ? __fmaf_rn(-e.lambda, s_second[d], o) : 0.f;      // (value_dim <= head_dim)
+  const float ss = tw_block_sum(v * v, red);
+  const float f = e.factor / sqrtf(ss / (float)e.value_dim + e.eps) * gate;
+  if (map) return;
+  for (int c = d; c < e.out_dim; c += half) out[(size_t)token * ldo + (size_t)head * e.out_dim + c] = tw_from_float<T>(c == d ? v * f : 0.f);
 }
 
 // =====================================================================================
@@ -1636,8 +1687,9 @@ extern "C" long tw_attn_decode_workspace_floats(int n_seqs, int q_heads, int hea
 template <typename T> struct IsBf16 { static constexpr bool value = false; };
 template <> struct IsBf16<bf16_t> { static constexpr bool value = true; };
 
+// maps: null, or what becomes of pairs of heads (splits > 1; a.out then is that result)
 template <typename T>
-static int decode_launch(AttnArgs a, int n_seqs, int generic, hipStream_t stream) {
+static int decode_launch(AttnArgs a, int n_seqs, int generic, const MapsEnd* maps, hipStream_t stream) {
   const int G = a.q_heads / a.kv_heads;
   dim3 grid(a.splits, a.kv_heads * ((G + 15) / 16), n_seqs);
   if (IsBf16<T>::value && a.page_shift >= 3 && !generic) {
@@ -1662,6 +1714,11 @@ static int decode_launch(AttnArgs a, int n_seqs, int generic, hipStream_t stream
     attn_decode_kernel<T, 16, 4><<<grid, 256, 0, stream>>>(a);
   int err = TW_LAUNCH_RESULT();
   if (err || a.splits == 1) return err;
+  if (maps) {
+    attn_decode_difference_kernel<T><<<dim3(a.q_heads / 2, n_seqs), 2 * ((a.head_dim + 63) / 64 * 64), 0, stream>>>(
+        a.part_o, a.part_ml, a.q_start, a.seq0, (T*)a.out, a.ldo, a.q_heads / 2, a.head_dim, a.splits, *maps);
+    return TW_LAUNCH_RESULT();
+  }
   const dim3 rgrid(a.q_heads, n_seqs);
   if (a.out_f32)
     attn_decode_reduce_kernel<float><<<rgrid, TW_REDUCE_THREADS, 0, stream>>>(
@@ -1675,12 +1732,12 @@ static int decode_launch(AttnArgs a, int n_seqs, int generic, hipStream_t stream
 // Sequences seq0 .. seq0 + n_seqs - 1 must each have exactly one token in this step.
 // `workspace` holds tw_attn_decode_workspace_floats floats when splits > 1.
 // generic != 0 forces the kernel that takes every type and page size.
-extern "C" int tw_attn_decode(int dtype, const void* q, long ldq, const void* keys, const void* values,
+static int attn_decode(int dtype, const void* q, long ldq, const void* keys, const void* values,
                               const int* block_table, int table_stride, const int* q_start,
                               const int* kv_len, int seq0, int n_seqs, void* out, long ldo,
                               float* workspace, long workspace_floats, int q_heads, int kv_heads,
                               int head_dim, int page_size, int window, int chunk, float scale, float softcap, int splits,
-                              int generic, const float* sink, const float* gate, int out_f32, hipStream_t stream) {
+                              int generic, const float* sink, const float* gate, int out_f32, const MapsEnd* maps, hipStream_t stream) {
   AttnArgs a;
   a.q = q; a.ldq = ldq; a.keys = keys; a.values = values; a.block_table = block_table;
   a.table_stride = table_stride; a.q_start = q_start; a.kv_len = kv_len; a.seq0 = seq0;
@@ -1693,8 +1750,10 @@ extern "C" int tw_attn_decode(int dtype, const void* q, long ldq, const void* ke
   a.page_shift = -1;
   for (int sh = 0; sh < 20; ++sh)
     if ((1 << sh) == page_size) a.page_shift = sh;
+  if (maps) a.ldo = (long)q_heads * head_dim;                  // (the ranges' kernel does not write out)
   int err = check_common(a);
   if (err) return err;
+  a.ldo = ldo;
   TW_REQUIRE(n_seqs >= 0 && seq0 >= 0 && splits >= 1 && splits <= 64 && n_seqs <= 65535);
   if (n_seqs == 0) return 0;
   if (splits > 1) {
@@ -1703,9 +1762,32 @@ extern "C" int tw_attn_decode(int dtype, const void* q, long ldq, const void* ke
     a.part_o = workspace;
     a.part_ml = workspace + (size_t)n_seqs * q_heads * splits * head_dim;
   }
-  if (dtype == TW_DTYPE_F32) return decode_launch<float>(a, n_seqs, generic, stream);
-  if (dtype == TW_DTYPE_BF16) return decode_launch<bf16_t>(a, n_seqs, generic, stream);
+  if (dtype == TW_DTYPE_F32) return decode_launch<float>(a, n_seqs, generic, maps, stream);
+  if (dtype == TW_DTYPE_BF16) return decode_launch<bf16_t>(a, n_seqs, generic, maps, stream);
   return TW_ERR_BAD_ARGUMENT;
+}
+extern "C" int tw_attn_decode(int dtype, const void* q, long ldq, const void* keys, const void* values,
+                              const int* block_table, int table_stride, const int* q_start,
+                              const int* kv_len, int seq0, int n_seqs, void* out, long ldo,
+                              float* workspace, long workspace_floats, int q_heads, int kv_heads,
+                              int head_dim, int page_size, int window, int chunk, float scale, float softcap, int splits,
+                              int generic, const float* sink, const float* gate, int out_f32, hipStream_t stream) {
+  return attn_decode(dtype, q, ldq, keys, values, block_table, table_stride, q_start, kv_len, seq0, n_seqs, out, ldo, workspace, workspace_floats,
+                     q_heads, kv_heads, head_dim, page_size, window, chunk, scale, softcap, splits, generic, sink, gate, out_f32, nullptr, stream);
+}
+
+// The same over key ranges (splits > 1), followed by tw_map_difference: q_heads heads are pairs of maps, out [tokens][q_heads / 2][out_dim] in
+// q's type.
+extern "C" int tw_attn_decode_difference(int dtype, const void* q, long ldq, const void* keys, const void* values, const int* block_table,
+                                         int table_stride, const int* q_start, const int* kv_len, int seq0, int n_seqs, void* out, long ldo,
+                                         float* workspace, long workspace_floats, int q_heads, int kv_heads, int head_dim, int page_size, int chunk,
+                                         float scale, int splits, int value_dim, int out_dim, float lambda, float factor, float eps,
+                                         const float* gate, hipStream_t stream) {
+  TW_REQUIRE(splits > 1 && q_heads > 0 && q_heads % 2 == 0 && value_dim > 0 && value_dim <= head_dim && out_dim >= value_dim && out_dim <= 256);
+  TW_REQUIRE(ldo >= (long)(q_heads / 2) * out_dim && eps > 0.f);
+  const MapsEnd maps{gate, value_dim, out_dim, lambda, factor, eps};
+  return attn_decode(dtype, q, ldq, keys, values, block_table, table_stride, q_start, kv_len, seq0, n_seqs, out, ldo, workspace, workspace_floats,
+                     q_heads, kv_heads, head_dim, page_size, 0, chunk, scale, 0.f, splits, 0, nullptr, nullptr, 0, &maps, stream);
 }
 
 template <typename T>

@@ -21,10 +21,12 @@ TILE_TOKENS = 128          # most tokens that one tile of rows of the prompt ker
 
 
 def paged_attention(ctx, q, keys, values, group, out, q_heads, kv_heads, head_dim, scale, window=0, softcap=0.0, chunk=0, sink=None,
-                    gate=None):
+                    gate=None, difference=None):
     """A step's causal attention over a cache group's pages: one-token sequences through the split-KV decode kernel, prompt
     portions through the prefill kernel. q [n, >= q_heads * head_dim], out [n, q_heads * head_dim]; keys and values as
-    `ctx.cache.keys_values` gives them. chunk, sink, gate and a float32 out: see `ops.attn_decode`."""
+    `ctx.cache.keys_values` gives them. chunk, sink, gate and a float32 out: see `ops.attn_decode`. difference: the result and the further
+    arguments of `ops.attn_decode_difference`, which takes a step of one-token sequences alone where it merges key ranges; out is then
+    not written and None returned."""
     n = ctx.n_tokens
     extras = dict(chunk=chunk, sink=sink, gate=gate)
     span = window or chunk                                 # most keys a query sees (0: all before it)
@@ -37,6 +39,11 @@ def paged_attention(ctx, q, keys, values, group, out, q_heads, kv_heads, head_di
         if splits > 1:
             floats = ops.attn_decode_workspace_floats(ctx.n_decode, q_heads, head_dim, most)
             ws = ctx.workspace.get("attn.split", (floats,), torch.float32)
+            if difference is not None and ctx.n_seqs == ctx.n_decode:
+                result, further = difference
+                ops.attn_decode_difference(q, keys, values, group.block_table, ctx.q_start, ctx.kv_len, 0, ctx.n_decode, result, q_heads // 2,
+                                           kv_heads, head_dim, scale, splits, ws, chunk=chunk, **further)
+                return None
         ops.attn_decode(q, keys, values, group.block_table, ctx.q_start, ctx.kv_len, 0, ctx.n_decode, out,
                         q_heads, kv_heads, head_dim, scale, window=window,
                         splits=splits, workspace=ws, softcap=softcap, **extras)

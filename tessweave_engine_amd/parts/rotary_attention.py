@@ -155,5 +155,7 @@ class DifferentialAttention(RotaryAttention):
         n, H = ctx.n_tokens, self.q_heads
         q, keys, values, group, gate = self._finish(ctx, run, proj, bias, 1.0)
         maps = ctx.scratch("rotary.maps", (n, 2 * H * self.head_dev), torch.float32)
-        paged_attention(ctx, q, keys, values, group, maps, 2 * H, self.kv_heads, self.head_dev, self.scale, chunk=self.chunk or 0)
-        ops.map_difference(maps, out, H, self.value_dim, self.weight, (1.0 - self.diff) * scale, self.eps, gate=gate)
+        further = dict(value_dim=self.value_dim, weight=self.weight, factor=(1.0 - self.diff) * scale, eps=self.eps, gate=gate)
+        if paged_attention(ctx, q, keys, values, group, maps, 2 * H, self.kv_heads, self.head_dev, self.scale, chunk=self.chunk or 0,
+                           difference=(out, further)) is not None:
+            ops.map_difference(maps, out, H, **further)

@@ -942,3 +942,35 @@ def test_greedy_generation_through_the_scheduler(device, tmp_path, name):
                 assert token == int(top.indices[t, 0]), (t, token)
                 clear += 1
     assert clear > 100
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("heads,kv_heads,head_dim,value_dim,out_dim,splits", [(1, 1, 16, 16, 16, 2), (3, 2, 48, 40, 40, 8), (4, 4, 64, 64, 72, 9), (8, 4, 128, 96, 96, 10),
+                                                                              (2, 1, 144, 130, 136, 17), (2, 2, 256, 250, 256, 64)])
+@pytest.mark.parametrize("gated,chunk", [(True, 0), (False, 32)])
+def test_ranges_merged_into_a_difference(device, dtype, heads, kv_heads, head_dim, value_dim, out_dim, splits, gated, chunk):
+    """Against the two kernels it stands for; sequences of one key (ranges without any) and of more than the ranges hold together."""
+    from tessweave_engine_amd.kernels import ops
+    g, lens, page = torch.Generator().manual_seed(3), [1, 9, 33, 700], 16
+    rand = lambda *shape: torch.randn(shape, generator=g)       # noqa: E731
+    q = rand(len(lens), 2 * heads * head_dim).to(dtype).to(device)
+    pages = (max(lens) + page - 1) // page
+    keys, values = rand(4 * pages, kv_heads, page, head_dim).to(dtype).to(device), rand(4 * pages, kv_heads, head_dim, page).to(dtype).to(device)
+    table = torch.randperm(4 * pages, generator=g).to(torch.int32).view(4, pages).to(device)
+    start, kv_len = torch.arange(5, dtype=torch.int32, device=device), torch.tensor(lens, dtype=torch.int32, device=device)
+    gate = torch.rand((4, heads), generator=g).to(device) if gated else None
+    ws = torch.empty(ops.attn_decode_workspace_floats(4, 2 * heads, head_dim, splits), device=device)
+    maps = torch.empty(4, 2 * heads * head_dim, device=device)
+    ops.attn_decode(q, keys, values, table, start, kv_len, 0, 4, maps, 2 * heads, kv_heads, head_dim, 0.11, splits=splits, workspace=ws, chunk=chunk)
+    want = torch.empty(4, heads * out_dim, dtype=dtype, device=device)
+    ops.map_difference(maps, want, heads, value_dim, 0.4, 0.7, 1e-5, gate=gate)
+    wide = torch.full((4, heads * out_dim + 8), float("nan"), dtype=dtype, device=device)
+    out = ops.attn_decode_difference(q, keys, values, table, start, kv_len, 0, 4, wide[:, :heads * out_dim], heads, kv_heads, head_dim, 0.11, splits, ws,
+                                     value_dim, 0.4, 0.7, 1e-5, gate=gate, chunk=chunk)
+    # unit rows times at most 0.7: 64 ranges added in another order are 64 roundings of 2^-24 off at most, the norm's factor as much again
+    # (one element's share of it), and what is rounded to bfloat16 may fall the other way
+    bound = 2.0 ** -16 + (2.0 ** -8 * want.float().abs() if dtype == torch.bfloat16 else 0)
+    assert ((out.float() - want.float()).abs() <= bound).all() and wide[:, heads * out_dim:].isnan().all()
+    assert not out.view(4, heads, out_dim)[:, :, value_dim:].any()
+    with pytest.raises(Exception):
+        ops.attn_decode_difference(q, keys, values, table, start, kv_len, 0, 4, out, heads, kv_heads, head_dim, 0.11, 1, ws, value_dim, 0.4, 0.7, 1e-5)
