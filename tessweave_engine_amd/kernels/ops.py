@@ -660,6 +660,26 @@ def attn_decode(q, keys, values, block_table, q_start, kv_len, seq0, n_seqs, out
     return out
 
 
+def attn_decode_difference(q, keys, values, block_table, q_start, kv_len, seq0, n_seqs, out, heads, kv_heads, head_dim, scale, splits,
+                           workspace, value_dim, weight, factor, eps, gate=None, chunk=0):
+    """`attn_decode` over key ranges (splits > 1) for heads of two maps each, then `map_difference` of what it gives, in q's type: the
+    kernel that merges the ranges forms the difference."""
+    nq, wq, ldq = _rows(q, "q")
+    no, wo, ldo = _rows(out, "out")
+    _check_attention(q, keys, values, block_table, q_start, kv_len, q[:, :2 * heads * head_dim], 2 * heads, kv_heads, head_dim)
+    _need(out.dtype == q.dtype and no == nq and wo % heads == 0 and value_dim <= min(head_dim, wo // heads) and wo // heads <= 256,
+          "attn_decode_difference shapes do not agree")
+    _need(gate is None or (gate.dtype == torch.float32 and gate.is_contiguous() and tuple(gate.shape) == (nq, heads)), "gate must be float32 [rows of q, heads]")
+    _need(seq0 + n_seqs <= kv_len.numel() and seq0 + n_seqs <= block_table.shape[0], "sequence range exceeds the metadata")
+    _need(splits > 1 and workspace.dtype == torch.float32, "attn_decode_difference merges key ranges from a float32 workspace")
+    check(library().tw_attn_decode_difference(
+        dtype_id(q.dtype), _dev(q), ldq, _dev(keys), _dev(values), _dev(block_table, torch.int32, "block_table"), block_table.stride(0),
+        _dev(q_start, torch.int32, "q_start"), _dev(kv_len, torch.int32, "kv_len"), seq0, n_seqs, _dev(out), ldo, _dev(workspace),
+        workspace.numel(), 2 * heads, kv_heads, head_dim, keys.shape[2], int(chunk or 0), float(scale), int(splits), int(value_dim), wo // heads,
+        float(weight), float(factor), float(eps), _dev(gate) if gate is not None else None, _stream()), "attn_decode_difference")
+    return out
+
+
 def attn_prefill_split(n_seqs, q_heads, kv_heads, max_q_len, max_kv_len, tile_rows=0):
     """(max_chunks, kv_chunk, tile_rows): how the fast prefill kernel would cut the keys of a tile into
     chunks that separate workgroups take (max_chunks == 1: not at all) for a launch of this shape, and the
@@ -683,26 +703,6 @@ def attn_prefill(q, keys, values, block_table, q_start, kv_len, seq0, n_seqs, ma
 
     stats float32 [rows of q, q_heads, 2]: gets what each row's softmax was taken against (a scaled
     score) and the row's sum relative to it, for `attn_kept_keys`.
-
-def attn_decode_difference(q, keys, values, block_table, q_start, kv_len, seq0, n_seqs, out, heads, kv_heads, head_dim, scale, splits,
-                           workspace, value_dim, weight, factor, eps, gate=None, chunk=0):
-    """`attn_decode` over key ranges (splits > 1) for heads of two maps each, then `map_difference` of what it gives, in q's type: the
-    kernel that merges the ranges forms the difference."""
-    nq, wq, ldq = _rows(q, "q")
-    no, wo, ldo = _rows(out, "out")
-    _check_attention(q, keys, values, block_table, q_start, kv_len, q[:, :2 * heads * head_dim], 2 * heads, kv_heads, head_dim)
-    _need(out.dtype == q.dtype and no == nq and wo % heads == 0 and value_dim <= min(head_dim, wo // heads) and wo // heads <= 256,
-          "attn_decode_difference shapes do not agree")
-    _need(gate is None or (gate.dtype == torch.float32 and gate.is_contiguous() and tuple(gate.shape) == (nq, heads)), "gate must be float32 [rows of q, heads]")
-    _need(seq0 + n_seqs <= kv_len.numel() and seq0 + n_seqs <= block_table.shape[0], "sequence range exceeds the metadata")
-    _need(splits > 1 and workspace.dtype == torch.float32, "attn_decode_difference merges key ranges from a float32 workspace")
-    check(library().tw_attn_decode_difference(
-        dtype_id(q.dtype), _dev(q), ldq, _dev(keys), _dev(values), _dev(block_table, torch.int32, "block_table"), block_table.stride(0),
-        _dev(q_start, torch.int32, "q_start"), _dev(kv_len, torch.int32, "kv_len"), seq0, n_seqs, _dev(out), ldo, _dev(workspace),
-        workspace.numel(), 2 * heads, kv_heads, head_dim, keys.shape[2], int(chunk or 0), float(scale), int(splits), int(value_dim), wo // heads,
-        float(weight), float(factor), float(eps), _dev(gate) if gate is not None else None, _stream()), "attn_decode_difference")
-    return out
-
 
     split = (max_chunks, kv_chunk[, tile_rows]) from attn_prefill_split with a float32 workspace of
     attn_prefill_workspace_floats(rows of q, ...) lets the fast bfloat16 kernel cut long key ranges
