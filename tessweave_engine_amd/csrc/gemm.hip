@@ -562,6 +562,8 @@ __global__ __launch_bounds__(TW_CU_WAVES * 64) void gemm_stream_cu_kernel(
 // Bound by the weights' latency and bytes, and by the activations that every workgroup reads from L2 (with K
 // above 4096 these cost more than they save).
 // =====================================================================================
+// HALVES: the gated form with eight gate and eight up rows a workgroup, one fragment of both (each eight weight rows of a fragment are a
+// cache line): where pairs of 16 leave CUs idle, or a second round nearly empty (see narrow_halves). The same sums in the same order.
 // ACT: the residual's stride names an activation (a form of its own: its code in the plain form cost that 0.15 us a launch).
 // In: RowNorms where A's rows are to be multiplied by their norms' factors.
 // End: what the epilogue does with a finished element.
@@ -593,7 +595,7 @@ struct EndRotate {
 template <class End> struct IsLeave { static constexpr bool value = false, after = false; };
 template <bool A> struct IsLeave<EndLeave<A>> { static constexpr bool value = true, after = A; };
 
-template <typename T, typename OutT, int WAVES, bool GLU, bool ACT = false, class In = RowsAsTheyAre, class End = EndPlain>
+template <typename T, typename OutT, int WAVES, bool GATED, bool ACT = false, class In = RowsAsTheyAre, class End = EndPlain, bool HALVES = false>
 __global__ __launch_bounds__(WAVES * 64) void gemm_narrow_kernel(const T* __restrict__ A, long lda,
                                                                  const T* __restrict__ W, long ldw,
                                                                  const float* __restrict__ bias,
@@ -602,7 +604,8 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_narrow_kernel(const T* __rest
   typedef typename Elem<T>::Frag Frag;
   constexpr bool NORMED = std::is_same<In, RowNorms>::value, ROTATE = std::is_same<End, EndRotate>::value;
   constexpr bool LEAVE = IsLeave<End>::value, AFTER = IsLeave<End>::after;
-  static_assert(!(GLU && (ROTATE || LEAVE)), "the gated form finishes plain outputs");
+  static_assert(!(GATED && (ROTATE || LEAVE)) && (GATED || !HALVES), "the gated form finishes plain outputs");
+  constexpr bool GLU = GATED && !HALVES;
   constexpr int EPF = Elem<T>::kPerFrag, U = 4, NT = GLU ? 2 : 1;
   __shared__ float sums[NT * WAVES * 16 * 16];
   __shared__ float rinv[16], rinv_before[16];
@@ -625,6 +628,12 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_narrow_kernel(const T* __rest
   const T* w_base = W + ((size_t)blockIdx.x * NT * ldw * 64 + lane) * EPF;
   if constexpr (ROTATE) {
     const int n = column(r);
+    w_base = W + ((size_t)(n >> 4) * ldw * 64 + g * 16 + (n & 15)) * EPF;
+  }
+  // HALVES: place i of 16 is gate row i, or up row i - 8, of this workgroup's eight
+  auto half_row = [&](int i) { return ((blockIdx.x & ~1) + (i >> 3)) * 16 + (blockIdx.x & 1) * 8 + (i & 7); };
+  if constexpr (HALVES) {
+    const int n = half_row(r);
     w_base = W + ((size_t)(n >> 4) * ldw * 64 + g * 16 + (n & 15)) * EPF;
   }
   const size_t w_tile = (size_t)ldw * 64 * EPF;
@@ -664,11 +673,11 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_narrow_kernel(const T* __rest
   load(1, U);
   // what the epilogue adds, requested behind the first weights: thread t < 256 finishes row t / 16, column t % 16
   const int row = tid >> 4, c = tid & 15, col = ROTATE ? column(c) : blockIdx.x * 16 + c;
-  const bool store = row < M && col < N / NT;
+  const bool store = row < M && col < N / NT;                                   // (HALVES: a row's 16 places, N is a multiple of 32)
   float add[NT], res = 0.f;
 #pragma unroll
-  for (int t = 0; t < NT; ++t) add[t] = store && bias ? bias[ROTATE ? col : (blockIdx.x * NT + t) * 16 + c] : 0.f;
-  if (!GLU && store && residual) res = residual[(size_t)row * ldr + col];
+  for (int t = 0; t < NT; ++t) add[t] = store && bias ? bias[ROTATE ? col : HALVES ? half_row(c) : (blockIdx.x * NT + t) * 16 + c] : 0.f;
+  if (!GATED && store && residual) res = residual[(size_t)row * ldr + col];
   float weight = 0.f, weight2 = 0.f, before_weight = 0.f, scale = 1.f;
   if constexpr (LEAVE) {
     if (store) {
@@ -727,6 +736,9 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_narrow_kernel(const T* __rest
   }
   if constexpr (GLU) {
     C[(size_t)row * ldc + col] = tw_from_float<OutT>(tw_glu(v[0], v[1], ldr));
+  } else if constexpr (HALVES) {
+    const float up = tw_dpp<TW_ROTATE_8>(v[0]);                // the row's other eight
+    if (c < 8) C[(size_t)row * ldc + blockIdx.x * 8 + c] = tw_from_float<OutT>(tw_glu(v[0], up, ldr));
   } else if constexpr (LEAVE) {
     if constexpr (AFTER) {
       v[0] *= scale;
@@ -1049,11 +1061,26 @@ static int launch_skinny_lds_m(const T* A, long lda, const T* W, long ldw, const
 // and 0.4 % behind the better of the two. (us, K ranges or two waves a column / whole K, at 1 and 8 rows: bf16 9216 x 2048 11.3 / 8.2, 11.6 /
 // 8.9, 12288 x 2048 13.0 / 9.9, 13.4 / 9.9; 2048 x 5632 with a residual 9.4 / 7.1, 9.7 / 9.0; float32 8192 x 2048 18.8 / 13.9, 19.4 / 14.3, 10304 x
 // 2048 21.3 / 18.0, 22.2 / 19.2, 2048 x 4096 13.2 / 11.2, 13.2 / 12.3.)
+// Gated: 16 gate and 16 up rows a workgroup, or eight of either in one fragment (HALVES), twice the workgroups that each read the
+// activations? What the fullest CU reads decides, in rows of weights (an activation's row counts for as much as below); in bfloat16 only
+// where halves are one workgroup a CU at most. (us, back to back, pairs or two waves a column / halves, 1, 4, 8 rows: bf16 2048 x 4096
+// 7.3 / 5.9, 7.8 / 6.3, 8.5 / 6.9, 4096 x 2048 5.2 / 4.8, 5.5 / 4.9, 5.8 / 5.2; float32 2048 x 2048 9.1 / 6.3, 9.6 / 6.7, 10.1 / 7.2, 3648 x 2896 15.7 / 10.8,
+// 15.3 / 11.6 at 8, 9728 x 896 10.4 / 9.1, 10.4 / 9.6, 10.5 / 10.5, 11264 x 1024 12.5 / 9.8, 12.0 / 10.0, 12.0 / 10.8, x 2048 23.1 / 20.3, 23.0 / 20.7, 23.0 / 21.1. Left
+// to pairs: bf16 9728 x 896 5.7 / 5.8, 6.1 / 6.5 at 8 rows, 16384 x 2048 12.1 / 12.5, 12.3 / 13.7; and 11264 x 2048, 10.0 / 9.6, 10.8 / 10.4 back to back,
+// but a captured step of four such layers of one row is 4 us slower with halves.)
+static double narrow_row_share(int epf, bool glu) { return epf == 8 ? 1.33 : glu ? 0.73 : 0.87; }
+static bool narrow_halves(int M, int N, int K, int epf) {
+  const int groups = N / 16;
+  const double rows = narrow_row_share(epf, true) * M;
+  if (groups > 256 && epf == 8) return false;
+  return (16 + rows) * tw_div_up(groups, 256) < 0.95 * (32 + rows) * tw_div_up(groups, 512);
+}
 static double narrow_us(int M, int N, int K, int epf, bool glu) {
-  const int size = 16 / epf, steps = tw_div_up(K / epf, 4), groups = glu ? N / 32 : tw_div_up(N, 16);
+  const bool pairs = glu && !narrow_halves(M, N, K, epf);
+  const int size = 16 / epf, steps = tw_div_up(K / epf, 4), groups = pairs ? N / 32 : tw_div_up(N, 16);
   const int waves = steps <= 48 ? 4 : steps <= 96 ? 8 : 16;            // (see launch_narrow)
   const double covered = (double)tw_div_up(tw_div_up(steps, waves), 4) * 4 * waves * 64;      // bytes of a row
-  const double cu = 1e-3 * (size == 2 ? (glu ? 0.0187 : 0.0195) : 0.0254) * ((glu ? 32 : 16) + (size == 2 ? 1.33 : glu ? 0.73 : 0.87) * M) * covered * tw_div_up(groups, 256);
+  const double cu = 1e-3 * (size == 2 ? (glu ? 0.0187 : 0.0195) : 0.0254) * ((pairs ? 32 : 16) + narrow_row_share(epf, glu) * M) * covered * tw_div_up(groups, 256);
   const double memory = 1e-6 * N * (double)K * size / (size == 2 ? 6.57 : 6.14);
   return (size == 2 ? (glu ? 2.66 : 2.80) : glu ? 2.81 : 2.97) + sqrt(sqrt(cu * cu * cu * cu + memory * memory * memory * memory));
 }
@@ -1082,7 +1109,8 @@ static bool narrow_pays(int M, int N, int K, int epf, bool glu, bool sums) {
   if (groups <= 256 ? steps <= (M > 8 && groups < 96 && !glu ? 96 : 128)
       : glu ? steps >= 28 && steps <= (groups < 512 && epf == 4 ? 32 : 64) && (M <= 8 || groups >= 512)
             : groups <= 512 && steps >= 16 && steps <= 64) return true;
-  const bool beyond = groups >= 576 || steps > (groups <= 256 ? 144 : 72);      // (by an eighth: what lies at the lines stays where it is)
+  // (by an eighth: what lies at the lines stays where it is; float32's are those of pairs, halves are estimated from workgroups of eight waves on)
+  const bool beyond = groups >= 576 || steps > (groups <= 256 ? 144 : 72) || (glu && epf == 4 && steps > 48 && narrow_halves(M, N, K, epf));
   return beyond && steps >= 28 && narrow_us(M, N, K, epf, glu) < (epf == 4 ? 0.93 : 0.9) * skinny_us(M, N, K, epf, glu);
 }
 
@@ -1109,14 +1137,22 @@ static bool narrow_act_pays(int M, int N, int K, int epf) {
 template <typename T, typename OutT, bool GLU, bool ACT = false, class In = RowsAsTheyAre, class End = EndPlain>
 static int launch_narrow(const T* A, long lda, const T* W, long ldw, const float* bias, const float* residual, long ldr,
                          OutT* C, long ldc, int M, int N, int K, hipStream_t stream, In norms = In{}, End end = End{}) {
-  const int steps = tw_div_up(K / Elem<T>::kPerFrag, 4), groups = GLU ? N / 32 : tw_div_up(N, 16);
-  if (steps <= 48)
-    gemm_narrow_kernel<T, OutT, 4, GLU, ACT, In, End><<<groups, 256, 0, stream>>>(A, lda, W, ldw, bias, residual, ldr, C, ldc, M, N, K, norms, end);
-  else if (steps <= 96)
-    gemm_narrow_kernel<T, OutT, 8, GLU, ACT, In, End><<<groups, 512, 0, stream>>>(A, lda, W, ldw, bias, residual, ldr, C, ldc, M, N, K, norms, end);
-  else
-    gemm_narrow_kernel<T, OutT, 16, GLU, ACT, In, End><<<groups, 1024, 0, stream>>>(A, lda, W, ldw, bias, residual, ldr, C, ldc, M, N, K, norms, end);
-  return TW_LAUNCH_RESULT();
+  const int steps = tw_div_up(K / Elem<T>::kPerFrag, 4);
+  auto run = [&](auto halves) {
+    constexpr bool H = decltype(halves)::value;
+    const int groups = GLU && !H ? N / 32 : tw_div_up(N, 16);
+    if (steps <= 48)
+      gemm_narrow_kernel<T, OutT, 4, GLU, ACT, In, End, H><<<groups, 256, 0, stream>>>(A, lda, W, ldw, bias, residual, ldr, C, ldc, M, N, K, norms, end);
+    else if (steps <= 96)
+      gemm_narrow_kernel<T, OutT, 8, GLU, ACT, In, End, H><<<groups, 512, 0, stream>>>(A, lda, W, ldw, bias, residual, ldr, C, ldc, M, N, K, norms, end);
+    else
+      gemm_narrow_kernel<T, OutT, 16, GLU, ACT, In, End, H><<<groups, 1024, 0, stream>>>(A, lda, W, ldw, bias, residual, ldr, C, ldc, M, N, K, norms, end);
+    return TW_LAUNCH_RESULT();
+  };
+  if constexpr (GLU) {
+    if (narrow_halves(M, N, K, Elem<T>::kPerFrag)) return run(std::true_type{});
+  }
+  return run(std::false_type{});
 }
 
 // force: 0 = choose, 1 = generic, 3 = tiled 128x128, 4 = tiled 128x256, 5 = skinny, 6 = tiled 256x256,

@@ -786,6 +786,25 @@ def test_linear_of_few_rows_over_whole_k(ops, device, dtype, m, n, k):
         torch.testing.assert_close(out.double().cpu(), g * torch.sigmoid(g) * u, atol=bound, rtol=1e-5 if dtype == torch.float32 else 2.0 ** -7)
 
 
+# eight gate and eight up rows a workgroup, or 16 of either: one workgroup a CU at most, one more, the second round of pairs' first, K of
+# four, eight and sixteen waves and ragged; rows on either side
+@pytest.mark.parametrize("m,n,k", [(1, 32, 64), (16, 96, 72), (7, 4096, 1024), (7, 4128, 520), (3, 8192, 512), (3, 8224, 2016), (3, 8224, 2048), (8, 9728, 896),
+                                   (16, 11264, 2048), (8, 11264, 2056), (2, 2048, 4096)])
+@pytest.mark.parametrize("dtype", DTYPES)
+def test_linear_glu_of_few_rows_in_halves(ops, device, dtype, m, n, k):
+    x, w = rand((m, k), dtype, device, 1.0, seed=1), rand((n, k), dtype, device, k ** -0.5, seed=2)
+    bias = rand((n,), torch.float32, device, 0.5, seed=3)
+    sums = (x.double() @ w.double().T + bias.double()).view(m, n // 32, 2, 16)
+    gate, up = sums[:, :, 0].reshape(m, -1), sums[:, :, 1].reshape(m, -1)
+    want = gate * torch.sigmoid(gate) * up
+    # float32 sums of unit size are off by less than 2^-18 (K up to 4,096), silu's slope is below 1.1; bfloat16 rounds once more
+    bound = 2.0 ** -18 * (1.1 * up.abs() + gate.abs() + 1) + (2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -20) * want.abs()
+    for force in (ops.GEMM_AUTO, ops.GEMM_NARROW):
+        wide = torch.full((m, n // 2 + 8), float("nan"), dtype=dtype, device=device)
+        ops.linear_glu(x, ops.shuffle_weight(w), wide[:, :n // 2], bias=bias, force=force)
+        assert ((wide[:, :n // 2].double() - want).abs() <= bound).all() and wide[:, n // 2:].isnan().all()
+
+
 @pytest.mark.parametrize("m,n,k", [(1024, 3584, 16384), (1100, 3000, 12288), (2048, 3584, 8192)])
 def test_linear_large_tiles_over_k_ranges(ops, device, m, n, k):
     """Many rows, few columns, long K (a down projection): the chosen plan may be 256x256 tiles whose K is
