@@ -44,6 +44,7 @@ struct RowNorms {
   float width, eps;
 };
 struct RowsAsTheyAre {};
+struct RowsRounded {};        // A holds float32 rows, rounded to the product's type as they are read
 #define TW_NORM_MAX_SUMS 256
 
 // THREADS / 16 lanes a row add its sums up: `request` asks for all of them (clamped, so that no load has a predicate), `finish`
@@ -592,6 +593,17 @@ struct EndRotate {
   void *keys, *values;
   int q_heads, kv_heads, head_dim, rot, page_size, write_cache, adjacent;
 };
+// EndTokenGate  C = gelu_tanh(sum + bias) * table[token of the row][offset + column], as token_gate_kernel: with rows rounded as they are read the
+//              launches in front of and behind a layer's small product from the stream to its token input go (128 x 2048, one row, in captured
+//              steps: 3.5 us a layer).
+template <typename T>
+struct EndTokenGate {
+  const T* table; long ld;
+  const int *ids, *feed;
+  int n_feed, vocab, offset;
+};
+template <class End> struct IsTokenGate { static constexpr bool value = false; };
+template <typename T> struct IsTokenGate<EndTokenGate<T>> { static constexpr bool value = true; };
 template <class End> struct IsLeave { static constexpr bool value = false, after = false; };
 template <bool A> struct IsLeave<EndLeave<A>> { static constexpr bool value = true, after = A; };
 
@@ -603,7 +615,8 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_narrow_kernel(const T* __rest
                                                                  int M, int N, int K, In norms, End end) {
   typedef typename Elem<T>::Frag Frag;
   constexpr bool NORMED = std::is_same<In, RowNorms>::value, ROTATE = std::is_same<End, EndRotate>::value;
-  constexpr bool LEAVE = IsLeave<End>::value, AFTER = IsLeave<End>::after;
+  constexpr bool LEAVE = IsLeave<End>::value, AFTER = IsLeave<End>::after, TOKEN_GATE = IsTokenGate<End>::value;
+  constexpr bool ROUND = std::is_same<In, RowsRounded>::value;
   static_assert(!(GATED && (ROTATE || LEAVE)) && (GATED || !HALVES), "the gated form finishes plain outputs");
   constexpr bool GLU = GATED && !HALVES;
   constexpr int EPF = Elem<T>::kPerFrag, U = 4, NT = GLU ? 2 : 1;
@@ -637,7 +650,8 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_narrow_kernel(const T* __rest
     w_base = W + ((size_t)(n >> 4) * ldw * 64 + g * 16 + (n & 15)) * EPF;
   }
   const size_t w_tile = (size_t)ldw * 64 * EPF;
-  const T* x_base = A + (size_t)min(r, M - 1) * lda;                            // (rows past M: never stored)
+  const T* x_base = A + (size_t)min(r, M - 1) * (ROUND ? 0 : lda);               // (rows past M: never stored)
+  const float* x_wide = reinterpret_cast<const float*>(A) + (size_t)min(r, M - 1) * lda;     // (ROUND)
 
   RowNormLoads<WAVES * 64> norm_sums, before_sums;
   if constexpr (NORMED) norm_sums.request(norms, M);
@@ -646,7 +660,9 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_narrow_kernel(const T* __rest
   }
   // Loads carry no predicate: steps are clamped to the last one and chunks to the last chunk, and activations
   // past either are replaced by zeros before the product.
-  Frag wf[2][NT][U], xf[2][U];
+  struct Wide { f32x4 part[EPF / 4]; };
+  std::conditional_t<ROUND, Wide, Frag> xf[2][U];
+  Frag wf[2][NT][U];
   auto load = [&](const int buf, int i0) {
 #pragma unroll
     for (int u = 0; u < U; ++u) {
@@ -654,7 +670,23 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_narrow_kernel(const T* __rest
 #pragma unroll
       for (int t = 0; t < NT; ++t)
         wf[buf][t][u] = tw_load_frag_stream(w_base + t * w_tile + (size_t)min(s, steps - 1) * 64 * EPF);
-      xf[buf][u] = tw_load_frag(x_base + (size_t)min(s * 4 + g, chunks - 1) * EPF);
+      const size_t at = (size_t)min(s * 4 + g, chunks - 1) * EPF;
+      if constexpr (ROUND) {
+#pragma unroll
+        for (int i = 0; i < EPF / 4; ++i) xf[buf][u].part[i] = *reinterpret_cast<const f32x4*>(x_wide + at + 4 * i);
+      } else {
+        xf[buf][u] = tw_load_frag(x_base + at);
+      }
+    }
+  };
+  auto fragment = [&](const int buf, int u) {
+    if constexpr (ROUND) {
+      Frag f;
+#pragma unroll
+      for (int i = 0; i < EPF; ++i) f[i] = tw_from_float<T>(xf[buf][u].part[i / 4][i % 4]);
+      return f;
+    } else {
+      return xf[buf][u];
     }
   };
   f32x4 acc[NT];
@@ -664,7 +696,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_narrow_kernel(const T* __rest
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       const int s = wave + (i0 + u) * WAVES;
-      const Frag x = s * 4 + g < chunks ? xf[buf][u] : Elem<T>::zero();
+      const Frag x = s * 4 + g < chunks ? fragment(buf, u) : Elem<T>::zero();
 #pragma unroll
       for (int t = 0; t < NT; ++t) tw_mma16(acc[t], wf[buf][t][u], x);
     }
@@ -687,6 +719,15 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_narrow_kernel(const T* __rest
         if (end.before.sums) before_weight = end.before_weight[col];
         if (end.scale) scale = end.scale[col];
       }
+    }
+  }
+  float token_value = 0.f;
+  if constexpr (TOKEN_GATE) {
+    if (store) {
+      int id = end.ids[row];
+      if (id < 0) id = (end.feed && -1 - id < end.n_feed) ? end.feed[-1 - id] : 0;
+      id = id < 0 ? 0 : (id >= end.vocab ? end.vocab - 1 : id);
+      token_value = tw_to_float(end.table[(size_t)id * end.ld + end.offset + col]);
     }
   }
   float turn_cos = 1.f, turn_sin = 0.f;
@@ -775,6 +816,8 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_narrow_kernel(const T* __rest
       else
         static_cast<T*>(end.values)[((page * end.kv_heads + kh) * end.head_dim + d) * end.page_size + off] = out;
     }
+  } else if constexpr (TOKEN_GATE) {
+    C[(size_t)row * ldc + col] = tw_from_float<OutT>(tw_gelu_tanh(v[0]) * token_value);
   } else {
     if constexpr (ACT) v[0] = tw_act(v[0], ldr);
     else if (residual) v[0] += res;
@@ -1436,6 +1479,24 @@ extern "C" int tw_linear_leave(int dtype, const void* A, long lda, const void* W
   const EndLeave<false> without = {weight, weight2, rows, rows2, sums, before, nullptr, nullptr, 1.f};
   if (dtype == TW_DTYPE_F32) return after ? run(float{}, with) : run(float{}, without);
   return after ? run(bf16_t{}, with) : run(bf16_t{}, without);
+}
+
+// C [M][N] (the weight's type) = gelu_tanh(round(A) W^T + bias) * table[token of the row][offset ..] for float32 rows A of the stream; tokens as
+// tw_token_gate. Where the product alone takes the kernel with the whole of K a workgroup.
+extern "C" int tw_linear_token_gate_pays(int dtype, int M, int N, int K) {
+  const int epf = dtype == TW_DTYPE_F32 ? 4 : 8;
+  return M >= 1 && M <= 16 && N > 0 && K > 0 && K % epf == 0 && narrow_pays(M, N, K, epf, false, false) ? 1 : 0;
+}
+extern "C" int tw_linear_token_gate(int dtype, const float* A, long lda, const void* W, long ldw, const float* bias, void* C, long ldc, int M,
+                                    int N, int K, const void* table, long ld_table, const int* ids, const int* feed, int n_feed, int vocab,
+                                    int offset, hipStream_t stream) {
+  TW_REQUIRE(few_rows_ok(dtype, A, lda, W, ldw, M, N, K) && lda % 4 == 0 && C != nullptr && ldc >= N);
+  TW_REQUIRE(table && ids && vocab > 0 && offset >= 0 && offset + N <= ld_table);
+  if (dtype == TW_DTYPE_F32)
+    return launch_narrow<float, float, false>(A, lda, (const float*)W, ldw, bias, nullptr, 0, (float*)C, ldc, M, N, K, stream, RowsAsTheyAre{},
+                                              EndTokenGate<float>{(const float*)table, ld_table, ids, feed, n_feed, vocab, offset});
+  return launch_narrow<bf16_t, bf16_t, false>((const bf16_t*)A, lda, (const bf16_t*)W, ldw, bias, nullptr, 0, (bf16_t*)C, ldc, M, N, K, stream, RowsRounded{},
+                                              EndTokenGate<bf16_t>{(const bf16_t*)table, ld_table, ids, feed, n_feed, vocab, offset});
 }
 
 extern "C" int tw_linear_rotate_pays(int dtype, int M, int N, int K) {

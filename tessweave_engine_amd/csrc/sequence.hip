@@ -11,10 +11,6 @@
 #include "rope_tables.h"
 #include <type_traits>
 
-__device__ __forceinline__ float tw_gelu_tanh(float z) {
-  return 0.5f * z * (1.f + tanhf(0.7978845608028654f * (z + 0.044715f * z * z * z)));
-}
-
 __device__ __forceinline__ float tw_sigmoid(float z) { return 1.f / (1.f + expf(-z)); }
 
 // The sequence that owns token row `row` (q_start is ascending, q_start[n_seqs] = n_tokens).

@@ -231,6 +231,10 @@ __device__ __forceinline__ float tw_block_sum(float v, float* lds /* 16 floats *
   return total;
 }
 
+__device__ __forceinline__ float tw_gelu_tanh(float z) {
+  return 0.5f * z * (1.f + tanhf(0.7978845608028654f * (z + 0.044715f * z * z * z)));
+}
+
 static inline int tw_div_up(long a, long b) { return (int)((a + b - 1) / b); }
 
 #define TW_REQUIRE(cond)                      \

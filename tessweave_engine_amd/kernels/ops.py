@@ -554,6 +554,30 @@ def linear_leave(x, weight, stream, norm_weight, eps, rows, sums, bias=None, sec
     return NormedRows(rows, sums, eps, second=NormedRows(second[1], sums, eps) if second is not None else None)
 
 
+def linear_token_gate_pays(x, weight):
+    """Is `linear_token_gate` there for these float32 rows, and no slower a product than `linear`?"""
+    return (_few_rows_of_shuffled(x, weight) and weight.shape[1] % (16 // weight.dtype.itemsize) == 0
+            and (x.stride(0) if x.shape[0] > 1 else x.shape[1]) % (16 // weight.dtype.itemsize) == 0
+            and bool(library().tw_linear_token_gate_pays(dtype_id(weight.dtype), x.shape[0], *weight.shape)))
+
+
+def linear_token_gate(x, weight, table, ids, offset, out, feed=None, bias=None):
+    """out[n, c] = gelu_tanh(x rounded to the weight's type @ weight.T (+ bias)) * table[ids[n], offset + c]: `round_rows`, `linear` into
+    float32 and `token_gate` for up to 16 float32 rows in one kernel."""
+    m, k, lda = _rows(x, "x")
+    n, k2, w_ptr, ldw, shuffled, w_dtype = _weight_args(weight)
+    mo, no, ldo = _rows(out, "out")
+    _need(x.dtype == torch.float32 and k == k2 and shuffled and w_dtype == table.dtype == out.dtype and (mo, no) == (m, n) and ids.numel() >= m,
+          "linear_token_gate shapes do not agree")
+    _need(table.dim() == 2 and table.is_contiguous() and 0 <= offset and offset + n <= table.shape[1], "the table must be contiguous and hold the asked columns")
+    _need(bias is None or (bias.numel() == n and bias.is_contiguous()), "bias has the wrong size")
+    check(library().tw_linear_token_gate(
+        dtype_id(w_dtype), _dev(x), lda, w_ptr, ldw, _dev(bias, torch.float32, "bias") if bias is not None else None, _dev(out), ldo, m, n, k,
+        _dev(table), table.shape[1], _dev(ids, torch.int32, "ids"), _dev(feed, torch.int32, "feed") if feed is not None else None,
+        feed.numel() if feed is not None else 0, table.shape[0], int(offset), _stream()), "linear_token_gate")
+    return out
+
+
 def linear_rotate_pays(x, weight, rot):
     """Is `linear_rotate` there for these operands, and faster than split-K sums that `rope_kv_write` finishes?"""
     rows = x.rows if isinstance(x, NormedRows) else x

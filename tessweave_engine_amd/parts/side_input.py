@@ -62,12 +62,15 @@ class TokenSideInput(Part):
     def forward(self, ctx, x):
         """y float32 [n, hidden] for the residual stream x; the caller norms and adds it."""
         n = x.shape[0]
+        g = ctx.scratch("side.g", (n, self.dim))
+        y = ctx.scratch("side.y", (n, self.hidden), torch.float32)
+        gate, bias = self.gate.weights[0], self.gate.biases[0] if self.gate.biases else None
+        if ops.linear_token_gate_pays(x, gate):
+            ops.linear_token_gate(x, gate, self.table.weight, ctx.token_ids, self.layer * self.dim, g, feed=ctx.token_feed, bias=bias)
+            return self.proj.forward(ctx, g, y)
         rounded = ctx.scratch("side.x", (n, self.hidden))
         ops.round_rows(x, rounded)
         pre = ctx.scratch("side.pre", (n, self.dim), torch.float32)
         self.gate.forward(ctx, rounded, pre)
-        g = ctx.scratch("side.g", (n, self.dim))
         ops.token_gate(pre, self.table.weight, ctx.token_ids, self.layer * self.dim, g, feed=ctx.token_feed)
-        y = ctx.scratch("side.y", (n, self.hidden), torch.float32)
-        self.proj.forward(ctx, g, y)
-        return y
+        return self.proj.forward(ctx, g, y)

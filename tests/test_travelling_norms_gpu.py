@@ -210,3 +210,22 @@ def test_experts_sums_behind_a_norm(ops, device, dtype, n, c, top, splits):
     ops.moe_experts(out, ids, weights, gate, up, down, 0.0, x, scratch, kind="silu", more=more, norm=(norm, 1e-6, out))
     assert torch.equal(x, want)
     torch.testing.assert_close(out.float(), wanted.float(), atol=0, rtol=2.0 ** -7 if dtype == torch.bfloat16 else 1e-6)     # (a last place: sums in another order)
+
+
+# rows, columns, K: one and all rows of a tile, ragged columns, K of four, eight and sixteen waves, and ragged
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("m,n,k,with_bias", [(1, 128, 2048, False), (16, 64, 256, True), (5, 24, 1032, True), (9, 256, 4096, False), (2, 16, 3072, True)])
+def test_product_gated_by_tokens(ops, device, dtype, m, n, k, with_bias):
+    """The same bits as the three kernels it stands for; token ids past the table, fed ones and fed ones past the feed."""
+    x, weight = rand((m, k + 8), torch.float32, device)[:, :k], ops.shuffle_weight(rand((n, k), dtype, device, k ** -0.5, 1))
+    table, bias = rand((37, 3 * n), dtype, device, 1.0, 2), rand((n,), torch.float32, device, 0.1, 3) if with_bias else None
+    ids = torch.tensor([5, -1, 36, 99, -3, -7, 0, 12, 12, 1, 2, 3, 4, -2, 6, 7][:m], dtype=torch.int32, device=device)
+    feed = torch.tensor([11, 36, 50], dtype=torch.int32, device=device)
+    rounded, pre, want = torch.empty(m, k, dtype=dtype, device=device), torch.empty(m, n, device=device), torch.empty(m, n, dtype=dtype, device=device)
+    ops.round_rows(x.contiguous(), rounded)
+    ops.linear(rounded, weight, pre, bias=bias, force=ops.GEMM_NARROW)
+    for offset, fed in ((0, feed), (2 * n, None)):
+        ops.token_gate(pre, table, ids, offset, want, feed=fed)
+        wide = torch.full((m, n + 8), float("nan"), dtype=dtype, device=device)
+        got = ops.linear_token_gate(x, weight, table, ids, offset, wide[:, :n], feed=fed, bias=bias)
+        assert torch.equal(got, want) and wide[:, n:].isnan().all()
