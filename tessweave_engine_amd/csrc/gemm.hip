@@ -572,7 +572,8 @@ __global__ __launch_bounds__(TW_CU_WAVES * 64) void gemm_stream_cu_kernel(
 //   EndLeave   C (float32, the residual stream) = sum + bias + residual, and beside it what a norm that travels needs: the rows times
 //              the next norm's weight in T (times a second weight too where two norms read the stream), and each 16 columns' sum of
 //              squares. AFTER: the stream itself is such a normed row, C = alpha * residual * rinv * before_weight + scale * (sum + bias).
-//   EndRotate  the packed product of queries, keys and values: q and k are rotated, q goes to C, k and v to the cache's pages. A
+//   EndRotate  the packed product of queries, keys and values: q and k are rotated, q goes to C, k and v to the cache's pages, and what lies behind
+//              them (another mixer's columns) to C. A
 //              workgroup's 16 columns are then eight of a head's first rotated half and the eight they turn with (each eight weight
 //              rows of a fragment are a cache line, so the loads are as wide as before), so that no other kernel has to bring the
 //              two halves together: it was 2.5 to 4 us behind every such product.
@@ -806,7 +807,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_narrow_kernel(const T* __rest
       out = tw_from_float<T>(high ? b : a);
     }
     const int head = blockIdx.x / (end.head_dim / 16), d = col - head * end.head_dim;
-    if (head < end.q_heads) {
+    if (head < end.q_heads || head >= end.q_heads + 2 * end.kv_heads) {
       C[(size_t)row * ldc + col] = out;
     } else if (slot >= 0) {
       const size_t page = slot / end.page_size;
@@ -1506,13 +1507,14 @@ extern "C" int tw_linear_rotate_pays(int dtype, int M, int N, int K) {
 
 // The packed product of queries, keys and values of up to 16 rows, finished as tw_rope_kv_write finishes it: qkv [M][ld] = round(A W^T +
 // bias), q rotated in place; rotated k and v to the pages of the rows' slots (write_cache; the k and v columns of qkv are not written).
-// sums: null, or the rows' norms as tw_linear_normed. rot: a multiple of 16.
+// sums: null, or the rows' norms as tw_linear_normed. rot: a multiple of 16. behind: columns of the product behind the values (a multiple of 16),
+// which stay as they are.
 extern "C" int tw_linear_rotate(int dtype, const void* A, long lda, const float* sums, int count, int width, float eps, const void* W, long ldw,
                                 const float* bias, void* qkv, long ld, int M, int K, const float* cos_t, const float* sin_t, const int* slots,
                                 void* keys, void* values, int q_heads, int kv_heads, int head_dim, int rot, int page_size, int write_cache,
-                                int adjacent, hipStream_t stream) {
-  TW_REQUIRE(q_heads > 0 && kv_heads > 0 && head_dim > 0 && head_dim % 16 == 0 && page_size > 0);
-  const int N = (q_heads + 2 * kv_heads) * head_dim;
+                                int adjacent, int behind, hipStream_t stream) {
+  TW_REQUIRE(q_heads > 0 && kv_heads > 0 && head_dim > 0 && head_dim % 16 == 0 && page_size > 0 && behind >= 0 && behind % 16 == 0);
+  const int N = (q_heads + 2 * kv_heads) * head_dim + behind;
   TW_REQUIRE(few_rows_ok(dtype, A, lda, W, ldw, M, N, K) && qkv != nullptr && ld >= N && rot >= 0 && rot % 16 == 0 && rot <= head_dim);
   TW_REQUIRE(rot == 0 || (cos_t && sin_t));
   TW_REQUIRE(!write_cache || (slots && keys && values));

@@ -52,7 +52,7 @@ _SIGNATURES = {
     "tw_linear_token_gate_pays": (I, [I, I, I, I]),
     "tw_linear_token_gate": (I, [I, P, L, P, L, P, P, L, I, I, I, P, L, P, P, I, I, I, P]),
     "tw_linear_rotate_pays": (I, [I, I, I, I]),
-    "tw_linear_rotate": (I, [I, P, L, P, I, I, F, P, L, P, P, L, I, I, P, P, P, P, P, I, I, I, I, I, I, I, P]),
+    "tw_linear_rotate": (I, [I, P, L, P, I, I, F, P, L, P, P, L, I, I, P, P, P, P, P, I, I, I, I, I, I, I, I, P]),
     "tw_attn_decode_splits": (I, [I, I, I, I, I, I]),
     "tw_attn_decode_most_splits": (I, [I, I, I, I, I, I, I]),
     "tw_attn_decode_workspace_floats": (L, [I, I, I, I]),

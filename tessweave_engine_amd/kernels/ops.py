@@ -587,13 +587,15 @@ def linear_rotate_pays(x, weight, rot):
 
 def linear_rotate(x, weight, qkv, cos, sin, slots, keys, values, q_heads, kv_heads, head_dim, page_size, write_cache=True, bias=None, adjacent=False):
     """The packed product of queries, keys and values of up to 16 rows (`NormedRows` or plain ones), with what `rope_kv_write` does behind it
-    in its epilogue: the q columns of qkv are written rotated, k and v go to the pages only."""
+    in its epilogue: the q columns of qkv are written rotated, k and v go to the pages only. cos, sin may be None (nothing turns), and further
+    columns may lie behind the values (a multiple of 16), which are written as they are."""
     rows = x.rows if isinstance(x, NormedRows) else x
     m, k, lda = _rows(rows, "x")
     n, k2, w_ptr, ldw, shuffled, w_dtype = _weight_args(weight)
     mo, no, ld = _rows(qkv, "qkv")
     _need(k == k2 and shuffled and rows.dtype == w_dtype == qkv.dtype and (mo, no) == (m, n) and m <= 16, "linear_rotate takes up to 16 rows of a shuffled weight's type")
-    _need(n == (q_heads + 2 * kv_heads) * head_dim and head_dim % 16 == 0, "qkv width does not match the head counts")
+    behind = n - (q_heads + 2 * kv_heads) * head_dim
+    _need(behind >= 0 and behind % 16 == 0 and head_dim % 16 == 0, "qkv width does not match the head counts")
     half = cos.shape[1] if cos is not None else 0
     _need(2 * half <= head_dim and half % 8 == 0, "linear_rotate turns multiples of 16 elements of a head")
     if half:
@@ -609,7 +611,7 @@ def linear_rotate(x, weight, qkv, cos, sin, slots, keys, values, q_heads, kv_hea
         dtype_id(w_dtype), _dev(rows), lda, *norms, w_ptr, ldw, _dev(bias, f32, "bias") if bias is not None else None, _dev(qkv), ld, m, k,
         _dev(cos, f32, "cos") if half else None, _dev(sin, f32, "sin") if half else None, _dev(slots, torch.int32, "slots") if write_cache else None,
         _dev(keys) if write_cache else None, _dev(values) if write_cache else None, q_heads, kv_heads, head_dim, 2 * half, page_size,
-        1 if write_cache else 0, 1 if adjacent else 0, _stream()), "linear_rotate")
+        1 if write_cache else 0, 1 if adjacent else 0, behind, _stream()), "linear_rotate")
     return qkv
 
 

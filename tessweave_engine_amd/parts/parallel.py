@@ -43,8 +43,15 @@ class MixerBranch(Part):
     takes_partials: proj may also be float32 [splits, n, columns] split-K sums of the product (a view into those of all
     branches), which the branch adds up itself, with `bias` (float32 [columns], or None) then given apart. (Without, a
     bias is in proj already, and `bias` is not given.)
+
+    stores(ctx, run): None, or (queries' heads, key and value heads, head size, keys, values, slots) where the branch's columns begin with
+    those of queries, keys and values and the latter two are wanted in the pages alone, as they are: the product may then write
+    them there, and `stored=True` tells the branch so.
     """
     takes_partials = False
+
+    def stores(self, ctx, run):
+        return None
 
     def in_matrices(self):
         raise NotImplementedError
@@ -115,12 +122,18 @@ class MixedHeadAttention(MixerBranch):
     def cache_need(self):
         return CacheNeed(paged=PagedKV(self.kv_heads, self.key_dev, self.window, self.value_dev))
 
-    def forward(self, ctx, run, proj, out, scale):
+    def stores(self, ctx, run):
+        if not run.writes_cache or self.key_dev != self.value_dev:
+            return None
+        keys, values, g = ctx.cache.keys_values(run.cache_slot)
+        return self.q_heads, self.kv_heads, self.key_dev, keys, values, ctx.groups[g].slot_mapping
+
+    def forward(self, ctx, run, proj, out, scale, stored=False):
         H, G, D, E = self.q_heads, self.kv_heads, self.key_dev, self.value_dev
         keys, values, g = ctx.cache.keys_values(run.cache_slot)
         values = values.view(values.shape[0], G, E, ctx.cache.page_size)
         group = ctx.groups[g]
-        if run.writes_cache:
+        if run.writes_cache and not stored:
             ops.kv_store(proj, H * D, (H + G) * D, group.slot_mapping, keys, values, G, D, E)
         window = self.window or 0
         common = dict(window=window, talk=self.talk, sink=self.sink, slopes=self.slopes, out_scale=scale)
@@ -295,8 +308,15 @@ class ParallelMixer(Mixer):
             extra = [dict(bias=bias[c0:c0 + w] if bias is not None else None) for c0, w in self.in_columns]
         else:
             proj = ctx.scratch("parallel.proj", (n, sum(self.proj.device_out)), self.proj_dtype)
-            self.proj.forward(ctx, h, proj)
             extra = [{} for _ in self.branches]
+            stores = self.branches[0].stores(ctx, run) if n <= 16 and proj.dtype == h.dtype and self.proj.takes_normed else None
+            if stores is not None and ops.linear_rotate_pays(h, self.proj.weights[0], 0):
+                q_heads, kv_heads, size, keys, values, slots = stores
+                ops.linear_rotate(h, self.proj.weights[0], proj, None, None, slots, keys, values, q_heads, kv_heads, size, ctx.cache.page_size,
+                                  bias=self.proj.biases[0] if self.proj.biases else None)
+                extra[0]["stored"] = True
+            else:
+                self.proj.forward(ctx, h, proj)
         for b, (c0, w), (o0, ow), scale, more in zip(self.branches, self.in_columns, self.out_columns, self.scales, extra):
             b.forward(ctx, run, proj[..., c0:c0 + w], joined[:, o0:o0 + ow], scale, **more)
 

@@ -229,3 +229,22 @@ def test_product_gated_by_tokens(ops, device, dtype, m, n, k, with_bias):
         wide = torch.full((m, n + 8), float("nan"), dtype=dtype, device=device)
         got = ops.linear_token_gate(x, weight, table, ids, offset, wide[:, :n], feed=fed, bias=bias)
         assert torch.equal(got, want) and wide[:, n:].isnan().all()
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("m,q_heads,kv_heads,dim,behind,k", [(1, 16, 4, 128, 4096, 2048), (16, 3, 1, 16, 16, 72), (5, 2, 2, 48, 144, 3000)])
+def test_product_that_fills_the_cache_with_columns_behind(ops, device, dtype, m, q_heads, kv_heads, dim, behind, k):
+    """Against the same product, then `kv_store`: the same bits."""
+    width, page = (q_heads + 2 * kv_heads) * dim + behind, 16
+    x, w, bias = rand((m, k), dtype, device), ops.shuffle_weight(rand((width, k), dtype, device, k ** -0.5, 1)), rand((width,), torch.float32, device, 0.1, 2)
+    slots = torch.tensor([(5 * i + 3) % (4 * page) if i != 4 else -1 for i in range(m)], dtype=torch.int32, device=device)
+    keys = torch.full((4, kv_heads, page, dim), -9.0, dtype=dtype, device=device)
+    values = torch.full((4, kv_heads, dim, page), -9.0, dtype=dtype, device=device)
+    want, want_keys, want_values = torch.empty(m, width, dtype=dtype, device=device), keys.clone(), values.clone()
+    ops.linear(x, w, want, bias=bias, force=ops.GEMM_NARROW)
+    ops.kv_store(want, q_heads * dim, (q_heads + kv_heads) * dim, slots, want_keys, want_values, kv_heads, dim, dim)
+    out = torch.full((m, width + 8), -9.0, dtype=dtype, device=device)
+    ops.linear_rotate(x, w, out[:, :width], None, None, slots, keys, values, q_heads, kv_heads, dim, page, bias=bias)
+    assert torch.equal(keys, want_keys) and torch.equal(values, want_values)
+    q, kv = q_heads * dim, (q_heads + 2 * kv_heads) * dim
+    assert torch.equal(out[:, :q], want[:, :q]) and torch.equal(out[:, kv:width], want[:, kv:]) and (out[:, width:] == -9).all()
