@@ -8,6 +8,14 @@
 // Also here: the square of relu, in place, for a feed-forward without a gate.
 #include "tw_common.h"
 
+// The rows a kernel has just written to the stream, behind the one RMS norm that reads them next as well (a model's last: its own launch in a
+// captured step, 3 us): out[n] = v / sqrt(mean(v^2) + eps) * w. w null: no such norm.
+struct NextNorm {
+  const float* w;
+  void* out;
+  float eps;
+};
+
 struct ResidualNormArgs {
   float* x;                 // [n][hidden]
   const float* y; long ldy; // [n][ldy] or null
@@ -18,6 +26,7 @@ struct ResidualNormArgs {
   int hidden;
   float alpha, eps;
   const float* before;      // [hidden] or null: x stands for before * unit(x) (few rows: the kernel of four consecutive elements)
+  NextNorm next;                         // (rows of whole groups of four alone)
 };
 
 // Four columns of split-K partial sums, `stride` apart, requested up to eight at a time and added in index order. (Four, two and
@@ -79,6 +88,26 @@ __device__ __forceinline__ void sub_store4(T* dst, f32x4 r, bool whole) {
 template <typename T>
 __device__ __forceinline__ bool sub_whole4(const void* out) { return (uintptr_t)out % (4 * sizeof(T)) == 0; }
 
+template <typename T, int PER>
+__device__ __forceinline__ void sub_next_norm(const NextNorm& next, const f32x4 (&v)[PER], int hidden, float* lds) {
+  const int chunks = hidden / 4;
+  f32x4 wv[PER];
+  float ss = 0.f;
+#pragma unroll
+  for (int i = 0; i < PER; ++i) {
+    const int c = threadIdx.x + i * blockDim.x;
+    wv[i] = *reinterpret_cast<const f32x4*>(next.w + 4 * min(c, chunks - 1));
+    if (c < chunks) ss += ((v[i][0] * v[i][0] + v[i][1] * v[i][1]) + v[i][2] * v[i][2]) + v[i][3] * v[i][3];
+  }
+  const float scale = 1.0f / sqrtf(tw_block_sum(ss, lds) / (float)hidden + next.eps);
+#pragma unroll
+  for (int i = 0; i < PER; ++i) {
+    const int c = threadIdx.x + i * blockDim.x;
+    if (c < chunks) sub_store4((T*)next.out + (size_t)blockIdx.x * hidden + 4 * c, v[i] * scale * wv[i], sub_whole4<T>(next.out));
+  }
+}
+static bool next_norm_ok(const NextNorm& n) { return n.w == nullptr || (n.out && n.eps > 0.f && (uintptr_t)n.w % 16 == 0); }
+
 // PER groups of four consecutive elements a thread, the row in registers between the two passes.
 template <typename T, int PER, bool EARLY>
 __global__ __launch_bounds__(1024) void residual_norm_vec4_kernel(ResidualNormArgs a) {
@@ -139,7 +168,9 @@ __global__ __launch_bounds__(1024) void residual_norm_vec4_kernel(ResidualNormAr
     for (int e = 0; e < 4; ++e) r[e] = v[i][e] * rinv * wv[i][e];
     *reinterpret_cast<f32x4*>(x + 4 * c) = r;
     if (a.out) sub_store4((T*)a.out + (size_t)row * a.hidden + 4 * c, r, sub_whole4<T>(a.out));
+    v[i] = r;
   }
+  if (a.next.w) sub_next_norm<T>(a.next, v, a.hidden, lds);
 }
 
 // Any row length: the sums are parked in x between the two passes (a thread reads back only what it wrote).
@@ -200,12 +231,14 @@ static void residual_norm_launch(const ResidualNormArgs& a, int n, hipStream_t s
 
 extern "C" int tw_residual_norm(int out_dtype, float* x, const float* y, long ldy, const float* add, int splits,
                                 long add_stride, const float* scale, const float* w, void* out, int n, int hidden,
-                                float alpha, float eps, const float* before, hipStream_t stream) {
+                                float alpha, float eps, const float* before, const float* next_w, void* next_out, float next_eps,
+                                hipStream_t stream) {
   TW_REQUIRE(x && w && n >= 0 && hidden > 0 && eps > 0.f);
   TW_REQUIRE(add == nullptr || (splits > 0 && add_stride >= (long)n * hidden));
   TW_REQUIRE(y == nullptr || ldy >= hidden);
   if (n == 0) return 0;
-  ResidualNormArgs a{x, add ? nullptr : y, ldy, add, splits, (size_t)add_stride, scale, w, out, hidden, alpha, eps, before};
+  ResidualNormArgs a{x, add ? nullptr : y, ldy, add, splits, (size_t)add_stride, scale, w, out, hidden, alpha, eps, before, {next_w, next_out, next_eps}};
+  TW_REQUIRE(next_norm_ok(a.next) && (!next_w || (residual_rows_aligned(a) && hidden <= 4 * 4096)));
   TW_REQUIRE(!before || (n <= TW_EARLY_ROWS && residual_rows_aligned(a) && (uintptr_t)before % 16 == 0 && hidden <= 4 * 4096));
   if (out_dtype == TW_DTYPE_BF16) residual_norm_launch<bf16_t>(a, n, stream);
   else if (out_dtype == TW_DTYPE_F32) residual_norm_launch<float>(a, n, stream);
@@ -270,6 +303,7 @@ struct AddNormedArgs {
   void* out;
   int hidden;
   float mult, eps;
+  NextNorm next;                         // (rows of whole groups of four alone)
 };
 
 // Four columns a thread and group, PER groups a thread, one block a row. Everything a row needs is requested before the first
@@ -313,7 +347,9 @@ __global__ __launch_bounds__(1024) void add_normed_vec4_kernel(AddNormedArgs a) 
     for (int e = 0; e < 4; ++e) r[e] = __fmaf_rn(v[i][e] * f, wv[i][e], xv[i][e]);
     *reinterpret_cast<f32x4*>(x + 4 * c) = r;
     if (a.out) sub_store4((T*)a.out + (size_t)row * a.hidden + 4 * c, r, sub_whole4<T>(a.out));
+    v[i] = r;
   }
+  if (a.next.w) sub_next_norm<T>(a.next, v, a.hidden, lds);
 }
 
 // Any row: W columns a thread and round (four where the result's rows allow: longer rows than the above and streams or weights
@@ -389,6 +425,12 @@ __global__ __launch_bounds__(1024) void add_normed_kernel(AddNormedArgs a) {
   }
 }
 
+// Whole rows in registers, groups of four?
+static bool add_normed_whole(const AddNormedArgs& a) {
+  auto ok = [](const void* p) { return (uintptr_t)p % 16 == 0; };            // (null is)
+  return a.hidden % 4 == 0 && ok(a.x) && ok(a.w) && ok(a.y) && a.ldy % 4 == 0 && ok(a.add) && a.add_stride % 4 == 0 && a.hidden <= 4 * 4096;
+}
+
 template <typename T>
 static void add_normed_launch(const AddNormedArgs& a, int n, hipStream_t stream) {
   auto ok = [](const void* p) { return (uintptr_t)p % 16 == 0; };            // (null is)
@@ -396,7 +438,7 @@ static void add_normed_launch(const AddNormedArgs& a, int n, hipStream_t stream)
   const bool whole = ok(a.x) && ok(a.w);
   // (a result that is one row is read column by column where the stream and the weight have to be, partial sums are not)
   const bool vec = a.hidden % 4 == 0 && ok(a.y) && a.ldy % 4 == 0 && ok(a.add) && a.add_stride % 4 == 0 && (whole || a.add);
-  if (vec && whole && chunks <= 4096) {
+  if (add_normed_whole(a)) {
     const int per = chunks <= 1024 ? 1 : chunks <= 2048 ? 2 : 4;
     const int threads = (tw_div_up(chunks, per) + 63) / 64 * 64;
     if (per == 1) add_normed_vec4_kernel<T, 1><<<n, threads, 0, stream>>>(a);
@@ -412,12 +454,14 @@ static void add_normed_launch(const AddNormedArgs& a, int n, hipStream_t stream)
 }
 
 extern "C" int tw_add_normed(int out_dtype, float* x, const float* y, long ldy, const float* add, int splits, long add_stride,
-                             const float* w, void* out, int n, int hidden, float mult, float eps, hipStream_t stream) {
+                             const float* w, void* out, int n, int hidden, float mult, float eps, const float* next_w, void* next_out, float next_eps,
+                             hipStream_t stream) {
   TW_REQUIRE(x && w && (y || add) && n >= 0 && hidden > 0 && eps > 0.f);
   TW_REQUIRE(add == nullptr || (splits > 0 && add_stride >= (long)n * hidden));
   TW_REQUIRE(add != nullptr || ldy >= hidden);
   if (n == 0) return 0;
-  AddNormedArgs a{x, add ? nullptr : y, ldy, add, splits, (size_t)add_stride, w, out, hidden, mult, eps};
+  AddNormedArgs a{x, add ? nullptr : y, ldy, add, splits, (size_t)add_stride, w, out, hidden, mult, eps, {next_w, next_out, next_eps}};
+  TW_REQUIRE(next_norm_ok(a.next) && (!next_w || add_normed_whole(a)));
   if (out_dtype == TW_DTYPE_BF16) add_normed_launch<bf16_t>(a, n, stream);
   else if (out_dtype == TW_DTYPE_F32) add_normed_launch<float>(a, n, stream);
   else return TW_ERR_BAD_ARGUMENT;

@@ -1077,12 +1077,28 @@ def attn_mixed(q, keys, values, block_table, q_start, kv_len, seq0, n_seqs, max_
 
 # ---- norm after the sum, relu squared, hashed pair embedding ----------------------------------------------------------
 
-def residual_norm(x, weight, eps, out=None, y=None, add=None, scale=None, alpha=1.0, before=None):
+def can_norm_next(x, *weights):
+    """Can `residual_norm` or `add_normed` of X put its new rows behind a further norm? (whole groups of four, up to 16,384 elements)"""
+    return (x.shape[1] % 4 == 0 and x.shape[1] <= 16384 and x.is_contiguous() and x.data_ptr() % 16 == 0
+            and all(w is None or w.data_ptr() % 16 == 0 for w in weights))
+
+
+def _next_norm(next_norm, x, out):
+    """Pointers and eps of next_norm = (weight, eps, rows): the new x behind that RMS norm too, in the rows' type (that of `out`, if there is one)."""
+    if next_norm is None:
+        return None, None, 0.0
+    weight, eps, rows = next_norm
+    _need(can_norm_next(x, weight) and weight.numel() == x.shape[1] and weight.is_contiguous(), "these rows cannot be normed here")
+    _need(rows.is_contiguous() and rows.shape == x.shape and (out is None or out.dtype == rows.dtype), "the normed rows must be [n, hidden], of out's type")
+    return _dev(weight, torch.float32, "weight"), _dev(rows), float(eps)
+
+
+def residual_norm(x, weight, eps, out=None, y=None, add=None, scale=None, alpha=1.0, before=None, next_norm=None):
     """x <- weight * unit(alpha * x + scale * y), unit(v) = v / sqrt(mean(v^2) + eps); x float32 [n, hidden] in place.
     before (float32 [hidden], for `can_leave_norms` rows): before * unit(x) takes the place of x.
 
     y: float32 [n, hidden] (rows may be strided), or add: float32 [splits, n, hidden] partial sums added up here;
-    scale: float32 [hidden] or None; out: the normed rows once more, rounded to its type (the compute type)."""
+    scale: float32 [hidden] or None; out: the normed rows once more, rounded to its type (the compute type). next_norm: see `_next_norm`."""
     _need(x.dim() == 2 and x.is_contiguous() and x.dtype == torch.float32, "residual_norm: x must be contiguous float32 [n, hidden]")
     n, hidden = x.shape
     _need(weight.numel() == hidden and weight.dtype == torch.float32 and weight.is_contiguous(), "the norm weight must be float32 [hidden]")
@@ -1100,7 +1116,7 @@ def residual_norm(x, weight, eps, out=None, y=None, add=None, scale=None, alpha=
         _need(scale.numel() == hidden and scale.dtype == torch.float32 and scale.is_contiguous(), "scale must be float32 [hidden]")
     if before is not None:
         _need(can_leave_norms(n, hidden) and before.numel() == hidden and before.is_contiguous(), "before must be [hidden], of rows whose norms can travel")
-    out_dtype = F32
+    out_dtype, following = F32 if next_norm is None else dtype_id(next_norm[2].dtype), _next_norm(next_norm, x, out)
     if out is not None:
         _need(out.is_contiguous() and tuple(out.shape) == (n, hidden), "out must be contiguous [n, hidden]")
         out_dtype = dtype_id(out.dtype)
@@ -1108,7 +1124,7 @@ def residual_norm(x, weight, eps, out=None, y=None, add=None, scale=None, alpha=
                                      _dev(add) if add is not None else None, splits, stride,
                                      _dev(scale) if scale is not None else None, _dev(weight),
                                      _dev(out) if out is not None else None, n, hidden, float(alpha), float(eps),
-                                     _dev(before, torch.float32, "before") if before is not None else None, _stream()),
+                                     _dev(before, torch.float32, "before") if before is not None else None, *following, _stream()),
           "residual_norm")
     return x
 
@@ -1611,11 +1627,11 @@ def moe_experts(h, ids, weights, gate, up, down, limit, x, scratch, kind="swish_
 
 # ---- a norm on a sublayer's result, output gates, convolved and normed queries and keys, the mLSTM ------------------------
 
-def add_normed(x, weight, eps, mult=1.0, y=None, add=None, out=None):
+def add_normed(x, weight, eps, mult=1.0, y=None, add=None, out=None, next_norm=None):
     """x <- x + mult * weight * unit(y), unit(v) = v / sqrt(mean(v^2) + eps); x float32 [n, hidden] in place.
 
     y: float32 [n, hidden] (rows may be strided), or add: float32 [splits, n, hidden] partial sums added up here;
-    out: the new x once more, rounded to its type (the compute type)."""
+    out: the new x once more, rounded to its type (the compute type). next_norm: see `_next_norm`."""
     _need(x.dim() == 2 and x.is_contiguous() and x.dtype == torch.float32, "add_normed: x must be contiguous float32 [n, hidden]")
     n, hidden = x.shape
     _need(weight.numel() == hidden and weight.dtype == torch.float32 and weight.is_contiguous(), "the norm weight must be float32 [hidden]")
@@ -1628,13 +1644,13 @@ def add_normed(x, weight, eps, mult=1.0, y=None, add=None, out=None):
         _need(add.dim() == 3 and add.is_contiguous() and tuple(add.shape[1:]) == (n, hidden) and add.dtype == torch.float32,
               "partial sums must be float32 [splits, n, hidden]")
         splits, stride = add.shape[0], n * hidden
-    out_dtype = F32
+    out_dtype, following = F32 if next_norm is None else dtype_id(next_norm[2].dtype), _next_norm(next_norm, x, out)
     if out is not None:
         _need(out.is_contiguous() and tuple(out.shape) == (n, hidden), "out must be contiguous [n, hidden]")
         out_dtype = dtype_id(out.dtype)
     check(library().tw_add_normed(out_dtype, _dev(x), _dev(y) if y is not None else None, ldy,
                                   _dev(add) if add is not None else None, splits, stride, _dev(weight),
-                                  _dev(out) if out is not None else None, n, hidden, float(mult), float(eps), _stream()),
+                                  _dev(out) if out is not None else None, n, hidden, float(mult), float(eps), *following, _stream()),
           "add_normed")
     return x
 

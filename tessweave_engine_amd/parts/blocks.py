@@ -51,6 +51,17 @@ def leaving(ctx, x, sublayer, entry):
         ctx.norm_ahead = None
 
 
+def next_norm(ctx, x, *weights):
+    """What `ops.residual_norm` and `ops.add_normed` take as next_norm behind a block's last sublayer, if one norm reads the stream next (captured
+    steps) and these rows allow it: the normed rows are then left for it under NORMED_STREAM."""
+    norm = ctx.norm_behind
+    if not isinstance(norm, RMSNorm) or norm.size != x.shape[1] or not ops.can_norm_next(x, norm.weight, *weights):
+        return None
+    rows = ctx.scratch("norm.out", tuple(x.shape))
+    ctx.shared[NORMED_STREAM] = (norm, rows)
+    return norm.weight, norm.eps, rows
+
+
 def normalise(norm, ctx, x, pending=None, rows=None):
     """NORM of X; PENDING partial sums go to a norm that folds them, and are folded here for one that does not
     (which only happens when parts are driven by hand: a model defers sums only if all its norms fold them)."""
@@ -203,7 +214,7 @@ class PostNormBlock(Block):
     def entry(self):
         return (), (self.mixer,)
 
-    def _sublayer(self, ctx, x, part, args, norm, scale, readers, behind):
+    def _sublayer(self, ctx, x, part, args, norm, scale, readers, behind, last):
         """x <- norm(alpha * x + scale * PART(rows)), ARGS what the part takes before its rows. BEHIND: `ops.NormedRows` where x is still
         the rows of a norm that travels (None: x is the stream). Returns the same of the new stream."""
         result = ctx.scratch("sublayer.result", (ctx.n_tokens, self.hidden), torch.float32)
@@ -217,16 +228,17 @@ class PostNormBlock(Block):
             return left
         rounded = ctx.scratch("stream.rounded", (ctx.n_tokens, self.hidden)) if ctx.dtype != torch.float32 else None
         ops.residual_norm(x, norm.weight, norm.eps, out=rounded, y=result if left is None else None, add=left, scale=scale, alpha=self.alpha,
-                          before=behind.norm.weight if behind is not None else None)
+                          before=behind.norm.weight if behind is not None else None, next_norm=next_norm(ctx, x, norm.weight, scale) if last else None)
         ctx.shared[ROUNDED_STREAM] = rounded if rounded is not None else x
         return None
 
     def forward(self, ctx, run, x, pending=None):
         behind = pending if isinstance(pending, ops.NormedRows) else fold_pending(x, pending)
         follows = ctx.entry_behind[1] if ctx.entry_behind is not None and not ctx.entry_behind[0] else ()      # (a block that reads the stream as it is)
-        behind = self._sublayer(ctx, x, self.mixer, (run,), self.mixer_norm, self.mixer_scale, (self.ffn,) if self.ffn is not None else follows, behind)
+        behind = self._sublayer(ctx, x, self.mixer, (run,), self.mixer_norm, self.mixer_scale, (self.ffn,) if self.ffn is not None else follows, behind,
+                                self.ffn is None)
         if self.ffn is not None:
-            behind = self._sublayer(ctx, x, self.ffn, (), self.ffn_norm, self.ffn_scale, follows, behind)
+            behind = self._sublayer(ctx, x, self.ffn, (), self.ffn_norm, self.ffn_scale, follows, behind, True)
         return behind
 
 
@@ -272,20 +284,20 @@ class ResultNormBlock(Block):
     def entry(self):
         return (), ()                     # (reads the stream as it is; nothing is left for it in place of sums)
 
-    def _sublayer(self, ctx, x, norm, result, pending):
+    def _sublayer(self, ctx, x, norm, result, pending, last):
         rounded = ctx.scratch("stream.rounded", (ctx.n_tokens, self.hidden)) if ctx.dtype != torch.float32 else None
         ops.add_normed(x, norm.weight, norm.eps, mult=self.mult, y=result if pending is None else None, add=pending,
-                       out=rounded)
+                       out=rounded, next_norm=next_norm(ctx, x, norm.weight) if last else None)
         ctx.shared[ROUNDED_STREAM] = rounded if rounded is not None else x
 
     def forward(self, ctx, run, x, pending=None):
         pending = fold_pending(x, pending)
         result = ctx.scratch("sublayer.result", (ctx.n_tokens, self.hidden), torch.float32)
         left = self.mixer.forward(ctx, run, self._rounded(ctx, x), result, accumulate=False)
-        self._sublayer(ctx, x, self.mixer_norm, result, left)
+        self._sublayer(ctx, x, self.mixer_norm, result, left, self.ffn is None)
         if self.ffn is not None:
             left = self.ffn.forward(ctx, self._rounded(ctx, x), result, accumulate=False)
-            self._sublayer(ctx, x, self.ffn_norm, result, left)
+            self._sublayer(ctx, x, self.ffn_norm, result, left, True)
         return None
 
 

@@ -248,3 +248,24 @@ def test_product_that_fills_the_cache_with_columns_behind(ops, device, dtype, m,
     assert torch.equal(keys, want_keys) and torch.equal(values, want_values)
     q, kv = q_heads * dim, (q_heads + 2 * kv_heads) * dim
     assert torch.equal(out[:, :q], want[:, :q]) and torch.equal(out[:, kv:width], want[:, kv:]) and (out[:, width:] == -9).all()
+
+
+# one and many rows, either side of the line up to which weights are requested with the row; one, two and four groups a thread
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("n,hidden,splits", [(1, 64, 3), (8, 2048, 4), (16, 4100, 0), (300, 896, 2), (5, 8196, 1), (3, 16384, 0)])
+def test_rows_behind_the_next_norm_as_well(ops, device, dtype, n, hidden, splits):
+    x, w, w2 = rand((n, hidden), torch.float32, device, 2.0), 1 + rand((hidden,), torch.float32, device, 0.1, 1), 1 + rand((hidden,), torch.float32, device, 0.1, 2)
+    parts = rand((max(splits, 1), n, hidden), torch.float32, device, 1.0, 3)
+    source = dict(add=parts) if splits else dict(y=parts[0])
+    for step in (ops.residual_norm, ops.add_normed):
+        alone, both, rows = x.clone(), x.clone(), torch.full((n, hidden), float("nan"), dtype=dtype, device=device)
+        outs = [torch.empty(n, hidden, dtype=dtype, device=device) for _ in range(2)]
+        step(alone, w, 1e-6, out=outs[0], **source)
+        step(both, w, 1e-6, out=outs[1], next_norm=(w2, 1e-5, rows), **source)
+        assert torch.equal(alone, both) and torch.equal(*outs)
+        want = both.double() / torch.sqrt((both.double() ** 2).mean(-1, keepdim=True) + 1e-5) * w2.double()
+        # the sum of squares, its root and two products: a few 2^-24 of the value, and one rounding to the type
+        assert ((rows.double() - want).abs() <= (BITS[dtype] + 2.0 ** -20) * want.abs()).all()
+        step(x.clone(), w, 1e-6, next_norm=(w2, 1e-5, rows), **source)                     # (without the rows as they are)
+        with pytest.raises(Exception):
+            step(x[:, 1:].contiguous(), w[1:].contiguous(), 1e-6, y=parts[0][:, 1:], next_norm=(w2[1:].contiguous(), 1e-5, rows[:, 1:].contiguous()))
