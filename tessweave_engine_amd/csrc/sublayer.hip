@@ -25,7 +25,8 @@ struct ResidualNormArgs {
   void* out;                // [n][hidden], compute type, or null
   int hidden;
   float alpha, eps;
-  const float* before;      // [hidden] or null: x stands for before * unit(x) (few rows: the kernel of four consecutive elements)
+  const float* before;      // [hidden] or null: x stands for before * unit(x) (few rows: the kernel of four consecutive elements),
+  float before_eps;         // whose eps is that of the norm the rows are behind
   NextNorm next;                         // (rows of whole groups of four alone)
 };
 
@@ -134,7 +135,7 @@ __global__ __launch_bounds__(1024) void residual_norm_vec4_kernel(ResidualNormAr
         for (int e = 0; e < 4; ++e) ss = __fmaf_rn(xv[i][e], xv[i][e], ss);
       }
     }
-    const float unit = 1.f / sqrtf(tw_block_sum(ss, lds) / (float)a.hidden + a.eps);
+    const float unit = 1.f / sqrtf(tw_block_sum(ss, lds) / (float)a.hidden + a.before_eps);
 #pragma unroll
     for (int i = 0; i < PER; ++i) xv[i] = f32x4{xv[i][0] * unit * bv[i][0], xv[i][1] * unit * bv[i][1], xv[i][2] * unit * bv[i][2], xv[i][3] * unit * bv[i][3]};
     ss = 0.f;
@@ -231,15 +232,15 @@ static void residual_norm_launch(const ResidualNormArgs& a, int n, hipStream_t s
 
 extern "C" int tw_residual_norm(int out_dtype, float* x, const float* y, long ldy, const float* add, int splits,
                                 long add_stride, const float* scale, const float* w, void* out, int n, int hidden,
-                                float alpha, float eps, const float* before, const float* next_w, void* next_out, float next_eps,
-                                hipStream_t stream) {
+                                float alpha, float eps, const float* before, float before_eps, const float* next_w, void* next_out,
+                                float next_eps, hipStream_t stream) {
   TW_REQUIRE(x && w && n >= 0 && hidden > 0 && eps > 0.f);
   TW_REQUIRE(add == nullptr || (splits > 0 && add_stride >= (long)n * hidden));
   TW_REQUIRE(y == nullptr || ldy >= hidden);
   if (n == 0) return 0;
-  ResidualNormArgs a{x, add ? nullptr : y, ldy, add, splits, (size_t)add_stride, scale, w, out, hidden, alpha, eps, before, {next_w, next_out, next_eps}};
+  ResidualNormArgs a{x, add ? nullptr : y, ldy, add, splits, (size_t)add_stride, scale, w, out, hidden, alpha, eps, before, before_eps, {next_w, next_out, next_eps}};
   TW_REQUIRE(next_norm_ok(a.next) && (!next_w || (residual_rows_aligned(a) && hidden <= 4 * 4096)));
-  TW_REQUIRE(!before || (n <= TW_EARLY_ROWS && residual_rows_aligned(a) && (uintptr_t)before % 16 == 0 && hidden <= 4 * 4096));
+  TW_REQUIRE(!before || (before_eps > 0.f && n <= TW_EARLY_ROWS && residual_rows_aligned(a) && (uintptr_t)before % 16 == 0 && hidden <= 4 * 4096));
   if (out_dtype == TW_DTYPE_BF16) residual_norm_launch<bf16_t>(a, n, stream);
   else if (out_dtype == TW_DTYPE_F32) residual_norm_launch<float>(a, n, stream);
   else return TW_ERR_BAD_ARGUMENT;

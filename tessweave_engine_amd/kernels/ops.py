@@ -1095,7 +1095,7 @@ def _next_norm(next_norm, x, out):
 
 def residual_norm(x, weight, eps, out=None, y=None, add=None, scale=None, alpha=1.0, before=None, next_norm=None):
     """x <- weight * unit(alpha * x + scale * y), unit(v) = v / sqrt(mean(v^2) + eps); x float32 [n, hidden] in place.
-    before (float32 [hidden], for `can_leave_norms` rows): before * unit(x) takes the place of x.
+    before = (weight, eps) of another norm, for `can_leave_norms` rows: weight * unit(x), with that eps, takes the place of x.
 
     y: float32 [n, hidden] (rows may be strided), or add: float32 [splits, n, hidden] partial sums added up here;
     scale: float32 [hidden] or None; out: the normed rows once more, rounded to its type (the compute type). next_norm: see `_next_norm`."""
@@ -1114,6 +1114,7 @@ def residual_norm(x, weight, eps, out=None, y=None, add=None, scale=None, alpha=
         splits, stride = add.shape[0], n * hidden
     if scale is not None:
         _need(scale.numel() == hidden and scale.dtype == torch.float32 and scale.is_contiguous(), "scale must be float32 [hidden]")
+    before, before_eps = before if before is not None else (None, 0.0)
     if before is not None:
         _need(can_leave_norms(n, hidden) and before.numel() == hidden and before.is_contiguous(), "before must be [hidden], of rows whose norms can travel")
     out_dtype, following = F32 if next_norm is None else dtype_id(next_norm[2].dtype), _next_norm(next_norm, x, out)
@@ -1124,7 +1125,7 @@ def residual_norm(x, weight, eps, out=None, y=None, add=None, scale=None, alpha=
                                      _dev(add) if add is not None else None, splits, stride,
                                      _dev(scale) if scale is not None else None, _dev(weight),
                                      _dev(out) if out is not None else None, n, hidden, float(alpha), float(eps),
-                                     _dev(before, torch.float32, "before") if before is not None else None, *following, _stream()),
+                                     _dev(before, torch.float32, "before") if before is not None else None, float(before_eps), *following, _stream()),
           "residual_norm")
     return x
 

@@ -20,7 +20,7 @@ import pytest
 import torch
 
 import plain_dinutar as plain
-from dinutar_util import CONFIGS, Driver, make_weights, row_error, write_folder
+from dinutar_util import CONFIGS, Driver, config, latent, make_weights, retention, row_error, write_folder
 
 pytestmark = pytest.mark.gpu
 
@@ -466,6 +466,26 @@ def test_token_by_token(model, dtype, graphs):
     if graphs and d.model.graph_safe_model:
         assert d.stepper.graph_replays > 0
     d.close()
+
+
+def test_token_by_token_with_norms_of_different_eps(tmp_path, device):
+    """Blocks take norms of any eps: captured steps, where a norm may travel with the product behind it, against eager ones. (float32: the
+    factors differ by several times between the eps, and sums in another order by 2e-5 of the logits' spread.) Products that leave their
+    rows and products that do not: a width of 64s, wide and narrow feed-forwards, none at all."""
+    c = config([latent(2, 16, 16, 32, 32, 0.25, ff=192), retention(2, 32, 32, [0.9, 0.99], 32, ff=64), latent(4, 16, 16, 16, 32, 0.2), latent(2, 16, 16, 32, 32, 0.25, ff=128)],
+               width=128, vocab=97, alpha=1.3, scale=0.7, buckets=7, mul_prev=5, mul_cur=3)
+    folder = write_folder(tmp_path, c, make_weights(c, seed=4))
+    tokens, got = {"a": [(7 * i + 3) % 97 for i in range(14)], "b": [(5 * i + 1) % 97 for i in range(14)]}, []
+    for graphs in (True, False):
+        d = Driver(folder, "float32", pages=24, page_size=4, graphs=graphs)
+        norms = [norm for block in d.model.blocks for norm in (block.mixer_norm, block.ffn_norm) if norm is not None]
+        for norm, eps in zip(norms, (0.9, 1e-6, 0.2, 1e-5, 2.0, 0.4, 1e-6)):
+            norm.eps = eps
+        got.append(d.run([[("a", 1), ("b", 1)] for _ in range(14)], tokens))
+        assert graphs == (d.stepper.graph_replays > 0)
+        d.close()
+    for rid in tokens:
+        check_rows(row_error(got[0][rid], got[1][rid]), "float32")
 
 
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])

@@ -141,13 +141,15 @@ def test_rotated_product(ops, device, dtype, with_norms, m, q_heads, kv_heads, d
 
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("hidden", [64, 2048, 4096])
-def test_residual_norm_of_rows_behind_a_norm(ops, device, dtype, hidden):
+@pytest.mark.parametrize("eps", [(1e-6, 1e-6), (3.0, 1e-6), (1e-6, 0.5)])
+def test_residual_norm_of_rows_behind_a_norm(ops, device, dtype, hidden, eps):
+    """Two norms behind one another, each with its own eps."""
     x, y = rand((16, hidden), torch.float32, device, 3.0), rand((3, 16, hidden), torch.float32, device, 1.0, 1)
     w, before, scale = (1 + rand((hidden,), torch.float32, device, 0.1, s) for s in (2, 3, 4))
     out = torch.empty(16, hidden, dtype=dtype, device=device)
-    unit = lambda v: v / torch.sqrt((v ** 2).mean(-1, keepdim=True) + 1e-6)       # noqa: E731
-    want = unit(0.7 * unit(x.double()) * before.double() + scale.double() * y.double().sum(0)) * w.double()
-    ops.residual_norm(x, w, 1e-6, out=out, add=y, scale=scale, alpha=0.7, before=before)
+    unit = lambda v, eps: v / torch.sqrt((v ** 2).mean(-1, keepdim=True) + eps)       # noqa: E731
+    want = unit(0.7 * unit(x.double(), eps[0]) * before.double() + scale.double() * y.double().sum(0), eps[1]) * w.double()
+    ops.residual_norm(x, w, eps[1], out=out, add=y, scale=scale, alpha=0.7, before=(before, eps[0]))
     torch.testing.assert_close(x.double(), want, atol=3e-6, rtol=3e-6)             # (as this kernel's other forms)
     torch.testing.assert_close(out, x.to(dtype), atol=0, rtol=0)
 
