@@ -65,7 +65,7 @@ __global__ __launch_bounds__(256) void norm_gate_kernel(NormGateArgs a) {
       const float f = KIND == TW_GATE_SIGMOID_BEHIND ? sig : g[i][e] * sig;
       if (KIND == TW_GATE_SILU_BEFORE) v[i][e] *= f;
       else g[i][e] = f;
-      ss = __fmaf_rn(mine ? v[i][e] : 0.f, v[i][e], ss);
+      ss = mine ? __fmaf_rn(v[i][e], v[i][e], ss) : ss;      // (0 times an infinity read again would be a NaN)
     }
   }
   const float sum = THREADS == 32 ? ng_half_wave_sum(ss) : THREADS == 64 ? tw_wave_sum(ss) : tw_block_sum(ss, lds);

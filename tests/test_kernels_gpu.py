@@ -1431,3 +1431,23 @@ def test_units_normed_and_gated(ops, device, dtype, n, parts, size, pitch, offse
     ops.gate_group_norm(y, z, w, out, parts, 1e-5, after=True, scale=0.6)
     want = unit(cut(y)) * w.double().view(parts, size) * torch.sigmoid(cut(z)) * 0.6
     torch.testing.assert_close(out.double().view_as(want), want, **close)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("size", [124, 132, 260, 516, 1028, 128])          # (all but the last: lanes past the end read its last group again)
+def test_an_infinity_in_a_units_last_group(ops, device, dtype, size):
+    """Over an infinite root mean square every finite element is 0, and the infinite one no number; the units beside it are as without it."""
+    n, parts = 2, 3
+    y, z = rand((n, parts * size), torch.float32, device, 2.0), rand((n, parts * size), torch.float32, device, 2.0, 1)
+    w, at = 1 + rand((parts * size,), torch.float32, device, 0.1, 2), 2 * size - 2
+    forms = [lambda out: ops.unit_gate(y, z.to(dtype), out, parts, size, size, 1e-5), lambda out: ops.head_norm_gate(y, z, w, out, parts, size, 1e-5),
+             lambda out: ops.head_norm_gate(y, z, w[:size].contiguous(), out, parts, size, 1e-5, gate_activation="sigmoid"),
+             lambda out: ops.gate_group_norm(y, z, w, out, parts, 1e-5), lambda out: ops.gate_group_norm(y, z, w, out, parts, 1e-5, after=True)]
+    want = [form(torch.empty(n, parts * size, dtype=dtype, device=device)) for form in forms]
+    y[1, at] = float("inf")
+    for form, plain in zip(forms, want):
+        got = form(torch.empty(n, parts * size, dtype=dtype, device=device))
+        plain[1, size:2 * size] = 0
+        assert got[1, at].isnan()
+        got[1, at] = 0
+        assert torch.equal(got, plain)
