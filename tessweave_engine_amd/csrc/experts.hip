@@ -132,7 +132,7 @@ __global__ __launch_bounds__(64 * WAVES) void moe_route_kernel(const T* __restri
     int mine = 0;
     float weight = 0.f;
     for (int r = 0; r < top; ++r) {
-      const float best = tw_wave_max(v);
+      const float best = fmaxf(tw_wave_max(v), -INFINITY);            // (64 logits that are all NaN: no number is the largest)
       const unsigned long long holders = __ballot(v == best);
       const int at = min(holders ? __ffsll((long long)holders) - 1 : X - 1, X - 1);      // (no logit compares as the largest if all are NaN)
       const float chosen = mode == 2 ? share : best;

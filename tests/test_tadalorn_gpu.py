@@ -232,6 +232,29 @@ def test_router_with_bias_and_softmax_over_the_chosen(device, C, X, top):
         assert not (chosen[both] == 2).any()
 
 
+@pytest.mark.parametrize("X", [5, 63, 64, 65])                       # (up to 64: an expert a lane)
+@pytest.mark.parametrize("weighting", ["sigmoid", "softmax_chosen"])
+def test_router_over_logits_that_are_no_numbers(device, X, weighting):
+    """NaN is never the largest: the other logits are chosen first, then the lowest of those that are -inf or taken already, and the last expert
+    where there is none but NaN."""
+    from tessweave_engine_amd.kernels import ops
+    nan, inf, top = float("nan"), float("inf"), 3
+    for case in ([nan] * X, [nan] * (X - 1) + [2.0], [nan, 1.0, nan, 3.0] + [nan] * (X - 4), [-inf] * X, [-inf] * (X - 1) + [nan],
+                 [0.5, inf] + [0.5] * (X - 2), [nan] * (X - 2) + [-inf, nan]):
+        ids, weights = torch.empty(1, top, dtype=torch.int32, device=device), torch.empty(1, top, device=device)
+        ops.moe_route(torch.ones(1, 32, device=device), torch.zeros(X, 32, device=device), top, ids, weights, bias=torch.tensor(case, device=device), weighting=weighting)
+        z, want, best = list(case), [], []
+        for _ in range(top):
+            finite = [v for v in z if v == v]
+            best.append(max(finite, default=-inf))
+            want.append(z.index(best[-1]) if finite else X - 1)
+            z[want[-1]] = -inf
+        assert ids[0].tolist() == want, case
+        best = torch.tensor(best, dtype=torch.float64)
+        expected = torch.sigmoid(best) if weighting == "sigmoid" else torch.exp(best - best[0]) / torch.exp(best - best[0]).sum()
+        torch.testing.assert_close(weights[0].cpu().double(), expected, atol=1e-6, rtol=0, equal_nan=True)
+
+
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 @pytest.mark.parametrize("n,C,X,top,F", [(1, 88, 5, 2, 40), (9, 128, 16, 4, 64), (300, 96, 3, 3, 24), (130, 72, 64, 1, 100), (17, 64, 2, 1, 32)])
 def test_grouped_experts_without_a_gate(device, dtype, n, C, X, top, F):
