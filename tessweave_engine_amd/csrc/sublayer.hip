@@ -25,7 +25,7 @@ struct ResidualNormArgs {
   void* out;                // [n][hidden], compute type, or null
   int hidden;
   float alpha, eps;
-  const float* before;      // [hidden] or null: x stands for before * unit(x) (few rows: the kernel of four consecutive elements),
+  const float* before;      // [hidden] or null: x stands for before * unit(x),
   float before_eps;         // whose eps is that of the norm the rows are behind
   NextNorm next;                         // (rows of whole groups of four alone)
 };
@@ -180,7 +180,12 @@ __global__ void residual_norm_kernel(ResidualNormArgs a) {
   __shared__ float lds[16];
   const int row = blockIdx.x;
   float* x = a.x + (size_t)row * a.hidden;
-  float ss = 0.f;
+  float ss = 0.f, unit = 1.f;
+  if (a.before) {
+    for (int c = threadIdx.x; c < a.hidden; c += blockDim.x) ss = __fmaf_rn(x[c], x[c], ss);
+    unit = 1.f / sqrtf(tw_block_sum(ss, lds) / (float)a.hidden + a.before_eps);
+    ss = 0.f;
+  }
   for (int c = threadIdx.x; c < a.hidden; c += blockDim.x) {
     float yv = 0.f;
     if (a.add) {
@@ -189,7 +194,7 @@ __global__ void residual_norm_kernel(ResidualNormArgs a) {
       yv = a.y[(size_t)row * a.ldy + c];
     }
     if (a.scale) yv *= a.scale[c];
-    const float v = __fmaf_rn(a.alpha, x[c], yv);
+    const float v = __fmaf_rn(a.alpha, a.before ? x[c] * unit * a.before[c] : x[c], yv);
     x[c] = v;
     ss = __fmaf_rn(v, v, ss);
   }
@@ -207,14 +212,14 @@ static bool residual_rows_aligned(const ResidualNormArgs& a) {
   return a.hidden % 4 == 0 && (uintptr_t)a.x % 16 == 0 && (uintptr_t)a.w % 16 == 0 &&
          (!a.y || ((uintptr_t)a.y % 16 == 0 && a.ldy % 4 == 0)) &&
          (!a.add || ((uintptr_t)a.add % 16 == 0 && a.add_stride % 4 == 0)) &&
-         (!a.scale || (uintptr_t)a.scale % 16 == 0);
+         (!a.scale || (uintptr_t)a.scale % 16 == 0) && (!a.before || (uintptr_t)a.before % 16 == 0);
 }
 
 template <typename T>
 static void residual_norm_launch(const ResidualNormArgs& a, int n, hipStream_t stream) {
   const bool aligned = residual_rows_aligned(a);
   const int chunks = a.hidden / 4;
-  if (aligned && chunks <= 4096) {
+  if (aligned && chunks <= 4096 && (!a.before || n <= TW_EARLY_ROWS)) {
     const int per = chunks <= 1024 ? 1 : (chunks <= 2048 ? 2 : 4);
     int threads = (chunks + per - 1) / per;
     threads = (threads + 63) / 64 * 64;
@@ -239,8 +244,8 @@ extern "C" int tw_residual_norm(int out_dtype, float* x, const float* y, long ld
   TW_REQUIRE(y == nullptr || ldy >= hidden);
   if (n == 0) return 0;
   ResidualNormArgs a{x, add ? nullptr : y, ldy, add, splits, (size_t)add_stride, scale, w, out, hidden, alpha, eps, before, before_eps, {next_w, next_out, next_eps}};
-  TW_REQUIRE(next_norm_ok(a.next) && (!next_w || (residual_rows_aligned(a) && hidden <= 4 * 4096)));
-  TW_REQUIRE(!before || (before_eps > 0.f && n <= TW_EARLY_ROWS && residual_rows_aligned(a) && (uintptr_t)before % 16 == 0 && hidden <= 4 * 4096));
+  TW_REQUIRE(!before || before_eps > 0.f);
+  TW_REQUIRE(next_norm_ok(a.next) && (!next_w || (residual_rows_aligned(a) && hidden <= 4 * 4096 && (!before || n <= TW_EARLY_ROWS))));
   if (out_dtype == TW_DTYPE_BF16) residual_norm_launch<bf16_t>(a, n, stream);
   else if (out_dtype == TW_DTYPE_F32) residual_norm_launch<float>(a, n, stream);
   else return TW_ERR_BAD_ARGUMENT;

@@ -118,8 +118,13 @@ def _rope_tables(positions, tables):
     return arg
 
 
-def can_embed_begin(table):
-    return table.shape[1] % 16 == 0 and table.is_contiguous() and table.data_ptr() % 16 == 0
+def _aligned(*tensors):
+    return all(t is None or t.data_ptr() % 16 == 0 for t in tensors)
+
+
+def can_embed_begin(table, *weights):
+    """Does `embed_begin` take rows of this table, with these norms' weights? (aligned ones)"""
+    return table.shape[1] % 16 == 0 and table.is_contiguous() and _aligned(table, *weights)
 
 
 def embed_begin(ids, table, out, feed=None, norm=None, second=None, sums=None, eps=0.0, rounded=None, positions=None, tables=()):
@@ -128,7 +133,8 @@ def embed_begin(ids, table, out, feed=None, norm=None, second=None, sums=None, e
     tables: rotary tables of POSITIONS, (inv_freq, rest or None, cos, sin, magnitude) each (see `rope_table`)."""
     n = ids.numel()
     vocab, hidden = table.shape
-    _need(can_embed_begin(table) and out.is_contiguous() and tuple(out.shape) == (n, hidden), "embed_begin takes rows of a multiple of 16 elements")
+    _need(can_embed_begin(table, *(p[0] for p in (norm, second) if p is not None)) and out.is_contiguous() and tuple(out.shape) == (n, hidden),
+          "embed_begin takes aligned rows of a multiple of 16 elements and aligned weights")
     _need(norm is None or (rounded is None and can_leave_norms(n, hidden) and sums is not None and sums.is_contiguous()
                            and tuple(sums.shape) == (n, hidden // 16)), "the norm of these rows cannot travel")
     for w, r in [p for p in (norm, second) if p is not None] + ([(None, rounded)] if rounded is not None else []):
@@ -1079,8 +1085,7 @@ def attn_mixed(q, keys, values, block_table, q_start, kv_len, seq0, n_seqs, max_
 
 def can_norm_next(x, *weights):
     """Can `residual_norm` or `add_normed` of X put its new rows behind a further norm? (whole groups of four, up to 16,384 elements)"""
-    return (x.shape[1] % 4 == 0 and x.shape[1] <= 16384 and x.is_contiguous() and x.data_ptr() % 16 == 0
-            and all(w is None or w.data_ptr() % 16 == 0 for w in weights))
+    return x.shape[1] % 4 == 0 and x.shape[1] <= 16384 and x.is_contiguous() and _aligned(x, *weights)
 
 
 def _next_norm(next_norm, x, out):
@@ -1569,9 +1574,9 @@ MOE_KINDS = {"swish_limited": 0, "gelu": 1, "silu": 2, "relu_squared": 3}
 MOE_PLAIN = ("gelu", "relu_squared")           # kinds without a gate
 
 
-def can_moe_norm(h, x):
-    """Can `moe_experts` norm the rows it adds to? (aligned rows of up to 4,096 elements)"""
-    return (x.shape[1] <= 4096 and x.shape[1] % 4 == 0 and x.is_contiguous() and h.is_contiguous() and x.data_ptr() % 16 == 0 and h.data_ptr() % 16 == 0)
+def can_moe_norm(h, x, weight):
+    """Can `moe_experts` put the rows it adds to behind the norm of WEIGHT? (aligned rows of up to 4,096 elements)"""
+    return x.shape[1] <= 4096 and x.shape[1] % 4 == 0 and x.is_contiguous() and h.is_contiguous() and _aligned(x, h, weight)
 
 
 def moe_experts(h, ids, weights, gate, up, down, limit, x, scratch, kind="swish_limited", accumulate=True, more=None, norm=None):
@@ -1606,7 +1611,7 @@ def moe_experts(h, ids, weights, gate, up, down, limit, x, scratch, kind="swish_
               "more must be float32 [splits, n, C]")
     if norm is not None:
         weight, norm_eps, normed = norm
-        _need(x is not None and accumulate and can_moe_norm(h, x) and weight.is_contiguous() and weight.numel() == C, "these rows cannot be normed here")
+        _need(x is not None and accumulate and can_moe_norm(h, x, weight) and weight.is_contiguous() and weight.numel() == C, "these rows cannot be normed here")
         _need(normed.is_contiguous() and tuple(normed.shape) == (n, C) and normed.dtype == h.dtype, "the normed rows must be [n, C] of h's type")
     capacity = moe_capacity(n * top, X)
     pos = scratch("moe.pos", (n * top,), torch.int32)

@@ -227,8 +227,9 @@ class PostNormBlock(Block):
         if isinstance(left, ops.NormedRows):
             return left
         rounded = ctx.scratch("stream.rounded", (ctx.n_tokens, self.hidden)) if ctx.dtype != torch.float32 else None
+        before = behind.norm.weight if behind is not None else None
         ops.residual_norm(x, norm.weight, norm.eps, out=rounded, y=result if left is None else None, add=left, scale=scale, alpha=self.alpha,
-                          before=(behind.norm.weight, behind.eps) if behind is not None else None, next_norm=next_norm(ctx, x, norm.weight, scale) if last else None)
+                          before=(before, behind.eps) if behind is not None else None, next_norm=next_norm(ctx, x, norm.weight, scale, before) if last else None)
         ctx.shared[ROUNDED_STREAM] = rounded if rounded is not None else x
         return None
 

@@ -34,10 +34,13 @@ class TokenEmbedding(Part):
         return ops.embed_gather(ctx.token_ids, self.weight, self._stream(ctx), feed=ctx.token_feed)
 
     def forward(self, ctx):
-        if not ctx.capturing or not ops.can_embed_begin(self.weight):
+        if not ctx.capturing:
+            return self.gather(ctx)
+        norms, readers = ctx.entry_behind or (None, ())
+        if not ops.can_embed_begin(self.weight, *(norm.weight for norm in norms or ())):
             return self.gather(ctx)
         # a step of one-token rows: the rotary tables, and the rows as their first reader wants them, are formed in the same launch
-        x, norms, readers = self._stream(ctx), *(ctx.entry_behind or (None, ()))
+        x = self._stream(ctx)
         options, ahead = {}, norm_ahead(ctx, x, norms, readers) if norms else None
         if ahead is not None:
             rows, sums = ahead.buffers(ctx, self.weight.dtype)

@@ -153,7 +153,7 @@ class RoutedExperts(FeedForward):
             rows, pos = ops.moe_experts(h, ids, weights, self.gate, self.up, self.down, self.limit, None, scratch, kind=self.kind)
             return ApartResult(pending, (rows, pos, weights), wrote)
         norm, behind = None, getattr(ctx, "norm_closing", None)
-        if behind is not None and accumulate and behind.size == self.hidden and ops.can_moe_norm(h, x):
+        if behind is not None and accumulate and behind.size == self.hidden and ops.can_moe_norm(h, x, behind.weight):
             norm = (behind.weight, behind.eps, ctx.scratch("norm.out", (n, self.hidden)))      # (the last kernel norms what it wrote)
             ctx.shared[NORMED_STREAM] = (behind, norm[2])
         ops.moe_experts(h, ids, weights, self.gate, self.up, self.down, self.limit, x, scratch, kind=self.kind,

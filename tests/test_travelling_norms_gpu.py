@@ -154,6 +154,64 @@ def test_residual_norm_of_rows_behind_a_norm(ops, device, dtype, hidden, eps):
     torch.testing.assert_close(out, x.to(dtype), atol=0, rtol=0)
 
 
+def misaligned(t):
+    """The same values four bytes behind a multiple of 16."""
+    flat = torch.empty(t.numel() + 1, dtype=t.dtype, device=t.device)
+    assert flat.data_ptr() % 16 == 0
+    flat[1:] = t.reshape(-1)
+    return flat[1:].view(t.shape)
+
+
+@pytest.mark.parametrize("which", ["w", "scale", "before", "all"])
+def test_residual_norm_of_rows_behind_a_norm_with_any_weights(ops, device, which):
+    """As with aligned ones, but for the order of the sums of squares."""
+    x, y = rand((5, 896), torch.float32, device, 3.0), rand((3, 5, 896), torch.float32, device, 1.0, 1)
+    given = {k: 1 + rand((896,), torch.float32, device, 0.1, i) for i, k in enumerate(("w", "scale", "before"))}
+    want, out = x.clone(), torch.empty(5, 896, dtype=torch.bfloat16, device=device)
+    ops.residual_norm(want, given["w"], 1e-6, add=y, scale=given["scale"], alpha=0.7, before=(given["before"], 0.5))
+    given = {k: misaligned(v) if which in (k, "all") else v for k, v in given.items()}
+    ops.residual_norm(x, given["w"], 1e-6, out=out, add=y, scale=given["scale"], alpha=0.7, before=(given["before"], 0.5))
+    torch.testing.assert_close(x, want, atol=1e-6, rtol=1e-6)
+    assert torch.equal(out, x.to(torch.bfloat16))
+
+
+DESIGNS = [("qwen2", "A"), ("qwen2", "B"), ("kanavik", "wide"), ("dinutar", "wide"), ("rufusun", "wide"), ("tadalorn", "wide"), ("darolix", "wide"), ("darolix", "odd"),
+           ("vulosun", "wide")]
+
+
+@pytest.mark.parametrize("design,name", DESIGNS)
+def test_captured_steps_with_norm_weights_anywhere(device, tmp_path, design, name):
+    """Weights that were bound as slices of a larger buffer need not be aligned: captured float32 steps against eager ones with aligned weights,
+    to 2e-5 of the logits' spread (sums in other orders). Tadalorn's mLSTM divides by a sum that may nearly cancel, which moves a row in any
+    order of operations: one of its rows may lie beyond that, none beyond 1e-3 (as in the design's own tests)."""
+    import importlib
+    from kanavik_util import Driver, row_error
+    from tessweave_engine_amd.parts.base import Norm
+    from tessweave_engine_amd.parts.model import walk
+    if design == "qwen2":
+        from tiny_configs import make_folder
+        make_folder(str(tmp_path), name)
+        folder = str(tmp_path)
+    else:
+        util = importlib.import_module(design + "_util")
+        config = util.CONFIGS[name]
+        folder = util.write_folder(tmp_path, config, util.make_weights(config, seed=3))
+    got = []
+    for graphs in (False, True):
+        d = Driver(folder, "float32", pages=24, page_size=4, graphs=graphs)
+        tokens = {rid: [(s * i + 3) % d.model.vocab_size for i in range(12)] for rid, s in (("a", 7), ("b", 5))}
+        if graphs:
+            for part in walk(d.model):
+                for attribute in ("weight", "bias") if isinstance(part, Norm) else ("mixer_scale", "ffn_scale"):
+                    if getattr(part, attribute, None) is not None:
+                        setattr(part, attribute, misaligned(getattr(part, attribute)))
+        got.append(d.run([[("a", 1), ("b", 1)] for _ in range(12)], tokens))
+        assert (d.stepper.graph_replays > 0) == (graphs and d.model.graph_safe_model)
+        d.close()
+    errors = sorted(e for rid in tokens for e in row_error(got[1][rid], got[0][rid]).tolist())
+    assert errors[-2 if design == "tadalorn" else -1] < 2e-5 and errors[-1] < 1e-3
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("n,hidden,form", [(1, 64, "norm"), (16, 896, "two norms"), (3, 4096, "norm"), (40, 2064, "rounded"), (5, 16, "rows alone"), (16, 3072, "no tables")])
 def test_embed_begin(ops, device, dtype, n, hidden, form):
