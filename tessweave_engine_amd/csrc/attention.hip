@@ -1635,27 +1635,34 @@ static int check_common(const AttnArgs& a) {
 
 // Key ranges per (sequence, kv head) of the decode kernels: the number with the least estimated time. `units` (sequence, kv head) pairs
 // with s ranges each are units * s workgroups, in turns of 256. A workgroup costs its start and merge (its waves' chain: the lengths, the page, the keys)
-// and a rate per key that is a CU's own, the slower the more CUs read at once; all together are no faster than memory. More than one range costs the
-// kernel that merges them. Measured with the cache in HBM, in a captured graph (us; ranges 1 / 2 / 4 / 8 / 16, the merge included):
+// and a rate per key that is a CU's own, the slower the more CUs read at once (a full turn reads as slowly whatever follows it: without that,
+// two turns of which the second is half empty look cheaper than a full one); all together are no faster than memory. More than one range costs
+// the kernel that merges them. Measured with the cache in HBM, in a captured graph (us; ranges 1 / 2 / 4 / 8 / 16, the merge included):
 //   bf16, heads of 128 over 4     1 x 150 keys    5.8 / 7.8 / 7.5 / 7.4 / 7.7       1 x 500   10.7 / 10.1 / 8.5 / 7.8 / 7.8      1 x 4000   56 / 34 / 21 / 14 / 11
 //                                 8 x 1000      18.8 / 14.8 / 11.4 / 10.4 / 10.6   24 x 1000   20.7 / 16.9 / 17.3 / 18.4 / 20    64 x 1000   26.7 / 30.7 / 30.9 / 35 / 42
 //   bf16, heads of 64 over 2      1 x 300         5.3 / 7.3 / 6.9 / 6.8 / 6.8       8 x 2000   17.5 / 13.7 / 10.4 / 9.0 / 8.3
 //   float32, heads of 128 over 4  4 x 60          8.7 / 11.8 / 11.4 / 11.3 / 11.5   4 x 300   21.6 / 19.5 / 16.2 / 12.6 / 12.6   8 x 1000   52 / 35 / 25 / 20 / 23
 // (At least 256 keys a range, whatever they weigh, and the fewest turns took 2 / 2 / 16, 4 / 2 / 1, 2 / 8 and 1 / 2 / 4 of these.)
+// Longer ones (us; in brackets the ranges):
+//   bf16, heads of 128 over 4     8 x 6,144 [8 / 13 / 16] 23.3 / 26.2 / 24.5   8 x 12,288 [8 / 12 / 16] 39 / 46 / 39   8 x 32,768 [8 / 11 / 16] 89 / 109 / 90
+//                                 5 x 12,288 [12 / 20] 28.8 / 32   9 x 6,144 [7 / 11 / 14] 26.0 / 29.8 / 26.6   12 x 12,288 [5 / 8 / 10] 55 / 63 / 57   32 x 6,144 [2 / 3 / 4] 70 / 82 / 78
+//   float32, heads of 128 over 4  8 x 3,072 [8 / 16] 35 / 42   4 x 12,288 [16 / 32] 53 / 66
+// Over 166 shapes of 1 to 64 sequences of 192 to 32,768 keys, either type, the choice is 0.9 % behind the fastest of twenty on average; over 156
+// random ones it takes 0.966 of the time of at least 256 keys a range and the fewest turns.
 extern "C" int tw_attn_decode_splits(int dtype, int n_seqs, int q_heads, int kv_heads, int head_dim, int max_kv_len) {
   const int G = q_heads / kv_heads;
   const long units = (long)n_seqs * kv_heads * ((G + 15) / 16);
   const bool f32 = dtype == TW_DTYPE_F32;
   const double start = f32 ? 1.5 + 0.039 * head_dim : 0.9 + 0.0125 * head_dim, key = (f32 ? 3.3e-4 : 1.06e-4) * head_dim;
   const double memory = 2.0 * head_dim * (f32 ? 4 : 2) * units * max_kv_len / 6.3e6;
+  auto turn = [&](long workgroups, int s) { return start + key * (1.0 + 0.0026 * (workgroups > 32 ? workgroups - 32 : 0)) * max_kv_len / s; };
   int most = tw_div_up(max_kv_len, 32);
   if (most > 64) most = 64;
   int best = 1;
   double best_us = 0;
   for (int s = 1; s <= most; ++s) {
-    const long workgroups = units * s, turns = tw_div_up(workgroups, 256);
-    const double busy = 1.0 + 0.0026 * ((workgroups < 256 ? workgroups : 256) > 32 ? (workgroups < 256 ? workgroups : 256) - 32 : 0);
-    double us = turns * (start + key * (turns == 1 ? busy : 1.0) * max_kv_len / s);
+    const long full = (units * s - 1) / 256;
+    double us = full * turn(256, s) + turn(units * s - 256 * full, s);
     if (us < start + memory) us = start + memory;
     if (s > 1) us += 2.65 + 0.05 * s + (s > 16 ? 0.11 * (s - 16) : 0.0);
     if (s == 1 || us < best_us) {

@@ -51,6 +51,24 @@ def test_key_ranges_of_mixed_heads_fill_whole_rounds(dtype, heads, kv_heads, dim
     assert ops.attn_mixed_splits(n, keys, heads, k, v) in good
 
 
+@pytest.mark.parametrize("dtype,heads,kv_heads,dim,n,good", [
+    ("bfloat16", 28, 4, 128, 5, {768: {8, 9, 10, 11, 12}, 6144: {11, 12}, 12288: {11, 12}, 32768: {12}}), ("bfloat16", 28, 4, 128, 7, {6144: {8, 9}, 12288: {8, 9}, 32768: {9}}),
+    ("bfloat16", 28, 4, 128, 8, {3072: {8}, 6144: {8}, 12288: {8, 16}, 32768: {8, 16}}), ("bfloat16", 28, 4, 128, 9, {3072: {7}, 6144: {7, 14}, 12288: {7}, 32768: {7}}),
+    ("bfloat16", 28, 4, 128, 12, {3072: {5}, 12288: {5}}), ("bfloat16", 28, 4, 128, 16, {1500: {4}, 3072: {4, 8}, 12288: {4, 8}}),
+    ("bfloat16", 28, 4, 128, 32, {768: {2, 3, 4}, 3072: {2}, 6144: {2}}), ("bfloat16", 14, 2, 64, 16, {3072: {8}, 12288: {8}}),
+    ("float32", 28, 4, 128, 8, {3072: {8}, 12288: {8}}), ("float32", 28, 4, 128, 4, {768: {12, 14, 16}, 12288: {16}}), ("float32", 14, 2, 64, 24, {3072: {5}, 12288: {5}})])
+def test_key_ranges_of_one_token_sequences_fill_whole_turns(dtype, heads, kv_heads, dim, n, good):
+    """The ranges measured within some 3 % of the fastest; a full turn and part of another is up to a quarter behind. And a captured step's
+    workspace holds what any length class up to the cache's asks for."""
+    kind = getattr(torch, dtype)
+    for keys, ranges in good.items():
+        assert ops.attn_decode_splits(n, heads, kv_heads, keys, dim, kind) in ranges, keys
+    for bound in (1 << i for i in range(4, 16)):
+        for span in (0, 100, 4096):
+            splits, most = ops.attn_decode_class_splits(n, heads, kv_heads, bound, 32768, span, dim, kind)
+            assert 1 <= splits <= most <= 64
+
+
 @pytest.mark.parametrize("heads,kv_heads,dim,value_dim,page", [(16, 4, 128, 128, 16), (1, 1, 64, 64, 32), (20, 10, 128, 128, 16), (16, 4, 128, 128, 24)])
 def test_no_length_has_more_key_ranges_than_a_workspace_is_sized_for(heads, kv_heads, dim, value_dim, page):
     """A captured step's workspace is sized once for all lengths up to the cache's."""
