@@ -7,6 +7,8 @@ back to a library routine.
 """
 from __future__ import annotations
 
+from functools import lru_cache
+
 import torch
 
 from .lib import ROPE_TABLES, RopeTables, library, check
@@ -626,9 +628,11 @@ def attn_decode_splits(n_seqs, q_heads, kv_heads, max_kv_len, head_dim=128, dtyp
     return int(library().tw_attn_decode_splits(dtype_id(dtype), n_seqs, q_heads, kv_heads, head_dim, max_kv_len))
 
 
+@lru_cache(maxsize=1024)
 def attn_decode_class_splits(n_seqs, q_heads, kv_heads, bound, capacity, span, head_dim, dtype):
     """(key ranges for steps whose longest sequence lies in the class up to BOUND keys, the most that any class up to CAPACITY asks for):
-    of a class the middle is taken, of which a query sees at most SPAN keys (0: all)."""
+    of a class the middle is taken, of which a query sees at most SPAN keys (0: all). (Numbers of the arguments alone, over a thousand
+    estimates a call: every layer of a step asks for the same.)"""
     span, shape = span or 1 << 30, (dtype_id(dtype), n_seqs, q_heads, kv_heads, head_dim)
     splits = int(library().tw_attn_decode_splits(*shape, min(max(1, bound * 3 // 4), span)))
     return splits, max(splits, int(library().tw_attn_decode_most_splits(*shape, capacity, span)))

@@ -69,6 +69,13 @@ def test_key_ranges_of_one_token_sequences_fill_whole_turns(dtype, heads, kv_hea
             assert 1 <= splits <= most <= 64
 
 
+def test_key_ranges_are_estimated_once_for_the_layers_of_a_step(monkeypatch):
+    shape = (13, 28, 4, 2048, 8192, 0, 128, torch.bfloat16)
+    want = ops.attn_decode_class_splits(*shape)
+    monkeypatch.setattr(ops, "library", lambda: pytest.fail("estimated again"))
+    assert ops.attn_decode_class_splits(*shape) == want
+
+
 @pytest.mark.parametrize("heads,kv_heads,dim,value_dim,page", [(16, 4, 128, 128, 16), (1, 1, 64, 64, 32), (20, 10, 128, 128, 16), (16, 4, 128, 128, 24)])
 def test_no_length_has_more_key_ranges_than_a_workspace_is_sized_for(heads, kv_heads, dim, value_dim, page):
     """A captured step's workspace is sized once for all lengths up to the cache's."""
