@@ -83,13 +83,6 @@ class WordUpload:
         check(library().tw_upload_words(*self._pointers, k, offsets, counts, _stream()), "upload_words")
 
 
-def upload_words(src, dst, segments):
-    """One `WordUpload`."""
-    segments = [(int(o), int(n)) for o, n in segments]
-    _need(all(o >= 0 and o + n <= dst.numel() for o, n in segments if n > 0), "upload_words: bad segments")
-    WordUpload(src, dst).run(segments)
-
-
 def embed_gather(ids, table, out, feed=None):
     """out[n, :] = float32(table[ids[n], :]); an id -1 - k stands for feed[k] (int32, on the device)."""
     n = ids.numel()

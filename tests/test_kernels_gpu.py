@@ -1451,3 +1451,25 @@ def test_an_infinity_in_a_units_last_group(ops, device, dtype, size):
         assert got[1, at].isnan()
         got[1, at] = 0
         assert torch.equal(got, plain)
+
+
+def test_words_are_fetched_in_segments(ops, device):
+    """One `WordUpload` for many steps: each fetches its own segments, whatever the last one's were; bad ones are refused, with nothing written."""
+    n = 5000
+    src, dst = torch.arange(1, n + 1, dtype=torch.int32).pin_memory(), torch.zeros(n, dtype=torch.int32, device=device)
+    upload, want = ops.WordUpload(src, dst), torch.zeros(n, dtype=torch.int32)
+    sixteen = [(300 * i, 1 + 17 * i) for i in range(16)]
+    for segments in ([], [(7, 0)], sixteen, [(4999, 1)], [(0, n)], [(3, 5), (100, 0), (64, 300)]):
+        dst.zero_()
+        want.zero_()
+        for o, c in segments:
+            want[o:o + c] = src[o:o + c]
+        upload.run(segments)
+        assert torch.equal(dst.cpu(), want)
+    for segments in ([*sixteen, (4990, 3)], [(-1, 2)], [(0, 1), (n - 1, 2)], [(n, 1)]):
+        with pytest.raises(ValueError):
+            upload.run(segments)
+    assert torch.equal(dst.cpu(), want)
+    for bad in ((src[1:], dst), (src.clone(), dst), (src, dst.long()), (src, src)):
+        with pytest.raises(ValueError):
+            ops.WordUpload(*bad)
