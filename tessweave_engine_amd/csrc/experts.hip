@@ -54,6 +54,9 @@ __device__ __forceinline__ f32x4 moe_four(const bf16_t* p) {
 // costs: few rows get many waves each, many rows share a read of the router; B pieces of 256 elements go out together, all of 2,048
 // where a wave has no more than its two experts). Then a wave a row chooses. (us, four pieces at a time and the choice through LDS / now: 4 rows,
 // 20 experts of 2,048, softmax 6.4 / 4.7; 1 row, 16 experts 4.9 / 4.0; 8 rows, 64 experts, eight chosen 14.2 / 9.5; 1,000 rows 9.9 / 6.9.)
+// Pieces behind a row's end are not read: a wave has many pairs of more than 64 experts, and each asked for up to seven pieces that it had no use for. Such
+// routers have 16 waves a row up to 512 rows, which are all there at once. (us, four waves and four pieces a round with the rest apart / every piece of
+// eight read / now: 512 rows of 256, 200 experts 21.9 / 41 / 20.3, 128 experts of 3,072 49 / 60 / 48, 65 rows of 1,024, 200 experts 31 / 42 / 21.)
 template <typename T, int R, int WAVES, int B>
 __global__ __launch_bounds__(64 * WAVES) void moe_route_kernel(const T* __restrict__ h, long ld_h, const float* __restrict__ router,
                                                                const float* __restrict__ bias, int mode, int n, int C, int X,
@@ -73,10 +76,12 @@ __global__ __launch_bounds__(64 * WAVES) void moe_route_kernel(const T* __restri
 #pragma unroll
     for (int r = 0; r < R; ++r) s0[r] = s1[r] = 0.f;
     if (vec) {
-      for (int c0 = 4 * lane; c0 < C; c0 += 256 * B) {
+      for (int first = 0; first < C; first += 256 * B) {
+        const int c0 = first + 4 * lane;
         f32x4 a[B], b[B], xv[R][B];
 #pragma unroll
         for (int j = 0; j < B; ++j) {
+          if (first + 256 * j >= C) break;                 // (the same for all lanes: no piece behind the row's end is read)
           const int c = min(c0 + 256 * j, C - 4);
           a[j] = *reinterpret_cast<const f32x4*>(w0 + c);
           b[j] = *reinterpret_cast<const f32x4*>(w1 + c);
@@ -267,7 +272,7 @@ extern "C" int tw_moe_route(int dtype, const void* h, long ld_h, const float* ro
 #define TW_MOE_ROUTE(T)                                                                                                 \
   do {                                                                                                                  \
     if (n <= 64 && X <= 32) moe_route_kernel<T, 1, 16, 8><<<n, 1024, 0, stream>>>((const T*)h, ld_h, router, bias, mode, n, C, X, top, ids, weights, groups, keep, scale); \
-    else if (n <= 64) moe_route_kernel<T, 1, 16, 4><<<n, 1024, 0, stream>>>((const T*)h, ld_h, router, bias, mode, n, C, X, top, ids, weights, groups, keep, scale); \
+    else if (n <= 64 || (n <= 512 && X > 64)) moe_route_kernel<T, 1, 16, 4><<<n, 1024, 0, stream>>>((const T*)h, ld_h, router, bias, mode, n, C, X, top, ids, weights, groups, keep, scale); \
     else if (n <= 512) moe_route_kernel<T, 1, 4, 8><<<n, 256, 0, stream>>>((const T*)h, ld_h, router, bias, mode, n, C, X, top, ids, weights, groups, keep, scale); \
     else moe_route_kernel<T, 4, 8, 2><<<tw_div_up(n, 4), 512, 0, stream>>>((const T*)h, ld_h, router, bias, mode, n, C, X, top, ids, weights, groups, keep, scale); \
   } while (0)

@@ -232,6 +232,25 @@ def test_router_with_bias_and_softmax_over_the_chosen(device, C, X, top):
         assert not (chosen[both] == 2).any()
 
 
+@pytest.mark.parametrize("C,X,groups", [(256, 20, 1), (1032, 33, 1), (2052, 64, 1), (3072, 65, 5), (600, 200, 1), (516, 128, 8)])
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+def test_a_routers_row_does_not_depend_on_the_others(device, C, X, groups, dtype):
+    """The same bits in steps of 1 to 513 rows, which have other numbers of waves and pieces in flight; against float64 sums."""
+    from tessweave_engine_amd.kernels import ops
+    g = torch.Generator().manual_seed(C)
+    h, router = torch.randn(513, C, generator=g).to(tdtype(dtype)).to(device), (torch.randn(X, C, generator=g) / math.sqrt(C)).to(device)
+    got = {}
+    for n in (1, 64, 65, 512, 513):
+        ids, weights = torch.empty(n, 3, dtype=torch.int32, device=device), torch.empty(n, 3, device=device)
+        ops.moe_route(h[:n], router, 3, ids, weights, groups=(groups, max(1, groups - 2)))
+        got[n] = ids, weights
+    for n in (1, 64, 65, 512):
+        assert all(torch.equal(a[:n], b) for a, b in zip(got[513], got[n]))
+    if groups == 1:
+        want = torch.sigmoid(torch.topk(h.double() @ router.double().T, 3, dim=-1).values)
+        assert (got[513][1].double() - want).abs().max() < 1e-5
+
+
 @pytest.mark.parametrize("X", [5, 63, 64, 65])                       # (up to 64: an expert a lane)
 @pytest.mark.parametrize("weighting", ["sigmoid", "softmax_chosen"])
 def test_router_over_logits_that_are_no_numbers(device, X, weighting):
