@@ -1159,15 +1159,24 @@ static bool narrow_pays(int M, int N, int K, int epf, bool glu, bool sums) {
 }
 
 // Whole K a workgroup where its epilogue spares the kernel that would add the K ranges' sums up anyway: a norm (EndLeave) or the
-// rotation and cache write (EndRotate), LAUNCH microseconds as a node of a captured step. (Four layers and a head, captured steps, us:
+// rotation and cache write (EndRotate), SPARES microseconds as a node of a captured step. (Four layers and a head, captured steps, us:
 // neither / norms that travel / rotation too, at 1, 8 and 16 rows: 896 wide with down products of 4,864 174 / 162 / 155, 188 / 180 / 172, 203 / 195 / 187;
 // 2,048 wide, 11,008: 318 / 303 / 295, 338 / 326 / 316, 363 / 351 / 342; 3,584 wide, 18,944, 1 and 8 rows: 584 / 559 / 561, 629 / 618 / 618. The
 // down products of the last at 8 rows, 3.4 us behind by estimate, gain 6 us a step; those of 2,048 x 11,008 at 4, 3 behind, 2.)
-static bool narrow_end_pays(int M, int N, int K, int epf, double launch) {
-  return M >= 1 && M <= 16 && N % 64 == 0 && K % epf == 0 && narrow_us(M, N, K, epf, false) < skinny_us(M, N, K, epf, false, false) + launch;
+// The rotation's kernel is 2.5 us, and its epilogue here takes 1 of them. Workgroups of 16 waves have a CU to themselves: further turns of them begin when
+// those before end, which the estimate leaves out, and pay for it unless a wave's k-steps are exactly the eight that are on their way from the start. (us, cold
+// weights, apart / here, 1 and 6 rows: bf16 7168 x 5120 18.5 / 18.6, 19.1 / 21.6; 10240 x 5120 24.1 / 26.9, 24.6 / 29.5; 10240 x 3584 18.9 / 19.6, 19.2 / 21.0;
+// float32 5120 x 3072 17.5 / 19.2, 18.1 / 21.1. One turn, eight waves, eight k-steps a wave: 4096 x 5120 13.8 / 10.9, 14.1 / 12.1; 9216 x 2048 12.7 / 9.8, 13.3 /
+// 10.9; 7168 x 4096 18.0 / 14.8, 19.2 / 16.2. Of 900 shapes of 1,152 to 10,240 x 896 to 8,192 and 1 to 16 rows the choice is 0.4 % behind the better of the two;
+// six are more than 2 % slower than apart, the most 6 %.)
+static bool narrow_end_pays(int M, int N, int K, int epf, double spares) {
+  if (M < 1 || M > 16 || N % 64 || K % epf) return false;
+  const int steps = tw_div_up(K / epf, 4);
+  const double turns = steps > 96 && steps != 128 ? 1.2 * (tw_div_up(N / 16, 256) - 1) : 0.0;
+  return narrow_us(M, N, K, epf, false) + turns < skinny_us(M, N, K, epf, false, false) + spares;
 }
 #define TW_LEAVE_SPARES_US 3.5
-#define TW_ROTATE_SPARES_US 1.5
+#define TW_ROTATE_SPARES_US 1.2
 
 // A plain product with an activation behind it, against the K ranges' sums and a kernel that adds them up and applies it (bf16, in a
 // captured graph, cold weights): 4096 x 2048 1 / 8 / 16 rows 7.6 / 4.2, 7.9 / 4.6, 8.5 / 5.2; 5632 x 2048 9.0 / 5.8, 9.5 / 6.6, 10.4 / 7.9;

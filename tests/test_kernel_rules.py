@@ -29,6 +29,16 @@ def test_sums_for_the_next_kernel_over_the_whole_of_k(dtype, m, n, k, whole):
     assert (library().tw_linear_partial_splits_rows(dtype, 1, m, n, k, k) == 1) == whole
 
 
+@pytest.mark.parametrize("dtype,n,k,here,apart", [(BF16, 7168, 5120, (), (3, 6, 10, 16)), (BF16, 10240, 5120, (), (1, 3, 6, 16)), (BF16, 10240, 3584, (), (1, 6, 16)),
+                                                  (BF16, 4608, 8192, (), (1, 6, 16)), (F32, 5120, 3072, (), (1, 3, 16)), (F32, 4608, 3584, (), (1, 6)),
+                                                  (BF16, 4096, 5120, (1, 6, 10), (16,)), (BF16, 9216, 2048, (1, 3, 6), (16,)), (BF16, 7168, 4096, (1, 3, 6), ()),
+                                                  (BF16, 1152, 896, (1, 8, 16), ()), (F32, 7168, 2048, (1, 3, 6), ()), (BF16, 7168, 3072, (1, 3, 6), (16,))])
+def test_products_that_rotate_where_they_are_faster(dtype, n, k, here, apart):
+    """Measured beside split sums that another kernel finishes; those kept apart are 1 to 40 % slower in one (and so are some near the line)."""
+    pays = library().tw_linear_rotate_pays
+    assert all(pays(dtype, m, n, k) for m in here) and not any(pays(dtype, m, n, k) for m in apart)
+
+
 @pytest.mark.parametrize("rows", [1, 8])
 def test_an_activation_behind_few_rows_asks_for_what_its_kernel_takes(rows):
     """Rows 2,050 elements apart are no multiple of 16 bytes apart, which the kernel refuses of a single row too."""
