@@ -32,7 +32,8 @@ __device__ __forceinline__ float ng_half_wave_sum(float v) {    // over a lane's
 // gate asked for behind the reduction, it was two or three trips.
 // (us in a captured graph, before / now: 8 rows of 8 heads of 256 3.3 / 2.4; 4 rows of 8 groups of 512 4.5 / 2.8; 4 rows
 // of 2,048 12.2 and 4.7 / 3.0; 2,048 rows of 16 heads of 128 13.1 / 9.3, 3,000 of 2,048 15.0 / 12.0. With a whole wave a unit of 128 half the
-// lanes had nothing: 14.2.)
+// lanes had nothing: 14.2. Many units of 516 to 768, of which a workgroup's threads have up to half too many: 8,192 of 640 element by element / a workgroup /
+// a wave a unit 14.3 / 15.7 / 10.5, 32,768 42 / 48 / 31; of up to 512 units the workgroup's chain is the shorter one, 2.7 and a wave's 3.1.)
 template <typename T, typename G, int THREADS, int PER, int KIND>
 __global__ __launch_bounds__(256) void norm_gate_kernel(NormGateArgs a) {
   typedef G Gate4 __attribute__((ext_vector_type(4)));
@@ -95,6 +96,7 @@ static bool norm_gate_launch(const NormGateArgs& a, hipStream_t stream) {
   if (a.size <= 128) norm_gate_kernel<T, G, 32, 1, KIND><<<tw_div_up(units, 8), 256, 0, stream>>>(a);
   else if (a.size <= 256) norm_gate_kernel<T, G, 64, 1, KIND><<<tw_div_up(units, 4), 256, 0, stream>>>(a);
   else if (a.size <= 512) norm_gate_kernel<T, G, 64, 2, KIND><<<tw_div_up(units, 4), 256, 0, stream>>>(a);
+  else if (a.size <= 768 && units >= 1024) norm_gate_kernel<T, G, 64, 3, KIND><<<tw_div_up(units, 4), 256, 0, stream>>>(a);
   else if (a.size <= 1024) norm_gate_kernel<T, G, 256, 1, KIND><<<(unsigned)units, 256, 0, stream>>>(a);
   else norm_gate_kernel<T, G, 256, 2, KIND><<<(unsigned)units, 256, 0, stream>>>(a);
   return true;

@@ -1473,3 +1473,18 @@ def test_words_are_fetched_in_segments(ops, device):
     for bad in ((src[1:], dst), (src.clone(), dst), (src, dst.long()), (src, src)):
         with pytest.raises(ValueError):
             ops.WordUpload(*bad)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("size", [516, 640, 768])
+def test_few_and_many_units_of_two_or_three_groups_a_lane(ops, device, dtype, size):
+    """Up to 1,023 units a workgroup each, from there a wave: against float64, and one infinity in a last group."""
+    close = tol(dtype, (4e-6, 4e-6), (1e-30, 2.0 ** -8))
+    for units in (1023, 1024, 1025):
+        y, z, w = rand((units, size), torch.float32, device, 2.0), rand((units, size), torch.float32, device, 2.0, 1), 1 + rand((size,), torch.float32, device, 0.1, 2)
+        got = ops.head_norm_gate(y, z, w, torch.empty(units, size, dtype=dtype, device=device), 1, size, 1e-5)
+        want = y.double() / torch.sqrt((y.double() ** 2).mean(-1, keepdim=True) + 1e-5) * w.double() * z.double() * torch.sigmoid(z.double())
+        torch.testing.assert_close(got.double(), want, **close)
+        y[-1, -3] = float("inf")
+        hit = ops.head_norm_gate(y, z, w, torch.empty_like(got), 1, size, 1e-5)
+        assert torch.equal(hit[:-1], got[:-1]) and hit[-1].isnan().sum() == 1 and hit[-1].nansum() == 0
