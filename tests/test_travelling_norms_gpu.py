@@ -212,6 +212,38 @@ def test_captured_steps_with_norm_weights_anywhere(device, tmp_path, design, nam
     assert errors[-2 if design == "tadalorn" else -1] < 2e-5 and errors[-1] < 1e-3
 
 
+@pytest.mark.parametrize("requests", [1, 16, 17])                       # (17: no norm travels)
+@pytest.mark.parametrize("ff,leaves", [(320, True), (8192, False)])      # (the second: a long K, where K ranges and a norm's kernel are faster)
+@pytest.mark.parametrize("design", ["qwen2", "dinutar"])
+def test_captured_steps_on_either_side_of_the_lines(ops, device, tmp_path, monkeypatch, design, ff, leaves, requests):
+    """Layers whose last product leaves its rows, does not, and steps of more rows than may be left, against eager steps: float32, sums in other
+    orders. The attention's product leaves its rows in all steps of up to 16."""
+    from kanavik_util import Driver, row_error
+    if design == "qwen2":
+        from tessweave_engine_amd.config import config_from_dict
+        from tessweave_engine_amd.weights import write_model_folder
+        from tiny_configs import TINY_B
+        folder = str(tmp_path)
+        write_model_folder(folder, config_from_dict(dict(TINY_B, intermediate_size=ff, rms_norm_eps=1e-3)), 3)
+    else:
+        from dinutar_util import config, latent, make_weights, retention, write_folder
+        c = config([latent(2, 16, 16, 32, 32, 0.25, ff=ff), retention(2, 32, 32, [0.9, 0.99], 32, ff=ff)], width=192, vocab=97, alpha=1.3, scale=0.7, buckets=7,
+                   mul_prev=5, mul_cur=3)
+        folder = write_folder(tmp_path, c, make_weights(c, seed=4))
+    got, widths = [], []
+    plain = ops.linear_leave
+    monkeypatch.setattr(ops, "linear_leave", lambda x, *a, **k: widths.append(x.shape[1]) or plain(x, *a, **k))
+    for graphs in (False, True):
+        d = Driver(folder, "float32", pages=64, page_size=4, max_requests=requests, graphs=graphs)
+        tokens = {f"r{i}": [(7 * i + 5 * j + 3) % d.model.vocab_size for j in range(6)] for i in range(requests)}
+        assert not widths
+        got.append(d.run([[(rid, 1) for rid in tokens] for _ in range(6)], tokens))
+        assert graphs == (d.stepper.graph_replays > 0)
+        d.close()
+    assert bool(widths) == (requests <= 16) and (ff in widths) == (leaves and requests <= 16)
+    assert max(row_error(got[1][rid], got[0][rid]).max() for rid in tokens) < 2e-5
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("n,hidden,form", [(1, 64, "norm"), (16, 896, "two norms"), (3, 4096, "norm"), (40, 2064, "rounded"), (5, 16, "rows alone"), (16, 3072, "no tables")])
 def test_embed_begin(ops, device, dtype, n, hidden, form):
