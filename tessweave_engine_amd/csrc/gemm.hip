@@ -1163,6 +1163,8 @@ static bool narrow_pays(int M, int N, int K, int epf, bool glu, bool sums) {
 // neither / norms that travel / rotation too, at 1, 8 and 16 rows: 896 wide with down products of 4,864 174 / 162 / 155, 188 / 180 / 172, 203 / 195 / 187;
 // 2,048 wide, 11,008: 318 / 303 / 295, 338 / 326 / 316, 363 / 351 / 342; 3,584 wide, 18,944, 1 and 8 rows: 584 / 559 / 561, 629 / 618 / 618. The
 // down products of the last at 8 rows, 3.4 us behind by estimate, gain 6 us a step; those of 2,048 x 11,008 at 4, 3 behind, 2.)
+// On either side of the line: of 600 random products of 512 to 4,096 columns and 1 to 16 rows with the product behind them, 470 leave their rows and take
+// 0.86 of the time, eleven of them more than 1 % longer, the most 7 %; the others would take 1.08, a tenth of them up to 10 % less.
 // The rotation's kernel is 2.5 us, and its epilogue here takes 1 of them. Workgroups of 16 waves have a CU to themselves: further turns of them begin when
 // those before end, which the estimate leaves out, and pay for it unless a wave's k-steps are exactly the eight that are on their way from the start. (us, cold
 // weights, apart / here, 1 and 6 rows: bf16 7168 x 5120 18.5 / 18.6, 19.1 / 21.6; 10240 x 5120 24.1 / 26.9, 24.6 / 29.5; 10240 x 3584 18.9 / 19.6, 19.2 / 21.0;
