@@ -109,8 +109,9 @@ __device__ __forceinline__ void sub_next_norm(const NextNorm& next, const f32x4 
 }
 static bool next_norm_ok(const NextNorm& n) { return n.w == nullptr || (n.out && n.eps > 0.f && (uintptr_t)n.w % 16 == 0); }
 
-// PER groups of four consecutive elements a thread, the row in registers between the two passes.
-template <typename T, int PER, bool EARLY>
+// PER groups of four consecutive elements a thread, the row in registers between the two passes. MORE: with a norm before or behind (a form
+// of its own: its branches cost every launch without them 0.1 us, and 300 rows of 3,072 0.3 of 4).
+template <typename T, int PER, bool EARLY, bool MORE>
 __global__ __launch_bounds__(1024) void residual_norm_vec4_kernel(ResidualNormArgs a) {
   __shared__ float lds[16];
   const int row = blockIdx.x;
@@ -125,7 +126,7 @@ __global__ __launch_bounds__(1024) void residual_norm_vec4_kernel(ResidualNormAr
     if (EARLY && a.scale) sv[i] = *reinterpret_cast<const f32x4*>(a.scale + 4 * c);
   }
   float ss = 0.f;
-  if (EARLY && a.before) {
+  if (EARLY && MORE && a.before) {
     f32x4 bv[PER];
 #pragma unroll
     for (int i = 0; i < PER; ++i) {
@@ -171,7 +172,7 @@ __global__ __launch_bounds__(1024) void residual_norm_vec4_kernel(ResidualNormAr
     if (a.out) sub_store4((T*)a.out + (size_t)row * a.hidden + 4 * c, r, sub_whole4<T>(a.out));
     v[i] = r;
   }
-  if (a.next.w) sub_next_norm<T>(a.next, v, a.hidden, lds);
+  if (MORE && a.next.w) sub_next_norm<T>(a.next, v, a.hidden, lds);
 }
 
 // Any row length: the sums are parked in x between the two passes (a thread reads back only what it wrote).
@@ -223,13 +224,15 @@ static void residual_norm_launch(const ResidualNormArgs& a, int n, hipStream_t s
     const int per = chunks <= 1024 ? 1 : (chunks <= 2048 ? 2 : 4);
     int threads = (chunks + per - 1) / per;
     threads = (threads + 63) / 64 * 64;
-#define TW_ROWS(PER) \
-  (n <= TW_EARLY_ROWS ? residual_norm_vec4_kernel<T, PER, true><<<n, threads, 0, stream>>>(a) \
-                      : residual_norm_vec4_kernel<T, PER, false><<<n, threads, 0, stream>>>(a))
+    const bool more = a.before || a.next.w;
+#define TW_FORM(PER, EARLY) \
+  (more ? residual_norm_vec4_kernel<T, PER, EARLY, true><<<n, threads, 0, stream>>>(a) : residual_norm_vec4_kernel<T, PER, EARLY, false><<<n, threads, 0, stream>>>(a))
+#define TW_ROWS(PER) (n <= TW_EARLY_ROWS ? TW_FORM(PER, true) : TW_FORM(PER, false))
     if (per == 1) TW_ROWS(1);
     else if (per == 2) TW_ROWS(2);
     else TW_ROWS(4);
 #undef TW_ROWS
+#undef TW_FORM
   } else {
     residual_norm_kernel<T><<<n, 256, 0, stream>>>(a);
   }
@@ -318,7 +321,8 @@ struct AddNormedArgs {
 // values in an array indexed by the round had them in scratch memory, asked for each partial sum after the last and for the
 // stream and the weight behind the row's sum. 8 rows of 2,048 with four partial sums 5.4 -> 3.1 us
 // (in a decode step's graph 10.6 -> 4.2), 2,048 rows 23.6 -> 17.6, without partial sums 16.1 -> 10.5.)
-template <typename T, int PER>
+// MORE: with a norm behind (a form of its own, as above).
+template <typename T, int PER, bool MORE>
 __global__ __launch_bounds__(1024) void add_normed_vec4_kernel(AddNormedArgs a) {
   __shared__ __attribute__((aligned(16))) float lds[16];
   const int row = blockIdx.x;
@@ -355,7 +359,7 @@ __global__ __launch_bounds__(1024) void add_normed_vec4_kernel(AddNormedArgs a) 
     if (a.out) sub_store4((T*)a.out + (size_t)row * a.hidden + 4 * c, r, sub_whole4<T>(a.out));
     v[i] = r;
   }
-  if (a.next.w) sub_next_norm<T>(a.next, v, a.hidden, lds);
+  if (MORE && a.next.w) sub_next_norm<T>(a.next, v, a.hidden, lds);
 }
 
 // Any row: W columns a thread and round (four where the result's rows allow: longer rows than the above and streams or weights
@@ -447,9 +451,12 @@ static void add_normed_launch(const AddNormedArgs& a, int n, hipStream_t stream)
   if (add_normed_whole(a)) {
     const int per = chunks <= 1024 ? 1 : chunks <= 2048 ? 2 : 4;
     const int threads = (tw_div_up(chunks, per) + 63) / 64 * 64;
-    if (per == 1) add_normed_vec4_kernel<T, 1><<<n, threads, 0, stream>>>(a);
-    else if (per == 2) add_normed_vec4_kernel<T, 2><<<n, threads, 0, stream>>>(a);
-    else add_normed_vec4_kernel<T, 4><<<n, threads, 0, stream>>>(a);
+#define TW_ROWS(PER) \
+  (a.next.w ? add_normed_vec4_kernel<T, PER, true><<<n, threads, 0, stream>>>(a) : add_normed_vec4_kernel<T, PER, false><<<n, threads, 0, stream>>>(a))
+    if (per == 1) TW_ROWS(1);
+    else if (per == 2) TW_ROWS(2);
+    else TW_ROWS(4);
+#undef TW_ROWS
   } else {
     // (many rows share the chip: a short one's few columns a thread then pay for the block's sums)
     const int units = vec ? chunks : a.hidden, most = n >= 512 && units <= 2048 ? 256 : 1024;
