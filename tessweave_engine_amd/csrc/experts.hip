@@ -786,17 +786,17 @@ struct MoeCombineArgs {
   int C, top, splits, accumulate;
 };
 
-// Columns c .. c + 3 of a row's sum. Of up to four choices at a time the rows' places go out together, then the rows.
+// Columns c .. c + 3 of a row's sum. Of up to four choices at a time the rows' places go out together, then the rows, and the row itself only where a
+// choice has none (2,048 rows of 2,048, two choices of eight experts, all launches 78.4 -> 76 us).
 template <typename T>
 __device__ __forceinline__ f32x4 moe_combined(const MoeCombineArgs& a, int row, int c) {
   f32x4 sum = {0.f, 0.f, 0.f, 0.f};
-  const f32x4 own = moe_four((const T*)a.h + (size_t)row * a.ld_h + c);
   if (a.more)
     for (int s = 0; s < a.splits; ++s) sum += *reinterpret_cast<const f32x4*>(a.more + s * a.more_stride + (size_t)row * a.C + c);
   for (int r0 = 0; r0 < a.top; r0 += 4) {
     int at[4];
     float w[4];
-    f32x4 y[4];
+    f32x4 y[4], own = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       const size_t item = (size_t)row * a.top + min(r0 + j, a.top - 1);
@@ -805,6 +805,7 @@ __device__ __forceinline__ f32x4 moe_combined(const MoeCombineArgs& a, int row, 
     }
 #pragma unroll
     for (int j = 0; j < 4; ++j) y[j] = *reinterpret_cast<const f32x4*>(a.ys + (size_t)max(at[j], 0) * a.ld_y + c);
+    if (min(min(at[0], at[1]), min(at[2], at[3])) < 0) own = moe_four((const T*)a.h + (size_t)row * a.ld_h + c);      // (the same for a row's lanes)
 #pragma unroll
     for (int j = 0; j < 4; ++j)
       if (r0 + j < a.top) sum += w[j] * (at[j] >= 0 ? y[j] : own);
