@@ -36,12 +36,11 @@ class TokenEmbedding(Part):
     def forward(self, ctx):
         if not ctx.capturing:
             return self.gather(ctx)
-        norms, readers = ctx.entry_behind or (None, ())
-        if not ops.can_embed_begin(self.weight, *(norm.weight for norm in norms or ())):
-            return self.gather(ctx)
         # a step of one-token rows: the rotary tables, and the rows as their first reader wants them, are formed in the same launch
-        x = self._stream(ctx)
+        x, norms, readers = self._stream(ctx), *(ctx.entry_behind or (None, ()))
         options, ahead = {}, norm_ahead(ctx, x, norms, readers) if norms else None
+        if not ops.can_embed_begin(self.weight, *(norm.weight for norm in (norms if ahead is not None else ()))):
+            return self.gather(ctx)
         if ahead is not None:
             rows, sums = ahead.buffers(ctx, self.weight.dtype)
             pairs = [(norm.weight, r) for norm, r in zip(norms, rows)]
