@@ -60,7 +60,7 @@ class Part:
     graph_safe = True
 
     #: may the rows a sublayer or a head is given be `ops.NormedRows` (see `NormAhead`)? Only parts whose first use of them is a
-    #: product say so.
+    #: product say so. (This and the next hold of the forward of the class that says them, see `in_force`.)
     takes_normed = False
 
     #: does a sublayer's `forward` end in ONE product into the stream that looks at `ctx.norm_ahead` (`Linear.forward_left`)? A part
@@ -115,6 +115,14 @@ class PositionEncoding(Part):
     def tables(self, ctx):
         """(cos, sin), float32 [n_tokens, rotary_dim / 2] each, from `ctx.positions`."""
         raise NotImplementedError
+
+
+def in_force(part, name):
+    """Does the class whose `forward` runs have NAME of its own? What a part says of its forward (`takes_normed`, `leaves_normed`, a norm's
+    `travels`, a block's `entry`) does not hold of another one: a subclass that overrides forward says it anew, or is run as ever."""
+    if "forward" in vars(part):
+        return False
+    return name in vars(next((cls for cls in type(part).__mro__ if "forward" in vars(cls)), object))
 
 
 class HeadHook(Part):
@@ -226,9 +234,11 @@ class NormAhead:
 def norm_ahead(ctx, stream, norms, readers, after=None):
     """A `NormAhead` if NORMS (each read by one of READERS) can travel in this step, else None."""
     n, width = stream.shape
-    if not ctx.capturing or not ops.can_leave_norms(n, width) or len({norm.eps for norm in norms}) != 1:       # (none: not here either)
+    if not ctx.capturing or not ops.can_leave_norms(n, width):
         return None
-    if not all(getattr(norm, "travels", False) and norm.size == width for norm in norms) or not all(r.takes_normed for r in readers):
+    if not all(in_force(norm, "travels") and norm.size == width for norm in norms) or not all(in_force(r, "takes_normed") and r.takes_normed for r in readers):
+        return None
+    if len({norm.eps for norm in norms}) != 1:       # (none: not here either)
         return None
     return NormAhead(norms, stream, after)
 
@@ -319,7 +329,7 @@ class StepContext:
         self.capturing = False       # launches may depend on kv_bound and capacities, not on this step's lengths
         self.norm_ahead = None       # NormAhead for the sublayer that runs now: the norms that read the stream behind it
         self.norm_behind = None      # the one norm that reads the stream behind the block that runs now, if only one does (captured steps)
-        self.norm_closing = None     # the same for a sublayer whose last kernel writes the stream as that norm will read it: it may norm
+        self.norm_closing = None     # the same for a sublayer that says `closes_norm`, whose last kernel writes the stream as that norm will read it: it may norm
                                      # it there and leave it under NORMED_STREAM
         self.tables_wanted = ()      # rotary encodings whose tables a layer will ask for: an embedding may form them with its rows
         self.entry_behind = None     # (norms, readers) of what runs behind the block that runs now, or None (see Block.entry)

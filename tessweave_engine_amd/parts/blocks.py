@@ -11,7 +11,7 @@ import torch
 from ..cache.spec import CacheNeed
 from ..kernels import ops
 from ..weights.spec import AVERAGE, ONE_PLUS_NORMAL, VECTOR, TensorSpec
-from .base import NORMED_STREAM, ROUNDED_STREAM, Block, fold_pending, norm_ahead
+from .base import NORMED_STREAM, ROUNDED_STREAM, Block, fold_pending, in_force, norm_ahead
 from .norms import LayerNorm, RMSNorm
 
 
@@ -41,10 +41,19 @@ class PreNormBlock(Block):
             return self.ffn.forward(ctx, h, x)
 
 
+def _leaves(sublayer):
+    return sublayer.leaves_normed and in_force(sublayer, "leaves_normed")
+
+
+def _own(norm, kind):
+    """Is NORM of KIND, with that class's forward?"""
+    return isinstance(norm, kind) and type(norm).forward is kind.forward and "forward" not in vars(norm)
+
+
 @contextmanager
 def leaving(ctx, x, sublayer, entry):
     """While SUBLAYER runs, whose last product may leave the stream X for the norms of ENTRY ((norms, readers), or None)."""
-    ctx.norm_ahead = norm_ahead(ctx, x, *entry) if entry is not None and sublayer.leaves_normed else None
+    ctx.norm_ahead = norm_ahead(ctx, x, *entry) if entry is not None and _leaves(sublayer) else None
     try:
         yield
     finally:
@@ -55,7 +64,7 @@ def next_norm(ctx, x, *weights):
     """What `ops.residual_norm` and `ops.add_normed` take as next_norm behind a block's last sublayer, if one norm reads the stream next (captured
     steps) and these rows allow it: the normed rows are then left for it under NORMED_STREAM."""
     norm = ctx.norm_behind
-    if not isinstance(norm, RMSNorm) or norm.size != x.shape[1] or not ops.can_norm_next(x, norm.weight, *weights):
+    if not _own(norm, RMSNorm) or norm.size != x.shape[1] or not ops.can_norm_next(x, norm.weight, *weights):
         return None
     rows = ctx.scratch("norm.out", tuple(x.shape))
     ctx.shared[NORMED_STREAM] = (norm, rows)
@@ -123,7 +132,7 @@ class ParallelBlock(Block):
             more = {"more": left} if left is not None and self.ffn.folds_beside else {}
             if left is not None and not more:
                 fold_pending(x, left)
-            ctx.norm_closing = ctx.norm_behind if isinstance(ctx.norm_behind, RMSNorm) else None
+            ctx.norm_closing = ctx.norm_behind if _own(ctx.norm_behind, RMSNorm) and in_force(self.ffn, "closes_norm") else None
             try:
                 return self.ffn.forward(ctx, h, x, **more)
             finally:
@@ -218,7 +227,7 @@ class PostNormBlock(Block):
         """x <- norm(alpha * x + scale * PART(rows)), ARGS what the part takes before its rows. BEHIND: `ops.NormedRows` where x is still
         the rows of a norm that travels (None: x is the stream). Returns the same of the new stream."""
         result = ctx.scratch("sublayer.result", (ctx.n_tokens, self.hidden), torch.float32)
-        if readers and part.leaves_normed:
+        if readers and _leaves(part):
             ctx.norm_ahead = norm_ahead(ctx, x, (norm,), readers, (behind, behind.norm.weight if behind is not None else None, self.alpha, scale))
         try:
             left = part.forward(ctx, *args, behind if behind is not None else self._rounded(ctx, x), result, accumulate=False)
@@ -348,7 +357,7 @@ class SandwichBlock(Block):
     def forward(self, ctx, run, x, pending=None):
         norm, h = ctx.shared.pop(NORMED_STREAM, (None, None))
         follows = self.next_norm
-        if follows is None and isinstance(ctx.norm_behind, LayerNorm) and ctx.norm_behind.size == self.hidden and ctx.norm_behind.eps == self.mixer_norm.eps:
+        if follows is None and _own(ctx.norm_behind, LayerNorm) and ctx.norm_behind.size == self.hidden and ctx.norm_behind.eps == self.mixer_norm.eps:
             follows = ctx.norm_behind         # (of a captured step, which wants every row)
         if norm is not self.mixer_norm or pending is not None:
             h = normalise(self.mixer_norm, ctx, x, pending)

@@ -34,7 +34,7 @@ class TokenEmbedding(Part):
         return ops.embed_gather(ctx.token_ids, self.weight, self._stream(ctx), feed=ctx.token_feed)
 
     def forward(self, ctx):
-        if not ctx.capturing:
+        if not ctx.capturing or type(self).forward is not TokenEmbedding.forward:       # (a subclass's forward goes on with the rows)
             return self.gather(ctx)
         # a step of one-token rows: the rotary tables, and the rows as their first reader wants them, are formed in the same launch
         x, norms, readers = self._stream(ctx), *(ctx.entry_behind or (None, ()))

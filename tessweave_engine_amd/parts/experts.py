@@ -41,6 +41,7 @@ ApartResult = namedtuple("ApartResult", "add pairs wrote")
 
 class RoutedExperts(FeedForward):
     folds_beside = True
+    closes_norm = True            # (see `StepContext.norm_closing`)
 
     def __init__(self, prefix, hidden, experts, top, intermediate, limit=None, shared=None, router_name="router",
                  expert_names=None, kind="swish_limited", weighting="sigmoid", router_bias=None, identity=0, correction=None,

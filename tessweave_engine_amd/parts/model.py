@@ -5,7 +5,7 @@ import torch
 
 from ..cache.spec import CacheLayout
 from ..kernels import ops
-from .base import EMBEDDING_OUTPUT, LEFT_ROWS, LayerRun, Mixer, Norm, Part, PositionEncoding
+from .base import EMBEDDING_OUTPUT, LEFT_ROWS, LayerRun, Mixer, Norm, Part, PositionEncoding, in_force
 from .blocks import normalise
 from .positions import RotaryEmbedding
 
@@ -127,14 +127,16 @@ class DecoderModel(Part):
         if i + 1 == len(self.schedule):
             return ((self.final_norm,), (self.head,)) if self.schedule else None
         following = self.schedule[i + 1]
-        return None if following.adds_embedding else self.blocks[following.block].entry()
+        block = self.blocks[following.block]
+        return None if following.adds_embedding or not in_force(block, "entry") else block.entry()
 
     def _norm_behind(self, i):
         """The one norm that reads the stream behind run I, or None (see `Block.first_norm`)."""
         if i + 1 == len(self.schedule):
             return self.final_norm
         following = self.schedule[i + 1]
-        return None if following.adds_embedding else self.blocks[following.block].first_norm
+        block = self.blocks[following.block]
+        return None if following.adds_embedding or not in_force(block, "first_norm") else block.first_norm
 
     # ---- one step -----------------------------------------------------------------
     def forward(self, ctx):

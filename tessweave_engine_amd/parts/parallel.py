@@ -23,7 +23,7 @@ import torch
 from ..cache.spec import CacheNeed, FixedState, PagedKV
 from ..kernels import ops
 from ..weights.spec import IDENTITY_PLUS_NORMAL, MATRIX, NORMAL, VECTOR, TensorSpec
-from .base import Mixer, Part
+from .base import Mixer, Part, in_force
 from .convolution import CausalConv
 from .linear import JoinedLinear, Linear
 
@@ -309,7 +309,7 @@ class ParallelMixer(Mixer):
         else:
             proj = ctx.scratch("parallel.proj", (n, sum(self.proj.device_out)), self.proj_dtype)
             extra = [{} for _ in self.branches]
-            stores = self.branches[0].stores(ctx, run) if n <= 16 and proj.dtype == h.dtype and self.proj.takes_normed else None
+            stores = self.branches[0].stores(ctx, run) if n <= 16 and in_force(self.branches[0], "stores") and proj.dtype == h.dtype and self.proj.takes_normed else None
             if stores is not None and ops.linear_rotate_pays(h, self.proj.weights[0], 0):
                 q_heads, kv_heads, size, keys, values, slots = stores
                 ops.linear_rotate(h, self.proj.weights[0], proj, None, None, slots, keys, values, q_heads, kv_heads, size, ctx.cache.page_size,

@@ -212,6 +212,82 @@ def test_captured_steps_with_norm_weights_anywhere(device, tmp_path, design, nam
     assert errors[-2 if design == "tadalorn" else -1] < 2e-5 and errors[-1] < 1e-3
 
 
+def remade(part, **members):
+    """PART with a class of its own that overrides MEMBERS."""
+    part.__class__ = type("Own" + type(part).__name__, (type(part),), members)
+
+
+@pytest.mark.parametrize("which", ["attention", "feed-forward", "norm", "last norm", "embedding", "head", "block", "experts", "branch", "post norm", "wrapped"])
+def test_parts_with_a_forward_of_their_own(device, tmp_path, which):
+    """A program's part that overrides `forward` of one of these is run as it is, whatever the part it comes from allows: captured float32 steps
+    against eager ones, to 2e-5 of the logits' spread."""
+    import importlib
+    from kanavik_util import Driver, row_error
+    design = {"experts": "darolix", "branch": "kanavik", "post norm": "dinutar"}.get(which, "qwen2")
+    if design == "qwen2":
+        from tiny_configs import make_folder
+        make_folder(str(tmp_path), "B320")
+        folder = str(tmp_path)
+    else:
+        util = importlib.import_module(design + "_util")
+        folder = util.write_folder(tmp_path, util.CONFIGS["wide"], util.make_weights(util.CONFIGS["wide"], seed=3))
+    got = []
+    for graphs in (False, True):
+        d = Driver(folder, "float32", pages=24, page_size=4, graphs=graphs)
+        blocks, head, embedding = d.model.blocks, d.model.head, d.model.embedding
+
+        def adds(base):
+            def forward(self, ctx, *args, **options):          # (the stream is the last of a sublayer's arguments)
+                left = base.forward(self, ctx, *args, **options)
+                args[-1].add_(0.25)
+                return left
+            return forward
+
+        def half(ctx, h):
+            return torch.mul(h, 0.5, out=ctx.workspace.get("half", tuple(h.shape), h.dtype))
+
+        def halves(base):
+            return lambda self, ctx, *args, **options: base.forward(self, ctx, *args, **options).mul_(0.5)
+        for block in blocks:
+            if which == "attention":
+                remade(block.mixer, forward=adds(type(block.mixer)))
+            elif which == "feed-forward":
+                remade(block.ffn, forward=adds(type(block.ffn)))
+            elif which == "norm":
+                remade(block.ffn_norm, forward=halves(type(block.ffn_norm)))
+            elif which == "post norm":
+                remade(block.mixer, forward=lambda self, ctx, run, h, x, accumulate=True, base=type(block.mixer):
+                       base.forward(self, ctx, run, half(ctx, h), x, accumulate=accumulate))
+            elif which == "experts" and getattr(block, "ffn", None) is not None:
+                remade(block.ffn, forward=adds(type(block.ffn)))
+            elif which == "branch":
+                base = type(block.mixer.branches[0])
+                remade(block.mixer.branches[0], forward=lambda self, ctx, run, proj, out, scale, base=base: base.forward(self, ctx, run, proj, out, 0.5 * scale))
+            elif which == "wrapped":
+                plain = block.mixer.forward
+                block.mixer.forward = lambda ctx, run, h, x, plain=plain: plain(ctx, run, half(ctx, h), x)
+        if which == "block":
+            base = type(blocks[1])
+
+            def forward(self, ctx, run, x, pending=None):
+                for part in pending if pending is not None else ():
+                    x.add_(part)
+                x.mul_(1.5)
+                return base.forward(self, ctx, run, x, None)
+            remade(blocks[1], forward=forward)
+        elif which == "last norm":
+            remade(d.model.final_norm, forward=halves(type(d.model.final_norm)))
+        elif which == "embedding":
+            remade(embedding, forward=lambda self, ctx, base=type(embedding): base.forward(self, ctx).mul_(3.0))
+        elif which == "head":
+            remade(head, forward=lambda self, ctx, h, base=type(head): base.forward(self, ctx, half(ctx, h)))
+        tokens = {rid: [(s * i + 3) % d.model.vocab_size for i in range(8)] for rid, s in (("a", 7), ("b", 5))}
+        got.append(d.run([[("a", 1), ("b", 1)] for _ in range(8)], tokens))
+        assert (d.stepper.graph_replays > 0) == graphs
+        d.close()
+    assert max(row_error(got[1][rid], got[0][rid]).max() for rid in tokens) < 2e-5
+
+
 @pytest.mark.parametrize("requests", [1, 16, 17])                       # (17: no norm travels)
 @pytest.mark.parametrize("ff,leaves", [(320, True), (8192, False)])      # (the second: a long K, where K ranges and a norm's kernel are faster)
 @pytest.mark.parametrize("design", ["qwen2", "dinutar"])
