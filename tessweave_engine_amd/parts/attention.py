@@ -138,7 +138,8 @@ class GroupedQueryAttention(Mixer):
         adjacent = self.position.pairing == "adjacent"
         keys, values, g = ctx.cache.keys_values(run.cache_slot)
         group = ctx.groups[g]
-        if n <= 16 and self.head_hook is None and self.qkv.takes_normed and ops.linear_rotate_pays(h, self.qkv.weights[0], self.position.rotary_dim):
+        rot = 2 * cos.shape[1] if cos is not None else 0
+        if n <= 16 and self.head_hook is None and self.qkv.takes_normed and ops.linear_rotate_pays(h, self.qkv.weights[0], rot):
             ops.linear_rotate(h, self.qkv.weights[0], qkv, cos, sin, group.slot_mapping, keys, values, self.q_heads, self.kv_heads, self.head_dim,
                               ctx.cache.page_size, write_cache=run.writes_cache, bias=self.qkv.biases[0] if self.qkv.biases else None,
                               adjacent=adjacent)

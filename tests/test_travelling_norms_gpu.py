@@ -288,6 +288,32 @@ def test_parts_with_a_forward_of_their_own(device, tmp_path, which):
     assert max(row_error(got[1][rid], got[0][rid]).max() for rid in tokens) < 2e-5
 
 
+@pytest.mark.parametrize("rot", [16, 20, 32])
+def test_an_encoding_that_gives_its_tables_alone(device, tmp_path, rot):
+    """How much of a head turns is what the tables say: an encoding need not name a size, and one that is no multiple of 16 is turned by the other
+    kernel. Against the engine's own encoding."""
+    from kanavik_util import Driver
+    from tessweave_engine_amd.parts.base import PositionEncoding
+    from tessweave_engine_amd.parts.positions import RotaryEmbedding
+    from tiny_configs import make_folder
+
+    class Tables(PositionEncoding):
+        def __init__(self, inner):
+            self.tables = inner.tables
+    make_folder(str(tmp_path), "B320")
+    got = []
+    for wrap in (lambda p: p, Tables):
+        d = Driver(str(tmp_path), "float32", pages=24, page_size=4)
+        for block in d.model.blocks:
+            encoding = RotaryEmbedding(32, 1e4, rotary_dim=rot)
+            encoding.bind({}, torch.float32, device)
+            block.mixer.position = wrap(encoding)
+        tokens = {"a": [(7 * i + 3) % d.model.vocab_size for i in range(12)]}
+        got.append(d.run([[("a", 5)]] + [[("a", 1)]] * 7, tokens)["a"])
+        d.close()
+    assert (got[0] == got[1]).all()
+
+
 @pytest.mark.parametrize("requests", [1, 16, 17])                       # (17: no norm travels)
 @pytest.mark.parametrize("ff,leaves", [(320, True), (8192, False)])      # (the second: a long K, where K ranges and a norm's kernel are faster)
 @pytest.mark.parametrize("design", ["qwen2", "dinutar"])
