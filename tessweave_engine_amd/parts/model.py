@@ -118,7 +118,7 @@ class DecoderModel(Part):
         """The rotary encodings whose tables some layer asks for in every step, each once."""
         if self._tables is None:
             self._tables = tuple({id(m.position): m.position for run in self.schedule for m in walk(self.blocks[run.block])
-                                  if isinstance(m, Mixer) and m.uses_tables and isinstance(m.position, RotaryEmbedding)}.values())
+                                  if isinstance(m, Mixer) and m.uses_tables and isinstance(m.position, RotaryEmbedding) and m.position.own_tables}.values())
         return self._tables
 
     def _entry_behind(self, i):

@@ -82,6 +82,11 @@ class RotaryEmbedding(PositionEncoding):
         shape = (ctx.n_tokens, self.rotary_dim // 2)
         return tuple(ctx.scratch(f"rotary.{name}.{id(self)}", shape, torch.float32) for name in ("cos", "sin"))
 
+    @property
+    def own_tables(self):
+        """Are `tables` this class's? (not a subclass's, which may need nothing of what these are formed from)"""
+        return type(self).tables is RotaryEmbedding.tables and "tables" not in vars(self)
+
     def table_job(self, ctx):
         """The step's tables as something its caller will form (see `ops.embed_begin`): they count as formed from here on."""
         cos, sin = ctx.shared["rotary", id(self)] = self._table_buffers(ctx)

@@ -217,7 +217,7 @@ def remade(part, **members):
     part.__class__ = type("Own" + type(part).__name__, (type(part),), members)
 
 
-@pytest.mark.parametrize("which", ["attention", "feed-forward", "norm", "last norm", "embedding", "head", "block", "experts", "branch", "post norm", "wrapped"])
+@pytest.mark.parametrize("which", ["attention", "feed-forward", "norm", "last norm", "embedding", "head", "block", "experts", "branch", "post norm", "wrapped", "encoding"])
 def test_parts_with_a_forward_of_their_own(device, tmp_path, which):
     """A program's part that overrides `forward` of one of these is run as it is, whatever the part it comes from allows: captured float32 steps
     against eager ones, to 2e-5 of the logits' spread."""
@@ -266,6 +266,16 @@ def test_parts_with_a_forward_of_their_own(device, tmp_path, which):
             elif which == "wrapped":
                 plain = block.mixer.forward
                 block.mixer.forward = lambda ctx, run, h, x, plain=plain: plain(ctx, run, half(ctx, h), x)
+        if which == "encoding":
+            angle = torch.arange(64, device=device)[:, None] * 0.3 ** torch.arange(16, device=device)[None]
+            kept = (angle.cos(), angle.sin())
+
+            def tables(self, ctx):
+                out = [ctx.workspace.get(name, (ctx.n_tokens, 16), torch.float32) for name in ("own.cos", "own.sin")]
+                return tuple(torch.index_select(t, 0, ctx.positions[0], out=o) for t, o in zip(kept, out))
+            for position in {id(block.mixer.position): block.mixer.position for block in blocks}.values():
+                remade(position, tables=tables)
+                position.inv_freq = position.rest = None
         if which == "block":
             base = type(blocks[1])
 
