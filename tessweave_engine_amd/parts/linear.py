@@ -7,6 +7,8 @@ products per layer become 4. `packed=False` keeps them apart (the reference's
 """
 from __future__ import annotations
 
+from functools import lru_cache
+
 import torch
 
 from ..kernels import ops
@@ -253,8 +255,9 @@ class Linear(Part):
     # ---- norms that travel with the product ---------------------------------------------------
     @property
     def takes_normed(self):
-        """May the input be `ops.NormedRows`? (one packed matrix in the kernels' layout)"""
-        return len(self.weights) == 1 and isinstance(self.weights[0], ops.ShuffledWeight)
+        """May the input be `ops.NormedRows`, and may another kernel take this product's place? (one packed matrix in the kernels' layout, with
+        this class's products: a subclass that adds to them, or replaces one, runs its own)"""
+        return len(self.weights) == 1 and isinstance(self.weights[0], ops.ShuffledWeight) and _own_products(type(self)) and PRODUCTS.isdisjoint(vars(self))
 
     def forward_left(self, ctx, x):
         """Add x @ W.T (+ bias) into the stream of `ctx.norm_ahead` and leave the rows for the norms that read it next, as
@@ -267,6 +270,14 @@ class Linear(Part):
         left = ops.linear_leave(x, self.weights[0], ahead.stream, first.weight, first.eps, rows[0], sums, bias=self.biases[0] if self.biases else None,
                                 second=(second.weight, rows[1]) if second is not None else None, after=ahead.after)
         return ahead.named(left)
+
+
+PRODUCTS = frozenset(("forward", "forward_glu", "forward_act", "forward_partials", "deferrable"))
+
+
+@lru_cache(maxsize=256)
+def _own_products(cls):
+    return all(getattr(cls, name) is getattr(Linear, name) for name in PRODUCTS)
 
 
 class JoinedLinear(Linear):

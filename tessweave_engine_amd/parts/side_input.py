@@ -65,7 +65,7 @@ class TokenSideInput(Part):
         g = ctx.scratch("side.g", (n, self.dim))
         y = ctx.scratch("side.y", (n, self.hidden), torch.float32)
         gate, bias = self.gate.weights[0], self.gate.biases[0] if self.gate.biases else None
-        if ops.linear_token_gate_pays(x, gate):
+        if self.gate.takes_normed and ops.linear_token_gate_pays(x, gate):
             ops.linear_token_gate(x, gate, self.table.weight, ctx.token_ids, self.layer * self.dim, g, feed=ctx.token_feed, bias=bias)
             return self.proj.forward(ctx, g, y)
         rounded = ctx.scratch("side.x", (n, self.hidden))

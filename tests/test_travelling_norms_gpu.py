@@ -298,6 +298,33 @@ def test_parts_with_a_forward_of_their_own(device, tmp_path, which):
     assert max(row_error(got[1][rid], got[0][rid]).max() for rid in tokens) < 2e-5
 
 
+@pytest.mark.parametrize("which", ["qkv", "o", "gate_up", "down", "side"])
+def test_products_of_their_own(device, tmp_path, which):
+    """A product that adds something of its own (and leaves no sums for another kernel to finish) does so for any number of rows: float32, a
+    prompt's 24 rows at once against 5 at a time and one by one, captured."""
+    from kanavik_util import CONFIGS, Driver, make_weights, row_error, write_folder
+    from tiny_configs import make_folder
+    if which == "side":
+        folder = write_folder(tmp_path, CONFIGS["odd"], make_weights(CONFIGS["odd"], seed=3))
+    else:
+        make_folder(str(tmp_path), "B320")
+        folder = str(tmp_path)
+    got, tokens = [], {"a": [(7 * i + 3) % 97 for i in range(24)]}
+    for schedule in ([24], [5, 5, 5, 5, 4], [1] * 24):
+        d = Driver(folder, "float32", pages=24, page_size=4)
+        for block in d.model.blocks:
+            part = block.side.gate if which == "side" else getattr(block.ffn if which in ("gate_up", "down") else block.mixer, which)
+            name, base = "forward_glu" if which == "gate_up" else "forward", type(part)
+
+            def product(self, ctx, x, out, *args, base=base, name=name, **options):
+                getattr(base, name)(self, ctx, x, out, *args, **options)
+                return out.add_(0.125)
+            remade(part, deferrable=lambda self, n: False, **{name: product})
+        got.append(d.run([[("a", n)] for n in schedule], tokens)["a"])
+        d.close()
+    assert max(row_error(got[1], got[0]).max(), row_error(got[2], got[0]).max()) < 2e-5
+
+
 @pytest.mark.parametrize("rot", [16, 20, 32])
 def test_an_encoding_that_gives_its_tables_alone(device, tmp_path, rot):
     """How much of a head turns is what the tables say: an encoding need not name a size, and one that is no multiple of 16 is turned by the other
