@@ -34,7 +34,8 @@ def paged_attention(ctx, q, keys, values, group, out, q_heads, kv_heads, head_di
         # A captured step is replayed for other lengths: the split count follows the step's length class (the kernel itself cuts
         # each sequence's own keys into that many ranges), and the scratch memory the most that any class asks for, so that it never
         # grows under a capture.
-        splits, most = ops.attn_decode_class_splits(ctx.n_decode, q_heads, kv_heads, ctx.kv_bound, ctx.kv_capacity, span, head_dim, q.dtype)
+        splits, most = ops.attn_decode_class_splits(ctx.n_decode, q_heads, kv_heads, ctx.kv_bound or ctx.max_kv_len, ctx.kv_capacity, span, head_dim,
+                                                     q.dtype)
         ws = None
         if splits > 1:
             floats = ops.attn_decode_workspace_floats(ctx.n_decode, q_heads, head_dim, most)

@@ -79,6 +79,19 @@ def test_key_ranges_of_one_token_sequences_fill_whole_turns(dtype, heads, kv_hea
             assert 1 <= splits <= most <= 64
 
 
+@pytest.mark.parametrize("bound,keys,want", [(0, 30000, 44), (32768, 30000, 44), (4096, 3000, 16)])
+def test_key_ranges_of_a_context_made_by_hand(monkeypatch, bound, keys, want):
+    """A context without a length class asks for its longest sequence's ranges."""
+    from types import SimpleNamespace
+    from tessweave_engine_amd.parts.attention import paged_attention
+    seen = []
+    monkeypatch.setattr(ops, "attn_decode", lambda *a, **k: seen.append(k["splits"]))
+    ctx = SimpleNamespace(n_decode=1, n_seqs=1, n_tokens=1, capturing=False, kv_bound=bound, max_kv_len=keys, kv_capacity=32768, q_start=None, kv_len=None,
+                          workspace=SimpleNamespace(get=lambda tag, shape, dtype: torch.empty(shape, dtype=dtype)))
+    paged_attention(ctx, torch.empty(1, 28 * 128, dtype=torch.bfloat16), None, None, SimpleNamespace(block_table=None), None, 28, 4, 128, 0.1)
+    assert abs(seen[0] - want) <= 3
+
+
 def test_key_ranges_are_estimated_once_for_the_layers_of_a_step(monkeypatch):
     shape = (13, 28, 4, 2048, 8192, 0, 128, torch.bfloat16)
     want = ops.attn_decode_class_splits(*shape)
