@@ -11,6 +11,7 @@ The reference has none of this: its layers are fixed attributes of one class
 from __future__ import annotations
 
 from dataclasses import dataclass
+from functools import lru_cache
 import math
 
 import torch
@@ -120,9 +121,12 @@ class PositionEncoding(Part):
 def in_force(part, name):
     """Does the class whose `forward` runs have NAME of its own? What a part says of its forward (`takes_normed`, `leaves_normed`, a norm's
     `travels`, a block's `entry`) does not hold of another one: a subclass that overrides forward says it anew, or is run as ever."""
-    if "forward" in vars(part):
-        return False
-    return name in vars(next((cls for cls in type(part).__mro__ if "forward" in vars(cls)), object))
+    return "forward" not in part.__dict__ and _says(type(part), name)
+
+
+@lru_cache(maxsize=1024)
+def _says(kind, name):
+    return name in vars(next((cls for cls in kind.__mro__ if "forward" in vars(cls)), object))
 
 
 class HeadHook(Part):

@@ -53,7 +53,7 @@ def _own(norm, kind):
 @contextmanager
 def leaving(ctx, x, sublayer, entry):
     """While SUBLAYER runs, whose last product may leave the stream X for the norms of ENTRY ((norms, readers), or None)."""
-    ctx.norm_ahead = norm_ahead(ctx, x, *entry) if entry is not None and _leaves(sublayer) else None
+    ctx.norm_ahead = norm_ahead(ctx, x, *entry) if ctx.capturing and entry is not None and _leaves(sublayer) else None
     try:
         yield
     finally:
@@ -227,7 +227,7 @@ class PostNormBlock(Block):
         """x <- norm(alpha * x + scale * PART(rows)), ARGS what the part takes before its rows. BEHIND: `ops.NormedRows` where x is still
         the rows of a norm that travels (None: x is the stream). Returns the same of the new stream."""
         result = ctx.scratch("sublayer.result", (ctx.n_tokens, self.hidden), torch.float32)
-        if readers and _leaves(part):
+        if ctx.capturing and readers and _leaves(part):
             ctx.norm_ahead = norm_ahead(ctx, x, (norm,), readers, (behind, behind.norm.weight if behind is not None else None, self.alpha, scale))
         try:
             left = part.forward(ctx, *args, behind if behind is not None else self._rounded(ctx, x), result, accumulate=False)

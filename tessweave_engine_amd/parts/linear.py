@@ -257,7 +257,7 @@ class Linear(Part):
     def takes_normed(self):
         """May the input be `ops.NormedRows`, and may another kernel take this product's place? (one packed matrix in the kernels' layout, with
         this class's products: a subclass that adds to them, or replaces one, runs its own)"""
-        return len(self.weights) == 1 and isinstance(self.weights[0], ops.ShuffledWeight) and _own_products(type(self)) and PRODUCTS.isdisjoint(vars(self))
+        return len(self.weights) == 1 and isinstance(self.weights[0], ops.ShuffledWeight) and _own_products(type(self)) and not PRODUCTS & self.__dict__.keys()
 
     def forward_left(self, ctx, x):
         """Add x @ W.T (+ bias) into the stream of `ctx.norm_ahead` and leave the rows for the norms that read it next, as
